@@ -381,7 +381,7 @@ def bench_prefill(args):
         "config": {"workload": "26-layer backbone prefill of 512 random token ids, causal GQA attention "
                                "(BASELINE.json configs[3])",
                    "layers": N_LAYERS, "seq_len": PREFILL_LEN, "weights": "bf16 N(0,0.02) seeded, truncated",
-                   "schedule": ("one launch per product and row pass", "one persistent launch per layer behind the attention")[args.prefill_mode]},
+                   "schedule": "one launch per product and row pass"},
         "tokens_per_s": round(PREFILL_LEN / (ms_step * 1e-3), 1),
         "tflops": round((gemm_fl + attn_fl) / ms_step / 1e9, 1),
         "roofline": {

@@ -415,7 +415,7 @@ extern "C" void tts_hip_set_decode_mode(int mode) {
 }
 extern "C" void tts_hip_set_prefill_mode(int mode) {
     if (mode != 0 && mode != 1) { vt_set_error("tts_hip_set_prefill_mode: unknown schedule %d", mode); return; }
-    g_vt.prefill_mode = mode;
+    /* both numbers name the one schedule there is (see the header) */
 }
 extern "C" void tts_hip_set_barrier_timeout(unsigned long long ticks) { g_vt.bar_timeout = ticks; }
 extern "C" void tts_hip_set_acoustic_grid(int workgroups) {
