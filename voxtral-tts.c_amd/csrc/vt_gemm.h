@@ -21,6 +21,15 @@ void vt_launch_gemm_ex(float *d_C, int ldc, size_t plane_stride, const uint16_t 
 int vt_gemm_frag_shape_ok(int N, int K, int splits);
 void vt_launch_gemm_frag(float *d_C, int ldc, size_t plane_stride, const uint16_t *d_Ahi, const uint16_t *d_Alo,
                          const uint16_t *d_Wf, int M, int N, int K, int splits);
+/* The same product for M <= 64 rows on 64-column tiles (vt_gemm_rows.hip), weights in the same fragment order:
+ * N % 64 == 0, K % 64 == 0; the cuts need not divide K. */
+int vt_gemm_rows_ok(int M, int N, int K);
+int vt_gemm_rows_cuts(int M, int N, int K, int most);
+void vt_launch_gemm_rows(float *d_C, int ldc, size_t plane_stride, const uint16_t *d_Ahi, const uint16_t *d_Alo,
+                         const uint16_t *d_Wf, int M, int N, int K, int splits);
+void vt_launch_gemm_rows_swiglu(uint16_t *d_hhi, uint16_t *d_hlo, int ldh, float *d_tail, const uint16_t *d_Ahi,
+                                const uint16_t *d_Alo, const uint16_t *d_Wf, int M, int n_main, int n_tail, int K,
+                                int tail_splits);
 /* row-major bf16 W[N, K] -> the fragment-order copy (same size); N % 32 == 0, K % 64 == 0.  pair: W holds
  * (gate, up) rows interleaved and every 64 fragment columns become 32 gates followed by their 32 ups
  * (N % 64 == 0), the order vt_launch_gemm_frag_swiglu expects. */

@@ -520,6 +520,13 @@ extern "C" void tts_hip_llm_prefill_out(const float *embeds, int seq_len, int st
      * 192 / 240 / 240 items */
     const int m_tiles = (seq_len + 127) / 128;
     const int fq = vt_prefill_cuts(m_tiles * (VT_QKV_DIM / 256), 4), fo = vt_prefill_cuts(m_tiles * (VT_DIM / 256), 8);
+    /* up to 64 rows: 64-column tiles (vt_gemm_rows.hip); gate|up runs whole tiles on every CU and the rest in K cuts */
+    const bool few = vt_gemm_rows_ok(seq_len, VT_DIM, VT_DIM);
+    const int wq = vt_gemm_rows_cuts(seq_len, VT_QKV_DIM, VT_DIM, 4), wo = vt_gemm_rows_cuts(seq_len, VT_DIM, VT_Q_DIM, 8);
+    const int wd = vt_gemm_rows_cuts(seq_len, VT_DIM, VT_FFN, 8);
+    const int few_main = (2 * VT_FFN / 64) / g_vt.n_cu * g_vt.n_cu * 64, few_tail = 2 * VT_FFN - few_main;
+    int few_cut = 1;                 /* as many cuts of the remaining tiles as give every CU at most one; their planes fit `part` */
+    while (few_cut < 8 && (few_cut + 1) * (few_tail / 64) <= g_vt.n_cu && (few_cut + 1) * few_tail <= 8 * VT_DIM) few_cut++;
     /* the 128 x 128 kernel on row-major weights (layers without a fragment copy) wants cuts that divide K */
     const int rq = m_tiles >= 3 ? 2 : 4, ro = m_tiles >= 3 ? 4 : 8;
     const int tail_cols = m_tiles == 4 ? 16 * 128 : 0;      /* part holds 4 x S x 2048 <= 8 x S x 3072 */
@@ -541,21 +548,27 @@ extern "C" void tts_hip_llm_prefill_out(const float *embeds, int seq_len, int st
         float *vc = g_hip.kv_cache_v_gpu + (size_t)l * g_vt.kv_max * VT_KV_DIM;
         const vt_layer_frag *F = &g_vt.h_frag[l];
         const bool frag = F->wqkv && F->wo && F->w13 && F->w2;
-        const int sp_qkv = frag ? fq : rq, sp_wo = frag ? fo : ro, sp_w2 = sp_wo;
-        if (frag) vt_launch_gemm_frag(wide, VT_QKV_DIM, S * VT_QKV_DIM, hi, lo, F->wqkv, seq_len, VT_QKV_DIM, VT_DIM, sp_qkv);
+        const bool rows = frag && few;
+        const int sp_qkv = rows ? wq : frag ? fq : rq, sp_wo = rows ? wo : frag ? fo : ro, sp_w2 = rows ? wd : frag ? fo : ro;
+        if (rows) vt_launch_gemm_rows(wide, VT_QKV_DIM, S * VT_QKV_DIM, hi, lo, F->wqkv, seq_len, VT_QKV_DIM, VT_DIM, sp_qkv);
+        else if (frag) vt_launch_gemm_frag(wide, VT_QKV_DIM, S * VT_QKV_DIM, hi, lo, F->wqkv, seq_len, VT_QKV_DIM, VT_DIM, sp_qkv);
         else vt_launch_gemm(wide, hi, lo, L->wqkv, seq_len, VT_QKV_DIM, VT_DIM, sp_qkv);
         /* k (rotated) and v into the cache and, with the earlier rows, into the attention's tile images; the
          * attention takes q from the product's planes itself */
         vt_pa_launch_image(img, wide, sp_qkv, S * VT_QKV_DIM, kc, vc, seq_len, start_pos);
         vt_launch_prefill_attention_raw(NULL, hi, lo, wide, VT_QKV_DIM, sp_qkv, S * VT_QKV_DIM, g_vt.d_rope, img,
                                         seq_len, start_pos, VT_ATT_SCALE);
-        if (frag) vt_launch_gemm_frag(part, VT_DIM, ps, hi, lo, F->wo, seq_len, VT_DIM, VT_Q_DIM, sp_wo);
+        if (rows) vt_launch_gemm_rows(part, VT_DIM, ps, hi, lo, F->wo, seq_len, VT_DIM, VT_Q_DIM, sp_wo);
+        else if (frag) vt_launch_gemm_frag(part, VT_DIM, ps, hi, lo, F->wo, seq_len, VT_DIM, VT_Q_DIM, sp_wo);
         else vt_launch_gemm(part, hi, lo, L->wo, seq_len, VT_DIM, VT_Q_DIM, sp_wo);
         vt_launch_residual_norm_split(x, part, sp_wo, ps, L->ffn_norm, hi, lo, seq_len);
         /* with the fragment copies the SiLU(gate) * up planes come out of the product itself, into the wide
          * area (free between q|k|v and the next layer), which the down projection then reads */
         uint16_t *h_hi = (uint16_t *)wide, *h_lo = h_hi + n_plane;
-        if (frag && m_tiles != 4) {
+        if (rows) {
+            vt_launch_gemm_rows_swiglu(h_hi, h_lo, VT_FFN, part, hi, lo, F->w13, seq_len, few_main, few_tail, VT_DIM, few_cut);
+            if (few_tail) vt_launch_swiglu_pair_tail(h_hi, h_lo, VT_FFN, few_main / 2, part, few_cut, S * few_tail, seq_len, few_tail);
+        } else if (frag && m_tiles != 4) {
             vt_launch_gemm_frag_swiglu(h_hi, h_lo, VT_FFN, NULL, hi, lo, F->w13, seq_len, 2 * VT_FFN, 0, VT_DIM, 1);
         } else if (frag) {
             /* 4 M tiles x 72 N tiles of 256 columns are 288 items for 256 CUs: the last 8 N tiles get their K cut
@@ -576,7 +589,8 @@ extern "C" void tts_hip_llm_prefill_out(const float *embeds, int seq_len, int st
             vt_launch_gemm(wide, hi, lo, L->w13, seq_len, 2 * VT_FFN, VT_DIM, 1);
             vt_launch_swiglu_split(hi, lo, wide, S * VT_FFN, 0, NULL, 0, 0);
         }
-        if (frag) vt_launch_gemm_frag(part, VT_DIM, ps, h_hi, h_lo, F->w2, seq_len, VT_DIM, VT_FFN, sp_w2);
+        if (rows) vt_launch_gemm_rows(part, VT_DIM, ps, h_hi, h_lo, F->w2, seq_len, VT_DIM, VT_FFN, sp_w2);
+        else if (frag) vt_launch_gemm_frag(part, VT_DIM, ps, h_hi, h_lo, F->w2, seq_len, VT_DIM, VT_FFN, sp_w2);
         else vt_launch_gemm(part, hi, lo, L->w2, seq_len, VT_DIM, VT_FFN, sp_w2);
         const float *next_norm = l + 1 < g_vt.n_dec_layers ? g_vt.h_layers[l + 1].attn_norm : NULL;
         vt_launch_residual_norm_split(x, part, sp_w2, ps, next_norm, hi, lo, seq_len);
