@@ -68,10 +68,15 @@ static float bench_prefill_kernel(int which, int iters) {
     const int S = 512;
     if (which == 4 && g_vt.kv_max < S) { vt_set_error("tts_hip_bench_kernel: KV cache shorter than 512"); return -1.f; }
     static const int NN[4] = {VT_QKV_DIM, VT_DIM, 2 * VT_FFN, VT_DIM}, KK[4] = {VT_DIM, VT_Q_DIM, VT_DIM, VT_FFN};
-    const int SP[4] = {vt_prefill_cuts(4 * (VT_QKV_DIM / 256), 4), vt_prefill_cuts(4 * (VT_DIM / 256), 8), 1,
-                       vt_prefill_cuts(4 * (VT_DIM / 256), 8)};
+    vt_gemm_plan plan[4];
+    size_t most = 0;
+    for (int i = 0; i < 4; i++) {
+        plan[i] = vt_gemm_frag_plan(S, NN[i], KK[i], i == 2);
+        const size_t n = (size_t)plan[i].cuts * NN[i];
+        most = n > most ? n : most;
+    }
     static const int RP[4] = {2, 4, 1, 4};            /* row-major weights: cuts that divide K */
-    const size_t n_out = (size_t)S * 2 * VT_FFN * 4, n_plane = (size_t)S * VT_FFN, n_q = (size_t)S * VT_Q_DIM;
+    const size_t n_out = (size_t)S * (most + 4 * 2 * VT_FFN), n_plane = (size_t)S * VT_FFN, n_q = (size_t)S * VT_Q_DIM;
     const size_t bytes = sizeof(float) * (n_out + n_q) + 2 * sizeof(uint16_t) * n_plane;
     unsigned char *base = (unsigned char *)vt_scratch(bytes);
     if (!base) return -1.f;
@@ -89,7 +94,7 @@ static float bench_prefill_kernel(int which, int iters) {
     unsigned char *img = NULL;
     if (which == 4) {
         if (!(img = vt_pa_image(S))) return -1.f;
-        vt_pa_launch_image(img, NULL, 0, 0, g_hip.kv_cache_k_gpu, g_hip.kv_cache_v_gpu, S, 0);
+        vt_pa_launch_image(img, NULL, 0, 0, 0, g_hip.kv_cache_k_gpu, g_hip.kv_cache_v_gpu, S, 0);
     }
     for (int it = -2; it < iters; it++) {
         if (it == 0 && vt_check(hipEventRecord(g_vt.ev0, g_vt.stream), "bench start")) return -1.f;
@@ -100,19 +105,17 @@ static float bench_prefill_kernel(int which, int iters) {
         const vt_layer_frag *F = &g_vt.h_frag[(it + 2) % g_vt.n_dec_layers];
         const uint16_t *Wf[4] = {F->wqkv, F->wo, F->w13, F->w2};
         const bool frag = F->wqkv && F->wo && F->w13 && F->w2;
-        if (which == 2 && frag) {                       /* as in the prefill: main part + K-cut tail */
-            const int tail = 8 * 256, main_cols = 2 * VT_FFN - tail;
+        if (which == 2 && frag) {
             uint16_t *h_hi = (uint16_t *)out, *h_lo = h_hi + n_plane;
-            vt_launch_gemm_frag_swiglu(h_hi, h_lo, VT_FFN, out + (size_t)S * 2 * VT_FFN, hi, lo, Wf[2], S, main_cols, tail, VT_DIM,
-                                       VT_W13_TAIL_CUT);
+            vt_launch_gemm_frag_swiglu(h_hi, h_lo, VT_FFN, out + (size_t)S * 2 * VT_FFN, hi, lo, Wf[2], S, 2 * VT_FFN, VT_DIM, plan[2]);
         } else if (which == 2) {
             const int tail = 16 * 128, main_cols = 2 * VT_FFN - tail;
             vt_launch_gemm_ex(out, 2 * VT_FFN, 0, hi, lo, W[2], S, main_cols, VT_DIM, 1);
             vt_launch_gemm_ex(out + (size_t)S * 2 * VT_FFN, tail, (size_t)S * tail, hi, lo,
                               W[2] + (size_t)main_cols * VT_DIM, S, tail, VT_DIM, 4);
-        } else if (which < 4 && frag) vt_launch_gemm_frag(out, NN[which], (size_t)S * NN[which], hi, lo, Wf[which], S, NN[which], KK[which], SP[which]);
+        } else if (which < 4 && frag) vt_launch_gemm_frag(out, NN[which], (size_t)S * NN[which], hi, lo, Wf[which], S, NN[which], KK[which], plan[which]);
         else if (which < 4) vt_launch_gemm(out, hi, lo, W[which], S, NN[which], KK[which], RP[which]);
-        else vt_launch_prefill_attention_raw(out, NULL, NULL, q, VT_Q_DIM, 1, 0, NULL, img, S, 0, VT_ATT_SCALE);
+        else vt_launch_prefill_attention_raw(out, NULL, NULL, q, VT_Q_DIM, 0, 1, 0, NULL, img, S, 0, VT_ATT_SCALE);
     }
     return timed_stop(iters);
 }

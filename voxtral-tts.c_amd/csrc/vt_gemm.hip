@@ -162,304 +162,7 @@ vt_gemm_mfma_kernel(float *C, const uint16_t *Ahi, const uint16_t *Alo, const ui
         }
 }
 
-/* ---- the same product, 128 x 256 tile, one workgroup per CU ---------------------------
- * What bounds the 128 x 128 kernel above is the LDS: a 64 x 64 wave tile reads 24 KB of fragments
- * (two activation planes and the weights) per 32 matrix instructions, three quarters of the LDS
- * bandwidth of a CU with four waves at it, and every K step is a store -> barrier -> read chain.
- * Here a wave owns 128 rows x 64 columns: the weights of its 64 columns are nobody else's in the
- * workgroup, so they go from global memory straight into the B operand registers, and only the
- * activation planes, which all four waves share, pass through the LDS: 8 KB of fragment reads per
- * 16 matrix instructions, half the LDS bandwidth.  Two LDS stages: the planes of K step kt + 1
- * are written while step kt is multiplied, one barrier per step; the global loads of step kt + 2
- * are in flight meanwhile (every request unconditional, so the waits count exactly).  One
- * workgroup of four waves per CU (a wave may then use the whole register file of its SIMD: 128
- * accumulator registers, two sets of weight registers, two sets of fragments).
- * The k order inside a matrix instruction is free as long as both operands agree: lane group g
- * (lane / 32) takes k = 32 g + 8 ks .. + 8 of the 64-wide step in slice ks.
- * A lane's operand is 8 consecutive k of ONE weight row, and the 32 lanes of a group are 32
- * different rows: read from the row-major matrix, every load instruction touches 32 lines 6 KB
- * apart, and the CU's address pipeline, not the matrix cores, sets the pace (measured: 434 against
- * 518 TFLOP/s).  The backbone therefore keeps a second copy of its matrices in fragment order,
- * written once at upload by vt_frag_layout_kernel: every load is then 1 KB of consecutive bytes.
- * Needs N % 256 == 0 and K % 128 == 0: a cut is a whole number of pairs of K steps, and the cuts of one
- * product may differ by one pair (64 steps in 5 cuts: 14, 14, 12, 12, 12), so that the cut count can be
- * chosen to fill the CUs (48 tiles x 5 = 240 items) rather than to divide K. */
-#define GW_TM 128
-#define GW_TN 256
-#define GW_PLANE (GW_TM * GM_ROWB)
-#define GW_STAGE (2 * GW_PLANE)
-#define GW_LDS (2 * GW_STAGE)
-
-struct gw_bregs { u32x4 v[2][4]; };          /* [column block][slice] */
-struct gw_aregs { u32x4 hi[4], lo[4]; };     /* staging: rows lr + 32 i */
-struct gw_frags { bf16x8 hi[4], lo[4]; };    /* one 16-wide slice of the 128 rows, both planes */
-
-/* A launch runs one or two sets of equal work items; workgroup i takes item i of each set in turn (a set
- * may have fewer items than the grid).  The second set lets a product whose tile count is not a multiple
- * of the CU count finish its last tiles as K cuts spread over all CUs inside the same launch. */
-struct gw_part {
-    float *C;                /* output of this set: `splits` planes, plane_stride floats apart, row pitch ldc */
-    const uint16_t *Wf;      /* fragment-order weights of the set's first column */
-    size_t plane_stride;
-    int ldc, n_tiles, splits, k_pairs;   /* k_pairs: K / 128, dealt out over the `splits` cuts */
-    /* gate|up product in the paired column order (vt_launch_frag_layout with pair = 1): instead of C, the
-     * (hi, lo) planes of SiLU(gate) * up, row pitch ldh; the set's first column is h column h_col0 */
-    uint16_t *h_hi, *h_lo;
-    int ldh, h_col0;
-};
-struct gw_plan { gw_part part[2]; int n_parts; };
-
-/* Item `id` of the set P (id < m_tiles * P.n_tiles * P.splits): one 128 x 256 tile over one K cut. */
-__device__ __forceinline__ void gw_run_item(const gw_part &P, int id, const uint16_t *Ahi, const uint16_t *Alo, int M,
-                                            int K, int m_tiles, unsigned char *lds) {
-    const int n_tiles = P.n_tiles, ldc = P.ldc, items = m_tiles * n_tiles * P.splits;
-    float *C = P.C;
-    const uint16_t *Wf = P.Wf;
-    const size_t plane_stride = P.plane_stride;
-    /* Slot id lands on XCD id % 8.  An XCD takes a run of consecutive items, M tile fastest, then N tile,
-     * then K cut: the M tiles of a (K cut, N tile) pair share its weights, the N tiles of a K cut share the
-     * activation planes of that cut, and both then leave the memory side once per XCD instead of once per
-     * workgroup (the two slices are the same size: 128 rows x 4 bytes against 256 rows x 2 bytes). */
-    const int li = (items & 7) == 0 ? (id & 7) * (items >> 3) + (id >> 3) : id;
-    const int mt = li % m_tiles, ci = li / m_tiles, nt = ci % n_tiles, sp = ci / n_tiles;
-    const int t = (int)threadIdx.x, lane = t & 63, wave = t >> 6;
-    const int lr = t >> 3, lc = t & 7;               /* staging: row lr + 32 i, 16-byte chunk lc */
-    /* K is dealt out in pairs of 64-wide steps; the first k_pairs % splits cuts take one pair more */
-    const int pq = P.k_pairs / P.splits, pr = P.k_pairs % P.splits;
-    const int k0 = 2 * GM_BK * (sp * pq + (sp < pr ? sp : pr)), tiles = 2 * (pq + (sp < pr ? 1 : 0));
-
-    /* rows past M read row 0 of the tile again: their products land in accumulator rows that are
-     * never stored (the rows of a matrix instruction do not mix), so nothing has to be zeroed */
-    const uint16_t *pa[4], *pl[4];
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const int gm = mt * GW_TM + lr + 32 * i;
-        const size_t ao = (size_t)(gm < M ? gm : mt * GW_TM) * K + k0 + lc * 8;
-        pa[i] = Ahi + ao;
-        pl[i] = Alo + ao;
-    }
-    const size_t b_blk = (size_t)32 * K;
-
-    auto fetch_a = [&](gw_aregs &r, int kt) {
-        const int adv = (kt < tiles ? kt : tiles - 1) * GM_BK;      /* past the end: the last step once more */
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            r.hi[i] = gm_ld(pa[i] + adv);
-            r.lo[i] = gm_ld(pl[i] + adv);
-        }
-    };
-    /* weights in fragment order (vt_frag_layout_kernel): the 1 KB of slice j of K step ks of column block
-     * nb is contiguous, lane l's 16 bytes at 16 l */
-    const uint16_t *pf = Wf + (size_t)(nt * GW_TN + 64 * wave) * K + (size_t)k0 * 32 + lane * 8;
-    auto fetch_b_slice = [&](gw_bregs &r, int kt, int j) {
-        const int adv = (kt < tiles ? kt : tiles - 1) * 2048;
-        r.v[0][j] = gm_ld(pf + adv + 512 * j);
-        r.v[1][j] = gm_ld(pf + b_blk + adv + 512 * j);
-    };
-    const int st_off = lr * GM_ROWB + lc * 16;
-    auto store_a = [&](const gw_aregs &r, int stage) {
-        unsigned char *base = lds + stage * GW_STAGE + st_off;
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            *reinterpret_cast<u32x4 *>(base + 32 * i * GM_ROWB) = r.hi[i];
-            *reinterpret_cast<u32x4 *>(base + GW_PLANE + 32 * i * GM_ROWB) = r.lo[i];
-        }
-    };
-
-    f32x16 acc[4][2];
-#pragma unroll
-    for (int a = 0; a < 4; a++)
-#pragma unroll
-        for (int b = 0; b < 2; b++)
-#pragma unroll
-            for (int v = 0; v < 16; v++) acc[a][b][v] = 0.f;
-
-    const int fa_off = (lane & 31) * GM_ROWB + (lane >> 5) * 64;
-    auto read_frags = [&](gw_frags &f, int stage, int ks) {
-        const unsigned char *base = lds + stage * GW_STAGE + fa_off + ks * 16;
-#pragma unroll
-        for (int a = 0; a < 4; a++) {
-            f.hi[a] = gm_frag(base + 32 * a * GM_ROWB);
-            f.lo[a] = gm_frag(base + GW_PLANE + 32 * a * GM_ROWB);
-        }
-    };
-    auto mma = [&](const gw_frags &f, const gw_bregs &rb, int ks) {
-        const bf16x8 b0 = __builtin_bit_cast(bf16x8, rb.v[0][ks]), b1 = __builtin_bit_cast(bf16x8, rb.v[1][ks]);
-#pragma unroll
-        for (int a = 0; a < 4; a++) {
-            acc[a][0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.lo[a], b0, acc[a][0], 0, 0, 0);
-            acc[a][1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.lo[a], b1, acc[a][1], 0, 0, 0);
-        }
-#pragma unroll
-        for (int a = 0; a < 4; a++) {
-            acc[a][0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.hi[a], b0, acc[a][0], 0, 0, 0);
-            acc[a][1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.hi[a], b1, acc[a][1], 0, 0, 0);
-        }
-    };
-
-    /* One K step: stage `stage` holds the planes of step kt and `cur` its weights; `ra` holds the planes
-     * of step kt + 1 (requested a step ago); f0 already holds the fragments of slice 0.  Four regions of
-     * sixteen matrix instructions each; the other instructions of a region (the fragment reads of the next
-     * slice, in the first region also the LDS stores of step kt + 1 and the plane requests of step kt + 2,
-     * in the others the two weight requests that refill the slice just used) are dealt out between the
-     * matrix instructions, one after every second, so that the matrix pipe never waits for a block of
-     * them to issue.  The step's one barrier stands in front of the last region: by then every wave has
-     * issued (and waited for) its stores into the other stage and its last reads of this one, so the first
-     * fragments of step kt + 1 are read under the last sixteen matrix instructions of step kt. */
-    gw_aregs ra;
-    gw_frags f0, f1;
-#define GW_FENCE() __builtin_amdgcn_sched_barrier(0)
-#define GW_MFMA2() __builtin_amdgcn_sched_group_barrier(0x008, 2, 0)
-#define GW_DSR1() __builtin_amdgcn_sched_group_barrier(0x100, 1, 0)
-#define GW_DSW1() __builtin_amdgcn_sched_group_barrier(0x200, 1, 0)
-#define GW_VMR1() __builtin_amdgcn_sched_group_barrier(0x020, 1, 0)
-    auto step = [&](int kt, int stage, gw_bregs &cur) {
-        GW_FENCE();
-        store_a(ra, stage ^ 1);
-        fetch_a(ra, kt + 2);
-        read_frags(f1, stage, 1);
-        mma(f0, cur, 0);
-#pragma unroll
-        for (int i = 0; i < 8; i++) { GW_MFMA2(); GW_DSR1(); GW_DSW1(); GW_VMR1(); }
-        GW_FENCE();
-        fetch_b_slice(cur, kt + 2, 0);
-        read_frags(f0, stage, 2);
-        mma(f1, cur, 1);
-#pragma unroll
-        for (int i = 0; i < 8; i++) { GW_MFMA2(); GW_DSR1(); if (i < 2) GW_VMR1(); }
-        GW_FENCE();
-        fetch_b_slice(cur, kt + 2, 1);
-        read_frags(f1, stage, 3);
-        mma(f0, cur, 2);
-#pragma unroll
-        for (int i = 0; i < 8; i++) { GW_MFMA2(); GW_DSR1(); if (i < 2) GW_VMR1(); }
-        GW_FENCE();
-        __syncthreads();
-        GW_FENCE();
-        fetch_b_slice(cur, kt + 2, 2);
-        read_frags(f0, stage ^ 1, 0);
-        mma(f1, cur, 3);
-#pragma unroll
-        for (int i = 0; i < 8; i++) { GW_MFMA2(); GW_DSR1(); if (i < 2) GW_VMR1(); }
-        GW_FENCE();
-        fetch_b_slice(cur, kt + 2, 3);
-    };
-
-    gw_bregs b0, b1;
-    fetch_a(ra, 0);
-#pragma unroll
-    for (int j = 0; j < 4; j++) fetch_b_slice(b0, 0, j);
-    store_a(ra, 0);
-    fetch_a(ra, 1);
-#pragma unroll
-    for (int j = 0; j < 4; j++) fetch_b_slice(b1, 1, j);
-    __syncthreads();
-    read_frags(f0, 0, 0);
-    for (int kt = 0; kt < tiles; kt += 2) {
-        step(kt, 0, b0);
-        step(kt + 1, 1, b1);
-    }
-#undef GW_MFMA2
-#undef GW_DSR1
-#undef GW_DSW1
-#undef GW_VMR1
-#undef GW_FENCE
-
-    /* accumulator element v of lane l: row 8*(v/4) + 4*(l/32) + v%4, column l%32 */
-    if (P.h_hi) {
-        /* a wave's two column blocks are the gates and the ups of the same 32 h columns
-         * (voxtral_tts_llm.c:346-350) */
-        const int hc = P.h_col0 + nt * (GW_TN / 2) + 32 * wave + (lane & 31);
-#pragma unroll
-        for (int a = 0; a < 4; a++)
-#pragma unroll
-            for (int v = 0; v < 16; v++) {
-                const int row = mt * GW_TM + 32 * a + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
-                const float g = acc[a][0][v], u = acc[a][1][v];
-                const float h = __fmul_rn(__fdiv_rn(g, __fadd_rn(1.0f, expf(-g))), u);
-                unsigned sh, sl;
-                vt_split_planes2(h, 0.f, sh, sl);
-                if (row < M) {
-                    P.h_hi[(size_t)row * P.ldh + hc] = (uint16_t)sh;
-                    P.h_lo[(size_t)row * P.ldh + hc] = (uint16_t)sl;
-                }
-            }
-    } else {
-    float *Cs = C + (size_t)sp * plane_stride;
-#pragma unroll
-    for (int a = 0; a < 4; a++)
-#pragma unroll
-        for (int b = 0; b < 2; b++) {
-            const int col = nt * GW_TN + 64 * wave + 32 * b + (lane & 31);
-#pragma unroll
-            for (int v = 0; v < 16; v++) {
-                const int row = mt * GW_TM + 32 * a + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
-                if (row < M) Cs[(size_t)row * ldc + col] = acc[a][b][v];
-            }
-        }
-    }
-    __syncthreads();                 /* the next item refills the LDS stages */
-}
-
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
-vt_gemm_wide_kernel(gw_plan plan, const uint16_t *Ahi, const uint16_t *Alo, int M, int K, int m_tiles) {
-    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-    const int id = (int)blockIdx.x;
-    for (int pi = 0; pi < plan.n_parts; pi++) {
-        const gw_part &P = plan.part[pi];
-        if (id < m_tiles * P.n_tiles * P.splits) gw_run_item(P, id, Ahi, Alo, M, K, m_tiles, lds);
-    }
-}
-
 static int gm_blocks(size_t n);
-
-int vt_gemm_frag_shape_ok(int N, int K, int splits) {
-    return N % GW_TN == 0 && K % (2 * GM_BK) == 0 && splits >= 1 && splits <= K / (2 * GM_BK);
-}
-
-static int gw_ready(void) {
-    static int attr_set = 0;
-    if (!attr_set) {
-        if (vt_check(hipFuncSetAttribute((const void *)vt_gemm_wide_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                         GW_LDS), "product LDS size"))
-            return 0;
-        attr_set = 1;
-    }
-    return 1;
-}
-
-void vt_launch_gemm_frag(float *d_C, int ldc, size_t plane_stride, const uint16_t *d_Ahi, const uint16_t *d_Alo,
-                         const uint16_t *d_Wf, int M, int N, int K, int splits) {
-    if (!gw_ready()) return;
-    const int m_tiles = (M + GW_TM - 1) / GW_TM;
-    gw_plan plan = {};
-    plan.n_parts = 1;
-    plan.part[0] = gw_part{d_C, d_Wf, plane_stride, ldc, N / GW_TN, splits, K / (2 * GM_BK), NULL, NULL, 0, 0};
-    hipLaunchKernelGGL(vt_gemm_wide_kernel, dim3(m_tiles * (N / GW_TN) * splits), dim3(256), GW_LDS, g_vt.stream,
-                       plan, d_Ahi, d_Alo, M, K, m_tiles);
-}
-
-/* gate|up product with the SiLU(gate) * up epilogue (weights in the paired fragment order): the first n_main
- * columns go straight into the planes d_hhi / d_hlo [M, ldh]; the other n_tail columns (0: none) have K cut
- * in tail_splits and leave fp32 planes d_tail [tail_splits][M, n_tail] in the paired column order, which
- * vt_launch_swiglu_pair_tail turns into the last n_tail / 2 plane columns.  One launch. */
-void vt_launch_gemm_frag_swiglu(uint16_t *d_hhi, uint16_t *d_hlo, int ldh, float *d_tail, const uint16_t *d_Ahi,
-                                const uint16_t *d_Alo, const uint16_t *d_Wf, int M, int n_main, int n_tail, int K,
-                                int tail_splits) {
-    if (!gw_ready()) return;
-    const int m_tiles = (M + GW_TM - 1) / GW_TM;
-    gw_plan plan = {};
-    plan.n_parts = n_tail > 0 ? 2 : 1;
-    plan.part[0] = gw_part{NULL, d_Wf, 0, 0, n_main / GW_TN, 1, K / (2 * GM_BK), d_hhi, d_hlo, ldh, 0};
-    int items = m_tiles * (n_main / GW_TN);
-    if (n_tail > 0) {
-        plan.part[1] = gw_part{d_tail, d_Wf + (size_t)n_main * K, (size_t)M * n_tail, n_tail, n_tail / GW_TN, tail_splits,
-                               K / (2 * GM_BK), NULL, NULL, 0, 0};
-        const int items1 = m_tiles * (n_tail / GW_TN) * tail_splits;
-        if (items1 > items) items = items1;
-    }
-    hipLaunchKernelGGL(vt_gemm_wide_kernel, dim3(items), dim3(256), GW_LDS, g_vt.stream, plan, d_Ahi, d_Alo, M, K, m_tiles);
-}
 
 /* Row-major W[N, K] (N % 32 == 0, K % 64 == 0) -> fragment order: the 16 bytes that lane l = 32 g + n % 32
  * feeds to slice j of K step ks of column block nb = n / 32, i.e. W[n][64 ks + 32 g + 8 j .. + 8], go to
@@ -523,12 +226,12 @@ void vt_launch_split(uint16_t *d_hi, uint16_t *d_lo, const float *d_x, size_t n)
 }
 
 /* One workgroup per row of 3072 floats (256 threads x 12):
- *   x[row] += part[0][row] + part[1][row] + ...   (splits > 0; fixed order)
- *   (hi, lo)[row] = split(rmsnorm(x[row]) * w)     (w != NULL)
+ *   x[row] += part[0][row] (+ part[1][row] + ... for the columns from col0 on)   (cuts > 0; fixed order)
+ *   (hi, lo)[row] = split(rmsnorm(x[row]) * w)                                   (w != NULL)
  * The residual add and the normalisation of voxtral_tts_llm.c:332-336,354 /
  * :338-341 in one pass over the row. */
 __global__ void __launch_bounds__(256)
-vt_residual_norm_split_kernel(float *x, const float *part, int splits, size_t part_stride,
+vt_residual_norm_split_kernel(float *x, const float *part, int col0, int cuts, size_t part_stride,
                               const float *w, uint16_t *hi, uint16_t *lo, float eps) {
     /* a thread owns 4 consecutive columns at 4 (t + 256 j): 16-byte loads and stores, 8-byte plane
      * stores (a quarter of the memory instructions of element-wise accesses) */
@@ -539,11 +242,13 @@ vt_residual_norm_split_kernel(float *x, const float *part, int splits, size_t pa
     float ss = 0.f;
 #pragma unroll
     for (int j = 0; j < NJ; j++) {
-        const size_t i = row * VT_DIM + 4 * ((size_t)threadIdx.x + 256 * j);
+        const int c = 4 * ((int)threadIdx.x + 256 * j);
+        const size_t i = row * VT_DIM + c;
         f32x4 a = *reinterpret_cast<const f32x4 *>(x + i);
-        if (splits > 0) {
+        if (cuts > 0) {
             f32x4 p = *reinterpret_cast<const f32x4 *>(part + i);
-            for (int s = 1; s < splits; s++) {
+            const int n = c < col0 ? 1 : cuts;
+            for (int s = 1; s < n; s++) {
                 const f32x4 q = *reinterpret_cast<const f32x4 *>(part + (size_t)s * part_stride + i);
                 p.x = __fadd_rn(p.x, q.x); p.y = __fadd_rn(p.y, q.y);
                 p.z = __fadd_rn(p.z, q.z); p.w = __fadd_rn(p.w, q.w);
@@ -573,10 +278,10 @@ vt_residual_norm_split_kernel(float *x, const float *part, int splits, size_t pa
     }
 }
 
-void vt_launch_residual_norm_split(float *d_x, const float *d_part, int splits, size_t part_stride,
+void vt_launch_residual_norm_split(float *d_x, const float *d_part, int col0, int cuts, size_t part_stride,
                                    const float *d_w, uint16_t *d_hi, uint16_t *d_lo, int rows) {
     hipLaunchKernelGGL(vt_residual_norm_split_kernel, dim3(rows), dim3(256), 0, g_vt.stream, d_x, d_part,
-                       splits, part_stride, d_w, d_hi, d_lo, VT_EPS);
+                       col0, cuts, part_stride, d_w, d_hi, d_lo, VT_EPS);
 }
 
 /* gu [rows, 2*ffn] with (gate, up) adjacent -> (hi, lo) planes of silu(gate)*up

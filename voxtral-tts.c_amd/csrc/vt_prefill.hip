@@ -4,10 +4,11 @@
  * voxtral_tts_llm.c:299-366).
  *
  * Per layer: RMSNorm into (hi, lo) bf16 planes -> q|k|v product on the matrix
- * cores -> RoPE + cache append -> causal attention on the fp32 matrix cores
- * -> output projection (K split in 2) -> residual + RMSNorm -> gate/up product
- * -> SiLU*up -> down projection (K split in 3) -> residual fused with the next
- * layer's RMSNorm.  Weights are the fused layouts of the decode path.
+ * cores -> RoPE + cache append -> causal attention on the matrix cores ->
+ * output projection -> residual + RMSNorm -> gate/up product with SiLU*up ->
+ * down projection -> residual fused with the next layer's RMSNorm.  Tiles and
+ * K cuts of the products follow the row count (vt_gemm_frag_plan); the kernels
+ * between them are told which columns are cut.
  */
 #include "vt_state.h"
 #include "vt_gemm.h"
@@ -70,18 +71,20 @@ __device__ __forceinline__ void pa_planes8(const f32x4 &a, const f32x4 &b, bf16x
  * 4*cg .. + 4 of the 8 keys that lane group sg meets in the second product (slot j: key 16*(j/4) + 4*sg +
  * j%4), so that the transposed V write is one 16-byte store per dim and plane.
  * Rows [start_pos, start_pos + S) come from the q|k|v product when qkv != NULL: the sum of `planes`
- * split-K planes (`plane_stride` floats apart, fixed order), k rotated (adjacent pairs,
+ * split-K planes (`plane_stride` floats apart, fixed order; only the columns from col0 on are cut, a multiple
+ * of 128), k rotated (adjacent pairs,
  * voxtral_tts_kernels.c:616-634; the table holds (cos, sin) per pair), and are appended to the cache on the
  * way (voxtral_tts_llm.c:317-324).  Earlier rows come from the cache; rows from kv_rows on are zeros (their
  * keys are masked).  qkv == NULL: all rows are in the cache (rope is not read). */
 __global__ void __launch_bounds__(256)
-vt_kv_image_kernel(unsigned char *img, int img_tiles, const float *qkv, int planes, size_t plane_stride,
+vt_kv_image_kernel(unsigned char *img, int img_tiles, const float *qkv, int col0, int planes, size_t plane_stride,
                    float *kc, float *vc, const float *rope, int start_pos, int kv_rows) {
     /* threads 0..127 make the K planes of the tile, threads 128..255 the V planes */
     const int tile = (int)blockIdx.x, kvh = (int)blockIdx.y;
     const bool is_v = threadIdx.x >= 128;
     const int tl = (int)threadIdx.x & 127, sg = tl >> 5, cg = tl & 31;
     const int col = kvh * VT_HEAD_DIM + 4 * cg;
+    if (VT_Q_DIM + (is_v ? VT_KV_DIM : 0) + kvh * VT_HEAD_DIM < col0) planes = 1;      /* a head whose columns are not cut */
     float *cache = is_v ? vc : kc;
     f32x4 r8[8];
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
@@ -165,7 +168,7 @@ vt_kv_image_kernel(unsigned char *img, int img_tiles, const float *qkv, int plan
 template <int NSPLIT, int HPW>
 __global__ void __launch_bounds__(64 * HPW * NSPLIT)
 vt_prefill_attention_kernel(float *out, uint16_t *out_hi, uint16_t *out_lo, const float *Q,
-                            int q_stride, int q_planes, size_t q_plane_stride, const float *rope,
+                            int q_stride, int q_col0, int q_planes, size_t q_plane_stride, const float *rope,
                             const unsigned char *img, int img_tiles, int S, int start_pos, float scale) {
     extern __shared__ __attribute__((aligned(16))) unsigned char pa_lds[];
     constexpr int GT = 64 * HPW;                         /* threads of a residue group */
@@ -185,6 +188,7 @@ vt_prefill_attention_kernel(float *out, uint16_t *out_hi, uint16_t *out_lo, cons
     const int q0 = qt * PA_QT;
     const int my_q = q0 + li;
     const int head = kvh * 4 + hsub * HPW + hq;
+    if (head * VT_HEAD_DIM < q_col0) q_planes = 1;       /* a head whose columns are not cut */
     unsigned char *Kt = pa_lds + (size_t)pz * PA_TILE_BYTES, *Vt = Kt + 2 * PA_KPLANE;   /* hi plane, then lo */
 
     /* this lane's query as the B operand of K Q^T: dims 8*g + 32*ks .. + 8 for K step ks, both planes */
@@ -459,19 +463,19 @@ unsigned char *vt_pa_image(int rows) {
 
 /* d_qkv != NULL: rows start_pos .. start_pos + S - 1 are taken from the q|k|v product (summed, k rotated)
  * and appended to the cache d_K / d_V; otherwise all start_pos + S rows are in the cache already */
-void vt_pa_launch_image(unsigned char *d_img, const float *d_qkv, int planes, size_t plane_stride, float *d_K,
-                            float *d_V, int S, int start_pos) {
+void vt_pa_launch_image(unsigned char *d_img, const float *d_qkv, int col0, int planes, size_t plane_stride, float *d_K,
+                        float *d_V, int S, int start_pos) {
     const int rows = start_pos + S;
     hipLaunchKernelGGL(vt_kv_image_kernel, dim3(pa_tiles(rows), VT_KV_HEADS), dim3(256), 0, g_vt.stream, d_img,
-                       pa_tiles(rows), d_qkv, planes, plane_stride, d_K, d_V, g_vt.d_rope, start_pos, rows);
+                       pa_tiles(rows), d_qkv, col0, planes, plane_stride, d_K, d_V, g_vt.d_rope, start_pos, rows);
 }
 
 /* Q rows are q_stride floats apart; out / (out_hi, out_lo) are [S,4096], each optional.  d_rope != NULL: d_Q
- * holds q_planes split-K planes (q_plane_stride floats apart) of the raw q product, to be summed and
+ * holds q_planes split-K planes (q_plane_stride floats apart; heads below column q_col0 have one) of the raw q product, to be summed and
  * rotated with the table rows start_pos .. by the kernel.  d_img: the tile images of the start_pos + S
  * cache rows (vt_kv_image_kernel). */
 void vt_launch_prefill_attention_raw(float *d_out, uint16_t *d_hi, uint16_t *d_lo, const float *d_Q,
-                                     int q_stride, int q_planes, size_t q_plane_stride, const float *d_rope,
+                                     int q_stride, int q_col0, int q_planes, size_t q_plane_stride, const float *d_rope,
                                      const unsigned char *d_img, int S, int start_pos, float scale) {
     static int attr_set = 0;
     if (!attr_set) {
@@ -483,7 +487,7 @@ void vt_launch_prefill_attention_raw(float *d_out, uint16_t *d_hi, uint16_t *d_l
     }
     hipLaunchKernelGGL((vt_prefill_attention_kernel<PA_NSPLIT, PA_HPW>),
                        dim3(VT_KV_HEADS * (4 / PA_HPW), (S + PA_QT - 1) / PA_QT), dim3(64 * PA_HPW * PA_NSPLIT),
-                       pa_lds_bytes(), g_vt.stream, d_out, d_hi, d_lo, d_Q, q_stride, q_planes, q_plane_stride, d_rope,
+                       pa_lds_bytes(), g_vt.stream, d_out, d_hi, d_lo, d_Q, q_stride, q_col0, q_planes, q_plane_stride, d_rope,
                        d_img, pa_tiles(start_pos + S), S, start_pos, scale);
 }
 
@@ -493,17 +497,11 @@ void vt_launch_prefill_attention(float *d_out, uint16_t *d_hi, uint16_t *d_lo, c
     unsigned char *img = vt_pa_image(start_pos + S);
     if (!img) return;
     /* (the image kernel only reads a cache that is complete) */
-    vt_pa_launch_image(img, NULL, 0, 0, const_cast<float *>(d_K), const_cast<float *>(d_V), S, start_pos);
-    vt_launch_prefill_attention_raw(d_out, d_hi, d_lo, d_Q, q_stride, 1, 0, NULL, img, S, start_pos, scale);
+    vt_pa_launch_image(img, NULL, 0, 0, 0, const_cast<float *>(d_K), const_cast<float *>(d_V), S, start_pos);
+    vt_launch_prefill_attention_raw(d_out, d_hi, d_lo, d_Q, q_stride, 0, 1, 0, NULL, img, S, start_pos, scale);
 }
 
 /* ---- backbone prefill ------------------------------------------------------------ */
-
-/* K cuts of a product of `tiles` output tiles: one item per CU at most, `most` planes at most */
-int vt_prefill_cuts(int tiles, int most) {
-    const int c = g_vt.n_cu / tiles;
-    return c < 1 ? 1 : c > most ? most : c;
-}
 
 extern "C" void tts_hip_llm_prefill_out(const float *embeds, int seq_len, int start_pos, float *out_x) {
     if (!g_vt.initialized || g_vt.n_dec_layers < 1) { vt_set_error("tts_hip_llm_prefill: no weights uploaded"); return; }
@@ -514,86 +512,67 @@ extern "C" void tts_hip_llm_prefill_out(const float *embeds, int seq_len, int st
     }
     const size_t S = (size_t)seq_len;
     hipStream_t st = g_vt.stream;
-    /* work area: x | wide f32 (qkv or gate/up) | q | partial planes | hi | lo */
-    /* K is cut into as many ranges as give every CU at most one item (M tiles x N tiles x cuts; the cuts
-     * need not divide K): 4 M tiles at 512 rows are 96 / 48 / 48 tiles for q|k|v / output / down, i.e.
-     * 192 / 240 / 240 items */
+    bool frag = true;                 /* every layer has its fragment-order copy (otherwise: the 128 x 128 kernel on row-major weights) */
+    for (int l = 0; l < g_vt.n_dec_layers; l++) {
+        const vt_layer_frag *F = &g_vt.h_frag[l];
+        frag = frag && F->wqkv && F->wo && F->w13 && F->w2;
+    }
     const int m_tiles = (seq_len + 127) / 128;
-    const int fq = vt_prefill_cuts(m_tiles * (VT_QKV_DIM / 256), 4), fo = vt_prefill_cuts(m_tiles * (VT_DIM / 256), 8);
-    /* up to 64 rows: 64-column tiles (vt_gemm_rows.hip); gate|up runs whole tiles on every CU and the rest in K cuts */
-    const bool few = vt_gemm_rows_ok(seq_len, VT_DIM, VT_DIM);
-    const int wq = vt_gemm_rows_cuts(seq_len, VT_QKV_DIM, VT_DIM, 4), wo = vt_gemm_rows_cuts(seq_len, VT_DIM, VT_Q_DIM, 8);
-    const int wd = vt_gemm_rows_cuts(seq_len, VT_DIM, VT_FFN, 8);
-    const int few_main = (2 * VT_FFN / 64) / g_vt.n_cu * g_vt.n_cu * 64, few_tail = 2 * VT_FFN - few_main;
-    int few_cut = 1;                 /* as many cuts of the remaining tiles as give every CU at most one; their planes fit `part` */
-    while (few_cut < 8 && (few_cut + 1) * (few_tail / 64) <= g_vt.n_cu && (few_cut + 1) * few_tail <= 8 * VT_DIM) few_cut++;
-    /* the 128 x 128 kernel on row-major weights (layers without a fragment copy) wants cuts that divide K */
-    const int rq = m_tiles >= 3 ? 2 : 4, ro = m_tiles >= 3 ? 4 : 8;
-    const int tail_cols = m_tiles == 4 ? 16 * 128 : 0;      /* part holds 4 x S x 2048 <= 8 x S x 3072 */
-    const size_t n_x = S * VT_DIM, n_wide = S * 4 * VT_QKV_DIM, n_part = 8 * S * VT_DIM;
-    const size_t n_plane = S * VT_FFN;                            /* bf16 elements per plane */
-    const size_t bytes = sizeof(float) * (n_x + n_wide + n_part) + 2 * sizeof(uint16_t) * n_plane;
+    vt_gemm_plan pq, po, pg, pd;      /* q|k|v, output, gate|up, down */
+    if (frag) {
+        pq = vt_gemm_frag_plan(seq_len, VT_QKV_DIM, VT_DIM, 0);
+        po = vt_gemm_frag_plan(seq_len, VT_DIM, VT_Q_DIM, 0);
+        pg = vt_gemm_frag_plan(seq_len, 2 * VT_FFN, VT_DIM, 1);
+        pd = vt_gemm_frag_plan(seq_len, VT_DIM, VT_FFN, 0);
+    } else {                          /* cuts that divide K */
+        pq = vt_gemm_plan{0, 0, 0, m_tiles >= 3 ? 2 : 4};
+        po = pd = vt_gemm_plan{0, 0, 0, m_tiles >= 3 ? 4 : 8};
+        /* 4 M tiles x 144 N tiles are 576 workgroups for 512 slots: the last 16 N tiles get their K cut in 4 */
+        pg = vt_gemm_plan{0, 0, 2 * VT_FFN - (m_tiles == 4 ? 16 * 128 : 0), 4};
+    }
+    /* work area: x | q|k|v planes (without fragment copies also the gate|up product) | planes of the output and
+     * down products | planes of the cut gate|up columns | bf16 planes: products' input, SiLU(gate) * up */
+    const int gu_tail = 2 * VT_FFN - pg.col0;
+    const size_t w_qkv = (size_t)pq.cuts * VT_QKV_DIM, w_gu = frag ? 0 : 2 * VT_FFN;
+    const size_t n_x = S * VT_DIM, n_wide = S * (w_qkv > w_gu ? w_qkv : w_gu), n_part = S * VT_DIM * (po.cuts > pd.cuts ? po.cuts : pd.cuts);
+    const size_t n_tail = S * gu_tail * pg.cuts, n_plane = S * VT_FFN;      /* bf16 elements per plane */
+    const size_t bytes = sizeof(float) * (n_x + n_wide + n_part + n_tail) + 4 * sizeof(uint16_t) * n_plane;
     float *x = (float *)vt_scratch(bytes);
     unsigned char *img = vt_pa_image(start_pos + seq_len);
     if (!x || !img) return;
-    float *wide = x + n_x, *part = wide + n_wide;
-    uint16_t *hi = (uint16_t *)(part + n_part), *lo = hi + n_plane;
+    float *wide = x + n_x, *part = wide + n_wide, *tail = part + n_part;
+    uint16_t *hi = (uint16_t *)(tail + n_tail), *lo = hi + n_plane, *h_hi = lo + n_plane, *h_lo = h_hi + n_plane;
     const size_t ps = S * VT_DIM;
 
     VT_TRYV(hipMemcpyAsync(x, embeds, sizeof(float) * n_x, hipMemcpyDefault, st));
-    vt_launch_residual_norm_split(x, NULL, 0, 0, g_vt.h_layers[0].attn_norm, hi, lo, seq_len);
+    vt_launch_residual_norm_split(x, NULL, 0, 0, 0, g_vt.h_layers[0].attn_norm, hi, lo, seq_len);
     for (int l = 0; l < g_vt.n_dec_layers; l++) {
         const vt_layer_dev *L = &g_vt.h_layers[l];
         float *kc = g_hip.kv_cache_k_gpu + (size_t)l * g_vt.kv_max * VT_KV_DIM;
         float *vc = g_hip.kv_cache_v_gpu + (size_t)l * g_vt.kv_max * VT_KV_DIM;
         const vt_layer_frag *F = &g_vt.h_frag[l];
-        const bool frag = F->wqkv && F->wo && F->w13 && F->w2;
-        const bool rows = frag && few;
-        const int sp_qkv = rows ? wq : frag ? fq : rq, sp_wo = rows ? wo : frag ? fo : ro, sp_w2 = rows ? wd : frag ? fo : ro;
-        if (rows) vt_launch_gemm_rows(wide, VT_QKV_DIM, S * VT_QKV_DIM, hi, lo, F->wqkv, seq_len, VT_QKV_DIM, VT_DIM, sp_qkv);
-        else if (frag) vt_launch_gemm_frag(wide, VT_QKV_DIM, S * VT_QKV_DIM, hi, lo, F->wqkv, seq_len, VT_QKV_DIM, VT_DIM, sp_qkv);
-        else vt_launch_gemm(wide, hi, lo, L->wqkv, seq_len, VT_QKV_DIM, VT_DIM, sp_qkv);
+        if (frag) vt_launch_gemm_frag(wide, VT_QKV_DIM, S * VT_QKV_DIM, hi, lo, F->wqkv, seq_len, VT_QKV_DIM, VT_DIM, pq);
+        else vt_launch_gemm(wide, hi, lo, L->wqkv, seq_len, VT_QKV_DIM, VT_DIM, pq.cuts);
         /* k (rotated) and v into the cache and, with the earlier rows, into the attention's tile images; the
          * attention takes q from the product's planes itself */
-        vt_pa_launch_image(img, wide, sp_qkv, S * VT_QKV_DIM, kc, vc, seq_len, start_pos);
-        vt_launch_prefill_attention_raw(NULL, hi, lo, wide, VT_QKV_DIM, sp_qkv, S * VT_QKV_DIM, g_vt.d_rope, img,
+        vt_pa_launch_image(img, wide, pq.col0, pq.cuts, S * VT_QKV_DIM, kc, vc, seq_len, start_pos);
+        vt_launch_prefill_attention_raw(NULL, hi, lo, wide, VT_QKV_DIM, pq.col0, pq.cuts, S * VT_QKV_DIM, g_vt.d_rope, img,
                                         seq_len, start_pos, VT_ATT_SCALE);
-        if (rows) vt_launch_gemm_rows(part, VT_DIM, ps, hi, lo, F->wo, seq_len, VT_DIM, VT_Q_DIM, sp_wo);
-        else if (frag) vt_launch_gemm_frag(part, VT_DIM, ps, hi, lo, F->wo, seq_len, VT_DIM, VT_Q_DIM, sp_wo);
-        else vt_launch_gemm(part, hi, lo, L->wo, seq_len, VT_DIM, VT_Q_DIM, sp_wo);
-        vt_launch_residual_norm_split(x, part, sp_wo, ps, L->ffn_norm, hi, lo, seq_len);
-        /* with the fragment copies the SiLU(gate) * up planes come out of the product itself, into the wide
-         * area (free between q|k|v and the next layer), which the down projection then reads */
-        uint16_t *h_hi = (uint16_t *)wide, *h_lo = h_hi + n_plane;
-        if (rows) {
-            vt_launch_gemm_rows_swiglu(h_hi, h_lo, VT_FFN, part, hi, lo, F->w13, seq_len, few_main, few_tail, VT_DIM, few_cut);
-            if (few_tail) vt_launch_swiglu_pair_tail(h_hi, h_lo, VT_FFN, few_main / 2, part, few_cut, S * few_tail, seq_len, few_tail);
-        } else if (frag && m_tiles != 4) {
-            vt_launch_gemm_frag_swiglu(h_hi, h_lo, VT_FFN, NULL, hi, lo, F->w13, seq_len, 2 * VT_FFN, 0, VT_DIM, 1);
-        } else if (frag) {
-            /* 4 M tiles x 72 N tiles of 256 columns are 288 items for 256 CUs: the last 8 N tiles get their K cut
-             * in VT_W13_TAIL_CUT and every workgroup takes one of those cuts after its whole tile, in the same
-             * launch, instead of 32 workgroups running a second round alone */
-            const int tail = 8 * 256, main_cols = 2 * VT_FFN - tail;
-            vt_launch_gemm_frag_swiglu(h_hi, h_lo, VT_FFN, part, hi, lo, F->w13, seq_len, main_cols, tail, VT_DIM, VT_W13_TAIL_CUT);
-            vt_launch_swiglu_pair_tail(h_hi, h_lo, VT_FFN, main_cols / 2, part, VT_W13_TAIL_CUT, S * tail, seq_len, tail);
-        } else if (tail_cols) {
-            /* 4 M tiles x 144 N tiles are 576 workgroups for 512 slots: the last 16 N tiles get their
-             * K cut in 4 instead of running as a nearly empty second round */
-            const int main_cols = 2 * VT_FFN - tail_cols;
-            vt_launch_gemm_ex(wide, 2 * VT_FFN, 0, hi, lo, L->w13, seq_len, main_cols, VT_DIM, 1);
-            vt_launch_gemm_ex(part, tail_cols, S * tail_cols, hi, lo, L->w13 + (size_t)main_cols * VT_DIM, seq_len,
-                              tail_cols, VT_DIM, 4);
-            vt_launch_swiglu_split(hi, lo, wide, S * VT_FFN, main_cols, part, 4, S * tail_cols);
+        if (frag) vt_launch_gemm_frag(part, VT_DIM, ps, hi, lo, F->wo, seq_len, VT_DIM, VT_Q_DIM, po);
+        else vt_launch_gemm(part, hi, lo, L->wo, seq_len, VT_DIM, VT_Q_DIM, po.cuts);
+        vt_launch_residual_norm_split(x, part, po.col0, po.cuts, ps, L->ffn_norm, hi, lo, seq_len);
+        if (frag) {
+            vt_launch_gemm_frag_swiglu(h_hi, h_lo, VT_FFN, tail, hi, lo, F->w13, seq_len, 2 * VT_FFN, VT_DIM, pg);
         } else {
-            vt_launch_gemm(wide, hi, lo, L->w13, seq_len, 2 * VT_FFN, VT_DIM, 1);
-            vt_launch_swiglu_split(hi, lo, wide, S * VT_FFN, 0, NULL, 0, 0);
+            vt_launch_gemm_ex(wide, 2 * VT_FFN, 0, hi, lo, L->w13, seq_len, pg.col0, VT_DIM, 1);
+            if (gu_tail)
+                vt_launch_gemm_ex(tail, gu_tail, S * gu_tail, hi, lo, L->w13 + (size_t)pg.col0 * VT_DIM, seq_len, gu_tail, VT_DIM, pg.cuts);
+            vt_launch_swiglu_split(h_hi, h_lo, wide, S * VT_FFN, pg.col0, tail, gu_tail ? pg.cuts : 0, S * gu_tail);
         }
-        if (rows) vt_launch_gemm_rows(part, VT_DIM, ps, h_hi, h_lo, F->w2, seq_len, VT_DIM, VT_FFN, sp_w2);
-        else if (frag) vt_launch_gemm_frag(part, VT_DIM, ps, h_hi, h_lo, F->w2, seq_len, VT_DIM, VT_FFN, sp_w2);
-        else vt_launch_gemm(part, hi, lo, L->w2, seq_len, VT_DIM, VT_FFN, sp_w2);
+        if (frag) vt_launch_gemm_frag(part, VT_DIM, ps, h_hi, h_lo, F->w2, seq_len, VT_DIM, VT_FFN, pd);
+        else vt_launch_gemm(part, h_hi, h_lo, L->w2, seq_len, VT_DIM, VT_FFN, pd.cuts);
         const float *next_norm = l + 1 < g_vt.n_dec_layers ? g_vt.h_layers[l + 1].attn_norm : NULL;
-        vt_launch_residual_norm_split(x, part, sp_w2, ps, next_norm, hi, lo, seq_len);
+        vt_launch_residual_norm_split(x, part, pd.col0, pd.cuts, ps, next_norm, hi, lo, seq_len);
     }
     VT_TRYV(hipGetLastError());
     VT_TRYV(hipStreamSynchronize(st));
