@@ -17,3 +17,30 @@ def test_prefill_row_counts_of_the_few_row_tiles(chunks):
 @pytest.mark.parametrize("chunks", [[96, 97], [128, 129], [192, 193], [225], [256, 257], [288, 289]])
 def test_prefill_row_counts_of_the_wide_tiles(chunks):
     _prefill_case(1, chunks, sum(chunks) + 4, lambda n: range(0, n, 3))
+
+
+def test_prefill_with_gates_far_from_zero():
+    """SiLU(gate) * up for gates of +-100 and more, where exp(-gate) over- and underflows: w1 scaled by 64, w2 by 2^-6."""
+    import numpy as np
+    import cases
+    import hipsupport as H
+    import vtsupport as S
+    layer = S.Layer(13)
+    for w, f in ((layer.w1, 64.0), (layer.w2, 2.0 ** -6)):           # powers of two: the bf16 values stay exact
+        w[...] = S.f32_to_bf16_trunc(S.bf16_to_f32(w) * np.float32(f))
+    norm = S.norm_weight(S.DIM, 98)
+    orc = cases.OracleBackend(threads=16)
+    orc.llm_open([layer], norm, 128, n_layers=1)
+    hip = H.Hip(kv_max=128)
+    try:
+        hip.upload_decoder([layer], norm, 1)
+        for s in (37, 80):                                           # both gate|up kernels
+            e = S.f32_normal((s, S.DIM), 90 + s)
+            rx, gx = orc.llm_prefill(e, want_x=True), hip.llm_prefill(e, want_x=True)
+            hip.check()
+            assert np.all(np.isfinite(gx))
+            for r in range(s):
+                mx, l2 = S.rel_errors(rx[r], gx[r])
+                assert mx < 1e-3 and l2 < 1e-3, (s, r, mx, l2)
+    finally:
+        hip.close()

@@ -314,10 +314,10 @@ __global__ void vt_swiglu_split_kernel(uint16_t *hi, uint16_t *lo, const float *
                 }
             }
         }
-        const float a = __fmul_rn(__fdiv_rn(g0.x, __fadd_rn(1.0f, expf(-g0.x))), g0.y);
-        const float b = __fmul_rn(__fdiv_rn(g0.z, __fadd_rn(1.0f, expf(-g0.z))), g0.w);
-        const float c = __fmul_rn(__fdiv_rn(g1.x, __fadd_rn(1.0f, expf(-g1.x))), g1.y);
-        const float d = __fmul_rn(__fdiv_rn(g1.z, __fadd_rn(1.0f, expf(-g1.z))), g1.w);
+        const float a = vt_silu_mul(g0.x, g0.y);
+        const float b = vt_silu_mul(g0.z, g0.w);
+        const float c = vt_silu_mul(g1.x, g1.y);
+        const float d = vt_silu_mul(g1.z, g1.w);
         u32x2 sph, spl;
         vt_split_planes4(a, b, c, d, sph, spl);
         reinterpret_cast<u32x2 *>(hi)[i] = sph;
@@ -350,10 +350,10 @@ __global__ void vt_swiglu_pair_tail_kernel(uint16_t *hi, uint16_t *lo, int ldh, 
             g.x = __fadd_rn(g.x, g2.x); g.y = __fadd_rn(g.y, g2.y); g.z = __fadd_rn(g.z, g2.z); g.w = __fadd_rn(g.w, g2.w);
             u.x = __fadd_rn(u.x, u2.x); u.y = __fadd_rn(u.y, u2.y); u.z = __fadd_rn(u.z, u2.z); u.w = __fadd_rn(u.w, u2.w);
         }
-        const float a = __fmul_rn(__fdiv_rn(g.x, __fadd_rn(1.0f, expf(-g.x))), u.x);
-        const float b = __fmul_rn(__fdiv_rn(g.y, __fadd_rn(1.0f, expf(-g.y))), u.y);
-        const float cc = __fmul_rn(__fdiv_rn(g.z, __fadd_rn(1.0f, expf(-g.z))), u.z);
-        const float d = __fmul_rn(__fdiv_rn(g.w, __fadd_rn(1.0f, expf(-g.w))), u.w);
+        const float a = vt_silu_mul(g.x, u.x);
+        const float b = vt_silu_mul(g.y, u.y);
+        const float cc = vt_silu_mul(g.z, u.z);
+        const float d = vt_silu_mul(g.w, u.w);
         u32x2 sph, spl;
         vt_split_planes4(a, b, cc, d, sph, spl);
         const size_t at = (size_t)row * ldh + h_col0 + 32 * blk + c;

@@ -240,18 +240,14 @@ vt_gemm_wide_kernel(gw_list list, const uint16_t *Ahi, const uint16_t *Alo, int 
         const int row0 = it.mt * TM + 32 * a + 8 * vq + 4 * (lane >> 5), c = lane & 31;
         if (P.h_hi) {
             /* a wave's two column blocks are the gates and the ups of the same 32 h columns (voxtral_tts_llm.c:346-350) */
-            const int hc = it.nt * (TN / 2) + 32 * cw + c;
+            const vt_h_quad h = vt_silu_mul_quad(q0, q1);
+            const size_t at = (size_t)(row0 + h.row) * P.ldh + it.nt * (TN / 2) + 32 * cw + (c & ~1);
 #pragma unroll
-            for (int v = 0; v < 4; v++) {
-                const float g = q0[v], u = q1[v];
-                const float h = __fmul_rn(__fdiv_rn(g, __fadd_rn(1.0f, expf(-g))), u);
-                unsigned sh, sl;
-                vt_split_planes2(h, 0.f, sh, sl);
-                if (row0 + v < M) {
-                    P.h_hi[(size_t)(row0 + v) * P.ldh + hc] = (uint16_t)sh;
-                    P.h_lo[(size_t)(row0 + v) * P.ldh + hc] = (uint16_t)sl;
+            for (int r = 0; r < 2; r++)
+                if (row0 + h.row + r < M) {
+                    *reinterpret_cast<unsigned *>(P.h_hi + at + (size_t)r * P.ldh) = h.hi[r];
+                    *reinterpret_cast<unsigned *>(P.h_lo + at + (size_t)r * P.ldh) = h.lo[r];
                 }
-            }
         } else {
             float *Cs = P.C + (size_t)it.sp * P.plane_stride + it.nt * TN + 64 * cw + c;
 #pragma unroll
