@@ -137,17 +137,16 @@ static float bench_acoustic_phase(int phase, int iters) {
 }
 
 static float bench_codec(int which, int iters) {
-    float *xn, *att, *h;
+    float *x;
     int *codes;
-    if (vt_codec_probe_buffers(&xn, &att, &h, &codes)) return -1.f;
-    const int frames = 200, T = frames * 8;
+    if (vt_codec_probe_buffers(&x, &codes)) return -1.f;
+    const int frames = 200, T = frames * 8, k = which == 3 ? 4096 : 1024;
     if (which == 4) {
         if (vt_check(hipMemsetAsync(codes, 0, (size_t)frames * 37 * sizeof(int), g_vt.stream), "bench clear")) return -1.f;
     } else {
         /* non-zero operands: on zeros the matrix cores draw less power and run at a higher clock */
-        bench_fill((uint16_t *)xn, NULL, (size_t)T * 1024 * 2);
-        bench_fill((uint16_t *)att, NULL, (size_t)T * 1024 * 2);
-        bench_fill((uint16_t *)h, NULL, (size_t)T * 4096 * 2);
+        bench_fill((uint16_t *)x, NULL, (size_t)T * k * 2);
+        vt_codec_probe_fill(x, k);
     }
     for (int it = -2; it < iters; it++) {
         if (it == 0 && vt_check(hipEventRecord(g_vt.ev0, g_vt.stream), "bench start")) return -1.f;

@@ -1,0 +1,109 @@
+/*
+ * vt_codec_gemm.hip - the codec decoder's products (fp32 weights, fp32 activations) on the fp16 matrix cores.
+ *
+ * Every fp32 operand is carried as two fp16 planes, hi = fp16(s x) and lo = fp16(s x - hi), with a power of two s
+ * per row that brings the row's largest magnitude to 2^13 .. 2^14: hi + lo then holds s x to 2^-24 of itself (2^-38
+ * of the row's largest where lo is subnormal), as good as fp32 does.  A product is hi hi + hi lo + lo hi, three
+ * matrix instructions on the same fp32 sums; the lo lo term left out is below 2^-24 of the product, the size of
+ * the rounding of every single addition.  Three fp16 instructions do 16 times the work of an fp32 one each, so the
+ * same product takes 3/16 of the matrix-core time; what it then runs into is the card's power limit.
+ * Measured against float64, error of a row over its l2 norm: 1.4e-7 .. 3.6e-7 (K 1024 .. 7168, rows and elements of
+ * log-normal magnitude) where a plain fp32 product has 2.7e-7 .. 1.1e-6: what remains is the fp32 sums.
+ * Rates, TFLOP/s of the product itself (v_mfma_f32_32x32x2f32 in 128 x 128 tiles before: 75 .. 105): gate|up
+ * 8192 x 1024 at 212 / 848 / 1696 / 8024 rows 150 / 287 / 290 / 335, down 1024 x 4096 111 / 227 / 282 / 336.
+ */
+#include "vt_gemm_tiles.h"
+
+/* ---- weights: row-major fp32 [N, K] -> fragment order, two fp16 planes --------------------------------------- */
+
+/* col_scale[n] = 2^-e, where row n is stored times 2^e */
+__global__ void __launch_bounds__(256) vt_codec_weight_scale_kernel(float *col_scale, const float *W, int K) {
+    __shared__ float red[4];
+    const size_t n = blockIdx.x;
+    float m = 0.f;
+    for (int k = threadIdx.x; k < K; k += 256) m = fmaxf(m, fabsf(W[n * K + k]));
+    for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) col_scale[n] = 1.0f / vt_f16_scale(fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])));
+}
+
+/* 16-byte slot (((n/32 * K/64 + ks) * 2 + plane) * 4 + j) * 64 + l holds elements 64 ks + 32 (l/32) + 8 j .. + 8 of row
+ * 32 (n/32) + l % 32 */
+__global__ void vt_codec_weight_layout_kernel(u32x4 *out, const float *W, const float *col_scale, size_t n_slots, int K) {
+    const int ksteps = K / 64;
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n_slots; i += (size_t)gridDim.x * blockDim.x) {
+        const int l = (int)(i & 63), j = (int)((i >> 6) & 3);
+        const size_t blk = i >> 8, n = blk / ksteps * 32 + (l & 31);
+        const int ks = (int)(blk % ksteps);
+        const float s = 1.0f / col_scale[n];
+        const f32x4 *p = reinterpret_cast<const f32x4 *>(W + n * K + 64 * ks + 32 * (l >> 5) + 8 * j);
+        const f32x4 a = p[0] * s, b = p[1] * s;
+        u32x2 h0, l0, h1, l1;
+        vt_split_f16x4(a, h0, l0);
+        vt_split_f16x4(b, h1, l1);
+        out[(blk * 2) * 256 + j * 64 + l] = u32x4{h0.x, h0.y, h1.x, h1.y};
+        out[(blk * 2 + 1) * 256 + j * 64 + l] = u32x4{l0.x, l0.y, l1.x, l1.y};
+    }
+}
+
+int vt_codec_weight_layout(uint16_t *d_Wf, float *d_col_scale, const float *d_W, int N, int K) {
+    if (vt_check(hipStreamSynchronize(NULL), "codec weight copy")) return -1;      /* d_W may have been copied from device memory */
+    hipLaunchKernelGGL(vt_codec_weight_scale_kernel, dim3(N), dim3(256), 0, g_vt.stream, d_col_scale, d_W, K);
+    const size_t n_slots = (size_t)N * K / 8;
+    hipLaunchKernelGGL(vt_codec_weight_layout_kernel, dim3((unsigned)((n_slots + 255) / 256 > 8192 ? 8192 : (n_slots + 255) / 256)), dim3(256), 0, g_vt.stream,
+                       (u32x4 *)d_Wf, d_W, d_col_scale, n_slots, K);
+    return vt_check(hipGetLastError(), "codec weight layout") || vt_check(hipStreamSynchronize(g_vt.stream), "codec weight layout") ? -1 : 0;
+}
+
+/* ---- launches -------------------------------------------------------------------------------------------------- */
+
+template <int NP>
+static void cg_rows(const gr_plan &plan, int grid, const uint16_t *d_hi, const uint16_t *d_lo, int M, int K) {
+    constexpr int NW = VT_CODEC_ROW_WAVES;
+    static int attr_set = 0;
+    const int lds = NW * 2 * 32 * ((NP + 3) / 4) * GM_STAGE_ROW;
+    if (!attr_set) {
+        if (vt_check(hipFuncSetAttribute((const void *)vt_gemm_rows_kernel<gm_f16x2, NP, NW>, hipFuncAttributeMaxDynamicSharedMemorySize, lds), "product LDS size"))
+            return;
+        attr_set = 1;
+    }
+    hipLaunchKernelGGL((vt_gemm_rows_kernel<gm_f16x2, NP, NW>), dim3(grid), dim3(64 * NW), lds, g_vt.stream, plan, d_hi, d_lo, M, K);
+}
+
+template <int MB, int CW>
+static void cg_wide(const gw_list &list, const uint16_t *d_hi, const uint16_t *d_lo, int M, int K) {
+    constexpr int LDS = 2 * (4 / CW) * 2 * 32 * MB * GM_STAGE_ROW;
+    static int attr_set = 0;
+    if (!attr_set) {
+        if (vt_check(hipFuncSetAttribute((const void *)vt_gemm_wide_kernel<gm_f16x2, MB, CW>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS), "product LDS size"))
+            return;
+        attr_set = 1;
+    }
+    const int items = list.m_tiles * list.part[0].n_tiles * list.part[0].splits;
+    hipLaunchKernelGGL((vt_gemm_wide_kernel<gm_f16x2, MB, CW>), dim3(items < g_vt.n_cu ? items : g_vt.n_cu), dim3(256), LDS, g_vt.stream, list, d_hi, d_lo, M, K);
+}
+
+void vt_launch_codec_gemm(float *d_C, int ldc, size_t plane_stride, const uint16_t *d_hi, const uint16_t *d_lo, const float *d_row_scale,
+                          const uint16_t *d_Wf, const float *d_col_scale, int M, int N, int K, const vt_gemm_plan &pl) {
+    if (pl.mb == 0) {
+        gr_plan plan = {};
+        plan.n_parts = 1;
+        plan.part[0] = gr_part{d_C, d_Wf, plane_stride, ldc, N / GR_TN, pl.cuts, NULL, NULL, 0, d_row_scale, d_col_scale};
+        const int items = plan.part[0].n_tiles * pl.cuts, grid = items < g_vt.n_cu ? items : g_vt.n_cu;
+        static void (*const launch[4])(const gr_plan &, int, const uint16_t *, const uint16_t *, int, int) = {cg_rows<2>, cg_rows<4>, cg_rows<6>, cg_rows<8>};
+        launch[(M + 15) / 16 - 1](plan, grid, d_hi, d_lo, M, K);
+        return;
+    }
+    gw_list list = {};
+    list.m_tiles = (M + 32 * pl.mb - 1) / (32 * pl.mb);
+    gw_part whole = {d_C, d_Wf, plane_stride, ldc, pl.col0 / (64 * pl.cw), 1, NULL, NULL, 0, d_row_scale, d_col_scale};
+    gw_part cut = {d_C + pl.col0, d_Wf + (size_t)pl.col0 * K * 2, plane_stride, ldc, (N - pl.col0) / (64 * pl.cw), pl.cuts, NULL, NULL, 0,
+                   d_row_scale, d_col_scale + pl.col0};
+    if (whole.n_tiles) list.part[list.n_parts++] = whole;
+    if (cut.n_tiles) list.part[list.n_parts++] = cut;
+    if (pl.mb == 4 && pl.cw == 4) cg_wide<4, 4>(list, d_hi, d_lo, M, K);
+    else if (pl.mb == 4) cg_wide<4, 2>(list, d_hi, d_lo, M, K);
+    else if (pl.cw == 4) cg_wide<3, 4>(list, d_hi, d_lo, M, K);
+    else cg_wide<3, 2>(list, d_hi, d_lo, M, K);
+}

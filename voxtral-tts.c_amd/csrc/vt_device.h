@@ -126,6 +126,29 @@ __device__ __forceinline__ void vt_split_planes4(float a, float b, float c, floa
     lo = u32x2{l0, l1};
 }
 
+/* fp32 -> two fp16 planes, for rows scaled by a power of two that brings the largest magnitude to 2^13 .. 2^14
+ * (vt_f16_scale of that magnitude): hi = fp16(x), lo = fp16(x - hi), both to nearest even, so that hi + lo is x to
+ * 2^-24 of itself where lo is normal and to 2^-25 absolute where it is not. */
+__device__ __forceinline__ float vt_f16_scale(float largest) {
+    int e;
+    (void)frexpf(largest, &e);                               /* largest = f 2^e, f in [0.5, 1) */
+    return largest > 0.f ? ldexpf(1.0f, 14 - (e < -100 ? -100 : e > 110 ? 110 : e)) : 1.0f;
+}
+typedef _Float16 vt_f16x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ void vt_split_f16x2(float a, float b, unsigned &hi, unsigned &lo) {
+    const vt_f16x2 h = {(_Float16)a, (_Float16)b};
+    const vt_f16x2 l = {(_Float16)__fsub_rn(a, (float)h.x), (_Float16)__fsub_rn(b, (float)h.y)};
+    hi = __builtin_bit_cast(unsigned, h);
+    lo = __builtin_bit_cast(unsigned, l);
+}
+__device__ __forceinline__ void vt_split_f16x4(const f32x4 &v, u32x2 &hi, u32x2 &lo) {
+    unsigned h0, l0, h1, l1;
+    vt_split_f16x2(v.x, v.y, h0, l0);
+    vt_split_f16x2(v.z, v.w, h1, l1);
+    hi = u32x2{h0, h1};
+    lo = u32x2{l0, l1};
+}
+
 /* Device-scope coherent accesses for the small vectors that workgroups hand
  * to each other inside one kernel.  Each XCD has its own L2, so such data is
  * written through to memory and read past the L2 (relaxed agent-scope

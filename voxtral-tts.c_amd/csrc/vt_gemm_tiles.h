@@ -1,0 +1,612 @@
+/*
+ * vt_gemm_tiles.h - the tile kernels of the sequence-level products C[M,N] = X[M,K] W[N,K]^T on the matrix cores,
+ * fp32 accumulation, for weights in fragment order (vt_launch_frag_layout): vt_gemm_wide_kernel and, for few rows,
+ * vt_gemm_rows_kernel.  Both are templates over the number format (gm_bf16, gm_f16x2 below).
+ */
+#ifndef VT_GEMM_TILES_H
+#define VT_GEMM_TILES_H
+
+#include "vt_state.h"
+#include "vt_gemm.h"
+
+typedef __bf16 gm_bf16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 gm_f16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+#define GM_STAGE_ROW 144                  /* bytes per staged row: 64 elements of 2 bytes + 16 (fragment reads cover all banks) */
+
+/* The backbone: bf16 weights as they are, fp32 activations as two bf16 planes (hi, lo) */
+struct gm_bf16 {
+    static constexpr int WP = 1;          /* weight planes */
+    static constexpr bool SCALED = false;
+    static __device__ __forceinline__ f32x16 mfma(const u32x4 &x, const u32x4 &w, const f32x16 &c) {
+        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(gm_bf16x8, x), __builtin_bit_cast(gm_bf16x8, w), c, 0, 0, 0);
+    }
+};
+/* The codec: fp32 weights and activations as two fp16 planes each, rows of both scaled by powers of two so that the
+ * planes stay in range; x w = hi hi + hi lo + lo hi (lo lo is below 2^-24 of the product).  The factors that
+ * undo the scaling, one per row and one per column, are applied to the sums. */
+struct gm_f16x2 {
+    static constexpr int WP = 2;
+    static constexpr bool SCALED = true;
+    static __device__ __forceinline__ f32x16 mfma(const u32x4 &x, const u32x4 &w, const f32x16 &c) {
+        return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(gm_f16x8, x), __builtin_bit_cast(gm_f16x8, w), c, 0, 0, 0);
+    }
+};
+
+template <int WP> struct gm_weights { u32x4 v[WP][2][4]; };       /* one 64-wide K step: [plane][block of 32 columns][16-wide slice] */
+template <int MB> struct gm_frags { u32x4 hi[MB], lo[MB]; };      /* one 16-wide slice of MB blocks of 32 rows, both planes */
+
+/* A request through a descriptor: one whose size is 0, and a byte offset beyond the size, load nothing (zeros) */
+__device__ __forceinline__ u32x4 gm_ldb(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
+    return __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0);
+}
+
+/* one slice: the small products first; 2 MB independent sums between two products into the same one */
+template <class T, int MB>
+__device__ __forceinline__ void gm_multiply(f32x16 (&acc)[MB][2], const gm_frags<MB> &f, const gm_weights<T::WP> &w, int ks) {
+    if constexpr (T::WP == 2) {
+#pragma unroll
+        for (int a = 0; a < MB; a++)
+#pragma unroll
+            for (int b = 0; b < 2; b++) acc[a][b] = T::mfma(f.hi[a], w.v[1][b][ks], acc[a][b]);
+    }
+#pragma unroll
+    for (int a = 0; a < MB; a++)
+#pragma unroll
+        for (int b = 0; b < 2; b++) acc[a][b] = T::mfma(f.lo[a], w.v[0][b][ks], acc[a][b]);
+#pragma unroll
+    for (int a = 0; a < MB; a++)
+#pragma unroll
+        for (int b = 0; b < 2; b++) acc[a][b] = T::mfma(f.hi[a], w.v[0][b][ks], acc[a][b]);
+}
+
+/* rows row0 .. + 3 of one column (q0) and of the column 32 further on (q1); C points at row 0 of the column */
+template <class T>
+__device__ __forceinline__ void gm_store_quad(float *C, int ldc, int row0, int M, const f32x4 &q0, const f32x4 &q1,
+                                              const float *row_scale, const float *col_scale) {
+    if constexpr (T::SCALED) {
+        const float s0 = col_scale[0], s1 = col_scale[32];
+#pragma unroll
+        for (int v = 0; v < 4; v++)
+            if (row0 + v < M) {
+                const float r = row_scale[row0 + v];
+                C[(size_t)(row0 + v) * ldc] = q0[v] * s0 * r;
+                C[(size_t)(row0 + v) * ldc + 32] = q1[v] * s1 * r;
+            }
+    } else {
+#pragma unroll
+        for (int v = 0; v < 4; v++)
+            if (row0 + v < M) {
+                C[(size_t)(row0 + v) * ldc] = q0[v];
+                C[(size_t)(row0 + v) * ldc + 32] = q1[v];
+            }
+    }
+}
+
+/* ---- more than 64 rows ---------------------------------------------------------------------------------
+ * A wave owns MB x 32 rows (MB 3 or 4) x 64 columns: the weights of its 64 columns are nobody else's among the
+ * waves that work on the same K step, so they go from global memory straight into the B operand registers, and
+ * only the activation planes pass through the LDS: 8 KB of fragment reads per 16 matrix instructions, half
+ * the LDS bandwidth (a 64 x 64 wave tile with both operands in LDS, vt_gemm_mfma_kernel, needs three quarters).
+ * One workgroup of four waves per CU (a wave may then use the whole register file of its SIMD: up to 128
+ * accumulator registers, two sets of weight registers, two sets of fragments), in one of two shapes:
+ *   CW = 4: four waves side by side, tile MB*32 x 256; the planes of one K step serve four waves;
+ *   CW = 2: two waves side by side and two K steps at a time, tile MB*32 x 128; the two halves of K are added
+ *           through LDS at the end.  Half the tile, for row counts whose 256-column tiles do not deal out over
+ *           the CUs, at the price of twice the plane traffic (L2 and LDS stores) per matrix instruction.
+ * Two LDS stages: the planes of the next step are written while this one is multiplied, one barrier per step;
+ * the global loads of the step after that are in flight meanwhile (every request unconditional, through
+ * descriptors whose size says whether there is anything to load, so the waits count exactly).
+ * The k order inside a matrix instruction is free as long as both operands agree: lane group g (lane / 32)
+ * takes k = 32 g + 8 ks .. + 8 of the 64-wide step in slice ks.
+ * A lane's operand is 8 consecutive k of ONE weight row, and the 32 lanes of a group are 32 different rows:
+ * read from the row-major matrix, every load instruction touches 32 lines 6 KB apart, and the CU's address
+ * pipeline, not the matrix cores, sets the pace (measured: 434 against 518 TFLOP/s).  The backbone therefore
+ * keeps a second copy of its matrices in fragment order, written once at upload by vt_frag_layout_kernel:
+ * every load is then 1 KB of consecutive bytes.
+ *
+ * A launch has at most one workgroup per CU, which walks its items: first whole tiles, as many rounds of them
+ * as every CU can take part in, then the tiles that are left as K cuts, so many that every CU gets one.  The
+ * first requests of an item go out in front of the stores of the one before it.  Only the columns of the cut
+ * tiles have more than one partial plane; whoever reads the result is told from which column on (vt_gemm_plan).
+ */
+
+/* One set of equal items: tiles of n_tiles x (row tiles), K in `splits` cuts */
+struct gw_part {
+    float *C;                             /* `splits` planes of [M, ldc], plane_stride floats apart */
+    const uint16_t *Wf;                   /* fragment-order weights of the set's first column */
+    size_t plane_stride;
+    int ldc, n_tiles, splits;
+    /* gate|up product in the paired column order (vt_launch_frag_layout with pair = 1): instead of C, the
+     * (hi, lo) planes of SiLU(gate) * up, row pitch ldh */
+    uint16_t *h_hi, *h_lo;
+    int ldh;
+    const float *row_scale, *col_scale;   /* T::SCALED: factors of the rows and of the set's columns */
+};
+struct gw_list { gw_part part[2]; int n_parts, m_tiles; };
+
+struct gw_item {
+    const unsigned char *w;               /* weights of the tile's first column */
+    int part, mt, nt, sp, s0, ns;         /* this cut's K steps: s0 .. s0 + ns - 1 (64 wide) */
+};
+
+template <int TN, int WP>
+__device__ __forceinline__ gw_item gw_item_at(const gw_list &list, int part, int id, int K) {
+    const gw_part &P = list.part[part];
+    /* Slot id lands on XCD id % 8.  An XCD takes a run of consecutive items, row tile fastest, then N tile,
+     * then K cut: the row tiles of a (K cut, N tile) pair share its weights, the N tiles of a K cut share the
+     * activation planes of that cut, and both leave the memory side once per XCD instead of once per workgroup. */
+    const int items = list.m_tiles * P.n_tiles * P.splits, x = id & 7, run = items >> 3, rem = items & 7;
+    const int li = x * run + min(x, rem) + (id >> 3);
+    gw_item it;
+    it.part = part;
+    it.mt = li % list.m_tiles;
+    const int ci = li / list.m_tiles;
+    it.nt = ci % P.n_tiles;
+    it.sp = ci / P.n_tiles;
+    const int steps = K / 64, q = steps / P.splits, r = steps % P.splits;
+    it.ns = q + (it.sp < r ? 1 : 0);
+    it.s0 = it.sp * q + min(it.sp, r);
+    it.w = (const unsigned char *)(P.Wf + (size_t)it.nt * TN * K * WP);
+    return it;
+}
+
+template <class T, int MB, int CW>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
+vt_gemm_wide_kernel(gw_list list, const uint16_t *Ahi, const uint16_t *Alo, int M, int K) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+    constexpr int WP = T::WP, KW = 4 / CW, TM = 32 * MB, TN = 64 * CW;
+    constexpr int NP = 4 * MB / CW;                        /* staging passes over a plane, 8 * CW rows each */
+    constexpr int PLANE = TM * GM_STAGE_ROW, GROUP = 2 * PLANE, STAGE = KW * GROUP;
+    const int lane = (int)threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int cw = wave % CW, kw = wave / CW;              /* column block of the tile; which of the KW K steps */
+    const int tg = (int)threadIdx.x - kw * 64 * CW;
+    const int lr = tg >> 3, lc = tg & 7;                   /* staging: row lr + 8 CW p, 16-byte chunk lc */
+    const int a_voff = (lr * K + lc * 8) * 2, a_pass = 16 * CW * K, blk_bytes = 64 * K * WP;
+    const int st_off = kw * GROUP + lr * GM_STAGE_ROW + lc * 16;
+    const int fa_off = kw * GROUP + (lane & 31) * GM_STAGE_ROW + (lane >> 5) * 64;
+
+    struct aregs { u32x4 hi[NP], lo[NP]; };                /* staged rows of one K step, both planes */
+    /* rows past M and steps past the cut's end: beyond the descriptor's size, nothing is loaded (zeros) */
+    auto fetch_a = [&](const gw_item &it, const uint16_t *plane, u32x4 (&r)[NP], int i) {
+        const int s = KW * i + kw, rows = min(M - it.mt * TM, TM);
+        const bool live = s < it.ns;
+        const __amdgpu_buffer_rsrc_t d = __builtin_amdgcn_make_buffer_rsrc((void *)(plane + (size_t)it.mt * TM * K), 0, live ? rows * K * 2 : 0, 0x00020000);
+        const int soff = live ? (it.s0 + s) * 128 : 0;
+#pragma unroll
+        for (int p = 0; p < NP; p++) r[p] = gm_ldb(d, a_voff + p * a_pass, soff);
+    };
+    auto fetch_b_slice = [&](const gw_item &it, gm_weights<WP> &r, int i, int j) {
+        const int s = KW * i + kw;
+        const bool live = s < it.ns;
+        const __amdgpu_buffer_rsrc_t d = __builtin_amdgcn_make_buffer_rsrc((void *)(it.w + (size_t)cw * 2 * blk_bytes), 0, live ? 2 * blk_bytes : 0, 0x00020000);
+        const int soff = live ? (it.s0 + s) * 4096 * WP : 0;
+#pragma unroll
+        for (int p = 0; p < WP; p++) {
+            r.v[p][0][j] = gm_ldb(d, lane * 16 + 1024 * j, soff + 4096 * p);
+            r.v[p][1][j] = gm_ldb(d, lane * 16 + 1024 * j, soff + 4096 * p + (live ? blk_bytes : 0));
+        }
+    };
+    auto store_a = [&](const u32x4 (&r)[NP], int at) {
+#pragma unroll
+        for (int p = 0; p < NP; p++) *reinterpret_cast<u32x4 *>(lds + at + st_off + 8 * CW * p * GM_STAGE_ROW) = r[p];
+    };
+    typedef gm_frags<MB> frags;
+    auto read_frags = [&](frags &f, int stage, int ks) {
+        const unsigned char *base = lds + stage * STAGE + fa_off + ks * 16;
+#pragma unroll
+        for (int a = 0; a < MB; a++) {
+            f.hi[a] = *reinterpret_cast<const u32x4 *>(base + 32 * a * GM_STAGE_ROW);
+            f.lo[a] = *reinterpret_cast<const u32x4 *>(base + PLANE + 32 * a * GM_STAGE_ROW);
+        }
+    };
+    f32x16 acc[MB][2];
+    auto mma = [&](const frags &f, const gm_weights<WP> &w, int ks) { gm_multiply<T, MB>(acc, f, w, ks); };
+
+    /* One step: stage `stage` holds the planes of step i and `cur` its weights; ra holds the planes of step
+     * i + 1 (requested two steps ago: with one step between request and store, the step takes as long as a load,
+     * 1.2 us, whatever the tile); f0 already holds the fragments of slice 0.  Four regions of 4 MB (6 MB with
+     * two weight planes) matrix instructions each; the other instructions of a region (the fragment reads of the next slice, in the first
+     * two also the LDS stores of a plane of step i + 1 and its requests of step i + 3, in all but the first the
+     * weight requests that refill the slice just used) are dealt out between the matrix instructions, one
+     * after every second or third, so that the matrix pipe never waits for a block of them to issue.  The step's one
+     * barrier stands in front of the last region: by then every wave has issued (and waited for) its stores
+     * into the other stage and its last reads of this one, so the first fragments of step i + 1 are read under
+     * the last matrix instructions of step i. */
+    gm_weights<WP> b0, b1;
+    aregs ra0, ra1;                       /* the rows of even and of odd steps */
+    frags f0, f1;
+#define GW_FENCE() __builtin_amdgcn_sched_barrier(0)
+#define GW_MFMA() __builtin_amdgcn_sched_group_barrier(0x008, 1 + WP, 0)
+#define GW_DSR1() __builtin_amdgcn_sched_group_barrier(0x100, 1, 0)
+#define GW_DSW1() __builtin_amdgcn_sched_group_barrier(0x200, 1, 0)
+#define GW_VMR1() __builtin_amdgcn_sched_group_barrier(0x020, 1, 0)
+    auto step = [&](const gw_item &it, int i, int stage, gm_weights<WP> &cur, aregs &ra) {
+        const int other = (stage ^ 1) * STAGE;
+        GW_FENCE();
+        store_a(ra.hi, other);
+        fetch_a(it, Ahi, ra.hi, i + 3);
+        read_frags(f1, stage, 1);
+        mma(f0, cur, 0);
+#pragma unroll
+        for (int k = 0; k < 2 * MB; k++) { GW_MFMA(); GW_DSR1(); if (k < NP) { GW_DSW1(); GW_VMR1(); } }
+        GW_FENCE();
+        store_a(ra.lo, other + PLANE);
+        fetch_a(it, Alo, ra.lo, i + 3);
+        fetch_b_slice(it, cur, i + 2, 0);
+        read_frags(f0, stage, 2);
+        mma(f1, cur, 1);
+#pragma unroll
+        for (int k = 0; k < 2 * MB; k++) { GW_MFMA(); GW_DSR1(); if (k < NP) { GW_DSW1(); GW_VMR1(); } if (k < 2 * WP) GW_VMR1(); }
+        GW_FENCE();
+        fetch_b_slice(it, cur, i + 2, 1);
+        read_frags(f1, stage, 3);
+        mma(f0, cur, 2);
+#pragma unroll
+        for (int k = 0; k < 2 * MB; k++) { GW_MFMA(); GW_DSR1(); if (k < 2 * WP) GW_VMR1(); }
+        GW_FENCE();
+        __syncthreads();
+        GW_FENCE();
+        fetch_b_slice(it, cur, i + 2, 2);
+        read_frags(f0, stage ^ 1, 0);
+        mma(f1, cur, 3);
+#pragma unroll
+        for (int k = 0; k < 2 * MB; k++) { GW_MFMA(); GW_DSR1(); if (k < 2 * WP) GW_VMR1(); }
+        GW_FENCE();
+        fetch_b_slice(it, cur, i + 2, 3);
+    };
+    /* the first requests of an item: the planes and weights of steps 0 and 1 */
+    auto begin = [&](const gw_item &it) {
+        fetch_a(it, Ahi, ra0.hi, 0);
+        fetch_a(it, Alo, ra0.lo, 0);
+#pragma unroll
+        for (int j = 0; j < 4; j++) fetch_b_slice(it, b0, 0, j);
+        fetch_a(it, Ahi, ra1.hi, 1);
+        fetch_a(it, Alo, ra1.lo, 1);
+#pragma unroll
+        for (int j = 0; j < 4; j++) fetch_b_slice(it, b1, 1, j);
+        GW_FENCE();
+    };
+    auto multiply = [&](const gw_item &it) {
+#pragma unroll
+        for (int a = 0; a < MB; a++)
+#pragma unroll
+            for (int b = 0; b < 2; b++)
+#pragma unroll
+                for (int v = 0; v < 16; v++) acc[a][b][v] = 0.f;
+        store_a(ra0.hi, 0);
+        store_a(ra0.lo, PLANE);
+        fetch_a(it, Ahi, ra0.hi, 2);
+        fetch_a(it, Alo, ra0.lo, 2);
+        GW_FENCE();
+        __syncthreads();
+        read_frags(f0, 0, 0);
+        const int n = (it.ns + KW - 1) / KW;
+        int i = 0;
+        for (; i + 1 < n; i += 2) {
+            step(it, i, 0, b0, ra1);
+            step(it, i + 1, 1, b1, ra0);
+        }
+        if (i < n) step(it, i, 0, b0, ra1);
+    };
+#undef GW_MFMA
+#undef GW_DSR1
+#undef GW_DSW1
+#undef GW_VMR1
+#undef GW_FENCE
+
+    /* accumulator element v of lane l: row 8*(v/4) + 4*(l/32) + v%4, column l%32; quad (a, vq) holds v = 4 vq .. + 3 */
+    auto emit = [&](const gw_part &P, const gw_item &it, int a, int vq, const f32x4 &q0, const f32x4 &q1) {
+        const int row0 = it.mt * TM + 32 * a + 8 * vq + 4 * (lane >> 5), c = lane & 31;
+        if (!T::SCALED && P.h_hi) {
+            /* a wave's two column blocks are the gates and the ups of the same 32 h columns (voxtral_tts_llm.c:346-350) */
+            const vt_h_quad h = vt_silu_mul_quad(q0, q1);
+            const size_t at = (size_t)(row0 + h.row) * P.ldh + it.nt * (TN / 2) + 32 * cw + (c & ~1);
+#pragma unroll
+            for (int r = 0; r < 2; r++)
+                if (row0 + h.row + r < M) {
+                    *reinterpret_cast<unsigned *>(P.h_hi + at + (size_t)r * P.ldh) = h.hi[r];
+                    *reinterpret_cast<unsigned *>(P.h_lo + at + (size_t)r * P.ldh) = h.lo[r];
+                }
+        } else {
+            const int col = it.nt * TN + 64 * cw + c;
+            gm_store_quad<T>(P.C + (size_t)it.sp * P.plane_stride + col, P.ldc, row0, M, q0, q1, P.row_scale, P.col_scale + col);
+        }
+    };
+    auto quad = [&](int a, int b, int vq) { return f32x4{acc[a][b][4 * vq], acc[a][b][4 * vq + 1], acc[a][b][4 * vq + 2], acc[a][b][4 * vq + 3]}; };
+    auto finish = [&](const gw_item &it) {
+        const gw_part &P = list.part[it.part];
+        if constexpr (KW == 1) {
+#pragma unroll
+            for (int a = 0; a < MB; a++)
+#pragma unroll
+                for (int vq = 0; vq < 4; vq++) emit(P, it, a, vq, quad(a, 0, vq), quad(a, 1, vq));
+        } else {
+            /* the two waves of a column block hold the sums over the even and the odd K steps: each parks the half
+             * of its quads that the other one finishes */
+            float *park = reinterpret_cast<float *>(lds) + (size_t)wave * (MB * 4 * 256);
+            const float *theirs = reinterpret_cast<const float *>(lds) + (size_t)(wave ^ CW) * (MB * 4 * 256);
+            __syncthreads();
+#pragma unroll
+            for (int a = 0; a < MB; a++)
+#pragma unroll
+                for (int h = 0; h < 2; h++)
+#pragma unroll
+                    for (int b = 0; b < 2; b++)
+                        *reinterpret_cast<f32x4 *>(park + (((a * 2 + h) * 2 + b) * 64 + lane) * 4) = kw == 0 ? quad(a, b, 2 + h) : quad(a, b, h);
+            __syncthreads();
+#pragma unroll
+            for (int a = 0; a < MB; a++)
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    f32x4 q[2];
+#pragma unroll
+                    for (int b = 0; b < 2; b++) {
+                        const f32x4 o = *reinterpret_cast<const f32x4 *>(theirs + (((a * 2 + h) * 2 + b) * 64 + lane) * 4);
+                        const f32x4 m = kw == 0 ? quad(a, b, h) : quad(a, b, 2 + h);
+                        q[b] = f32x4{__fadd_rn(m.x, o.x), __fadd_rn(m.y, o.y), __fadd_rn(m.z, o.z), __fadd_rn(m.w, o.w)};
+                    }
+                    emit(P, it, a, kw == 0 ? h : 2 + h, q[0], q[1]);
+                }
+        }
+    };
+
+    int part = 0, id = (int)blockIdx.x;
+    gw_item it = gw_item_at<TN, WP>(list, 0, id, K);
+    begin(it);
+    for (;;) {
+        multiply(it);
+        id += (int)gridDim.x;
+        while (part < list.n_parts && id >= list.m_tiles * list.part[part].n_tiles * list.part[part].splits) {
+            part++;
+            id = (int)blockIdx.x;
+        }
+        if (part >= list.n_parts) break;
+        const gw_item nx = gw_item_at<TN, WP>(list, part, id, K);
+        begin(nx);
+        finish(it);
+        __syncthreads();                  /* the next item stages over what this one read */
+        it = nx;
+    }
+    finish(it);
+}
+
+
+/* ---- up to 64 rows (a short prompt) -----------------------------------------------------------------------
+ * With so few rows the product is a weight stream: at 64 rows a CU needs 1024 of the 2900 cycles in which its
+ * share of HBM delivers 32 KB of weights.  What counts is that every CU has a share, and an equal one.  A tile
+ * of vt_gemm_wide_kernel is 256 columns wide, so gate|up has 72 of them for 256 CUs, and the other products
+ * can only give more CUs something to do by cutting K into many planes.  Here a workgroup owns 64 columns and
+ * its waves share K among themselves: wave w takes the 64-wide K steps w, w + NW, ... of the workgroup's range,
+ * keeps its own sums for all rows, and the waves' sums are added through LDS at the end (in wave order: the
+ * result does not depend on timing).  288 gate|up tiles (256 whole and the last 32 in 8 K cuts), 96 q|k|v tiles
+ * in 2 cuts, 48 output and down tiles in 4 and 5 then fill the chip with at most 5 planes.
+ *
+ * No two waves work on the same K step, so nobody shares anything before the end: a wave stages its own
+ * activation rows through its own piece of LDS (one stage; the LDS serves a wave's accesses in order, so the
+ * rows of the next step are written over those of this one behind its last reads) and there is no barrier in
+ * the K loop.  The weights of a step go straight into the B operand registers, two steps ahead.  Every request
+ * goes through a buffer descriptor whose size says whether there is anything to load: steps past a wave's last
+ * one and rows past M ask for nothing, without a branch (behind a branch the compiler would wait for all
+ * outstanding loads).
+ *
+ * What bounds it, from 26 layers in rotation: the stream plus about 4 us of launch, first latency, sums and
+ * stores, plus the activation rows, which every workgroup reads for itself at about 50 KB/us per CU (1.3 us per
+ * 8 rows in the gate|up product; that is why the passes over the rows are a template argument and the kernel is
+ * not used beyond 64 rows, where rows shared through LDS cost less).  us per launch, q|k|v / output / gate|up /
+ * down: 10.0 / 7.7 / 22.2 / 11.9 at 6 rows, 14.5 / 10.4 / 29.6 / 16.5 at 37, 15.5 / 11.5 / 34.1 / 18.8 at 64;
+ * vt_gemm_wide_kernel takes 21.7 / 16.8 / 62.1 / 27.9 at 37.
+ */
+#define GR_TN 64
+
+struct gr_part {
+    float *C;                             /* `splits` planes of [M, ldc], plane_stride floats apart */
+    const uint16_t *Wf;                   /* fragment-order weights of the part's first column */
+    size_t plane_stride;
+    int ldc, n_tiles, splits;
+    uint16_t *h_hi, *h_lo;                /* gate|up (paired column order): planes of SiLU(gate) * up instead of C */
+    int ldh;
+    const float *row_scale, *col_scale;   /* T::SCALED: factors of the rows and of the part's columns */
+};
+struct gr_plan { gr_part part[2]; int n_parts; };
+
+/* non-temporal: with this few rows the weights are read once */
+__device__ __forceinline__ u32x4 gr_ld_nt(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
+    return __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 2);
+}
+
+/* One workgroup's piece of a product: a 64-column tile over one K cut */
+struct gr_item {
+    const unsigned char *w;               /* weights of the tile */
+    int part, nt, sp, s0, n;              /* n: this wave's K steps s0 + wave + 8 i */
+};
+
+template <int NW, int WP>
+__device__ __forceinline__ gr_item gr_item_at(const gr_plan &plan, int part, int id, int K, int wave) {
+    const gr_part &P = plan.part[part];
+    /* slot id lands on XCD id % 8: an XCD takes a run of items, N tile fastest, i.e. few K cuts: the slice of
+     * the planes that its L2 has to fetch is that of its cuts */
+    const int items = P.n_tiles * P.splits;
+    const int li = (items & 7) == 0 ? (id & 7) * (items >> 3) + (id >> 3) : id;
+    gr_item it;
+    it.part = part;
+    it.nt = li % P.n_tiles;
+    it.sp = li / P.n_tiles;
+    const int steps = K / 64, q = steps / P.splits, rem = steps % P.splits;
+    const int ns = q + (it.sp < rem ? 1 : 0);
+    it.s0 = it.sp * q + min(it.sp, rem);
+    it.n = ns > wave ? (ns - wave + NW - 1) / NW : 0;
+    it.w = (const unsigned char *)(P.Wf + (size_t)it.nt * GR_TN * K * WP);
+    return it;
+}
+
+/* NP passes of 8 rows: M <= 8 NP; NW waves */
+template <class T, int NP, int NW>
+__global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW / 4, NW / 4)))
+vt_gemm_rows_kernel(gr_plan plan, const uint16_t *Ahi, const uint16_t *Alo, int M, int K) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+    constexpr int WP = T::WP;
+    constexpr int MB = (NP + 3) / 4;                                         /* blocks of 32 rows */
+    constexpr int PLANE = 32 * MB * GM_STAGE_ROW;
+    const int lane = (int)threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int blk_bytes = 64 * K * WP;                                       /* 32 columns x K x 2 bytes x planes */
+    const int a_bytes = M * K * 2;
+    unsigned char *mine = lds + wave * (2 * PLANE);
+    const int lr = lane >> 3, lc = lane & 7;                                 /* staging: row lr + 8 p, 16-byte chunk lc */
+    const int a_voff = (lr * K + lc * 8) * 2, a_pass = 16 * K;               /* byte distance of two passes */
+    const int st_off = lr * GM_STAGE_ROW + lc * 16;
+    const int fa_off = (lane & 31) * GM_STAGE_ROW + (lane >> 5) * 64;
+
+    u32x4 ra_hi[NP], ra_lo[NP];
+    auto fetch_a = [&](const gr_item &it, int i) {
+        const int soff = i < it.n ? (it.s0 + wave + NW * i) * 128 : 0;
+        const __amdgpu_buffer_rsrc_t h = __builtin_amdgcn_make_buffer_rsrc((void *)Ahi, 0, i < it.n ? a_bytes : 0, 0x00020000);
+        const __amdgpu_buffer_rsrc_t l = __builtin_amdgcn_make_buffer_rsrc((void *)Alo, 0, i < it.n ? a_bytes : 0, 0x00020000);
+#pragma unroll
+        for (int p = 0; p < NP; p++) {
+            ra_hi[p] = gm_ldb(h, a_voff + p * a_pass, soff);
+            ra_lo[p] = gm_ldb(l, a_voff + p * a_pass, soff);
+        }
+    };
+    auto fetch_b_slice = [&](const gr_item &it, gm_weights<WP> &r, int i, int j) {
+        const int soff = i < it.n ? (it.s0 + wave + NW * i) * 4096 * WP : 0;
+        const __amdgpu_buffer_rsrc_t w = __builtin_amdgcn_make_buffer_rsrc((void *)it.w, 0, i < it.n ? 2 * blk_bytes : 0, 0x00020000);
+#pragma unroll
+        for (int p = 0; p < WP; p++) {
+            r.v[p][0][j] = gr_ld_nt(w, lane * 16 + 1024 * j, soff + 4096 * p);
+            r.v[p][1][j] = gr_ld_nt(w, lane * 16 + 1024 * j, soff + 4096 * p + (i < it.n ? blk_bytes : 0));
+        }
+    };
+    auto store_a = [&]() {
+#pragma unroll
+        for (int p = 0; p < NP; p++) {
+            *reinterpret_cast<u32x4 *>(mine + st_off + 8 * p * GM_STAGE_ROW) = ra_hi[p];
+            *reinterpret_cast<u32x4 *>(mine + PLANE + st_off + 8 * p * GM_STAGE_ROW) = ra_lo[p];
+        }
+    };
+    typedef gm_frags<MB> frags;
+    auto read_frags = [&](frags &f, int ks) {
+#pragma unroll
+        for (int a = 0; a < MB; a++) {
+            f.hi[a] = *reinterpret_cast<const u32x4 *>(mine + fa_off + 32 * a * GM_STAGE_ROW + 16 * ks);
+            f.lo[a] = *reinterpret_cast<const u32x4 *>(mine + PLANE + fa_off + 32 * a * GM_STAGE_ROW + 16 * ks);
+        }
+    };
+    f32x16 acc[MB][2];
+    auto mma = [&](const frags &f, const gm_weights<WP> &w, int ks) { gm_multiply<T, MB>(acc, f, w, ks); };
+    gm_weights<WP> b0, b1;
+    frags f0, f1;
+    /* the first requests of an item: the rows of step 0, the weights of steps 0 and 1 */
+    auto begin = [&](const gr_item &it) {
+        fetch_a(it, 0);
+#pragma unroll
+        for (int j = 0; j < 4; j++) fetch_b_slice(it, b0, 0, j);
+#pragma unroll
+        for (int j = 0; j < 4; j++) fetch_b_slice(it, b1, 1, j);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    /* step i: the stage holds its rows, f0 their slice 0; ra holds the rows of step i + 1.  A slice's weight
+     * registers are requested again (step i + 2) as soon as the slice has been multiplied. */
+    auto step = [&](const gr_item &it, int i, gm_weights<WP> &cur) {
+        read_frags(f1, 1);
+        mma(f0, cur, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        fetch_b_slice(it, cur, i + 2, 0);
+        read_frags(f0, 2);
+        mma(f1, cur, 1);
+        __builtin_amdgcn_sched_barrier(0);
+        fetch_b_slice(it, cur, i + 2, 1);
+        read_frags(f1, 3);
+        mma(f0, cur, 2);
+        __builtin_amdgcn_sched_barrier(0);
+        fetch_b_slice(it, cur, i + 2, 2);
+        store_a();
+        fetch_a(it, i + 2);
+        read_frags(f0, 0);
+        mma(f1, cur, 3);
+        __builtin_amdgcn_sched_barrier(0);
+        fetch_b_slice(it, cur, i + 2, 3);
+    };
+    auto multiply = [&](const gr_item &it) {
+#pragma unroll
+        for (int a = 0; a < MB; a++)
+#pragma unroll
+            for (int b = 0; b < 2; b++)
+#pragma unroll
+                for (int v = 0; v < 16; v++) acc[a][b][v] = 0.f;
+        store_a();
+        fetch_a(it, 1);
+        __builtin_amdgcn_sched_barrier(0);
+        read_frags(f0, 0);
+        for (int i = 0; i < it.n; i += 2) {
+            step(it, i, b0);
+            step(it, i + 1, b1);          /* past the last one: zeros times zeros */
+        }
+    };
+    /* the waves' sums: parked as quads of accumulator elements over each wave's own stage, added in wave order */
+    auto finish = [&](const gr_item &it) {
+        const gr_part &P = plan.part[it.part];
+        float *park = reinterpret_cast<float *>(mine);
+#pragma unroll
+        for (int a = 0; a < MB; a++)
+#pragma unroll
+            for (int b = 0; b < 2; b++)
+#pragma unroll
+                for (int vq = 0; vq < 4; vq++)
+                    *reinterpret_cast<f32x4 *>(park + (((a * 4 + vq) * 2 + b) * 64 + lane) * 4) =
+                        f32x4{acc[a][b][4 * vq], acc[a][b][4 * vq + 1], acc[a][b][4 * vq + 2], acc[a][b][4 * vq + 3]};
+        __syncthreads();
+        /* wave w finishes the quads w, w + NW, ...: rows 8 q + 4 (lane / 32) + 0..3, column lane % 32 of both blocks */
+#pragma unroll
+        for (int qd = wave; qd < NP; qd += NW) {
+            f32x4 s[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+            for (int w = 0; w < NW; w++)
+#pragma unroll
+                for (int b = 0; b < 2; b++) {
+                    const f32x4 v = *reinterpret_cast<const f32x4 *>(lds + w * (2 * PLANE) + ((qd * 2 + b) * 64 + lane) * 16);
+                    s[b].x = __fadd_rn(s[b].x, v.x); s[b].y = __fadd_rn(s[b].y, v.y);
+                    s[b].z = __fadd_rn(s[b].z, v.z); s[b].w = __fadd_rn(s[b].w, v.w);
+                }
+            const int row0 = 8 * qd + 4 * (lane >> 5), c = lane & 31;
+            if (!T::SCALED && P.h_hi) {
+                const vt_h_quad h = vt_silu_mul_quad(s[0], s[1]);                /* voxtral_tts_llm.c:346-350 */
+                const size_t at = (size_t)(row0 + h.row) * P.ldh + it.nt * (GR_TN / 2) + (c & ~1);
+#pragma unroll
+                for (int r = 0; r < 2; r++)
+                    if (row0 + h.row + r < M) {
+                        *reinterpret_cast<unsigned *>(P.h_hi + at + (size_t)r * P.ldh) = h.hi[r];
+                        *reinterpret_cast<unsigned *>(P.h_lo + at + (size_t)r * P.ldh) = h.lo[r];
+                    }
+            } else {
+                const int col = it.nt * GR_TN + c;
+                gm_store_quad<T>(P.C + (size_t)it.sp * P.plane_stride + col, P.ldc, row0, M, s[0], s[1], P.row_scale, P.col_scale + col);
+            }
+        }
+    };
+
+    /* items blockIdx.x, + gridDim.x, ... of each part in turn; the first requests of the next item go out in
+     * front of the sums of this one */
+    int part = 0, id = (int)blockIdx.x;
+    gr_item it = gr_item_at<NW, WP>(plan, 0, id, K, wave);
+    begin(it);
+    for (;;) {
+        multiply(it);
+        id += (int)gridDim.x;
+        while (part < plan.n_parts && id >= plan.part[part].n_tiles * plan.part[part].splits) {
+            part++;
+            id = (int)blockIdx.x;
+        }
+        if (part >= plan.n_parts) break;
+        const gr_item nx = gr_item_at<NW, WP>(plan, part, id, K, wave);
+        begin(nx);
+        finish(it);
+        __syncthreads();                  /* the next item stages over the parked sums */
+        it = nx;
+    }
+    finish(it);
+}
+
+
+#endif /* VT_GEMM_TILES_H */

@@ -113,7 +113,8 @@ void vt_launch_prefill_attention(float *d_out, uint16_t *d_hi, uint16_t *d_lo, c
 #define VT_ATT_SCALE (1.0f / sqrtf((float)VT_HEAD_DIM))
 void vt_codec_free(void);
 /* single launches for the library's other translation units and its benchmark companion (vt_bench.hip) */
-int vt_codec_probe_buffers(float **xn, float **att, float **h, int **codes);
+int vt_codec_probe_buffers(float **x, int **codes);
+void vt_codec_probe_fill(const float *x, int k);
 int vt_codec_probe_launch(int which);
 int vt_ac_launch_layer_phase(int layer, int phase);
 float *vt_ac_work_area(size_t *n_floats);
