@@ -12,7 +12,7 @@
  *
  * A layer is four kernels, each a skinny product on the matrix cores
  * (v_mfma_f32_16x16x32_bf16, the 6 activation rows as (hi, lo) bf16 planes in
- * LDS, 12 weight rows at a time streamed straight from HBM into the B operand
+ * LDS, 12 weight rows at a time in fragment order streamed straight from HBM into the B operand
  * by one persistent workgroup per CU, its 8 waves splitting K):
  *   RMSNorm + q|k|v            -> qkv [6, 6144]
  *   attention (3x3 per head and branch) + output projection + residual
@@ -29,13 +29,6 @@
 #include <string.h>
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef __attribute__((address_space(1))) const u32x4 ac_gptr_u32x4;
-
-/* Two consecutive 16-byte loads of a lane share a 128-byte line (a load instruction
- * covers 16 weight rows x 64 bytes), so these are ordinary cached loads: the second
- * one must find the line the first one brought in. */
-__device__ __forceinline__ u32x4 ac_ldw(const uint16_t *p) { return *(ac_gptr_u32x4 *)p; }
-
 #define AC_ROWS    6
 #define AC_THREADS 512
 #define AC_WAVES   8
@@ -44,7 +37,7 @@ __device__ __forceinline__ u32x4 ac_ldw(const uint16_t *p) { return *(ac_gptr_u3
 enum { AC_QKV = 0, AC_WO = 1, AC_W13 = 2, AC_W2 = 3 };
 
 struct ac_phase_args {
-    const uint16_t *W;            /* [N, K] bf16 */
+    const uint16_t *W;            /* [N, K] bf16 in fragment order (vt_ac_layout_layer) */
     const float *in;              /* QKV/W13: tok [6,3072]; WO: qkv [6,6144]; W2: h [6,9216] */
     const float *gain;            /* RMSNorm gains (QKV, W13) */
     float *out;                   /* QKV: qkv; WO/W2: tok (residual, in place); W13: h */
@@ -238,10 +231,46 @@ __device__ __forceinline__ void ac_attention_to_planes(unsigned char *hi, unsign
  * the planes for each. */
 #define AC_RB 12
 
-template <int PH, int NL>
-__device__ __forceinline__ void ac_issue(u32x4 (&wreg)[NL], const uint16_t *p) {
+/* Weights in fragment order: per unit the 32-wide K slices one after the other, a slice (AC_SLICE bytes) as the 4 k
+ * groups x 12 rows of 16 bytes that lanes 16 kg + col load, so that a load instruction reads 768 consecutive bytes, each
+ * line once.  From the row-major matrix neighbouring lanes ask for different rows: 64 accesses of 16 bytes per
+ * instruction, which the CU's address path serves at about the rate the card's memory delivers, and every line
+ * twice: an acoustic frame took 1303 us from row-major weights and takes 1188 from these, results bit-identical.
+ * The lanes of the four spare columns ask beyond the descriptor's size, i.e. for nothing. */
+#define AC_SLICE (AC_RB * 64)
+
+__global__ void __launch_bounds__(256) vt_ac_weight_layout_kernel(u32x4 *out, const uint16_t *W, size_t n_slots, int K) {
+    const int slices = K / 32;
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n_slots; i += (size_t)gridDim.x * blockDim.x) {
+        const int at = (int)(i % (4 * AC_RB)), kg = at / AC_RB, col = at % AC_RB;
+        const size_t blk = i / (4 * AC_RB), unit = blk / slices;
+        out[i] = *reinterpret_cast<const u32x4 *>(W + (unit * AC_RB + col) * K + 32 * (blk % slices) + 8 * kg);
+    }
+}
+
+/* The matrices of one uploaded acoustic layer from row-major into fragment order */
+int vt_ac_layout_layer(vt_layer_dev *l) {
+    struct { const uint16_t **w; size_t n; int k; } m[4] = {
+        {&l->wqkv, VT_QKV_DIM, VT_DIM}, {&l->wo, VT_DIM, VT_Q_DIM}, {&l->w13, 2 * VT_FFN, VT_DIM}, {&l->w2, VT_DIM, VT_FFN}};
+    if (vt_check(hipStreamSynchronize(NULL), "acoustic weight copy")) return -1;     /* sources may have been device memory */
+    for (int i = 0; i < 4; i++) {
+        u32x4 *f = (u32x4 *)vt_dev_alloc(m[i].n * m[i].k * 2);
+        if (!f) return -1;
+        hipLaunchKernelGGL(vt_ac_weight_layout_kernel, dim3(4096), dim3(256), 0, g_vt.stream, f, *m[i].w, m[i].n * m[i].k / 8, m[i].k);
+        const int bad = vt_check(hipGetLastError(), "acoustic weight layout") || vt_check(hipStreamSynchronize(g_vt.stream), "acoustic weight layout");
+        (void)hipFree((void *)*m[i].w);
+        *m[i].w = (const uint16_t *)f;
+        if (bad) return -1;
+    }
+    return 0;
+}
+
+/* non-temporal: a frame's weights do not fit the L2, the activation rows do */
+template <int NL>
+__device__ __forceinline__ void ac_issue(u32x4 (&wreg)[NL], __amdgpu_buffer_rsrc_t unit, int voff, int soff) {
 #pragma unroll
-    for (int i = 0; i < NL; i++) wreg[i] = ac_ldw(p + 32 * i);
+    for (int i = 0; i < NL; i++)
+        wreg[i] = __builtin_amdgcn_raw_buffer_load_b128(unit, voff + AC_SLICE * (i % 5), soff + AC_SLICE * 5 * (i / 5), 2);
 }
 
 template <int NL>
@@ -331,10 +360,11 @@ vt_ac_phase_kernel(ac_phase_args a, int n_units) {
     const int G = (int)gridDim.x;
     int u = (int)blockIdx.x;
     if (u >= n_units) return;
-    /* this lane's weight row inside unit 0, at this wave's K slice; the four spare columns of
-     * the tile repeat row 0 (same cache lines, results unused) */
-    const uint16_t *wbase = a.W + (size_t)(live ? col : 0) * SH::KTOT + wave * SH::KW + 8 * kg;
-    const size_t unit_stride = (size_t)AC_RB * SH::KTOT;
+    const int w_voff = live ? (kg * AC_RB + col) * 16 : 0x40000000;      /* spare columns: beyond the size */
+    const int w_soff = __builtin_amdgcn_readfirstlane(wave) * SH::NL * AC_SLICE;
+    auto unit_at = [&](int unit) {
+        return __builtin_amdgcn_make_buffer_rsrc((void *)(a.W + (size_t)unit * AC_RB * SH::KTOT), 0, AC_RB * SH::KTOT * 2, 0x00020000);
+    };
     const int arow = col < AC_ROWS ? col : 0;          /* rows 6..15 of the A operand are don't-care */
     const unsigned char *fa = hi + arow * SH::PITCH + 2 * (wave * SH::KW + 8 * kg);
     const unsigned char *fl = lo + arow * SH::PITCH + 2 * (wave * SH::KW + 8 * kg);
@@ -367,12 +397,12 @@ vt_ac_phase_kernel(ac_phase_args a, int n_units) {
             /* every wave for itself: its K slice of the rows, no workgroup barrier before the products */
             ac_slice_regs<SH::KW> sr;
             ac_fetch_slice<SH::KW>(sr, a.in, VT_DIM, a.gain);
-            ac_issue<PH>(w0, wbase + u * unit_stride);
+            ac_issue(w0, unit_at(u), w_voff, w_soff);
             ac_slice_to_planes<true, SH::KW>(hi, lo, SH::PITCH, sr, red_ss);
         } else {
             ac_attn_regs ra;
             ac_fetch_attn(ra, a.in);
-            ac_issue<PH>(w0, wbase + u * unit_stride);
+            ac_issue(w0, unit_at(u), w_voff, w_soff);
             f32x4 *kvl = reinterpret_cast<f32x4 *>(ac_lds + 2 * SH::PLANE + SH::RED_BYTES);
             ac_stage_kv(kvl, ra);
             ac_attention_to_planes(hi, lo, SH::PITCH, ra, kvl);
@@ -395,7 +425,7 @@ vt_ac_phase_kernel(ac_phase_args a, int n_units) {
                 break;
             }
             {
-                ac_issue<PH>(w1, wbase + nx * unit_stride);
+                ac_issue(w1, unit_at(nx), w_voff, w_soff);
                 __builtin_amdgcn_sched_barrier(0);
                 f32x4 ah = zero4, al = zero4;
                 ac_consume(w0, fa, fl, ah, al);
@@ -412,7 +442,7 @@ vt_ac_phase_kernel(ac_phase_args a, int n_units) {
                 break;
             }
             {
-                ac_issue<PH>(w0, wbase + nx * unit_stride);
+                ac_issue(w0, unit_at(nx), w_voff, w_soff);
                 __builtin_amdgcn_sched_barrier(0);
                 f32x4 ah = zero4, al = zero4;
                 ac_consume(w1, fa, fl, ah, al);
@@ -423,18 +453,17 @@ vt_ac_phase_kernel(ac_phase_args a, int n_units) {
         }
     } else {
         for (; u < n_units; u += G) {
-            const uint16_t *wp = wbase + u * unit_stride;
             ac_slice_regs<SH::KW> sr;
             ac_fetch_slice<SH::KW>(sr, a.in, VT_FFN, NULL);
             u32x4 wreg[2][SH::NL];
-            ac_issue<PH>(wreg[0], wp);
+            ac_issue(wreg[0], unit_at(u), w_voff, w_soff);
             f32x4 ah = zero4, al = zero4;
 #pragma unroll
             for (int pass = 0; pass < SH::NPASS; pass++) {
                 ac_slice_to_planes<false, SH::KW>(hi, lo, SH::PITCH, sr, red_ss);
                 if (pass + 1 < SH::NPASS) {
                     ac_fetch_slice<SH::KW>(sr, a.in + (pass + 1) * SH::KP, VT_FFN, NULL);
-                    ac_issue<PH>(wreg[(pass + 1) & 1], wp + (pass + 1) * SH::KP);
+                    ac_issue(wreg[(pass + 1) & 1], unit_at(u), w_voff, w_soff + (pass + 1) * (SH::KP / 32) * AC_SLICE);
                 }
                 ac_consume(wreg[pass & 1], fa, fl, ah, al);
             }

@@ -372,7 +372,7 @@ extern "C" int tts_hip_upload_acoustic_weights(void *acoustic_ptr) {
     if (!(d->time_inv_freq = (float *)upload(ac->time_inv_freq, sizeof(float) * VT_DIM / 2))) return -1;
     VT_TRY(hipMemcpy(d->h_time_inv_freq, ac->time_inv_freq, sizeof d->h_time_inv_freq, hipMemcpyDefault));
     for (int i = 0; i < TTS_HIP_AC_LAYERS; i++)
-        if (upload_layer(&d->layers[i], &ac->layers[i])) return -1;
+        if (upload_layer(&d->layers[i], &ac->layers[i]) || vt_ac_layout_layer(&d->layers[i])) return -1;
     g_vt.ac_uploaded = 1;
     g_hip.ac_layers_uploaded = TTS_HIP_AC_LAYERS;
     return 0;

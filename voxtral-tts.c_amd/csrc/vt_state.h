@@ -26,7 +26,7 @@
 struct vt_layer_frag { uint16_t *wqkv, *wo, *w13, *w2; };
 
 struct vt_acoustic_dev {
-    vt_layer_dev layers[TTS_HIP_AC_LAYERS];
+    vt_layer_dev layers[TTS_HIP_AC_LAYERS];      /* matrices in the fragment order of the phase kernels */
     uint16_t *input_proj, *time_proj, *llm_proj, *semantic_out, *acoustic_out;
     float *semantic_bias;         /* NULL when the checkpoint has none */
     float *norm;
@@ -116,6 +116,7 @@ void vt_codec_free(void);
 int vt_codec_probe_buffers(float **x, int **codes);
 void vt_codec_probe_fill(const float *x, int k);
 int vt_codec_probe_launch(int which);
+int vt_ac_layout_layer(vt_layer_dev *l);
 int vt_ac_launch_layer_phase(int layer, int phase);
 float *vt_ac_work_area(size_t *n_floats);
 unsigned char *vt_pa_image(int rows);
