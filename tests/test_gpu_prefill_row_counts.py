@@ -44,3 +44,29 @@ def test_prefill_with_gates_far_from_zero():
                 assert mx < 1e-3 and l2 < 1e-3, (s, r, mx, l2)
     finally:
         hip.close()
+
+
+@pytest.mark.parametrize("chunks", [[1, 8], [37, 64], [65, 97], [226, 41]])
+def test_prefill_for_the_cache_alone(chunks):
+    """Without the rows the last layer is its k|v product only: the cache is the one of the whole prefill, the last
+    layer's up to the order of sums (K cuts of a 2048-column product; fp32 sums of 3072 products differ by ~3e-7)."""
+    import numpy as np
+    import hipsupport as H
+    import vtsupport as S
+    layers, got = [S.Layer(21), S.Layer(22)], []
+    hip = H.Hip(kv_max=sum(chunks) + 1)
+    try:
+        hip.upload_decoder(layers, S.norm_weight(S.DIM, 97), 2)
+        for want_x in (True, False):
+            hip.pos = 0
+            for i, n in enumerate(chunks):
+                hip.llm_prefill(S.f32_normal((n, S.DIM), 300 + i), want_x=want_x)
+            got.append([c[:2, :sum(chunks)].copy() for c in hip.kv(2)])
+            if want_x:
+                hip.set_kv(np.zeros((26, hip.kv_max, S.KV_DIM)), np.zeros((26, hip.kv_max, S.KV_DIM)))
+    finally:
+        hip.close()
+    for a, b in zip(*got):
+        assert np.array_equal(a[0], b[0])
+        mx, l2 = S.rel_errors(a[1].ravel(), b[1].ravel())
+        assert mx < 1e-5 and l2 < 3e-6, (mx, l2)
