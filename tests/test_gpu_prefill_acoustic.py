@@ -105,6 +105,19 @@ def test_velocity_memo_follows_the_reference_call_pattern(ac_session):
         assert not np.array_equal(vu2, vu)
 
 
+@pytest.mark.parametrize("scale", [0.0, 1e-4, 0.3, 1.0, 8.0])
+@pytest.mark.parametrize("t", [0.0, 6.0 / 7.0, 0.77])
+def test_velocity_over_latent_sizes(ac_session, scale, t):
+    """The first layer's q|k|v of the noise token comes from the latent directly (folded weights, the sum of squares
+    as a quadratic form): latents from none to large, times on the grid (projected ahead) and off it."""
+    hip, orc, ac = ac_session
+    x, h = S.f32_normal(S.ACOUSTIC_DIM, 81) * np.float32(scale), S.f32_normal(S.DIM, 82)
+    t = np.float32(t) if t == 0.77 else np.float32(round(t * 7)) / np.float32(7)
+    vc, vu = hip.predict_velocity_cfg(x, h, t)
+    assert_close(orc.predict_velocity(x, h, t), vc, "cond")
+    assert_close(orc.predict_velocity(x, np.zeros(S.DIM, np.float32), t), vu, "uncond")
+
+
 def test_acoustic_frames_codes_bit_exact(ac_session):
     """Sampled codes at a fixed seed: noise comes from the host RNG restated by
     the oracle (the reference draws it on the host too), the frame runs on the

@@ -8,7 +8,7 @@
  * run as one batch of 6 rows (2 branches x 3 tokens), so every weight is
  * streamed once per Euler step instead of twice.  Work that does not depend
  * on the step is hoisted: the projected LLM token is computed once per frame
- * and the 7 projected time tokens once per weight upload.
+ * and the 7 projected time tokens once per weight upload; both with their q|k|v of the first layer.
  *
  * A layer is four kernels, each a skinny product on the matrix cores
  * (v_mfma_f32_16x16x32_bf16, the 6 activation rows as (hi, lo) bf16 planes in
@@ -21,7 +21,7 @@
  * Two small kernels stand between the steps: one closes a step (final norm,
  * 36-wide output projection of both branches), the other applies the guided
  * Euler update and opens the next step (input projection of the new latent,
- * token assembly).
+ * token assembly, the first layer's q|k|v).
  */
 #include "vt_state.h"
 
@@ -481,11 +481,20 @@ vt_ac_phase_kernel(ac_phase_args a, int n_units) {
  * Two small launches: `back` closes a step (final norm of token 0 of both branches, the 72
  * dot products of the 36-wide output projection), `front` applies the guided Euler update,
  * quantises at the end of the frame, and opens the next step (36-term input projection of the
- * new latent, token assembly).  Both used to be one workgroup, which then pulled the two
- * 221 KB matrices through a single CU (18 us per step); spread over 5 and 3 workgroups the
+ * new latent, token assembly, q|k|v of the first layer).  Both used to be one workgroup, which then pulled the two
+ * 221 KB matrices through a single CU (18 us per step); spread over 5 and 36 workgroups the
  * same arithmetic, element for element, takes a few microseconds per launch.  The latent is
  * read from x_in and written to x_out by workgroup 0 only (every workgroup of `front` applies
- * the update for itself; in place, a late workgroup would apply it twice). */
+ * the update for itself; in place, a late workgroup would apply it twice).
+ *
+ * The first layer's q|k|v is not a pass over its 37.7 MB of weights per step: of the three tokens of a branch the
+ * time token depends on the weights only (its q|k|v is projected with it, once per upload), the LLM token on the
+ * frame only (once per frame), the zero token of the second branch has zeros, and the noise token is a linear
+ * function of the latent's 36 values: W diag(gain) W_in, summed in 64 bits at upload and kept in fp32 (0.9 MB),
+ * times x, times 1/rms of the noise token, whose sum of squares is x' (W_in' W_in) x, kept and done in 64 bits.
+ * Error of the noise token's q|k|v against 64 bits, over its l2 norm: 1.2e-7 (through the phase kernel's planes
+ * 2.4e-6).  us per frame 1188 -> 1141: seven launches of 9.5 us fewer, one more for the LLM token's q|k|v, `front`
+ * 3.8 -> 4.2. */
 
 struct ac_edge_args {
     const float *tok_in;          /* [6,3072] after the last layer (back) */
@@ -493,8 +502,12 @@ struct ac_edge_args {
     const float *norm;            /* final norm gains */
     const uint16_t *acoustic_out; /* [36,3072] */
     const uint16_t *input_proj;   /* [3072,36] */
+    const f32x4 *noise_qkv;       /* [9][6144] quads over the 36 latent values: W_qkv diag(gain) W_in of the first layer */
+    const double *noise_gram;     /* [36][36] W_in' W_in */
     const float *time_tok;        /* [3072] projected time token of the next step */
     const float *llm_tok;         /* [3072] projected LLM token */
+    const float *time_qkv, *llm_qkv;   /* [6144] the first layer's q|k|v of the two */
+    float *qkv_out;               /* [6,6144] the first layer's q|k|v of the next step (front, when do_front) */
     const float *x_in;            /* [36] latent */
     float *x_out;                 /* [36] latent after the update (== x_in values without do_euler) */
     float *vel;                   /* [72] cond | uncond velocities (written by back, read by front) */
@@ -504,7 +517,9 @@ struct ac_edge_args {
 };
 
 #define AC_BACK_WGS 5             /* x 16 waves >= 72 dot products */
-#define AC_FRONT_WGS 3            /* x 1024 threads = 3072 token columns */
+#define AC_FRONT_THREADS 256
+#define AC_FRONT_TOK_WGS (VT_DIM / AC_FRONT_THREADS)                 /* these assemble the token columns, the others q|k|v */
+#define AC_FRONT_WGS (AC_FRONT_TOK_WGS + VT_QKV_DIM / AC_FRONT_THREADS)
 
 __global__ void __launch_bounds__(1024)
 vt_ac_edge_back_kernel(ac_edge_args a) {
@@ -560,18 +575,30 @@ vt_ac_edge_back_kernel(ac_edge_args a) {
     if (mine && lane == 0) a.vel[o] = acc;
 }
 
-__global__ void __launch_bounds__(1024)
+__global__ void __launch_bounds__(AC_FRONT_THREADS)
 vt_ac_edge_front_kernel(ac_edge_args a) {
     __shared__ float s_vel[2 * VT_AC_DIM_IN];
     __shared__ float s_x[VT_AC_DIM_IN];
+    __shared__ double s_ss[VT_AC_DIM_IN];
     const int t = (int)threadIdx.x;
-    const int c = t + 1024 * (int)blockIdx.x;            /* this thread's token column */
-    /* the column's row of the input projection does not depend on the latent: requested first */
+    const bool tok = (int)blockIdx.x < AC_FRONT_TOK_WGS;
+    const int c = t + AC_FRONT_THREADS * ((int)blockIdx.x - (tok ? 0 : AC_FRONT_TOK_WGS));  /* this thread's token or q|k|v column */
+    /* what does not depend on the latent is requested first: the column's row of the input projection or of its
+     * product with the first layer's weights, the other tokens' values */
     u32x2 wr[VT_AC_DIM_IN / 4];
+    f32x4 wq[VT_AC_DIM_IN / 4];
+    float tm = 0.f, lt = 0.f;
     if (a.do_front) {
-        const u32x2 *p = reinterpret_cast<const u32x2 *>(a.input_proj + (size_t)c * VT_AC_DIM_IN);
+        if (tok) {
+            const u32x2 *p = reinterpret_cast<const u32x2 *>(a.input_proj + (size_t)c * VT_AC_DIM_IN);
 #pragma unroll
-        for (int k4 = 0; k4 < VT_AC_DIM_IN / 4; k4++) wr[k4] = p[k4];
+            for (int k4 = 0; k4 < VT_AC_DIM_IN / 4; k4++) wr[k4] = p[k4];
+        } else {
+#pragma unroll
+            for (int k4 = 0; k4 < VT_AC_DIM_IN / 4; k4++) wq[k4] = a.noise_qkv[(size_t)k4 * VT_QKV_DIM + c];
+        }
+        tm = tok ? a.time_tok[c] : a.time_qkv[c];
+        lt = tok ? a.llm_tok[c] : a.llm_qkv[c];
     }
     if (t < VT_AC_DIM_IN) s_x[t] = a.x_in[t];
     if (a.do_euler && t < 2 * VT_AC_DIM_IN) s_vel[t] = a.vel[t];
@@ -601,7 +628,7 @@ vt_ac_edge_front_kernel(ac_edge_args a) {
         }
     }
     __syncthreads();
-    if (a.do_front) {
+    if (a.do_front && tok) {
         /* tokens of both branches: [noise, time, llm] and [noise, time, 0]; the noise token is
          * the 36-term input projection in the CPU order (voxtral_tts_kernels.c:152-185) */
         float acc = 0.f;
@@ -613,14 +640,72 @@ vt_ac_edge_front_kernel(ac_edge_args a) {
             acc = __fadd_rn(acc, __fmul_rn(vt_bf16_lo(w.y), s_x[4 * k4 + 2]));
             acc = __fadd_rn(acc, __fmul_rn(vt_bf16_hi(w.y), s_x[4 * k4 + 3]));
         }
-        const float tm = a.time_tok[c];
-        a.tok_out[c] = acc;
-        a.tok_out[VT_DIM + c] = tm;
-        a.tok_out[2 * VT_DIM + c] = a.llm_tok[c];
-        a.tok_out[3 * VT_DIM + c] = acc;
-        a.tok_out[4 * VT_DIM + c] = tm;
-        a.tok_out[5 * VT_DIM + c] = 0.f;
+        const float rows[AC_ROWS] = {acc, tm, lt, acc, tm, 0.f};
+#pragma unroll
+        for (int m = 0; m < AC_ROWS; m++) a.tok_out[m * VT_DIM + c] = rows[m];
+    } else if (a.do_front) {
+        /* the noise token's sum of squares, a row of the quadratic form per thread */
+        if (t < VT_AC_DIM_IN) {
+            double r = 0.0;
+            for (int k = 0; k < VT_AC_DIM_IN; k++) r = fma(a.noise_gram[k * VT_AC_DIM_IN + t], (double)s_x[k], r);
+            s_ss[t] = r * (double)s_x[t];
+        }
+        __syncthreads();
+        double ss = 0.0;
+        for (int k = 0; k < VT_AC_DIM_IN; k++) ss += s_ss[k];
+        const float inv = 1.0f / sqrtf(fmaxf((float)ss, 0.f) / (float)VT_DIM + VT_EPS);
+        float acc = 0.f;
+#pragma unroll
+        for (int k4 = 0; k4 < VT_AC_DIM_IN / 4; k4++) {
+            const f32x4 w = wq[k4];
+            acc = fmaf(w.x, s_x[4 * k4], acc);
+            acc = fmaf(w.y, s_x[4 * k4 + 1], acc);
+            acc = fmaf(w.z, s_x[4 * k4 + 2], acc);
+            acc = fmaf(w.w, s_x[4 * k4 + 3], acc);
+        }
+        acc = __fmul_rn(acc, inv);
+        const float rows[AC_ROWS] = {acc, tm, lt, acc, tm, 0.f};
+#pragma unroll
+        for (int m = 0; m < AC_ROWS; m++) a.qkv_out[m * VT_QKV_DIM + c] = rows[m];
     }
+}
+
+/* At upload, in 64 bits: noise_qkv (a workgroup per row of the row-major W_qkv) and noise_gram (workgroup VT_QKV_DIM) */
+__global__ void __launch_bounds__(256)
+vt_ac_fold_kernel(float *noise_qkv, double *noise_gram, const uint16_t *wqkv, const float *gain, const uint16_t *win) {
+    __shared__ double s_part[7][VT_AC_DIM_IN];
+    const int n = (int)blockIdx.x, t = (int)threadIdx.x, k = t % VT_AC_DIM_IN, part = t / VT_AC_DIM_IN;
+    auto bf = [](uint16_t v) { return (double)__uint_as_float((unsigned)v << 16); };
+    if (n == VT_QKV_DIM) {
+        for (int e = t; e < VT_AC_DIM_IN * VT_AC_DIM_IN; e += 256) {
+            double acc = 0.0;
+            for (int d = 0; d < VT_DIM; d++)
+                acc = fma(bf(win[(size_t)d * VT_AC_DIM_IN + e / VT_AC_DIM_IN]), bf(win[(size_t)d * VT_AC_DIM_IN + e % VT_AC_DIM_IN]), acc);
+            noise_gram[e] = acc;
+        }
+        return;
+    }
+    if (part < 7) {                       /* 7 x 36 of the 256 threads */
+        double acc = 0.0;
+        for (int d = part; d < VT_DIM; d += 7)
+            acc = fma(bf(wqkv[(size_t)n * VT_DIM + d]) * (double)gain[d], bf(win[(size_t)d * VT_AC_DIM_IN + k]), acc);
+        s_part[part][k] = acc;
+    }
+    __syncthreads();
+    if (part == 0) {
+        double acc = 0.0;
+        for (int p = 0; p < 7; p++) acc += s_part[p][k];
+        noise_qkv[((size_t)(k / 4) * VT_QKV_DIM + n) * 4 + k % 4] = (float)acc;
+    }
+}
+
+/* Behind the upload of the acoustic weights, while the first layer's matrices are row-major */
+int vt_ac_fold_noise(void) {
+    vt_acoustic_dev *ac = &g_vt.ac;
+    if (vt_check(hipStreamSynchronize(NULL), "acoustic weight copy")) return -1;     /* sources may have been device memory */
+    hipLaunchKernelGGL(vt_ac_fold_kernel, dim3(VT_QKV_DIM + 1), dim3(256), 0, g_vt.stream, ac->noise_qkv, ac->noise_gram,
+                       ac->layers[0].wqkv, ac->layers[0].attn_norm, ac->input_proj);
+    return vt_check(hipGetLastError(), "acoustic fold") || vt_check(hipStreamSynchronize(g_vt.stream), "acoustic fold") ? -1 : 0;
 }
 
 /* First maximum of the masked semantic logits (voxtral_tts_acoustic.c:291-306):
@@ -656,19 +741,24 @@ __global__ void __launch_bounds__(1024) vt_semantic_argmax_kernel(const float *l
 /* device work area of the acoustic path, in floats */
 struct ac_work {
     float *tok, *qkv, *h, *llm_tok, *hidden, *x, *x2, *vel, *temb, *time_tok1, *logits;
+    float *llm_qkv, *time_qkv1;   /* the first layer's q|k|v of llm_tok and time_tok1 */
     int *codes;
 };
-#define AC_WORK_FLOATS (AC_ROWS * (VT_DIM + VT_QKV_DIM + VT_FFN) + 4 * VT_DIM + 64 + 128 + VT_SEM_PADDED + 64)
+/* llm_tok and time_tok1, llm_qkv and time_qkv1 are rows 0 and 1 of blocks of AC_ROWS rows: the q|k|v phase kernel
+ * projects all rows of a block, the others hold anything and are not read again */
+#define AC_WORK_FLOATS (AC_ROWS * (2 * VT_DIM + 2 * VT_QKV_DIM + VT_FFN) + 2 * VT_DIM + 64 + 128 + VT_SEM_PADDED + 64)
 
 static void carve(ac_work *w, float *base) {
     w->tok = base;
     w->qkv = w->tok + AC_ROWS * VT_DIM;
     w->h = w->qkv + AC_ROWS * VT_QKV_DIM;
     w->llm_tok = w->h + AC_ROWS * VT_FFN;
-    w->hidden = w->llm_tok + VT_DIM;
+    w->time_tok1 = w->llm_tok + VT_DIM;
+    w->llm_qkv = w->llm_tok + AC_ROWS * VT_DIM;
+    w->time_qkv1 = w->llm_qkv + VT_QKV_DIM;
+    w->hidden = w->llm_qkv + AC_ROWS * VT_QKV_DIM;
     w->temb = w->hidden + VT_DIM;
-    w->time_tok1 = w->temb + VT_DIM;
-    w->x = w->time_tok1 + VT_DIM;
+    w->x = w->temb + VT_DIM;
     w->vel = w->x + 64;
     w->x2 = w->vel + 80;                                 /* vel uses 72 of its 128 floats */
     w->logits = w->vel + 128;
@@ -693,12 +783,18 @@ static int launch_phase(const uint16_t *W, const float *in, const float *gain, f
     return 0;
 }
 
-/* the three layers on tok [6,3072] (in place) */
+/* the first layer's q|k|v of six rows */
+static int project_qkv(float *d_qkv, const float *d_tok) {
+    const vt_layer_dev *L = &g_vt.ac.layers[0];
+    return launch_phase<AC_QKV>(L->wqkv, d_tok, L->attn_norm, d_qkv, VT_QKV_DIM);
+}
+
+/* the three layers on tok [6,3072] (in place) and the first one's q|k|v, which `front` has written */
 static int run_layers(const ac_work *w) {
     const vt_acoustic_dev *ac = &g_vt.ac;
     for (int l = 0; l < TTS_HIP_AC_LAYERS; l++) {
         const vt_layer_dev *L = &ac->layers[l];
-        if (launch_phase<AC_QKV>(L->wqkv, w->tok, L->attn_norm, w->qkv, VT_QKV_DIM)) return -1;
+        if (l > 0 && launch_phase<AC_QKV>(L->wqkv, w->tok, L->attn_norm, w->qkv, VT_QKV_DIM)) return -1;
         if (launch_phase<AC_WO>(L->wo, w->qkv, NULL, w->tok, VT_DIM)) return -1;
         if (launch_phase<AC_W13>(L->w13, w->tok, L->ffn_norm, w->h, 2 * VT_FFN)) return -1;
         if (launch_phase<AC_W2>(L->w2, w->h, NULL, w->tok, VT_DIM)) return -1;
@@ -730,18 +826,21 @@ float *vt_ac_work_area(size_t *n_floats) {
 
 /* One step boundary.  The latent ping-pongs between w->x and w->x2: `flip` counts the front
  * launches of the frame so far; the caller keeps it. */
-static void launch_edge(const ac_work *w, const float *time_tok, const float *llm_tok, float dt, int back, int euler,
-                        int front, int fsq, int *flip) {
+struct ac_tokens { const float *time_tok, *time_qkv, *llm_tok, *llm_qkv; };
+
+static void launch_edge(const ac_work *w, const ac_tokens &tk, float dt, int back, int euler, int front, int fsq, int *flip) {
     const vt_acoustic_dev *ac = &g_vt.ac;
     ac_edge_args a;
     a.tok_in = w->tok; a.tok_out = w->tok; a.norm = ac->norm; a.acoustic_out = ac->acoustic_out;
-    a.input_proj = ac->input_proj; a.time_tok = time_tok; a.llm_tok = llm_tok; a.vel = w->vel;
+    a.input_proj = ac->input_proj; a.noise_qkv = reinterpret_cast<const f32x4 *>(ac->noise_qkv);
+    a.noise_gram = ac->noise_gram; a.qkv_out = w->qkv; a.vel = w->vel;
+    a.time_tok = tk.time_tok; a.time_qkv = tk.time_qkv; a.llm_tok = tk.llm_tok; a.llm_qkv = tk.llm_qkv;
     a.codes = w->codes; a.dt = dt; a.do_euler = euler; a.do_front = front; a.do_fsq = fsq;
     a.x_in = (*flip & 1) ? w->x2 : w->x;
     a.x_out = (*flip & 1) ? w->x : w->x2;
     if (back) hipLaunchKernelGGL(vt_ac_edge_back_kernel, dim3(AC_BACK_WGS), dim3(1024), 0, g_vt.stream, a);
     if (euler || front || fsq) {
-        hipLaunchKernelGGL(vt_ac_edge_front_kernel, dim3(front ? AC_FRONT_WGS : 1), dim3(1024), 0, g_vt.stream, a);
+        hipLaunchKernelGGL(vt_ac_edge_front_kernel, dim3(front ? AC_FRONT_WGS : 1), dim3(AC_FRONT_THREADS), 0, g_vt.stream, a);
         *flip += 1;
     }
 }
@@ -796,6 +895,8 @@ static int ensure_time_grid(float *d_temb) {
     float ts[AC_STEPS];
     for (int i = 0; i < AC_STEPS; i++) ts[i] = (float)i / (float)AC_STEPS;
     if (project_times(ac->time_tok, d_temb, ts, AC_STEPS)) return -1;
+    /* rows 0..5, then 2..7 for row 6 (row 7 is the LLM token's: projected whenever that is) */
+    if (project_qkv(ac->time_qkv, ac->time_tok) || project_qkv(ac->time_qkv + 2 * VT_QKV_DIM, ac->time_tok + 2 * VT_DIM)) return -1;
     ac->time_tok_ready = 1;
     s_memo.uncond_valid = s_memo.hidden_valid = 0;
     return 0;
@@ -817,26 +918,33 @@ static void predict(float *out_c, float *out_u, const float *x_t, const float *l
         return;
     }
     /* time token: from the grid when t is a grid point, else projected now */
-    const float *time_tok = w.time_tok1;
+    ac_tokens tk = {w.time_tok1, w.time_qkv1, NULL, NULL};
     int on_grid = 0;
     for (int i = 0; i < AC_STEPS && !on_grid; i++)
-        if (t_val == (float)i / (float)AC_STEPS) { time_tok = ac->time_tok + (size_t)i * VT_DIM; on_grid = 1; }
-    if (!on_grid && project_times(w.time_tok1, w.temb, &t_val, 1)) return;
+        if (t_val == (float)i / (float)AC_STEPS) {
+            tk.time_tok = ac->time_tok + (size_t)i * VT_DIM;
+            tk.time_qkv = ac->time_qkv + (size_t)i * VT_QKV_DIM;
+            on_grid = 1;
+        }
+    if (!on_grid && (project_times(w.time_tok1, w.temb, &t_val, 1) || project_qkv(w.llm_qkv, w.llm_tok))) return;
     /* LLM token: row AC_STEPS of the token cache */
     float *llm_tok = ac->time_tok + (size_t)AC_STEPS * VT_DIM;
+    tk.llm_tok = llm_tok;
+    tk.llm_qkv = ac->time_qkv + (size_t)AC_STEPS * VT_QKV_DIM;
     if (!s_memo.hidden_valid || memcmp(s_memo.hidden, llm_hidden, sizeof s_memo.hidden) != 0) {
         VT_TRYV(hipStreamSynchronize(st));
         memcpy(g_vt.h_pin, llm_hidden, sizeof(float) * VT_DIM);
         VT_TRYV(hipMemcpyAsync(w.hidden, g_vt.h_pin, sizeof(float) * VT_DIM, hipMemcpyHostToDevice, st));
         vt_launch_linear(llm_tok, w.hidden, ac->llm_proj, NULL, 1, VT_DIM, VT_DIM);
+        if (project_qkv(ac->time_qkv + 2 * VT_QKV_DIM, ac->time_tok + 2 * VT_DIM)) return;
         memcpy(s_memo.hidden, llm_hidden, sizeof s_memo.hidden);
         s_memo.hidden_valid = 1;
     }
     VT_TRYV(hipMemcpyAsync(w.x, x_t, sizeof(float) * VT_AC_DIM_IN, hipMemcpyDefault, st));
     int flip = 0;
-    launch_edge(&w, time_tok, llm_tok, 0.f, 0, 0, 1, 0, &flip);
+    launch_edge(&w, tk, 0.f, 0, 0, 1, 0, &flip);
     if (run_layers(&w)) return;
-    launch_edge(&w, time_tok, llm_tok, 0.f, 1, 0, 0, 0, &flip);
+    launch_edge(&w, tk, 0.f, 1, 0, 0, 0, &flip);
     VT_TRYV(hipGetLastError());
     VT_TRYV(hipStreamSynchronize(st));
     float vel[2 * VT_AC_DIM_IN];
@@ -878,14 +986,17 @@ static int enqueue_frame(ac_work *w, const float *d_or_h_hidden, const float *x0
     vt_launch_linear(w->logits, w->hidden, ac->semantic_out, ac->semantic_bias, 1, VT_DIM, VT_SEM_PADDED);
     hipLaunchKernelGGL(vt_semantic_argmax_kernel, dim3(1), dim3(1024), 0, st, w->logits, w->codes);
     vt_launch_linear(w->llm_tok, w->hidden, ac->llm_proj, NULL, 1, VT_DIM, VT_DIM);
+    if (project_qkv(w->llm_qkv, w->llm_tok)) return -1;
     /* the flow runs without waiting for the semantic code; an END_AUDIO frame discards it */
     int flip = 0;                                        /* 1 + AC_STEPS front launches: the latent ends in w->x */
-    launch_edge(w, ac->time_tok, w->llm_tok, 0.f, 0, 0, 1, 0, &flip);
+    ac_tokens tk = {ac->time_tok, ac->time_qkv, w->llm_tok, w->llm_qkv};
+    launch_edge(w, tk, 0.f, 0, 0, 1, 0, &flip);
     for (int s = 0; s < AC_STEPS; s++) {
         volatile float dt = ts[s + 1] - ts[s];
         if (run_layers(w)) return -1;
         const int last = s + 1 == AC_STEPS;
-        launch_edge(w, ac->time_tok + (size_t)(last ? s : s + 1) * VT_DIM, w->llm_tok, (float)dt, 1, 1, !last, last, &flip);
+        if (!last) { tk.time_tok += VT_DIM; tk.time_qkv += VT_QKV_DIM; }
+        launch_edge(w, tk, (float)dt, 1, 1, !last, last, &flip);
     }
     return vt_check(hipGetLastError(), "frame launch");
 }

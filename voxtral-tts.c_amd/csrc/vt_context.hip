@@ -198,7 +198,7 @@ static void teardown(void) {
     void *ptrs[] = {g_vt.d_layers, g_vt.d_dec_norm, g_vt.d_tok_emb, g_vt.ac.input_proj,
                     g_vt.ac.time_proj, g_vt.ac.llm_proj, g_vt.ac.semantic_out,
                     g_vt.ac.acoustic_out, g_vt.ac.semantic_bias, g_vt.ac.norm,
-                    g_vt.ac.time_inv_freq, g_vt.ac.time_tok, g_vt.ac.audio_emb, g_vt.ac.audio_offsets,
+                    g_vt.ac.time_inv_freq, g_vt.ac.time_tok, g_vt.ac.time_qkv, g_vt.ac.noise_qkv, g_vt.ac.noise_gram, g_vt.ac.audio_emb, g_vt.ac.audio_offsets,
                     g_hip.kv_cache_k_gpu, g_hip.kv_cache_v_gpu,
                     g_vt.d_rope, g_vt.d_x, g_vt.d_q, g_vt.d_attn, g_vt.d_h, g_vt.d_att_part,
                     g_vt.d_att_cnt, g_vt.d_embed, g_vt.d_hidden, g_vt.d_bar_flags,
@@ -352,7 +352,8 @@ extern "C" int tts_hip_upload_acoustic_weights(void *acoustic_ptr) {
     (void)hipStreamSynchronize(g_vt.stream);
     void **old[] = {(void **)&d->input_proj, (void **)&d->time_proj, (void **)&d->llm_proj,
                     (void **)&d->semantic_out, (void **)&d->acoustic_out, (void **)&d->semantic_bias,
-                    (void **)&d->norm, (void **)&d->time_inv_freq, (void **)&d->time_tok};
+                    (void **)&d->norm, (void **)&d->time_inv_freq, (void **)&d->time_tok, (void **)&d->time_qkv,
+                    (void **)&d->noise_qkv, (void **)&d->noise_gram};
     for (size_t i = 0; i < sizeof old / sizeof old[0]; i++) {
         if (*old[i]) (void)hipFree(*old[i]);
         *old[i] = NULL;              /* a failure below must not leave a freed pointer for the teardown */
@@ -361,6 +362,9 @@ extern "C" int tts_hip_upload_acoustic_weights(void *acoustic_ptr) {
     g_hip.ac_layers_uploaded = 0;
     d->time_tok_ready = 0;
     if (!(d->time_tok = (float *)vt_dev_alloc(sizeof(float) * 8 * VT_DIM))) return -1;
+    if (!(d->time_qkv = (float *)vt_dev_alloc(sizeof(float) * 8 * VT_QKV_DIM))) return -1;
+    if (!(d->noise_qkv = (float *)vt_dev_alloc(sizeof(float) * VT_AC_DIM_IN * VT_QKV_DIM))) return -1;
+    if (!(d->noise_gram = (double *)vt_dev_alloc(sizeof(double) * VT_AC_DIM_IN * VT_AC_DIM_IN))) return -1;
     if (!(d->input_proj = (uint16_t *)upload(ac->input_proj_bf16, (size_t)VT_DIM * VT_AC_DIM_IN * 2))) return -1;
     if (!(d->time_proj = (uint16_t *)upload(ac->time_proj_bf16, (size_t)VT_DIM * VT_DIM * 2))) return -1;
     if (!(d->llm_proj = (uint16_t *)upload(ac->llm_proj_bf16, (size_t)VT_DIM * VT_DIM * 2))) return -1;
@@ -372,7 +376,7 @@ extern "C" int tts_hip_upload_acoustic_weights(void *acoustic_ptr) {
     if (!(d->time_inv_freq = (float *)upload(ac->time_inv_freq, sizeof(float) * VT_DIM / 2))) return -1;
     VT_TRY(hipMemcpy(d->h_time_inv_freq, ac->time_inv_freq, sizeof d->h_time_inv_freq, hipMemcpyDefault));
     for (int i = 0; i < TTS_HIP_AC_LAYERS; i++)
-        if (upload_layer(&d->layers[i], &ac->layers[i]) || vt_ac_layout_layer(&d->layers[i])) return -1;
+        if (upload_layer(&d->layers[i], &ac->layers[i]) || (i == 0 && vt_ac_fold_noise()) || vt_ac_layout_layer(&d->layers[i])) return -1;
     g_vt.ac_uploaded = 1;
     g_hip.ac_layers_uploaded = TTS_HIP_AC_LAYERS;
     return 0;

@@ -33,6 +33,9 @@ struct vt_acoustic_dev {
     float *time_inv_freq;
     float h_time_inv_freq[VT_DIM / 2];
     float *time_tok;              /* [8, 3072]: projected time tokens of the Euler grid, then the last LLM token */
+    float *time_qkv;              /* [8, 6144]: the first layer's q|k|v of the rows of time_tok */
+    float *noise_qkv;             /* [9][6144][4]: the first layer's q|k|v of the noise token per latent value, before 1/rms */
+    double *noise_gram;           /* [36, 36]: sum of squares of the noise token as a quadratic form of the latent */
     int time_tok_ready;
     uint16_t *audio_emb;          /* [audio_rows, 3072] audio-code embedding table */
     int *audio_offsets;           /* [37] first row of every codebook, then 37 ints of staging for codes */
@@ -117,6 +120,7 @@ int vt_codec_probe_buffers(float **x, int **codes);
 void vt_codec_probe_fill(const float *x, int k);
 int vt_codec_probe_launch(int which);
 int vt_ac_layout_layer(vt_layer_dev *l);
+int vt_ac_fold_noise(void);
 int vt_ac_launch_layer_phase(int layer, int phase);
 float *vt_ac_work_area(size_t *n_floats);
 unsigned char *vt_pa_image(int rows);
