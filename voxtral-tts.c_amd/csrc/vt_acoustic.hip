@@ -43,17 +43,22 @@ struct ac_phase_args {
     float *out;                   /* QKV: qkv; WO/W2: tok (residual, in place); W13: h */
 };
 
-template <int PH> struct ac_shape {
+/* ROWS = 2: of the last layer only token 0 of either branch is read (`back`), so that from its attention on the
+ * phases work on the rows 0 and 3 alone: row m of a phase is row 3 m of its buffers.  us per phase with six rows and
+ * with two: output 9.2 / 7.2 (the attention is done by every workgroup for itself), gate|up 19.9 / 19.1, down
+ * 12.9 / 11.2; an acoustic frame 1141 / 1108. */
+template <int PH, int ROWS> struct ac_shape {
+    static constexpr int RS = ROWS == AC_ROWS ? 1 : 3;                /* buffer rows per row of the phase */
     static constexpr int KP = PH == AC_WO ? VT_Q_DIM : VT_DIM;      /* K per pass */
     static constexpr int NPASS = PH == AC_W2 ? 3 : 1;
     static constexpr int KTOT = KP * NPASS;
     static constexpr int KW = KP / AC_WAVES;                         /* K per wave and pass */
     static constexpr int NL = KW / 32;                               /* 16-byte loads per lane and pass */
     static constexpr int PITCH = KP * 2 + 16;                        /* bytes per plane row */
-    static constexpr int PLANE = AC_ROWS * PITCH;
+    static constexpr int PLANE = ROWS * PITCH;
     /* units a workgroup takes on a 256-workgroup grid (more on a smaller one: then the buffers are reused) */
     static constexpr int UNITS = PH == AC_W13 ? 6 : PH == AC_QKV ? 2 : 1;
-    static constexpr int RED_UNIT = AC_WAVES * AC_ROWS * 16;          /* floats: one unit's partial sums of all waves */
+    static constexpr int RED_UNIT = AC_WAVES * ROWS * 16;          /* floats: one unit's partial sums of all waves */
     static constexpr int RED_BYTES = 4 * (UNITS * RED_UNIT + AC_WAVES * 8);
     /* attention + output projection: the k|v columns of the 6 rows, shared by the 4 heads of a group */
     static constexpr int KV_BYTES = PH == AC_WO ? AC_ROWS * 2 * VT_KV_DIM * 4 : 0;
@@ -63,26 +68,26 @@ template <int PH> struct ac_shape {
 /* Activation rows are fetched into registers BEFORE the weight loads of a pass are
  * issued: a wave's loads return in order, so this way the planes can be built while
  * the weights are still streaming in. */
-struct ac_attn_regs { f32x4 q[3][4]; f32x4 kv[AC_ROWS * 2 * VT_KV_DIM / 4 / AC_THREADS]; };
+template <int NQ> struct ac_attn_regs { f32x4 q[NQ][4]; f32x4 kv[AC_ROWS * 2 * VT_KV_DIM / 4 / AC_THREADS]; };
 
 /* A wave's own K slice of the 6 rows.  The products of a wave read only the plane columns of its K slice
  * (wave w: columns w * KW .. + KW), so a wave that fetches, scales and converts exactly those columns
  * depends on no other wave before its first matrix instruction: no workgroup barrier between the rows'
  * arrival and the products.  Behind an RMSNorm the planes then hold x * gain and the result is multiplied
  * by 1/rms(x) in the epilogue, from the waves' partial sums of squares (red_ss[wave * 8 + m]). */
-template <int KW> struct ac_slice_regs {
+template <int KW, int ROWS> struct ac_slice_regs {
     static constexpr int NJ = (KW / 4 + 63) / 64;       /* 16-byte groups per lane and row */
-    f32x4 v[AC_ROWS][NJ];
+    f32x4 v[ROWS][NJ];
     f32x4 g[NJ];
 };
 
-template <int KW>
-__device__ __forceinline__ void ac_fetch_slice(ac_slice_regs<KW> &r, const float *src, int src_stride, const float *gain) {
-    constexpr int NJ = ac_slice_regs<KW>::NJ, G4 = KW / 4;
+template <int KW, int ROWS>
+__device__ __forceinline__ void ac_fetch_slice(ac_slice_regs<KW, ROWS> &r, const float *src, int src_stride, const float *gain) {
+    constexpr int NJ = ac_slice_regs<KW, ROWS>::NJ, G4 = KW / 4;
     const int lane = vt_lane(), c0 = vt_wave() * KW;
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f}, one = {1.f, 1.f, 1.f, 1.f};
 #pragma unroll
-    for (int m = 0; m < AC_ROWS; m++) {
+    for (int m = 0; m < ROWS; m++) {
         const f32x4 *row = reinterpret_cast<const f32x4 *>(src + (size_t)m * src_stride + c0);
 #pragma unroll
         for (int j = 0; j < NJ; j++) r.v[m][j] = (64 * (j + 1) <= G4 || lane + 64 * j < G4) ? row[lane + 64 * j] : zero;
@@ -96,14 +101,14 @@ __device__ __forceinline__ void ac_fetch_slice(ac_slice_regs<KW> &r, const float
     }
 }
 
-template <bool NORM, int KW>
+template <bool NORM, int KW, int ROWS>
 __device__ __forceinline__ void ac_slice_to_planes(unsigned char *hi, unsigned char *lo, int pitch,
-                                                   const ac_slice_regs<KW> &r, float *red_ss) {
-    constexpr int NJ = ac_slice_regs<KW>::NJ, G4 = KW / 4;
+                                                   const ac_slice_regs<KW, ROWS> &r, float *red_ss) {
+    constexpr int NJ = ac_slice_regs<KW, ROWS>::NJ, G4 = KW / 4;
     const int lane = vt_lane(), c0 = vt_wave() * KW;
     if (NORM) {
 #pragma unroll
-        for (int m = 0; m < AC_ROWS; m++) {
+        for (int m = 0; m < ROWS; m++) {
             float ss = 0.f;
 #pragma unroll
             for (int j = 0; j < NJ; j++) {
@@ -120,7 +125,7 @@ __device__ __forceinline__ void ac_slice_to_planes(unsigned char *hi, unsigned c
             const int c = c0 + 4 * (lane + 64 * j);
             const f32x4 g = r.g[j];
 #pragma unroll
-            for (int m = 0; m < AC_ROWS; m++) {
+            for (int m = 0; m < ROWS; m++) {
                 f32x4 v = r.v[m][j];
                 if (NORM) { v.x = __fmul_rn(v.x, g.x); v.y = __fmul_rn(v.y, g.y); v.z = __fmul_rn(v.z, g.z); v.w = __fmul_rn(v.w, g.w); }
                 u32x2 sph, spl;
@@ -143,7 +148,8 @@ __device__ __forceinline__ void ac_slice_to_planes(unsigned char *hi, unsigned c
  * kernel pull 295 KB of activations through its CU instead of 147 KB.
  * Wave w serves the query heads 4 w .. 4 w + 3 of both branches, i.e. kv head w: their outputs are exactly
  * the plane columns 512 w .. of the wave's own K slice, and the k|v rows they share are the wave's alone. */
-__device__ __forceinline__ void ac_fetch_attn(ac_attn_regs &r, const float *qkv) {
+template <int NQ>
+__device__ __forceinline__ void ac_fetch_attn(ac_attn_regs<NQ> &r, const float *qkv) {
     const int lane = vt_lane(), wave = vt_wave(), p = lane >> 3, sub = lane & 7;
     const int br = p >> 2, h = 4 * wave + (p & 3), d0 = sub * 16;
 #pragma unroll
@@ -153,7 +159,7 @@ __device__ __forceinline__ void ac_fetch_attn(ac_attn_regs &r, const float *qkv)
                                                    wave * VT_HEAD_DIM + 4 * g4);
     }
 #pragma unroll
-    for (int i = 0; i < 3; i++) {
+    for (int i = 0; i < NQ; i++) {
         const float *row = qkv + (size_t)(br * 3 + i) * VT_QKV_DIM;
 #pragma unroll
         for (int e = 0; e < 4; e++) r.q[i][e] = *reinterpret_cast<const f32x4 *>(row + h * VT_HEAD_DIM + d0 + 4 * e);
@@ -161,7 +167,8 @@ __device__ __forceinline__ void ac_fetch_attn(ac_attn_regs &r, const float *qkv)
 }
 
 /* the wave's k|v into its part of LDS as [row][k 32 | v 32] groups of 4 */
-__device__ __forceinline__ void ac_stage_kv(f32x4 *kvl, const ac_attn_regs &r) {
+template <int NQ>
+__device__ __forceinline__ void ac_stage_kv(f32x4 *kvl, const ac_attn_regs<NQ> &r) {
     f32x4 *mine = kvl + vt_wave() * (AC_ROWS * 64);
 #pragma unroll
     for (int j = 0; j < AC_ROWS; j++) mine[j * 64 + vt_lane()] = r.kv[j];
@@ -169,8 +176,10 @@ __device__ __forceinline__ void ac_stage_kv(f32x4 *kvl, const ac_attn_regs &r) {
     __builtin_amdgcn_wave_barrier();
 }
 
+/* NQ: the first NQ of the three queries of a branch */
+template <int NQ>
 __device__ __forceinline__ void ac_attention_to_planes(unsigned char *hi, unsigned char *lo, int pitch,
-                                                       const ac_attn_regs &r, const f32x4 *kvl) {
+                                                       const ac_attn_regs<NQ> &r, const f32x4 *kvl) {
     const int lane = vt_lane(), wave = vt_wave(), p = lane >> 3, sub = lane & 7;
     const int br = p >> 2, h = 4 * wave + (p & 3), d0 = sub * 16;
     const float scale = 1.0f / sqrtf((float)VT_HEAD_DIM);
@@ -185,7 +194,7 @@ __device__ __forceinline__ void ac_attention_to_planes(unsigned char *hi, unsign
             v[j][e] = mine[at + 32];
         }
 #pragma unroll
-    for (int i = 0; i < 3; i++) {
+    for (int i = 0; i < NQ; i++) {
         float s[3];
 #pragma unroll
         for (int j = 0; j < 3; j++) {
@@ -205,8 +214,8 @@ __device__ __forceinline__ void ac_attention_to_planes(unsigned char *hi, unsign
         const float mx = fmaxf(s[0], fmaxf(s[1], s[2]));
         const float p0 = expf(s[0] - mx), p1 = expf(s[1] - mx), p2 = expf(s[2] - mx);
         const float inv = __fdiv_rn(1.0f, (p0 + p1) + p2);
-        unsigned char *ph = hi + (br * 3 + i) * pitch + 2 * (h * VT_HEAD_DIM + d0);
-        unsigned char *pl = lo + (br * 3 + i) * pitch + 2 * (h * VT_HEAD_DIM + d0);
+        unsigned char *ph = hi + (br * NQ + i) * pitch + 2 * (h * VT_HEAD_DIM + d0);
+        unsigned char *pl = lo + (br * NQ + i) * pitch + 2 * (h * VT_HEAD_DIM + d0);
 #pragma unroll
         for (int e = 0; e < 4; e++) {
             const float o0 = __fmul_rn(fmaf(p2, v[2][e].x, fmaf(p1, v[1][e].x, p0 * v[0][e].x)), inv);
@@ -296,23 +305,24 @@ __device__ __forceinline__ float ac_inv_rms_of(const float *red_ss, int m) {
 }
 
 /* A wave leaves its partial sums of one unit in that unit's buffer; nobody waits. */
+template <int ROWS>
 __device__ __forceinline__ void ac_park_unit(float *red, f32x4 acc_hi, f32x4 acc_lo) {
     const int lane = vt_lane(), wave = vt_wave(), col = lane & 15, kg = lane >> 4;
     /* accumulator element v of lane l: activation row 4*(l/16) + v, weight row l%16 */
 #pragma unroll
     for (int v = 0; v < 4; v++) {
         const int m = 4 * kg + v;
-        if (m < AC_ROWS) red[(wave * AC_ROWS + m) * 16 + col] = acc_hi[v] + acc_lo[v];
+        if (m < ROWS) red[(wave * ROWS + m) * 16 + col] = acc_hi[v] + acc_lo[v];
     }
 }
 
 /* Behind the workgroup's barrier: cross-wave sums and epilogues of the `n` units parked in red (unit j of
  * them is weight rows (u0 + j * G) * 12 ..).  Thread t takes output element t % E of unit t / E. */
-template <int PH>
+template <int PH, int ROWS>
 __device__ __forceinline__ void ac_finish_units(const ac_phase_args &a, const float *red, int n, int u0, int G,
                                                 bool have_prev, float prev, const float *red_ss) {
-    typedef ac_shape<PH> SH;
-    constexpr int E = PH == AC_W13 ? AC_ROWS * 8 : AC_ROWS * 16;     /* threads per unit */
+    typedef ac_shape<PH, ROWS> SH;
+    constexpr int E = PH == AC_W13 ? ROWS * 8 : ROWS * 16;     /* threads per unit */
     for (int t = (int)threadIdx.x; t < n * E; t += AC_THREADS) {
         const int j = t / E, e = t % E;
         const float *r = red + j * SH::RED_UNIT;
@@ -323,33 +333,33 @@ __device__ __forceinline__ void ac_finish_units(const ac_phase_args &a, const fl
                 float g = 0.f, u = 0.f;
 #pragma unroll
                 for (int w = 0; w < AC_WAVES; w++) {
-                    g += r[(w * AC_ROWS + m) * 16 + 2 * c];
-                    u += r[(w * AC_ROWS + m) * 16 + 2 * c + 1];
+                    g += r[(w * ROWS + m) * 16 + 2 * c];
+                    u += r[(w * ROWS + m) * 16 + 2 * c + 1];
                 }
                 const float inv = ac_inv_rms_of(red_ss, m);
                 g = __fmul_rn(g, inv);
                 u = __fmul_rn(u, inv);
-                a.out[(size_t)m * VT_FFN + (n0 >> 1) + c] = __fmul_rn(__fdiv_rn(g, __fadd_rn(1.0f, expf(-g))), u);
+                a.out[(size_t)(m * SH::RS) * VT_FFN + (n0 >> 1) + c] = __fmul_rn(__fdiv_rn(g, __fadd_rn(1.0f, expf(-g))), u);
             }
         } else if ((e & 15) < AC_RB) {
             const int m = e >> 4, c = e & 15;
             float y = 0.f;
 #pragma unroll
-            for (int w = 0; w < AC_WAVES; w++) y += r[(w * AC_ROWS + m) * 16 + c];
+            for (int w = 0; w < AC_WAVES; w++) y += r[(w * ROWS + m) * 16 + c];
             if (PH == AC_QKV) {
-                a.out[(size_t)m * VT_QKV_DIM + n0 + c] = __fmul_rn(y, ac_inv_rms_of(red_ss, m));
+                a.out[(size_t)(m * SH::RS) * VT_QKV_DIM + n0 + c] = __fmul_rn(y, ac_inv_rms_of(red_ss, m));
             } else {
-                float *p = a.out + (size_t)m * VT_DIM + n0 + c;
+                float *p = a.out + (size_t)(m * SH::RS) * VT_DIM + n0 + c;
                 *p = __fadd_rn(have_prev && j == 0 ? prev : *p, y);
             }
         }
     }
 }
 
-template <int PH>
+template <int PH, int ROWS>
 __global__ void __launch_bounds__(AC_THREADS)
 vt_ac_phase_kernel(ac_phase_args a, int n_units) {
-    typedef ac_shape<PH> SH;
+    typedef ac_shape<PH, ROWS> SH;
     extern __shared__ __attribute__((aligned(16))) unsigned char ac_lds[];
     unsigned char *hi = ac_lds, *lo = ac_lds + SH::PLANE;
     float *red = reinterpret_cast<float *>(ac_lds + 2 * SH::PLANE);          /* UNITS x [8 waves][6][16] */
@@ -365,7 +375,7 @@ vt_ac_phase_kernel(ac_phase_args a, int n_units) {
     auto unit_at = [&](int unit) {
         return __builtin_amdgcn_make_buffer_rsrc((void *)(a.W + (size_t)unit * AC_RB * SH::KTOT), 0, AC_RB * SH::KTOT * 2, 0x00020000);
     };
-    const int arow = col < AC_ROWS ? col : 0;          /* rows 6..15 of the A operand are don't-care */
+    const int arow = col < ROWS ? col : 0;          /* rows 6..15 of the A operand are don't-care */
     const unsigned char *fa = hi + arow * SH::PITCH + 2 * (wave * SH::KW + 8 * kg);
     const unsigned char *fl = lo + arow * SH::PITCH + 2 * (wave * SH::KW + 8 * kg);
     const f32x4 zero4 = {0.f, 0.f, 0.f, 0.f};
@@ -377,8 +387,8 @@ vt_ac_phase_kernel(ac_phase_args a, int n_units) {
     float prev = 0.f;
     if (PH == AC_WO || PH == AC_W2) {
         const int t = (int)threadIdx.x;
-        const bool fin = t < AC_ROWS * 16 && (t & 15) < AC_RB;
-        prev = a.out[(size_t)(fin ? t >> 4 : 0) * VT_DIM + u * AC_RB + (fin ? t & 15 : 0)];
+        const bool fin = t < ROWS * 16 && (t & 15) < AC_RB;
+        prev = a.out[(size_t)((fin ? t >> 4 : 0) * SH::RS) * VT_DIM + u * AC_RB + (fin ? t & 15 : 0)];
     }
 
     /* behind an RMSNorm the planes hold x * gain; the epilogue multiplies by 1/rms(x) */
@@ -387,7 +397,7 @@ vt_ac_phase_kernel(ac_phase_args a, int n_units) {
     int k = 0, u0 = u;                                  /* units parked, and the first of them */
     auto flush = [&] {
         __syncthreads();
-        ac_finish_units<PH>(a, red, k, u0, G, RES && u0 == first_unit, prev, scale_ss);
+        ac_finish_units<PH, ROWS>(a, red, k, u0, G, RES && u0 == first_unit, prev, scale_ss);
         __syncthreads();                                /* the buffers are free again */
         u0 += k * G;
         k = 0;
@@ -395,12 +405,12 @@ vt_ac_phase_kernel(ac_phase_args a, int n_units) {
     if (SH::NPASS == 1) {
         if (PH != AC_WO) {
             /* every wave for itself: its K slice of the rows, no workgroup barrier before the products */
-            ac_slice_regs<SH::KW> sr;
-            ac_fetch_slice<SH::KW>(sr, a.in, VT_DIM, a.gain);
+            ac_slice_regs<SH::KW, ROWS> sr;
+            ac_fetch_slice(sr, a.in, VT_DIM * SH::RS, a.gain);
             ac_issue(w0, unit_at(u), w_voff, w_soff);
-            ac_slice_to_planes<true, SH::KW>(hi, lo, SH::PITCH, sr, red_ss);
+            ac_slice_to_planes<true>(hi, lo, SH::PITCH, sr, red_ss);
         } else {
-            ac_attn_regs ra;
+            ac_attn_regs<ROWS / 2> ra;
             ac_fetch_attn(ra, a.in);
             ac_issue(w0, unit_at(u), w_voff, w_soff);
             f32x4 *kvl = reinterpret_cast<f32x4 *>(ac_lds + 2 * SH::PLANE + SH::RED_BYTES);
@@ -420,7 +430,7 @@ vt_ac_phase_kernel(ac_phase_args a, int n_units) {
             if (nx >= n_units) {
                 f32x4 ah = zero4, al = zero4;
                 ac_consume(w0, fa, fl, ah, al);
-                ac_park_unit(red + k * SH::RED_UNIT, ah, al);
+                ac_park_unit<ROWS>(red + k * SH::RED_UNIT, ah, al);
                 k++;
                 break;
             }
@@ -429,7 +439,7 @@ vt_ac_phase_kernel(ac_phase_args a, int n_units) {
                 __builtin_amdgcn_sched_barrier(0);
                 f32x4 ah = zero4, al = zero4;
                 ac_consume(w0, fa, fl, ah, al);
-                ac_park_unit(red + k * SH::RED_UNIT, ah, al);
+                ac_park_unit<ROWS>(red + k * SH::RED_UNIT, ah, al);
                 if (++k == SH::UNITS) flush();
                 u = nx;
             }
@@ -437,7 +447,7 @@ vt_ac_phase_kernel(ac_phase_args a, int n_units) {
             if (nx >= n_units) {
                 f32x4 ah = zero4, al = zero4;
                 ac_consume(w1, fa, fl, ah, al);
-                ac_park_unit(red + k * SH::RED_UNIT, ah, al);
+                ac_park_unit<ROWS>(red + k * SH::RED_UNIT, ah, al);
                 k++;
                 break;
             }
@@ -446,34 +456,34 @@ vt_ac_phase_kernel(ac_phase_args a, int n_units) {
                 __builtin_amdgcn_sched_barrier(0);
                 f32x4 ah = zero4, al = zero4;
                 ac_consume(w1, fa, fl, ah, al);
-                ac_park_unit(red + k * SH::RED_UNIT, ah, al);
+                ac_park_unit<ROWS>(red + k * SH::RED_UNIT, ah, al);
                 if (++k == SH::UNITS) flush();
                 u = nx;
             }
         }
     } else {
         for (; u < n_units; u += G) {
-            ac_slice_regs<SH::KW> sr;
-            ac_fetch_slice<SH::KW>(sr, a.in, VT_FFN, NULL);
+            ac_slice_regs<SH::KW, ROWS> sr;
+            ac_fetch_slice(sr, a.in, VT_FFN * SH::RS, NULL);
             u32x4 wreg[2][SH::NL];
             ac_issue(wreg[0], unit_at(u), w_voff, w_soff);
             f32x4 ah = zero4, al = zero4;
 #pragma unroll
             for (int pass = 0; pass < SH::NPASS; pass++) {
-                ac_slice_to_planes<false, SH::KW>(hi, lo, SH::PITCH, sr, red_ss);
+                ac_slice_to_planes<false>(hi, lo, SH::PITCH, sr, red_ss);
                 if (pass + 1 < SH::NPASS) {
-                    ac_fetch_slice<SH::KW>(sr, a.in + (pass + 1) * SH::KP, VT_FFN, NULL);
+                    ac_fetch_slice(sr, a.in + (pass + 1) * SH::KP, VT_FFN * SH::RS, NULL);
                     ac_issue(wreg[(pass + 1) & 1], unit_at(u), w_voff, w_soff + (pass + 1) * (SH::KP / 32) * AC_SLICE);
                 }
                 ac_consume(wreg[pass & 1], fa, fl, ah, al);
             }
-            ac_park_unit(red + k * SH::RED_UNIT, ah, al);
+            ac_park_unit<ROWS>(red + k * SH::RED_UNIT, ah, al);
             if (++k == SH::UNITS) flush();
         }
     }
     if (k) {
         __syncthreads();
-        ac_finish_units<PH>(a, red, k, u0, G, RES && u0 == first_unit, prev, scale_ss);
+        ac_finish_units<PH, ROWS>(a, red, k, u0, G, RES && u0 == first_unit, prev, scale_ss);
     }
 }
 
@@ -765,12 +775,12 @@ static void carve(ac_work *w, float *base) {
     w->codes = (int *)(w->logits + VT_SEM_PADDED);
 }
 
-template <int PH>
+template <int PH, int ROWS = AC_ROWS>
 static int launch_phase(const uint16_t *W, const float *in, const float *gain, float *out, int n_rows) {
     static int attr_set = 0;
-    const int lds = ac_shape<PH>::LDS_BYTES;
+    const int lds = ac_shape<PH, ROWS>::LDS_BYTES;
     if (!attr_set) {
-        if (vt_check(hipFuncSetAttribute((const void *)vt_ac_phase_kernel<PH>,
+        if (vt_check(hipFuncSetAttribute((const void *)vt_ac_phase_kernel<PH, ROWS>,
                                          hipFuncAttributeMaxDynamicSharedMemorySize, lds), "acoustic LDS size"))
             return -1;
         attr_set = 1;
@@ -779,7 +789,7 @@ static int launch_phase(const uint16_t *W, const float *in, const float *gain, f
     const int n_units = n_rows / AC_RB;
     const int most = g_vt.ac_grid > 0 && g_vt.ac_grid < g_vt.n_cu ? g_vt.ac_grid : g_vt.n_cu;
     const int grid = n_units < most ? n_units : most;
-    hipLaunchKernelGGL(vt_ac_phase_kernel<PH>, dim3(grid), dim3(AC_THREADS), lds, g_vt.stream, a, n_units);
+    hipLaunchKernelGGL((vt_ac_phase_kernel<PH, ROWS>), dim3(grid), dim3(AC_THREADS), lds, g_vt.stream, a, n_units);
     return 0;
 }
 
@@ -795,6 +805,12 @@ static int run_layers(const ac_work *w) {
     for (int l = 0; l < TTS_HIP_AC_LAYERS; l++) {
         const vt_layer_dev *L = &ac->layers[l];
         if (l > 0 && launch_phase<AC_QKV>(L->wqkv, w->tok, L->attn_norm, w->qkv, VT_QKV_DIM)) return -1;
+        if (l + 1 == TTS_HIP_AC_LAYERS) {
+            if (launch_phase<AC_WO, 2>(L->wo, w->qkv, NULL, w->tok, VT_DIM)) return -1;
+            if (launch_phase<AC_W13, 2>(L->w13, w->tok, L->ffn_norm, w->h, 2 * VT_FFN)) return -1;
+            if (launch_phase<AC_W2, 2>(L->w2, w->h, NULL, w->tok, VT_DIM)) return -1;
+            break;
+        }
         if (launch_phase<AC_WO>(L->wo, w->qkv, NULL, w->tok, VT_DIM)) return -1;
         if (launch_phase<AC_W13>(L->w13, w->tok, L->ffn_norm, w->h, 2 * VT_FFN)) return -1;
         if (launch_phase<AC_W2>(L->w2, w->h, NULL, w->tok, VT_DIM)) return -1;
