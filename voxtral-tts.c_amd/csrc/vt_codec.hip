@@ -161,50 +161,165 @@ vt_codec_swiglu_kernel(cd_planes h, const float *__restrict__ gu, int col0, int 
     if (threadIdx.x == 0) h.inv[row] = 1.0f / s;
 }
 
-/* ALiBi causal sliding-window attention: one workgroup per token, one wave per head, the online softmax over the at
- * most `window` keys in the reference's order (voxtral_tts_kernels.c:527-596); the result as planes. */
+/* ALiBi causal sliding-window attention, the online softmax of a query over the at most `window` keys in ascending
+ * order (voxtral_tts_kernels.c:527-596); the result as planes.  A wave works for one head, eight lanes hold a row's 128
+ * dims (dims 32 e + 4 sub + 0..3 of lane sub), so that a score is 16 products per lane and three lane steps.  With a
+ * wave per (token, head), two dims per lane, it took six shuffles per key and waited for each key's rows in turn. */
+struct cd_head_row { f32x4 v[4]; };
+
+__device__ __forceinline__ cd_head_row cd_load_row(const float *p) {
+    cd_head_row r;
+#pragma unroll
+    for (int e = 0; e < 4; e++) r.v[e] = *(const f32x4 *)(p + 32 * e);
+    return r;
+}
+
+/* q . k over the eight lanes */
+__device__ __forceinline__ float cd_row_dot(const cd_head_row &q, const cd_head_row &k) {
+    float p = 0.f;
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) p = fmaf(q.v[e][i], k.v[e][i], p);
+    p += vt_dpp<0xB1>(p);                         /* lanes ^1 */
+    p += vt_dpp<0x4E>(p);                         /* lanes ^2 */
+    return p + vt_dpp<0x141>(p);                  /* the other quad of the eight */
+}
+
+struct cd_softmax {
+    float mx = -1e30f, se = 0.f;
+    cd_head_row o = {};
+    __device__ __forceinline__ void add(float sc, const cd_head_row &v) {
+        const float d = sc - mx, ex = expf(-fabsf(d)), c = d > 0.f ? ex : 1.0f, w = d > 0.f ? 1.0f : ex;
+        mx = d > 0.f ? sc : mx;
+        se = fmaf(se, c, w);
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) o.v[e][i] = fmaf(v.v[e][i], w, o.v[e][i] * c);
+    }
+};
+
+/* Many tokens: one workgroup for 16 of them, wave h for head h, eight lanes for two neighbouring tokens, which share
+ * all but two of their keys.  The rows of the next key are requested in front of the work on this one; with its
+ * value rows requested late instead (118 registers, two workgroups to a CU) the eight launches of 1003 frames took
+ * 258 us instead of 196: a workgroup's rows in flight are twice the L1 already.  us per launch at 4012 rows, window
+ * 8 / 8024 rows, window 16: 42 / 96 with the kernel below, 20 / 59 with this one. */
+/* Fewer rows than this: the kernel below.  Measured, this kernel / the one below: 848 rows, window 8, 11.3 / 11.3
+ * us; 1003 rows, window 2, 8 / 8.5; 1696 rows, window 16, 17.5 / 23.4; 168 rows, window 16, 16 / 5.5. */
+#define CD_ATT_TOKENS 16
+#define CD_ATT_SPLIT_BELOW 1024
 __global__ void __launch_bounds__(64 * CD_HEADS)
 vt_codec_attention_kernel(cd_planes out, const float *__restrict__ qkv, int T, int window,
                           const float *__restrict__ slopes, float scale) {
-    __shared__ float red[CD_HEADS];
-    const int i = blockIdx.x, h = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    __shared__ float red[CD_HEADS][CD_ATT_TOKENS];
+    const int h = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane >> 3, sub = lane & 7;
+    const int i0 = blockIdx.x * CD_ATT_TOKENS + 2 * g;
+    const bool live[2] = {i0 < T, i0 + 1 < T};
+    const int a = live[0] ? i0 : T - 1, b = a + 1;
     const float slope = slopes[h];
-    const float2 q = *(const float2 *)(qkv + (size_t)i * (3 * CD_DIM) + h * CD_HEAD_DIM + lane * 2);
-    const int j0 = (window > 0 && i - window + 1 > 0) ? i - window + 1 : 0;
-    float mx = -1e30f, se = 0.f;
-    float2 o = make_float2(0.f, 0.f);
-    for (int j = j0; j <= i; j++) {
-        const float *kr = qkv + (size_t)j * (3 * CD_DIM) + CD_DIM + h * CD_HEAD_DIM + lane * 2;
-        const float2 k = *(const float2 *)kr, v = *(const float2 *)(kr + CD_DIM);
-        float sc = q.x * k.x + q.y * k.y;
-        for (int s = 32; s > 0; s >>= 1) sc += __shfl_xor(sc, s);
-        sc = sc * scale + slope * (float)(j - i);
-        if (sc > mx) {
-            const float c = expf(mx - sc);
-            se = se * c + 1.0f;
-            o.x = o.x * c + v.x; o.y = o.y * c + v.y;
-            mx = sc;
-        } else {
-            const float w = expf(sc - mx);
-            se += w;
-            o.x += w * v.x; o.y += w * v.y;
+    const float *base = qkv + h * CD_HEAD_DIM + 4 * sub;
+    auto row = [&](int j, int part) { return cd_load_row(base + (size_t)j * (3 * CD_DIM) + part * CD_DIM); };
+    const cd_head_row qa = row(a, 0), qb = row(live[1] ? b : a, 0);
+    const int ja = (window > 0 && a - window + 1 > 0) ? a - window + 1 : 0, jb = (window > 0 && b - window + 1 > 0) ? b - window + 1 : 0;
+    cd_softmax sa, sb;
+    int j = ja;
+    cd_head_row k = row(j, 1), v = row(j, 2);
+    if (jb > ja) {                                /* the one key that only the first token sees */
+        const int nx = j < a ? j + 1 : live[1] ? b : a;
+        const cd_head_row nk = row(nx, 1), nv = row(nx, 2);
+        sa.add(cd_row_dot(qa, k) * scale + slope * (float)(j - a), v);
+        k = nk; v = nv;
+        j++;
+    }
+    for (; j <= a; j++) {
+        const int nx = j < a ? j + 1 : live[1] ? b : a;
+        const cd_head_row nk = row(nx, 1), nv = row(nx, 2);
+        const float ka = cd_row_dot(qa, k), kb = cd_row_dot(qb, k);
+        sa.add(ka * scale + slope * (float)(j - a), v);
+        sb.add(kb * scale + slope * (float)(j - b), v);
+        k = nk; v = nv;
+    }
+    if (live[1]) sb.add(cd_row_dot(qb, k) * scale, v);      /* the second token's own key */
+    cd_softmax *st[2] = {&sa, &sb};
+#pragma unroll
+    for (int t = 0; t < 2; t++) {
+        const float inv = st[t]->se > 0.f ? 1.0f / st[t]->se : 1.0f;
+        float m = 0.f;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            st[t]->o.v[e] *= inv;
+            m = fmaxf(m, cd_max4(st[t]->o.v[e]));
+        }
+        m = fmaxf(m, vt_dpp<0xB1>(m));
+        m = fmaxf(m, vt_dpp<0x4E>(m));
+        m = fmaxf(m, vt_dpp<0x141>(m));
+        if (sub == 0) red[h][2 * g + t] = m;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < 2; t++) {
+        float m = 0.f;
+#pragma unroll
+        for (int w = 0; w < CD_HEADS; w++) m = fmaxf(m, red[w][2 * g + t]);
+        const float s = vt_f16_scale(m);
+        if (live[t]) {
+#pragma unroll
+            for (int e = 0; e < 4; e++) cd_put4(out, (size_t)(i0 + t) * CD_DIM + h * CD_HEAD_DIM + 32 * e + 4 * sub, st[t]->o.v[e], s);
+            if (h == 0 && sub == 0) out.inv[i0 + t] = 1.0f / s;
         }
     }
+}
+
+/* Few tokens: one workgroup each, wave h for head h; its eight groups of eight lanes take every eighth key, so that
+ * a window of 16 is two keys deep, and merge their sums: each step hands half of what a lane still holds to its
+ * partner and keeps the other half, two dims per lane at the end. */
+__global__ void __launch_bounds__(64 * CD_HEADS)
+vt_codec_attention_split_kernel(cd_planes out, const float *__restrict__ qkv, int T, int window,
+                                const float *__restrict__ slopes, float scale) {
+    __shared__ float red[CD_HEADS];
+    const int i = blockIdx.x, h = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane >> 3, sub = lane & 7;
+    const float slope = slopes[h];
+    const float *base = qkv + h * CD_HEAD_DIM + 4 * sub;
+    const cd_head_row q = cd_load_row(base + (size_t)i * (3 * CD_DIM));
+    const int j0 = (window > 0 && i - window + 1 > 0) ? i - window + 1 : 0;
+    cd_softmax s;
+    for (int j = j0 + g; j <= i; j += 8) {
+        const float *kr = base + (size_t)j * (3 * CD_DIM) + CD_DIM;
+        const cd_head_row k = cd_load_row(kr), v = cd_load_row(kr + CD_DIM);
+        s.add(cd_row_dot(q, k) * scale + slope * (float)(j - i), v);
+    }
+    float mx = s.mx;
+    for (int o = 8; o < 64; o <<= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+    const float f = s.mx == mx ? 1.0f : expf(s.mx - mx);
+    float se = s.se * f;
+    for (int o = 8; o < 64; o <<= 1) se += __shfl_xor(se, o);
+    const bool b3 = lane & 8, b4 = lane & 16, b5 = lane & 32;
+    f32x4 r2[2], r1;
+#pragma unroll
+    for (int e = 0; e < 2; e++) {
+        const f32x4 keep = (b3 ? s.o.v[2 + e] : s.o.v[e]) * f, give = (b3 ? s.o.v[e] : s.o.v[2 + e]) * f;
+#pragma unroll
+        for (int n = 0; n < 4; n++) r2[e][n] = keep[n] + __shfl_xor(give[n], 8);
+    }
+#pragma unroll
+    for (int n = 0; n < 4; n++) r1[n] = (b4 ? r2[1][n] : r2[0][n]) + __shfl_xor(b4 ? r2[0][n] : r2[1][n], 16);
     const float inv = se > 0.f ? 1.0f / se : 1.0f;
-    o.x *= inv; o.y *= inv;
-    float m = fmaxf(fabsf(o.x), fabsf(o.y));
-    for (int s = 32; s > 0; s >>= 1) m = fmaxf(m, __shfl_xor(m, s));
+    const float x = ((b5 ? r1[2] : r1[0]) + __shfl_xor(b5 ? r1[0] : r1[2], 32)) * inv;
+    const float y = ((b5 ? r1[3] : r1[1]) + __shfl_xor(b5 ? r1[1] : r1[3], 32)) * inv;
+    float m = fmaxf(fabsf(x), fabsf(y));
+    for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
     if (lane == 0) red[h] = m;
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < CD_HEADS; k++) m = fmaxf(m, red[k]);
-    const float s = vt_f16_scale(m);
+    const float sc = vt_f16_scale(m);
     unsigned hi, lo;
-    vt_split_f16x2(o.x * s, o.y * s, hi, lo);
-    const size_t at = (size_t)i * CD_DIM + h * CD_HEAD_DIM + lane * 2;
+    vt_split_f16x2(x * sc, y * sc, hi, lo);
+    const size_t at = (size_t)i * CD_DIM + h * CD_HEAD_DIM + 32 * (2 * (int)b3 + (int)b4) + 4 * sub + 2 * (int)b5;
     *(unsigned *)(out.hi + at) = hi;
     *(unsigned *)(out.lo + at) = lo;
-    if (threadIdx.x == 0) out.inv[i] = 1.0f / s;
+    if (threadIdx.x == 0) out.inv[i] = 1.0f / sc;
 }
 
 /* codes [T, 37] -> the three shifted copies of the 292-wide embedding that the input
@@ -574,7 +689,11 @@ static int cd_enqueue(const int *d_codes, int n_frames, float *d_samples) {
                                    (size_t)T * 3 * CD_DIM, l->q_norm, l->k_norm)
         CD_BY_CUTS(pl.cuts, CALL);
 #undef CALL
-        hipLaunchKernelGGL(vt_codec_attention_kernel, dim3(T), dim3(64 * CD_HEADS), 0, g_vt.stream, g_cd.planes, g_cd.qkv, T, l->window, g_cd.slopes, scale);
+        if (T < CD_ATT_SPLIT_BELOW)
+            hipLaunchKernelGGL(vt_codec_attention_split_kernel, dim3(T), dim3(64 * CD_HEADS), 0, g_vt.stream, g_cd.planes, g_cd.qkv, T, l->window, g_cd.slopes, scale);
+        else
+            hipLaunchKernelGGL(vt_codec_attention_kernel, dim3((T + CD_ATT_TOKENS - 1) / CD_ATT_TOKENS), dim3(64 * CD_HEADS), 0, g_vt.stream, g_cd.planes,
+                               g_cd.qkv, T, l->window, g_cd.slopes, scale);
         pl = cd_gemm(T, l->wo);
         cd_row(pl, T, CD_DIM, g_cd.x, NULL, l->attn_scale, l->ffn_norm);
         pl = cd_gemm(T, l->w13);
