@@ -8,12 +8,15 @@
  * product writes the waveform ([T, 240] row-major is the sample order).  Weights are re-laid
  * once at upload:
  *   - q|k|v and gate|up are stacked into one [3072, 1024] and one [8192, 1024] matrix;
- *   - a causal conv1d (stride 1, taps K) becomes a product over the K shifted copies of the
- *     input: W'[oc][k * C_in + ic] = w[oc][ic][k], rows and K padded with zeros;
- *   - the transposed conv (taps 4, stride 2) becomes ONE product that writes both output
- *     phases: out[2j+p][oc] = sum_ic x[j][ic] w[ic][oc][p] + x[j-1][ic] w[ic][oc][p+2], i.e.
- *     W'[p * 1024 + oc][q * 1024 + ic] = w[ic][oc][p + 2q] against rows [x[j] | x[j-1]], and
- *     the [L, 2048] result IS the [2L, 1024] upsampled sequence.
+ *   - the input convolution (taps 3, 292 channels) becomes a product over the shifted copies of
+ *     the embedding: W'[oc][k * 292 + ic] = w[oc][ic][k], K padded with zeros;
+ *   - the others multiply every row with all taps, and the kernel that reads the result adds the
+ *     taps' columns of neighbouring rows.  Transposed (taps 4, stride 2): out[2j+p][oc] =
+ *     sum_ic x[j][ic] w[ic][oc][p] + x[j-1][ic] w[ic][oc][p+2], so W'[q * 2048 + p * 1024 + oc][ic]
+ *     = w[ic][oc][p + 2q].  Output (taps 7): W'[k * 256 + oc][ic] = w[oc][ic][k].  The sums are those
+ *     of a product over shifted copies of the rows, in two and seven pieces, without four launches that
+ *     write the copies (100 us of a 1003-frame decode); us per decode of 21 / 212 / 1003 frames:
+ *     731 / 1595 / 4983 -> 712 / 1558 / 4890.
  * Every product runs on the fp16 matrix cores with both operands as two fp16 planes
  * (vt_codec_gemm.hip); whoever produces a product's input leaves it as planes with one scale
  * per row.  Where a launch would not fill the chip K is cut, and the kernel that reads the
@@ -40,8 +43,9 @@
 #define CD_IN_TAPS 3
 #define CD_OUT_TAPS 7
 #define CD_IN_K 896           /* 3 * 292 = 876 padded to a multiple of 64 */
-#define CD_OUT_K (CD_OUT_TAPS * CD_DIM)
-#define CD_OUT_N 256          /* 240 padded to a multiple of 256 */
+#define CD_OUT_PITCH 256      /* a tap's 240 columns */
+#define CD_OUT_N (CD_OUT_TAPS * CD_OUT_PITCH)
+#define CD_UP_N (4 * CD_DIM)  /* (tap pair q, phase p, channel) */
 
 /* ---- row kernels ------------------------------------------------------------------------- */
 
@@ -86,32 +90,40 @@ __device__ __forceinline__ f32x4 cd_sum(const float *p, int n, size_t stride) {
     return v;
 }
 
-/* One row of 1024: val = the product's result (+ bias) (* scale) (+ residual) -> x_out; with a norm weight also
- * val * rsqrt(mean(val^2) + eps) * norm_w (tts_rms_norm, voxtral_tts_kernels.c:333-349) as planes.  A result row
- * of ldp columns may hold several rows of 1024 (the upsampling product); its columns from col0 on are cut. */
-template <int C>
+/* One row of 1024: val = the product's result (+ bias) (* scale) (+ residual).  With a norm weight val -> x_out and
+ * val * rsqrt(mean(val^2) + eps) * norm_w (tts_rms_norm, voxtral_tts_kernels.c:333-349) as planes; without one the
+ * rows go into a convolution next, val itself as planes.  UP: rows of the upsampling product, row 2 j + p is the sum of
+ * phase p's columns of row j and, for the other tap, of row j - 1.  The columns from col0 on are cut. */
+template <int C, bool UP>
 __global__ void __launch_bounds__(256)
 vt_codec_row_kernel(float *x_out, cd_planes xn, const float *x_in, const float *__restrict__ planes, int col0, int cuts,
-                    size_t plane_stride, int ldp, const float *__restrict__ bias, const float *__restrict__ scale,
+                    size_t plane_stride, const float *__restrict__ bias, const float *__restrict__ scale,
                     const float *__restrict__ norm_w, float eps) {
     __shared__ float red[4];
     const int row = blockIdx.x, c = threadIdx.x * 4;
     const size_t at = (size_t)row * CD_DIM + c;
     f32x4 r = {0.f, 0.f, 0.f, 0.f};
     if (x_in) r = *(const f32x4 *)(x_in + at);
-    f32x4 v = cd_sum<C>(planes + at, (int)(at % ldp) < col0 ? 1 : cuts, plane_stride);
+    f32x4 v;
+    if (UP) {
+        const int j = row >> 1, col = (row & 1) * CD_DIM + c;
+        v = cd_sum<C>(planes + (size_t)j * CD_UP_N + col, col < col0 ? 1 : cuts, plane_stride);
+        if (j > 0) v += cd_sum<C>(planes + (size_t)(j - 1) * CD_UP_N + 2 * CD_DIM + col, 2 * CD_DIM + col < col0 ? 1 : cuts, plane_stride);
+    } else {
+        v = cd_sum<C>(planes + at, c < col0 ? 1 : cuts, plane_stride);
+    }
     if (bias) v += *(const f32x4 *)(bias + c);
     if (scale) v *= *(const f32x4 *)(scale + c);
     v += r;
-    *(f32x4 *)(x_out + at) = v;
     if (norm_w) {
+        *(f32x4 *)(x_out + at) = v;
         const float ss = cd_block_sum(v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w, red);
         const float inv = 1.0f / sqrtf(ss / (float)CD_DIM + eps);
         v = v * inv * *(const f32x4 *)(norm_w + c);
-        const float s = vt_f16_scale(cd_block_max(cd_max4(v), red));
-        cd_put4(xn, at, v, s);
-        if (threadIdx.x == 0) xn.inv[row] = 1.0f / s;
     }
+    const float s = vt_f16_scale(cd_block_max(cd_max4(v), red));
+    cd_put4(xn, at, v, s);
+    if (threadIdx.x == 0) xn.inv[row] = 1.0f / s;
 }
 
 /* q|k|v [T, 3072] summed, with the RMSNorm over the whole 1024-wide q row and k row (tts_qk_norm,
@@ -358,52 +370,23 @@ vt_codec_embed_kernel(cd_planes a, const int *__restrict__ codes, const float *_
     if (threadIdx.x == 0) a.inv[t] = 1.0f / s;
 }
 
-/* x [T, 1024] -> a[t][k * 1024 + c] = x[src(t, k)][c] for the output convolution's causal taps (stride 1, left
- * reflection as above), as planes. */
-__global__ void __launch_bounds__(256)
-vt_codec_taps_kernel(cd_planes a, const float *__restrict__ x, int T) {
-    __shared__ float red[4];
+/* waveform row t: bias + the sum over the output convolution's taps k of tap k's columns of product row src(t, k),
+ * stride 1, left reflection as above */
+template <int C>
+__global__ void __launch_bounds__(64)
+vt_codec_wave_kernel(float *__restrict__ out, const float *__restrict__ planes, int col0, int cuts, size_t plane_stride,
+                     int T, const float *__restrict__ bias) {
     const int t = blockIdx.x, c = threadIdx.x * 4;
-    f32x4 v[CD_OUT_TAPS];
-    float m = 0.f;
+    if (c >= CD_PATCH) return;
+    f32x4 v = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int k = 0; k < CD_OUT_TAPS; k++) {
         int src = t + k - (CD_OUT_TAPS - 1);
         if (src < 0) src = -src;
-        v[k] = f32x4{0.f, 0.f, 0.f, 0.f};
-        if (src < T) v[k] = *(const f32x4 *)(x + (size_t)src * CD_DIM + c);
+        const int col = k * CD_OUT_PITCH + c;
+        const f32x4 p = cd_sum<C>(planes + (size_t)(src < T ? src : 0) * CD_OUT_N + col, col < col0 ? 1 : cuts, plane_stride);
+        if (src < T) v += p;
     }
-#pragma unroll
-    for (int k = 0; k < CD_OUT_TAPS; k++) m = fmaxf(m, cd_max4(v[k]));
-    const float s = vt_f16_scale(cd_block_max(m, red));
-#pragma unroll
-    for (int k = 0; k < CD_OUT_TAPS; k++) cd_put4(a, ((size_t)t * CD_OUT_TAPS + k) * CD_DIM + c, v[k], s);
-    if (threadIdx.x == 0) a.inv[t] = 1.0f / s;
-}
-
-/* x [L, 1024] -> a[j] = [x[j] | x[j-1]] (zero before the start), as planes: the operand of the
- * transposed convolution (voxtral_tts_kernels.c:274-327 with taps 4, stride 2). */
-__global__ void __launch_bounds__(256)
-vt_codec_pair_kernel(cd_planes a, const float *__restrict__ x, int L) {
-    __shared__ float red[4];
-    const int j = blockIdx.x, c = threadIdx.x * 4;
-    const f32x4 v = *(const f32x4 *)(x + (size_t)j * CD_DIM + c);
-    f32x4 p = {0.f, 0.f, 0.f, 0.f};
-    if (j > 0) p = *(const f32x4 *)(x + (size_t)(j - 1) * CD_DIM + c);
-    const float s = vt_f16_scale(cd_block_max(fmaxf(cd_max4(v), cd_max4(p)), red));
-    cd_put4(a, (size_t)j * 2 * CD_DIM + c, v, s);
-    cd_put4(a, (size_t)j * 2 * CD_DIM + CD_DIM + c, p, s);
-    if (threadIdx.x == 0) a.inv[j] = 1.0f / s;
-}
-
-/* waveform: [T, 240 of ldp] summed + bias */
-template <int C>
-__global__ void __launch_bounds__(64)
-vt_codec_wave_kernel(float *__restrict__ out, const float *__restrict__ planes, int col0, int cuts, size_t plane_stride,
-                     int ldp, const float *__restrict__ bias) {
-    const int t = blockIdx.x, c = threadIdx.x * 4;
-    if (c >= CD_PATCH) return;
-    f32x4 v = cd_sum<C>(planes + (size_t)t * ldp + c, c < col0 ? 1 : cuts, plane_stride);
     if (bias) v += *(const f32x4 *)(bias + c);
     *(f32x4 *)(out + (size_t)t * CD_PATCH + c) = v;
 }
@@ -425,8 +408,8 @@ static struct {
     float *slopes;                /* [8] */
     cd_matrix w_in;               /* [1024, 896] */
     cd_layer_dev layers[CD_LAYERS];
-    cd_matrix w_up[3];            /* [2048, 2048] */
-    cd_matrix w_out;              /* [256, 7168] */
+    cd_matrix w_up[3];            /* [4096, 1024] */
+    cd_matrix w_out;              /* [1792, 1024] */
     float *b_in, *b_up[3], *b_out;
     /* work area, grown to the largest decode so far and laid out anew by each (cd_carve) */
     unsigned char *work;
@@ -502,18 +485,18 @@ static int cd_matrix_from(cd_matrix *m, float *d, int n, int k) {
     return ok;
 }
 
-/* conv1d weight [out_ch, in_ch, taps] -> [n_pad, k_pad] with k = tap * in_ch + ic */
-static float *cd_upload_conv(const tts_hip_host_conv_t *cv, int n_pad, int k_pad) {
-    const size_t n = (size_t)cv->out_ch * cv->in_ch * cv->kernel;
-    float *h = cd_host(cv->weight, n);
-    float *r = (float *)calloc((size_t)n_pad * k_pad, sizeof(float));
+/* conv1d weight [out_ch, in_ch, taps] -> zeros [n, k_dim] but for element (oc, ic, k) at row oc + row_tap * k, column
+ * ic + col_tap * k */
+static float *cd_upload_conv(const tts_hip_host_conv_t *cv, int n, int k_dim, int row_tap, int col_tap) {
+    float *h = cd_host(cv->weight, (size_t)cv->out_ch * cv->in_ch * cv->kernel);
+    float *r = (float *)calloc((size_t)n * k_dim, sizeof(float));
     float *d = NULL;
     if (h && r) {
         for (int oc = 0; oc < cv->out_ch; oc++)
             for (int ic = 0; ic < cv->in_ch; ic++)
                 for (int k = 0; k < cv->kernel; k++)
-                    r[(size_t)oc * k_pad + (size_t)k * cv->in_ch + ic] = h[((size_t)oc * cv->in_ch + ic) * cv->kernel + k];
-        d = cd_upload(r, (size_t)n_pad * k_pad);
+                    r[(size_t)(oc + row_tap * k) * k_dim + ic + col_tap * k] = h[((size_t)oc * cv->in_ch + ic) * cv->kernel + k];
+        d = cd_upload(r, (size_t)n * k_dim);
     } else {
         vt_set_error("codec upload: out of host memory");
     }
@@ -521,8 +504,8 @@ static float *cd_upload_conv(const tts_hip_host_conv_t *cv, int n_pad, int k_pad
     return d;
 }
 
-/* transposed conv weight [in_ch, out_ch, 4] -> [2 * 1024, 2 * 1024]: row p * 1024 + oc, column
- * q * 1024 + ic holds w[ic][oc][p + 2q] */
+/* transposed conv weight [in_ch, out_ch, 4] -> [4 * 1024, 1024]: row q * 2048 + p * 1024 + oc, column ic holds
+ * w[ic][oc][p + 2q] */
 static float *cd_upload_convt(const tts_hip_host_conv_t *cv) {
     const size_t n = (size_t)CD_DIM * CD_DIM * 4;
     float *h = cd_host(cv->weight, n);
@@ -533,7 +516,7 @@ static float *cd_upload_convt(const tts_hip_host_conv_t *cv) {
             for (int oc = 0; oc < CD_DIM; oc++)
                 for (int k = 0; k < 4; k++) {
                     const int p = k & 1, q = k >> 1;
-                    r[((size_t)p * CD_DIM + oc) * (2 * CD_DIM) + (size_t)q * CD_DIM + ic] = h[((size_t)ic * CD_DIM + oc) * 4 + k];
+                    r[((size_t)(2 * q + p) * CD_DIM + oc) * CD_DIM + ic] = h[((size_t)ic * CD_DIM + oc) * 4 + k];
                 }
         d = cd_upload(r, n);
     } else {
@@ -580,12 +563,12 @@ extern "C" int tts_hip_upload_codec_weights(void *codec_ptr) {
     int ok = 1;
     ok &= (g_cd.sem = cd_upload(c->semantic_embedding, (size_t)CD_SEM_SIZE * CD_SEM_DIM)) != NULL;
     ok &= (g_cd.slopes = cd_upload(c->alibi_slopes, CD_HEADS)) != NULL;
-    ok &= cd_matrix_from(&g_cd.w_in, cd_upload_conv(&c->input_conv, CD_DIM, CD_IN_K), CD_DIM, CD_IN_K);
+    ok &= cd_matrix_from(&g_cd.w_in, cd_upload_conv(&c->input_conv, CD_DIM, CD_IN_K, 0, CD_EMBED), CD_DIM, CD_IN_K);
     g_cd.b_in = cd_upload_bias(c->input_conv.bias, CD_DIM, CD_DIM, 1);
-    ok &= cd_matrix_from(&g_cd.w_out, cd_upload_conv(&c->output_proj, CD_OUT_N, CD_OUT_K), CD_OUT_N, CD_OUT_K);
-    g_cd.b_out = cd_upload_bias(c->output_proj.bias, CD_PATCH, CD_OUT_N, 1);
+    ok &= cd_matrix_from(&g_cd.w_out, cd_upload_conv(&c->output_proj, CD_OUT_N, CD_DIM, CD_OUT_PITCH, 0), CD_OUT_N, CD_DIM);
+    g_cd.b_out = cd_upload_bias(c->output_proj.bias, CD_PATCH, CD_OUT_PITCH, 1);
     for (int i = 0; ok && i < 3; i++) {
-        ok &= cd_matrix_from(&g_cd.w_up[i], cd_upload_convt(&c->stage_convs[i]), 2 * CD_DIM, 2 * CD_DIM);
+        ok &= cd_matrix_from(&g_cd.w_up[i], cd_upload_convt(&c->stage_convs[i]), CD_UP_N, CD_DIM);
         g_cd.b_up[i] = cd_upload_bias(c->stage_convs[i].bias, CD_DIM, CD_DIM, 1);
     }
     for (int i = 0; ok && i < CD_LAYERS; i++) {
@@ -636,7 +619,7 @@ static int cd_reserve(int n_frames) {
         part = n > part ? n : part;
     }
     /* the pieces start at multiples of 256 bytes */
-    const size_t f = sizeof(float), sizes[] = {T * CD_DIM * f, T * 3 * CD_DIM * f, part * f, T * CD_PATCH * f, T * CD_OUT_K * 2, T * CD_OUT_K * 2,
+    const size_t f = sizeof(float), sizes[] = {T * CD_DIM * f, T * 3 * CD_DIM * f, part * f, T * CD_PATCH * f, T * CD_HID * 2, T * CD_HID * 2,
                                                (T + 4) * f, (size_t)n_frames * 37 * sizeof(int)};
     size_t total = 0, at[8];
     for (int i = 0; i < 8; i++) { at[i] = total; total += (sizes[i] + 255) & ~(size_t)255; }
@@ -664,13 +647,16 @@ static vt_gemm_plan cd_gemm(int M, const cd_matrix &w) {
 }
 
 /* CALL(C) with the instance that requests enough planes at once */
-#define CD_BY_CUTS(cuts, CALL) do { if ((cuts) <= 1) CALL(1); else if ((cuts) <= 2) CALL(2); else if ((cuts) <= 4) CALL(4); else CALL(VT_MAX_CUTS); } while (0)
+#define CD_BY_CUTS(cuts, CALL) do { if ((cuts) <= 1) { CALL(1); } else if ((cuts) <= 2) { CALL(2); } else if ((cuts) <= 4) { CALL(4); } else { CALL(VT_MAX_CUTS); } } while (0)
 
-/* M product rows of w.n columns = rows of 1024 -> x (bias or layer scale and residual), planes of its RMSNorm */
-static void cd_row(const vt_gemm_plan &pl, int M, int n, const float *x_in, const float *bias, const float *scale, const float *norm_w) {
-    const int rows = (int)((size_t)M * n / CD_DIM);
-#define CALL(C) hipLaunchKernelGGL(vt_codec_row_kernel<C>, dim3(rows), dim3(256), 0, g_vt.stream, g_cd.x, g_cd.planes, x_in, g_cd.part, pl.col0, pl.cuts, \
-                                   (size_t)M * n, n, bias, scale, norm_w, CD_EPS)
+/* M product rows (up: of the upsampling product, two rows of 1024 each) -> x (bias or layer scale and residual) and
+ * planes of its RMSNorm; norm_w NULL: its planes only */
+static void cd_row(const vt_gemm_plan &pl, int M, bool up, const float *x_in, const float *bias, const float *scale, const float *norm_w) {
+#define CALL(C) \
+    if (up) hipLaunchKernelGGL((vt_codec_row_kernel<C, true>), dim3(2 * M), dim3(256), 0, g_vt.stream, g_cd.x, g_cd.planes, x_in, g_cd.part, \
+                               pl.col0, pl.cuts, (size_t)M * CD_UP_N, bias, scale, norm_w, CD_EPS); \
+    else hipLaunchKernelGGL((vt_codec_row_kernel<C, false>), dim3(M), dim3(256), 0, g_vt.stream, g_cd.x, g_cd.planes, x_in, g_cd.part, \
+                            pl.col0, pl.cuts, (size_t)M * CD_DIM, bias, scale, norm_w, CD_EPS)
     CD_BY_CUTS(pl.cuts, CALL);
 #undef CALL
 }
@@ -681,7 +667,7 @@ static int cd_enqueue(const int *d_codes, int n_frames, float *d_samples) {
     const float scale = 1.0f / sqrtf((float)CD_HEAD_DIM);
     hipLaunchKernelGGL(vt_codec_embed_kernel, dim3(T), dim3(256), 0, g_vt.stream, g_cd.planes, d_codes, g_cd.sem, T);
     vt_gemm_plan pl = cd_gemm(T, g_cd.w_in);
-    cd_row(pl, T, CD_DIM, NULL, g_cd.b_in, NULL, g_cd.layers[0].attention_norm);
+    cd_row(pl, T, false, NULL, g_cd.b_in, NULL, g_cd.layers[0].attention_norm);
     for (int li = 0; li < CD_LAYERS; li++) {
         const cd_layer_dev *l = &g_cd.layers[li];
         pl = cd_gemm(T, l->wqkv);
@@ -695,25 +681,23 @@ static int cd_enqueue(const int *d_codes, int n_frames, float *d_samples) {
             hipLaunchKernelGGL(vt_codec_attention_kernel, dim3((T + CD_ATT_TOKENS - 1) / CD_ATT_TOKENS), dim3(64 * CD_HEADS), 0, g_vt.stream, g_cd.planes,
                                g_cd.qkv, T, l->window, g_cd.slopes, scale);
         pl = cd_gemm(T, l->wo);
-        cd_row(pl, T, CD_DIM, g_cd.x, NULL, l->attn_scale, l->ffn_norm);
+        cd_row(pl, T, false, g_cd.x, NULL, l->attn_scale, l->ffn_norm);
         pl = cd_gemm(T, l->w13);
 #define CALL(C) hipLaunchKernelGGL(vt_codec_swiglu_kernel<C>, dim3(T), dim3(256), 0, g_vt.stream, g_cd.planes, g_cd.part, pl.col0, pl.cuts, (size_t)T * 2 * CD_HID)
         CD_BY_CUTS(pl.cuts, CALL);
 #undef CALL
         pl = cd_gemm(T, l->w2);
         const int last_of_stage = (li & 1) == 1;
-        cd_row(pl, T, CD_DIM, g_cd.x, NULL, l->ffn_scale, last_of_stage ? NULL : g_cd.layers[li + 1].attention_norm);
+        cd_row(pl, T, false, g_cd.x, NULL, l->ffn_scale, last_of_stage ? NULL : g_cd.layers[li + 1].attention_norm);
         if (last_of_stage && li < CD_LAYERS - 1) {
             const int st = li / 2;
-            hipLaunchKernelGGL(vt_codec_pair_kernel, dim3(T), dim3(256), 0, g_vt.stream, g_cd.planes, g_cd.x, T);
             pl = cd_gemm(T, g_cd.w_up[st]);
-            cd_row(pl, T, 2 * CD_DIM, NULL, g_cd.b_up[st], NULL, g_cd.layers[li + 1].attention_norm);       /* [T, 2048] is [2T, 1024] */
+            cd_row(pl, T, true, NULL, g_cd.b_up[st], NULL, g_cd.layers[li + 1].attention_norm);
             T *= 2;
         }
     }
-    hipLaunchKernelGGL(vt_codec_taps_kernel, dim3(T), dim3(256), 0, g_vt.stream, g_cd.planes, g_cd.x, T);
     pl = cd_gemm(T, g_cd.w_out);
-#define CALL(C) hipLaunchKernelGGL(vt_codec_wave_kernel<C>, dim3(T), dim3(64), 0, g_vt.stream, d_samples, g_cd.part, pl.col0, pl.cuts, (size_t)T * CD_OUT_N, CD_OUT_N, g_cd.b_out)
+#define CALL(C) hipLaunchKernelGGL(vt_codec_wave_kernel<C>, dim3(T), dim3(64), 0, g_vt.stream, d_samples, g_cd.part, pl.col0, pl.cuts, (size_t)T * CD_OUT_N, T, g_cd.b_out)
     CD_BY_CUTS(pl.cuts, CALL);
 #undef CALL
     return vt_check(hipGetLastError(), "codec launch");
