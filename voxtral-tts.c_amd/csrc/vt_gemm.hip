@@ -225,37 +225,55 @@ void vt_launch_split(uint16_t *d_hi, uint16_t *d_lo, const float *d_x, size_t n)
     hipLaunchKernelGGL(vt_split_kernel, dim3(gm_blocks(n / 2)), dim3(256), 0, g_vt.stream, d_hi, d_lo, d_x, n / 2);
 }
 
+/* CALL(P) with P = planes, 1 .. VT_MAX_CUTS */
+#define GM_BY_PLANES(planes, CALL) do { switch (planes) { case 1: CALL(1); break; case 2: CALL(2); break; case 3: CALL(3); break; \
+    case 4: CALL(4); break; case 5: CALL(5); break; case 6: CALL(6); break; case 7: CALL(7); break; default: CALL(8); } } while (0)
+static_assert(VT_MAX_CUTS == 8, "GM_BY_PLANES");
+
 /* One workgroup per row of 3072 floats (256 threads x 12):
- *   x[row] += part[0][row] (+ part[1][row] + ... for the columns from col0 on)   (cuts > 0; fixed order)
+ *   x[row] += part[0][row] (+ part[1][row] + ... for the columns from col0 on)   (C > 0 cuts; fixed order)
  *   (hi, lo)[row] = split(rmsnorm(x[row]) * w)                                   (w != NULL)
  * The residual add and the normalisation of voxtral_tts_llm.c:332-336,354 /
- * :338-341 in one pass over the row. */
+ * :338-341 in one pass over the row.  Up to a few hundred rows a launch is one chain of memory latencies per
+ * workgroup, so everything is requested in front of the first sum (columns that are not cut ask for plane 0 again);
+ * with the planes in a loop that waited for each of them a launch took 8.5 us at 226 rows and takes 6.0 to 6.6 now; us per
+ * prefill of 37 / 226 / 512 / 1531 rows 2632 / 4414 / 7236 / 20457 -> 2481 / 4326 / 7186 / 20181, results the same. */
+template <int C>
 __global__ void __launch_bounds__(256)
-vt_residual_norm_split_kernel(float *x, const float *part, int col0, int cuts, size_t part_stride,
+vt_residual_norm_split_kernel(float *x, const float *part, int col0, size_t part_stride,
                               const float *w, uint16_t *hi, uint16_t *lo, float eps) {
     /* a thread owns 4 consecutive columns at 4 (t + 256 j): 16-byte loads and stores, 8-byte plane
      * stores (a quarter of the memory instructions of element-wise accesses) */
     __shared__ float red[4];
     const size_t row = blockIdx.x;
     constexpr int NJ = VT_DIM / 1024;
-    f32x4 v[NJ];
-    float ss = 0.f;
+    f32x4 v[NJ], g[NJ], p[NJ][C > 0 ? C : 1];
 #pragma unroll
     for (int j = 0; j < NJ; j++) {
         const int c = 4 * ((int)threadIdx.x + 256 * j);
         const size_t i = row * VT_DIM + c;
-        f32x4 a = *reinterpret_cast<const f32x4 *>(x + i);
-        if (cuts > 0) {
-            f32x4 p = *reinterpret_cast<const f32x4 *>(part + i);
-            const int n = c < col0 ? 1 : cuts;
-            for (int s = 1; s < n; s++) {
-                const f32x4 q = *reinterpret_cast<const f32x4 *>(part + (size_t)s * part_stride + i);
-                p.x = __fadd_rn(p.x, q.x); p.y = __fadd_rn(p.y, q.y);
-                p.z = __fadd_rn(p.z, q.z); p.w = __fadd_rn(p.w, q.w);
-            }
-            a.x = __fadd_rn(a.x, p.x); a.y = __fadd_rn(a.y, p.y);
-            a.z = __fadd_rn(a.z, p.z); a.w = __fadd_rn(a.w, p.w);
-            *reinterpret_cast<f32x4 *>(x + i) = a;
+        v[j] = *reinterpret_cast<const f32x4 *>(x + i);
+#pragma unroll
+        for (int s = 0; s < C; s++) p[j][s] = *reinterpret_cast<const f32x4 *>(part + (c < col0 ? 0 : s) * part_stride + i);
+        g[j] = v[j];
+        if (w) g[j] = *reinterpret_cast<const f32x4 *>(w + c);
+    }
+    float ss = 0.f;
+#pragma unroll
+    for (int j = 0; j < NJ; j++) {
+        const int c = 4 * ((int)threadIdx.x + 256 * j);
+        f32x4 a = v[j];
+        if (C > 0) {
+            f32x4 q = p[j][0];
+#pragma unroll
+            for (int s = 1; s < C; s++)
+                if (c >= col0) {
+                    q.x = __fadd_rn(q.x, p[j][s].x); q.y = __fadd_rn(q.y, p[j][s].y);
+                    q.z = __fadd_rn(q.z, p[j][s].z); q.w = __fadd_rn(q.w, p[j][s].w);
+                }
+            a.x = __fadd_rn(a.x, q.x); a.y = __fadd_rn(a.y, q.y);
+            a.z = __fadd_rn(a.z, q.z); a.w = __fadd_rn(a.w, q.w);
+            *reinterpret_cast<f32x4 *>(x + row * VT_DIM + c) = a;
         }
         v[j] = a;
         ss = fmaf(a.x, a.x, ss); ss = fmaf(a.y, a.y, ss);
@@ -270,9 +288,9 @@ vt_residual_norm_split_kernel(float *x, const float *part, int col0, int cuts, s
 #pragma unroll
     for (int j = 0; j < NJ; j++) {
         const int c = 4 * ((int)threadIdx.x + 256 * j);
-        const f32x4 g = *reinterpret_cast<const f32x4 *>(w + c);
         u32x2 sph, spl;
-        vt_split_planes4(__fmul_rn(__fmul_rn(v[j].x, inv), g.x), __fmul_rn(__fmul_rn(v[j].y, inv), g.y), __fmul_rn(__fmul_rn(v[j].z, inv), g.z), __fmul_rn(__fmul_rn(v[j].w, inv), g.w), sph, spl);
+        vt_split_planes4(__fmul_rn(__fmul_rn(v[j].x, inv), g[j].x), __fmul_rn(__fmul_rn(v[j].y, inv), g[j].y),
+                         __fmul_rn(__fmul_rn(v[j].z, inv), g[j].z), __fmul_rn(__fmul_rn(v[j].w, inv), g[j].w), sph, spl);
         *reinterpret_cast<u32x2 *>(hi + row * VT_DIM + c) = sph;
         *reinterpret_cast<u32x2 *>(lo + row * VT_DIM + c) = spl;
     }
@@ -280,8 +298,11 @@ vt_residual_norm_split_kernel(float *x, const float *part, int col0, int cuts, s
 
 void vt_launch_residual_norm_split(float *d_x, const float *d_part, int col0, int cuts, size_t part_stride,
                                    const float *d_w, uint16_t *d_hi, uint16_t *d_lo, int rows) {
-    hipLaunchKernelGGL(vt_residual_norm_split_kernel, dim3(rows), dim3(256), 0, g_vt.stream, d_x, d_part,
-                       col0, cuts, part_stride, d_w, d_hi, d_lo, VT_EPS);
+#define CALL(C) hipLaunchKernelGGL(vt_residual_norm_split_kernel<C>, dim3(rows), dim3(256), 0, g_vt.stream, d_x, d_part, \
+                                   col0, part_stride, d_w, d_hi, d_lo, VT_EPS)
+    if (cuts <= 0) CALL(0);
+    else GM_BY_PLANES(cuts, CALL);
+#undef CALL
 }
 
 /* gu [rows, 2*ffn] with (gate, up) adjacent -> (hi, lo) planes of silu(gate)*up
@@ -334,21 +355,27 @@ void vt_launch_swiglu_split(uint16_t *d_hi, uint16_t *d_lo, const float *d_gu, s
 /* The K-cut tail of the paired gate|up product: tail [planes][rows, tw] fp32 in the paired column order
  * (of every 64 columns the first 32 are gates, the other 32 the ups of the same h columns) -> the
  * (hi, lo) planes of SiLU(gate) * up at h columns h_col0 .. h_col0 + tw/2 (row pitch ldh).  A thread owns 4
- * consecutive h columns. */
+ * consecutive h columns and requests all its planes at once. */
+template <int P>
 __global__ void vt_swiglu_pair_tail_kernel(uint16_t *hi, uint16_t *lo, int ldh, int h_col0, const float *tail,
-                                           int planes, size_t stride, int rows, int tw) {
+                                           size_t stride, int rows, int tw) {
     const int per_row = tw / 8;                                   /* threads per row */
     const size_t total = (size_t)rows * per_row;
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (size_t)gridDim.x * blockDim.x) {
         const int row = (int)(i / per_row), q = (int)(i % per_row);
         const int blk = q >> 3, c = (q & 7) * 4;
         const float *tp = tail + (size_t)row * tw + 64 * blk + c;
-        f32x4 g = *reinterpret_cast<const f32x4 *>(tp), u = *reinterpret_cast<const f32x4 *>(tp + 32);
-        for (int p = 1; p < planes; p++) {
-            const f32x4 g2 = *reinterpret_cast<const f32x4 *>(tp + p * stride);
-            const f32x4 u2 = *reinterpret_cast<const f32x4 *>(tp + p * stride + 32);
-            g.x = __fadd_rn(g.x, g2.x); g.y = __fadd_rn(g.y, g2.y); g.z = __fadd_rn(g.z, g2.z); g.w = __fadd_rn(g.w, g2.w);
-            u.x = __fadd_rn(u.x, u2.x); u.y = __fadd_rn(u.y, u2.y); u.z = __fadd_rn(u.z, u2.z); u.w = __fadd_rn(u.w, u2.w);
+        f32x4 gs[P], us[P];
+#pragma unroll
+        for (int p = 0; p < P; p++) {
+            gs[p] = *reinterpret_cast<const f32x4 *>(tp + p * stride);
+            us[p] = *reinterpret_cast<const f32x4 *>(tp + p * stride + 32);
+        }
+        f32x4 g = gs[0], u = us[0];
+#pragma unroll
+        for (int p = 1; p < P; p++) {
+            g.x = __fadd_rn(g.x, gs[p].x); g.y = __fadd_rn(g.y, gs[p].y); g.z = __fadd_rn(g.z, gs[p].z); g.w = __fadd_rn(g.w, gs[p].w);
+            u.x = __fadd_rn(u.x, us[p].x); u.y = __fadd_rn(u.y, us[p].y); u.z = __fadd_rn(u.z, us[p].z); u.w = __fadd_rn(u.w, us[p].w);
         }
         const float a = vt_silu_mul(g.x, u.x);
         const float b = vt_silu_mul(g.y, u.y);
@@ -364,8 +391,10 @@ __global__ void vt_swiglu_pair_tail_kernel(uint16_t *hi, uint16_t *lo, int ldh, 
 
 void vt_launch_swiglu_pair_tail(uint16_t *d_hi, uint16_t *d_lo, int ldh, int h_col0, const float *d_tail, int planes,
                                 size_t stride, int rows, int tw) {
-    hipLaunchKernelGGL(vt_swiglu_pair_tail_kernel, dim3(gm_blocks((size_t)rows * tw / 8)), dim3(256), 0, g_vt.stream,
-                       d_hi, d_lo, ldh, h_col0, d_tail, planes, stride, rows, tw);
+#define CALL(P) hipLaunchKernelGGL(vt_swiglu_pair_tail_kernel<P>, dim3(gm_blocks((size_t)rows * tw / 8)), dim3(256), 0, g_vt.stream, \
+                                   d_hi, d_lo, ldh, h_col0, d_tail, stride, rows, tw)
+    GM_BY_PLANES(planes, CALL);
+#undef CALL
 }
 
 /* C = sum of `splits` partial planes (fixed order), for callers that want the plain product. */
