@@ -46,6 +46,41 @@ def test_prefill_with_gates_far_from_zero():
         hip.close()
 
 
+def test_prefill_with_gates_near_the_ends_of_fp32():
+    """Gates of -1e37 leave SiLU(gate) * up = 0 and gates of 2.8e38 times an up of 0 as well: h columns of both kinds
+    between ordinary ones.  Channel 0 of the normalised rows is about 37 everywhere (the first embedding column is 50, the
+    attention adds nothing), so a w1 row that reads it alone gives all rows the same gate, to a few per cent."""
+    import numpy as np
+    import cases
+    import hipsupport as H
+    import vtsupport as S
+    layer = S.Layer(14)
+    layer.wo[...] = 0
+    x0 = 50.0 / np.sqrt((50.0 ** 2 + S.DIM - 1) / S.DIM) * float(layer.ffn_norm[0])
+    for cols, gate in ((slice(0, None, 3), -1e37), (slice(1, None, 97), 2.8e38)):
+        w = np.zeros(S.DIM, np.float32)
+        w[0] = gate / x0
+        layer.w1[cols] = S.f32_to_bf16_trunc(w)
+    layer.w3[1::97] = 0
+    norm = S.norm_weight(S.DIM, 98)
+    orc = cases.OracleBackend(threads=16)
+    orc.llm_open([layer], norm, 192, n_layers=1)
+    hip = H.Hip(kv_max=192)
+    try:
+        hip.upload_decoder([layer], norm, 1)
+        for s in (37, 80):                                           # both gate|up kernels, whole tiles and cut ones
+            e = S.f32_normal((s, S.DIM), 95 + s)
+            e[:, 0] = 50.0
+            rx, gx = orc.llm_prefill(e, want_x=True), hip.llm_prefill(e, want_x=True)
+            hip.check()
+            assert np.all(np.isfinite(rx)) and np.all(np.isfinite(gx))
+            for r in range(s):
+                mx, l2 = S.rel_errors((rx - e)[r, 1:], (gx - e)[r, 1:])
+                assert mx < 1e-3 and l2 < 1e-3, (s, r, mx, l2)
+    finally:
+        hip.close()
+
+
 @pytest.mark.parametrize("chunks", [[1, 8], [37, 64], [65, 97], [226, 41]])
 def test_prefill_for_the_cache_alone(chunks):
     """Without the rows the last layer is its k|v product only: the cache is the one of the whole prefill, the last

@@ -163,8 +163,7 @@ vt_codec_swiglu_kernel(cd_planes h, const float *__restrict__ gu, int col0, int 
         const int c = 4 * ((int)threadIdx.x + 256 * j);
         const float *p = gu + (size_t)row * (2 * CD_HID) + c;
         const f32x4 g = cd_sum<C>(p, c < col0 ? 1 : cuts, plane_stride), u = cd_sum<C>(p + CD_HID, CD_HID + c < col0 ? 1 : cuts, plane_stride);
-#pragma unroll
-        for (int i = 0; i < 4; i++) v[j][i] = vt_silu_mul(g[i], u[i]);
+        v[j] = vt_silu_mul4(g, u);
         m = fmaxf(m, cd_max4(v[j]));
     }
     const float s = vt_f16_scale(cd_block_max(m, red));

@@ -65,23 +65,35 @@ void vt_launch_swiglu_split(uint16_t *d_hi, uint16_t *d_lo, const float *d_gu, s
 void vt_launch_sum_planes(float *d_out, const float *d_part, int splits, size_t stride, size_t n);
 
 #ifdef __HIPCC__
-/* SiLU(gate) * up (voxtral_tts_kernels.c's tts_silu and tts_mul_inplace) for results that go on as (hi, lo) planes:
- * exp2 of the product with log2(e) and the product's rounding error carried on to first order, the quotient from
- * the reciprocal estimate with one Newton step and one correction of the quotient; both good to about one ulp
- * (2^-23; the planes keep 2^-17).  A third of the instructions of expf and an IEEE division: as the epilogue of
- * a 128 x 256 gate|up tile those took 5 of its 7.5 us.  The exponent stops at 2^120 (gate < -83), where the
- * result is below 1e-34 and its planes are as good as zero. */
-__device__ __forceinline__ float vt_silu_mul(float g, float u) {
-    const float log2e = 1.44269504f, log2e_lo = 1.92596303e-8f;     /* log2(e) = their sum */
-    const float t = fminf(__fmul_rn(-g, log2e), 120.f);
-    const float r = fmaf(-g, log2e_lo, fmaf(-g, log2e, -t));        /* what the product's rounding left out (clamped t: unused) */
+/* SiLU(gate) * up (voxtral_tts_kernels.c's tts_silu and tts_mul_inplace), four at a time.  The quotient
+ * g / (1 + exp(-g)) with exp2 of the product with log2(e), the product's rounding error carried on to first order, a
+ * denominator in two floats, and the reciprocal estimate with one correction of the quotient.  Largest error against 64
+ * bits, and of g / (1 + expf(-g)) with an IEEE division: 1.36e-7 / 1.84e-7 for g in -83 .. 0, 0.91e-7 / 1.50e-7 above.
+ * A third of the instructions of that formula: as the epilogue of a 128 x 256 gate|up tile it took 5 of its 7.5 us. */
+__device__ __forceinline__ float vt_silu_mul_small(float g, float u) {       /* |g| < VT_SILU_SMALL, or NaN */
+    const float log2e = 1.44269504f, log2e_lo = 1.92596303e-8f;              /* log2(e) = their sum */
+    const float t = __fmul_rn(-g, log2e);
+    const float r = fmaf(-g, log2e_lo, fmaf(-g, log2e, -t));                 /* what the product's rounding left out */
     const float e = __builtin_amdgcn_exp2f(t);
-    const float d = 1.0f + (t < 120.f ? fmaf(e, r * 0.693147181f, e) : e);
-    float y = __builtin_amdgcn_rcpf(d);
-    y = fmaf(fmaf(-d, y, 1.0f), y, y);
+    const float d = __fadd_rn(1.0f, e);                                      /* the denominator is d + dl */
+    const float dl = fmaf(e, r * 0.693147181f, fminf(e, 1.0f) - (d - fmaxf(e, 1.0f)));
+    const float y = __builtin_amdgcn_rcpf(d);
     float q = g * y;
-    q = fmaf(fmaf(-q, d, g), y, q);
+    q = fmaf(fmaf(-q, dl, fmaf(-q, d, g)), y, q);
     return q * u;
+}
+#define VT_SILU_SMALL 83.0f       /* exp(-g) and its reciprocal stay normal, with room for the quotient */
+__device__ __forceinline__ f32x4 vt_silu_mul4(const f32x4 &g, const f32x4 &u) {
+    f32x4 h;
+#pragma unroll
+    for (int v = 0; v < 4; v++) h[v] = vt_silu_mul_small(g[v], u[v]);
+    /* beyond, infinities included, the formula itself (rare: skipped by waves that have no such gate) */
+    if (__builtin_expect(fmaxf(fmaxf(fabsf(g.x), fabsf(g.y)), fmaxf(fabsf(g.z), fabsf(g.w))) >= VT_SILU_SMALL, 0)) {
+#pragma unroll
+        for (int v = 0; v < 4; v++)
+            if (fabsf(g[v]) >= VT_SILU_SMALL) h[v] = __fmul_rn(__fdiv_rn(g[v], __fadd_rn(1.0f, expf(-g[v]))), u[v]);
+    }
+    return h;
 }
 
 /* Four gates and ups of one column (rows v = 0..3; the neighbouring lane holds the next column) -> plane words of two
@@ -89,9 +101,7 @@ __device__ __forceinline__ float vt_silu_mul(float g, float u) {
  * stores, two per quad instead of four of 2 bytes.  The words belong to columns c & ~1 and c | 1. */
 struct vt_h_quad { unsigned hi[2], lo[2]; int row; };
 __device__ __forceinline__ vt_h_quad vt_silu_mul_quad(const f32x4 &g, const f32x4 &u) {
-    float h[4];
-#pragma unroll
-    for (int v = 0; v < 4; v++) h[v] = vt_silu_mul(g[v], u[v]);
+    const f32x4 h = vt_silu_mul4(g, u);
     const bool odd = threadIdx.x & 1;
     vt_h_quad o;
     o.row = odd ? 2 : 0;

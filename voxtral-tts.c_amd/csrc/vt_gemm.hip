@@ -335,12 +335,9 @@ __global__ void vt_swiglu_split_kernel(uint16_t *hi, uint16_t *lo, const float *
                 }
             }
         }
-        const float a = vt_silu_mul(g0.x, g0.y);
-        const float b = vt_silu_mul(g0.z, g0.w);
-        const float c = vt_silu_mul(g1.x, g1.y);
-        const float d = vt_silu_mul(g1.z, g1.w);
+        const f32x4 h = vt_silu_mul4(f32x4{g0.x, g0.z, g1.x, g1.z}, f32x4{g0.y, g0.w, g1.y, g1.w});
         u32x2 sph, spl;
-        vt_split_planes4(a, b, c, d, sph, spl);
+        vt_split_planes4(h.x, h.y, h.z, h.w, sph, spl);
         reinterpret_cast<u32x2 *>(hi)[i] = sph;
         reinterpret_cast<u32x2 *>(lo)[i] = spl;
     }
@@ -377,12 +374,9 @@ __global__ void vt_swiglu_pair_tail_kernel(uint16_t *hi, uint16_t *lo, int ldh, 
             g.x = __fadd_rn(g.x, gs[p].x); g.y = __fadd_rn(g.y, gs[p].y); g.z = __fadd_rn(g.z, gs[p].z); g.w = __fadd_rn(g.w, gs[p].w);
             u.x = __fadd_rn(u.x, us[p].x); u.y = __fadd_rn(u.y, us[p].y); u.z = __fadd_rn(u.z, us[p].z); u.w = __fadd_rn(u.w, us[p].w);
         }
-        const float a = vt_silu_mul(g.x, u.x);
-        const float b = vt_silu_mul(g.y, u.y);
-        const float cc = vt_silu_mul(g.z, u.z);
-        const float d = vt_silu_mul(g.w, u.w);
+        const f32x4 h = vt_silu_mul4(g, u);
         u32x2 sph, spl;
-        vt_split_planes4(a, b, cc, d, sph, spl);
+        vt_split_planes4(h.x, h.y, h.z, h.w, sph, spl);
         const size_t at = (size_t)row * ldh + h_col0 + 32 * blk + c;
         *reinterpret_cast<u32x2 *>(hi + at) = sph;
         *reinterpret_cast<u32x2 *>(lo + at) = spl;
