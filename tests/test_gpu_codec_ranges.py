@@ -1,0 +1,39 @@
+"""The codec's products hold an fp32 operand as two fp16 planes and an exponent per row.  What fp32 arithmetic takes in
+its stride: rows whose values stand near either end of fp32."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import codecsupport as K
+import hipsupport as H
+import vtsupport as S
+from test_gpu_codec import hip_decode
+from test_gpu_codec_planes import close
+
+pytestmark = pytest.mark.gpu
+
+
+def decode_both(hc, frames):
+    S.oracle().orc_set_threads(16)
+    cs = hc.struct()
+    hip = H.Hip(kv_max=8)
+    try:
+        assert hip.lib.tts_hip_upload_codec_weights(C.addressof(cs)) == 0, hip.lib.tts_hip_last_error()
+        for n in frames:
+            codes = K.random_codes(n, 60 + n)
+            print(f"codec of {n} frames", flush=True)
+            close(K.oracle_decode(cs, codes), hip_decode(hip, codes))
+    finally:
+        hip.close()
+        S.oracle().orc_set_threads(1)
+
+
+def test_rows_near_the_ends_of_fp32():
+    """The residual stream of the second stage at 1e34 (its RMSNorms overflow and give zeros, as on the CPU) between
+    convolutions of 2^113 and 2^-113 times ordinary weights."""
+    hc = K.HostCodec(9, distinct_layers=1)
+    for conv, f in ((hc.stage_convs[0], 2.0 ** 113), (hc.stage_convs[1], 2.0 ** -113)):
+        conv.weight *= np.float32(f)
+    hc.stage_convs[0].bias *= np.float32(2.0 ** 113)
+    decode_both(hc, (5, 40))

@@ -18,7 +18,7 @@
  *     write the copies (100 us of a 1003-frame decode); us per decode of 21 / 212 / 1003 frames:
  *     731 / 1595 / 4983 -> 712 / 1558 / 4890.
  * Every product runs on the fp16 matrix cores with both operands as two fp16 planes
- * (vt_codec_gemm.hip); whoever produces a product's input leaves it as planes with one scale
+ * (vt_codec_gemm.hip); whoever produces a product's input leaves it as planes with one exponent
  * per row.  Where a launch would not fill the chip K is cut, and the kernel that reads the
  * result adds the partial planes in a fixed order, next to bias / layer scale / residual and
  * the next RMSNorm.
@@ -66,12 +66,12 @@ __device__ __forceinline__ float cd_block_max(float v, float *red) {
 }
 __device__ __forceinline__ float cd_max4(const f32x4 &v) { return fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))); }
 
-/* A product's input: two fp16 planes [rows, K] and the factor that undoes the scaling, per row */
-struct cd_planes { uint16_t *hi, *lo; float *inv; };
+/* A product's input: two fp16 planes [rows, K] of the rows times 2^exp, an exponent per row */
+struct cd_planes { uint16_t *hi, *lo; int *exp; };
 
-__device__ __forceinline__ void cd_put4(const cd_planes &p, size_t at, const f32x4 &v, float scale) {
+__device__ __forceinline__ void cd_put4(const cd_planes &p, size_t at, const f32x4 &v, int e) {
     u32x2 h, l;
-    vt_split_f16x4(v * scale, h, l);
+    vt_split_f16x4(vt_ldexp4(v, e), h, l);
     *(u32x2 *)(p.hi + at) = h;
     *(u32x2 *)(p.lo + at) = l;
 }
@@ -121,9 +121,9 @@ vt_codec_row_kernel(float *x_out, cd_planes xn, const float *x_in, const float *
         const float inv = 1.0f / sqrtf(ss / (float)CD_DIM + eps);
         v = v * inv * *(const f32x4 *)(norm_w + c);
     }
-    const float s = vt_f16_scale(cd_block_max(cd_max4(v), red));
-    cd_put4(xn, at, v, s);
-    if (threadIdx.x == 0) xn.inv[row] = 1.0f / s;
+    const int e = vt_f16_exp(cd_block_max(cd_max4(v), red));
+    cd_put4(xn, at, v, e);
+    if (threadIdx.x == 0) xn.exp[row] = e;
 }
 
 /* q|k|v [T, 3072] summed, with the RMSNorm over the whole 1024-wide q row and k row (tts_qk_norm,
@@ -166,10 +166,10 @@ vt_codec_swiglu_kernel(cd_planes h, const float *__restrict__ gu, int col0, int 
         v[j] = vt_silu_mul4(g, u);
         m = fmaxf(m, cd_max4(v[j]));
     }
-    const float s = vt_f16_scale(cd_block_max(m, red));
+    const int e = vt_f16_exp(cd_block_max(m, red));
 #pragma unroll
-    for (int j = 0; j < CD_HID / 1024; j++) cd_put4(h, (size_t)row * CD_HID + 4 * ((int)threadIdx.x + 256 * j), v[j], s);
-    if (threadIdx.x == 0) h.inv[row] = 1.0f / s;
+    for (int j = 0; j < CD_HID / 1024; j++) cd_put4(h, (size_t)row * CD_HID + 4 * ((int)threadIdx.x + 256 * j), v[j], e);
+    if (threadIdx.x == 0) h.exp[row] = e;
 }
 
 /* ALiBi causal sliding-window attention, the online softmax of a query over the at most `window` keys in ascending
@@ -273,11 +273,11 @@ vt_codec_attention_kernel(cd_planes out, const float *__restrict__ qkv, int T, i
         float m = 0.f;
 #pragma unroll
         for (int w = 0; w < CD_HEADS; w++) m = fmaxf(m, red[w][2 * g + t]);
-        const float s = vt_f16_scale(m);
+        const int ex = vt_f16_exp(m);
         if (live[t]) {
 #pragma unroll
-            for (int e = 0; e < 4; e++) cd_put4(out, (size_t)(i0 + t) * CD_DIM + h * CD_HEAD_DIM + 32 * e + 4 * sub, st[t]->o.v[e], s);
-            if (h == 0 && sub == 0) out.inv[i0 + t] = 1.0f / s;
+            for (int e = 0; e < 4; e++) cd_put4(out, (size_t)(i0 + t) * CD_DIM + h * CD_HEAD_DIM + 32 * e + 4 * sub, st[t]->o.v[e], ex);
+            if (h == 0 && sub == 0) out.exp[i0 + t] = ex;
         }
     }
 }
@@ -324,13 +324,13 @@ vt_codec_attention_split_kernel(cd_planes out, const float *__restrict__ qkv, in
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < CD_HEADS; k++) m = fmaxf(m, red[k]);
-    const float sc = vt_f16_scale(m);
+    const int ex = vt_f16_exp(m);
     unsigned hi, lo;
-    vt_split_f16x2(x * sc, y * sc, hi, lo);
+    vt_split_f16x2(__builtin_amdgcn_ldexpf(x, ex), __builtin_amdgcn_ldexpf(y, ex), hi, lo);
     const size_t at = (size_t)i * CD_DIM + h * CD_HEAD_DIM + 32 * (2 * (int)b3 + (int)b4) + 4 * sub + 2 * (int)b5;
     *(unsigned *)(out.hi + at) = hi;
     *(unsigned *)(out.lo + at) = lo;
-    if (threadIdx.x == 0) out.inv[i] = 1.0f / sc;
+    if (threadIdx.x == 0) out.exp[i] = ex;
 }
 
 /* codes [T, 37] -> the three shifted copies of the 292-wide embedding that the input
@@ -364,9 +364,9 @@ vt_codec_embed_kernel(cd_planes a, const int *__restrict__ codes, const float *_
                 }
             }
         }
-    const float s = vt_f16_scale(cd_block_max(cd_max4(v), red));
-    if (base < CD_IN_K) cd_put4(a, (size_t)t * CD_IN_K + base, v, s);
-    if (threadIdx.x == 0) a.inv[t] = 1.0f / s;
+    const int e = vt_f16_exp(cd_block_max(cd_max4(v), red));
+    if (base < CD_IN_K) cd_put4(a, (size_t)t * CD_IN_K + base, v, e);
+    if (threadIdx.x == 0) a.exp[t] = e;
 }
 
 /* waveform row t: bias + the sum over the output convolution's taps k of tap k's columns of product row src(t, k),
@@ -392,8 +392,8 @@ vt_codec_wave_kernel(float *__restrict__ out, const float *__restrict__ planes, 
 
 /* ---- device state -------------------------------------------------------------------------- */
 
-/* A product's weights in fragment order and the factors of its columns */
-struct cd_matrix { uint16_t *wf; float *inv; int n, k; };
+/* A product's weights in fragment order and the exponents of its columns */
+struct cd_matrix { uint16_t *wf; int *exp; int n, k; };
 
 struct cd_layer_dev {
     cd_matrix wqkv, wo, w13, w2;
@@ -422,8 +422,9 @@ static void cd_free_ptr(float **p) { if (*p) (void)hipFree(*p); *p = NULL; }
 
 static void cd_free_matrix(cd_matrix *m) {
     if (m->wf) (void)hipFree(m->wf);
-    cd_free_ptr(&m->inv);
+    if (m->exp) (void)hipFree(m->exp);
     m->wf = NULL;
+    m->exp = NULL;
 }
 
 void vt_codec_free(void) {
@@ -478,8 +479,8 @@ static int cd_matrix_from(cd_matrix *m, float *d, int n, int k) {
     int ok = d != NULL;
     m->n = n; m->k = k;
     ok = ok && (m->wf = (uint16_t *)vt_dev_alloc((size_t)n * k * 2 * sizeof(uint16_t))) != NULL;
-    ok = ok && (m->inv = (float *)vt_dev_alloc((size_t)n * sizeof(float))) != NULL;
-    ok = ok && vt_codec_weight_layout(m->wf, m->inv, d, n, k) == 0;
+    ok = ok && (m->exp = (int *)vt_dev_alloc((size_t)n * sizeof(int))) != NULL;
+    ok = ok && vt_codec_weight_layout(m->wf, m->exp, d, n, k) == 0;
     if (d) (void)hipFree(d);
     return ok;
 }
@@ -633,7 +634,7 @@ static int cd_reserve(int n_frames) {
     g_cd.qkv = (float *)(g_cd.work + at[1]);
     g_cd.part = (float *)(g_cd.work + at[2]);
     g_cd.wave = (float *)(g_cd.work + at[3]);
-    g_cd.planes = cd_planes{(uint16_t *)(g_cd.work + at[4]), (uint16_t *)(g_cd.work + at[5]), (float *)(g_cd.work + at[6])};
+    g_cd.planes = cd_planes{(uint16_t *)(g_cd.work + at[4]), (uint16_t *)(g_cd.work + at[5]), (int *)(g_cd.work + at[6])};
     g_cd.codes = (int *)(g_cd.work + at[7]);
     return 0;
 }
@@ -641,7 +642,7 @@ static int cd_reserve(int n_frames) {
 /* the product of the rows in g_cd.planes with w -> g_cd.part, row pitch w.n, planes M * w.n floats apart */
 static vt_gemm_plan cd_gemm(int M, const cd_matrix &w) {
     const vt_gemm_plan pl = cd_plan(M, w);
-    vt_launch_codec_gemm(g_cd.part, w.n, (size_t)M * w.n, g_cd.planes.hi, g_cd.planes.lo, g_cd.planes.inv, w.wf, w.inv, M, w.n, w.k, pl);
+    vt_launch_codec_gemm(g_cd.part, w.n, (size_t)M * w.n, g_cd.planes.hi, g_cd.planes.lo, g_cd.planes.exp, w.wf, w.exp, M, w.n, w.k, pl);
     return pl;
 }
 
@@ -752,9 +753,9 @@ __global__ void __launch_bounds__(256) vt_codec_probe_planes_kernel(cd_planes p,
     __shared__ float red[4];
     float m = 0.f;
     for (int c = threadIdx.x * 4; c < k; c += 1024) m = fmaxf(m, cd_max4(*(const f32x4 *)(x + (size_t)blockIdx.x * k + c)));
-    const float s = vt_f16_scale(cd_block_max(m, red));
-    for (int c = threadIdx.x * 4; c < k; c += 1024) cd_put4(p, (size_t)blockIdx.x * k + c, *(const f32x4 *)(x + (size_t)blockIdx.x * k + c), s);
-    if (threadIdx.x == 0) p.inv[blockIdx.x] = 1.0f / s;
+    const int e = vt_f16_exp(cd_block_max(m, red));
+    for (int c = threadIdx.x * 4; c < k; c += 1024) cd_put4(p, (size_t)blockIdx.x * k + c, *(const f32x4 *)(x + (size_t)blockIdx.x * k + c), e);
+    if (threadIdx.x == 0) p.exp[blockIdx.x] = e;
 }
 
 void vt_codec_probe_fill(const float *x, int k) {

@@ -16,8 +16,8 @@
 
 /* ---- weights: row-major fp32 [N, K] -> fragment order, two fp16 planes --------------------------------------- */
 
-/* col_scale[n] = 2^-e, where row n is stored times 2^e */
-__global__ void __launch_bounds__(256) vt_codec_weight_scale_kernel(float *col_scale, const float *W, int K) {
+/* row n is stored times 2^col_exp[n] */
+__global__ void __launch_bounds__(256) vt_codec_weight_exp_kernel(int *col_exp, const float *W, int K) {
     __shared__ float red[4];
     const size_t n = blockIdx.x;
     float m = 0.f;
@@ -25,20 +25,19 @@ __global__ void __launch_bounds__(256) vt_codec_weight_scale_kernel(float *col_s
     for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
     __syncthreads();
-    if (threadIdx.x == 0) col_scale[n] = 1.0f / vt_f16_scale(fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])));
+    if (threadIdx.x == 0) col_exp[n] = vt_f16_exp(fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])));
 }
 
 /* 16-byte slot (((n/32 * K/64 + ks) * 2 + plane) * 4 + j) * 64 + l holds elements 64 ks + 32 (l/32) + 8 j .. + 8 of row
  * 32 (n/32) + l % 32 */
-__global__ void vt_codec_weight_layout_kernel(u32x4 *out, const float *W, const float *col_scale, size_t n_slots, int K) {
+__global__ void vt_codec_weight_layout_kernel(u32x4 *out, const float *W, const int *col_exp, size_t n_slots, int K) {
     const int ksteps = K / 64;
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n_slots; i += (size_t)gridDim.x * blockDim.x) {
         const int l = (int)(i & 63), j = (int)((i >> 6) & 3);
         const size_t blk = i >> 8, n = blk / ksteps * 32 + (l & 31);
         const int ks = (int)(blk % ksteps);
-        const float s = 1.0f / col_scale[n];
         const f32x4 *p = reinterpret_cast<const f32x4 *>(W + n * K + 64 * ks + 32 * (l >> 5) + 8 * j);
-        const f32x4 a = p[0] * s, b = p[1] * s;
+        const f32x4 a = vt_ldexp4(p[0], col_exp[n]), b = vt_ldexp4(p[1], col_exp[n]);
         u32x2 h0, l0, h1, l1;
         vt_split_f16x4(a, h0, l0);
         vt_split_f16x4(b, h1, l1);
@@ -47,12 +46,12 @@ __global__ void vt_codec_weight_layout_kernel(u32x4 *out, const float *W, const 
     }
 }
 
-int vt_codec_weight_layout(uint16_t *d_Wf, float *d_col_scale, const float *d_W, int N, int K) {
+int vt_codec_weight_layout(uint16_t *d_Wf, int *d_col_exp, const float *d_W, int N, int K) {
     if (vt_check(hipStreamSynchronize(NULL), "codec weight copy")) return -1;      /* d_W may have been copied from device memory */
-    hipLaunchKernelGGL(vt_codec_weight_scale_kernel, dim3(N), dim3(256), 0, g_vt.stream, d_col_scale, d_W, K);
+    hipLaunchKernelGGL(vt_codec_weight_exp_kernel, dim3(N), dim3(256), 0, g_vt.stream, d_col_exp, d_W, K);
     const size_t n_slots = (size_t)N * K / 8;
     hipLaunchKernelGGL(vt_codec_weight_layout_kernel, dim3((unsigned)((n_slots + 255) / 256 > 8192 ? 8192 : (n_slots + 255) / 256)), dim3(256), 0, g_vt.stream,
-                       (u32x4 *)d_Wf, d_W, d_col_scale, n_slots, K);
+                       (u32x4 *)d_Wf, d_W, d_col_exp, n_slots, K);
     return vt_check(hipGetLastError(), "codec weight layout") || vt_check(hipStreamSynchronize(g_vt.stream), "codec weight layout") ? -1 : 0;
 }
 
@@ -84,12 +83,12 @@ static void cg_wide(const gw_list &list, const uint16_t *d_hi, const uint16_t *d
     hipLaunchKernelGGL((vt_gemm_wide_kernel<gm_f16x2, MB, CW>), dim3(items < g_vt.n_cu ? items : g_vt.n_cu), dim3(256), LDS, g_vt.stream, list, d_hi, d_lo, M, K);
 }
 
-void vt_launch_codec_gemm(float *d_C, int ldc, size_t plane_stride, const uint16_t *d_hi, const uint16_t *d_lo, const float *d_row_scale,
-                          const uint16_t *d_Wf, const float *d_col_scale, int M, int N, int K, const vt_gemm_plan &pl) {
+void vt_launch_codec_gemm(float *d_C, int ldc, size_t plane_stride, const uint16_t *d_hi, const uint16_t *d_lo, const int *d_row_exp,
+                          const uint16_t *d_Wf, const int *d_col_exp, int M, int N, int K, const vt_gemm_plan &pl) {
     if (pl.mb == 0) {
         gr_plan plan = {};
         plan.n_parts = 1;
-        plan.part[0] = gr_part{d_C, d_Wf, plane_stride, ldc, N / GR_TN, pl.cuts, NULL, NULL, 0, d_row_scale, d_col_scale};
+        plan.part[0] = gr_part{d_C, d_Wf, plane_stride, ldc, N / GR_TN, pl.cuts, NULL, NULL, 0, d_row_exp, d_col_exp};
         const int items = plan.part[0].n_tiles * pl.cuts, grid = items < g_vt.n_cu ? items : g_vt.n_cu;
         static void (*const launch[4])(const gr_plan &, int, const uint16_t *, const uint16_t *, int, int) = {cg_rows<2>, cg_rows<4>, cg_rows<6>, cg_rows<8>};
         launch[(M + 15) / 16 - 1](plan, grid, d_hi, d_lo, M, K);
@@ -97,9 +96,9 @@ void vt_launch_codec_gemm(float *d_C, int ldc, size_t plane_stride, const uint16
     }
     gw_list list = {};
     list.m_tiles = (M + 32 * pl.mb - 1) / (32 * pl.mb);
-    gw_part whole = {d_C, d_Wf, plane_stride, ldc, pl.col0 / (64 * pl.cw), 1, NULL, NULL, 0, d_row_scale, d_col_scale};
+    gw_part whole = {d_C, d_Wf, plane_stride, ldc, pl.col0 / (64 * pl.cw), 1, NULL, NULL, 0, d_row_exp, d_col_exp};
     gw_part cut = {d_C + pl.col0, d_Wf + (size_t)pl.col0 * K * 2, plane_stride, ldc, (N - pl.col0) / (64 * pl.cw), pl.cuts, NULL, NULL, 0,
-                   d_row_scale, d_col_scale + pl.col0};
+                   d_row_exp, d_col_exp + pl.col0};
     if (whole.n_tiles) list.part[list.n_parts++] = whole;
     if (cut.n_tiles) list.part[list.n_parts++] = cut;
     if (pl.mb == 4 && pl.cw == 4) cg_wide<4, 4>(list, d_hi, d_lo, M, K);

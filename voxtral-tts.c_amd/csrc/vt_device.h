@@ -127,12 +127,15 @@ __device__ __forceinline__ void vt_split_planes4(float a, float b, float c, floa
 }
 
 /* fp32 -> two fp16 planes, for rows scaled by a power of two that brings the largest magnitude to 2^13 .. 2^14
- * (vt_f16_scale of that magnitude): hi = fp16(x), lo = fp16(x - hi), both to nearest even, so that hi + lo is x to
+ * (vt_f16_exp of that magnitude): hi = fp16(x), lo = fp16(x - hi), both to nearest even, so that hi + lo is x to
  * 2^-24 of itself where lo is normal and to 2^-25 absolute where it is not. */
-__device__ __forceinline__ float vt_f16_scale(float largest) {
-    int e;
-    (void)frexpf(largest, &e);                               /* largest = f 2^e, f in [0.5, 1) */
-    return largest > 0.f ? ldexpf(1.0f, 14 - (e < -100 ? -100 : e > 110 ? 110 : e)) : 1.0f;
+/* An exponent and not a factor: 2^14 / largest and its inverse need not be floats, and no product of two factors is
+ * made on the way back. */
+__device__ __forceinline__ int vt_f16_exp(float largest) {
+    return largest > 0.f ? 14 - __builtin_amdgcn_frexp_expf(largest) : 0;      /* largest = f 2^e, f in [0.5, 1) */
+}
+__device__ __forceinline__ f32x4 vt_ldexp4(const f32x4 &v, int e) {
+    return f32x4{__builtin_amdgcn_ldexpf(v.x, e), __builtin_amdgcn_ldexpf(v.y, e), __builtin_amdgcn_ldexpf(v.z, e), __builtin_amdgcn_ldexpf(v.w, e)};
 }
 typedef _Float16 vt_f16x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ void vt_split_f16x2(float a, float b, unsigned &hi, unsigned &lo) {

@@ -24,8 +24,8 @@ struct gm_bf16 {
     }
 };
 /* The codec: fp32 weights and activations as two fp16 planes each, rows of both scaled by powers of two so that the
- * planes stay in range; x w = hi hi + hi lo + lo hi (lo lo is below 2^-24 of the product).  The factors that
- * undo the scaling, one per row and one per column, are applied to the sums. */
+ * planes stay in range; x w = hi hi + hi lo + lo hi (lo lo is below 2^-24 of the product).  The scaling is
+ * undone on the sums by its exponents, one per row and one per column. */
 struct gm_f16x2 {
     static constexpr int WP = 2;
     static constexpr bool SCALED = true;
@@ -64,15 +64,15 @@ __device__ __forceinline__ void gm_multiply(f32x16 (&acc)[MB][2], const gm_frags
 /* rows row0 .. + 3 of one column (q0) and of the column 32 further on (q1); C points at row 0 of the column */
 template <class T>
 __device__ __forceinline__ void gm_store_quad(float *C, int ldc, int row0, int M, const f32x4 &q0, const f32x4 &q1,
-                                              const float *row_scale, const float *col_scale) {
+                                              const int *row_exp, const int *col_exp) {
     if constexpr (T::SCALED) {
-        const float s0 = col_scale[0], s1 = col_scale[32];
+        const int e0 = col_exp[0], e1 = col_exp[32];
 #pragma unroll
         for (int v = 0; v < 4; v++)
             if (row0 + v < M) {
-                const float r = row_scale[row0 + v];
-                C[(size_t)(row0 + v) * ldc] = q0[v] * s0 * r;
-                C[(size_t)(row0 + v) * ldc + 32] = q1[v] * s1 * r;
+                const int e = row_exp[row0 + v];
+                C[(size_t)(row0 + v) * ldc] = __builtin_amdgcn_ldexpf(q0[v], -e0 - e);
+                C[(size_t)(row0 + v) * ldc + 32] = __builtin_amdgcn_ldexpf(q1[v], -e1 - e);
             }
     } else {
 #pragma unroll
@@ -122,7 +122,7 @@ struct gw_part {
      * (hi, lo) planes of SiLU(gate) * up, row pitch ldh */
     uint16_t *h_hi, *h_lo;
     int ldh;
-    const float *row_scale, *col_scale;   /* T::SCALED: factors of the rows and of the set's columns */
+    const int *row_exp, *col_exp;         /* T::SCALED: exponents of the rows and of the set's columns */
 };
 struct gw_list { gw_part part[2]; int n_parts, m_tiles; };
 
@@ -311,7 +311,7 @@ vt_gemm_wide_kernel(gw_list list, const uint16_t *Ahi, const uint16_t *Alo, int 
                 }
         } else {
             const int col = it.nt * TN + 64 * cw + c;
-            gm_store_quad<T>(P.C + (size_t)it.sp * P.plane_stride + col, P.ldc, row0, M, q0, q1, P.row_scale, P.col_scale + col);
+            gm_store_quad<T>(P.C + (size_t)it.sp * P.plane_stride + col, P.ldc, row0, M, q0, q1, P.row_exp, P.col_exp + col);
         }
     };
     auto quad = [&](int a, int b, int vq) { return f32x4{acc[a][b][4 * vq], acc[a][b][4 * vq + 1], acc[a][b][4 * vq + 2], acc[a][b][4 * vq + 3]}; };
@@ -407,7 +407,7 @@ struct gr_part {
     int ldc, n_tiles, splits;
     uint16_t *h_hi, *h_lo;                /* gate|up (paired column order): planes of SiLU(gate) * up instead of C */
     int ldh;
-    const float *row_scale, *col_scale;   /* T::SCALED: factors of the rows and of the part's columns */
+    const int *row_exp, *col_exp;         /* T::SCALED: exponents of the rows and of the part's columns */
 };
 struct gr_plan { gr_part part[2]; int n_parts; };
 
@@ -581,7 +581,7 @@ vt_gemm_rows_kernel(gr_plan plan, const uint16_t *Ahi, const uint16_t *Alo, int 
                     }
             } else {
                 const int col = it.nt * GR_TN + c;
-                gm_store_quad<T>(P.C + (size_t)it.sp * P.plane_stride + col, P.ldc, row0, M, s[0], s[1], P.row_scale, P.col_scale + col);
+                gm_store_quad<T>(P.C + (size_t)it.sp * P.plane_stride + col, P.ldc, row0, M, s[0], s[1], P.row_exp, P.col_exp + col);
             }
         }
     };
