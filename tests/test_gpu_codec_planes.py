@@ -1,7 +1,7 @@
 """The codec's products run on two fp16 planes per fp32 operand, each row scaled by a power of two, on tiles and K
 cuts that follow the row count.  Frame counts whose four stages (1, 2, 4, 8 rows a frame) fall on the edges of the
 tiles (16, 32, 48, 64 rows of the few-row kernel, then 96- and 128-row tiles), and magnitudes far outside the
-range of fp16.  The bound: an operand is carried to 2^-24, a product's left-out term is below 2^-24 of it, and the
+range of fp16.  The bound: an operand is carried to 2^-23, a product's left-out term is at most 2^-22 of it, and the
 sums are fp32 as on the CPU, whose own sequential sums differ from these by a few 1e-6 of the waveform's rms
 (measured 4e-6 in l2, 2e-5 at most per sample); four times that."""
 import ctypes as C

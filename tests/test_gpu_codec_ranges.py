@@ -1,5 +1,6 @@
 """The codec's products hold an fp32 operand as two fp16 planes and an exponent per row.  What fp32 arithmetic takes in
-its stride: rows whose values stand near either end of fp32."""
+its stride: rows whose values stand near either end of fp32, and rows of values that are far apart, whose small ones
+still carry the result because the large ones meet zeros."""
 import ctypes as C
 
 import numpy as np
@@ -36,4 +37,20 @@ def test_rows_near_the_ends_of_fp32():
     for conv, f in ((hc.stage_convs[0], 2.0 ** 113), (hc.stage_convs[1], 2.0 ** -113)):
         conv.weight *= np.float32(f)
     hc.stage_convs[0].bias *= np.float32(2.0 ** 113)
+    decode_both(hc, (5, 40))
+
+
+@pytest.mark.parametrize("log2", [20, 24])
+def test_rows_of_values_far_apart(log2):
+    """One channel of the normalised rows 2^20 and 2^24 times the others, which no weight reads, and weights as far from
+    the rest of their rows at a channel that is zero: the result is that of the small values, whose 24 bits count."""
+    f = np.float32(2.0 ** log2)
+    hc = K.HostCodec(11, distinct_layers=1)
+    l = hc.layers[0]
+    for norm, weights in ((l.attention_norm, (l.wq, l.wk, l.wv)), (l.ffn_norm, (l.w1, l.w3))):
+        norm[5] = f
+        norm[6] = 0
+        for w in weights:
+            w[:, 5] = 0
+            w[:, 6] = f * np.abs(w).max(axis=1)
     decode_both(hc, (5, 40))

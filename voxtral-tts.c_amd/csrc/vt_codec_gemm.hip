@@ -1,14 +1,20 @@
 /*
  * vt_codec_gemm.hip - the codec decoder's products (fp32 weights, fp32 activations) on the fp16 matrix cores.
  *
- * Every fp32 operand is carried as two fp16 planes, hi = fp16(s x) and lo = fp16(s x - hi), with a power of two s
- * per row that brings the row's largest magnitude to 2^13 .. 2^14: hi + lo then holds s x to 2^-24 of itself (2^-38
- * of the row's largest where lo is subnormal), as good as fp32 does.  A product is hi hi + hi lo + lo hi, three
- * matrix instructions on the same fp32 sums; the lo lo term left out is below 2^-24 of the product, the size of
- * the rounding of every single addition.  Three fp16 instructions do 16 times the work of an fp32 one each, so the
+ * Every fp32 operand is carried as two fp16 planes, hi = fp16(s x) and lo = fp16(2^6 (s x - hi)), with a power of two s
+ * per row that brings the row's largest magnitude to 2^14 .. 2^15: hi + 2^-6 lo then holds s x to 2^-23 of itself down
+ * to 2^-22 of the row's largest, and to 2^-46 of that below.  A product is hi hi + hi lo + lo hi, three matrix
+ * instructions on the same fp32 sums; the lo lo term left out is at most 2^-22 of the product.  An operand so has up to
+ * one bit less than fp32, and the sums have fewer roundings (one per instruction, not one per product): where they
+ * matter more, the result is closer to 64 bits than with fp32 instructions.
+ * Three fp16 instructions do 16 times the work of an fp32 one each, so the
  * same product takes 3/16 of the matrix-core time; what it then runs into is the card's power limit.
  * Measured against float64, error of a row over its l2 norm: 1.4e-7 .. 3.6e-7 (K 1024 .. 7168, rows and elements of
  * log-normal magnitude) where a plain fp32 product has 2.7e-7 .. 1.1e-6: what remains is the fp32 sums.
+ * The 2^6 is for rows with values far apart whose large ones meet zeros.  Error of the operands and the left-out term
+ * alone, K = 1024, one channel 1 / 2^16 / 2^20 / 2^24 times the others: 0.75 / 0.75 / 0.77 / 2.4e-7 of the result, and
+ * 0.75 / 1.2 / 17 / 209e-7 without it; fp32 sums in order have 5.7e-7.  hi times 2^-6, which it takes, costs 0.7 / 1.6 / 1.5 %
+ * of a decode of 21 / 212 / 1003 frames.
  * Rates, TFLOP/s of the product itself (v_mfma_f32_32x32x2f32 in 128 x 128 tiles before: 75 .. 105): gate|up
  * 8192 x 1024 at 212 / 848 / 1696 / 8024 rows 150 / 287 / 290 / 335, down 1024 x 4096 111 / 227 / 282 / 336.
  */

@@ -126,13 +126,15 @@ __device__ __forceinline__ void vt_split_planes4(float a, float b, float c, floa
     lo = u32x2{l0, l1};
 }
 
-/* fp32 -> two fp16 planes, for rows scaled by a power of two that brings the largest magnitude to 2^13 .. 2^14
- * (vt_f16_exp of that magnitude): hi = fp16(x), lo = fp16(x - hi), both to nearest even, so that hi + lo is x to
- * 2^-24 of itself where lo is normal and to 2^-25 absolute where it is not. */
-/* An exponent and not a factor: 2^14 / largest and its inverse need not be floats, and no product of two factors is
+/* fp32 -> two fp16 planes, for rows times 2^vt_f16_exp(their largest magnitude), which is then 2^14 .. 2^15:
+ * hi = fp16(x), lo = fp16(2^VT_F16_LO_EXP (x - hi)), both to nearest even, so that hi + 2^-VT_F16_LO_EXP lo is x to 2^-23
+ * of itself where both are normal, i.e. down to 2^-22 of the row's largest (without the factor: to 2^-16 of it), and to
+ * 2^-46 of the largest below.
+ * An exponent and not a factor: 2^15 / largest and its inverse need not be floats, and no product of two factors is
  * made on the way back. */
+#define VT_F16_LO_EXP 6
 __device__ __forceinline__ int vt_f16_exp(float largest) {
-    return largest > 0.f ? 14 - __builtin_amdgcn_frexp_expf(largest) : 0;      /* largest = f 2^e, f in [0.5, 1) */
+    return largest > 0.f ? 15 - __builtin_amdgcn_frexp_expf(largest) : 0;      /* largest = f 2^e, f in [0.5, 1) */
 }
 __device__ __forceinline__ f32x4 vt_ldexp4(const f32x4 &v, int e) {
     return f32x4{__builtin_amdgcn_ldexpf(v.x, e), __builtin_amdgcn_ldexpf(v.y, e), __builtin_amdgcn_ldexpf(v.z, e), __builtin_amdgcn_ldexpf(v.w, e)};
@@ -140,7 +142,8 @@ __device__ __forceinline__ f32x4 vt_ldexp4(const f32x4 &v, int e) {
 typedef _Float16 vt_f16x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ void vt_split_f16x2(float a, float b, unsigned &hi, unsigned &lo) {
     const vt_f16x2 h = {(_Float16)a, (_Float16)b};
-    const vt_f16x2 l = {(_Float16)__fsub_rn(a, (float)h.x), (_Float16)__fsub_rn(b, (float)h.y)};
+    const float up = (float)(1 << VT_F16_LO_EXP);
+    const vt_f16x2 l = {(_Float16)(__fsub_rn(a, (float)h.x) * up), (_Float16)(__fsub_rn(b, (float)h.y) * up)};
     hi = __builtin_bit_cast(unsigned, h);
     lo = __builtin_bit_cast(unsigned, l);
 }

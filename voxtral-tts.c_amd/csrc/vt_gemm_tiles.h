@@ -23,9 +23,12 @@ struct gm_bf16 {
         return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(gm_bf16x8, x), __builtin_bit_cast(gm_bf16x8, w), c, 0, 0, 0);
     }
 };
-/* The codec: fp32 weights and activations as two fp16 planes each, rows of both scaled by powers of two so that the
- * planes stay in range; x w = hi hi + hi lo + lo hi (lo lo is below 2^-24 of the product).  The scaling is
- * undone on the sums by its exponents, one per row and one per column. */
+/* The codec: fp32 weights and activations as two fp16 planes each (vt_split_f16x2), rows of both scaled by powers of
+ * two so that the planes stay in range; x w = hi hi + hi lo + lo hi (lo lo is at most 2^-22 of the product).  The lo
+ * planes are kept 2^6 larger, for small values in rows with a large one, and meet hi times 2^-6, made in registers
+ * beside the matrix instructions.  (Dealt out between them by number, as the memory instructions are, it costs 3.5 %
+ * of a decode instead of 2; in front of them 2.5.)  The scaling is undone on the sums by its exponents, one per row
+ * and one per column. */
 struct gm_f16x2 {
     static constexpr int WP = 2;
     static constexpr bool SCALED = true;
@@ -42,23 +45,40 @@ __device__ __forceinline__ u32x4 gm_ldb(__amdgpu_buffer_rsrc_t r, int voff, int 
     return __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0);
 }
 
-/* one slice: the small products first; 2 MB independent sums between two products into the same one */
+__device__ __forceinline__ u32x4 gm_down(const u32x4 &hi) {
+    return __builtin_bit_cast(u32x4, __builtin_bit_cast(gm_f16x8, hi) * (_Float16)(1.0f / (1 << VT_F16_LO_EXP)));
+}
+
+/* one slice; 2 MB independent sums between two products into the same one */
 template <class T, int MB>
 __device__ __forceinline__ void gm_multiply(f32x16 (&acc)[MB][2], const gm_frags<MB> &f, const gm_weights<T::WP> &w, int ks) {
     if constexpr (T::WP == 2) {
 #pragma unroll
         for (int a = 0; a < MB; a++)
 #pragma unroll
-            for (int b = 0; b < 2; b++) acc[a][b] = T::mfma(f.hi[a], w.v[1][b][ks], acc[a][b]);
+            for (int b = 0; b < 2; b++) acc[a][b] = T::mfma(f.hi[a], w.v[0][b][ks], acc[a][b]);
+        const u32x4 wd[2] = {gm_down(w.v[0][0][ks]), gm_down(w.v[0][1][ks])};
+#pragma unroll
+        for (int a = 0; a < MB; a++)
+#pragma unroll
+            for (int b = 0; b < 2; b++) acc[a][b] = T::mfma(f.lo[a], wd[b], acc[a][b]);
+#pragma unroll
+        for (int a = 0; a < MB; a++) {
+            const u32x4 d = gm_down(f.hi[a]);
+#pragma unroll
+            for (int b = 0; b < 2; b++) acc[a][b] = T::mfma(d, w.v[1][b][ks], acc[a][b]);
+        }
+    } else {
+        /* the small products first */
+#pragma unroll
+        for (int a = 0; a < MB; a++)
+#pragma unroll
+            for (int b = 0; b < 2; b++) acc[a][b] = T::mfma(f.lo[a], w.v[0][b][ks], acc[a][b]);
+#pragma unroll
+        for (int a = 0; a < MB; a++)
+#pragma unroll
+            for (int b = 0; b < 2; b++) acc[a][b] = T::mfma(f.hi[a], w.v[0][b][ks], acc[a][b]);
     }
-#pragma unroll
-    for (int a = 0; a < MB; a++)
-#pragma unroll
-        for (int b = 0; b < 2; b++) acc[a][b] = T::mfma(f.lo[a], w.v[0][b][ks], acc[a][b]);
-#pragma unroll
-    for (int a = 0; a < MB; a++)
-#pragma unroll
-        for (int b = 0; b < 2; b++) acc[a][b] = T::mfma(f.hi[a], w.v[0][b][ks], acc[a][b]);
 }
 
 /* rows row0 .. + 3 of one column (q0) and of the column 32 further on (q1); C points at row 0 of the column */
