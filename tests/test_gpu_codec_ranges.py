@@ -1,10 +1,11 @@
 """The codec's products hold an fp32 operand as two fp16 planes and an exponent per row.  What fp32 arithmetic takes in
 its stride: rows whose values stand near either end of fp32, and rows of values that are far apart, whose small ones
-still carry the result because the large ones meet zeros."""
+still carry the result because the large ones meet zeros.  And the memory that a decode takes."""
 import ctypes as C
 
 import numpy as np
 import pytest
+import torch
 
 import codecsupport as K
 import hipsupport as H
@@ -54,3 +55,27 @@ def test_rows_of_values_far_apart(log2):
             w[:, 5] = 0
             w[:, 6] = f * np.abs(w).max(axis=1)
     decode_both(hc, (5, 40))
+
+
+def test_work_area_follows_the_frame_count():
+    """A product's partial planes hold the cut columns only.  527 frames, whose last gate|up product has 256 of 8192
+    columns in 6 cuts, need the 138 MB of that product, a quarter and 17 MB more for cut planes, and the 142 MB of the
+    other buffers; 20 MB are left for what the runtime takes.  A decode then finds room where a longer one did."""
+    hip = H.Hip(kv_max=8)
+    try:
+        cs = K.HostCodec(5, distinct_layers=1).struct()
+        assert hip.lib.tts_hip_upload_codec_weights(C.addressof(cs)) == 0, hip.lib.tts_hip_last_error()
+
+        def used_by(n):
+            before = torch.cuda.mem_get_info()[0]
+            hip_decode(hip, K.random_codes(n, n))
+            return before - torch.cuda.mem_get_info()[0]
+
+        used_by(9)                     # the runtime takes some memory of its own with the first launches of a kernel
+        used_by(65)
+        assert used_by(527) <= 352e6
+        used_by(612)
+        for n in (527, 288, 575):
+            assert used_by(n) <= 20e6, n
+    finally:
+        hip.close()

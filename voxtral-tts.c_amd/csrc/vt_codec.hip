@@ -76,10 +76,18 @@ __device__ __forceinline__ void cd_put4(const cd_planes &p, size_t at, const f32
     *(u32x2 *)(p.lo + at) = l;
 }
 
-/* A product's result at one place: `n` partial planes, in order.  Up to C of them, all requested before the first is
- * used (one after the other they cost a memory latency each); those that do not exist repeat plane 0. */
+/* A product's result as vt_launch_codec_gemm leaves it: the columns below col0, [rows, col0], and behind them `cuts`
+ * partial planes of the others, [rows, n - col0] */
+struct cd_product { const float *p; int rows, n, col0, cuts; };
+
+/* Four columns of a row, partial planes in order.  Up to C of them, all requested before the first is used (one after
+ * the other they cost a memory latency each); those that do not exist repeat plane 0. */
 template <int C>
-__device__ __forceinline__ f32x4 cd_sum(const float *p, int n, size_t stride) {
+__device__ __forceinline__ f32x4 cd_sum(const cd_product &r, int row, int col) {
+    const bool cut = col >= r.col0;
+    const int pitch = cut ? r.n - r.col0 : r.col0, n = cut ? r.cuts : 1;
+    const size_t stride = (size_t)r.rows * pitch;
+    const float *p = r.p + (cut ? (size_t)r.rows * r.col0 : 0) + (size_t)row * pitch + (cut ? col - r.col0 : col);
     f32x4 q[C];
 #pragma unroll
     for (int s = 0; s < C; s++) q[s] = *(const f32x4 *)(p + (s < n ? s : 0) * stride);
@@ -93,12 +101,11 @@ __device__ __forceinline__ f32x4 cd_sum(const float *p, int n, size_t stride) {
 /* One row of 1024: val = the product's result (+ bias) (* scale) (+ residual).  With a norm weight val -> x_out and
  * val * rsqrt(mean(val^2) + eps) * norm_w (tts_rms_norm, voxtral_tts_kernels.c:333-349) as planes; without one the
  * rows go into a convolution next, val itself as planes.  UP: rows of the upsampling product, row 2 j + p is the sum of
- * phase p's columns of row j and, for the other tap, of row j - 1.  The columns from col0 on are cut. */
+ * phase p's columns of row j and, for the other tap, of row j - 1. */
 template <int C, bool UP>
 __global__ void __launch_bounds__(256)
-vt_codec_row_kernel(float *x_out, cd_planes xn, const float *x_in, const float *__restrict__ planes, int col0, int cuts,
-                    size_t plane_stride, const float *__restrict__ bias, const float *__restrict__ scale,
-                    const float *__restrict__ norm_w, float eps) {
+vt_codec_row_kernel(float *x_out, cd_planes xn, const float *x_in, cd_product in, const float *__restrict__ bias,
+                    const float *__restrict__ scale, const float *__restrict__ norm_w, float eps) {
     __shared__ float red[4];
     const int row = blockIdx.x, c = threadIdx.x * 4;
     const size_t at = (size_t)row * CD_DIM + c;
@@ -107,10 +114,10 @@ vt_codec_row_kernel(float *x_out, cd_planes xn, const float *x_in, const float *
     f32x4 v;
     if (UP) {
         const int j = row >> 1, col = (row & 1) * CD_DIM + c;
-        v = cd_sum<C>(planes + (size_t)j * CD_UP_N + col, col < col0 ? 1 : cuts, plane_stride);
-        if (j > 0) v += cd_sum<C>(planes + (size_t)(j - 1) * CD_UP_N + 2 * CD_DIM + col, 2 * CD_DIM + col < col0 ? 1 : cuts, plane_stride);
+        v = cd_sum<C>(in, j, col);
+        if (j > 0) v += cd_sum<C>(in, j - 1, 2 * CD_DIM + col);
     } else {
-        v = cd_sum<C>(planes + at, c < col0 ? 1 : cuts, plane_stride);
+        v = cd_sum<C>(in, row, c);
     }
     if (bias) v += *(const f32x4 *)(bias + c);
     if (scale) v *= *(const f32x4 *)(scale + c);
@@ -130,14 +137,13 @@ vt_codec_row_kernel(float *x_out, cd_planes xn, const float *x_in, const float *
  * voxtral_tts_kernels.c:351-355, eps 1e-6) when the layer has those weights. */
 template <int C>
 __global__ void __launch_bounds__(256)
-vt_codec_qkv_kernel(float *__restrict__ qkv, const float *__restrict__ planes, int col0, int cuts, size_t plane_stride,
-                    const float *__restrict__ q_norm, const float *__restrict__ k_norm) {
+vt_codec_qkv_kernel(float *__restrict__ qkv, cd_product in, const float *__restrict__ q_norm, const float *__restrict__ k_norm) {
     __shared__ float red[4];
     const int row = blockIdx.x, c = threadIdx.x * 4;
     const size_t at = (size_t)row * (3 * CD_DIM) + c;
     f32x4 v[3];
 #pragma unroll
-    for (int part = 0; part < 3; part++) v[part] = cd_sum<C>(planes + at + part * CD_DIM, part * CD_DIM + c < col0 ? 1 : cuts, plane_stride);
+    for (int part = 0; part < 3; part++) v[part] = cd_sum<C>(in, row, part * CD_DIM + c);
 #pragma unroll
     for (int part = 0; part < 3; part++) {
         const float *nw = part == 0 ? q_norm : part == 1 ? k_norm : nullptr;
@@ -153,7 +159,7 @@ vt_codec_qkv_kernel(float *__restrict__ qkv, const float *__restrict__ planes, i
 /* gate|up [T, 8192] -> h = silu(gate) * up [T, 4096] (tts_silu, tts_mul_inplace) as planes; one workgroup per row */
 template <int C>
 __global__ void __launch_bounds__(256)
-vt_codec_swiglu_kernel(cd_planes h, const float *__restrict__ gu, int col0, int cuts, size_t plane_stride) {
+vt_codec_swiglu_kernel(cd_planes h, cd_product gu) {
     __shared__ float red[4];
     const int row = blockIdx.x;
     f32x4 v[CD_HID / 1024];
@@ -161,8 +167,7 @@ vt_codec_swiglu_kernel(cd_planes h, const float *__restrict__ gu, int col0, int 
 #pragma unroll
     for (int j = 0; j < CD_HID / 1024; j++) {
         const int c = 4 * ((int)threadIdx.x + 256 * j);
-        const float *p = gu + (size_t)row * (2 * CD_HID) + c;
-        const f32x4 g = cd_sum<C>(p, c < col0 ? 1 : cuts, plane_stride), u = cd_sum<C>(p + CD_HID, CD_HID + c < col0 ? 1 : cuts, plane_stride);
+        const f32x4 g = cd_sum<C>(gu, row, c), u = cd_sum<C>(gu, row, CD_HID + c);
         v[j] = vt_silu_mul4(g, u);
         m = fmaxf(m, cd_max4(v[j]));
     }
@@ -373,8 +378,7 @@ vt_codec_embed_kernel(cd_planes a, const int *__restrict__ codes, const float *_
  * stride 1, left reflection as above */
 template <int C>
 __global__ void __launch_bounds__(64)
-vt_codec_wave_kernel(float *__restrict__ out, const float *__restrict__ planes, int col0, int cuts, size_t plane_stride,
-                     int T, const float *__restrict__ bias) {
+vt_codec_wave_kernel(float *__restrict__ out, cd_product in, const float *__restrict__ bias) {
     const int t = blockIdx.x, c = threadIdx.x * 4;
     if (c >= CD_PATCH) return;
     f32x4 v = {0.f, 0.f, 0.f, 0.f};
@@ -382,9 +386,8 @@ vt_codec_wave_kernel(float *__restrict__ out, const float *__restrict__ planes, 
     for (int k = 0; k < CD_OUT_TAPS; k++) {
         int src = t + k - (CD_OUT_TAPS - 1);
         if (src < 0) src = -src;
-        const int col = k * CD_OUT_PITCH + c;
-        const f32x4 p = cd_sum<C>(planes + (size_t)(src < T ? src : 0) * CD_OUT_N + col, col < col0 ? 1 : cuts, plane_stride);
-        if (src < T) v += p;
+        const f32x4 p = cd_sum<C>(in, src < in.rows ? src : 0, k * CD_OUT_PITCH + c);
+        if (src < in.rows) v += p;
     }
     if (bias) v += *(const f32x4 *)(bias + c);
     *(f32x4 *)(out + (size_t)t * CD_PATCH + c) = v;
@@ -604,12 +607,19 @@ extern "C" int tts_hip_upload_codec_weights(void *codec_ptr) {
  * upsampling products, output convolution */
 static vt_gemm_plan cd_plan(int M, const cd_matrix &w) { return vt_codec_gemm_plan(M, w.n, w.k); }
 
-/* floats that a product's partial planes take */
-static size_t cd_part_floats(int M, const cd_matrix &w) { return (size_t)M * w.n * cd_plan(M, w).cuts; }
+/* floats that a product's result takes (cd_product) */
+static size_t cd_part_floats(int M, const cd_matrix &w) {
+    const vt_gemm_plan pl = cd_plan(M, w);
+    return (size_t)M * (pl.col0 + (size_t)(w.n - pl.col0) * pl.cuts);
+}
 
 static int cd_reserve(int n_frames) {
     const size_t T = (size_t)n_frames * 8;
-    size_t part = cd_part_floats(n_frames, g_cd.w_in);
+    /* the gate|up product of the last stage and what cut planes add to it on 256 CUs, whatever the row count: a
+     * decode finds room where a longer one did */
+    size_t part = T * (2 * CD_HID + 2 * CD_HID / 4) + ((size_t)4 << 20);
+    const size_t n_in = cd_part_floats(n_frames, g_cd.w_in);
+    part = n_in > part ? n_in : part;
     for (int st = 0; st < 4; st++) {
         const int M = n_frames << st;
         const cd_layer_dev *l = &g_cd.layers[2 * st];
@@ -639,25 +649,25 @@ static int cd_reserve(int n_frames) {
     return 0;
 }
 
-/* the product of the rows in g_cd.planes with w -> g_cd.part, row pitch w.n, planes M * w.n floats apart */
-static vt_gemm_plan cd_gemm(int M, const cd_matrix &w) {
+/* the product of the rows in g_cd.planes with w, in g_cd.part */
+static cd_product cd_gemm(int M, const cd_matrix &w) {
     const vt_gemm_plan pl = cd_plan(M, w);
-    vt_launch_codec_gemm(g_cd.part, w.n, (size_t)M * w.n, g_cd.planes.hi, g_cd.planes.lo, g_cd.planes.exp, w.wf, w.exp, M, w.n, w.k, pl);
-    return pl;
+    vt_launch_codec_gemm(g_cd.part, g_cd.planes.hi, g_cd.planes.lo, g_cd.planes.exp, w.wf, w.exp, M, w.n, w.k, pl);
+    return cd_product{g_cd.part, M, w.n, pl.col0, pl.cuts};
 }
 
 /* CALL(C) with the instance that requests enough planes at once */
 #define CD_BY_CUTS(cuts, CALL) do { if ((cuts) <= 1) { CALL(1); } else if ((cuts) <= 2) { CALL(2); } else if ((cuts) <= 4) { CALL(4); } else { CALL(VT_MAX_CUTS); } } while (0)
 
-/* M product rows (up: of the upsampling product, two rows of 1024 each) -> x (bias or layer scale and residual) and
+/* the rows of a product (up: of the upsampling product, two rows of 1024 each) -> x (bias or layer scale and residual) and
  * planes of its RMSNorm; norm_w NULL: its planes only */
-static void cd_row(const vt_gemm_plan &pl, int M, bool up, const float *x_in, const float *bias, const float *scale, const float *norm_w) {
+static void cd_row(const cd_product &in, bool up, const float *x_in, const float *bias, const float *scale, const float *norm_w) {
 #define CALL(C) \
-    if (up) hipLaunchKernelGGL((vt_codec_row_kernel<C, true>), dim3(2 * M), dim3(256), 0, g_vt.stream, g_cd.x, g_cd.planes, x_in, g_cd.part, \
-                               pl.col0, pl.cuts, (size_t)M * CD_UP_N, bias, scale, norm_w, CD_EPS); \
-    else hipLaunchKernelGGL((vt_codec_row_kernel<C, false>), dim3(M), dim3(256), 0, g_vt.stream, g_cd.x, g_cd.planes, x_in, g_cd.part, \
-                            pl.col0, pl.cuts, (size_t)M * CD_DIM, bias, scale, norm_w, CD_EPS)
-    CD_BY_CUTS(pl.cuts, CALL);
+    if (up) hipLaunchKernelGGL((vt_codec_row_kernel<C, true>), dim3(2 * in.rows), dim3(256), 0, g_vt.stream, g_cd.x, g_cd.planes, x_in, in, bias, \
+                               scale, norm_w, CD_EPS); \
+    else hipLaunchKernelGGL((vt_codec_row_kernel<C, false>), dim3(in.rows), dim3(256), 0, g_vt.stream, g_cd.x, g_cd.planes, x_in, in, bias, \
+                            scale, norm_w, CD_EPS)
+    CD_BY_CUTS(in.cuts, CALL);
 #undef CALL
 }
 
@@ -666,39 +676,38 @@ static int cd_enqueue(const int *d_codes, int n_frames, float *d_samples) {
     int T = n_frames;
     const float scale = 1.0f / sqrtf((float)CD_HEAD_DIM);
     hipLaunchKernelGGL(vt_codec_embed_kernel, dim3(T), dim3(256), 0, g_vt.stream, g_cd.planes, d_codes, g_cd.sem, T);
-    vt_gemm_plan pl = cd_gemm(T, g_cd.w_in);
-    cd_row(pl, T, false, NULL, g_cd.b_in, NULL, g_cd.layers[0].attention_norm);
+    cd_product p = cd_gemm(T, g_cd.w_in);
+    cd_row(p, false, NULL, g_cd.b_in, NULL, g_cd.layers[0].attention_norm);
     for (int li = 0; li < CD_LAYERS; li++) {
         const cd_layer_dev *l = &g_cd.layers[li];
-        pl = cd_gemm(T, l->wqkv);
-#define CALL(C) hipLaunchKernelGGL(vt_codec_qkv_kernel<C>, dim3(T), dim3(256), 0, g_vt.stream, g_cd.qkv, g_cd.part, pl.col0, pl.cuts, \
-                                   (size_t)T * 3 * CD_DIM, l->q_norm, l->k_norm)
-        CD_BY_CUTS(pl.cuts, CALL);
+        p = cd_gemm(T, l->wqkv);
+#define CALL(C) hipLaunchKernelGGL(vt_codec_qkv_kernel<C>, dim3(T), dim3(256), 0, g_vt.stream, g_cd.qkv, p, l->q_norm, l->k_norm)
+        CD_BY_CUTS(p.cuts, CALL);
 #undef CALL
         if (T < CD_ATT_SPLIT_BELOW)
             hipLaunchKernelGGL(vt_codec_attention_split_kernel, dim3(T), dim3(64 * CD_HEADS), 0, g_vt.stream, g_cd.planes, g_cd.qkv, T, l->window, g_cd.slopes, scale);
         else
             hipLaunchKernelGGL(vt_codec_attention_kernel, dim3((T + CD_ATT_TOKENS - 1) / CD_ATT_TOKENS), dim3(64 * CD_HEADS), 0, g_vt.stream, g_cd.planes,
                                g_cd.qkv, T, l->window, g_cd.slopes, scale);
-        pl = cd_gemm(T, l->wo);
-        cd_row(pl, T, false, g_cd.x, NULL, l->attn_scale, l->ffn_norm);
-        pl = cd_gemm(T, l->w13);
-#define CALL(C) hipLaunchKernelGGL(vt_codec_swiglu_kernel<C>, dim3(T), dim3(256), 0, g_vt.stream, g_cd.planes, g_cd.part, pl.col0, pl.cuts, (size_t)T * 2 * CD_HID)
-        CD_BY_CUTS(pl.cuts, CALL);
+        p = cd_gemm(T, l->wo);
+        cd_row(p, false, g_cd.x, NULL, l->attn_scale, l->ffn_norm);
+        p = cd_gemm(T, l->w13);
+#define CALL(C) hipLaunchKernelGGL(vt_codec_swiglu_kernel<C>, dim3(T), dim3(256), 0, g_vt.stream, g_cd.planes, p)
+        CD_BY_CUTS(p.cuts, CALL);
 #undef CALL
-        pl = cd_gemm(T, l->w2);
+        p = cd_gemm(T, l->w2);
         const int last_of_stage = (li & 1) == 1;
-        cd_row(pl, T, false, g_cd.x, NULL, l->ffn_scale, last_of_stage ? NULL : g_cd.layers[li + 1].attention_norm);
+        cd_row(p, false, g_cd.x, NULL, l->ffn_scale, last_of_stage ? NULL : g_cd.layers[li + 1].attention_norm);
         if (last_of_stage && li < CD_LAYERS - 1) {
             const int st = li / 2;
-            pl = cd_gemm(T, g_cd.w_up[st]);
-            cd_row(pl, T, true, NULL, g_cd.b_up[st], NULL, g_cd.layers[li + 1].attention_norm);
+            p = cd_gemm(T, g_cd.w_up[st]);
+            cd_row(p, true, NULL, g_cd.b_up[st], NULL, g_cd.layers[li + 1].attention_norm);
             T *= 2;
         }
     }
-    pl = cd_gemm(T, g_cd.w_out);
-#define CALL(C) hipLaunchKernelGGL(vt_codec_wave_kernel<C>, dim3(T), dim3(64), 0, g_vt.stream, d_samples, g_cd.part, pl.col0, pl.cuts, (size_t)T * CD_OUT_N, T, g_cd.b_out)
-    CD_BY_CUTS(pl.cuts, CALL);
+    p = cd_gemm(T, g_cd.w_out);
+#define CALL(C) hipLaunchKernelGGL(vt_codec_wave_kernel<C>, dim3(T), dim3(64), 0, g_vt.stream, d_samples, p, g_cd.b_out)
+    CD_BY_CUTS(p.cuts, CALL);
 #undef CALL
     return vt_check(hipGetLastError(), "codec launch");
 }

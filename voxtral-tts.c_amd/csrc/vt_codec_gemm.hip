@@ -89,12 +89,12 @@ static void cg_wide(const gw_list &list, const uint16_t *d_hi, const uint16_t *d
     hipLaunchKernelGGL((vt_gemm_wide_kernel<gm_f16x2, MB, CW>), dim3(items < g_vt.n_cu ? items : g_vt.n_cu), dim3(256), LDS, g_vt.stream, list, d_hi, d_lo, M, K);
 }
 
-void vt_launch_codec_gemm(float *d_C, int ldc, size_t plane_stride, const uint16_t *d_hi, const uint16_t *d_lo, const int *d_row_exp,
+void vt_launch_codec_gemm(float *d_C, const uint16_t *d_hi, const uint16_t *d_lo, const int *d_row_exp,
                           const uint16_t *d_Wf, const int *d_col_exp, int M, int N, int K, const vt_gemm_plan &pl) {
     if (pl.mb == 0) {
         gr_plan plan = {};
         plan.n_parts = 1;
-        plan.part[0] = gr_part{d_C, d_Wf, plane_stride, ldc, N / GR_TN, pl.cuts, NULL, NULL, 0, d_row_exp, d_col_exp};
+        plan.part[0] = gr_part{d_C, d_Wf, (size_t)M * N, N, N / GR_TN, pl.cuts, NULL, NULL, 0, d_row_exp, d_col_exp};
         const int items = plan.part[0].n_tiles * pl.cuts, grid = items < g_vt.n_cu ? items : g_vt.n_cu;
         static void (*const launch[4])(const gr_plan &, int, const uint16_t *, const uint16_t *, int, int) = {cg_rows<2>, cg_rows<4>, cg_rows<6>, cg_rows<8>};
         launch[(M + 15) / 16 - 1](plan, grid, d_hi, d_lo, M, K);
@@ -102,8 +102,8 @@ void vt_launch_codec_gemm(float *d_C, int ldc, size_t plane_stride, const uint16
     }
     gw_list list = {};
     list.m_tiles = (M + 32 * pl.mb - 1) / (32 * pl.mb);
-    gw_part whole = {d_C, d_Wf, plane_stride, ldc, pl.col0 / (64 * pl.cw), 1, NULL, NULL, 0, d_row_exp, d_col_exp};
-    gw_part cut = {d_C + pl.col0, d_Wf + (size_t)pl.col0 * K * 2, plane_stride, ldc, (N - pl.col0) / (64 * pl.cw), pl.cuts, NULL, NULL, 0,
+    gw_part whole = {d_C, d_Wf, 0, pl.col0, pl.col0 / (64 * pl.cw), 1, NULL, NULL, 0, d_row_exp, d_col_exp};
+    gw_part cut = {d_C + (size_t)M * pl.col0, d_Wf + (size_t)pl.col0 * K * 2, (size_t)M * (N - pl.col0), N - pl.col0, (N - pl.col0) / (64 * pl.cw), pl.cuts, NULL, NULL, 0,
                    d_row_exp, d_col_exp + pl.col0};
     if (whole.n_tiles) list.part[list.n_parts++] = whole;
     if (cut.n_tiles) list.part[list.n_parts++] = cut;

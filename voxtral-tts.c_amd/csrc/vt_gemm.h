@@ -42,10 +42,11 @@ void vt_launch_gemm_rows_swiglu(uint16_t *d_hhi, uint16_t *d_hlo, int ldh, float
                                 int tail_splits);
 /* The codec's products (vt_codec_gemm.hip): activations as two fp16 planes [M, K] with an exponent per row, weights in
  * fragment order with an exponent per column, from fp32 W[N, K] by vt_codec_weight_layout (d_Wf: 2 N K elements; 0 / -1).
- * N % 64 == 0 (more than 64 rows: % 256), K % 64 == 0; d_row_exp readable up to a multiple of 4 rows. */
+ * N % 64 == 0 (more than 64 rows: % 256), K % 64 == 0.  d_C: [M, pl.col0] and, behind it, pl.cuts planes of
+ * [M, N - pl.col0]. */
 vt_gemm_plan vt_codec_gemm_plan(int M, int N, int K);
 int vt_codec_weight_layout(uint16_t *d_Wf, int *d_col_exp, const float *d_W, int N, int K);
-void vt_launch_codec_gemm(float *d_C, int ldc, size_t plane_stride, const uint16_t *d_hi, const uint16_t *d_lo, const int *d_row_exp,
+void vt_launch_codec_gemm(float *d_C, const uint16_t *d_hi, const uint16_t *d_lo, const int *d_row_exp,
                           const uint16_t *d_Wf, const int *d_col_exp, int M, int N, int K, const vt_gemm_plan &pl);
 /* row-major bf16 W[N, K] -> the fragment-order copy (same size); N % 32 == 0, K % 64 == 0.  pair: W holds
  * (gate, up) rows interleaved and every 64 fragment columns become 32 gates followed by their 32 ups
