@@ -193,18 +193,16 @@ def test_prefill_chunks_three_layers():
 
 
 def test_prefill_row_counts_with_uneven_k_cuts():
-    """300 rows are 3 row tiles: the output and down products then run in 7 K cuts of 5 or 4 (11 or 10)
-    pairs of steps and q|k|v in 3; 650 rows (6 tiles) take 3 cuts and none."""
+    """300 rows are 4 tiles of 96: the output product then runs in 5 K cuts of 13 or 12 steps, the down product in 4
+    and q|k|v in 2; 650 rows (7 tiles) take 3, 3 and none."""
     _prefill_case(1, [300, 650], 960, lambda n: range(0, n, 7))
 
 
 @pytest.mark.parametrize("chunks", [[512], [64], [130, 7], [300], [1, 650]])
-def test_prefill_schedules_agree_bit_for_bit(chunks):
-    """Schedule 1 runs everything behind a layer's attention as one persistent launch whose work items
-    wait for each other per block of 128 rows; schedule 0 is one launch per product and row pass.  Same K
-    cuts, same tile walk, same sums in the same order: cache rows and residual stream must be equal bit
-    for bit, run after run (3 layers, so that the q|k|v product of the next layer inside the persistent
-    launch and the last layer without one are both walked)."""
+def test_prefill_is_reproducible_bit_for_bit(chunks):
+    """Tiles, K cuts and the order of all sums follow from the row count alone: three runs over cleared caches, under
+    either number of the one schedule, leave the same residual stream and cache rows.  (Against the
+    oracle: the tests around this one.)"""
     layers = [S.Layer(11), S.Layer(12)]
     norm = S.norm_weight(S.DIM, 98)
     n_layers, kv_max = 3, sum(chunks) + 8
@@ -220,7 +218,7 @@ def test_prefill_schedules_agree_bit_for_bit(chunks):
             hip.pos = 0
             xs = []
             for ci, s in enumerate(chunks):
-                print(f"prefill schedule {mode}, chunk of {s} rows at {hip.pos}", flush=True)
+                print(f"prefill run {run}, chunk of {s} rows at {hip.pos}", flush=True)
                 xs.append(hip.llm_prefill(S.f32_normal((s, S.DIM), 60 + ci), want_x=True))
             gk, gv = hip.kv()
             outs[run] = (np.concatenate(xs), gk[:n_layers].copy(), gv[:n_layers].copy())
@@ -228,9 +226,21 @@ def test_prefill_schedules_agree_bit_for_bit(chunks):
             for a, b, what in zip(outs[0], outs[run], ("residual stream", "k rows", "v rows")):
                 assert np.all(np.isfinite(a)), what
                 assert np.array_equal(a, b), (what, run, float(np.abs(a - b).max()))
-        hip.lib.tts_hip_set_prefill_mode(7)
-        assert b"tts_hip_set_prefill_mode" in hip.lib.tts_hip_last_error()
-        hip.err0 = hip.lib.tts_hip_error_count()
     finally:
-        hip.lib.tts_hip_set_prefill_mode(0)
+        hip.close()
+
+
+def test_prefill_against_the_oracle_at_the_reproduced_row_counts():
+    _prefill_case(2, [64], 68, lambda n: range(0, n, 3))
+    _prefill_case(2, [130, 7], 141, lambda n: range(0, n, 3))
+
+
+def test_unknown_prefill_schedule_is_an_error():
+    hip = H.Hip(kv_max=8)
+    try:
+        n0 = hip.lib.tts_hip_error_count()
+        hip.lib.tts_hip_set_prefill_mode(7)
+        assert hip.lib.tts_hip_error_count() == n0 + 1
+        assert b"tts_hip_set_prefill_mode" in hip.lib.tts_hip_last_error()
+    finally:
         hip.close()
