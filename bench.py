@@ -292,10 +292,11 @@ GEMM_SHAPES = (("q|k|v", 6144, 3072), ("output", 3072, 4096), ("gate|up", 18432,
 
 
 def prefill_flops(seq):
-    """Algorithmic flops of a 26-layer prefill: 2 M N K per projection plus the causal
-    attention (QK^T and PV over the visible keys of each query, 32 heads of 128)."""
-    gemm = 2 * seq * LAYER_WEIGHT_ELEMS * N_LAYERS
-    attn = 4 * S.HEAD_DIM * S.HEADS * (seq * (seq + 1) // 2) * N_LAYERS
+    """Algorithmic flops of a prefill for the cache (tts_hip_llm_prefill): 2 M N K per projection of 25 layers plus
+    their causal attention (QK^T and PV over the visible keys of each query, 32 heads of 128), and of the last
+    layer its k|v product, behind which the cache is complete."""
+    gemm = 2 * seq * (LAYER_WEIGHT_ELEMS * (N_LAYERS - 1) + 2 * S.KV_DIM * S.DIM)
+    attn = 4 * S.HEAD_DIM * S.HEADS * (seq * (seq + 1) // 2) * (N_LAYERS - 1)
     return gemm, attn
 
 
@@ -350,7 +351,6 @@ def bench_prefill(args):
     hip.upload_decoder(layers, final_norm, N_LAYERS)
     t_up = time.time() - t0
     d_e = H.DevBuf.from_numpy(lib, embeds)
-    lib.tts_hip_set_prefill_mode(args.prefill_mode)
     for _ in range(W):
         lib.tts_hip_llm_prefill(d_e.ptr, PREFILL_LEN, 0)
     lib.tts_hip_sync()
@@ -381,7 +381,8 @@ def bench_prefill(args):
         "config": {"workload": "26-layer backbone prefill of 512 random token ids, causal GQA attention "
                                "(BASELINE.json configs[3])",
                    "layers": N_LAYERS, "seq_len": PREFILL_LEN, "weights": "bf16 N(0,0.02) seeded, truncated",
-                   "schedule": "one launch per product and row pass"},
+                   "schedule": "one launch per product and row pass; the call fills the cache, so of the last layer only the "
+                               "k|v product is done and counted"},
         "tokens_per_s": round(PREFILL_LEN / (ms_step * 1e-3), 1),
         "tflops": round((gemm_fl + attn_fl) / ms_step / 1e9, 1),
         "roofline": {
@@ -436,10 +437,13 @@ AC_PHASES = (("q|k|v", 10, 2 * 6144 * 3072), ("attention+output", 11, 2 * 3072 *
 
 def acoustic_frame_bytes():
     """Algorithmic HBM bytes of one frame: 7 Euler steps x 3 layers of bf16 weights (each streamed
-    once per step for both guidance branches), the 36-wide in/out projections per step, the semantic
+    once per step for both guidance branches; the first layer's q|k|v once per frame, for the LLM token, and per step
+    its fp32 product with the input projection instead), the 36-wide in/out projections per step, the semantic
     head and the LLM-token projection once per frame.  Time tokens are cached per upload."""
-    per_step = 3 * AC_LAYER_BYTES + 2 * (S.DIM * S.ACOUSTIC_DIM * 2) + 6 * S.DIM * 4
-    return 7 * per_step + 8320 * S.DIM * 2 + S.DIM * S.DIM * 2
+    qkv = 2 * (S.Q_DIM + 2 * S.KV_DIM) * S.DIM
+    folded = 4 * (S.Q_DIM + 2 * S.KV_DIM) * S.ACOUSTIC_DIM
+    per_step = 3 * AC_LAYER_BYTES - qkv + folded + 2 * (S.DIM * S.ACOUSTIC_DIM * 2) + 6 * S.DIM * 4
+    return 7 * per_step + qkv + 8320 * S.DIM * 2 + S.DIM * S.DIM * 2
 
 
 def bench_acoustic(args):
@@ -1063,8 +1067,6 @@ def main():
     ap.add_argument("--workload", choices=("decode", "prefill", "acoustic", "frame", "codec", "matvec", "layer"), default="decode",
                     help="decode = the headline metric; prefill / acoustic = the other two configurations")
     ap.add_argument("--mode", type=int, default=0, choices=(0, 1), help="0 persistent kernel, 1 per-phase kernels")
-    ap.add_argument("--prefill-mode", type=int, default=0, choices=(0, 1),
-                    help="--workload prefill: 0 one launch per product and row pass, 1 one persistent launch per layer")
     ap.add_argument("--cpu-seconds", type=float, default=12.0, help="budget of the CPU baseline leg (0 = skip)")
     ap.add_argument("--no-workloads", action="store_true",
                     help="leave the short runs of the other configurations out of the default line")

@@ -1,7 +1,7 @@
 """Audio codec decoder on the device (tts_codec_decode, voxtral_tts_codec.c:389-503) against
 the oracle, which is bit-equal to the compiled reference on these inputs
-(tests/test_oracle_golden.py).  The device sums every dot product on the fp32 matrix cores in
-another order than the CPU loop, so the bar is the floating-point one: max |d| / rms and
+(tests/test_oracle_golden.py).  The device sums every dot product on the fp16 matrix cores, two
+planes per operand, in another order than the CPU loop, so the bar is the floating-point one: max |d| / rms and
 relative L2 of the waveform <= 1e-3."""
 import ctypes as C
 

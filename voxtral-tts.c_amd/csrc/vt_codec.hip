@@ -529,14 +529,14 @@ static float *cd_upload_convt(const tts_hip_host_conv_t *cv) {
     return d;
 }
 
-static float *cd_upload_bias(const float *bias, int n, int n_pad, int repeat) {
+static float *cd_upload_bias(const float *bias, int n, int n_pad) {
     if (!bias) return NULL;
     float *h = cd_host(bias, n);
-    float *r = (float *)calloc((size_t)n_pad * repeat, sizeof(float));
+    float *r = (float *)calloc(n_pad, sizeof(float));
     float *d = NULL;
     if (h && r) {
-        for (int k = 0; k < repeat; k++) memcpy(r + (size_t)k * n_pad, h, n * sizeof(float));
-        d = cd_upload(r, (size_t)n_pad * repeat);
+        memcpy(r, h, n * sizeof(float));
+        d = cd_upload(r, n_pad);
     }
     free(h); free(r);
     return d;
@@ -567,12 +567,12 @@ extern "C" int tts_hip_upload_codec_weights(void *codec_ptr) {
     ok &= (g_cd.sem = cd_upload(c->semantic_embedding, (size_t)CD_SEM_SIZE * CD_SEM_DIM)) != NULL;
     ok &= (g_cd.slopes = cd_upload(c->alibi_slopes, CD_HEADS)) != NULL;
     ok &= cd_matrix_from(&g_cd.w_in, cd_upload_conv(&c->input_conv, CD_DIM, CD_IN_K, 0, CD_EMBED), CD_DIM, CD_IN_K);
-    g_cd.b_in = cd_upload_bias(c->input_conv.bias, CD_DIM, CD_DIM, 1);
+    g_cd.b_in = cd_upload_bias(c->input_conv.bias, CD_DIM, CD_DIM);
     ok &= cd_matrix_from(&g_cd.w_out, cd_upload_conv(&c->output_proj, CD_OUT_N, CD_DIM, CD_OUT_PITCH, 0), CD_OUT_N, CD_DIM);
-    g_cd.b_out = cd_upload_bias(c->output_proj.bias, CD_PATCH, CD_OUT_PITCH, 1);
+    g_cd.b_out = cd_upload_bias(c->output_proj.bias, CD_PATCH, CD_OUT_PITCH);
     for (int i = 0; ok && i < 3; i++) {
         ok &= cd_matrix_from(&g_cd.w_up[i], cd_upload_convt(&c->stage_convs[i]), CD_UP_N, CD_DIM);
-        g_cd.b_up[i] = cd_upload_bias(c->stage_convs[i].bias, CD_DIM, CD_DIM, 1);
+        g_cd.b_up[i] = cd_upload_bias(c->stage_convs[i].bias, CD_DIM, CD_DIM);
     }
     for (int i = 0; ok && i < CD_LAYERS; i++) {
         const tts_hip_host_codec_layer_t *s = &c->transformers[i];

@@ -439,7 +439,7 @@ __device__ __forceinline__ u32x4 gr_ld_nt(__amdgpu_buffer_rsrc_t r, int voff, in
 /* One workgroup's piece of a product: a 64-column tile over one K cut */
 struct gr_item {
     const unsigned char *w;               /* weights of the tile */
-    int part, nt, sp, s0, n;              /* n: this wave's K steps s0 + wave + 8 i */
+    int part, nt, sp, s0, n;              /* n: this wave's K steps s0 + wave + NW i */
 };
 
 template <int NW, int WP>
