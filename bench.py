@@ -292,12 +292,18 @@ GEMM_SHAPES = (("q|k|v", 6144, 3072), ("output", 3072, 4096), ("gate|up", 18432,
 
 
 def prefill_flops(seq):
-    """Algorithmic flops of a prefill for the cache (tts_hip_llm_prefill): 2 M N K per projection of 25 layers plus
-    their causal attention (QK^T and PV over the visible keys of each query, 32 heads of 128), and of the last
-    layer its k|v product, behind which the cache is complete."""
-    gemm = 2 * seq * (LAYER_WEIGHT_ELEMS * (N_LAYERS - 1) + 2 * S.KV_DIM * S.DIM)
-    attn = 4 * S.HEAD_DIM * S.HEADS * (seq * (seq + 1) // 2) * (N_LAYERS - 1)
+    """Algorithmic flops of a 26-layer prefill: 2 M N K per projection plus the causal
+    attention (QK^T and PV over the visible keys of each query, 32 heads of 128)."""
+    gemm = 2 * seq * LAYER_WEIGHT_ELEMS * N_LAYERS
+    attn = 4 * S.HEAD_DIM * S.HEADS * (seq * (seq + 1) // 2) * N_LAYERS
     return gemm, attn
+
+
+def cache_prefill_flops(seq):
+    """The same for a prefill that fills the cache (tts_hip_llm_prefill): 25 layers, and of the last one its k|v
+    product, behind which the cache is complete."""
+    gemm, attn = prefill_flops(seq)
+    return gemm - 2 * seq * (LAYER_WEIGHT_ELEMS - 2 * S.KV_DIM * S.DIM), attn // N_LAYERS * (N_LAYERS - 1)
 
 
 REF_LINEARS = (("wq", S.Q_DIM, S.DIM), ("wk", S.KV_DIM, S.DIM), ("wv", S.KV_DIM, S.DIM), ("wo", S.DIM, S.Q_DIM),
@@ -360,7 +366,7 @@ def bench_prefill(args):
     ms_step = BL().tts_hip_timer_stop_ms() / K
     lib.tts_hip_sync()
     hip.check()
-    gemm_fl, attn_fl = prefill_flops(PREFILL_LEN)
+    gemm_fl, attn_fl = cache_prefill_flops(PREFILL_LEN)
     # the dominant kernel alone, per projection shape, timed by the library with events
     per_shape = {}
     for i, (name, n, k) in enumerate(GEMM_SHAPES):
@@ -958,7 +964,7 @@ def other_workloads(hip, kv_max):
     for _ in range(8):
         lib.tts_hip_llm_prefill(d_e.ptr, PREFILL_LEN, 0)
     ms = BL().tts_hip_timer_stop_ms() / 8
-    gemm_fl, attn_fl = prefill_flops(PREFILL_LEN)
+    gemm_fl, attn_fl = cache_prefill_flops(PREFILL_LEN)
     ms_layer = sum(BL().tts_hip_bench_kernel(i, 26) for i in range(4))
     achieved = 2.0 * PREFILL_LEN * LAYER_WEIGHT_ELEMS / ms_layer / 1e9
     w["prefill, 512 tokens x 26 layers"] = {
