@@ -16,7 +16,7 @@
  * 0.75 / 1.2 / 17 / 209e-7 without it; fp32 sums in order have 5.7e-7.  hi times 2^-6, which it takes, costs 0.7 / 1.6 / 1.5 %
  * of a decode of 21 / 212 / 1003 frames.
  * Rates, TFLOP/s of the product itself (v_mfma_f32_32x32x2f32 in 128 x 128 tiles before: 75 .. 105): gate|up
- * 8192 x 1024 at 212 / 848 / 1696 / 8024 rows 150 / 287 / 290 / 335, down 1024 x 4096 111 / 227 / 282 / 336.
+ * 8192 x 1024 at 212 / 848 / 1696 / 8024 rows 152 / 281 / 292 / 331, down 1024 x 4096 105 / 242 / 282 / 391.
  */
 #include "vt_gemm_tiles.h"
 

@@ -127,7 +127,7 @@ __device__ __forceinline__ void gm_store_quad(float *C, int ldc, int row0, int M
  * every load is then 1 KB of consecutive bytes.
  *
  * A launch has at most one workgroup per CU, which walks its items: first whole tiles, as many rounds of them
- * as every CU can take part in, then the tiles that are left as K cuts, so many that every CU gets one.  The
+ * as every CU can take part in, then the tiles that are left as K cuts, of which a CU gets one or none.  The
  * first requests of an item go out in front of the stores of the one before it.  Only the columns of the cut
  * tiles have more than one partial plane; whoever reads the result is told from which column on (vt_gemm_plan).
  */
