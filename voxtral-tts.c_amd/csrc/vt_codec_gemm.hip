@@ -9,12 +9,11 @@
  * matter more, the result is closer to 64 bits than with fp32 instructions.
  * Three fp16 instructions do 16 times the work of an fp32 one each, so the
  * same product takes 3/16 of the matrix-core time; what it then runs into is the card's power limit.
- * Measured against float64, error of a row over its l2 norm: 1.4e-7 .. 3.6e-7 (K 1024 .. 7168, rows and elements of
- * log-normal magnitude) where a plain fp32 product has 2.7e-7 .. 1.1e-6: what remains is the fp32 sums.
- * The 2^6 is for rows with values far apart whose large ones meet zeros.  Error of the operands and the left-out term
- * alone, K = 1024, one channel 1 / 2^16 / 2^20 / 2^24 times the others: 0.75 / 0.75 / 0.77 / 2.4e-7 of the result, and
- * 0.75 / 1.2 / 17 / 209e-7 without it; fp32 sums in order have 5.7e-7.  hi times 2^-6, which it takes, costs 0.7 / 1.6 / 1.5 %
- * of a decode of 21 / 212 / 1003 frames.
+ * Measured against float64, error of a row over its l2 norm, K 1024 / 4096: 1.4e-7 / 2.1e-7, worst row 2.7e-7 / 4.0e-7
+ * (rows and elements of log-normal magnitude), where fp32 sums in order have 5.7e-7 / 1.1e-6, worst 1.6e-6 / 1.9e-6.
+ * The 2^6 is for rows with values far apart whose large ones meet zeros: with one channel of the activations and one of
+ * the weights 2^20 / 2^24 times the others, 1.4e-7 / 4.4e-7 at K = 1024 (2.1e-7 / 4.6e-7 at 4096); without it the operands alone
+ * leave 2.4e-6 / 3.7e-5 at K = 1024.  hi times 2^-6, which it takes, costs 0.7 / 1.6 / 1.5 % of a decode of 21 / 212 / 1003 frames.
  * Rates, TFLOP/s of the product itself (v_mfma_f32_32x32x2f32 in 128 x 128 tiles before: 75 .. 105): gate|up
  * 8192 x 1024 at 212 / 848 / 1696 / 8024 rows 152 / 281 / 292 / 331, down 1024 x 4096 105 / 242 / 282 / 391.
  */
