@@ -80,12 +80,12 @@ static void cg_wide(const gw_list &list, const uint16_t *d_hi, const uint16_t *d
     constexpr int LDS = 2 * (4 / CW) * 2 * 32 * MB * GM_STAGE_ROW;
     static int attr_set = 0;
     if (!attr_set) {
-        if (vt_check(hipFuncSetAttribute((const void *)vt_gemm_wide_kernel<gm_f16x2, MB, CW>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS), "product LDS size"))
+        if (vt_check(hipFuncSetAttribute((const void *)vt_gemm_wide_kernel<gm_f16x2, MB, CW, 2>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS), "product LDS size"))
             return;
         attr_set = 1;
     }
     const int items = list.m_tiles * list.part[0].n_tiles * list.part[0].splits;
-    hipLaunchKernelGGL((vt_gemm_wide_kernel<gm_f16x2, MB, CW>), dim3(items < g_vt.n_cu ? items : g_vt.n_cu), dim3(256), LDS, g_vt.stream, list, d_hi, d_lo, M, K);
+    hipLaunchKernelGGL((vt_gemm_wide_kernel<gm_f16x2, MB, CW, 2>), dim3(items < g_vt.n_cu ? items : g_vt.n_cu), dim3(256), LDS, g_vt.stream, list, d_hi, d_lo, M, K);
 }
 
 void vt_launch_codec_gemm(float *d_C, const uint16_t *d_hi, const uint16_t *d_lo, const int *d_row_exp,
@@ -101,13 +101,11 @@ void vt_launch_codec_gemm(float *d_C, const uint16_t *d_hi, const uint16_t *d_lo
     }
     gw_list list = {};
     list.m_tiles = (M + 32 * pl.mb - 1) / (32 * pl.mb);
-    gw_part whole = {d_C, d_Wf, 0, pl.col0, pl.col0 / (64 * pl.cw), 1, NULL, NULL, 0, d_row_exp, d_col_exp};
-    gw_part cut = {d_C + (size_t)M * pl.col0, d_Wf + (size_t)pl.col0 * K * 2, (size_t)M * (N - pl.col0), N - pl.col0, (N - pl.col0) / (64 * pl.cw), pl.cuts, NULL, NULL, 0,
+    gw_part whole = {d_C, d_Wf, 0, pl.col0, pl.col0 / pl.tn, 1, NULL, NULL, 0, d_row_exp, d_col_exp};
+    gw_part cut = {d_C + (size_t)M * pl.col0, d_Wf + (size_t)pl.col0 * K * 2, (size_t)M * (N - pl.col0), N - pl.col0, (N - pl.col0) / pl.tn, pl.cuts, NULL, NULL, 0,
                    d_row_exp, d_col_exp + pl.col0};
     if (whole.n_tiles) list.part[list.n_parts++] = whole;
     if (cut.n_tiles) list.part[list.n_parts++] = cut;
-    if (pl.mb == 4 && pl.cw == 4) cg_wide<4, 4>(list, d_hi, d_lo, M, K);
-    else if (pl.mb == 4) cg_wide<4, 2>(list, d_hi, d_lo, M, K);
-    else if (pl.cw == 4) cg_wide<3, 4>(list, d_hi, d_lo, M, K);
-    else cg_wide<3, 2>(list, d_hi, d_lo, M, K);
+    static void (*const launch[2][2])(const gw_list &, const uint16_t *, const uint16_t *, int, int) = {{cg_wide<3, 2>, cg_wide<3, 4>}, {cg_wide<4, 2>, cg_wide<4, 4>}};
+    launch[pl.mb - 3][pl.tn == 256](list, d_hi, d_lo, M, K);
 }

@@ -18,9 +18,10 @@ void vt_launch_gemm_ex(float *d_C, int ldc, size_t plane_stride, const uint16_t 
                        const uint16_t *d_W, int M, int N, int K, int splits);
 /* How a product of the backbone is done on fragment-order weights (vt_launch_frag_layout): the columns below
  * col0 as whole tiles (one plane), the others with K in `cuts` cuts (that many partial planes, to be added in
- * order by whoever reads the result).  mb, cw: the tile (vt_gemm_wide.hip; mb 0: vt_gemm_rows.hip). */
+ * order by whoever reads the result).  mb, tn: the tile, 32 mb rows x tn columns
+ * (vt_gemm_wide.hip; mb 0: vt_gemm_rows.hip).  col0 is a multiple of 128. */
 #define VT_MAX_CUTS 8
-struct vt_gemm_plan { int mb, cw, col0, cuts; };
+struct vt_gemm_plan { int mb, tn, col0, cuts; };
 /* N % 256 == 0, K % 64 == 0; swiglu: for vt_launch_gemm_frag_swiglu */
 vt_gemm_plan vt_gemm_frag_plan(int M, int N, int K, int swiglu);
 void vt_launch_gemm_frag(float *d_C, int ldc, size_t plane_stride, const uint16_t *d_Ahi, const uint16_t *d_Alo,

@@ -37,7 +37,7 @@ struct gm_f16x2 {
     }
 };
 
-template <int WP> struct gm_weights { u32x4 v[WP][2][4]; };       /* one 64-wide K step: [plane][block of 32 columns][16-wide slice] */
+template <int WP, int NB> struct gm_weights { u32x4 v[WP][NB][4]; };      /* one 64-wide K step: [plane][block of 32 columns][16-wide slice] */
 template <int MB> struct gm_frags { u32x4 hi[MB], lo[MB]; };      /* one 16-wide slice of MB blocks of 32 rows, both planes */
 
 /* A request through a descriptor: one whose size is 0, and a byte offset beyond the size, load nothing (zeros) */
@@ -49,72 +49,71 @@ __device__ __forceinline__ u32x4 gm_down(const u32x4 &hi) {
     return __builtin_bit_cast(u32x4, __builtin_bit_cast(gm_f16x8, hi) * (_Float16)(1.0f / (1 << VT_F16_LO_EXP)));
 }
 
-/* one slice; 2 MB independent sums between two products into the same one */
-template <class T, int MB>
-__device__ __forceinline__ void gm_multiply(f32x16 (&acc)[MB][2], const gm_frags<MB> &f, const gm_weights<T::WP> &w, int ks) {
+/* one slice; MB NB independent sums between two products into the same one */
+template <class T, int MB, int NB>
+__device__ __forceinline__ void gm_multiply(f32x16 (&acc)[MB][NB], const gm_frags<MB> &f, const gm_weights<T::WP, NB> &w, int ks) {
     if constexpr (T::WP == 2) {
 #pragma unroll
         for (int a = 0; a < MB; a++)
 #pragma unroll
-            for (int b = 0; b < 2; b++) acc[a][b] = T::mfma(f.hi[a], w.v[0][b][ks], acc[a][b]);
-        const u32x4 wd[2] = {gm_down(w.v[0][0][ks]), gm_down(w.v[0][1][ks])};
+            for (int b = 0; b < NB; b++) acc[a][b] = T::mfma(f.hi[a], w.v[0][b][ks], acc[a][b]);
+        u32x4 wd[NB];
+#pragma unroll
+        for (int b = 0; b < NB; b++) wd[b] = gm_down(w.v[0][b][ks]);
 #pragma unroll
         for (int a = 0; a < MB; a++)
 #pragma unroll
-            for (int b = 0; b < 2; b++) acc[a][b] = T::mfma(f.lo[a], wd[b], acc[a][b]);
+            for (int b = 0; b < NB; b++) acc[a][b] = T::mfma(f.lo[a], wd[b], acc[a][b]);
 #pragma unroll
         for (int a = 0; a < MB; a++) {
             const u32x4 d = gm_down(f.hi[a]);
 #pragma unroll
-            for (int b = 0; b < 2; b++) acc[a][b] = T::mfma(d, w.v[1][b][ks], acc[a][b]);
+            for (int b = 0; b < NB; b++) acc[a][b] = T::mfma(d, w.v[1][b][ks], acc[a][b]);
         }
     } else {
         /* the small products first */
 #pragma unroll
         for (int a = 0; a < MB; a++)
 #pragma unroll
-            for (int b = 0; b < 2; b++) acc[a][b] = T::mfma(f.lo[a], w.v[0][b][ks], acc[a][b]);
+            for (int b = 0; b < NB; b++) acc[a][b] = T::mfma(f.lo[a], w.v[0][b][ks], acc[a][b]);
 #pragma unroll
         for (int a = 0; a < MB; a++)
 #pragma unroll
-            for (int b = 0; b < 2; b++) acc[a][b] = T::mfma(f.hi[a], w.v[0][b][ks], acc[a][b]);
+            for (int b = 0; b < NB; b++) acc[a][b] = T::mfma(f.hi[a], w.v[0][b][ks], acc[a][b]);
     }
 }
 
-/* rows row0 .. + 3 of one column (q0) and of the column 32 further on (q1); C points at row 0 of the column */
-template <class T>
-__device__ __forceinline__ void gm_store_quad(float *C, int ldc, int row0, int M, const f32x4 &q0, const f32x4 &q1,
-                                              const int *row_exp, const int *col_exp) {
+/* rows row0 .. + 3 of NB columns 32 apart; C and col_exp point at the first of them, C at its row 0 */
+template <class T, int NB>
+__device__ __forceinline__ void gm_store_quad(float *C, int ldc, int row0, int M, const f32x4 (&q)[NB], const int *row_exp, const int *col_exp) {
+    int e[NB];
     if constexpr (T::SCALED) {
-        const int e0 = col_exp[0], e1 = col_exp[32];
 #pragma unroll
-        for (int v = 0; v < 4; v++)
-            if (row0 + v < M) {
-                const int e = row_exp[row0 + v];
-                C[(size_t)(row0 + v) * ldc] = __builtin_amdgcn_ldexpf(q0[v], -e0 - e);
-                C[(size_t)(row0 + v) * ldc + 32] = __builtin_amdgcn_ldexpf(q1[v], -e1 - e);
-            }
-    } else {
-#pragma unroll
-        for (int v = 0; v < 4; v++)
-            if (row0 + v < M) {
-                C[(size_t)(row0 + v) * ldc] = q0[v];
-                C[(size_t)(row0 + v) * ldc + 32] = q1[v];
-            }
+        for (int b = 0; b < NB; b++) e[b] = col_exp[32 * b];
     }
+#pragma unroll
+    for (int v = 0; v < 4; v++)
+        if (row0 + v < M) {
+            const int er = T::SCALED ? row_exp[row0 + v] : 0;
+#pragma unroll
+            for (int b = 0; b < NB; b++)
+                C[(size_t)(row0 + v) * ldc + 32 * b] = T::SCALED ? __builtin_amdgcn_ldexpf(q[b][v], -e[b] - er) : q[b][v];
+        }
 }
 
 /* ---- more than 64 rows ---------------------------------------------------------------------------------
- * A wave owns MB x 32 rows (MB 3 or 4) x 64 columns: the weights of its 64 columns are nobody else's among the
+ * A wave owns MB x 32 rows (MB 3 or 4) x 64 or 96 columns: the weights of its columns are nobody else's among the
  * waves that work on the same K step, so they go from global memory straight into the B operand registers, and
  * only the activation planes pass through the LDS: 8 KB of fragment reads per 16 matrix instructions, half
  * the LDS bandwidth (a 64 x 64 wave tile with both operands in LDS, vt_gemm_mfma_kernel, needs three quarters).
  * One workgroup of four waves per CU (a wave may then use the whole register file of its SIMD: up to 128
- * accumulator registers, two sets of weight registers, two sets of fragments), in one of two shapes:
+ * accumulator registers, 192 with 96 columns, two sets of weight registers, two sets of fragments), in one of these shapes:
  *   CW = 4: four waves side by side, tile MB*32 x 256; the planes of one K step serve four waves;
- *   CW = 2: two waves side by side and two K steps at a time, tile MB*32 x 128; the two halves of K are added
- *           through LDS at the end.  Half the tile, for row counts whose 256-column tiles do not deal out over
- *           the CUs, at the price of twice the plane traffic (L2 and LDS stores) per matrix instruction.
+ *   CW = 2: two waves side by side and two K steps at a time, tile MB*32 x 128 (NB = 2 blocks of 32 columns per wave) or
+ *           x 192 (NB = 3); the two halves of K are added through LDS at the end.  For row counts whose 256-column
+ *           tiles do not deal out over the CUs, at the price of more plane traffic (L2 and LDS stores) per matrix
+ *           instruction: operand bytes per cycle of matrix instructions 32 (128 x 256), 37 (128 x 192), 47 (128 x 128).
+ *           With 192 columns a step is half as long again, and the planes of 128 rows are requested one step ahead.
  * Two LDS stages: the planes of the next step are written while this one is multiplied, one barrier per step;
  * the global loads of the step after that are in flight meanwhile (every request unconditional, through
  * descriptors whose size says whether there is anything to load, so the waits count exactly).
@@ -172,12 +171,13 @@ __device__ __forceinline__ gw_item gw_item_at(const gw_list &list, int part, int
     return it;
 }
 
-template <class T, int MB, int CW>
+template <class T, int MB, int CW, int NB>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
 vt_gemm_wide_kernel(gw_list list, const uint16_t *Ahi, const uint16_t *Alo, int M, int K) {
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-    constexpr int WP = T::WP, KW = 4 / CW, TM = 32 * MB, TN = 64 * CW;
+    constexpr int WP = T::WP, KW = 4 / CW, TM = 32 * MB, TN = 32 * NB * CW;
     constexpr int NP = 4 * MB / CW;                        /* staging passes over a plane, 8 * CW rows each */
+    constexpr int AHEAD = MB * NB > 8 && CW == 2 ? 1 : 2;  /* steps between the request of a step's planes and their store (registers) */
     constexpr int PLANE = TM * GM_STAGE_ROW, GROUP = 2 * PLANE, STAGE = KW * GROUP;
     const int lane = (int)threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int cw = wave % CW, kw = wave / CW;              /* column block of the tile; which of the KW K steps */
@@ -197,16 +197,15 @@ vt_gemm_wide_kernel(gw_list list, const uint16_t *Ahi, const uint16_t *Alo, int 
 #pragma unroll
         for (int p = 0; p < NP; p++) r[p] = gm_ldb(d, a_voff + p * a_pass, soff);
     };
-    auto fetch_b_slice = [&](const gw_item &it, gm_weights<WP> &r, int i, int j) {
+    auto fetch_b_slice = [&](const gw_item &it, gm_weights<WP, NB> &r, int i, int j) {
         const int s = KW * i + kw;
         const bool live = s < it.ns;
-        const __amdgpu_buffer_rsrc_t d = __builtin_amdgcn_make_buffer_rsrc((void *)(it.w + (size_t)cw * 2 * blk_bytes), 0, live ? 2 * blk_bytes : 0, 0x00020000);
+        const __amdgpu_buffer_rsrc_t d = __builtin_amdgcn_make_buffer_rsrc((void *)(it.w + (size_t)cw * NB * blk_bytes), 0, live ? NB * blk_bytes : 0, 0x00020000);
         const int soff = live ? (it.s0 + s) * 4096 * WP : 0;
 #pragma unroll
-        for (int p = 0; p < WP; p++) {
-            r.v[p][0][j] = gm_ldb(d, lane * 16 + 1024 * j, soff + 4096 * p);
-            r.v[p][1][j] = gm_ldb(d, lane * 16 + 1024 * j, soff + 4096 * p + (live ? blk_bytes : 0));
-        }
+        for (int p = 0; p < WP; p++)
+#pragma unroll
+            for (int b = 0; b < NB; b++) r.v[p][b][j] = gm_ldb(d, lane * 16 + 1024 * j, soff + 4096 * p + (live ? b * blk_bytes : 0));
     };
     auto store_a = [&](const u32x4 (&r)[NP], int at) {
 #pragma unroll
@@ -221,8 +220,8 @@ vt_gemm_wide_kernel(gw_list list, const uint16_t *Ahi, const uint16_t *Alo, int 
             f.lo[a] = *reinterpret_cast<const u32x4 *>(base + PLANE + 32 * a * GM_STAGE_ROW);
         }
     };
-    f32x16 acc[MB][2];
-    auto mma = [&](const frags &f, const gm_weights<WP> &w, int ks) { gm_multiply<T, MB>(acc, f, w, ks); };
+    f32x16 acc[MB][NB];
+    auto mma = [&](const frags &f, const gm_weights<WP, NB> &w, int ks) { gm_multiply<T, MB, NB>(acc, f, w, ks); };
 
     /* One step: stage `stage` holds the planes of step i and `cur` its weights; ra holds the planes of step
      * i + 1 (requested two steps ago: with one step between request and store, the step takes as long as a load,
@@ -234,37 +233,37 @@ vt_gemm_wide_kernel(gw_list list, const uint16_t *Ahi, const uint16_t *Alo, int 
      * barrier stands in front of the last region: by then every wave has issued (and waited for) its stores
      * into the other stage and its last reads of this one, so the first fragments of step i + 1 are read under
      * the last matrix instructions of step i. */
-    gm_weights<WP> b0, b1;
-    aregs ra0, ra1;                       /* the rows of even and of odd steps */
+    gm_weights<WP, NB> b0, b1;
+    aregs ra0, ra1;                       /* the rows of even and of odd steps (AHEAD 1: ra0 of all) */
     frags f0, f1;
 #define GW_FENCE() __builtin_amdgcn_sched_barrier(0)
-#define GW_MFMA() __builtin_amdgcn_sched_group_barrier(0x008, 1 + WP, 0)
+#define GW_MFMA() __builtin_amdgcn_sched_group_barrier(0x008, NB * (1 + WP) / 2, 0)
 #define GW_DSR1() __builtin_amdgcn_sched_group_barrier(0x100, 1, 0)
 #define GW_DSW1() __builtin_amdgcn_sched_group_barrier(0x200, 1, 0)
 #define GW_VMR1() __builtin_amdgcn_sched_group_barrier(0x020, 1, 0)
-    auto step = [&](const gw_item &it, int i, int stage, gm_weights<WP> &cur, aregs &ra) {
+    auto step = [&](const gw_item &it, int i, int stage, gm_weights<WP, NB> &cur, aregs &ra) {
         const int other = (stage ^ 1) * STAGE;
         GW_FENCE();
         store_a(ra.hi, other);
-        fetch_a(it, Ahi, ra.hi, i + 3);
+        fetch_a(it, Ahi, ra.hi, i + 1 + AHEAD);
         read_frags(f1, stage, 1);
         mma(f0, cur, 0);
 #pragma unroll
         for (int k = 0; k < 2 * MB; k++) { GW_MFMA(); GW_DSR1(); if (k < NP) { GW_DSW1(); GW_VMR1(); } }
         GW_FENCE();
         store_a(ra.lo, other + PLANE);
-        fetch_a(it, Alo, ra.lo, i + 3);
+        fetch_a(it, Alo, ra.lo, i + 1 + AHEAD);
         fetch_b_slice(it, cur, i + 2, 0);
         read_frags(f0, stage, 2);
         mma(f1, cur, 1);
 #pragma unroll
-        for (int k = 0; k < 2 * MB; k++) { GW_MFMA(); GW_DSR1(); if (k < NP) { GW_DSW1(); GW_VMR1(); } if (k < 2 * WP) GW_VMR1(); }
+        for (int k = 0; k < 2 * MB; k++) { GW_MFMA(); GW_DSR1(); if (k < NP) { GW_DSW1(); GW_VMR1(); } if (k < NB * WP) GW_VMR1(); }
         GW_FENCE();
         fetch_b_slice(it, cur, i + 2, 1);
         read_frags(f1, stage, 3);
         mma(f0, cur, 2);
 #pragma unroll
-        for (int k = 0; k < 2 * MB; k++) { GW_MFMA(); GW_DSR1(); if (k < 2 * WP) GW_VMR1(); }
+        for (int k = 0; k < 2 * MB; k++) { GW_MFMA(); GW_DSR1(); if (k < NB * WP) GW_VMR1(); }
         GW_FENCE();
         __syncthreads();
         GW_FENCE();
@@ -272,7 +271,7 @@ vt_gemm_wide_kernel(gw_list list, const uint16_t *Ahi, const uint16_t *Alo, int 
         read_frags(f0, stage ^ 1, 0);
         mma(f1, cur, 3);
 #pragma unroll
-        for (int k = 0; k < 2 * MB; k++) { GW_MFMA(); GW_DSR1(); if (k < 2 * WP) GW_VMR1(); }
+        for (int k = 0; k < 2 * MB; k++) { GW_MFMA(); GW_DSR1(); if (k < NB * WP) GW_VMR1(); }
         GW_FENCE();
         fetch_b_slice(it, cur, i + 2, 3);
     };
@@ -282,8 +281,10 @@ vt_gemm_wide_kernel(gw_list list, const uint16_t *Ahi, const uint16_t *Alo, int 
         fetch_a(it, Alo, ra0.lo, 0);
 #pragma unroll
         for (int j = 0; j < 4; j++) fetch_b_slice(it, b0, 0, j);
-        fetch_a(it, Ahi, ra1.hi, 1);
-        fetch_a(it, Alo, ra1.lo, 1);
+        if constexpr (AHEAD == 2) {
+            fetch_a(it, Ahi, ra1.hi, 1);
+            fetch_a(it, Alo, ra1.lo, 1);
+        }
 #pragma unroll
         for (int j = 0; j < 4; j++) fetch_b_slice(it, b1, 1, j);
         GW_FENCE();
@@ -292,23 +293,24 @@ vt_gemm_wide_kernel(gw_list list, const uint16_t *Ahi, const uint16_t *Alo, int 
 #pragma unroll
         for (int a = 0; a < MB; a++)
 #pragma unroll
-            for (int b = 0; b < 2; b++)
+            for (int b = 0; b < NB; b++)
 #pragma unroll
                 for (int v = 0; v < 16; v++) acc[a][b][v] = 0.f;
         store_a(ra0.hi, 0);
         store_a(ra0.lo, PLANE);
-        fetch_a(it, Ahi, ra0.hi, 2);
-        fetch_a(it, Alo, ra0.lo, 2);
+        fetch_a(it, Ahi, ra0.hi, AHEAD);
+        fetch_a(it, Alo, ra0.lo, AHEAD);
         GW_FENCE();
         __syncthreads();
         read_frags(f0, 0, 0);
         const int n = (it.ns + KW - 1) / KW;
+        aregs &odd = AHEAD == 2 ? ra1 : ra0;
         int i = 0;
         for (; i + 1 < n; i += 2) {
-            step(it, i, 0, b0, ra1);
+            step(it, i, 0, b0, odd);
             step(it, i + 1, 1, b1, ra0);
         }
-        if (i < n) step(it, i, 0, b0, ra1);
+        if (i < n) step(it, i, 0, b0, odd);
     };
 #undef GW_MFMA
 #undef GW_DSR1
@@ -316,58 +318,64 @@ vt_gemm_wide_kernel(gw_list list, const uint16_t *Ahi, const uint16_t *Alo, int 
 #undef GW_VMR1
 #undef GW_FENCE
 
-    /* accumulator element v of lane l: row 8*(v/4) + 4*(l/32) + v%4, column l%32; quad (a, vq) holds v = 4 vq .. + 3 */
-    auto emit = [&](const gw_part &P, const gw_item &it, int a, int vq, const f32x4 &q0, const f32x4 &q1) {
+    /* accumulator element v of lane l: row 8*(v/4) + 4*(l/32) + v%4, column l%32; quads (a, vq) hold v = 4 vq .. + 3 */
+    auto emit = [&](const gw_part &P, const gw_item &it, int a, int vq, const f32x4 (&q)[NB]) {
         const int row0 = it.mt * TM + 32 * a + 8 * vq + 4 * (lane >> 5), c = lane & 31;
-        if (!T::SCALED && P.h_hi) {
-            /* a wave's two column blocks are the gates and the ups of the same 32 h columns (voxtral_tts_llm.c:346-350) */
-            const vt_h_quad h = vt_silu_mul_quad(q0, q1);
-            const size_t at = (size_t)(row0 + h.row) * P.ldh + it.nt * (TN / 2) + 32 * cw + (c & ~1);
+        if constexpr (!T::SCALED && NB == 2) {
+            if (P.h_hi) {
+                /* a wave's two column blocks are the gates and the ups of the same 32 h columns (voxtral_tts_llm.c:346-350) */
+                const vt_h_quad h = vt_silu_mul_quad(q[0], q[1]);
+                const size_t at = (size_t)(row0 + h.row) * P.ldh + it.nt * (TN / 2) + 32 * cw + (c & ~1);
 #pragma unroll
-            for (int r = 0; r < 2; r++)
-                if (row0 + h.row + r < M) {
-                    *reinterpret_cast<unsigned *>(P.h_hi + at + (size_t)r * P.ldh) = h.hi[r];
-                    *reinterpret_cast<unsigned *>(P.h_lo + at + (size_t)r * P.ldh) = h.lo[r];
-                }
-        } else {
-            const int col = it.nt * TN + 64 * cw + c;
-            gm_store_quad<T>(P.C + (size_t)it.sp * P.plane_stride + col, P.ldc, row0, M, q0, q1, P.row_exp, P.col_exp + col);
+                for (int r = 0; r < 2; r++)
+                    if (row0 + h.row + r < M) {
+                        *reinterpret_cast<unsigned *>(P.h_hi + at + (size_t)r * P.ldh) = h.hi[r];
+                        *reinterpret_cast<unsigned *>(P.h_lo + at + (size_t)r * P.ldh) = h.lo[r];
+                    }
+                return;
+            }
         }
+        const int col = it.nt * TN + 32 * NB * cw + c;
+        gm_store_quad<T, NB>(P.C + (size_t)it.sp * P.plane_stride + col, P.ldc, row0, M, q, P.row_exp, P.col_exp + col);
     };
-    auto quad = [&](int a, int b, int vq) { return f32x4{acc[a][b][4 * vq], acc[a][b][4 * vq + 1], acc[a][b][4 * vq + 2], acc[a][b][4 * vq + 3]}; };
+    auto quads = [&](f32x4 (&q)[NB], int a, int vq) {
+#pragma unroll
+        for (int b = 0; b < NB; b++) q[b] = f32x4{acc[a][b][4 * vq], acc[a][b][4 * vq + 1], acc[a][b][4 * vq + 2], acc[a][b][4 * vq + 3]};
+    };
     auto finish = [&](const gw_item &it) {
         const gw_part &P = list.part[it.part];
+        f32x4 q[NB];
         if constexpr (KW == 1) {
 #pragma unroll
             for (int a = 0; a < MB; a++)
 #pragma unroll
-                for (int vq = 0; vq < 4; vq++) emit(P, it, a, vq, quad(a, 0, vq), quad(a, 1, vq));
+                for (int vq = 0; vq < 4; vq++) { quads(q, a, vq); emit(P, it, a, vq, q); }
         } else {
             /* the two waves of a column block hold the sums over the even and the odd K steps: each parks the half
              * of its quads that the other one finishes */
-            float *park = reinterpret_cast<float *>(lds) + (size_t)wave * (MB * 4 * 256);
-            const float *theirs = reinterpret_cast<const float *>(lds) + (size_t)(wave ^ CW) * (MB * 4 * 256);
-            __syncthreads();
-#pragma unroll
-            for (int a = 0; a < MB; a++)
-#pragma unroll
-                for (int h = 0; h < 2; h++)
-#pragma unroll
-                    for (int b = 0; b < 2; b++)
-                        *reinterpret_cast<f32x4 *>(park + (((a * 2 + h) * 2 + b) * 64 + lane) * 4) = kw == 0 ? quad(a, b, 2 + h) : quad(a, b, h);
+            float *park = reinterpret_cast<float *>(lds) + (size_t)wave * (MB * NB * 2 * 256);
+            const float *theirs = reinterpret_cast<const float *>(lds) + (size_t)(wave ^ CW) * (MB * NB * 2 * 256);
             __syncthreads();
 #pragma unroll
             for (int a = 0; a < MB; a++)
 #pragma unroll
                 for (int h = 0; h < 2; h++) {
-                    f32x4 q[2];
+                    if (kw == 0) quads(q, a, 2 + h); else quads(q, a, h);
 #pragma unroll
-                    for (int b = 0; b < 2; b++) {
-                        const f32x4 o = *reinterpret_cast<const f32x4 *>(theirs + (((a * 2 + h) * 2 + b) * 64 + lane) * 4);
-                        const f32x4 m = kw == 0 ? quad(a, b, h) : quad(a, b, 2 + h);
+                    for (int b = 0; b < NB; b++) *reinterpret_cast<f32x4 *>(park + (((a * 2 + h) * NB + b) * 64 + lane) * 4) = q[b];
+                }
+            __syncthreads();
+#pragma unroll
+            for (int a = 0; a < MB; a++)
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    if (kw == 0) quads(q, a, h); else quads(q, a, 2 + h);
+#pragma unroll
+                    for (int b = 0; b < NB; b++) {
+                        const f32x4 o = *reinterpret_cast<const f32x4 *>(theirs + (((a * 2 + h) * NB + b) * 64 + lane) * 4), m = q[b];
                         q[b] = f32x4{__fadd_rn(m.x, o.x), __fadd_rn(m.y, o.y), __fadd_rn(m.z, o.z), __fadd_rn(m.w, o.w)};
                     }
-                    emit(P, it, a, kw == 0 ? h : 2 + h, q[0], q[1]);
+                    emit(P, it, a, kw == 0 ? h : 2 + h, q);
                 }
         }
     };
@@ -384,8 +392,9 @@ vt_gemm_wide_kernel(gw_list list, const uint16_t *Ahi, const uint16_t *Alo, int 
         }
         if (part >= list.n_parts) break;
         const gw_item nx = gw_item_at<TN, WP>(list, part, id, K);
-        begin(nx);
+        if constexpr (AHEAD == 2) begin(nx);
         finish(it);
+        if constexpr (AHEAD == 1) begin(nx);      /* no registers for them beside the sums */
         __syncthreads();                  /* the next item stages over what this one read */
         it = nx;
     }
@@ -489,7 +498,7 @@ vt_gemm_rows_kernel(gr_plan plan, const uint16_t *Ahi, const uint16_t *Alo, int 
             ra_lo[p] = gm_ldb(l, a_voff + p * a_pass, soff);
         }
     };
-    auto fetch_b_slice = [&](const gr_item &it, gm_weights<WP> &r, int i, int j) {
+    auto fetch_b_slice = [&](const gr_item &it, gm_weights<WP, 2> &r, int i, int j) {
         const int soff = i < it.n ? (it.s0 + wave + NW * i) * 4096 * WP : 0;
         const __amdgpu_buffer_rsrc_t w = __builtin_amdgcn_make_buffer_rsrc((void *)it.w, 0, i < it.n ? 2 * blk_bytes : 0, 0x00020000);
 #pragma unroll
@@ -514,8 +523,8 @@ vt_gemm_rows_kernel(gr_plan plan, const uint16_t *Ahi, const uint16_t *Alo, int 
         }
     };
     f32x16 acc[MB][2];
-    auto mma = [&](const frags &f, const gm_weights<WP> &w, int ks) { gm_multiply<T, MB>(acc, f, w, ks); };
-    gm_weights<WP> b0, b1;
+    auto mma = [&](const frags &f, const gm_weights<WP, 2> &w, int ks) { gm_multiply<T, MB, 2>(acc, f, w, ks); };
+    gm_weights<WP, 2> b0, b1;
     frags f0, f1;
     /* the first requests of an item: the rows of step 0, the weights of steps 0 and 1 */
     auto begin = [&](const gr_item &it) {
@@ -528,7 +537,7 @@ vt_gemm_rows_kernel(gr_plan plan, const uint16_t *Ahi, const uint16_t *Alo, int 
     };
     /* step i: the stage holds its rows, f0 their slice 0; ra holds the rows of step i + 1.  A slice's weight
      * registers are requested again (step i + 2) as soon as the slice has been multiplied. */
-    auto step = [&](const gr_item &it, int i, gm_weights<WP> &cur) {
+    auto step = [&](const gr_item &it, int i, gm_weights<WP, 2> &cur) {
         read_frags(f1, 1);
         mma(f0, cur, 0);
         __builtin_amdgcn_sched_barrier(0);
@@ -601,7 +610,7 @@ vt_gemm_rows_kernel(gr_plan plan, const uint16_t *Ahi, const uint16_t *Alo, int 
                     }
             } else {
                 const int col = it.nt * GR_TN + c;
-                gm_store_quad<T>(P.C + (size_t)it.sp * P.plane_stride + col, P.ldc, row0, M, s[0], s[1], P.row_exp, P.col_exp + col);
+                gm_store_quad<T, 2>(P.C + (size_t)it.sp * P.plane_stride + col, P.ldc, row0, M, s, P.row_exp, P.col_exp + col);
             }
         }
     };

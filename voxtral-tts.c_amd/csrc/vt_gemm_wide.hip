@@ -7,58 +7,64 @@
 /* ---- plans and launches ---------------------------------------------------------------------------- */
 
 /* What a product is expected to take, in us, for the choice between tiles and cuts.  A round of items takes as
- * long as the operands of its steps need to arrive (step_us: a step of the 128-column tile does as much as one of
- * the 256-column tile but moves 1.5 times the bytes) and 1.5 us for sums and stores, but no less than the card's
- * power limit lets the matrix cores of its items run (pflops, executed, padding included: the 128-column tile pays
- * for its bytes here, too); a launch takes 5 us; cut planes are written and read once more.  Measured against every
- * tile and cut count at 65 .. 1531 rows of the backbone's products and 84 .. 8024 of the codec's, the plan taken is
- * 1.8 and 1.0 % behind the fastest on average, at worst 9.7 % (output, 512 rows: 192 items on 256 CUs where 240 are
- * faster) and 17 % (the codec's q|k|v at 212 rows: 192 items, 216 faster). */
+ * long as the operands of its steps need to arrive (step_us: a step of the 128- and 192-column tiles is two K steps, half
+ * of the waves at each) and item_us for sums and stores, but no less than the card's
+ * power limit lets the matrix cores of its items run (pflops, executed, padding included: narrow tiles pay
+ * for their bytes here, too); a launch takes 5 us; cut planes are written and read once more.
+ * The backbone's 192 columns divide 6144 and 3072 into 32 and 16 tiles, so that 1, 2, 4, .. row tiles fill the 256 CUs
+ * where 256-column tiles come in multiples of 192 items: q|k|v / output / down at 700 rows 57.5 / 40.7 / 79.4 -> 51.1 / 37.2 /
+ * 72.5 us, at 1000 75.0 / 53.3 / 104.9 -> 68.5 / 49.2 / 97.0, output / down at 1531 73.3 / 149.4 -> 67.1 / 140.6.
+ * Measured against every tile and cut count at 65 .. 1531 rows of the backbone's products and 84 .. 8024 of the codec's, the plan taken is
+ * 1.0 % behind the fastest on average in both, at worst 11 % (q|k|v at 600 rows, whole 192-column tiles on 224 CUs instead
+ * of 240 cut ones) and 17 % (the codec's q|k|v at 212 rows: 192 items, 216 faster). */
 struct gw_format {
     int products;                         /* matrix instructions per pair of operands */
-    float launch_us, item_us;
-    float step_us[2][2];                  /* [256, 128 columns][96, 128 rows] */
-    float pflops[2];                      /* [256, 128 columns] */
+    float launch_us, item_us, planes;     /* planes: passes over a cut column's planes */
+    float step_us[3][2];                  /* [128, 192, 256 columns][96, 128 rows]; 0: tile not used */
+    float pflops[3];                      /* [128, 192, 256 columns] */
 };
-static const gw_format gw_backbone = {2, 5.0f, 1.5f, {{1.05f, 1.30f}, {1.6f, 2.0f}}, {1.12f, 1.0f}};
-static const gw_format gw_codec = {3, 6.0f, 2.0f, {{2.0f, 2.5f}, {2.0f, 2.6f}}, {1.10f, 0.88f}};
+static const gw_format gw_backbone = {2, 5.0f, 2.8f, 1.45f, {{1.28f, 0.f}, {1.97f, 2.96f}, {1.15f, 1.65f}}, {0.91f, 1.07f, 1.21f}};
+static const gw_format gw_codec = {3, 6.0f, 2.0f, 1.2f, {{2.0f, 2.6f}, {0.f, 0.f}, {2.0f, 2.5f}}, {0.88f, 0.f, 1.10f}};
 
 static float gw_rounds(int items, float item_us, float power_us) {
     const int full = items / g_vt.n_cu, rem = items % g_vt.n_cu;
     return full * fmaxf(item_us, g_vt.n_cu * power_us) + (rem ? fmaxf(item_us, rem * power_us) : 0.f);
 }
 
-static float gw_cost(const gw_format &f, int M, int N, int K, int mb, int cw, int n_main, int cuts, int swiglu) {
-    const int kw = 4 / cw, mt = (M + 32 * mb - 1) / (32 * mb), narrow = cw == 2;
-    const float t_step = f.step_us[narrow][mb - 3];
-    const float tile_us = 2.f * f.products * (32 * mb) * (64 * cw) * (float)K / (f.pflops[narrow] * 1e9f);
-    const int rest = N / (64 * cw) - n_main;
+static float gw_cost(const gw_format &f, int M, int N, int K, int mb, int tn, int n_main, int cuts, int swiglu) {
+    const int kw = tn < 256 ? 2 : 1, mt = (M + 32 * mb - 1) / (32 * mb), w = tn / 64 - 2;
+    const float t_step = f.step_us[w][mb - 3];
+    const float tile_us = 2.f * f.products * (32 * mb) * tn * (float)K / (f.pflops[w] * 1e9f);
+    const int rest = N / tn - n_main;
     float t = f.launch_us + gw_rounds(mt * n_main, (float)((K / 64 + kw - 1) / kw) * t_step + f.item_us, tile_us);
     if (rest) {
         t += gw_rounds(mt * rest * cuts, (float)((K / 64 + cuts * kw - 1) / (cuts * kw)) * t_step + f.item_us, tile_us / cuts);
-        if (cuts > 1 || swiglu) t += 1.2f * cuts * M * (float)(rest * 64 * cw) * 4.f / 4.5e6f + (swiglu ? 4.5f : 0.f);
+        if (cuts > 1 || swiglu) t += f.planes * cuts * M * (float)(rest * tn) * 4.f / 4.5e6f + (swiglu ? 4.5f : 0.f);
     }
     return t;
 }
 
 static vt_gemm_plan gw_plan(const gw_format &f, int M, int N, int K, int swiglu) {
-    vt_gemm_plan best = {0, 1, 0, 1};
+    vt_gemm_plan best = {0, 64, 0, 1};
     float best_cost = 0.f;
     for (int mb = 3; mb <= 4; mb++)
-        for (int cw = 2; cw <= 4; cw += 2) {
-            const int mt = (M + 32 * mb - 1) / (32 * mb), nt = N / (64 * cw);
+        for (int tn = 128; tn <= 256; tn += 64) {
+            /* 192 columns: gates and ups come in blocks of 64, which a wave's 96 columns do not end with */
+            if (N % tn || f.step_us[tn / 64 - 2][mb - 3] == 0.f || (tn == 192 && swiglu)) continue;
+            const int mt = (M + 32 * mb - 1) / (32 * mb), nt = N / tn;
             /* whole tiles: as many as make full rounds over the CUs, or one round fewer, or all */
             const int full = mt * nt / g_vt.n_cu;
             for (int pick = 0; pick < 3; pick++) {
                 int n_main = pick == 2 ? nt : (full - pick) * g_vt.n_cu / mt;
                 if (n_main < 0 || n_main > nt) continue;
+                if (n_main * tn % 128) n_main--;          /* heads of 128 columns are cut or not */
                 for (int cuts = 1; cuts <= VT_MAX_CUTS && cuts <= K / 64; cuts++) {
                     if (n_main == nt && cuts > 1) break;
                     if (swiglu && n_main < nt && cuts == 1) continue;
-                    const float c = gw_cost(f, M, N, K, mb, cw, n_main, cuts, swiglu);
+                    const float c = gw_cost(f, M, N, K, mb, tn, n_main, cuts, swiglu);
                     if (best_cost == 0.f || c < best_cost) {
                         best_cost = c;
-                        best = vt_gemm_plan{mb, cw, n_main * 64 * cw, n_main == nt ? 1 : cuts};
+                        best = vt_gemm_plan{mb, tn, n_main * tn, n_main == nt ? 1 : cuts};
                     }
                 }
             }
@@ -67,7 +73,7 @@ static vt_gemm_plan gw_plan(const gw_format &f, int M, int N, int K, int swiglu)
 }
 
 vt_gemm_plan vt_gemm_frag_plan(int M, int N, int K, int swiglu) {
-    vt_gemm_plan best = {0, 1, 0, 1};
+    vt_gemm_plan best = {0, 64, 0, 1};
     if (vt_gemm_rows_ok(M, N, K)) {
         if (swiglu) {
             best.col0 = N / 64 / g_vt.n_cu * g_vt.n_cu * 64;
@@ -82,36 +88,35 @@ vt_gemm_plan vt_gemm_frag_plan(int M, int N, int K, int swiglu) {
 }
 
 vt_gemm_plan vt_codec_gemm_plan(int M, int N, int K) {
-    if (vt_gemm_rows_ok(M, N, K)) return vt_gemm_plan{0, 1, 0, vt_gemm_rows_cuts(VT_CODEC_ROW_WAVES, N, K, VT_MAX_CUTS)};
+    if (vt_gemm_rows_ok(M, N, K)) return vt_gemm_plan{0, 64, 0, vt_gemm_rows_cuts(VT_CODEC_ROW_WAVES, N, K, VT_MAX_CUTS)};
     return gw_plan(gw_codec, M, N, K, 0);
 }
 
-template <int MB, int CW>
+template <int MB, int CW, int NB>
 static void gw_launch(const gw_list &list, const uint16_t *d_Ahi, const uint16_t *d_Alo, int M, int K) {
     constexpr int LDS = 2 * (4 / CW) * 2 * 32 * MB * GM_STAGE_ROW;
     static int attr_set = 0;
     if (!attr_set) {
-        if (vt_check(hipFuncSetAttribute((const void *)vt_gemm_wide_kernel<gm_bf16, MB, CW>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS), "product LDS size"))
+        if (vt_check(hipFuncSetAttribute((const void *)vt_gemm_wide_kernel<gm_bf16, MB, CW, NB>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS), "product LDS size"))
             return;
         attr_set = 1;
     }
     const int items = list.m_tiles * list.part[0].n_tiles * list.part[0].splits;      /* every workgroup takes an item of the first part */
-    hipLaunchKernelGGL((vt_gemm_wide_kernel<gm_bf16, MB, CW>), dim3(items < g_vt.n_cu ? items : g_vt.n_cu), dim3(256), LDS, g_vt.stream, list, d_Ahi, d_Alo, M, K);
+    hipLaunchKernelGGL((vt_gemm_wide_kernel<gm_bf16, MB, CW, NB>), dim3(items < g_vt.n_cu ? items : g_vt.n_cu), dim3(256), LDS, g_vt.stream, list, d_Ahi, d_Alo, M, K);
 }
 
 static void gw_run(const vt_gemm_plan &pl, gw_part whole, gw_part cut, const uint16_t *d_Ahi, const uint16_t *d_Alo, int M, int N, int K) {
     gw_list list = {};
     list.m_tiles = (M + 32 * pl.mb - 1) / (32 * pl.mb);
-    whole.n_tiles = pl.col0 / (64 * pl.cw);
+    whole.n_tiles = pl.col0 / pl.tn;
     whole.splits = 1;
-    cut.n_tiles = (N - pl.col0) / (64 * pl.cw);
+    cut.n_tiles = (N - pl.col0) / pl.tn;
     cut.splits = pl.cuts;
     if (whole.n_tiles) list.part[list.n_parts++] = whole;
     if (cut.n_tiles) list.part[list.n_parts++] = cut;
-    if (pl.mb == 4 && pl.cw == 4) gw_launch<4, 4>(list, d_Ahi, d_Alo, M, K);
-    else if (pl.mb == 4) gw_launch<4, 2>(list, d_Ahi, d_Alo, M, K);
-    else if (pl.cw == 4) gw_launch<3, 4>(list, d_Ahi, d_Alo, M, K);
-    else gw_launch<3, 2>(list, d_Ahi, d_Alo, M, K);
+    static void (*const launch[2][3])(const gw_list &, const uint16_t *, const uint16_t *, int, int) = {
+        {gw_launch<3, 2, 2>, gw_launch<3, 2, 3>, gw_launch<3, 4, 2>}, {NULL, gw_launch<4, 2, 3>, gw_launch<4, 4, 2>}};
+    launch[pl.mb - 3][pl.tn / 64 - 2](list, d_Ahi, d_Alo, M, K);
 }
 
 void vt_launch_gemm_frag(float *d_C, int ldc, size_t plane_stride, const uint16_t *d_Ahi, const uint16_t *d_Alo,
