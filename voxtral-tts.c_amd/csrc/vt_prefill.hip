@@ -16,40 +16,41 @@
 #include <math.h>
 
 
-/* ---- causal attention, 16 queries x 32 keys per matrix-core tile ----------------
+/* ---- causal attention, 32 query rows x 32 keys per matrix-core tile ----------------
  * (tts_causal_attention, voxtral_tts_kernels.c:403-465, for head_dim 128 and four
  * query heads per KV head.)
  *
- * Workgroup = (KV head, HPW of its 4 query heads, block of 16 queries), HPW*NSPLIT
- * waves: wave = (query head, key-tile residue).  The waves of one residue share 32-key
- * K and V tiles in LDS, as (hi, lo) planes laid out as the matrix instructions want them: K as
- * [key][dim] (a lane's operand is 8 consecutive dims of a key), V transposed as [dim][lane
- * group][8 key slots] (a lane's operand is the 8 keys of its group for one dim).  The planes are
- * made once per layer, by vt_kv_image_kernel, in exactly this layout; a workgroup copies a tile's
- * 37 KB image into its LDS (converting in here cost every step 1450 of its 5900 cycles, and every
- * tile is used by 34 workgroups on average).  Both products run on the bf16 matrix cores
- * (v_mfma_f32_16x16x32_bf16) with every fp32 operand split in (hi, lo) bf16 planes as in
- * the projections: a b = hi_a hi_b + hi_a lo_b + lo_a hi_b, 16 mantissa bits per operand,
- * fp32 accumulation; three such instructions take 3/16 of the time of the fp32 ones they
- * replace.  Scores are computed transposed, S^T = K Q^T, so that a lane owns one query:
- * lane l holds query l%16 and the keys 4*(l/16) + v of each 16-key block in accumulator
- * element v.  The softmax state is then per lane (two exchanges across the four lane
- * groups per tile), and the eight probabilities a lane holds are exactly its share of the
- * reduction index of the second product O^T = V^T P^T (the k order inside a matrix
- * instruction is free as long as both operands agree: slot j of lane group g stands for
- * key 16*(j/4) + 4*g + j%4).  Residues are merged through LDS at the end.
- * 16-query blocks give 32 blocks per KV head at 512 queries: with HPW = 2 that is 512
- * workgroups whose work grows with the block index (causal), enough to keep 256 CUs
- * busy when long and short blocks follow each other. */
-#define PA_QT 16                  /* queries per workgroup */
-#define PA_KROW 272               /* bytes per key of a K plane: 128 bf16 + 16 (16-byte reads over 16 keys cover all banks) */
-#define PA_VROW 80                /* bytes per dim of a V plane: 4 lane groups x 8 key slots + 16 */
-/* Dim d of V is row d of its plane: the 16 lanes that a 16-byte LDS read serves together (dims 16 b + li of
- * a block) then start 20 li dwords apart, which are 16 different groups of four banks.  (While the tiles were
- * converted in here the rows were skewed to keep the transposed writes free of bank conflicts.) */
-#define PA_KPLANE (32 * PA_KROW)
-#define PA_VPLANE (VT_HEAD_DIM * PA_VROW)
-#define PA_TILE_BYTES (2 * PA_KPLANE + 2 * PA_VPLANE)
+ * Workgroup = (KV head, block of QB queries of its four query heads), eight waves.  A wave holds 32 query rows: QB = 32
+ * queries of one head, or QB = 16 queries of two heads; the NS = 2 or 4 waves with the same rows take the key
+ * tiles in turn (tile modulo NS) and merge at the end.  The waves of a residue share a tile of 32 keys in LDS.  Both
+ * products run on the bf16 matrix cores (v_mfma_f32_32x32x16_bf16) with every fp32 operand split in (hi, lo) bf16
+ * planes as in the projections: a b = hi_a hi_b + hi_a lo_b + lo_a hi_b, 16 mantissa bits per operand, fp32 accumulation.
+ * Scores are computed transposed, S^T = K Q^T, so that a lane owns one query row: lane l holds row l%32 and the keys
+ * 8*(v/4) + 4*(l/32) + v%4 in accumulator element v.  The softmax state is then per lane (one exchange between the
+ * two lane groups per tile), and the sixteen probabilities a lane holds are exactly its share of the reduction index
+ * of the second product O^T = V^T P^T (the k order inside a matrix instruction is free as long as both operands
+ * agree: slot j of lane group g in the instruction of key half t stands for key 16 t + 8*(j/4) + 4 g + j%4).
+ *
+ * A tile of K and V is 32 KB of operands in the order in which the instructions take them (1 KB per instruction and
+ * plane, lane l at byte 16 l), made once per layer by vt_kv_image_kernel; a workgroup copies tiles from
+ * memory straight into LDS (buffer loads to LDS, no registers).  Two arrays, not two halves of one: the compiler then
+ * knows that reading one does not have to wait for what arrives in the other.
+ *
+ * What bounds it: 48 matrix instructions of 32 cycles per wave and tile beside 32 KB of LDS reads and about 250 vector
+ * instructions, two waves per SIMD: 2.0 to 2.3 us per NS tiles, 1.28 of them matrix instructions at 2.4 GHz; and
+ * 7 to 9 us in front and behind (queries 2.1, their planes 1.5, merge and stores 2.5: each of them code that is run once and
+ * comes from memory).  us per launch inside a prefill of 37 / 226 / 512 / 1531 rows: 7.7 / 12.2 / 17.8 /
+ * 63.2, where 16 queries per wave on 16 x 16 x 32 instructions, four waves and tiles copied through registers took 9.0 / 15.8 /
+ * 24.5 / 125.5. */
+/* Queries per workgroup: 16 as long as that gives the CUs more to do at once (twice the workgroups, each half as many
+ * rounds of tiles), 32 from where every CU is busy either way and the tiles are copied half as often.  us per launch
+ * at 37 / 226 / 512 / 1000 / 1531 / 3000 rows, 16: 7.5 / 10.5 / 16.4 / 34.4 / 70.1 / 236.7, 32: 9.0 / 14.3 / 22.4 / 39.5 /
+ * 63.0 / 210.5. */
+#define PA_SHORT_QT 16
+#define PA_LONG_QT 32
+#define PA_SHORT_ROWS 1200
+#define PA_PLANE 8192             /* bytes of a plane of a tile: 8 slices of K, 4 dim blocks x 2 key halves of V, 1 KB each */
+#define PA_TILE_BYTES (4 * PA_PLANE)                  /* K hi, K lo, V hi, V lo */
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
@@ -64,18 +65,18 @@ __device__ __forceinline__ void pa_planes8(const f32x4 &a, const f32x4 &b, bf16x
     lo = __builtin_bit_cast(bf16x8, u32x4{l0, l1, l2, l3});
 }
 
-/* K and V of one layer as the attention wants them in its LDS: per (kv head, tile of 32 keys) the image
- * [K hi plane | K lo plane | V hi plane | V lo plane] described above, img[kvh][tile], so that the attention
- * copies a tile instead of converting it (every tile is read by all later query blocks of 4 heads: at 512
- * rows 34 times on average).  Workgroup = (tile, kv head), 128 threads for K and 128 for V; thread (sg, cg) owns the dims
- * 4*cg .. + 4 of the 8 keys that lane group sg meets in the second product (slot j: key 16*(j/4) + 4*sg +
- * j%4), so that the transposed V write is one 16-byte store per dim and plane.
+/* K and V of one layer as the attention wants them in its LDS: per (kv head, tile of 32 keys) the operands described
+ * above, img[kvh][tile].  K: slice ks of lane l = key l%32, dims 16 ks + 8 (l/32) .. + 8; V: dim block b and key half t of
+ * lane l = dim 32 b + l%32, keys 16 t + 4 (l/32) + 0..3 and the four 8 further on.  Workgroup = (tile, kv head), 128
+ * threads for K and 128 for V; thread (sg, cg) owns the dims 4*cg .. + 4 of the 8 keys that lane group sg % 2 meets in
+ * key half sg / 2, so that the transposed V write is one 16-byte store per dim and plane.
  * Rows [start_pos, start_pos + S) come from the q|k|v product when qkv != NULL: the sum of `planes`
  * split-K planes (`plane_stride` floats apart, fixed order; only the columns from col0 on are cut, a multiple
  * of 128), k rotated (adjacent pairs,
  * voxtral_tts_kernels.c:616-634; the table holds (cos, sin) per pair), and are appended to the cache on the
  * way (voxtral_tts_llm.c:317-324).  Earlier rows come from the cache; rows from kv_rows on are zeros (their
  * keys are masked).  qkv == NULL: all rows are in the cache (rope is not read). */
+__device__ __forceinline__ int pa_key(int sg, int i) { return 16 * (sg >> 1) + 4 * (sg & 1) + 8 * (i >> 2) + (i & 3); }
 __global__ void __launch_bounds__(256)
 vt_kv_image_kernel(unsigned char *img, int img_tiles, const float *qkv, int col0, int planes, size_t plane_stride,
                    float *kc, float *vc, const float *rope, int start_pos, int kv_rows) {
@@ -94,7 +95,7 @@ vt_kv_image_kernel(unsigned char *img, int img_tiles, const float *qkv, int col0
         f32x4 cs[8];
 #pragma unroll
         for (int i = 0; i < 8; i++) {
-            const int row = 16 * (i >> 2) + 4 * sg + (i & 3);
+            const int row = pa_key(sg, i);
             r8[i] = *reinterpret_cast<const f32x4 *>(src + (size_t)row * VT_QKV_DIM);
             cs[i] = is_v ? zero : *reinterpret_cast<const f32x4 *>(rope + (size_t)(tile * 32 + row) * VT_HEAD_DIM + 4 * cg);
         }
@@ -102,7 +103,7 @@ vt_kv_image_kernel(unsigned char *img, int img_tiles, const float *qkv, int col0
             f32x4 w[8];
 #pragma unroll
             for (int i = 0; i < 8; i++)
-                w[i] = *reinterpret_cast<const f32x4 *>(src + p * plane_stride + (size_t)(16 * (i >> 2) + 4 * sg + (i & 3)) * VT_QKV_DIM);
+                w[i] = *reinterpret_cast<const f32x4 *>(src + p * plane_stride + (size_t)pa_key(sg, i) * VT_QKV_DIM);
 #pragma unroll
             for (int i = 0; i < 8; i++) {
                 r8[i].x = __fadd_rn(r8[i].x, w[i].x); r8[i].y = __fadd_rn(r8[i].y, w[i].y);
@@ -111,7 +112,7 @@ vt_kv_image_kernel(unsigned char *img, int img_tiles, const float *qkv, int col0
         }
 #pragma unroll
         for (int i = 0; i < 8; i++) {
-            const int r = tile * 32 + 16 * (i >> 2) + 4 * sg + (i & 3);
+            const int r = tile * 32 + pa_key(sg, i);
             if (!is_v) {
                 const f32x4 k = r8[i], c = cs[i];
                 r8[i] = f32x4{__fsub_rn(__fmul_rn(k.x, c.x), __fmul_rn(k.y, c.y)), __fadd_rn(__fmul_rn(k.x, c.y), __fmul_rn(k.y, c.x)),
@@ -122,7 +123,7 @@ vt_kv_image_kernel(unsigned char *img, int img_tiles, const float *qkv, int col0
     } else {
 #pragma unroll
         for (int i = 0; i < 8; i++) {
-            const int r = tile * 32 + 16 * (i >> 2) + 4 * sg + (i & 3);
+            const int r = tile * 32 + pa_key(sg, i);
             if (r >= kv_rows) {
                 r8[i] = zero;
             } else if (qkv && r >= start_pos) {
@@ -144,305 +145,293 @@ vt_kv_image_kernel(unsigned char *img, int img_tiles, const float *qkv, int col0
             }
         }
     }
-    unsigned char *Kt = img + ((size_t)kvh * img_tiles + tile) * PA_TILE_BYTES, *Vt = Kt + 2 * PA_KPLANE;
+    unsigned char *Kt = img + ((size_t)kvh * img_tiles + tile) * PA_TILE_BYTES, *Vt = Kt + 2 * PA_PLANE;
     if (!is_v) {
 #pragma unroll
         for (int i = 0; i < 8; i++) {
-            const int row = 16 * (i >> 2) + 4 * sg + (i & 3);
             u32x2 h, l;
             vt_split_planes4(r8[i].x, r8[i].y, r8[i].z, r8[i].w, h, l);
-            *reinterpret_cast<u32x2 *>(Kt + row * PA_KROW + 8 * cg) = h;
-            *reinterpret_cast<u32x2 *>(Kt + PA_KPLANE + row * PA_KROW + 8 * cg) = l;
+            unsigned char *at = Kt + (cg >> 2) * 1024 + ((cg >> 1) & 1) * 512 + pa_key(sg, i) * 16 + (cg & 1) * 8;
+            *reinterpret_cast<u32x2 *>(at) = h;
+            *reinterpret_cast<u32x2 *>(at + PA_PLANE) = l;
         }
     } else {
 #pragma unroll
         for (int d = 0; d < 4; d++) {
             bf16x8 h, l;
             pa_planes8(f32x4{r8[0][d], r8[1][d], r8[2][d], r8[3][d]}, f32x4{r8[4][d], r8[5][d], r8[6][d], r8[7][d]}, h, l);
-            *reinterpret_cast<bf16x8 *>(Vt + (4 * cg + d) * PA_VROW + 16 * sg) = h;
-            *reinterpret_cast<bf16x8 *>(Vt + PA_VPLANE + (4 * cg + d) * PA_VROW + 16 * sg) = l;
+            unsigned char *at = Vt + ((cg >> 3) * 2 + (sg >> 1)) * 1024 + ((sg & 1) * 32 + (4 * cg + d) % 32) * 16;
+            *reinterpret_cast<bf16x8 *>(at) = h;
+            *reinterpret_cast<bf16x8 *>(at + PA_PLANE) = l;
         }
     }
 }
 
-template <int NSPLIT, int HPW>
-__global__ void __launch_bounds__(64 * HPW * NSPLIT)
+typedef float pa_f32x16 __attribute__((ext_vector_type(16)));
+__device__ __forceinline__ pa_f32x16 pa_mfma(const bf16x8 &a, const bf16x8 &b, const pa_f32x16 &c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+/* the larger of this lane's value and that of the lane 32 away */
+__device__ __forceinline__ float pa_max_halves(float x) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
+template <int QB>
+__global__ void __launch_bounds__(512)
 vt_prefill_attention_kernel(float *out, uint16_t *out_hi, uint16_t *out_lo, const float *Q,
                             int q_stride, int q_col0, int q_planes, size_t q_plane_stride, const float *rope,
                             const unsigned char *img, int img_tiles, int S, int start_pos, float scale) {
-    extern __shared__ __attribute__((aligned(16))) unsigned char pa_lds[];
-    constexpr int GT = 64 * HPW;                         /* threads of a residue group */
-    constexpr int NCH = PA_TILE_BYTES / 16;              /* 16-byte chunks of a tile image */
-    constexpr int NLD = (NCH + GT - 1) / GT;             /* chunks per thread and tile */
-    const int kvh = (int)blockIdx.x / (4 / HPW), hsub = (int)blockIdx.x % (4 / HPW);
-    /* The last query block has the most keys.  Workgroups are handed to the CUs in launch order, one per
-     * CU and then a second one each: the first half of the launch takes the long blocks in descending
-     * order, the second half the short ones in ascending order, so that every CU gets a long block and
-     * the short one that makes up the same total. */
-    const int ny = (int)gridDim.y, half = (ny + 1) / 2;
-    const int qt = (int)blockIdx.y < half ? ny - 1 - (int)blockIdx.y : (int)blockIdx.y - half;
-    const int t = (int)threadIdx.x, lane = t & 63, wave = t >> 6;
-    const int hq = wave % HPW, pz = wave / HPW;
-    const int tl = hq * 64 + lane;                       /* thread index inside the residue group */
-    const int g = lane >> 4, li = lane & 15;
-    const int q0 = qt * PA_QT;
-    const int my_q = q0 + li;
-    const int head = kvh * 4 + hsub * HPW + hq;
-    if (head * VT_HEAD_DIM < q_col0) q_planes = 1;       /* a head whose columns are not cut */
-    unsigned char *Kt = pa_lds + (size_t)pz * PA_TILE_BYTES, *Vt = Kt + 2 * PA_KPLANE;   /* hi plane, then lo */
-
-    /* this lane's query as the B operand of K Q^T: dims 8*g + 32*ks .. + 8 for K step ks, both planes */
-    bf16x8 qhi[4], qlo[4];
-    {
-        /* Q as it is, or (rope != NULL) the raw product: the sum of q_planes split-K planes, rotated here
-         * (adjacent pairs, voxtral_tts_kernels.c:616-634; the table holds (cos, sin) per pair).  All
-         * requests of a plane go out before the first value is used: inside a prefill every one of them
-         * goes to memory, and one after the other they were 7 us of a 27 us launch. */
-        const int qrow = my_q < S ? my_q : S - 1;
-        const float *qp = Q + (size_t)qrow * q_stride + head * VT_HEAD_DIM + 8 * g;
-        f32x4 qa[4], qb[4];
-#pragma unroll
-        for (int ks = 0; ks < 4; ks++) {
-            qa[ks] = reinterpret_cast<const f32x4 *>(qp + 32 * ks)[0];
-            qb[ks] = reinterpret_cast<const f32x4 *>(qp + 32 * ks)[1];
-        }
-        if (rope) {
-            const float *cs = rope + (size_t)(start_pos + qrow) * VT_HEAD_DIM + 8 * g;
-            f32x4 c0[4], c1[4];
-#pragma unroll
-            for (int ks = 0; ks < 4; ks++) {
-                c0[ks] = reinterpret_cast<const f32x4 *>(cs + 32 * ks)[0];
-                c1[ks] = reinterpret_cast<const f32x4 *>(cs + 32 * ks)[1];
-            }
-            for (int p = 1; p < q_planes; p++) {
-                f32x4 a2[4], b2[4];
-#pragma unroll
-                for (int ks = 0; ks < 4; ks++) {
-                    a2[ks] = reinterpret_cast<const f32x4 *>(qp + p * q_plane_stride + 32 * ks)[0];
-                    b2[ks] = reinterpret_cast<const f32x4 *>(qp + p * q_plane_stride + 32 * ks)[1];
-                }
-#pragma unroll
-                for (int ks = 0; ks < 4; ks++) {
-                    f32x4 &a = qa[ks], &b = qb[ks];
-                    a.x = __fadd_rn(a.x, a2[ks].x); a.y = __fadd_rn(a.y, a2[ks].y); a.z = __fadd_rn(a.z, a2[ks].z); a.w = __fadd_rn(a.w, a2[ks].w);
-                    b.x = __fadd_rn(b.x, b2[ks].x); b.y = __fadd_rn(b.y, b2[ks].y); b.z = __fadd_rn(b.z, b2[ks].z); b.w = __fadd_rn(b.w, b2[ks].w);
-                }
-            }
-#pragma unroll
-            for (int ks = 0; ks < 4; ks++) {
-                const f32x4 a = qa[ks], b = qb[ks];
-                qa[ks] = f32x4{__fsub_rn(__fmul_rn(a.x, c0[ks].x), __fmul_rn(a.y, c0[ks].y)), __fadd_rn(__fmul_rn(a.x, c0[ks].y), __fmul_rn(a.y, c0[ks].x)),
-                               __fsub_rn(__fmul_rn(a.z, c0[ks].z), __fmul_rn(a.w, c0[ks].w)), __fadd_rn(__fmul_rn(a.z, c0[ks].w), __fmul_rn(a.w, c0[ks].z))};
-                qb[ks] = f32x4{__fsub_rn(__fmul_rn(b.x, c1[ks].x), __fmul_rn(b.y, c1[ks].y)), __fadd_rn(__fmul_rn(b.x, c1[ks].y), __fmul_rn(b.y, c1[ks].x)),
-                               __fsub_rn(__fmul_rn(b.z, c1[ks].z), __fmul_rn(b.w, c1[ks].w)), __fadd_rn(__fmul_rn(b.z, c1[ks].w), __fmul_rn(b.w, c1[ks].z))};
-            }
-        }
-#pragma unroll
-        for (int ks = 0; ks < 4; ks++) pa_planes8(qa[ks], qb[ks], qhi[ks], qlo[ks]);
-    }
-    f32x4 o[8];
-#pragma unroll
-    for (int b = 0; b < 8; b++) o[b] = f32x4{0.f, 0.f, 0.f, 0.f};
-    float m = -1e30f, lsum = 0.f;
-
-    const int last_q = (q0 + PA_QT - 1 < S ? q0 + PA_QT - 1 : S - 1) + start_pos;
+    constexpr int HW = QB / 8, NS = 8 / HW;              /* waves of a residue, residues */
+    /* QB 32: a tile of each residue of the even and of the odd steps; QB 16: K and V of a tile of each residue */
+    __shared__ __attribute__((aligned(16))) unsigned char pa_a[65536], pa_b[65536];
+    __shared__ f32x2 pa_ml[8][64];
+    const int kvh = (int)blockIdx.x;
+    const int qt = (int)gridDim.y - 1 - (int)blockIdx.y;         /* the blocks with the most keys first */
+    const int t = (int)threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int hq = wave % HW, pz = wave / HW;
+    const int g = lane >> 5, li = lane & 31;
+    const int q0 = qt * QB;
+    const int my_q = q0 + li % QB;
+    const int last_q = (q0 + QB - 1 < S ? q0 + QB - 1 : S - 1) + start_pos;
     const int ntiles = last_q / 32 + 1;                  /* key tiles 0 .. ntiles-1 are visible */
-    const int nsteps = (ntiles + NSPLIT - 1) / NSPLIT;
+    const int nsteps = (ntiles + NS - 1) / NS;
 
-    /* staging: a tile arrives as the image vt_kv_image_kernel made of it, which is what the LDS holds:
-     * the threads of a residue group copy its 16-byte chunks tl, tl + GT, ...  Buffer loads: the tile as the
-     * scalar offset, the thread's chunk as a vector offset that never changes (no 64-bit address arithmetic
-     * per load); the chunks past the end of a tile belong to nobody and are never stored. */
-    u32x4 rt[NLD];
+    /* the waves of a residue copy KB kilobytes of its tile, from `from` of the tile on, 1 KB per wave and request; a tile
+     * past the last visible one lies beyond the descriptor's end: zeros, which nobody reads */
     const __amdgpu_buffer_rsrc_t t_rs = __builtin_amdgcn_make_buffer_rsrc(
-        (void *)(img + (size_t)kvh * img_tiles * PA_TILE_BYTES), 0, img_tiles * PA_TILE_BYTES, 0x00020000);
-    int voff[NLD];
+        (void *)(img + (size_t)kvh * img_tiles * PA_TILE_BYTES), 0, ntiles * PA_TILE_BYTES, 0x00020000);
+    constexpr int KB = QB == 32 ? 32 : 16;
+    auto fetch = [&](unsigned char *buf, int step, int from) {
+        const int soff = (step * NS + pz) * PA_TILE_BYTES + from;
 #pragma unroll
-    for (int i = 0; i < NLD; i++) voff[i] = 16 * (tl + GT * i < NCH ? tl + GT * i : NCH - 1);
-    /* A tile is requested in four parts, dealt out over the step: a wave's requests are accepted at the
-     * pace at which the CU's address unit works them off (16 cycles per 1 KB request, all waves of the CU
-     * together), and all of them in a row hold the wave's own matrix instructions up behind them. */
-    auto fetch_part = [&](int tile, int part) {
-        const int soff = __builtin_amdgcn_readfirstlane(tile) * PA_TILE_BYTES;
-#pragma unroll
-        for (int i = (part * NLD) / 4; i < ((part + 1) * NLD) / 4; i++)
-            rt[i] = __builtin_amdgcn_raw_buffer_load_b128(t_rs, voff[i], soff, 0);
+        for (int i = 0; i < KB / HW; i++)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(t_rs, (__attribute__((address_space(3))) void *)(buf + pz * KB * 1024 + (i * HW + hq) * 1024), 16,
+                                                     (i * HW + hq) * 1024 + lane * 16, soff, 0, 0);
     };
-    auto fetch = [&](int tile) {
-#pragma unroll
-        for (int part = 0; part < 4; part++) fetch_part(tile, part);
-    };
-    /* Every request of the loop below is unconditional (a tile index beyond the last visible one
-     * is clamped: that tile is fetched again, out of the L2, and never stored): behind a
-     * conditional request the compiler waits for all outstanding loads before the next use of
-     * anything loaded, here the query registers, i.e. before the products of every step. */
-    fetch(pz < ntiles ? pz : ntiles - 1);
+    fetch(pa_a, 0, 0);
 
-    /* The workgroups of one blockIdx.x run on one XCD and walk the same K and V rows, tile by tile, at the
-     * same pace: left alone, every tile is a miss in that XCD's L2 for all of them at the moment they need
-     * it, and each step pays the full memory latency.  So they first touch all the rows between them, one
-     * 128-byte line per lane and request (K and V rows are 4 lines each), which starts every line on its way
-     * into the L2 at once.  The values are dropped at the end of the kernel. */
-    unsigned warm[4];
-    {   /* (behind the query and the first tile: a wave's loads return in order, and these go all the way to memory) */
-        const int n_lines = ((start_pos + S + 31) / 32) * (PA_TILE_BYTES / 128), stride = (int)(gridDim.y * blockDim.x);
-        const unsigned char *mine = img + (size_t)kvh * img_tiles * PA_TILE_BYTES;
+    /* The queries of the four heads, QB rows x 512 columns: Q as it is, or (rope != NULL) the raw product: the sum of
+     * q_planes split-K planes, rotated here (adjacent pairs, voxtral_tts_kernels.c:616-634; the table holds (cos, sin)
+     * per pair).  Fetched once per workgroup, whole 128-byte lines per eight lanes, and handed to the waves through LDS as
+     * the B operands of K Q^T: lane l holds row l%32, dims 16*ks + 8*(l/32) .. + 8 in slice ks.  (A wave fetching its
+     * own operands touches 64 pieces of 16 bytes per request: 10 us of a launch.) */
+    bf16x8 qhi[8], qlo[8];
+    {
+        constexpr int NR = QB / 8, N = 2 * NR;                               /* row groups of 8, quads per thread */
+        const int qh = wave >> 1, r = lane >> 3, qd = lane & 7;              /* wave w: columns 64 w .. + 64 */
+        const int planes = rope && (kvh * 4 + qh) * VT_HEAD_DIM >= q_col0 ? q_planes : 1;       /* a head whose columns are not cut has one */
+        const float *qp = Q + (kvh * 4 + qh) * VT_HEAD_DIM + (wave & 1) * 64 + 4 * qd;
+        size_t row[NR];
+        f32x4 a[N], c[N];
 #pragma unroll
-        for (int k = 0; k < 4; k++) {
-            int j = (int)blockIdx.y * (int)blockDim.x + t + k * stride;
-            j = j < n_lines ? j : n_lines - 1;
-            warm[k] = *reinterpret_cast<const unsigned *>(mine + (size_t)j * 128);
-        }
-    }
-
-    for (int step = 0; step < nsteps; step++) {
-        const int tile = step * NSPLIT + pz;
-        const bool valid = tile < ntiles;
-        __syncthreads();
-        if (valid) {
+        for (int i = 0; i < NR; i++) row[i] = (size_t)min(q0 + 8 * i + r, S - 1);
 #pragma unroll
-            for (int i = 0; i < NLD; i++)
-                if (GT * (i + 1) <= NCH || tl + GT * i < NCH) *reinterpret_cast<u32x4 *>(Kt + 16 * (tl + GT * i)) = rt[i];
-        }
-        __syncthreads();
-        const int nxt = tile + NSPLIT < ntiles ? tile + NSPLIT : ntiles - 1;
-        fetch_part(nxt, 0);
-        __builtin_amdgcn_sched_barrier(0);
-        if (!valid) {
-            fetch_part(nxt, 1); fetch_part(nxt, 2); fetch_part(nxt, 3);
-            continue;
-        }
-
-        /* S^T = K Q^T: K step ks pairs the dims 8*g + 32*ks .. + 8 of key 16*kb + li and of the query */
-        f32x4 s[2];
+        for (int i = 0; i < N; i++) a[i] = *reinterpret_cast<const f32x4 *>(qp + row[i % NR] * q_stride + 32 * (i / NR));
+        if (rope) {
 #pragma unroll
-        for (int kb = 0; kb < 2; kb++) {
-            s[kb] = f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int i = 0; i < N; i++)
+                c[i] = *reinterpret_cast<const f32x4 *>(rope + (start_pos + row[i % NR]) * VT_HEAD_DIM + (wave & 1) * 64 + 32 * (i / NR) + 4 * qd);
+            for (int p = 1; p < planes; p++) {
+                f32x4 b[N];
 #pragma unroll
-            for (int ks = 0; ks < 4; ks++) {
-                const unsigned char *kp = Kt + (16 * kb + li) * PA_KROW + 16 * g + 64 * ks;
-                const bf16x8 khi = *reinterpret_cast<const bf16x8 *>(kp);
-                const bf16x8 klo = *reinterpret_cast<const bf16x8 *>(kp + PA_KPLANE);
-                s[kb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(klo, qhi[ks], s[kb], 0, 0, 0);
-                s[kb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(khi, qlo[ks], s[kb], 0, 0, 0);
-                s[kb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(khi, qhi[ks], s[kb], 0, 0, 0);
+                for (int i = 0; i < N; i++) b[i] = *reinterpret_cast<const f32x4 *>(qp + p * q_plane_stride + row[i % NR] * q_stride + 32 * (i / NR));
+#pragma unroll
+                for (int i = 0; i < N; i++) {
+                    a[i].x = __fadd_rn(a[i].x, b[i].x); a[i].y = __fadd_rn(a[i].y, b[i].y);
+                    a[i].z = __fadd_rn(a[i].z, b[i].z); a[i].w = __fadd_rn(a[i].w, b[i].w);
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < N; i++) {
+                const f32x4 q = a[i], k = c[i];
+                a[i] = f32x4{__fsub_rn(__fmul_rn(q.x, k.x), __fmul_rn(q.y, k.y)), __fadd_rn(__fmul_rn(q.x, k.y), __fmul_rn(q.y, k.x)),
+                             __fsub_rn(__fmul_rn(q.z, k.z), __fmul_rn(q.w, k.w)), __fadd_rn(__fmul_rn(q.z, k.w), __fmul_rn(q.w, k.z))};
             }
         }
-        __builtin_amdgcn_sched_barrier(0);
-        fetch_part(nxt, 1);
-        __builtin_amdgcn_sched_barrier(0);
-        /* online softmax for this lane's query; element v of block kb is key 16*kb + 4*g + v */
-        const int qpos = start_pos + my_q;
+#pragma unroll
+        for (int i = 0; i < N; i++) {
+            u32x2 h, l;
+            vt_split_planes4(a[i].x, a[i].y, a[i].z, a[i].w, h, l);
+            /* dims 64 (w%2) + 32 (i/NR) + 4 qd: slice 4 (w%2) + 2 (i/NR) + qd/4, lane group (qd/2)%2, half qd%2 of its 16 bytes */
+            const int col = 8 * (i % NR) + r + (QB == 16 ? 16 * (qh & 1) : 0), grp = QB == 16 ? qh >> 1 : qh;
+            unsigned char *at = pa_b + grp * 16384 + (4 * (wave & 1) + 2 * (i / NR) + (qd >> 2)) * 1024 + ((qd >> 1 & 1) * 32 + col) * 16 + (qd & 1) * 8;
+            *reinterpret_cast<u32x2 *>(at) = h;
+            *reinterpret_cast<u32x2 *>(at + PA_PLANE) = l;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int ks = 0; ks < 8; ks++) {
+            qhi[ks] = *reinterpret_cast<const bf16x8 *>(pa_b + hq * 16384 + ks * 1024 + lane * 16);
+            qlo[ks] = *reinterpret_cast<const bf16x8 *>(pa_b + hq * 16384 + PA_PLANE + ks * 1024 + lane * 16);
+        }
+    }
+    pa_f32x16 o[4];
+#pragma unroll
+    for (int b = 0; b < 4; b++)
+#pragma unroll
+        for (int v = 0; v < 16; v++) o[b][v] = 0.f;
+    /* scores in units of log2: exp2 of a difference is the exponential */
+    const float to_log2 = __fmul_rn(scale, 1.44269504f);
+    float m = -1e30f, lsum = 0.f;
+    const int qpos = start_pos + my_q;
+
+    pa_f32x16 s;
+    auto scores = [&](const unsigned char *Kt) {         /* S^T = K Q^T */
+#pragma unroll
+        for (int v = 0; v < 16; v++) s[v] = 0.f;
+#pragma unroll
+        for (int ks = 0; ks < 8; ks++) {
+            const bf16x8 khi = *reinterpret_cast<const bf16x8 *>(Kt + lane * 16 + 1024 * ks);
+            const bf16x8 klo = *reinterpret_cast<const bf16x8 *>(Kt + lane * 16 + PA_PLANE + 1024 * ks);
+            s = pa_mfma(klo, qhi[ks], s);
+            s = pa_mfma(khi, qlo[ks], s);
+            s = pa_mfma(khi, qhi[ks], s);
+        }
+    };
+    auto weigh = [&](const unsigned char *Vt, int tile) {
+        /* online softmax for this lane's query row; element v is key 8*(v/4) + 4*g + v%4.  A score that is no number counts
+         * as masked. */
         float mx = -1e30f;
 #pragma unroll
-        for (int kb = 0; kb < 2; kb++)
+        for (int v = 0; v < 16; v++) s[v] = fmaxf(__fmul_rn(s[v], to_log2), -3e38f);
+        if (tile * 32 + 31 > start_pos + q0) {           /* the tile reaches beyond the first query */
 #pragma unroll
-            for (int v = 0; v < 4; v++) {
-                const int kpos = tile * 32 + 16 * kb + 4 * g + v;
-                s[kb][v] = kpos <= qpos ? __fmul_rn(s[kb][v], scale) : -3e38f;
-                mx = fmaxf(mx, s[kb][v]);
-            }
-        mx = fmaxf(mx, __shfl_xor(mx, 16));
-        mx = fmaxf(mx, __shfl_xor(mx, 32));
-        const float mn = fmaxf(m, mx);
-        const float corr = __expf(m - mn);
-        float psum = 0.f;
-#pragma unroll
-        for (int kb = 0; kb < 2; kb++)
-#pragma unroll
-            for (int v = 0; v < 4; v++) {
-                s[kb][v] = s[kb][v] > -1e38f ? __expf(s[kb][v] - mn) : 0.f;
-                psum += s[kb][v];
-            }
-        lsum = fmaf(lsum, corr, psum);
-        m = mn;
-#pragma unroll
-        for (int b = 0; b < 8; b++) o[b] = o[b] * corr;
-        /* O^T += V^T P^T: slot j of this lane group is key 16*(j/4) + 4*g + j%4, whose probability is
-         * s[j/4][j%4]; the A operand of dim block b is that key's column 16*b + li of V */
-        bf16x8 phi, plo;
-        pa_planes8(s[0], s[1], phi, plo);
-        __builtin_amdgcn_sched_barrier(0);
-        fetch_part(nxt, 2);
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int b = 0; b < 8; b++) {
-            const unsigned char *vp = Vt + (16 * b + li) * PA_VROW + 16 * g;
-            const bf16x8 vhi = *reinterpret_cast<const bf16x8 *>(vp);
-            const bf16x8 vlo = *reinterpret_cast<const bf16x8 *>(vp + PA_VPLANE);
-            o[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vlo, phi, o[b], 0, 0, 0);
-            o[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vhi, plo, o[b], 0, 0, 0);
-            o[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vhi, phi, o[b], 0, 0, 0);
+            for (int v = 0; v < 16; v++) s[v] = tile * 32 + 8 * (v >> 2) + 4 * g + (v & 3) <= qpos ? s[v] : -3e38f;
         }
-        __builtin_amdgcn_sched_barrier(0);
-        fetch_part(nxt, 3);
-    }
-
-    /* merge the residues: residue r > 0 parks (m, l, O) in LDS, residue 0 folds them in */
-    if (NSPLIT > 1) {
-        __syncthreads();
-        float *park = reinterpret_cast<float *>(pa_lds);  /* [NSPLIT-1][HPW][34][64 lanes] */
-        for (int r = 1; r < NSPLIT; r++) {
-            float *slot = park + ((size_t)((r - 1) * HPW + hq) * 34) * 64 + lane;
-            if (pz == r) {
-                slot[0] = m;
-                slot[64] = lsum;
 #pragma unroll
-                for (int b = 0; b < 8; b++)
+        for (int v = 0; v < 16; v++) mx = fmaxf(mx, s[v]);
+        mx = pa_max_halves(mx);
+        /* The sums stay relative to an earlier maximum while the new one is at most 2^8 above it: probabilities and sums keep
+         * their relative precision, and most tiles leave O as it is. */
+        if (__any(mx > m + 8.0f)) {
+            const float mn = fmaxf(m, mx), corr = __builtin_amdgcn_exp2f(m - mn);
+            m = mn;
+            lsum *= corr;
 #pragma unroll
-                    for (int v = 0; v < 4; v++) slot[(2 + b * 4 + v) * 64] = o[b][v];
+            for (int b = 0; b < 4; b++) o[b] = o[b] * corr;
+        }
+#pragma unroll
+        for (int v = 0; v < 16; v++) {
+            s[v] = __builtin_amdgcn_exp2f(s[v] - m);
+            lsum += s[v];
+        }
+        /* O^T += V^T P^T */
+#pragma unroll
+        for (int kt = 0; kt < 2; kt++) {
+            bf16x8 phi, plo;
+            pa_planes8(f32x4{s[8 * kt], s[8 * kt + 1], s[8 * kt + 2], s[8 * kt + 3]}, f32x4{s[8 * kt + 4], s[8 * kt + 5], s[8 * kt + 6], s[8 * kt + 7]}, phi, plo);
+#pragma unroll
+            for (int b = 0; b < 4; b++) {
+                const bf16x8 vhi = *reinterpret_cast<const bf16x8 *>(Vt + lane * 16 + (b * 2 + kt) * 1024);
+                const bf16x8 vlo = *reinterpret_cast<const bf16x8 *>(Vt + lane * 16 + PA_PLANE + (b * 2 + kt) * 1024);
+                o[b] = pa_mfma(vlo, phi, o[b]);
+                o[b] = pa_mfma(vhi, plo, o[b]);
+                o[b] = pa_mfma(vhi, phi, o[b]);
             }
-            __syncthreads();
-            if (pz == 0) {
-                const float m2 = slot[0], l2 = slot[64];
-                const float mn = fmaxf(m, m2);
-                const float c1 = __expf(m - mn), c2 = __expf(m2 - mn);
-                lsum = fmaf(lsum, c1, l2 * c2);
-                m = mn;
-#pragma unroll
-                for (int b = 0; b < 8; b++)
-#pragma unroll
-                    for (int v = 0; v < 4; v++) o[b][v] = fmaf(o[b][v], c1, slot[(2 + b * 4 + v) * 64] * c2);
-            }
-            __syncthreads();
+        }
+    };
+    /* every wave waits for what it asked for, then for all the others: they have then also read what is written next */
+#define PA_LANDED() do { __builtin_amdgcn_s_waitcnt(0x0f70); __syncthreads(); } while (0)     /* vmcnt(0) */
+    PA_LANDED();
+    if constexpr (QB == 32) {
+        /* the next tile arrives while this one is worked on: one barrier per tile */
+        const unsigned char *even = pa_a + pz * PA_TILE_BYTES, *odd = pa_b + pz * PA_TILE_BYTES;
+        for (int step = 0; step < nsteps; step += 2) {
+            fetch(pa_b, step + 1, 0);
+            if (step * NS + pz < ntiles) { scores(even); weigh(even + 2 * PA_PLANE, step * NS + pz); }
+            PA_LANDED();
+            fetch(pa_a, step + 2, 0);
+            if ((step + 1) * NS + pz < ntiles) { scores(odd); weigh(odd + 2 * PA_PLANE, (step + 1) * NS + pz); }
+            PA_LANDED();
+        }
+    } else {
+        /* V of a tile arrives under its scores, K of the next one under the rest */
+        for (int step = 0; step < nsteps; step++) {
+            const int tile = step * NS + pz;
+            fetch(pa_b, step, 2 * PA_PLANE);
+            if (tile < ntiles) scores(pa_a + pz * 2 * PA_PLANE);
+            PA_LANDED();
+            fetch(pa_a, step + 1, 0);
+            if (tile < ntiles) weigh(pa_b + pz * 2 * PA_PLANE, tile);
+            PA_LANDED();
         }
     }
-    asm volatile("" ::"v"(warm[0]), "v"(warm[1]), "v"(warm[2]), "v"(warm[3]));
-    if (pz != 0 || my_q >= S) return;
-    float L = lsum + __shfl_xor(lsum, 16);
-    L += __shfl_xor(L, 32);
-    const float inv = L > 0.f ? __fdiv_rn(1.0f, L) : 0.f;
-    const size_t ob = (size_t)my_q * VT_Q_DIM + head * VT_HEAD_DIM;
+#undef PA_LANDED
+
+    /* Merge: of the NS waves with the same rows, wave pz finishes 128 / NS dims.  Each parks its sums, 16 quads of
+     * dims (behind the last barrier nobody reads tiles); they are added in the order of the residues. */
+    constexpr int NB = 4 / NS;                           /* dim blocks that a wave finishes */
+    auto park = [&](int w, int b, int v) {
+        return reinterpret_cast<f32x4 *>((w < 4 ? pa_a : pa_b) + (w & 3) * 16384 + (4 * b + v) * 1024 + lane * 16);
+    };
 #pragma unroll
-    for (int b = 0; b < 8; b++) {
-        const int d = 16 * b + 4 * g;
-        f32x4 r;
-        r.x = __fmul_rn(o[b][0], inv);
-        r.y = __fmul_rn(o[b][1], inv);
-        r.z = __fmul_rn(o[b][2], inv);
-        r.w = __fmul_rn(o[b][3], inv);
-        if (out) *reinterpret_cast<f32x4 *>(out + ob + d) = r;
-        if (out_hi) {
-            u32x2 sph, spl;
-            vt_split_planes4(r.x, r.y, r.z, r.w, sph, spl);
-            u32x2 ph = sph, pl = spl;
-            *reinterpret_cast<u32x2 *>(out_hi + ob + d) = ph;
-            *reinterpret_cast<u32x2 *>(out_lo + ob + d) = pl;
+    for (int b = 0; b < 4; b++)
+#pragma unroll
+        for (int v = 0; v < 4; v++) *park(wave, b, v) = f32x4{o[b][4 * v], o[b][4 * v + 1], o[b][4 * v + 2], o[b][4 * v + 3]};
+    pa_ml[wave][lane] = f32x2{m, lsum};
+    __syncthreads();
+    float c[NS], inv;
+    {
+        f32x2 ml[NS];
+#pragma unroll
+        for (int r = 0; r < NS; r++) ml[r] = pa_ml[r * HW + hq][lane];
+        float mn = ml[0].x, L = 0.f;
+#pragma unroll
+        for (int r = 1; r < NS; r++) mn = fmaxf(mn, ml[r].x);
+#pragma unroll
+        for (int r = 0; r < NS; r++) {
+            c[r] = __builtin_amdgcn_exp2f(ml[r].x - mn);
+            L = fmaf(ml[r].y, c[r], L);
+        }
+        L += __shfl_xor(L, 32);
+        inv = L > 0.f ? __fdiv_rn(1.0f, L) : 0.f;
+    }
+    f32x4 res[NB][4];
+#pragma unroll
+    for (int b = 0; b < NB; b++)
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            f32x4 x = *park(hq, NB * pz + b, v) * c[0];
+#pragma unroll
+            for (int r = 1; r < NS; r++) {
+                const f32x4 y = *park(r * HW + hq, NB * pz + b, v);
+                x = f32x4{fmaf(y.x, c[r], x.x), fmaf(y.y, c[r], x.y), fmaf(y.z, c[r], x.z), fmaf(y.w, c[r], x.w)};
+            }
+            res[b][v] = x * inv;
+        }
+    const int hd = QB == 16 ? 2 * hq + (li >> 4) : hq;   /* this lane's head of the four */
+    if (out && my_q < S) {
+#pragma unroll
+        for (int b = 0; b < NB; b++)
+#pragma unroll
+            for (int v = 0; v < 4; v++)
+                *reinterpret_cast<f32x4 *>(out + (size_t)my_q * VT_Q_DIM + (kvh * 4 + hd) * VT_HEAD_DIM + 32 * (NB * pz + b) + 8 * v + 4 * g) = res[b][v];
+    }
+    if (!out_hi) return;
+    __syncthreads();
+    /* the planes leave through LDS, as whole lines: rows of 256 bytes, [query][head], 16-byte piece i at place i ^ query % 16 */
+#pragma unroll
+    for (int b = 0; b < NB; b++)
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            u32x2 h, l;
+            vt_split_planes4(res[b][v].x, res[b][v].y, res[b][v].z, res[b][v].w, h, l);
+            const int at = ((li % QB) * 4 + hd) * 256 + (((4 * (NB * pz + b) + v) ^ (li & 15)) * 16) + 8 * g;
+            *reinterpret_cast<u32x2 *>(pa_a + at) = h;
+            *reinterpret_cast<u32x2 *>(pa_b + at) = l;
+        }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < QB / 8; i++) {                   /* a wave stores one query's four heads */
+        const int r = 8 * i + wave;
+        if (q0 + r < S) {
+            const size_t at = (size_t)(q0 + r) * VT_Q_DIM + kvh * 4 * VT_HEAD_DIM + 8 * lane;
+            const int from = (r * 4 + (lane >> 4)) * 256 + (((lane & 15) ^ (r & 15)) * 16);
+            *reinterpret_cast<u32x4 *>(out_hi + at) = *reinterpret_cast<const u32x4 *>(pa_a + from);
+            *reinterpret_cast<u32x4 *>(out_lo + at) = *reinterpret_cast<const u32x4 *>(pa_b + from);
         }
     }
-}
-
-#ifndef PA_NSPLIT
-#define PA_NSPLIT 2
-#endif
-#ifndef PA_HPW
-#define PA_HPW 2
-#endif
-
-static size_t pa_lds_bytes(void) {
-    size_t tiles = (size_t)PA_NSPLIT * PA_TILE_BYTES;
-    size_t park = sizeof(float) * (size_t)(PA_NSPLIT - 1) * PA_HPW * 34 * 64;
-    return tiles > park ? tiles : park;
 }
 
 /* Tiles of 32 keys that cover `rows` cache rows, and the tile images of one layer's K and V (a buffer of the
@@ -477,18 +466,14 @@ void vt_pa_launch_image(unsigned char *d_img, const float *d_qkv, int col0, int 
 void vt_launch_prefill_attention_raw(float *d_out, uint16_t *d_hi, uint16_t *d_lo, const float *d_Q,
                                      int q_stride, int q_col0, int q_planes, size_t q_plane_stride, const float *d_rope,
                                      const unsigned char *d_img, int S, int start_pos, float scale) {
-    static int attr_set = 0;
-    if (!attr_set) {
-        if (vt_check(hipFuncSetAttribute((const void *)vt_prefill_attention_kernel<PA_NSPLIT, PA_HPW>,
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)pa_lds_bytes()),
-                     "attention LDS size"))
-            return;
-        attr_set = 1;
-    }
-    hipLaunchKernelGGL((vt_prefill_attention_kernel<PA_NSPLIT, PA_HPW>),
-                       dim3(VT_KV_HEADS * (4 / PA_HPW), (S + PA_QT - 1) / PA_QT), dim3(64 * PA_HPW * PA_NSPLIT),
-                       pa_lds_bytes(), g_vt.stream, d_out, d_hi, d_lo, d_Q, q_stride, q_col0, q_planes, q_plane_stride, d_rope,
-                       d_img, pa_tiles(start_pos + S), S, start_pos, scale);
+    const bool lng = S > PA_SHORT_ROWS;
+    const int qb = lng ? PA_LONG_QT : PA_SHORT_QT;
+    const dim3 grid(VT_KV_HEADS, (S + qb - 1) / qb);
+#define CALL(QB) hipLaunchKernelGGL(vt_prefill_attention_kernel<QB>, grid, dim3(512), 0, g_vt.stream, d_out, d_hi, d_lo, d_Q, q_stride, q_col0, \
+                                    q_planes, q_plane_stride, d_rope, d_img, pa_tiles(start_pos + S), S, start_pos, scale)
+    if (lng) CALL(PA_LONG_QT);
+    else CALL(PA_SHORT_QT);
+#undef CALL
 }
 
 void vt_launch_prefill_attention(float *d_out, uint16_t *d_hi, uint16_t *d_lo, const float *d_Q,
