@@ -1,6 +1,6 @@
 """Causal attention of a prompt at the edges of its kernels (16 queries per workgroup up to 1200 rows, 32 beyond): a block
-with one query more, key tiles that begin before the first new row, and scores that grow along the keys, by less and by more
-than the 2^8 that the running maximum may lag behind.  Against float64."""
+with one query more, key tiles that begin before the first new row, and scores that grow along the keys, so that the
+running maximum changes with every tile.  Against float64."""
 import ctypes as C
 
 import numpy as np

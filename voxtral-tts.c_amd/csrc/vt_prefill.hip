@@ -40,12 +40,12 @@
  * instructions, two waves per SIMD: 2.0 to 2.3 us per NS tiles, 1.28 of them matrix instructions at 2.4 GHz; and
  * 7 to 9 us in front and behind (queries 2.1, their planes 1.5, merge and stores 2.5: each of them code that is run once and
  * comes from memory).  us per launch inside a prefill of 37 / 226 / 512 / 1531 rows: 7.7 / 12.2 / 17.8 /
- * 63.2, where 16 queries per wave on 16 x 16 x 32 instructions, four waves and tiles copied through registers took 9.0 / 15.8 /
+ * 65.6, where 16 queries per wave on 16 x 16 x 32 instructions, four waves and tiles copied through registers took 9.0 / 15.8 /
  * 24.5 / 125.5. */
 /* Queries per workgroup: 16 as long as that gives the CUs more to do at once (twice the workgroups, each half as many
  * rounds of tiles), 32 from where every CU is busy either way and the tiles are copied half as often.  us per launch
  * at 37 / 226 / 512 / 1000 / 1531 / 3000 rows, 16: 7.5 / 10.5 / 16.4 / 34.4 / 70.1 / 236.7, 32: 9.0 / 14.3 / 22.4 / 39.5 /
- * 63.0 / 210.5. */
+ * 65.4 / 213.8. */
 #define PA_SHORT_QT 16
 #define PA_LONG_QT 32
 #define PA_SHORT_ROWS 1200
@@ -302,9 +302,9 @@ vt_prefill_attention_kernel(float *out, uint16_t *out_hi, uint16_t *out_lo, cons
 #pragma unroll
         for (int v = 0; v < 16; v++) mx = fmaxf(mx, s[v]);
         mx = pa_max_halves(mx);
-        /* The sums stay relative to an earlier maximum while the new one is at most 2^8 above it: probabilities and sums keep
-         * their relative precision, and most tiles leave O as it is. */
-        if (__any(mx > m + 8.0f)) {
+        /* (Letting the maximum lag by up to 2^8, so that fewer tiles rescale the sums, makes the results' error against 64 bits
+         * 2.5 % larger: a probability of exactly 1 has no rounding error, and a row's largest one no longer is.) */
+        if (__any(mx > m)) {
             const float mn = fmaxf(m, mx), corr = __builtin_amdgcn_exp2f(m - mn);
             m = mn;
             lsum *= corr;
@@ -312,10 +312,9 @@ vt_prefill_attention_kernel(float *out, uint16_t *out_hi, uint16_t *out_lo, cons
             for (int b = 0; b < 4; b++) o[b] = o[b] * corr;
         }
 #pragma unroll
-        for (int v = 0; v < 16; v++) {
-            s[v] = __builtin_amdgcn_exp2f(s[v] - m);
-            lsum += s[v];
-        }
+        for (int v = 0; v < 16; v++) s[v] = __builtin_amdgcn_exp2f(s[v] - m);
+        lsum += (((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]))) +
+                (((s[8] + s[9]) + (s[10] + s[11])) + ((s[12] + s[13]) + (s[14] + s[15])));
         /* O^T += V^T P^T */
 #pragma unroll
         for (int kt = 0; kt < 2; kt++) {
