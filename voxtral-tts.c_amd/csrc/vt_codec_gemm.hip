@@ -63,7 +63,7 @@ int vt_codec_weight_layout(uint16_t *d_Wf, int *d_col_exp, const float *d_W, int
 /* ---- launches -------------------------------------------------------------------------------------------------- */
 
 template <int NP>
-static void cg_rows(const gr_plan &plan, int grid, const uint16_t *d_hi, const uint16_t *d_lo, int M, int K) {
+static void cg_rows(const gr_list &plan, int grid, const uint16_t *d_hi, const uint16_t *d_lo, int M, int K) {
     constexpr int NW = VT_CODEC_ROW_WAVES;
     static int attr_set = 0;
     const int lds = NW * 2 * 32 * ((NP + 3) / 4) * GM_STAGE_ROW;
@@ -91,11 +91,9 @@ static void cg_wide(const gw_list &list, const uint16_t *d_hi, const uint16_t *d
 void vt_launch_codec_gemm(float *d_C, const uint16_t *d_hi, const uint16_t *d_lo, const int *d_row_exp,
                           const uint16_t *d_Wf, const int *d_col_exp, int M, int N, int K, const vt_gemm_plan &pl) {
     if (pl.mb == 0) {
-        gr_plan plan = {};
-        plan.n_parts = 1;
-        plan.part[0] = gr_part{d_C, d_Wf, (size_t)M * N, N, N / GR_TN, pl.cuts, NULL, NULL, 0, d_row_exp, d_col_exp};
-        const int items = plan.part[0].n_tiles * pl.cuts, grid = items < g_vt.n_cu ? items : g_vt.n_cu;
-        static void (*const launch[4])(const gr_plan &, int, const uint16_t *, const uint16_t *, int, int) = {cg_rows<2>, cg_rows<4>, cg_rows<6>, cg_rows<8>};
+        const gr_list plan = {d_C, d_Wf, (size_t)M * N, N, N / GR_TN, pl.cuts, d_row_exp, d_col_exp};
+        const int items = plan.n_tiles * pl.cuts, grid = items < g_vt.n_cu ? items : g_vt.n_cu;
+        static void (*const launch[4])(const gr_list &, int, const uint16_t *, const uint16_t *, int, int) = {cg_rows<2>, cg_rows<4>, cg_rows<6>, cg_rows<8>};
         launch[(M + 15) / 16 - 1](plan, grid, d_hi, d_lo, M, K);
         return;
     }

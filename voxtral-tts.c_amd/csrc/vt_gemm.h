@@ -22,7 +22,7 @@ void vt_launch_gemm_ex(float *d_C, int ldc, size_t plane_stride, const uint16_t 
  * (vt_gemm_wide.hip; mb 0: vt_gemm_rows.hip).  col0 is a multiple of 128. */
 #define VT_MAX_CUTS 8
 struct vt_gemm_plan { int mb, tn, col0, cuts; };
-/* N % 256 == 0, K % 64 == 0; swiglu: for vt_launch_gemm_frag_swiglu */
+/* K % 64 == 0; N % 256 == 0, up to 64 rows N % 96 == 0 (swiglu: % 288); swiglu: for vt_launch_gemm_frag_swiglu */
 vt_gemm_plan vt_gemm_frag_plan(int M, int N, int K, int swiglu);
 void vt_launch_gemm_frag(float *d_C, int ldc, size_t plane_stride, const uint16_t *d_Ahi, const uint16_t *d_Alo,
                          const uint16_t *d_Wf, int M, int N, int K, const vt_gemm_plan &pl);
@@ -30,17 +30,14 @@ void vt_launch_gemm_frag(float *d_C, int ldc, size_t plane_stride, const uint16_
  * columns from pl.col0 on pass through d_tail [pl.cuts][M, N - pl.col0] and a second launch */
 void vt_launch_gemm_frag_swiglu(uint16_t *d_hhi, uint16_t *d_hlo, int ldh, float *d_tail, const uint16_t *d_Ahi,
                                 const uint16_t *d_Alo, const uint16_t *d_Wf, int M, int N, int K, const vt_gemm_plan &pl);
-/* The same product for M <= 64 rows on 64-column tiles (vt_gemm_rows.hip), weights in the same fragment order:
- * N % 64 == 0, K % 64 == 0; the cuts need not divide K. */
+/* The same for M <= 64 rows on strips of 96 columns, or 288 for the gate|up product (vt_gemm_rows.hip), weights in the same
+ * fragment order: N a multiple of those; the cuts need not divide K. */
 int vt_gemm_rows_ok(int M, int N, int K);
-int vt_gemm_rows_waves(int M);
-int vt_gemm_rows_cuts(int waves, int N, int K, int most);      /* waves of a workgroup */
+vt_gemm_plan vt_gemm_few_rows_plan(int N, int swiglu);
+void vt_launch_gemm_few_rows(float *d_C, int ldc, size_t plane_stride, const uint16_t *d_Ahi, const uint16_t *d_Alo,
+                             const uint16_t *d_Wf, int M, int N, int K, const vt_gemm_plan &pl);
+int vt_gemm_rows_cuts(int waves, int N, int K, int most);      /* waves of a workgroup of vt_gemm_rows_kernel */
 #define VT_CODEC_ROW_WAVES 4     /* with two weight planes a wave's registers do not fit two waves per SIMD */
-void vt_launch_gemm_rows(float *d_C, int ldc, size_t plane_stride, const uint16_t *d_Ahi, const uint16_t *d_Alo,
-                         const uint16_t *d_Wf, int M, int N, int K, int splits);
-void vt_launch_gemm_rows_swiglu(uint16_t *d_hhi, uint16_t *d_hlo, int ldh, float *d_tail, const uint16_t *d_Ahi,
-                                const uint16_t *d_Alo, const uint16_t *d_Wf, int M, int n_main, int n_tail, int K,
-                                int tail_splits);
 /* The codec's products (vt_codec_gemm.hip): activations as two fp16 planes [M, K] with an exponent per row, weights in
  * fragment order with an exponent per column, from fp32 W[N, K] by vt_codec_weight_layout (d_Wf: 2 N K elements; 0 / -1).
  * N % 64 == 0 (more than 64 rows: % 256), K % 64 == 0.  d_C: [M, pl.col0] and, behind it, pl.cuts planes of

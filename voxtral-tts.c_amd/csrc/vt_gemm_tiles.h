@@ -402,15 +402,12 @@ vt_gemm_wide_kernel(gw_list list, const uint16_t *Ahi, const uint16_t *Alo, int 
 }
 
 
-/* ---- up to 64 rows (a short prompt) -----------------------------------------------------------------------
- * With so few rows the product is a weight stream: at 64 rows a CU needs 1024 of the 2900 cycles in which its
- * share of HBM delivers 32 KB of weights.  What counts is that every CU has a share, and an equal one.  A tile
- * of vt_gemm_wide_kernel is 256 columns wide, so gate|up has 72 of them for 256 CUs, and the other products
- * can only give more CUs something to do by cutting K into many planes.  Here a workgroup owns 64 columns and
+/* ---- up to 64 rows (the codec's first stages) ---------------------------------------------------------------
+ * With so few rows the product is a weight stream, and what counts is that every CU has a share of it, and an equal one.  A
+ * workgroup owns 64 columns and
  * its waves share K among themselves: wave w takes the 64-wide K steps w, w + NW, ... of the workgroup's range,
  * keeps its own sums for all rows, and the waves' sums are added through LDS at the end (in wave order: the
- * result does not depend on timing).  288 gate|up tiles (256 whole and the last 32 in 8 K cuts), 96 q|k|v tiles
- * in 2 cuts, 48 output and down tiles in 4 and 5 then fill the chip with at most 5 planes.
+ * result does not depend on timing).
  *
  * No two waves work on the same K step, so nobody shares anything before the end: a wave stages its own
  * activation rows through its own piece of LDS (one stage; the LDS serves a wave's accesses in order, so the
@@ -419,26 +416,16 @@ vt_gemm_wide_kernel(gw_list list, const uint16_t *Ahi, const uint16_t *Alo, int 
  * goes through a buffer descriptor whose size says whether there is anything to load: steps past a wave's last
  * one and rows past M ask for nothing, without a branch (behind a branch the compiler would wait for all
  * outstanding loads).
- *
- * What bounds it, from 26 layers in rotation: the stream plus about 4 us of launch, first latency, sums and
- * stores, plus the activation rows, which every workgroup reads for itself at about 50 KB/us per CU (1.3 us per
- * 8 rows in the gate|up product; that is why the passes over the rows are a template argument and the kernel is
- * not used beyond 64 rows, where rows shared through LDS cost less).  us per launch, q|k|v / output / gate|up /
- * down: 10.0 / 7.7 / 22.2 / 11.9 at 6 rows, 14.5 / 10.4 / 29.6 / 16.5 at 37, 15.5 / 11.5 / 34.1 / 18.8 at 64;
- * vt_gemm_wide_kernel takes 21.7 / 16.8 / 62.1 / 27.9 at 37.
  */
 #define GR_TN 64
 
-struct gr_part {
+struct gr_list {
     float *C;                             /* `splits` planes of [M, ldc], plane_stride floats apart */
-    const uint16_t *Wf;                   /* fragment-order weights of the part's first column */
+    const uint16_t *Wf;                   /* fragment-order weights */
     size_t plane_stride;
     int ldc, n_tiles, splits;
-    uint16_t *h_hi, *h_lo;                /* gate|up (paired column order): planes of SiLU(gate) * up instead of C */
-    int ldh;
-    const int *row_exp, *col_exp;         /* T::SCALED: exponents of the rows and of the part's columns */
+    const int *row_exp, *col_exp;         /* T::SCALED: exponents of the rows and of the columns */
 };
-struct gr_plan { gr_part part[2]; int n_parts; };
 
 /* non-temporal: with this few rows the weights are read once */
 __device__ __forceinline__ u32x4 gr_ld_nt(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
@@ -448,18 +435,16 @@ __device__ __forceinline__ u32x4 gr_ld_nt(__amdgpu_buffer_rsrc_t r, int voff, in
 /* One workgroup's piece of a product: a 64-column tile over one K cut */
 struct gr_item {
     const unsigned char *w;               /* weights of the tile */
-    int part, nt, sp, s0, n;              /* n: this wave's K steps s0 + wave + NW i */
+    int nt, sp, s0, n;                    /* n: this wave's K steps s0 + wave + NW i */
 };
 
 template <int NW, int WP>
-__device__ __forceinline__ gr_item gr_item_at(const gr_plan &plan, int part, int id, int K, int wave) {
-    const gr_part &P = plan.part[part];
+__device__ __forceinline__ gr_item gr_item_at(const gr_list &P, int id, int K, int wave) {
     /* slot id lands on XCD id % 8: an XCD takes a run of items, N tile fastest, i.e. few K cuts: the slice of
      * the planes that its L2 has to fetch is that of its cuts */
     const int items = P.n_tiles * P.splits;
     const int li = (items & 7) == 0 ? (id & 7) * (items >> 3) + (id >> 3) : id;
     gr_item it;
-    it.part = part;
     it.nt = li % P.n_tiles;
     it.sp = li / P.n_tiles;
     const int steps = K / 64, q = steps / P.splits, rem = steps % P.splits;
@@ -473,7 +458,7 @@ __device__ __forceinline__ gr_item gr_item_at(const gr_plan &plan, int part, int
 /* NP passes of 8 rows: M <= 8 NP; NW waves */
 template <class T, int NP, int NW>
 __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW / 4, NW / 4)))
-vt_gemm_rows_kernel(gr_plan plan, const uint16_t *Ahi, const uint16_t *Alo, int M, int K) {
+vt_gemm_rows_kernel(gr_list P, const uint16_t *Ahi, const uint16_t *Alo, int M, int K) {
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     constexpr int WP = T::WP;
     constexpr int MB = (NP + 3) / 4;                                         /* blocks of 32 rows */
@@ -575,7 +560,6 @@ vt_gemm_rows_kernel(gr_plan plan, const uint16_t *Ahi, const uint16_t *Alo, int 
     };
     /* the waves' sums: parked as quads of accumulator elements over each wave's own stage, added in wave order */
     auto finish = [&](const gr_item &it) {
-        const gr_part &P = plan.part[it.part];
         float *park = reinterpret_cast<float *>(mine);
 #pragma unroll
         for (int a = 0; a < MB; a++)
@@ -599,36 +583,20 @@ vt_gemm_rows_kernel(gr_plan plan, const uint16_t *Ahi, const uint16_t *Alo, int 
                     s[b].z = __fadd_rn(s[b].z, v.z); s[b].w = __fadd_rn(s[b].w, v.w);
                 }
             const int row0 = 8 * qd + 4 * (lane >> 5), c = lane & 31;
-            if (!T::SCALED && P.h_hi) {
-                const vt_h_quad h = vt_silu_mul_quad(s[0], s[1]);                /* voxtral_tts_llm.c:346-350 */
-                const size_t at = (size_t)(row0 + h.row) * P.ldh + it.nt * (GR_TN / 2) + (c & ~1);
-#pragma unroll
-                for (int r = 0; r < 2; r++)
-                    if (row0 + h.row + r < M) {
-                        *reinterpret_cast<unsigned *>(P.h_hi + at + (size_t)r * P.ldh) = h.hi[r];
-                        *reinterpret_cast<unsigned *>(P.h_lo + at + (size_t)r * P.ldh) = h.lo[r];
-                    }
-            } else {
-                const int col = it.nt * GR_TN + c;
-                gm_store_quad<T, 2>(P.C + (size_t)it.sp * P.plane_stride + col, P.ldc, row0, M, s, P.row_exp, P.col_exp + col);
-            }
+            const int col = it.nt * GR_TN + c;
+            gm_store_quad<T, 2>(P.C + (size_t)it.sp * P.plane_stride + col, P.ldc, row0, M, s, P.row_exp, P.col_exp + col);
         }
     };
 
-    /* items blockIdx.x, + gridDim.x, ... of each part in turn; the first requests of the next item go out in
-     * front of the sums of this one */
-    int part = 0, id = (int)blockIdx.x;
-    gr_item it = gr_item_at<NW, WP>(plan, 0, id, K, wave);
+    /* items blockIdx.x, + gridDim.x, ...; the first requests of the next item go out in front of the sums of this one */
+    int id = (int)blockIdx.x;
+    gr_item it = gr_item_at<NW, WP>(P, id, K, wave);
     begin(it);
     for (;;) {
         multiply(it);
         id += (int)gridDim.x;
-        while (part < plan.n_parts && id >= plan.part[part].n_tiles * plan.part[part].splits) {
-            part++;
-            id = (int)blockIdx.x;
-        }
-        if (part >= plan.n_parts) break;
-        const gr_item nx = gr_item_at<NW, WP>(plan, part, id, K, wave);
+        if (id >= P.n_tiles * P.splits) break;
+        const gr_item nx = gr_item_at<NW, WP>(P, id, K, wave);
         begin(nx);
         finish(it);
         __syncthreads();                  /* the next item stages over the parked sums */

@@ -73,18 +73,7 @@ static vt_gemm_plan gw_plan(const gw_format &f, int M, int N, int K, int swiglu)
 }
 
 vt_gemm_plan vt_gemm_frag_plan(int M, int N, int K, int swiglu) {
-    vt_gemm_plan best = {0, 64, 0, 1};
-    if (vt_gemm_rows_ok(M, N, K)) {
-        if (swiglu) {
-            best.col0 = N / 64 / g_vt.n_cu * g_vt.n_cu * 64;
-            const int rest = (N - best.col0) / 64;
-            while (rest && best.cuts < VT_MAX_CUTS && (best.cuts + 1) * rest <= g_vt.n_cu) best.cuts++;
-        } else {
-            best.cuts = vt_gemm_rows_cuts(vt_gemm_rows_waves(M), N, K, VT_MAX_CUTS);
-        }
-        return best;
-    }
-    return gw_plan(gw_backbone, M, N, K, swiglu);
+    return vt_gemm_rows_ok(M, N, K) ? vt_gemm_few_rows_plan(N, swiglu) : gw_plan(gw_backbone, M, N, K, swiglu);
 }
 
 vt_gemm_plan vt_codec_gemm_plan(int M, int N, int K) {
@@ -121,7 +110,7 @@ static void gw_run(const vt_gemm_plan &pl, gw_part whole, gw_part cut, const uin
 
 void vt_launch_gemm_frag(float *d_C, int ldc, size_t plane_stride, const uint16_t *d_Ahi, const uint16_t *d_Alo,
                          const uint16_t *d_Wf, int M, int N, int K, const vt_gemm_plan &pl) {
-    if (pl.mb == 0) { vt_launch_gemm_rows(d_C, ldc, plane_stride, d_Ahi, d_Alo, d_Wf, M, N, K, pl.cuts); return; }
+    if (pl.mb == 0) { vt_launch_gemm_few_rows(d_C, ldc, plane_stride, d_Ahi, d_Alo, d_Wf, M, N, K, pl); return; }
     gw_run(pl, gw_part{d_C, d_Wf, plane_stride, ldc, 0, 0, NULL, NULL, 0, NULL, NULL},
            gw_part{d_C + pl.col0, d_Wf + (size_t)pl.col0 * K, plane_stride, ldc, 0, 0, NULL, NULL, 0, NULL, NULL}, d_Ahi, d_Alo, M, N, K);
 }
@@ -130,7 +119,7 @@ void vt_launch_gemm_frag_swiglu(uint16_t *d_hhi, uint16_t *d_hlo, int ldh, float
                                 const uint16_t *d_Alo, const uint16_t *d_Wf, int M, int N, int K, const vt_gemm_plan &pl) {
     const int tail = N - pl.col0;
     if (pl.mb == 0)
-        vt_launch_gemm_rows_swiglu(d_hhi, d_hlo, ldh, d_tail, d_Ahi, d_Alo, d_Wf, M, pl.col0, tail, K, pl.cuts);
+        vt_launch_gemm_few_rows(d_tail, N, (size_t)M * N, d_Ahi, d_Alo, d_Wf, M, N, K, pl);
     else
         gw_run(pl, gw_part{NULL, d_Wf, 0, 0, 0, 0, d_hhi, d_hlo, ldh, NULL, NULL},
                gw_part{d_tail, d_Wf + (size_t)pl.col0 * K, (size_t)M * tail, tail, 0, 0, NULL, NULL, 0, NULL, NULL}, d_Ahi, d_Alo, M, N, K);

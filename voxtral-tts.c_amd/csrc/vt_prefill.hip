@@ -85,65 +85,52 @@ vt_kv_image_kernel(unsigned char *img, int img_tiles, const float *qkv, int col0
     const bool is_v = threadIdx.x >= 128;
     const int tl = (int)threadIdx.x & 127, sg = tl >> 5, cg = tl & 31;
     const int col = kvh * VT_HEAD_DIM + 4 * cg;
-    if (VT_Q_DIM + (is_v ? VT_KV_DIM : 0) + kvh * VT_HEAD_DIM < col0) planes = 1;      /* a head whose columns are not cut */
+    const int wide_col = VT_Q_DIM + (is_v ? VT_KV_DIM : 0) + col;                /* in the product's rows */
+    if (!qkv || VT_Q_DIM + (is_v ? VT_KV_DIM : 0) + kvh * VT_HEAD_DIM < col0) planes = 1;      /* a head whose columns are not cut */
     float *cache = is_v ? vc : kc;
-    f32x4 r8[8];
+    f32x4 r8[8], cs[8];
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-    if (qkv && tile * 32 >= start_pos && tile * 32 + 32 <= kv_rows) {
-        /* a tile of new rows only (all but the first and the last one of a chunk): every request up front */
-        const float *src = qkv + (size_t)(tile * 32 - start_pos) * VT_QKV_DIM + VT_Q_DIM + (is_v ? VT_KV_DIM : 0) + col;
-        f32x4 cs[8];
+    /* Every request up front (a row that is not there asks for the last one, a plane that is not there for the last one again):
+     * with one row or plane after the other a launch at 37 rows in four cuts took 7.3 us. */
+    const float *src[8];
+    bool fresh[8];
 #pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const int row = pa_key(sg, i);
-            r8[i] = *reinterpret_cast<const f32x4 *>(src + (size_t)row * VT_QKV_DIM);
-            cs[i] = is_v ? zero : *reinterpret_cast<const f32x4 *>(rope + (size_t)(tile * 32 + row) * VT_HEAD_DIM + 4 * cg);
-        }
-        for (int p = 1; p < planes; p++) {
-            f32x4 w[8];
+    for (int i = 0; i < 8; i++) {
+        const int r = min(tile * 32 + pa_key(sg, i), kv_rows - 1);
+        fresh[i] = qkv && r >= start_pos;
+        src[i] = fresh[i] ? qkv + (size_t)(r - start_pos) * VT_QKV_DIM + wide_col : cache + (size_t)r * VT_KV_DIM + col;
+        r8[i] = *reinterpret_cast<const f32x4 *>(src[i]);
+        cs[i] = qkv && !is_v ? *reinterpret_cast<const f32x4 *>(rope + (size_t)r * VT_HEAD_DIM + 4 * cg) : zero;
+    }
+    for (int p = 1; p < planes; p += 3) {
+        f32x4 w[3][8];
 #pragma unroll
-            for (int i = 0; i < 8; i++)
-                w[i] = *reinterpret_cast<const f32x4 *>(src + p * plane_stride + (size_t)pa_key(sg, i) * VT_QKV_DIM);
+        for (int z = 0; z < 3; z++)
 #pragma unroll
-            for (int i = 0; i < 8; i++) {
-                r8[i].x = __fadd_rn(r8[i].x, w[i].x); r8[i].y = __fadd_rn(r8[i].y, w[i].y);
-                r8[i].z = __fadd_rn(r8[i].z, w[i].z); r8[i].w = __fadd_rn(r8[i].w, w[i].w);
+            for (int i = 0; i < 8; i++) w[z][i] = *reinterpret_cast<const f32x4 *>(src[i] + (fresh[i] ? min(p + z, planes - 1) * plane_stride : 0));
+#pragma unroll
+        for (int z = 0; z < 3; z++)
+            if (p + z < planes) {
+#pragma unroll
+                for (int i = 0; i < 8; i++)
+                    if (fresh[i]) {
+                        r8[i].x = __fadd_rn(r8[i].x, w[z][i].x); r8[i].y = __fadd_rn(r8[i].y, w[z][i].y);
+                        r8[i].z = __fadd_rn(r8[i].z, w[z][i].z); r8[i].w = __fadd_rn(r8[i].w, w[z][i].w);
+                    }
             }
-        }
+    }
 #pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const int r = tile * 32 + pa_key(sg, i);
+    for (int i = 0; i < 8; i++) {
+        const int r = tile * 32 + pa_key(sg, i);
+        if (fresh[i]) {
             if (!is_v) {
                 const f32x4 k = r8[i], c = cs[i];
                 r8[i] = f32x4{__fsub_rn(__fmul_rn(k.x, c.x), __fmul_rn(k.y, c.y)), __fadd_rn(__fmul_rn(k.x, c.y), __fmul_rn(k.y, c.x)),
                               __fsub_rn(__fmul_rn(k.z, c.z), __fmul_rn(k.w, c.w)), __fadd_rn(__fmul_rn(k.z, c.w), __fmul_rn(k.w, c.z))};
             }
-            *reinterpret_cast<f32x4 *>(cache + (size_t)r * VT_KV_DIM + col) = r8[i];
+            if (r < kv_rows) *reinterpret_cast<f32x4 *>(cache + (size_t)r * VT_KV_DIM + col) = r8[i];
         }
-    } else {
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const int r = tile * 32 + pa_key(sg, i);
-            if (r >= kv_rows) {
-                r8[i] = zero;
-            } else if (qkv && r >= start_pos) {
-                const float *src = qkv + (size_t)(r - start_pos) * VT_QKV_DIM + VT_Q_DIM + (is_v ? VT_KV_DIM : 0) + col;
-                f32x4 k = *reinterpret_cast<const f32x4 *>(src);
-                for (int p = 1; p < planes; p++) {
-                    const f32x4 k2 = *reinterpret_cast<const f32x4 *>(src + p * plane_stride);
-                    k.x = __fadd_rn(k.x, k2.x); k.y = __fadd_rn(k.y, k2.y); k.z = __fadd_rn(k.z, k2.z); k.w = __fadd_rn(k.w, k2.w);
-                }
-                if (!is_v) {
-                    const f32x4 c = *reinterpret_cast<const f32x4 *>(rope + (size_t)r * VT_HEAD_DIM + 4 * cg);
-                    k = f32x4{__fsub_rn(__fmul_rn(k.x, c.x), __fmul_rn(k.y, c.y)), __fadd_rn(__fmul_rn(k.x, c.y), __fmul_rn(k.y, c.x)),
-                              __fsub_rn(__fmul_rn(k.z, c.z), __fmul_rn(k.w, c.w)), __fadd_rn(__fmul_rn(k.z, c.w), __fmul_rn(k.w, c.z))};
-                }
-                *reinterpret_cast<f32x4 *>(cache + (size_t)r * VT_KV_DIM + col) = k;
-                r8[i] = k;
-            } else {
-                r8[i] = *reinterpret_cast<const f32x4 *>(cache + (size_t)r * VT_KV_DIM + col);
-            }
-        }
+        if (r >= kv_rows) r8[i] = zero;
     }
     unsigned char *Kt = img + ((size_t)kvh * img_tiles + tile) * PA_TILE_BYTES, *Vt = Kt + 2 * PA_PLANE;
     if (!is_v) {
@@ -503,9 +490,10 @@ extern "C" void tts_hip_llm_prefill_out(const float *embeds, int seq_len, int st
     }
     const int m_tiles = (seq_len + 127) / 128;
     vt_gemm_plan pq, po, pg, pd;      /* q|k|v, output, gate|up, down */
-    vt_gemm_plan pkv = {};            /* k|v alone */
+    vt_gemm_plan pkv = {};            /* k|v alone: its columns, with the last 64 of q where strips of 96 take them */
+    const int kv0 = vt_gemm_rows_ok(seq_len, VT_QKV_DIM, VT_DIM) ? VT_Q_DIM - 64 : VT_Q_DIM;
     if (frag) {
-        pkv = vt_gemm_frag_plan(seq_len, 2 * VT_KV_DIM, VT_DIM, 0);
+        pkv = vt_gemm_frag_plan(seq_len, VT_QKV_DIM - kv0, VT_DIM, 0);
         pq = vt_gemm_frag_plan(seq_len, VT_QKV_DIM, VT_DIM, 0);
         po = vt_gemm_frag_plan(seq_len, VT_DIM, VT_Q_DIM, 0);
         pg = vt_gemm_frag_plan(seq_len, 2 * VT_FFN, VT_DIM, 1);
@@ -541,9 +529,9 @@ extern "C" void tts_hip_llm_prefill_out(const float *embeds, int seq_len, int st
             /* the caller wants the cache only: behind the last layer's k and v nothing of it is read, and q is not
              * either.  25.08 of 26 layers' products remain: prefills of
              * 37, 226, 512, 1531 rows take 0.968, 0.950, 0.974, 0.944 of their time. */
-            vt_launch_gemm_frag(wide + VT_Q_DIM, VT_QKV_DIM, S * VT_QKV_DIM, hi, lo, F->wqkv + (size_t)VT_Q_DIM * VT_DIM,
-                                seq_len, 2 * VT_KV_DIM, VT_DIM, pkv);
-            vt_pa_launch_image(img, wide, VT_Q_DIM + pkv.col0, pkv.cuts, S * VT_QKV_DIM, kc, vc, seq_len, start_pos);
+            vt_launch_gemm_frag(wide + kv0, VT_QKV_DIM, S * VT_QKV_DIM, hi, lo, F->wqkv + (size_t)kv0 * VT_DIM,
+                                seq_len, VT_QKV_DIM - kv0, VT_DIM, pkv);
+            vt_pa_launch_image(img, wide, kv0 + pkv.col0, pkv.cuts, S * VT_QKV_DIM, kc, vc, seq_len, start_pos);
             break;
         }
         if (frag) vt_launch_gemm_frag(wide, VT_QKV_DIM, S * VT_QKV_DIM, hi, lo, F->wqkv, seq_len, VT_QKV_DIM, VT_DIM, pq);
