@@ -345,7 +345,14 @@ vt_codec_attention_split_kernel(cd_planes out, const float *__restrict__ qkv, in
 __global__ void __launch_bounds__(256)
 vt_codec_embed_kernel(cd_planes a, const int *__restrict__ codes, const float *__restrict__ sem, int T) {
     __shared__ float red[4];
+    __shared__ int code[CD_IN_TAPS][37];
     const int t = blockIdx.x, base = threadIdx.x * 4;
+    /* each code once (they may lie in host memory) */
+    if (threadIdx.x < CD_IN_TAPS * 37) {
+        const int k = threadIdx.x / 37, src = abs(t + k - (CD_IN_TAPS - 1));
+        code[k][threadIdx.x % 37] = src < T ? codes[(size_t)src * 37 + threadIdx.x % 37] : 0;
+    }
+    __syncthreads();
     f32x4 v = {0.f, 0.f, 0.f, 0.f};
     if (base < CD_IN_K)
 #pragma unroll
@@ -353,16 +360,13 @@ vt_codec_embed_kernel(cd_planes a, const int *__restrict__ codes, const float *_
             const int idx = base + i;
             if (idx < CD_IN_TAPS * CD_EMBED) {
                 const int k = idx / CD_EMBED, c = idx % CD_EMBED;
-                int src = t + k - (CD_IN_TAPS - 1);
-                if (src < 0) src = -src;
-                if (src < T) {
-                    const int *fc = codes + (size_t)src * 37;
+                if (abs(t + k - (CD_IN_TAPS - 1)) < T) {
                     if (c < CD_SEM_DIM) {
-                        int s = fc[0] - 2;
+                        int s = code[k][0] - 2;
                         s = s < 0 ? 0 : s >= CD_SEM_SIZE ? CD_SEM_SIZE - 1 : s;
                         v[i] = sem[(size_t)s * CD_SEM_DIM + c];
                     } else {
-                        int q = fc[c - CD_SEM_DIM + 1] - 2;
+                        int q = code[k][c - CD_SEM_DIM + 1] - 2;
                         q = q < 0 ? 0 : q > 20 ? 20 : q;
                         v[i] = (float)q * 2.0f / 20.0f - 1.0f;
                     }
@@ -374,12 +378,12 @@ vt_codec_embed_kernel(cd_planes a, const int *__restrict__ codes, const float *_
     if (threadIdx.x == 0) a.exp[t] = e;
 }
 
-/* waveform row t: bias + the sum over the output convolution's taps k of tap k's columns of product row src(t, k),
+/* waveform row t, t0 + 0 .. of a launch: bias + the sum over the output convolution's taps k of tap k's columns of product row src(t, k),
  * stride 1, left reflection as above */
 template <int C>
 __global__ void __launch_bounds__(64)
-vt_codec_wave_kernel(float *__restrict__ out, cd_product in, const float *__restrict__ bias) {
-    const int t = blockIdx.x, c = threadIdx.x * 4;
+vt_codec_wave_kernel(float *__restrict__ out, cd_product in, const float *__restrict__ bias, int t0) {
+    const int t = t0 + blockIdx.x, c = threadIdx.x * 4;
     if (c >= CD_PATCH) return;
     f32x4 v = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -404,6 +408,8 @@ struct cd_layer_dev {
     int window;
 };
 
+#define CD_WAVE_PARTS 16
+
 static struct {
     int uploaded;
     float *sem;                   /* [8192, 256] */
@@ -418,6 +424,9 @@ static struct {
     size_t work_bytes;
     float *x, *qkv, *part, *wave;
     cd_planes planes;
+    unsigned char *host;          /* pinned: the waveform of the largest decode so far and its codes (7828 bytes a frame) */
+    size_t host_bytes;
+    hipEvent_t written[CD_WAVE_PARTS];
     int *codes;
 } g_cd;
 
@@ -442,6 +451,9 @@ void vt_codec_free(void) {
     for (int i = 0; i < 3; i++) { cd_free_matrix(&g_cd.w_up[i]); cd_free_ptr(&g_cd.b_up[i]); }
     cd_free_matrix(&g_cd.w_out); cd_free_ptr(&g_cd.b_out);
     if (g_cd.work) (void)hipFree(g_cd.work);
+    if (g_cd.host) (void)hipHostFree(g_cd.host);
+    for (int i = 0; i < CD_WAVE_PARTS; i++)
+        if (g_cd.written[i]) (void)hipEventDestroy(g_cd.written[i]);
     memset(&g_cd, 0, sizeof g_cd);
 }
 
@@ -671,11 +683,11 @@ static void cd_row(const cd_product &in, bool up, const float *x_in, const float
 #undef CALL
 }
 
-/* the whole decoder on the library's stream: d_codes [n_frames, 37] -> d_samples [n_frames * 1920] */
-static int cd_enqueue(const int *d_codes, int n_frames, float *d_samples) {
+/* the decoder up to the output convolution's product, on the library's stream: codes [n_frames, 37] */
+static cd_product cd_enqueue(const int *codes, int n_frames) {
     int T = n_frames;
     const float scale = 1.0f / sqrtf((float)CD_HEAD_DIM);
-    hipLaunchKernelGGL(vt_codec_embed_kernel, dim3(T), dim3(256), 0, g_vt.stream, g_cd.planes, d_codes, g_cd.sem, T);
+    hipLaunchKernelGGL(vt_codec_embed_kernel, dim3(T), dim3(256), 0, g_vt.stream, g_cd.planes, codes, g_cd.sem, T);
     cd_product p = cd_gemm(T, g_cd.w_in);
     cd_row(p, false, NULL, g_cd.b_in, NULL, g_cd.layers[0].attention_norm);
     for (int li = 0; li < CD_LAYERS; li++) {
@@ -705,12 +717,18 @@ static int cd_enqueue(const int *d_codes, int n_frames, float *d_samples) {
             T *= 2;
         }
     }
-    p = cd_gemm(T, g_cd.w_out);
-#define CALL(C) hipLaunchKernelGGL(vt_codec_wave_kernel<C>, dim3(T), dim3(64), 0, g_vt.stream, d_samples, p, g_cd.b_out)
+    return cd_gemm(T, g_cd.w_out);
+}
+
+/* rows t0 .. t1 - 1 of the waveform from that product */
+static int cd_wave(float *samples, const cd_product &p, int t0, int t1) {
+#define CALL(C) hipLaunchKernelGGL(vt_codec_wave_kernel<C>, dim3(t1 - t0), dim3(64), 0, g_vt.stream, samples, p, g_cd.b_out, t0)
     CD_BY_CUTS(p.cuts, CALL);
 #undef CALL
     return vt_check(hipGetLastError(), "codec launch");
 }
+
+static int cd_enqueue_all(const int *codes, int n_frames, float *d_samples) { return cd_wave(d_samples, cd_enqueue(codes, n_frames), 0, n_frames * 8); }
 
 static int cd_ready(const char *who, int n_frames) {
     if (!g_vt.initialized || !g_cd.uploaded) { vt_set_error("%s: codec weights not uploaded", who); return -1; }
@@ -719,11 +737,27 @@ static int cd_ready(const char *who, int n_frames) {
     return 0;
 }
 
+/* pinned memory and the events of the waveform's parts */
+#define CD_WAVE_PART_BYTES (480 << 10)
+static int cd_host(size_t bytes) {
+    for (int i = 0; i < CD_WAVE_PARTS; i++)
+        if (!g_cd.written[i] && vt_check(hipEventCreateWithFlags(&g_cd.written[i], hipEventDisableTiming), "codec event")) return -1;
+    if (bytes <= g_cd.host_bytes) return 0;
+    (void)hipStreamSynchronize(g_vt.stream);
+    if (g_cd.host) (void)hipHostFree(g_cd.host);
+    g_cd.host_bytes = 0;
+    g_cd.host = NULL;
+    bytes = (bytes + ((1 << 20) - 1)) & ~(size_t)((1 << 20) - 1);
+    if (vt_check(hipHostMalloc((void **)&g_cd.host, bytes, hipHostMallocDefault), "codec host memory")) { g_cd.host = NULL; return -1; }
+    g_cd.host_bytes = bytes;
+    return 0;
+}
+
 /* device codes -> device waveform (n_frames * 1920 floats), asynchronous on the library's stream */
 extern "C" int tts_hip_codec_decode_device(const int *d_codes, int n_frames, float *d_samples) {
     if (cd_ready("tts_hip_codec_decode_device", n_frames)) return -1;
     if (!d_codes || !d_samples) { vt_set_error("tts_hip_codec_decode_device: NULL buffer"); return -1; }
-    return cd_enqueue(d_codes, n_frames, d_samples);
+    return cd_enqueue_all(d_codes, n_frames, d_samples);
 }
 
 /* replaces tts_codec_decode (voxtral_tts_codec.c:389): host codes [n_frames, 37] -> a malloc'ed
@@ -733,13 +767,29 @@ extern "C" void tts_hip_codec_decode(const int *codes, int n_frames, float **out
     if (out_n_samples) *out_n_samples = 0;
     if (!codes || !out_samples || !out_n_samples) { vt_set_error("tts_hip_codec_decode: NULL argument"); return; }
     if (cd_ready("tts_hip_codec_decode", n_frames)) return;
-    const int n = n_frames * 8 * CD_PATCH;
+    const int rows = n_frames * 8, n = rows * CD_PATCH;
+    const size_t code_bytes = (size_t)n_frames * 37 * sizeof(int);
+    if (cd_host((size_t)n * sizeof(float) + code_bytes)) { vt_set_error("tts_hip_codec_decode: out of host memory"); return; }
     float *s = (float *)malloc((size_t)n * sizeof(float));
     if (!s) { vt_set_error("tts_hip_codec_decode: out of host memory"); return; }
-    if (vt_check(hipMemcpyAsync(g_cd.codes, codes, (size_t)n_frames * 37 * sizeof(int), hipMemcpyHostToDevice, g_vt.stream), "codes copy") ||
-        cd_enqueue(g_cd.codes, n_frames, g_cd.wave) ||
-        vt_check(hipMemcpyAsync(s, g_cd.wave, (size_t)n * sizeof(float), hipMemcpyDeviceToHost, g_vt.stream), "waveform copy") ||
-        vt_check(hipStreamSynchronize(g_vt.stream), "codec decode")) {
+    /* Codes and samples cross through pinned memory that the kernels read and write themselves; the caller's buffer is filled
+     * part by part behind the last kernel's launches.  Where the codes and the waveform were copied
+     * from and into pageable memory, calls of 2 / 21 / 212 / 1003 frames took 508 / 737 / 1630 / 5020 us; 453 / 695 / 1596 / 4791
+     * now, of which 8 / 21 / 95 / 273 behind the device's work. */
+    float *wave = (float *)g_cd.host;
+    int *host_codes = (int *)(wave + n);
+    memcpy(host_codes, codes, code_bytes);
+    const cd_product p = cd_enqueue(host_codes, n_frames);
+    int parts = (int)((size_t)n * sizeof(float) / CD_WAVE_PART_BYTES), bad = 0;
+    parts = parts < 1 ? 1 : parts < CD_WAVE_PARTS ? parts : CD_WAVE_PARTS;
+    auto first = [&](int i) { return (int)((long long)rows * i / parts); };
+    for (int i = 0; i < parts && !bad; i++)
+        bad = cd_wave(wave, p, first(i), first(i + 1)) || (i + 1 < parts && vt_check(hipEventRecord(g_cd.written[i], g_vt.stream), "codec decode"));
+    for (int i = 0; i < parts && !bad; i++) {
+        bad = vt_check(i + 1 < parts ? hipEventSynchronize(g_cd.written[i]) : hipStreamSynchronize(g_vt.stream), "codec decode");
+        if (!bad) memcpy(s + (size_t)first(i) * CD_PATCH, wave + (size_t)first(i) * CD_PATCH, (size_t)(first(i + 1) - first(i)) * CD_PATCH * sizeof(float));
+    }
+    if (bad) {
         free(s);
         return;
     }
@@ -775,7 +825,7 @@ int vt_codec_probe_launch(int which) {
     const int frames = 200;
     const cd_layer_dev *l = &g_cd.layers[CD_LAYERS - 1];
     const cd_matrix *w[4] = {&l->wqkv, &l->wo, &l->w13, &l->w2};
-    if (which == 4) return cd_enqueue(g_cd.codes, frames, g_cd.wave);
+    if (which == 4) return cd_enqueue_all(g_cd.codes, frames, g_cd.wave);
     if (which < 0 || which > 3) return -1;
     (void)cd_gemm(frames * 8, *w[which]);
     return 0;
