@@ -177,7 +177,10 @@ vt_gemm_wide_kernel(gw_list list, const uint16_t *Ahi, const uint16_t *Alo, int 
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     constexpr int WP = T::WP, KW = 4 / CW, TM = 32 * MB, TN = 32 * NB * CW;
     constexpr int NP = 4 * MB / CW;                        /* staging passes over a plane, 8 * CW rows each */
-    constexpr int AHEAD = MB * NB > 8 && CW == 2 ? 1 : 2;  /* steps between the request of a step's planes and their store (registers) */
+    constexpr int AHEAD = MB * NB > 9 ? 1 : 2;             /* steps between the request of a step's planes and their store (registers) */
+    /* The first requests of an item go out in front of the stores of the one before it, where registers for both are left (where
+     * they were not, a launch's first loads were spilled one by one, each behind a wait: 5 us). */
+    constexpr bool EARLY = CW == 4 || MB == 3;
     constexpr int PLANE = TM * GM_STAGE_ROW, GROUP = 2 * PLANE, STAGE = KW * GROUP;
     const int lane = (int)threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int cw = wave % CW, kw = wave / CW;              /* column block of the tile; which of the KW K steps */
@@ -382,8 +385,9 @@ vt_gemm_wide_kernel(gw_list list, const uint16_t *Ahi, const uint16_t *Alo, int 
 
     int part = 0, id = (int)blockIdx.x;
     gw_item it = gw_item_at<TN, WP>(list, 0, id, K);
-    begin(it);
+    if constexpr (EARLY) begin(it);
     for (;;) {
+        if constexpr (!EARLY) begin(it);
         multiply(it);
         id += (int)gridDim.x;
         while (part < list.n_parts && id >= list.m_tiles * list.part[part].n_tiles * list.part[part].splits) {
@@ -392,9 +396,8 @@ vt_gemm_wide_kernel(gw_list list, const uint16_t *Ahi, const uint16_t *Alo, int 
         }
         if (part >= list.n_parts) break;
         const gw_item nx = gw_item_at<TN, WP>(list, part, id, K);
-        if constexpr (AHEAD == 2) begin(nx);
+        if constexpr (EARLY) begin(nx);
         finish(it);
-        if constexpr (AHEAD == 1) begin(nx);      /* no registers for them beside the sums */
         __syncthreads();                  /* the next item stages over what this one read */
         it = nx;
     }
