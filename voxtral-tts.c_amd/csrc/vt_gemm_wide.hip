@@ -15,8 +15,8 @@
  * where 256-column tiles come in multiples of 192 items: q|k|v / output / down at 700 rows 57.5 / 40.7 / 79.4 -> 51.1 / 37.2 /
  * 72.5 us, at 1000 75.0 / 53.3 / 104.9 -> 68.5 / 49.2 / 97.0, output / down at 1531 73.3 / 149.4 -> 67.1 / 140.6.
  * Measured against every tile and cut count at 65 .. 1531 rows of the backbone's products and 84 .. 8024 of the codec's, the plan taken is
- * 1.0 % behind the fastest on average in both, at worst 11 % (q|k|v at 600 rows, whole 192-column tiles on 224 CUs instead
- * of 240 cut ones) and 17 % (the codec's q|k|v at 212 rows: 192 items, 216 faster). */
+ * 0.9 and 0.4 % behind the fastest on average, at worst 9 % (q|k|v at 600 rows, whole 192-column tiles on 224 CUs instead
+ * of 240 cut ones) and 5 %. */
 struct gw_format {
     int products;                         /* matrix instructions per pair of operands */
     float launch_us, item_us, planes;     /* planes: passes over a cut column's planes */
@@ -24,7 +24,7 @@ struct gw_format {
     float pflops[3];                      /* [128, 192, 256 columns] */
 };
 static const gw_format gw_backbone = {2, 5.0f, 2.8f, 1.45f, {{1.28f, 0.f}, {1.97f, 2.96f}, {1.15f, 1.65f}}, {0.91f, 1.07f, 1.21f}};
-static const gw_format gw_codec = {3, 6.0f, 2.0f, 1.2f, {{2.0f, 2.6f}, {0.f, 0.f}, {2.0f, 2.5f}}, {0.88f, 0.f, 1.10f}};
+static const gw_format gw_codec = {3, 6.0f, 1.0f, 1.4f, {{1.76f, 2.81f}, {0.f, 0.f}, {1.89f, 2.44f}}, {0.865f, 0.f, 0.98f}};
 
 static float gw_rounds(int items, float item_us, float power_us) {
     const int full = items / g_vt.n_cu, rem = items % g_vt.n_cu;
