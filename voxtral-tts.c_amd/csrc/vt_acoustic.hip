@@ -506,6 +506,9 @@ vt_ac_phase_kernel(ac_phase_args a, int n_units) {
  * 2.4e-6).  us per frame 1188 -> 1141: seven launches of 9.5 us fewer, one more for the LLM token's q|k|v, `front`
  * 3.8 -> 4.2. */
 
+/* A frame's results in host memory, written by its last kernel */
+struct ac_frame_out { int codes[1 + VT_AC_DIM_IN]; float x[VT_AC_DIM_IN]; int abort; };
+
 struct ac_edge_args {
     const float *tok_in;          /* [6,3072] after the last layer (back) */
     float *tok_out;               /* [6,3072] for the next step (front, when do_front) */
@@ -522,6 +525,9 @@ struct ac_edge_args {
     float *x_out;                 /* [36] latent after the update (== x_in values without do_euler) */
     float *vel;                   /* [72] cond | uncond velocities (written by back, read by front) */
     int *codes;                   /* [37] (FSQ codes at 1..36 when do_fsq) */
+    const float *logits;          /* the frame's semantic logits: one workgroup more leaves the first maximum in codes[0] */
+    ac_frame_out *host;           /* what the caller gets, in pinned memory (when do_fsq) */
+    const int *abort;             /* the backbone step's "gave up" word */
     float dt;
     int do_euler, do_front, do_fsq;
 };
@@ -585,12 +591,42 @@ vt_ac_edge_back_kernel(ac_edge_args a) {
     if (mine && lane == 0) a.vel[o] = acc;
 }
 
+/* First maximum of the masked semantic logits (voxtral_tts_acoustic.c:291-306):
+ * index 0 and indices >= 8194 are forced to -1e30; ties keep the lowest index.  One workgroup of `front`. */
+__device__ __forceinline__ void ac_semantic_argmax(const float *logits, int *out_code) {
+    __shared__ float sv[AC_FRONT_THREADS];
+    __shared__ int si[AC_FRONT_THREADS];
+    float best = -1e30f;              /* value of the masked slot 0 */
+    int bi = 0;
+#pragma unroll 11
+    for (int i = (int)threadIdx.x; i < VT_SEM_VALID_END; i += AC_FRONT_THREADS) {
+        const float v = i == 0 ? -1e30f : logits[i];
+        if (v > best) { best = v; bi = i; }          /* ascending i per thread: first max kept */
+    }
+    sv[threadIdx.x] = best;
+    si[threadIdx.x] = bi;
+    __syncthreads();
+    for (int s = AC_FRONT_THREADS / 2; s > 0; s >>= 1) {
+        if ((int)threadIdx.x < s) {
+            const float v = sv[threadIdx.x + s];
+            const int j = si[threadIdx.x + s];
+            if (v > sv[threadIdx.x] || (v == sv[threadIdx.x] && j < si[threadIdx.x])) {
+                sv[threadIdx.x] = v;
+                si[threadIdx.x] = j;
+            }
+        }
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) *out_code = si[0];
+}
+
 __global__ void __launch_bounds__(AC_FRONT_THREADS)
 vt_ac_edge_front_kernel(ac_edge_args a) {
     __shared__ float s_vel[2 * VT_AC_DIM_IN];
     __shared__ float s_x[VT_AC_DIM_IN];
     __shared__ double s_ss[VT_AC_DIM_IN];
     const int t = (int)threadIdx.x;
+    if (a.logits && blockIdx.x + 1 == gridDim.x) { ac_semantic_argmax(a.logits, a.codes); return; }
     const bool tok = (int)blockIdx.x < AC_FRONT_TOK_WGS;
     const int c = t + AC_FRONT_THREADS * ((int)blockIdx.x - (tok ? 0 : AC_FRONT_TOK_WGS));  /* this thread's token or q|k|v column */
     /* what does not depend on the latent is requested first: the column's row of the input projection or of its
@@ -634,6 +670,9 @@ vt_ac_edge_front_kernel(ac_edge_args a) {
                 if (q < 0) q = 0;
                 if (q > 20) q = 20;
                 a.codes[t + 1] = q + 2;
+                a.host->codes[t + 1] = q + 2;
+                a.host->x[t] = xn;
+                if (t == 0) { a.host->codes[0] = a.codes[0]; a.host->abort = *a.abort; }
             }
         }
     }
@@ -718,39 +757,12 @@ int vt_ac_fold_noise(void) {
     return vt_check(hipGetLastError(), "acoustic fold") || vt_check(hipStreamSynchronize(g_vt.stream), "acoustic fold") ? -1 : 0;
 }
 
-/* First maximum of the masked semantic logits (voxtral_tts_acoustic.c:291-306):
- * index 0 and indices >= 8194 are forced to -1e30; ties keep the lowest index. */
-__global__ void __launch_bounds__(1024) vt_semantic_argmax_kernel(const float *logits, int *out_code) {
-    __shared__ float sv[1024];
-    __shared__ int si[1024];
-    float best = -1e30f;              /* value of the masked slot 0 */
-    int bi = 0;
-    for (int i = (int)threadIdx.x; i < VT_SEM_PADDED; i += (int)blockDim.x) {
-        const float v = (i == 0 || i >= VT_SEM_VALID_END) ? -1e30f : logits[i];
-        if (v > best) { best = v; bi = i; }          /* ascending i per thread: first max kept */
-    }
-    sv[threadIdx.x] = best;
-    si[threadIdx.x] = bi;
-    __syncthreads();
-    for (int s = (int)blockDim.x / 2; s > 0; s >>= 1) {
-        if ((int)threadIdx.x < s) {
-            const float v = sv[threadIdx.x + s];
-            const int j = si[threadIdx.x + s];
-            if (v > sv[threadIdx.x] || (v == sv[threadIdx.x] && j < si[threadIdx.x])) {
-                sv[threadIdx.x] = v;
-                si[threadIdx.x] = j;
-            }
-        }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) *out_code = si[0];
-}
-
 /* ---- host side ---------------------------------------------------------------------- */
 
 /* device work area of the acoustic path, in floats */
 struct ac_work {
     float *tok, *qkv, *h, *llm_tok, *hidden, *x, *x2, *vel, *temb, *time_tok1, *logits;
+    const float *x0;              /* a frame's noise, in pinned memory: read once */
     float *llm_qkv, *time_qkv1;   /* the first layer's q|k|v of llm_tok and time_tok1 */
     int *codes;
 };
@@ -773,6 +785,7 @@ static void carve(ac_work *w, float *base) {
     w->x2 = w->vel + 80;                                 /* vel uses 72 of its 128 floats */
     w->logits = w->vel + 128;
     w->codes = (int *)(w->logits + VT_SEM_PADDED);
+    w->x0 = NULL;
 }
 
 template <int PH, int ROWS = AC_ROWS>
@@ -844,7 +857,7 @@ float *vt_ac_work_area(size_t *n_floats) {
  * launches of the frame so far; the caller keeps it. */
 struct ac_tokens { const float *time_tok, *time_qkv, *llm_tok, *llm_qkv; };
 
-static void launch_edge(const ac_work *w, const ac_tokens &tk, float dt, int back, int euler, int front, int fsq, int *flip) {
+static void launch_edge(const ac_work *w, const ac_tokens &tk, float dt, int back, int euler, int front, int fsq, int *flip, const float *logits = NULL) {
     const vt_acoustic_dev *ac = &g_vt.ac;
     ac_edge_args a;
     a.tok_in = w->tok; a.tok_out = w->tok; a.norm = ac->norm; a.acoustic_out = ac->acoustic_out;
@@ -852,11 +865,14 @@ static void launch_edge(const ac_work *w, const ac_tokens &tk, float dt, int bac
     a.noise_gram = ac->noise_gram; a.qkv_out = w->qkv; a.vel = w->vel;
     a.time_tok = tk.time_tok; a.time_qkv = tk.time_qkv; a.llm_tok = tk.llm_tok; a.llm_qkv = tk.llm_qkv;
     a.codes = w->codes; a.dt = dt; a.do_euler = euler; a.do_front = front; a.do_fsq = fsq;
-    a.x_in = (*flip & 1) ? w->x2 : w->x;
+    a.logits = logits;
+    a.host = (ac_frame_out *)(g_vt.h_pin + VT_PIN_FRAME);
+    a.abort = g_vt.d_abort;
+    a.x_in = *flip == 0 && w->x0 ? w->x0 : (*flip & 1) ? w->x2 : w->x;
     a.x_out = (*flip & 1) ? w->x : w->x2;
     if (back) hipLaunchKernelGGL(vt_ac_edge_back_kernel, dim3(AC_BACK_WGS), dim3(1024), 0, g_vt.stream, a);
     if (euler || front || fsq) {
-        hipLaunchKernelGGL(vt_ac_edge_front_kernel, dim3(front ? AC_FRONT_WGS : 1), dim3(AC_FRONT_THREADS), 0, g_vt.stream, a);
+        hipLaunchKernelGGL(vt_ac_edge_front_kernel, dim3((front ? AC_FRONT_WGS : 1) + (logits ? 1 : 0)), dim3(AC_FRONT_THREADS), 0, g_vt.stream, a);
         *flip += 1;
     }
 }
@@ -985,10 +1001,17 @@ extern "C" void tts_hip_predict_velocity_cfg(float *out_v_cond, float *out_v_unc
     predict(out_v_cond, out_v_uncond, x_t, llm_hidden, t_val);
 }
 
-/* Enqueues one frame: semantic head + argmax, 7 guided Euler steps, FSQ.  d_or_h_hidden may
- * be a host or a device pointer.  Codes end up in w->codes, the latent in w->x; nothing is
- * synchronised. */
-static int enqueue_frame(ac_work *w, const float *d_or_h_hidden, const float *x0) {
+/* n floats of pinned memory, a kernel's launch instead of a copy's */
+__global__ void vt_ac_fetch_kernel(float *out, const float *in, int n) {
+    const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    if (i < n) out[i] = in[i];
+}
+
+/* Enqueues one frame: semantic head + argmax, 7 guided Euler steps, FSQ.  The hidden state is the caller's (h_hidden, host)
+ * or the backbone step's (d_hidden).  Codes end up in w->codes, the latent in w->x and both in the pinned ac_frame_out;
+ * nothing is synchronised.  The frame's only traffic with the host is what its kernels read and write there: five
+ * copies of 144 bytes to 12 KB, the argmax in a launch of its own and the hidden state copied on the device were 9 us of a frame. */
+static int enqueue_frame(ac_work *w, const float *h_hidden, const float *d_hidden, const float *x0) {
     hipStream_t st = g_vt.stream;
     vt_acoustic_dev *ac = &g_vt.ac;
     float *base = (float *)vt_scratch(sizeof(float) * AC_WORK_FLOATS);
@@ -997,16 +1020,20 @@ static int enqueue_frame(ac_work *w, const float *d_or_h_hidden, const float *x0
     float ts[AC_STEPS + 1];
     for (int i = 0; i <= AC_STEPS; i++) ts[i] = (float)i / (float)AC_STEPS;
     if (ensure_time_grid(w->temb)) return -1;            /* the projected time tokens depend on the weights only */
-    if (vt_check(hipMemcpyAsync(w->hidden, d_or_h_hidden, sizeof(float) * VT_DIM, hipMemcpyDefault, st), "frame hidden")) return -1;
-    if (vt_check(hipMemcpyAsync(w->x, x0, sizeof(float) * VT_AC_DIM_IN, hipMemcpyDefault, st), "frame noise")) return -1;
-    vt_launch_linear(w->logits, w->hidden, ac->semantic_out, ac->semantic_bias, 1, VT_DIM, VT_SEM_PADDED);
-    hipLaunchKernelGGL(vt_semantic_argmax_kernel, dim3(1), dim3(1024), 0, st, w->logits, w->codes);
-    vt_launch_linear(w->llm_tok, w->hidden, ac->llm_proj, NULL, 1, VT_DIM, VT_DIM);
+    memcpy(g_vt.h_pin + VT_PIN_X0, x0, sizeof(float) * VT_AC_DIM_IN);
+    w->x0 = g_vt.h_pin + VT_PIN_X0;
+    if (h_hidden) {
+        memcpy(g_vt.h_pin + VT_PIN_HIDDEN, h_hidden, sizeof(float) * VT_DIM);
+        hipLaunchKernelGGL(vt_ac_fetch_kernel, dim3(VT_DIM / 256), dim3(256), 0, st, w->hidden, g_vt.h_pin + VT_PIN_HIDDEN, VT_DIM);
+        d_hidden = w->hidden;
+    }
+    vt_launch_linear(w->logits, d_hidden, ac->semantic_out, ac->semantic_bias, 1, VT_DIM, VT_SEM_PADDED);
+    vt_launch_linear(w->llm_tok, d_hidden, ac->llm_proj, NULL, 1, VT_DIM, VT_DIM);
     if (project_qkv(w->llm_qkv, w->llm_tok)) return -1;
     /* the flow runs without waiting for the semantic code; an END_AUDIO frame discards it */
     int flip = 0;                                        /* 1 + AC_STEPS front launches: the latent ends in w->x */
     ac_tokens tk = {ac->time_tok, ac->time_qkv, w->llm_tok, w->llm_qkv};
-    launch_edge(w, tk, 0.f, 0, 0, 1, 0, &flip);
+    launch_edge(w, tk, 0.f, 0, 0, 1, 0, &flip, w->logits);
     for (int s = 0; s < AC_STEPS; s++) {
         volatile float dt = ts[s + 1] - ts[s];
         if (run_layers(w)) return -1;
@@ -1017,22 +1044,16 @@ static int enqueue_frame(ac_work *w, const float *d_or_h_hidden, const float *x0
     return vt_check(hipGetLastError(), "frame launch");
 }
 
-static void finish_frame(const ac_work *w, int *out_codes, float *out_x) {
-    /* codes, latent and the backbone step's "gave up" word come back through pinned memory behind ONE wait
-     * (three blocking copies were 1 % of a turn of the generation loop) */
-    hipStream_t st = g_vt.stream;
-    int *pin_codes = (int *)g_vt.h_pin, *pin_flag = (int *)(g_vt.h_pin + 128);
-    float *pin_x = g_vt.h_pin + 64;
-    VT_TRYV(hipMemcpyAsync(pin_codes, w->codes, sizeof(int) * (1 + VT_AC_DIM_IN), hipMemcpyDeviceToHost, st));
-    VT_TRYV(hipMemcpyAsync(pin_x, w->x, sizeof(float) * VT_AC_DIM_IN, hipMemcpyDeviceToHost, st));
-    VT_TRYV(hipMemcpyAsync(pin_flag, g_vt.d_abort, sizeof(int), hipMemcpyDeviceToHost, st));
-    VT_TRYV(hipStreamSynchronize(st));
+static void finish_frame(int *out_codes, float *out_x) {
+    const ac_frame_out *pin = (const ac_frame_out *)(g_vt.h_pin + VT_PIN_FRAME);
+    VT_TRYV(hipGetLastError());
+    VT_TRYV(hipStreamSynchronize(g_vt.stream));
     if (g_vt.step_pending) {                /* the backbone step in front of this frame: was it abandoned? */
         g_vt.step_pending = 0;
-        if (pin_flag[0]) { (void)vt_step_poll_abort_now(); return; }
+        if (pin->abort) { (void)vt_step_poll_abort_now(); return; }
     }
-    memcpy(out_codes, pin_codes, sizeof(int) * (1 + VT_AC_DIM_IN));
-    if (out_x) memcpy(out_x, pin_x, sizeof(float) * VT_AC_DIM_IN);
+    memcpy(out_codes, pin->codes, sizeof(int) * (1 + VT_AC_DIM_IN));
+    if (out_x) memcpy(out_x, pin->x, sizeof(float) * VT_AC_DIM_IN);
     if (out_codes[0] == 1) {                            /* END_AUDIO */
         for (int i = 1; i <= VT_AC_DIM_IN; i++) out_codes[i] = 2;
         if (out_x) memset(out_x, 0, sizeof(float) * VT_AC_DIM_IN);
@@ -1043,8 +1064,8 @@ extern "C" void tts_hip_acoustic_frame(int *out_codes, const float *llm_hidden, 
                                        float *out_x) {
     if (!ac_ready("tts_hip_acoustic_frame")) return;
     ac_work w;
-    if (enqueue_frame(&w, llm_hidden, x0)) return;
-    finish_frame(&w, out_codes, out_x);
+    if (enqueue_frame(&w, llm_hidden, NULL, x0)) return;
+    finish_frame(out_codes, out_x);
 }
 
 /* ---- audio-code embedding and the per-frame loop -------------------------------------- */
@@ -1113,9 +1134,9 @@ extern "C" void tts_hip_generate_frame(int *out_codes, float *d_embed, const flo
     if (g_vt.n_dec_layers < 1) { vt_set_error("tts_hip_generate_frame: no backbone weights uploaded"); return; }
     if (vt_run_step(g_vt.d_layers, g_vt.n_dec_layers, 0, g_vt.d_dec_norm, d_embed, g_vt.d_hidden, pos)) return;
     ac_work w;
-    if (enqueue_frame(&w, g_vt.d_hidden, x0)) return;
+    if (enqueue_frame(&w, NULL, g_vt.d_hidden, x0)) return;
     vt_acoustic_dev *ac = &g_vt.ac;
     hipLaunchKernelGGL(vt_audio_embed_kernel, dim3(VT_DIM / 256), dim3(256), 0, g_vt.stream, d_embed, ac->audio_emb,
                        ac->audio_offsets, w.codes, ac->audio_rows);
-    finish_frame(&w, out_codes, NULL);
+    finish_frame(out_codes, NULL);
 }

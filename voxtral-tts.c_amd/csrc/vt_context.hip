@@ -132,7 +132,7 @@ static int init_context(int kv_cache_max) {
         VT_TRY(hipMemset(*bufs[i].p, 0, bufs[i].bytes));
     }
     g_vt.bar_epoch = 0;
-    VT_TRY(hipHostMalloc((void **)&g_vt.h_pin, sizeof(float) * (2 * VT_DIM + 64), hipHostMallocDefault));
+    VT_TRY(hipHostMalloc((void **)&g_vt.h_pin, sizeof(float) * VT_PIN_FLOATS, hipHostMallocDefault));
     VT_TRY(hipDeviceSynchronize());
 
     g_hip.n_cu = g_vt.n_cu;

@@ -79,7 +79,7 @@ struct vt_state {
     unsigned long long bar_timeout; /* spin budget of a barrier in 100 MHz ticks; 0 = default */
     int *d_abort;
     uint16_t *d_dummy;            /* small resident block requested in place of a layer beyond the last */
-    float *h_pin;                 /* pinned staging: [3072 in][3072 out + flag] */
+    float *h_pin;                 /* pinned staging: [3072 in][3072 out + flag], and a frame's hidden state, noise and results */
 
     /* generic scratch (prefill / acoustic / linear) */
     void *d_scratch;
@@ -90,6 +90,12 @@ struct vt_state {
     int error_count;
     char last_error[512];
 };
+
+/* floats into h_pin; the last part holds an ac_frame_out */
+#define VT_PIN_HIDDEN (2 * VT_DIM + 64)
+#define VT_PIN_X0 (VT_PIN_HIDDEN + VT_DIM)
+#define VT_PIN_FRAME (VT_PIN_X0 + 64)
+#define VT_PIN_FLOATS (VT_PIN_FRAME + 128)
 
 extern vt_state g_vt;
 
