@@ -13,8 +13,10 @@
 #include <stdlib.h>
 
 /* ---- linear: y[s,o] = bias[o] + sum_k W[o,k] x[s,k] ------------------------- */
-/* One wave per output row; up to S rows of x share each weight load. */
-template <int S>
+/* One wave per output row and up to S rows of x, which share each weight load: shapes that the kernels below do not take.
+ * GROUPS: more than S rows, group blockIdx.y of them (known to start at 0 otherwise, which is 6 % of 36 x 3072 at 5 rows;
+ * 36 x 3072 at 300 rows took 258 us when a wave went through all groups, 11 now on the matrix cores). */
+template <int S, bool GROUPS>
 __global__ void __launch_bounds__(256)
 vt_linear_kernel(float *y, const float *x, const uint16_t *W, const float *bias,
                  int seq_len, int in_dim, int out_dim, int vec_ok) {
@@ -22,7 +24,7 @@ vt_linear_kernel(float *y, const float *x, const uint16_t *W, const float *bias,
     if (row >= out_dim) return;
     const int lane = vt_lane();
     const uint16_t *wr = W + (size_t)row * in_dim;
-    for (int s0 = 0; s0 < seq_len; s0 += S) {
+    for (int s0 = GROUPS ? (int)blockIdx.y * S : 0; s0 < seq_len; s0 += GROUPS ? (int)gridDim.y * S : S) {
         float acc[S];
 #pragma unroll
         for (int s = 0; s < S; s++) acc[s] = 0.f;
@@ -175,20 +177,190 @@ static int matvec_launch(float *d_y, const float *d_x, const uint16_t *d_W, cons
     return 1;
 }
 
+/* ---- a few rows: fp32 on the matrix cores ------------------------------------------------------------------
+ * y[s,o] for up to 16 rows s per workgroup row (blockIdx.y): a stream of W like the single-row product, on
+ * v_mfma_f32_16x16x4_f32, so that operands, products and sums are fp32 (bf16 weights widened exactly).  A workgroup owns
+ * rows_per_wg consecutive rows of W, its eight waves share K: wave w keeps its K slice of x in registers as the B operand,
+ * 16 weight rows at a time come as the A operand (lane l: row l%16, 8 consecutive k of group l/16; the k order inside an
+ * instruction is free as long as both operands agree), and the waves' sums are added through LDS in wave order, one barrier
+ * per 16 rows.  A wave's piece of 16 rows comes in P parts of H lines of 128 bytes per row, by buffer loads straight into three LDS
+ * buffers of its own: eight lanes bring a line (lane i its 16-byte piece i%8 ^ row%8, so that eight lanes reading one piece
+ * of eight rows meet all banks), two parts are on their way while one is multiplied, and a wave waits for nothing but its own loads.
+ * (Loaded into the operands directly, an instruction touches 64 pieces of 16 bytes, and the CU's address path takes
+ * twice as long as the stream.)  Three arrays, so that the compiler knows that reading one need not wait for the others.  K of
+ * more than 512 H P takes its slices in passes.
+ * An instruction does 16 weight rows and 16 rows of x in 32 cycles, so that a CU could take 38 KB of weights per us, half
+ * as much again as its share of HBM.  us per call at 2 / 5 / 8 / 16 rows, 9216 x 3072: 18.2 / 18.7 / 19.0 / 21.0; 131072 x 3072: 145 / 143 / 144 / 149; with a wave per
+ * weight row and, from 8 rows on, planes, tiles and partial sums in three launches: 14 / 25 / 24 / 25 and 195 / 329 / 184 / 198. */
+#define LR_ROWS 16
+template <int N> struct lr_int { static constexpr int v = N; };
+template <int H, int P>
+__global__ void __launch_bounds__(512)
+vt_linear_rows_kernel(float *y, const float *x, const uint16_t *W, const float *bias, int seq_len, int in_dim, int out_dim, int rows_per_wg) {
+    constexpr int PART = 2048 * H, KW = 64 * H * P;      /* bytes of a wave's part; k of a wave and pass */
+    __shared__ __attribute__((aligned(16))) unsigned char buf0[8 * PART], buf1[8 * PART], buf2[8 * PART];
+    __shared__ float red[8][256];
+    const int lane = (int)threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), li = lane & 15, g = lane >> 4;
+    const int s0 = (int)blockIdx.y * LR_ROWS, ns = min(LR_ROWS, seq_len - s0);
+    const int row0 = (int)blockIdx.x * rows_per_wg, rows = min(rows_per_wg, out_dim - row0);
+    const int passes = in_dim / (8 * KW), per_block = passes * P, n = (rows + 15) / 16 * per_block;
+    const __amdgpu_buffer_rsrc_t xd = __builtin_amdgcn_make_buffer_rsrc((void *)(x + (size_t)s0 * in_dim), 0, ns * in_dim * 4, 0x00020000);
+    f32x4 xr[2 * H * P][2];
+    auto load_x = [&](int pass) {
+#pragma unroll
+        for (int i = 0; i < 2 * H * P; i++)
+#pragma unroll
+            for (int h = 0; h < 2; h++)
+                xr[i][h] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(xd, (li * in_dim + 8 * g + 4 * h) * 4, ((pass * 8 + wave) * KW + 32 * i) * 4, 0));
+    };
+    /* part t: block t / per_block, pass, part of the pass; past the last one: zeros, which nobody reads */
+    const int w_voff = (lane >> 3) * in_dim * 2 + ((lane & 7) ^ (lane >> 3)) * 16;
+    auto ask = [&](unsigned char *buf, int t) {
+        const int b = t / per_block, pass = t % per_block / P, part = t % P, left = min(rows - 16 * b, 16);
+        const __amdgpu_buffer_rsrc_t d = __builtin_amdgcn_make_buffer_rsrc((void *)(W + (size_t)(row0 + (t < n ? 16 * b : 0)) * in_dim), 0, t < n ? left * in_dim * 2 : 0, 0x00020000);
+#pragma unroll
+        for (int j = 0; j < 2 * H; j++)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(d, (__attribute__((address_space(3))) void *)(buf + wave * PART + j * 1024), 16, w_voff + (j & 1) * 16 * in_dim,
+                                                     ((pass * 8 + wave) * KW + part * 64 * H + 64 * (j >> 1)) * 2, 0, 2);
+    };
+    f32x4 acc[4];
+    auto multiply = [&](const unsigned char *buf, auto part) {
+        u32x4 w[2 * H];
+#pragma unroll
+        for (int i = 0; i < 2 * H; i++)
+            w[i] = *reinterpret_cast<const u32x4 *>(buf + wave * PART + ((i >> 1) * 16 + li) * 128 + ((4 * (i & 1) + g) ^ (li & 7)) * 16);
+#pragma unroll
+        for (int i = 0; i < 2 * H; i++)
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                const unsigned u = w[i][j / 2];
+                acc[j & 3] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(j & 1 ? u & 0xffff0000u : u << 16), xr[2 * H * decltype(part)::v + i][j / 4][j % 4], acc[j & 3], 0, 0, 0);
+            }
+    };
+    /* accumulator element v of lane l: weight row 4 (l/16) + v, row l%16 of x.  Bare barriers: __syncthreads() would wait for
+     * the parts on their way. */
+    auto finish = [&](int b) {
+        const f32x4 q = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();                                        /* the block before has been summed */
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int v = 0; v < 4; v++) red[wave][li * 16 + 4 * g + v] = q[v];
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(0xc07f);                                  /* lgkmcnt(0) */
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        const int t = (int)threadIdx.x, s = t >> 4, r = 16 * b + (t & 15);
+        if (t < 256 && s < ns && r < rows) {
+            float sum = red[0][t];
+#pragma unroll
+            for (int w = 1; w < 8; w++) sum = __fadd_rn(sum, red[w][t]);
+            y[(size_t)(s0 + s) * out_dim + row0 + r] = bias ? __fadd_rn(bias[row0 + r], sum) : sum;
+        }
+    };
+    auto item = [&](int t, auto part, const unsigned char *here, unsigned char *later) {
+        if (t % per_block == 0)
+#pragma unroll
+            for (int a = 0; a < 4; a++) acc[a] = f32x4{0.f, 0.f, 0.f, 0.f};
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(0x0f70 | (2 * H));                        /* vmcnt: the next part may be on its way */
+        asm volatile("" ::: "memory");
+        ask(later, t + 2);
+        asm volatile("" ::: "memory");
+        multiply(here, part);
+        if (passes > 1 && t % P == P - 1) load_x((t + 1) % per_block / P);
+        if (t % per_block == per_block - 1) finish(t / per_block);
+    };
+    load_x(0);
+    asm volatile("" ::: "memory");
+    ask(buf0, 0);
+    ask(buf1, 1);
+    constexpr int Q = P - 1;                             /* parts alternate 0, Q */
+    for (int t = 0; t < n; t += 6) {
+        item(t, lr_int<0>(), buf0, buf2);
+        if (t + 1 >= n) break;
+        item(t + 1, lr_int<Q>(), buf1, buf0);
+        if (t + 2 >= n) break;
+        item(t + 2, lr_int<0>(), buf2, buf1);
+        if (t + 3 >= n) break;
+        item(t + 3, lr_int<Q>(), buf0, buf2);
+        if (t + 4 >= n) break;
+        item(t + 4, lr_int<0>(), buf1, buf0);
+        if (t + 5 >= n) break;
+        item(t + 5, lr_int<Q>(), buf2, buf1);
+    }
+    __builtin_amdgcn_s_waitcnt(0x0f70);                  /* nothing arrives in the buffers any more */
+}
+
+/* Whole lines for eight waves, 16-byte loads; and where it is the fastest: against a wave per weight row from 8 rows on, from 4
+ * on matrices of 8 M weights and at 2 on those of 128 M (us at 3 / 4 rows, wave per row and this: 4096 x 3072 7 / 9 and 8.8 / 9.0,
+ * 9216 x 3072 17 / 21 and 18.3 / 18.5; 1024 x 3072 at 5 / 7 rows 7 / 8 and 8 / 8.5), against planes and tiles while a
+ * workgroup's rows of x stay below half a megabyte (3072 x 9216 at 12 / 16 rows: 28 / 28 and 26.9 / 30.2). */
+static int linear_rows_ok(const float *d_x, const uint16_t *d_W, int seq_len, int in_dim, int out_dim) {
+    if (in_dim % 512 != 0 || (((uintptr_t)d_W | (uintptr_t)d_x) & 15)) return 0;
+    const size_t weights = (size_t)out_dim * in_dim;
+    return seq_len >= 8 || (seq_len >= 4 && weights >= (size_t)1 << 23) || (seq_len >= 2 && weights >= (size_t)1 << 27);
+}
+static int linear_rows_before_planes(const float *d_x, const uint16_t *d_W, int seq_len, int in_dim, int out_dim) {
+    return seq_len <= LR_ROWS && (size_t)seq_len * in_dim <= 12 * 9216 && linear_rows_ok(d_x, d_W, seq_len, in_dim, out_dim);
+}
+
+static void linear_rows(float *d_y, const float *d_x, const uint16_t *d_W, const float *d_bias, int seq_len, int in_dim, int out_dim) {
+    const int n_cu = g_vt.n_cu > 0 ? g_vt.n_cu : 256, k = in_dim / 512;
+    const int groups = (seq_len + LR_ROWS - 1) / LR_ROWS, wgs = groups < n_cu ? n_cu / groups : 1;
+    const int rows_per_wg = (out_dim + wgs - 1) / wgs;
+    const dim3 grid((out_dim + rows_per_wg - 1) / rows_per_wg, groups);
+#define CALL(H, P) hipLaunchKernelGGL((vt_linear_rows_kernel<H, P>), grid, dim3(512), 0, g_vt.stream, d_y, d_x, d_W, d_bias, seq_len, in_dim, out_dim, rows_per_wg)
+    if (k % 6 == 0) CALL(3, 2);
+    else if (k % 4 == 0) CALL(2, 2);
+    else if (k % 2 == 0) CALL(1, 2);
+    else CALL(1, 1);
+#undef CALL
+}
+
+/* ---- K of up to 64: a thread per output column, four rows of x through LDS -----------------------------------
+ * (3072 x 36 at 300 rows: 71 us with a wave per output column that went through the rows, 6 with this one.) */
+#define LN_K 64
+#define LN_ROWS 4
+__global__ void __launch_bounds__(256)
+vt_linear_narrow_kernel(float *y, const float *x, const uint16_t *W, const float *bias, int seq_len, int in_dim, int out_dim) {
+    __shared__ float xs[LN_ROWS][LN_K];
+    const int s0 = (int)blockIdx.y * LN_ROWS, ns = min(LN_ROWS, seq_len - s0), o = (int)(blockIdx.x * 256 + threadIdx.x);
+    for (int i = threadIdx.x; i < LN_ROWS * in_dim; i += 256) xs[i / in_dim][i % in_dim] = i / in_dim < ns ? x[(size_t)s0 * in_dim + i] : 0.f;
+    __syncthreads();
+    if (o >= out_dim) return;
+    const uint16_t *wr = W + (size_t)o * in_dim;
+    float acc[LN_ROWS] = {};
+    for (int k = 0; k < in_dim; k++) {
+        const float w = __uint_as_float((unsigned)wr[k] << 16);
+#pragma unroll
+        for (int s = 0; s < LN_ROWS; s++) acc[s] = fmaf(w, xs[s][k], acc[s]);
+    }
+#pragma unroll
+    for (int s = 0; s < LN_ROWS; s++)
+        if (s < ns) y[(size_t)(s0 + s) * out_dim + o] = bias ? __fadd_rn(bias[o], acc[s]) : acc[s];
+}
+
 void vt_launch_linear(float *d_y, const float *d_x, const uint16_t *d_W, const float *d_bias,
                       int seq_len, int in_dim, int out_dim) {
     if (seq_len == 1 && matvec_launch(d_y, d_x, d_W, d_bias, in_dim, out_dim)) return;
-    const int vec_ok = (in_dim % 8 == 0) && (((uintptr_t)d_W | (uintptr_t)d_x) % 16 == 0);
-    const dim3 grid((out_dim + 3) / 4), block(256);
-    if (seq_len == 1)
-        hipLaunchKernelGGL(vt_linear_kernel<1>, grid, block, 0, g_vt.stream, d_y, d_x, d_W, d_bias,
-                           seq_len, in_dim, out_dim, vec_ok);
-    else if (seq_len <= 4)
-        hipLaunchKernelGGL(vt_linear_kernel<4>, grid, block, 0, g_vt.stream, d_y, d_x, d_W, d_bias,
-                           seq_len, in_dim, out_dim, vec_ok);
-    else
-        hipLaunchKernelGGL(vt_linear_kernel<8>, grid, block, 0, g_vt.stream, d_y, d_x, d_W, d_bias,
-                           seq_len, in_dim, out_dim, vec_ok);
+    const int most = 1 << 17;                        /* rows per launch: they are the grid's second dimension */
+    for (; seq_len > most; seq_len -= most, d_x += (size_t)most * in_dim, d_y += (size_t)most * out_dim)
+        vt_launch_linear(d_y, d_x, d_W, d_bias, most, in_dim, out_dim);
+    if (linear_rows_ok(d_x, d_W, seq_len, in_dim, out_dim)) { linear_rows(d_y, d_x, d_W, d_bias, seq_len, in_dim, out_dim); return; }
+    if (seq_len > 1 && in_dim <= LN_K) {
+        hipLaunchKernelGGL(vt_linear_narrow_kernel, dim3((out_dim + 255) / 256, (seq_len + LN_ROWS - 1) / LN_ROWS), dim3(256), 0, g_vt.stream, d_y, d_x, d_W, d_bias,
+                           seq_len, in_dim, out_dim);
+        return;
+    }
+    const int vec_ok = (in_dim % 8 == 0) && (((uintptr_t)d_W | (uintptr_t)d_x) % 16 == 0), rows = seq_len == 1 ? 1 : seq_len <= 4 ? 4 : 8;
+    const dim3 grid((out_dim + 3) / 4, (seq_len + rows - 1) / rows), block(256);
+#define CALL(S, G) hipLaunchKernelGGL((vt_linear_kernel<S, G>), grid, block, 0, g_vt.stream, d_y, d_x, d_W, d_bias, seq_len, in_dim, out_dim, vec_ok)
+    if (rows == 1) CALL(1, false);
+    else if (rows == 4) CALL(4, false);
+    else if (seq_len <= 8) CALL(8, false);
+    else CALL(8, true);
+#undef CALL
 }
 
 /* Rows of activations against an aligned weight matrix go to the matrix cores:
@@ -198,7 +370,7 @@ void vt_launch_linear(float *d_y, const float *d_x, const uint16_t *d_W, const f
  * planes) the launches need; linear_mfma_run queues them on that work area. */
 static int linear_mfma_plan(const float *d_y, const float *d_x, const uint16_t *d_W, int seq_len, int in_dim,
                             int out_dim, int *splits_out, size_t *bytes_out) {
-    if (seq_len < 8 || !vt_gemm_shape_ok(seq_len, out_dim, in_dim, 1) ||
+    if (seq_len < 8 || linear_rows_before_planes(d_x, d_W, seq_len, in_dim, out_dim) || !vt_gemm_shape_ok(seq_len, out_dim, in_dim, 1) ||
         (((uintptr_t)d_W | (uintptr_t)d_x | (uintptr_t)d_y) & 15))
         return 0;
     const int tiles = ((seq_len + 127) / 128) * (out_dim / 128);
