@@ -21,9 +21,14 @@ void vt_launch_gemm_ex(float *d_C, int ldc, size_t plane_stride, const uint16_t 
  * order by whoever reads the result).  mb, tn: the tile, 32 mb rows x tn columns
  * (vt_gemm_wide.hip; mb 0: vt_gemm_rows.hip).  col0 is a multiple of 128. */
 #define VT_MAX_CUTS 8
-struct vt_gemm_plan { int mb, tn, col0, cuts; };
+struct vt_gemm_plan { int mb, tn, col0, cuts, row_major; };      /* row_major: W as it is (vt_gemm_row_major_plan) */
 /* K % 64 == 0; N % 256 == 0, up to 64 rows N % 96 == 0 (swiglu: % 288); swiglu: for vt_launch_gemm_frag_swiglu */
 vt_gemm_plan vt_gemm_frag_plan(int M, int N, int K, int swiglu);
+/* The same on row-major weights W[N, K], N % 128 == 0, K % 64 == 0, in at most `most` cuts: d_y [M, N]; d_part: pl.cuts planes of
+ * [M, N - pl.col0] (pl.cuts 1: not used) */
+vt_gemm_plan vt_gemm_row_major_plan(int M, int N, int K, int most);
+void vt_launch_gemm_row_major(float *d_y, float *d_part, const uint16_t *d_Ahi, const uint16_t *d_Alo, const uint16_t *d_W, int M, int N, int K,
+                              const vt_gemm_plan &pl);
 void vt_launch_gemm_frag(float *d_C, int ldc, size_t plane_stride, const uint16_t *d_Ahi, const uint16_t *d_Alo,
                          const uint16_t *d_Wf, int M, int N, int K, const vt_gemm_plan &pl);
 /* gate|up product on paired weights with SiLU(gate) * up as its epilogue -> planes d_hhi / d_hlo [M, ldh]; the

@@ -31,6 +31,8 @@ int vt_gemm_rows_cuts(int nw, int N, int K, int most) {
  * i%8 ^ row%8 of its 128-byte line, so that eight lanes reading one piece of eight rows meet all banks).  Three arrays, so that
  * the compiler knows that reading one need not wait for the others; the number of requests per wave is fixed (what is
  * past the end brings zeros, what a wave has no part in goes to a spare kilobyte), so the waits count exactly.
+ * Row-major weights (a caller's own, FRAG false): the same, a lane's 16 bytes from its own row, a line's four requests behind one
+ * another; their last strip may have one or two blocks of columns.
  * us per launch inside a prefill of 37 rows, q|k|v / output / gate|up / down: 13.0 / 11.6 / 23.5 / 15.8, on the 64-column tiles
  * 15.2 / 11.1 / 29.9 / 17.4; whole prefills of 6 / 24 / 37 / 64 rows 1829 / 2199 / 2473 / 2763 -> 1785 / 1994 / 2340 / 2737. */
 #define GS_WAVES 9
@@ -38,9 +40,9 @@ int vt_gemm_rows_cuts(int nw, int N, int K, int most) {
 
 template <int N> struct gs_int { static constexpr int v = N; };
 
-template <int NP, int KW>
+template <int NP, int KW, bool FRAG>
 __global__ void __launch_bounds__(64 * GS_WAVES)
-vt_gemm_strip_kernel(float *C, int ldc, size_t plane_stride, const uint16_t *Ahi, const uint16_t *Alo, const uint16_t *Wf, int M, int K,
+vt_gemm_strip_kernel(float *C, int ldc, size_t plane_stride, const uint16_t *Ahi, const uint16_t *Alo, const uint16_t *Wf, int M, int N, int K,
                      int strips, int cuts) {
     constexpr int MG = (NP + 1) / 2, CB = GS_WAVES / KW, STEP = MG * 4096, BUF = GS_CHUNK * STEP;
     constexpr int SPW = GS_CHUNK / KW, D = 3;                                /* a wave's steps per chunk; steps ahead */
@@ -67,13 +69,15 @@ vt_gemm_strip_kernel(float *C, int ldc, size_t plane_stride, const uint16_t *Ahi
         }
     };
     const unsigned char *w = (const unsigned char *)Wf + (size_t)(strip * CB + cb) * 64 * K;
+    const int w_voff = (lane & 31) * K * 2 + (lane >> 5) * 64;               /* row-major weights: a lane's own row */
+    const bool here = FRAG || (strip * CB + cb) * 32 < N;                    /* of these the last strip may have less than its columns */
     u32x4 ring[D][4];
     auto request = [&](u32x4 (&r)[4], int i) {                               /* this wave's i-th step */
         const int k = i * KW + kw;
-        const bool live = k < ns;
+        const bool live = k < ns && here;
         const __amdgpu_buffer_rsrc_t d = __builtin_amdgcn_make_buffer_rsrc((void *)w, 0, live ? 64 * K : 0, 0x00020000);
 #pragma unroll
-        for (int j = 0; j < 4; j++) r[j] = gr_ld_nt(d, lane * 16 + 1024 * j, live ? (s0 + k) * 4096 : 0);
+        for (int j = 0; j < 4; j++) r[j] = FRAG ? gr_ld_nt(d, lane * 16 + 1024 * j, live ? (s0 + k) * 4096 : 0) : gm_ldb(d, w_voff + 16 * j, live ? (s0 + k) * 128 : 0);
     };
     f32x16 acc[MG];
 #pragma unroll
@@ -94,7 +98,7 @@ vt_gemm_strip_kernel(float *C, int ldc, size_t plane_stride, const uint16_t *Ahi
      * chunk c + 2, which every wave has read as those of chunk c - 1 when all have met here.  (A bare barrier:
      * __syncthreads() waits for all rows on their way, those of chunk c + 1 too.  What a wave has read from LDS it has multiplied by then,
      * and the empty statements keep requests and reads on their side of it.) */
-    auto body = [&](int c, const unsigned char *here, unsigned char *next, auto slot, auto after) {
+    auto body = [&](int c, const unsigned char *rows, unsigned char *next, auto slot, auto after) {
         __builtin_amdgcn_sched_barrier(0);
         __builtin_amdgcn_s_waitcnt(0x0f70 | (decltype(after)::v & 15) | (decltype(after)::v >> 4 << 14));
         __builtin_amdgcn_s_barrier();
@@ -106,7 +110,7 @@ vt_gemm_strip_kernel(float *C, int ldc, size_t plane_stride, const uint16_t *Ahi
 #pragma unroll
         for (int j = 0; j < SPW; j++) {
             const int at = (decltype(slot)::v + j) % D;
-            multiply(here, KW == 1 ? j : kw, ring[at]);
+            multiply(rows, KW == 1 ? j : kw, ring[at]);
             request(ring[at], c * SPW + j + D);
             asm volatile("" ::: "memory");
         }
@@ -135,7 +139,7 @@ vt_gemm_strip_kernel(float *C, int ldc, size_t plane_stride, const uint16_t *Ahi
         const int row0 = 8 * qd + 4 * (lane >> 5);
 #pragma unroll
         for (int v = 0; v < 4; v++)
-            if (row0 + v < M) out[(size_t)(row0 + v) * ldc] = x[v];
+            if (row0 + v < M && here) out[(size_t)(row0 + v) * ldc] = x[v];
     };
     auto quad = [&](int qd) {
         const f32x16 &p = acc[qd / 2];
@@ -176,22 +180,23 @@ vt_gemm_strip_kernel(float *C, int ldc, size_t plane_stride, const uint16_t *Ahi
 #define GS_WIDE 288
 #define GS_NARROW 96
 
-template <int NP, int KW>
+template <int NP, int KW, bool FRAG>
 static void gs_launch(float *d_C, int ldc, size_t plane_stride, const uint16_t *d_Ahi, const uint16_t *d_Alo, const uint16_t *d_Wf, int M, int N, int K, int cuts) {
-    const int strips = N / (32 * GS_WAVES / KW);
-    hipLaunchKernelGGL((vt_gemm_strip_kernel<NP, KW>), dim3(strips * cuts), dim3(64 * GS_WAVES), 0, g_vt.stream, d_C, ldc, plane_stride, d_Ahi, d_Alo, d_Wf, M, K,
+    const int tn = 32 * GS_WAVES / KW, strips = (N + tn - 1) / tn;
+    hipLaunchKernelGGL((vt_gemm_strip_kernel<NP, KW, FRAG>), dim3(strips * cuts), dim3(64 * GS_WAVES), 0, g_vt.stream, d_C, ldc, plane_stride, d_Ahi, d_Alo, d_Wf, M, N, K,
                        strips, cuts);
 }
 
 vt_gemm_plan vt_gemm_few_rows_plan(int N, int swiglu) {
-    const int tn = swiglu ? GS_WIDE : GS_NARROW, cuts = g_vt.n_cu / (N / tn);
+    const int tn = swiglu ? GS_WIDE : GS_NARROW, cuts = g_vt.n_cu / ((N + tn - 1) / tn);
     return vt_gemm_plan{0, tn, 0, cuts < 1 ? 1 : cuts < VT_MAX_CUTS ? cuts : VT_MAX_CUTS};
 }
 
 void vt_launch_gemm_few_rows(float *d_C, int ldc, size_t plane_stride, const uint16_t *d_Ahi, const uint16_t *d_Alo,
                              const uint16_t *d_Wf, int M, int N, int K, const vt_gemm_plan &pl) {
     typedef void (*fn)(float *, int, size_t, const uint16_t *, const uint16_t *, const uint16_t *, int, int, int, int);
-    static const fn launch[2][8] = {{gs_launch<1, 1>, gs_launch<2, 1>, gs_launch<3, 1>, gs_launch<4, 1>, gs_launch<5, 1>, gs_launch<6, 1>, gs_launch<7, 1>, gs_launch<8, 1>},
-                                    {gs_launch<1, 3>, gs_launch<2, 3>, gs_launch<3, 3>, gs_launch<4, 3>, gs_launch<5, 3>, gs_launch<6, 3>, gs_launch<7, 3>, gs_launch<8, 3>}};
-    launch[pl.tn == GS_NARROW][(M + 7) / 8 - 1](d_C, ldc, plane_stride, d_Ahi, d_Alo, d_Wf, M, N, K, pl.cuts);
+#define GS_BY_ROWS(KW, FRAG) {gs_launch<1, KW, FRAG>, gs_launch<2, KW, FRAG>, gs_launch<3, KW, FRAG>, gs_launch<4, KW, FRAG>, gs_launch<5, KW, FRAG>, gs_launch<6, KW, FRAG>, \
+                              gs_launch<7, KW, FRAG>, gs_launch<8, KW, FRAG>}
+    static const fn launch[3][8] = {GS_BY_ROWS(1, true), GS_BY_ROWS(3, true), GS_BY_ROWS(3, false)};
+    launch[pl.tn == GS_WIDE ? 0 : pl.row_major ? 2 : 1][(M + 7) / 8 - 1](d_C, ldc, plane_stride, d_Ahi, d_Alo, d_Wf, M, N, K, pl.cuts);
 }

@@ -171,7 +171,8 @@ __device__ __forceinline__ gw_item gw_item_at(const gw_list &list, int part, int
     return it;
 }
 
-template <class T, int MB, int CW, int NB>
+/* FRAG false: row-major weights (WP 1), a caller's own: the same operands, a lane's 16 bytes of each slice from its own row */
+template <class T, int MB, int CW, int NB, bool FRAG = true>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
 vt_gemm_wide_kernel(gw_list list, const uint16_t *Ahi, const uint16_t *Alo, int M, int K) {
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
@@ -190,6 +191,8 @@ vt_gemm_wide_kernel(gw_list list, const uint16_t *Ahi, const uint16_t *Alo, int 
     const int st_off = kw * GROUP + lr * GM_STAGE_ROW + lc * 16;
     const int fa_off = kw * GROUP + (lane & 31) * GM_STAGE_ROW + (lane >> 5) * 64;
 
+    const int w_voff = FRAG ? lane * 16 : (lane & 31) * K * 2 + (lane >> 5) * 64;
+
     struct aregs { u32x4 hi[NP], lo[NP]; };                /* staged rows of one K step, both planes */
     /* rows past M and steps past the cut's end: beyond the descriptor's size, nothing is loaded (zeros) */
     auto fetch_a = [&](const gw_item &it, const uint16_t *plane, u32x4 (&r)[NP], int i) {
@@ -204,11 +207,11 @@ vt_gemm_wide_kernel(gw_list list, const uint16_t *Ahi, const uint16_t *Alo, int 
         const int s = KW * i + kw;
         const bool live = s < it.ns;
         const __amdgpu_buffer_rsrc_t d = __builtin_amdgcn_make_buffer_rsrc((void *)(it.w + (size_t)cw * NB * blk_bytes), 0, live ? NB * blk_bytes : 0, 0x00020000);
-        const int soff = live ? (it.s0 + s) * 4096 * WP : 0;
+        const int soff = live ? (it.s0 + s) * (FRAG ? 4096 * WP : 128) : 0;
 #pragma unroll
         for (int p = 0; p < WP; p++)
 #pragma unroll
-            for (int b = 0; b < NB; b++) r.v[p][b][j] = gm_ldb(d, lane * 16 + 1024 * j, soff + 4096 * p + (live ? b * blk_bytes : 0));
+            for (int b = 0; b < NB; b++) r.v[p][b][j] = gm_ldb(d, w_voff + (FRAG ? 1024 : 16) * j, soff + 4096 * p + (live ? b * blk_bytes : 0));
     };
     auto store_a = [&](const u32x4 (&r)[NP], int at) {
 #pragma unroll

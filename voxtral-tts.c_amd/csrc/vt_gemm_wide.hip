@@ -44,7 +44,7 @@ static float gw_cost(const gw_format &f, int M, int N, int K, int mb, int tn, in
     return t;
 }
 
-static vt_gemm_plan gw_plan(const gw_format &f, int M, int N, int K, int swiglu) {
+static vt_gemm_plan gw_plan(const gw_format &f, int M, int N, int K, int swiglu, int most = VT_MAX_CUTS) {
     vt_gemm_plan best = {0, 64, 0, 1};
     float best_cost = 0.f;
     for (int mb = 3; mb <= 4; mb++)
@@ -58,7 +58,7 @@ static vt_gemm_plan gw_plan(const gw_format &f, int M, int N, int K, int swiglu)
                 int n_main = pick == 2 ? nt : (full - pick) * g_vt.n_cu / mt;
                 if (n_main < 0 || n_main > nt) continue;
                 if (n_main * tn % 128) n_main--;          /* heads of 128 columns are cut or not */
-                for (int cuts = 1; cuts <= VT_MAX_CUTS && cuts <= K / 64; cuts++) {
+                for (int cuts = 1; cuts <= most && cuts <= K / 64; cuts++) {
                     if (n_main == nt && cuts > 1) break;
                     if (swiglu && n_main < nt && cuts == 1) continue;
                     const float c = gw_cost(f, M, N, K, mb, tn, n_main, cuts, swiglu);
@@ -81,17 +81,17 @@ vt_gemm_plan vt_codec_gemm_plan(int M, int N, int K) {
     return gw_plan(gw_codec, M, N, K, 0);
 }
 
-template <int MB, int CW, int NB>
+template <int MB, int CW, int NB, bool FRAG = true>
 static void gw_launch(const gw_list &list, const uint16_t *d_Ahi, const uint16_t *d_Alo, int M, int K) {
     constexpr int LDS = 2 * (4 / CW) * 2 * 32 * MB * GM_STAGE_ROW;
     static int attr_set = 0;
     if (!attr_set) {
-        if (vt_check(hipFuncSetAttribute((const void *)vt_gemm_wide_kernel<gm_bf16, MB, CW, NB>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS), "product LDS size"))
+        if (vt_check(hipFuncSetAttribute((const void *)vt_gemm_wide_kernel<gm_bf16, MB, CW, NB, FRAG>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS), "product LDS size"))
             return;
         attr_set = 1;
     }
     const int items = list.m_tiles * list.part[0].n_tiles * list.part[0].splits;      /* every workgroup takes an item of the first part */
-    hipLaunchKernelGGL((vt_gemm_wide_kernel<gm_bf16, MB, CW, NB>), dim3(items < g_vt.n_cu ? items : g_vt.n_cu), dim3(256), LDS, g_vt.stream, list, d_Ahi, d_Alo, M, K);
+    hipLaunchKernelGGL((vt_gemm_wide_kernel<gm_bf16, MB, CW, NB, FRAG>), dim3(items < g_vt.n_cu ? items : g_vt.n_cu), dim3(256), LDS, g_vt.stream, list, d_Ahi, d_Alo, M, K);
 }
 
 static void gw_run(const vt_gemm_plan &pl, gw_part whole, gw_part cut, const uint16_t *d_Ahi, const uint16_t *d_Alo, int M, int N, int K) {
@@ -103,9 +103,57 @@ static void gw_run(const vt_gemm_plan &pl, gw_part whole, gw_part cut, const uin
     cut.splits = pl.cuts;
     if (whole.n_tiles) list.part[list.n_parts++] = whole;
     if (cut.n_tiles) list.part[list.n_parts++] = cut;
-    static void (*const launch[2][3])(const gw_list &, const uint16_t *, const uint16_t *, int, int) = {
-        {gw_launch<3, 2, 2>, gw_launch<3, 2, 3>, gw_launch<3, 4, 2>}, {NULL, gw_launch<4, 2, 3>, gw_launch<4, 4, 2>}};
-    launch[pl.mb - 3][pl.tn / 64 - 2](list, d_Ahi, d_Alo, M, K);
+    static void (*const launch[2][2][3])(const gw_list &, const uint16_t *, const uint16_t *, int, int) = {
+        {{gw_launch<3, 2, 2>, gw_launch<3, 2, 3>, gw_launch<3, 4, 2>}, {NULL, gw_launch<4, 2, 3>, gw_launch<4, 4, 2>}},
+        {{gw_launch<3, 2, 2, false>, gw_launch<3, 2, 3, false>, gw_launch<3, 4, 2, false>}, {NULL, gw_launch<4, 2, 3, false>, gw_launch<4, 4, 2, false>}}};
+    launch[pl.row_major][pl.mb - 3][pl.tn / 64 - 2](list, d_Ahi, d_Alo, M, K);
+}
+
+/* The cost constants are those of fragment order: a lane's own row costs four times the lines per request, and with the steps
+ * 15 % or a cut column's planes twice as dear the plans were no better at 65 to 300 rows.  A step's four requests of a line
+ * stand one in each of its regions, as with fragments: all in the last one, 42 us instead of 39 for 9216 x 3072 at 150 rows.
+ * Strips up to 64 rows, beyond 32 only while they are one per CU (32768 x 3072 at 64 rows: 63 us, tiles 52) */
+vt_gemm_plan vt_gemm_row_major_plan(int M, int N, int K, int most) {
+    vt_gemm_plan pl;
+    if (vt_gemm_rows_ok(M, N, K) && (M <= 32 || N <= 96 * g_vt.n_cu)) {
+        pl = vt_gemm_few_rows_plan(N, 0);
+        if (pl.cuts > most) pl.cuts = most;
+        if (pl.cuts > K / 64) pl.cuts = K / 64;
+    } else {
+        pl = gw_plan(gw_backbone, M, N, K, 0, most);
+        if (pl.cuts == 1) pl.col0 = N;
+    }
+    pl.row_major = 1;
+    return pl;
+}
+
+/* y[:, col0 ..] = the planes' sum, in order, all of them requested in front of the first addition: a chain of memory latencies */
+__global__ void __launch_bounds__(256) vt_sum_cut_columns_kernel(float *y, const float *part, int cuts, int M, int N, int col0) {
+    const int w = (N - col0) / 4;
+    const size_t n = (size_t)M * w;
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
+        f32x4 q[VT_MAX_CUTS];
+#pragma unroll
+        for (int p = 0; p < VT_MAX_CUTS; p++) q[p] = reinterpret_cast<const f32x4 *>(part)[(p < cuts ? p : 0) * n + i];
+        f32x4 v = q[0];
+#pragma unroll
+        for (int p = 1; p < VT_MAX_CUTS; p++)
+            if (p < cuts) { v.x = __fadd_rn(v.x, q[p].x); v.y = __fadd_rn(v.y, q[p].y); v.z = __fadd_rn(v.z, q[p].z); v.w = __fadd_rn(v.w, q[p].w); }
+        *reinterpret_cast<f32x4 *>(y + i / w * N + col0 + i % w * 4) = v;
+    }
+}
+
+void vt_launch_gemm_row_major(float *d_y, float *d_part, const uint16_t *d_Ahi, const uint16_t *d_Alo, const uint16_t *d_W, int M, int N, int K,
+                              const vt_gemm_plan &pl) {
+    const int cut = N - pl.col0;
+    const size_t plane = (size_t)M * cut;
+    if (pl.mb == 0) vt_launch_gemm_few_rows(pl.cuts > 1 ? d_part : d_y, N, plane, d_Ahi, d_Alo, d_W, M, N, K, pl);
+    else gw_run(pl, gw_part{d_y, d_W, 0, N, 0, 0, NULL, NULL, 0, NULL, NULL},
+                gw_part{d_part, d_W + (size_t)pl.col0 * K, plane, cut, 0, 0, NULL, NULL, 0, NULL, NULL}, d_Ahi, d_Alo, M, N, K);
+    if (pl.cuts > 1) {
+        const size_t n = plane / 4;
+        hipLaunchKernelGGL(vt_sum_cut_columns_kernel, dim3((unsigned)((n + 255) / 256 > 4096 ? 4096 : (n + 255) / 256)), dim3(256), 0, g_vt.stream, d_y, d_part, pl.cuts, M, N, pl.col0);
+    }
 }
 
 void vt_launch_gemm_frag(float *d_C, int ldc, size_t plane_stride, const uint16_t *d_Ahi, const uint16_t *d_Alo,

@@ -294,15 +294,16 @@ vt_linear_rows_kernel(float *y, const float *x, const uint16_t *W, const float *
 
 /* Whole lines for eight waves, 16-byte loads; and where it is the fastest: against a wave per weight row from 8 rows on, from 4
  * on matrices of 8 M weights and at 2 on those of 128 M (us at 3 / 4 rows, wave per row and this: 4096 x 3072 7 / 9 and 8.8 / 9.0,
- * 9216 x 3072 17 / 21 and 18.3 / 18.5; 1024 x 3072 at 5 / 7 rows 7 / 8 and 8 / 8.5), against planes and tiles while a
- * workgroup's rows of x stay below half a megabyte (3072 x 9216 at 12 / 16 rows: 28 / 28 and 26.9 / 30.2). */
+ * 9216 x 3072 17 / 21 and 18.3 / 18.5; 1024 x 3072 at 5 / 7 rows 7 / 8 and 8 / 8.5), against planes
+ * and strips while a workgroup's rows of x stay below 200 KB (16 rows of 9216 x 3072 and 131072 x 3072 21 / 149, strips at 17 rows 18 / 185,
+ * of 4096 x 3072 11.5 / 13; 3072 x 4096 at 12 / 16 rows 13 / 15.3, strips 12.6 at 17; 3072 x 9216 at 12 rows 27, strips 16). */
 static int linear_rows_ok(const float *d_x, const uint16_t *d_W, int seq_len, int in_dim, int out_dim) {
     if (in_dim % 512 != 0 || (((uintptr_t)d_W | (uintptr_t)d_x) & 15)) return 0;
     const size_t weights = (size_t)out_dim * in_dim;
     return seq_len >= 8 || (seq_len >= 4 && weights >= (size_t)1 << 23) || (seq_len >= 2 && weights >= (size_t)1 << 27);
 }
 static int linear_rows_before_planes(const float *d_x, const uint16_t *d_W, int seq_len, int in_dim, int out_dim) {
-    return seq_len <= LR_ROWS && (size_t)seq_len * in_dim <= 12 * 9216 && linear_rows_ok(d_x, d_W, seq_len, in_dim, out_dim);
+    return seq_len <= LR_ROWS && (size_t)seq_len * in_dim <= 12 * 4096 && linear_rows_ok(d_x, d_W, seq_len, in_dim, out_dim);
 }
 
 static void linear_rows(float *d_y, const float *d_x, const uint16_t *d_W, const float *d_bias, int seq_len, int in_dim, int out_dim) {
@@ -363,47 +364,78 @@ void vt_launch_linear(float *d_y, const float *d_x, const uint16_t *d_W, const f
 #undef CALL
 }
 
-/* Rows of activations against an aligned weight matrix go to the matrix cores:
- * (hi, lo) planes of x, K cut into enough ranges to fill the device, partial
- * planes summed in a fixed order.  linear_mfma_plan says whether the shape qualifies, into how
- * many ranges K is cut and how many bytes of work area (partial planes, then the two activation
- * planes) the launches need; linear_mfma_run queues them on that work area. */
+/* Rows of activations against an aligned weight matrix go to the matrix cores: (hi, lo) planes of x, products, partial
+ * planes summed in a fixed order.  linear_mfma_plan says whether the shape qualifies, how the product is divided and how many
+ * bytes of work area (partial planes, then the two activation planes) the launches need; linear_mfma_run queues them on that
+ * work area.  The products are the backbone's strips and tiles on the caller's weights as they lie (equal_cuts 0), or tiles
+ * of 128 x 128 whose K is cut into equal ranges.
+ * The fixed work area of the entry point without allocation holds what equal ranges that make 192 such tiles take, and a shape
+ * beyond that is refused there: where it holds that, the plan is one that fits too. */
+#define VT_STATIC_SCRATCH_BYTES ((size_t)16 << 20)
+struct linear_plan { vt_gemm_plan tiles; int equal_cuts; size_t bytes; };
+
+static size_t linear_part_bytes(const linear_plan &p, int seq_len, int out_dim) {
+    const int cuts = p.equal_cuts ? p.equal_cuts : p.tiles.cuts, col0 = p.equal_cuts ? 0 : p.tiles.col0;
+    return cuts > 1 ? sizeof(float) * seq_len * (size_t)(out_dim - col0) * cuts : 0;
+}
+
+/* 128 x 128 tiles, two workgroups per CU, stage the weights through LDS in whole lines; the others read a lane's own row and have
+ * one workgroup per CU.  us, these and the others, 9216 x 3072 at 17 / 64 / 96 / 150 / 300 / 700 rows: 26 / 28 / 30 / 53 / 65 / 103
+ * and 18 / 25 / 29 / 39 / 59 / 87; 3072 x 9216 27 / 31 / 33 / 55 / 72 / 141 and 17 / 23 / 29 / 37 / 57 / 105; 1024 x 3072 15 / 17 / 18 /
+ * 21 / 22 / 31 and 11 / 14 / 16 / 18 / 22 / 29.  The 128 x 128 tiles stay the faster ones
+ *   for 97 to 128 rows, one of their tiles and two of 96 rows (9216 x 3072 at 110: 32 and 37);
+ *   with two full rounds of them, unless the others have a quarter fewer rows to pad (131072 x 3072 at 37 / 65 / 150 / 300 rows: 203 /
+ *   215 / 412 / 641 and 215 / 228 / 378 / 677);
+ *   for columns that are no multiple of 192 or 256, beyond 512 rows (8320 x 3072 at 700 / 1500: 100 / 187 and 106 / 199);
+ *   beyond 256 rows of few columns (1024 x 3072 at 300 rows, 24 tiles: 21.4 and 22.3; at 700, 48 tiles: 31 and 29). */
+static int linear_equal_cuts(int M, int N, int tiles) {
+    const int pad96 = (M + 95) / 96 * 96, pad128 = (M + 127) / 128 * 128;
+    return (M > 96 && M <= 128) || (tiles >= 4 * g_vt.n_cu && (M <= 128 || 4 * pad96 > 3 * pad128)) || (M > 512 && N % 192 != 0 && N % 256 != 0) ||
+           (M > 256 && tiles <= 24);
+}
+
 static int linear_mfma_plan(const float *d_y, const float *d_x, const uint16_t *d_W, int seq_len, int in_dim,
-                            int out_dim, int *splits_out, size_t *bytes_out) {
+                            int out_dim, linear_plan *p) {
     if (seq_len < 8 || linear_rows_before_planes(d_x, d_W, seq_len, in_dim, out_dim) || !vt_gemm_shape_ok(seq_len, out_dim, in_dim, 1) ||
         (((uintptr_t)d_W | (uintptr_t)d_x | (uintptr_t)d_y) & 15))
         return 0;
     const int tiles = ((seq_len + 127) / 128) * (out_dim / 128);
-    int splits = 1;
+    p->equal_cuts = 1;
     static const int cand[] = {2, 3, 4, 6, 8};
-    for (int i = 0; i < 5 && tiles * splits < 192; i++)
-        if (vt_gemm_shape_ok(seq_len, out_dim, in_dim, cand[i])) splits = cand[i];
-    const size_t n_in = (size_t)seq_len * in_dim, n_out = (size_t)seq_len * out_dim;
-    const size_t part_bytes = splits > 1 ? sizeof(float) * n_out * splits : 0;
-    *splits_out = splits;
-    *bytes_out = part_bytes + 2 * sizeof(uint16_t) * n_in;
+    for (int i = 0; i < 5 && tiles * p->equal_cuts < 192; i++)
+        if (vt_gemm_shape_ok(seq_len, out_dim, in_dim, cand[i])) p->equal_cuts = cand[i];
+    const size_t planes = 2 * sizeof(uint16_t) * (size_t)seq_len * in_dim, equal = linear_part_bytes(*p, seq_len, out_dim) + planes;
+    p->bytes = equal;
+    if (linear_equal_cuts(seq_len, out_dim, tiles)) return 1;
+    p->equal_cuts = 0;
+    for (int most = VT_MAX_CUTS;; most = p->tiles.cuts - 1) {
+        p->tiles = vt_gemm_row_major_plan(seq_len, out_dim, in_dim, most);
+        const size_t bytes = linear_part_bytes(*p, seq_len, out_dim) + planes;
+        if (bytes > p->bytes) p->bytes = bytes;
+        if (p->tiles.cuts == 1 || equal > VT_STATIC_SCRATCH_BYTES || bytes <= VT_STATIC_SCRATCH_BYTES) break;
+        p->bytes = equal;
+    }
     return 1;
 }
 
 static void linear_mfma_run(unsigned char *base, float *d_y, const float *d_x, const uint16_t *d_W, int seq_len,
-                            int in_dim, int out_dim, int splits) {
+                            int in_dim, int out_dim, const linear_plan &p) {
     const size_t n_in = (size_t)seq_len * in_dim, n_out = (size_t)seq_len * out_dim;
-    const size_t part_bytes = splits > 1 ? sizeof(float) * n_out * splits : 0;
-    float *part = splits > 1 ? (float *)base : d_y;
-    uint16_t *hi = (uint16_t *)(base + part_bytes), *lo = hi + n_in;
+    float *part = (float *)base;
+    uint16_t *hi = (uint16_t *)(base + linear_part_bytes(p, seq_len, out_dim)), *lo = hi + n_in;
     vt_launch_split(hi, lo, d_x, n_in);
-    vt_launch_gemm(part, hi, lo, d_W, seq_len, out_dim, in_dim, splits);
-    if (splits > 1) vt_launch_sum_planes(d_y, part, splits, n_out, n_out);
+    if (!p.equal_cuts) vt_launch_gemm_row_major(d_y, part, hi, lo, d_W, seq_len, out_dim, in_dim, p.tiles);
+    else vt_launch_gemm(p.equal_cuts > 1 ? part : d_y, hi, lo, d_W, seq_len, out_dim, in_dim, p.equal_cuts);
+    if (p.equal_cuts > 1) vt_launch_sum_planes(d_y, part, p.equal_cuts, n_out, n_out);
 }
 
 /* Returns 0 when the shape does not qualify, 1 when queued, -1 on error. */
 static int linear_mfma(float *d_y, const float *d_x, const uint16_t *d_W, int seq_len, int in_dim, int out_dim) {
-    int splits;
-    size_t bytes;
-    if (!linear_mfma_plan(d_y, d_x, d_W, seq_len, in_dim, out_dim, &splits, &bytes)) return 0;
-    unsigned char *base = (unsigned char *)vt_scratch(bytes);
+    linear_plan plan;
+    if (!linear_mfma_plan(d_y, d_x, d_W, seq_len, in_dim, out_dim, &plan)) return 0;
+    unsigned char *base = (unsigned char *)vt_scratch(plan.bytes);
     if (!base) return -1;
-    linear_mfma_run(base, d_y, d_x, d_W, seq_len, in_dim, out_dim, splits);
+    linear_mfma_run(base, d_y, d_x, d_W, seq_len, in_dim, out_dim, plan);
     return 1;
 }
 
@@ -416,7 +448,6 @@ static int linear_mfma(float *d_y, const float *d_x, const uint16_t *d_W, int se
  * last call's contents; nothing in it has to start at zero (the activation planes and every
  * element of every partial plane that is read are written by the call itself).  Calls that overlap
  * on one device would share the array: the library has one stream and is not thread-safe. */
-#define VT_STATIC_SCRATCH_BYTES ((size_t)16 << 20)
 #define VT_STATIC_MAX_DEVICES 16
 static __device__ __align__(256) unsigned char vt_static_scratch[VT_STATIC_SCRATCH_BYTES];
 static unsigned char *s_static_ptr[VT_STATIC_MAX_DEVICES];
@@ -450,21 +481,20 @@ extern "C" int tts_hip_linear_bf16_noalloc(float *d_y, const float *d_x, int seq
         vt_set_error("tts_hip_linear_bf16_noalloc: bad arguments");
         return -1;
     }
-    int splits;
-    size_t bytes;
-    if (!linear_mfma_plan(d_y, d_x, (const uint16_t *)d_W, seq_len, in_dim, out_dim, &splits, &bytes)) {
+    linear_plan plan;
+    if (!linear_mfma_plan(d_y, d_x, (const uint16_t *)d_W, seq_len, in_dim, out_dim, &plan)) {
         /* few rows or an unaligned shape: the row kernels, which use no work area at all */
         vt_launch_linear(d_y, d_x, (const uint16_t *)d_W, NULL, seq_len, in_dim, out_dim);
         return vt_check(hipGetLastError(), "tts_hip_linear_bf16_noalloc") ? -1 : 0;
     }
-    if (bytes > VT_STATIC_SCRATCH_BYTES) {
+    if (plan.bytes > VT_STATIC_SCRATCH_BYTES) {
         vt_set_error("tts_hip_linear_bf16_noalloc: %d x %d x %d needs %zu bytes of work area, the fixed one has %zu; "
-                     "use tts_hip_linear_bf16", seq_len, out_dim, in_dim, bytes, (size_t)VT_STATIC_SCRATCH_BYTES);
+                     "use tts_hip_linear_bf16", seq_len, out_dim, in_dim, plan.bytes, (size_t)VT_STATIC_SCRATCH_BYTES);
         return -1;
     }
     unsigned char *base = static_scratch();
     if (!base) return -1;
-    linear_mfma_run(base, d_y, d_x, (const uint16_t *)d_W, seq_len, in_dim, out_dim, splits);
+    linear_mfma_run(base, d_y, d_x, (const uint16_t *)d_W, seq_len, in_dim, out_dim, plan);
     return vt_check(hipGetLastError(), "tts_hip_linear_bf16_noalloc") ? -1 : 0;
 }
 
