@@ -133,6 +133,7 @@ static int init_context(int kv_cache_max) {
     }
     g_vt.bar_epoch = 0;
     VT_TRY(hipHostMalloc((void **)&g_vt.h_pin, sizeof(float) * VT_PIN_FLOATS, hipHostMallocDefault));
+    if (vt_gemm_row_major_prepare()) return -1;
     VT_TRY(hipDeviceSynchronize());
 
     g_hip.n_cu = g_vt.n_cu;

@@ -81,15 +81,28 @@ vt_gemm_plan vt_codec_gemm_plan(int M, int N, int K) {
     return gw_plan(gw_codec, M, N, K, 0);
 }
 
+template <int MB, int CW>
+struct gw_lds { static constexpr int bytes = 2 * (4 / CW) * 2 * 32 * MB * GM_STAGE_ROW; };
+
+template <int MB, int CW, int NB, bool FRAG = true>
+static int gw_prepare(void) {
+    static int attr_device = -1;
+    if (attr_device == g_vt.device) return 0;
+    if (vt_check(hipFuncSetAttribute((const void *)vt_gemm_wide_kernel<gm_bf16, MB, CW, NB, FRAG>, hipFuncAttributeMaxDynamicSharedMemorySize, gw_lds<MB, CW>::bytes), "product LDS size"))
+        return -1;
+    attr_device = g_vt.device;
+    return 0;
+}
+
+/* With the context: a product on a caller's weights may be the first call inside a stream capture */
+int vt_gemm_row_major_prepare(void) {
+    return gw_prepare<3, 2, 2, false>() || gw_prepare<3, 2, 3, false>() || gw_prepare<3, 4, 2, false>() || gw_prepare<4, 2, 3, false>() || gw_prepare<4, 4, 2, false>() ? -1 : 0;
+}
+
 template <int MB, int CW, int NB, bool FRAG = true>
 static void gw_launch(const gw_list &list, const uint16_t *d_Ahi, const uint16_t *d_Alo, int M, int K) {
-    constexpr int LDS = 2 * (4 / CW) * 2 * 32 * MB * GM_STAGE_ROW;
-    static int attr_set = 0;
-    if (!attr_set) {
-        if (vt_check(hipFuncSetAttribute((const void *)vt_gemm_wide_kernel<gm_bf16, MB, CW, NB, FRAG>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS), "product LDS size"))
-            return;
-        attr_set = 1;
-    }
+    constexpr int LDS = gw_lds<MB, CW>::bytes;
+    if (gw_prepare<MB, CW, NB, FRAG>()) return;
     const int items = list.m_tiles * list.part[0].n_tiles * list.part[0].splits;      /* every workgroup takes an item of the first part */
     hipLaunchKernelGGL((vt_gemm_wide_kernel<gm_bf16, MB, CW, NB, FRAG>), dim3(items < g_vt.n_cu ? items : g_vt.n_cu), dim3(256), LDS, g_vt.stream, list, d_Ahi, d_Alo, M, K);
 }
