@@ -153,7 +153,7 @@ void tts_hip_causal_attention_decode(float *d_out, const float *d_Q, const float
                                      int kv_cache_stride);
 /* replaces tts_cuda_causal_attention_prefill (voxtral_tts_cuda.h:142-145).  With the model's head
  * counts and 8 or more queries it runs on the matrix cores, from tile images of K and V that a first
- * kernel writes into a buffer of the library's own (8 x ceil((start_pos + seq_len) / 32) x 37 KB,
+ * kernel writes into a buffer of the library's own (8 x ceil((start_pos + seq_len) / 32) x 32 KB,
  * allocated when a call needs more than any before it). */
 void tts_hip_causal_attention_prefill(float *d_out, const float *d_Q, const float *d_K,
                                       const float *d_V, int seq_len, int start_pos,
