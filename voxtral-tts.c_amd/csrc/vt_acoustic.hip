@@ -1007,8 +1007,9 @@ __global__ void vt_ac_fetch_kernel(float *out, const float *in, int n) {
     if (i < n) out[i] = in[i];
 }
 
-/* Enqueues one frame: semantic head + argmax, 7 guided Euler steps, FSQ.  The hidden state is the caller's (h_hidden, host)
- * or the backbone step's (d_hidden).  Codes end up in w->codes, the latent in w->x and both in the pinned ac_frame_out;
+/* Enqueues one frame: semantic head + argmax, 7 guided Euler steps, FSQ.  The hidden state is the caller's (h_hidden)
+ * or the backbone step's (d_hidden).  What the caller holds in pageable memory is read here and now; device and pinned memory
+ * (whose contents may still be on their way on the stream) goes through a copy on the stream.  Codes end up in w->codes, the latent in w->x and both in the pinned ac_frame_out;
  * nothing is synchronised.  The frame's only traffic with the host is what its kernels read and write there: five
  * copies of 144 bytes to 12 KB, the argmax in a launch of its own and the hidden state copied on the device were 9 us of a frame. */
 static int enqueue_frame(ac_work *w, const float *h_hidden, const float *d_hidden, const float *x0) {
@@ -1020,11 +1021,16 @@ static int enqueue_frame(ac_work *w, const float *h_hidden, const float *d_hidde
     float ts[AC_STEPS + 1];
     for (int i = 0; i <= AC_STEPS; i++) ts[i] = (float)i / (float)AC_STEPS;
     if (ensure_time_grid(w->temb)) return -1;            /* the projected time tokens depend on the weights only */
-    memcpy(g_vt.h_pin + VT_PIN_X0, x0, sizeof(float) * VT_AC_DIM_IN);
-    w->x0 = g_vt.h_pin + VT_PIN_X0;
+    w->x0 = NULL;
+    if (vt_pageable(x0)) {
+        memcpy(g_vt.h_pin + VT_PIN_X0, x0, sizeof(float) * VT_AC_DIM_IN);
+        w->x0 = g_vt.h_pin + VT_PIN_X0;
+    } else if (vt_check(hipMemcpyAsync(w->x, x0, sizeof(float) * VT_AC_DIM_IN, hipMemcpyDefault, st), "frame noise")) return -1;
     if (h_hidden) {
-        memcpy(g_vt.h_pin + VT_PIN_HIDDEN, h_hidden, sizeof(float) * VT_DIM);
-        hipLaunchKernelGGL(vt_ac_fetch_kernel, dim3(VT_DIM / 256), dim3(256), 0, st, w->hidden, g_vt.h_pin + VT_PIN_HIDDEN, VT_DIM);
+        if (vt_pageable(h_hidden)) {
+            memcpy(g_vt.h_pin + VT_PIN_HIDDEN, h_hidden, sizeof(float) * VT_DIM);
+            hipLaunchKernelGGL(vt_ac_fetch_kernel, dim3(VT_DIM / 256), dim3(256), 0, st, w->hidden, g_vt.h_pin + VT_PIN_HIDDEN, VT_DIM);
+        } else if (vt_check(hipMemcpyAsync(w->hidden, h_hidden, sizeof(float) * VT_DIM, hipMemcpyDefault, st), "frame hidden")) return -1;
         d_hidden = w->hidden;
     }
     vt_launch_linear(w->logits, d_hidden, ac->semantic_out, ac->semantic_bias, 1, VT_DIM, VT_SEM_PADDED);

@@ -778,7 +778,8 @@ extern "C" void tts_hip_codec_decode(const int *codes, int n_frames, float **out
      * now, of which 8 / 21 / 95 / 273 behind the device's work. */
     float *wave = (float *)g_cd.host;
     int *host_codes = (int *)(wave + n);
-    memcpy(host_codes, codes, code_bytes);
+    if (vt_pageable(codes)) memcpy(host_codes, codes, code_bytes);
+    else if (vt_check(hipMemcpyAsync(host_codes, codes, code_bytes, hipMemcpyDefault, g_vt.stream), "codes copy")) { free(s); return; }
     const cd_product p = cd_enqueue(host_codes, n_frames);
     int parts = (int)((size_t)n * sizeof(float) / CD_WAVE_PART_BYTES), bad = 0;
     parts = parts < 1 ? 1 : parts < CD_WAVE_PARTS ? parts : CD_WAVE_PARTS;

@@ -78,6 +78,13 @@ static int build_rope_table(int kv_max) {
 
 static void teardown(void);
 
+int vt_pageable(const void *p) {
+    hipPointerAttribute_t a;
+    if (hipPointerGetAttributes(&a, p) == hipSuccess) return a.type == hipMemoryTypeUnregistered;
+    (void)hipGetLastError();                             /* how some runtimes say that they do not know the address */
+    return 1;
+}
+
 static int init_context(int kv_cache_max) {
     int n = 0;
     if (hipGetDeviceCount(&n) != hipSuccess || n == 0) {

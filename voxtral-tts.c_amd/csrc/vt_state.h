@@ -101,6 +101,7 @@ extern vt_state g_vt;
 
 void vt_set_error(const char *fmt, ...);
 int vt_check(hipError_t e, const char *what);
+int vt_pageable(const void *p);           /* host memory that the runtime does not know; 0: device, managed and pinned memory */
 void *vt_scratch(size_t bytes);      /* grows on demand; contents undefined */
 void *vt_dev_alloc(size_t bytes);
 
