@@ -15,8 +15,8 @@
  * where 256-column tiles come in multiples of 192 items: q|k|v / output / down at 700 rows 57.5 / 40.7 / 79.4 -> 51.1 / 37.2 /
  * 72.5 us, at 1000 75.0 / 53.3 / 104.9 -> 68.5 / 49.2 / 97.0, output / down at 1531 73.3 / 149.4 -> 67.1 / 140.6.
  * Measured against every tile and cut count at 65 .. 1531 rows of the backbone's products and 84 .. 8024 of the codec's, the plan taken is
- * 0.9 and 0.4 % behind the fastest on average, at worst 9 % (q|k|v at 600 rows, whole 192-column tiles on 224 CUs instead
- * of 240 cut ones) and 5 %. */
+ * 0.9 to 1.0 and 0.4 % behind the fastest on average, at worst 9 to 12 % (q|k|v at 600 rows, whole 192-column tiles on 224 CUs
+ * instead of 240 cut ones; output at 256 rows) and 5 to 6 %, on two boxes. */
 struct gw_format {
     int products;                         /* matrix instructions per pair of operands */
     float launch_us, item_us, planes;     /* planes: passes over a cut column's planes */
