@@ -219,7 +219,7 @@ void tts_hip_predict_velocity_cfg(float *out_v_cond, float *out_v_uncond, const 
 /* One audio frame on the device: semantic head + argmax, 7 Euler steps with
  * CFG from the caller's noise x0[36], FSQ quantisation -> codes[37]
  * (voxtral_tts_acoustic.c:268-373).  Host pointers; synchronous.  out_x
- * (optional) receives the final latent. */
+ * (optional) receives the final latent; another NULL is refused. */
 void tts_hip_acoustic_frame(int *out_codes, const float *llm_hidden, const float *x0,
                             float *out_x);
 

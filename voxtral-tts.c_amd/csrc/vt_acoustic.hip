@@ -1069,6 +1069,7 @@ static void finish_frame(int *out_codes, float *out_x) {
 extern "C" void tts_hip_acoustic_frame(int *out_codes, const float *llm_hidden, const float *x0,
                                        float *out_x) {
     if (!ac_ready("tts_hip_acoustic_frame")) return;
+    if (!out_codes || !llm_hidden || !x0) { vt_set_error("tts_hip_acoustic_frame: NULL argument"); return; }
     ac_work w;
     if (enqueue_frame(&w, llm_hidden, NULL, x0)) return;
     finish_frame(out_codes, out_x);
@@ -1137,6 +1138,7 @@ extern "C" void tts_hip_audio_embed(float *out_embed, const int *codes) {
  * caller keeps the RNG).  Returns the codes; after an END_AUDIO frame d_embed is not meaningful. */
 extern "C" void tts_hip_generate_frame(int *out_codes, float *d_embed, const float *x0, int pos) {
     if (!ac_ready("tts_hip_generate_frame") || !embed_ready("tts_hip_generate_frame")) return;
+    if (!out_codes || !d_embed || !x0) { vt_set_error("tts_hip_generate_frame: NULL argument"); return; }
     if (g_vt.n_dec_layers < 1) { vt_set_error("tts_hip_generate_frame: no backbone weights uploaded"); return; }
     if (vt_run_step(g_vt.d_layers, g_vt.n_dec_layers, 0, g_vt.d_dec_norm, d_embed, g_vt.d_hidden, pos)) return;
     ac_work w;
