@@ -8,6 +8,7 @@
  */
 #include "vt_state.h"
 #include "vt_gemm.h"
+#include "vt_requests.h"
 
 #include <math.h>
 #include <stdlib.h>
@@ -216,12 +217,12 @@ vt_linear_rows_kernel(float *y, const float *x, const uint16_t *W, const float *
     /* part t: block t / per_block, pass, part of the pass; past the last one: zeros, which nobody reads */
     const int w_voff = (lane >> 3) * in_dim * 2 + ((lane & 7) ^ (lane >> 3)) * 16;
     auto ask = [&](unsigned char *buf, int t) {
-        const int b = t / per_block, pass = t % per_block / P, part = t % P, left = min(rows - 16 * b, 16);
-        const __amdgpu_buffer_rsrc_t d = __builtin_amdgcn_make_buffer_rsrc((void *)(W + (size_t)(row0 + (t < n ? 16 * b : 0)) * in_dim), 0, t < n ? left * in_dim * 2 : 0, 0x00020000);
+        const vt_request q = vt_rows_request(t, n, H, P, passes, rows, in_dim, wave);
+        const __amdgpu_buffer_rsrc_t d = __builtin_amdgcn_make_buffer_rsrc((void *)(W + (size_t)(row0 + 16 * vt_rows_block(t, n, P, passes)) * in_dim), 0, q.bytes, 0x00020000);
 #pragma unroll
         for (int j = 0; j < 2 * H; j++)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(d, (__attribute__((address_space(3))) void *)(buf + wave * PART + j * 1024), 16, w_voff + (j & 1) * 16 * in_dim,
-                                                     ((pass * 8 + wave) * KW + part * 64 * H + 64 * (j >> 1)) * 2, 0, 2);
+                                                     q.soff + (t < n ? 128 * (j >> 1) : 0), 0, 2);
     };
     f32x4 acc[4];
     auto multiply = [&](const unsigned char *buf, auto part) {

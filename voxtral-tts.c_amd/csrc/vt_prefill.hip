@@ -12,6 +12,7 @@
  */
 #include "vt_state.h"
 #include "vt_gemm.h"
+#include "vt_requests.h"
 
 #include <math.h>
 
@@ -184,17 +185,16 @@ vt_prefill_attention_kernel(float *out, uint16_t *out_hi, uint16_t *out_lo, cons
     const int ntiles = last_q / 32 + 1;                  /* key tiles 0 .. ntiles-1 are visible */
     const int nsteps = (ntiles + NS - 1) / NS;
 
-    /* the waves of a residue copy KB kilobytes of its tile, from `from` of the tile on, 1 KB per wave and request; a tile
-     * past the last visible one lies beyond the descriptor's end: zeros, which nobody reads */
-    const __amdgpu_buffer_rsrc_t t_rs = __builtin_amdgcn_make_buffer_rsrc(
-        (void *)(img + (size_t)kvh * img_tiles * PA_TILE_BYTES), 0, ntiles * PA_TILE_BYTES, 0x00020000);
+    /* the waves of a residue copy KB kilobytes of its tile, from `from` of the tile on, 1 KB per wave and request; for a tile
+     * past the last visible one: zeros, which nobody reads */
     constexpr int KB = QB == 32 ? 32 : 16;
     auto fetch = [&](unsigned char *buf, int step, int from) {
-        const int soff = (step * NS + pz) * PA_TILE_BYTES + from;
+        const vt_request rq = vt_tile_request(step * NS + pz, ntiles, PA_TILE_BYTES, from);
+        const __amdgpu_buffer_rsrc_t t_rs = __builtin_amdgcn_make_buffer_rsrc((void *)(img + (size_t)kvh * img_tiles * PA_TILE_BYTES), 0, rq.bytes, 0x00020000);
 #pragma unroll
         for (int i = 0; i < KB / HW; i++)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(t_rs, (__attribute__((address_space(3))) void *)(buf + pz * KB * 1024 + (i * HW + hq) * 1024), 16,
-                                                     (i * HW + hq) * 1024 + lane * 16, soff, 0, 0);
+                                                     (i * HW + hq) * 1024 + lane * 16, rq.soff, 0, 0);
     };
     fetch(pa_a, 0, 0);
 

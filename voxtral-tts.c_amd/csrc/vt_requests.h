@@ -1,0 +1,30 @@
+/*
+ * vt_requests.h - which bytes the kernels' requests through a buffer descriptor ask for where some of them have nothing to
+ * bring: the number of requests is fixed (the waits count them), so one for a tile past the last visible one, or for a part past
+ * a workgroup's last, still goes out.  Such a request has size 0 AND scalar offset 0: whether the hardware's range check
+ * takes the scalar offset into account (and how, where that is the larger one) then makes no difference.  Pure integer
+ * functions, compiled for the device by hipcc and for the host by any C++ compiler; a host test walks every request.
+ */
+#ifndef VT_REQUESTS_H
+#define VT_REQUESTS_H
+
+#include "vt_rowsplit.h"
+
+struct vt_request { int bytes, soff; };   /* the descriptor's size and the scalar offset */
+
+/* Prefill attention: `from` bytes into tile `tile` of the ntiles that are visible, counted from tile 0 */
+VT_HD vt_request vt_tile_request(int tile, int ntiles, int tile_bytes, int from) {
+    const bool live = tile < ntiles;
+    return vt_request{live ? ntiles * tile_bytes : 0, live ? tile * tile_bytes + from : 0};
+}
+
+/* Linear layers of a few rows: part t of a workgroup's n, i.e. part t % P of pass t / P % passes over K of a block of 16 of its
+ * `rows` weight rows, H lines of 128 bytes per row; counted from the block's first row (t >= n: none) */
+VT_HD int vt_rows_block(int t, int n, int P, int passes) { return t < n ? t / (P * passes) : 0; }
+VT_HD vt_request vt_rows_request(int t, int n, int H, int P, int passes, int rows, int in_dim, int wave) {
+    const int left = rows - 16 * vt_rows_block(t, n, P, passes), pass = t % (P * passes) / P, part = t % P;
+    const bool live = t < n;
+    return vt_request{live ? (left < 16 ? left : 16) * in_dim * 2 : 0, live ? ((pass * 8 + wave) * P + part) * 128 * H : 0};
+}
+
+#endif /* VT_REQUESTS_H */
