@@ -321,26 +321,50 @@ static void linear_rows(float *d_y, const float *d_x, const uint16_t *d_W, const
 }
 
 /* ---- K of up to 64: a thread per output column, four rows of x through LDS -----------------------------------
- * (3072 x 36 at 300 rows: 71 us with a wave per output column that went through the rows, 6 with this one.) */
+ * (3072 x 36 at 300 rows: 71 us with a wave per output column that went through the rows, 6 with this one.)
+ * Sixteen sums per output, added as a tree: no larger an error than a wave's 64 lanes and theirs (relative to the norm, at
+ * K = 16 / 36 / 50 / 64: 6.0e-8 / 6.3e-8 / 6.5e-8 / 6.8e-8, the wave 6.0e-8 / 6.7e-8 / 6.9e-8 / 7.1e-8; one chain 7.4e-8 / 1.09e-7 /
+ * 1.27e-7 / 1.45e-7, four sums 5.6e-8 / 6.9e-8 / 7.6e-8 / 8.3e-8). */
 #define LN_K 64
 #define LN_ROWS 4
+#define LN_SUMS 16
 __global__ void __launch_bounds__(256)
 vt_linear_narrow_kernel(float *y, const float *x, const uint16_t *W, const float *bias, int seq_len, int in_dim, int out_dim) {
-    __shared__ float xs[LN_ROWS][LN_K];
+    __shared__ float xs[LN_ROWS][LN_K];                  /* zeros behind K and behind the last row */
     const int s0 = (int)blockIdx.y * LN_ROWS, ns = min(LN_ROWS, seq_len - s0), o = (int)(blockIdx.x * 256 + threadIdx.x);
-    for (int i = threadIdx.x; i < LN_ROWS * in_dim; i += 256) xs[i / in_dim][i % in_dim] = i / in_dim < ns ? x[(size_t)s0 * in_dim + i] : 0.f;
+    const int xr = (int)threadIdx.x / LN_K, xk = (int)threadIdx.x % LN_K;
+    xs[xr][xk] = xr < ns && xk < in_dim ? x[(size_t)(s0 + xr) * in_dim + xk] : 0.f;
     __syncthreads();
     if (o >= out_dim) return;
     const uint16_t *wr = W + (size_t)o * in_dim;
-    float acc[LN_ROWS] = {};
-    for (int k = 0; k < in_dim; k++) {
-        const float w = __uint_as_float((unsigned)wr[k] << 16);
+    float acc[LN_ROWS][LN_SUMS] = {};
+    auto add = [&](int k0, const unsigned (&w)[LN_SUMS]) {
 #pragma unroll
-        for (int s = 0; s < LN_ROWS; s++) acc[s] = fmaf(w, xs[s][k], acc[s]);
+        for (int j = 0; j < LN_SUMS; j++)
+#pragma unroll
+            for (int s = 0; s < LN_ROWS; s++) acc[s][j] = fmaf(__uint_as_float(w[j] << 16), xs[s][k0 + j], acc[s][j]);
+    };
+    int k = 0;
+    for (; k + LN_SUMS <= in_dim; k += LN_SUMS) {
+        unsigned w[LN_SUMS];
+#pragma unroll
+        for (int j = 0; j < LN_SUMS; j++) w[j] = wr[k + j];
+        add(k, w);
+    }
+    if (k < in_dim) {
+        unsigned w[LN_SUMS];
+#pragma unroll
+        for (int j = 0; j < LN_SUMS; j++) w[j] = k + j < in_dim ? wr[k + j] : 0u;
+        add(k, w);
     }
 #pragma unroll
-    for (int s = 0; s < LN_ROWS; s++)
-        if (s < ns) y[(size_t)(s0 + s) * out_dim + o] = bias ? __fadd_rn(bias[o], acc[s]) : acc[s];
+    for (int s = 0; s < LN_ROWS; s++) {
+#pragma unroll
+        for (int n = LN_SUMS / 2; n > 0; n /= 2)
+#pragma unroll
+            for (int j = 0; j < n; j++) acc[s][j] = __fadd_rn(acc[s][j], acc[s][j + n]);
+        if (s < ns) y[(size_t)(s0 + s) * out_dim + o] = bias ? __fadd_rn(bias[o], acc[s][0]) : acc[s][0];
+    }
 }
 
 void vt_launch_linear(float *d_y, const float *d_x, const uint16_t *d_W, const float *d_bias,
