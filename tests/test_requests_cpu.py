@@ -40,7 +40,7 @@ int main(void) {
                 for (int t = 0; t < n + 2; t++)
                     for (int wave = 0; wave < 8; wave++) {
                         const vt_request r = vt_rows_request(t, n, H, P, passes, rows, in_dim, wave);
-                        const int first = 16 * vt_rows_block(t, n, P, passes);
+                        const int first = 16 * r.block;
                         if (first >= rows) { bad++; printf("block %d of %d rows\n", first, rows); }
                         /* the last row that the descriptor holds, all lines of the part; rows behind it lie beyond its size */
                         const int last = (rows - first < 16 ? rows - first : 16) - 1;

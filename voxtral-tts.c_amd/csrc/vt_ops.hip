@@ -218,7 +218,7 @@ vt_linear_rows_kernel(float *y, const float *x, const uint16_t *W, const float *
     const int w_voff = (lane >> 3) * in_dim * 2 + ((lane & 7) ^ (lane >> 3)) * 16;
     auto ask = [&](unsigned char *buf, int t) {
         const vt_request q = vt_rows_request(t, n, H, P, passes, rows, in_dim, wave);
-        const __amdgpu_buffer_rsrc_t d = __builtin_amdgcn_make_buffer_rsrc((void *)(W + (size_t)(row0 + 16 * vt_rows_block(t, n, P, passes)) * in_dim), 0, q.bytes, 0x00020000);
+        const __amdgpu_buffer_rsrc_t d = __builtin_amdgcn_make_buffer_rsrc((void *)(W + (size_t)(row0 + 16 * q.block) * in_dim), 0, q.bytes, 0x00020000);
 #pragma unroll
         for (int j = 0; j < 2 * H; j++)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(d, (__attribute__((address_space(3))) void *)(buf + wave * PART + j * 1024), 16, w_voff + (j & 1) * 16 * in_dim,

@@ -10,21 +10,20 @@
 
 #include "vt_rowsplit.h"
 
-struct vt_request { int bytes, soff; };   /* the descriptor's size and the scalar offset */
+struct vt_request { int block, bytes, soff; };       /* which block of rows; the descriptor's size; the scalar offset */
 
 /* Prefill attention: `from` bytes into tile `tile` of the ntiles that are visible, counted from tile 0 */
 VT_HD vt_request vt_tile_request(int tile, int ntiles, int tile_bytes, int from) {
     const bool live = tile < ntiles;
-    return vt_request{live ? ntiles * tile_bytes : 0, live ? tile * tile_bytes + from : 0};
+    return vt_request{0, live ? ntiles * tile_bytes : 0, live ? tile * tile_bytes + from : 0};
 }
 
 /* Linear layers of a few rows: part t of a workgroup's n, i.e. part t % P of pass t / P % passes over K of a block of 16 of its
  * `rows` weight rows, H lines of 128 bytes per row; counted from the block's first row (t >= n: none) */
-VT_HD int vt_rows_block(int t, int n, int P, int passes) { return t < n ? t / (P * passes) : 0; }
 VT_HD vt_request vt_rows_request(int t, int n, int H, int P, int passes, int rows, int in_dim, int wave) {
-    const int left = rows - 16 * vt_rows_block(t, n, P, passes), pass = t % (P * passes) / P, part = t % P;
     const bool live = t < n;
-    return vt_request{live ? (left < 16 ? left : 16) * in_dim * 2 : 0, live ? ((pass * 8 + wave) * P + part) * 128 * H : 0};
+    const int block = t / (P * passes), at = t - block * (P * passes), left = rows - 16 * block;
+    return vt_request{live ? block : 0, live ? (left < 16 ? left : 16) * in_dim * 2 : 0, live ? ((at / P * 8 + wave) * P + at % P) * 128 * H : 0};
 }
 
 #endif /* VT_REQUESTS_H */
