@@ -51,3 +51,10 @@ def compare(hip, m, n, k, group):
 @pytest.mark.parametrize("m,n,k", [(2, 3072, 36), (5, 3072, 64), (300, 300, 36), (40, 257, 63), (7, 1000, 16), (9, 999, 50), (33, 200, 5)])
 def test_short_rows(hip, m, n, k):
     compare(hip, m, n, k, 1)
+
+
+# the fp32 matrix instructions: each kernel (K / 512 a multiple of 6, of 4, even, odd), one pass over K and several
+@pytest.mark.parametrize("m,n,k", [(16, 36, 3072), (8, 50, 9216), (12, 60, 4096), (8, 70, 2048), (9, 100, 1024), (16, 50, 5120), (20, 100, 512),
+                                   (8, 60, 2560), (4, 3072, 3072)])
+def test_a_few_rows(hip, m, n, k):
+    compare(hip, m, n, k, 8)

@@ -183,17 +183,23 @@ static int matvec_launch(float *d_y, const float *d_x, const uint16_t *d_W, cons
  * v_mfma_f32_16x16x4_f32, so that operands, products and sums are fp32 (bf16 weights widened exactly).  A workgroup owns
  * rows_per_wg consecutive rows of W, its eight waves share K: wave w keeps its K slice of x in registers as the B operand,
  * 16 weight rows at a time come as the A operand (lane l: row l%16, 8 consecutive k of group l/16; the k order inside an
- * instruction is free as long as both operands agree), and the waves' sums are added through LDS in wave order, one barrier
+ * instruction is free as long as both operands agree), and the waves' sums are added through LDS, one barrier
  * per 16 rows.  A wave's piece of 16 rows comes in P parts of H lines of 128 bytes per row, by buffer loads straight into three LDS
  * buffers of its own: eight lanes bring a line (lane i its 16-byte piece i%8 ^ row%8, so that eight lanes reading one piece
  * of eight rows meet all banks), two parts are on their way while one is multiplied, and a wave waits for nothing but its own loads.
  * (Loaded into the operands directly, an instruction touches 64 pieces of 16 bytes, and the CU's address path takes
  * twice as long as the stream.)  Three arrays, so that the compiler knows that reading one need not wait for the others.  K of
  * more than 512 H P takes its slices in passes.
+ * An instruction adds its four products to the sum one after another.  Eight sums per wave, taken in turn, and trees over these
+ * and over the waves make chains of K / 64 as in a wave per weight row, and the same error against 64 bits: relative to the norm
+ * 1.42e-7 at K = 3072, 2.25e-7 at 9216 (four sums and the waves in turn: 1.89e-7 and 3.1e-7; sixteen: 1.15e-7 and 1.69e-7, 3 to 5 %
+ * slower).  A block's sums start with the first part's instructions where that part has a copy of its own (H 3, which is 4 to
+ * 8 % faster); with smaller parts, of which few follow one another, the copy's code costs more than clearing the sums.
  * An instruction does 16 weight rows and 16 rows of x in 32 cycles, so that a CU could take 38 KB of weights per us, half
- * as much again as its share of HBM.  us per call at 2 / 5 / 8 / 16 rows, 9216 x 3072: 18.2 / 18.7 / 19.0 / 21.0; 131072 x 3072: 145 / 143 / 144 / 149; with a wave per
- * weight row and, from 8 rows on, planes, tiles and partial sums in three launches: 14 / 25 / 24 / 25 and 195 / 329 / 184 / 198. */
+ * as much again as its share of HBM.  us per call at 4 / 5 / 8 / 16 rows, 9216 x 3072: 17.2 / 17.5 / 18.2 / 20.3, at 2 / 5 / 16 rows 131072 x 3072:
+ * 135 / 134 / 142; with a wave per weight row and, from 8 rows on, planes, tiles and partial sums in three launches: 21 / 25 / 24 / 24 and 192 / 328 / 196. */
 #define LR_ROWS 16
+#define LR_SUMS 8                         /* a wave's sums; 2 H 8 instructions per part are a multiple */
 template <int N> struct lr_int { static constexpr int v = N; };
 template <int H, int P>
 __global__ void __launch_bounds__(512)
@@ -224,8 +230,8 @@ vt_linear_rows_kernel(float *y, const float *x, const uint16_t *W, const float *
             __builtin_amdgcn_raw_ptr_buffer_load_lds(d, (__attribute__((address_space(3))) void *)(buf + wave * PART + j * 1024), 16, w_voff + (j & 1) * 16 * in_dim,
                                                      q.soff + (t < n ? 128 * (j >> 1) : 0), 0, 2);
     };
-    f32x4 acc[4];
-    auto multiply = [&](const unsigned char *buf, auto part) {
+    f32x4 acc[LR_SUMS];
+    auto multiply = [&](const unsigned char *buf, auto part, auto first) {
         u32x4 w[2 * H];
 #pragma unroll
         for (int i = 0; i < 2 * H; i++)
@@ -235,13 +241,19 @@ vt_linear_rows_kernel(float *y, const float *x, const uint16_t *W, const float *
 #pragma unroll
             for (int j = 0; j < 8; j++) {
                 const unsigned u = w[i][j / 2];
-                acc[j & 3] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(j & 1 ? u & 0xffff0000u : u << 16), xr[2 * H * decltype(part)::v + i][j / 4][j % 4], acc[j & 3], 0, 0, 0);
+                f32x4 &a = acc[(8 * i + j) % LR_SUMS];
+                a = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(j & 1 ? u & 0xffff0000u : u << 16), xr[2 * H * decltype(part)::v + i][j / 4][j % 4],
+                                                         decltype(first)::v && 8 * i + j < LR_SUMS ? f32x4{0.f, 0.f, 0.f, 0.f} : a, 0, 0, 0);
             }
     };
     /* accumulator element v of lane l: weight row 4 (l/16) + v, row l%16 of x.  Bare barriers: __syncthreads() would wait for
      * the parts on their way. */
     auto finish = [&](int b) {
-        const f32x4 q = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+#pragma unroll
+        for (int n = LR_SUMS / 2; n > 0; n /= 2)
+#pragma unroll
+            for (int a = 0; a < n; a++) acc[a] = acc[a] + acc[a + n];
+        const f32x4 q = acc[0];
         asm volatile("" ::: "memory");
         __builtin_amdgcn_s_barrier();                                        /* the block before has been summed */
         asm volatile("" ::: "memory");
@@ -253,22 +265,28 @@ vt_linear_rows_kernel(float *y, const float *x, const uint16_t *W, const float *
         asm volatile("" ::: "memory");
         const int t = (int)threadIdx.x, s = t >> 4, r = 16 * b + (t & 15);
         if (t < 256 && s < ns && r < rows) {
-            float sum = red[0][t];
+            float part[8];
 #pragma unroll
-            for (int w = 1; w < 8; w++) sum = __fadd_rn(sum, red[w][t]);
+            for (int w = 0; w < 8; w++) part[w] = red[w][t];
+#pragma unroll
+            for (int w = 4; w > 0; w /= 2)
+#pragma unroll
+                for (int a = 0; a < w; a++) part[a] = __fadd_rn(part[a], part[a + w]);
+            const float sum = part[0];
             y[(size_t)(s0 + s) * out_dim + row0 + r] = bias ? __fadd_rn(bias[row0 + r], sum) : sum;
         }
     };
     auto item = [&](int t, auto part, const unsigned char *here, unsigned char *later) {
-        if (t % per_block == 0)
+        if (H < 3 && t % per_block == 0)
 #pragma unroll
-            for (int a = 0; a < 4; a++) acc[a] = f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int a = 0; a < LR_SUMS; a++) acc[a] = f32x4{0.f, 0.f, 0.f, 0.f};
         asm volatile("" ::: "memory");
         __builtin_amdgcn_s_waitcnt(0x0f70 | (2 * H));                        /* vmcnt: the next part may be on its way */
         asm volatile("" ::: "memory");
         ask(later, t + 2);
         asm volatile("" ::: "memory");
-        multiply(here, part);
+        if (H == 3 && decltype(part)::v == 0 && t % per_block == 0) multiply(here, part, lr_int<1>());
+        else multiply(here, part, lr_int<0>());
         if (passes > 1 && t % P == P - 1) load_x((t + 1) % per_block / P);
         if (t % per_block == per_block - 1) finish(t / per_block);
     };
