@@ -339,13 +339,14 @@ static void linear_rows(float *d_y, const float *d_x, const uint16_t *d_W, const
 }
 
 /* ---- K of up to 64: a thread per output column, four rows of x through LDS -----------------------------------
- * (3072 x 36 at 300 rows: 71 us with a wave per output column that went through the rows, 6 with this one.)
- * Sixteen sums per output, added as a tree: no larger an error than a wave's 64 lanes and theirs (relative to the norm, at
- * K = 16 / 36 / 50 / 64: 6.0e-8 / 6.3e-8 / 6.5e-8 / 6.8e-8, the wave 6.0e-8 / 6.7e-8 / 6.9e-8 / 7.1e-8; one chain 7.4e-8 / 1.09e-7 /
- * 1.27e-7 / 1.45e-7, four sums 5.6e-8 / 6.9e-8 / 7.6e-8 / 8.3e-8). */
+ * (3072 x 36 at 300 rows: 71 us with a wave per output column that went through the rows, 7 with this one.)
+ * Sixteen sums per output, eight for K up to 48, added as a tree: no larger an error than a wave's 64 lanes and theirs (relative to
+ * the norm, at K = 16 / 36 / 50 / 64: 5.6e-8 / 6.3e-8 / 6.5e-8 / 6.8e-8, the wave 6.0e-8 / 6.7e-8 / 6.9e-8 / 7.1e-8; one chain 7.4e-8 /
+ * 1.09e-7 / 1.27e-7 / 1.45e-7).  What bounds a launch of few rows is code that is run once and comes from memory: 3072 x 36 takes 3.5 us
+ * with eight sums, 4.1 with sixteen, 3.3 with one chain. */
 #define LN_K 64
 #define LN_ROWS 4
-#define LN_SUMS 16
+template <int SUMS, bool REST>                           /* REST: K is no multiple of SUMS */
 __global__ void __launch_bounds__(256)
 vt_linear_narrow_kernel(float *y, const float *x, const uint16_t *W, const float *bias, int seq_len, int in_dim, int out_dim) {
     __shared__ float xs[LN_ROWS][LN_K];                  /* zeros behind K and behind the last row */
@@ -355,34 +356,45 @@ vt_linear_narrow_kernel(float *y, const float *x, const uint16_t *W, const float
     __syncthreads();
     if (o >= out_dim) return;
     const uint16_t *wr = W + (size_t)o * in_dim;
-    float acc[LN_ROWS][LN_SUMS] = {};
-    auto add = [&](int k0, const unsigned (&w)[LN_SUMS]) {
+    float acc[LN_ROWS][SUMS] = {};
+    auto add = [&](int k0, int j, unsigned w) {
 #pragma unroll
-        for (int j = 0; j < LN_SUMS; j++)
-#pragma unroll
-            for (int s = 0; s < LN_ROWS; s++) acc[s][j] = fmaf(__uint_as_float(w[j] << 16), xs[s][k0 + j], acc[s][j]);
+        for (int s = 0; s < LN_ROWS; s++) acc[s][j] = fmaf(__uint_as_float(w << 16), xs[s][k0 + j], acc[s][j]);
     };
     int k = 0;
-    for (; k + LN_SUMS <= in_dim; k += LN_SUMS) {
-        unsigned w[LN_SUMS];
+#pragma unroll 1
+    for (; k + SUMS <= in_dim; k += SUMS) {
+        uint16_t w[SUMS];
+        __builtin_memcpy(w, wr + k, sizeof w);
 #pragma unroll
-        for (int j = 0; j < LN_SUMS; j++) w[j] = wr[k + j];
-        add(k, w);
+        for (int j = 0; j < SUMS; j++) add(k, j, w[j]);
     }
-    if (k < in_dim) {
-        unsigned w[LN_SUMS];
+    if constexpr (REST) {
+        unsigned w[SUMS - 1];
 #pragma unroll
-        for (int j = 0; j < LN_SUMS; j++) w[j] = k + j < in_dim ? wr[k + j] : 0u;
-        add(k, w);
+        for (int j = 0; j < SUMS - 1; j++) w[j] = k + j < in_dim ? wr[k + j] : 0u;
+#pragma unroll
+        for (int j = 0; j < SUMS - 1; j++) add(k, j, w[j]);
     }
 #pragma unroll
     for (int s = 0; s < LN_ROWS; s++) {
 #pragma unroll
-        for (int n = LN_SUMS / 2; n > 0; n /= 2)
+        for (int n = SUMS / 2; n > 0; n /= 2)
 #pragma unroll
             for (int j = 0; j < n; j++) acc[s][j] = __fadd_rn(acc[s][j], acc[s][j + n]);
         if (s < ns) y[(size_t)(s0 + s) * out_dim + o] = bias ? __fadd_rn(bias[o], acc[s][0]) : acc[s][0];
     }
+}
+
+static void linear_narrow(float *d_y, const float *d_x, const uint16_t *d_W, const float *d_bias, int seq_len, int in_dim, int out_dim) {
+    const dim3 grid((out_dim + 255) / 256, (seq_len + LN_ROWS - 1) / LN_ROWS);
+#define CALL(SUMS) do { \
+        if (in_dim % SUMS) hipLaunchKernelGGL((vt_linear_narrow_kernel<SUMS, true>), grid, dim3(256), 0, g_vt.stream, d_y, d_x, d_W, d_bias, seq_len, in_dim, out_dim); \
+        else hipLaunchKernelGGL((vt_linear_narrow_kernel<SUMS, false>), grid, dim3(256), 0, g_vt.stream, d_y, d_x, d_W, d_bias, seq_len, in_dim, out_dim); \
+    } while (0)
+    if (in_dim <= 48) CALL(8);
+    else CALL(16);
+#undef CALL
 }
 
 void vt_launch_linear(float *d_y, const float *d_x, const uint16_t *d_W, const float *d_bias,
@@ -392,11 +404,9 @@ void vt_launch_linear(float *d_y, const float *d_x, const uint16_t *d_W, const f
     for (; seq_len > most; seq_len -= most, d_x += (size_t)most * in_dim, d_y += (size_t)most * out_dim)
         vt_launch_linear(d_y, d_x, d_W, d_bias, most, in_dim, out_dim);
     if (linear_rows_ok(d_x, d_W, seq_len, in_dim, out_dim)) { linear_rows(d_y, d_x, d_W, d_bias, seq_len, in_dim, out_dim); return; }
-    if (seq_len > 1 && in_dim <= LN_K) {
-        hipLaunchKernelGGL(vt_linear_narrow_kernel, dim3((out_dim + 255) / 256, (seq_len + LN_ROWS - 1) / LN_ROWS), dim3(256), 0, g_vt.stream, d_y, d_x, d_W, d_bias,
-                           seq_len, in_dim, out_dim);
-        return;
-    }
+    /* K of up to 64: few rows of few columns are a wave's work each (3072 x 36 at 2 rows 2.7 us, narrow 3.4, at 5 3.5 both; 3072 x 64
+     * at 2 / 5 2.9 / 4.0 and 4.4 / 4.6; 9216 x 16 at 2 4.0 and 2.7) */
+    if (seq_len > (out_dim > 4096 ? 1 : in_dim <= 48 ? 4 : 8) && in_dim <= LN_K) { linear_narrow(d_y, d_x, d_W, d_bias, seq_len, in_dim, out_dim); return; }
     const int vec_ok = (in_dim % 8 == 0) && (((uintptr_t)d_W | (uintptr_t)d_x) % 16 == 0), rows = seq_len == 1 ? 1 : seq_len <= 4 ? 4 : 8;
     const dim3 grid((out_dim + 3) / 4, (seq_len + rows - 1) / rows), block(256);
 #define CALL(S, G) hipLaunchKernelGGL((vt_linear_kernel<S, G>), grid, block, 0, g_vt.stream, d_y, d_x, d_W, d_bias, seq_len, in_dim, out_dim, vec_ok)
