@@ -1050,10 +1050,13 @@ static int enqueue_frame(ac_work *w, const float *h_hidden, const float *d_hidde
     return vt_check(hipGetLastError(), "frame launch");
 }
 
-static void finish_frame(int *out_codes, float *out_x) {
+/* bad: what enqueue_frame returned.  Waits in front of every return, also behind a frame that was queued in part: its kernels read
+ * the pinned noise and hidden state that the next call fills and, where they are pinned, the caller's own. */
+static void finish_frame(int bad, int *out_codes, float *out_x) {
     const ac_frame_out *pin = (const ac_frame_out *)(g_vt.h_pin + VT_PIN_FRAME);
-    VT_TRYV(hipGetLastError());
+    bad = bad || vt_check(hipGetLastError(), "frame launch");
     VT_TRYV(hipStreamSynchronize(g_vt.stream));
+    if (bad) return;
     if (g_vt.step_pending) {                /* the backbone step in front of this frame: was it abandoned? */
         g_vt.step_pending = 0;
         if (pin->abort) { (void)vt_step_poll_abort_now(); return; }
@@ -1071,8 +1074,7 @@ extern "C" void tts_hip_acoustic_frame(int *out_codes, const float *llm_hidden, 
     if (!ac_ready("tts_hip_acoustic_frame")) return;
     if (!out_codes || !llm_hidden || !x0) { vt_set_error("tts_hip_acoustic_frame: NULL argument"); return; }
     ac_work w;
-    if (enqueue_frame(&w, llm_hidden, NULL, x0)) return;
-    finish_frame(out_codes, out_x);
+    finish_frame(enqueue_frame(&w, llm_hidden, NULL, x0), out_codes, out_x);
 }
 
 /* ---- audio-code embedding and the per-frame loop -------------------------------------- */
@@ -1142,9 +1144,10 @@ extern "C" void tts_hip_generate_frame(int *out_codes, float *d_embed, const flo
     if (g_vt.n_dec_layers < 1) { vt_set_error("tts_hip_generate_frame: no backbone weights uploaded"); return; }
     if (vt_run_step(g_vt.d_layers, g_vt.n_dec_layers, 0, g_vt.d_dec_norm, d_embed, g_vt.d_hidden, pos)) return;
     ac_work w;
-    if (enqueue_frame(&w, NULL, g_vt.d_hidden, x0)) return;
+    const int bad = enqueue_frame(&w, NULL, g_vt.d_hidden, x0);
     vt_acoustic_dev *ac = &g_vt.ac;
-    hipLaunchKernelGGL(vt_audio_embed_kernel, dim3(VT_DIM / 256), dim3(256), 0, g_vt.stream, d_embed, ac->audio_emb,
-                       ac->audio_offsets, w.codes, ac->audio_rows);
-    finish_frame(out_codes, NULL);
+    if (!bad)
+        hipLaunchKernelGGL(vt_audio_embed_kernel, dim3(VT_DIM / 256), dim3(256), 0, g_vt.stream, d_embed, ac->audio_emb,
+                           ac->audio_offsets, w.codes, ac->audio_rows);
+    finish_frame(bad, out_codes, NULL);
 }
