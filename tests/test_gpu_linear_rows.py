@@ -17,7 +17,9 @@ def hip():
     h.close()
 
 
-@pytest.mark.parametrize("n,k", [(36, 3072), (1000, 4096), (9216, 3072), (3072, 9216), (17, 256), (300, 1280), (3072, 36), (257, 64), (5, 1), (36, 100)])
+@pytest.mark.parametrize("n,k", [(36, 3072), (1000, 4096), (9216, 3072), (3072, 9216), (17, 256), (300, 1280), (3072, 36), (257, 64), (5, 1), (36, 100),
+                                 # each instance (K / 512 a multiple of 4, even, odd) with more than 16 rows per workgroup at 49 rows, in passes over K
+                                 (1111, 8192), (1300, 1024), (1200, 5120), (1100, 2560)])
 @pytest.mark.parametrize("m", [1, 2, 7, 15, 16, 17, 49])
 def test_rows(hip, m, n, k):
     W = S.bf16_normal((n, k), 4000 + n + k)
