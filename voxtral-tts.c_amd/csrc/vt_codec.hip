@@ -422,12 +422,13 @@ static struct {
     /* work area, grown to the largest decode so far and laid out anew by each (cd_carve) */
     unsigned char *work;
     size_t work_bytes;
-    float *x, *qkv, *part, *wave;
+    float *x, *qkv, *part;
     cd_planes planes;
     unsigned char *host;          /* pinned: the waveform of the largest decode so far and its codes (7828 bytes a frame) */
     size_t host_bytes;
     hipEvent_t written[CD_WAVE_PARTS];
-    int *codes;
+    float *probe_wave;            /* vt_codec_probe_buffers */
+    int *probe_codes;
 } g_cd;
 
 static void cd_free_ptr(float **p) { if (*p) (void)hipFree(*p); *p = NULL; }
@@ -452,6 +453,8 @@ void vt_codec_free(void) {
     cd_free_matrix(&g_cd.w_out); cd_free_ptr(&g_cd.b_out);
     if (g_cd.work) (void)hipFree(g_cd.work);
     if (g_cd.host) (void)hipHostFree(g_cd.host);
+    cd_free_ptr(&g_cd.probe_wave);
+    if (g_cd.probe_codes) (void)hipFree(g_cd.probe_codes);
     for (int i = 0; i < CD_WAVE_PARTS; i++)
         if (g_cd.written[i]) (void)hipEventDestroy(g_cd.written[i]);
     memset(&g_cd, 0, sizeof g_cd);
@@ -641,10 +644,9 @@ static int cd_reserve(int n_frames) {
         part = n > part ? n : part;
     }
     /* the pieces start at multiples of 256 bytes */
-    const size_t f = sizeof(float), sizes[] = {T * CD_DIM * f, T * 3 * CD_DIM * f, part * f, T * CD_PATCH * f, T * CD_HID * 2, T * CD_HID * 2,
-                                               (T + 4) * f, (size_t)n_frames * 37 * sizeof(int)};
-    size_t total = 0, at[8];
-    for (int i = 0; i < 8; i++) { at[i] = total; total += (sizes[i] + 255) & ~(size_t)255; }
+    const size_t f = sizeof(float), sizes[] = {T * CD_DIM * f, T * 3 * CD_DIM * f, part * f, T * CD_HID * 2, T * CD_HID * 2, (T + 4) * f};
+    size_t total = 0, at[6];
+    for (int i = 0; i < 6; i++) { at[i] = total; total += (sizes[i] + 255) & ~(size_t)255; }
     if (total > g_cd.work_bytes) {
         (void)hipStreamSynchronize(g_vt.stream);
         if (g_cd.work) (void)hipFree(g_cd.work);
@@ -655,9 +657,7 @@ static int cd_reserve(int n_frames) {
     g_cd.x = (float *)(g_cd.work + at[0]);
     g_cd.qkv = (float *)(g_cd.work + at[1]);
     g_cd.part = (float *)(g_cd.work + at[2]);
-    g_cd.wave = (float *)(g_cd.work + at[3]);
-    g_cd.planes = cd_planes{(uint16_t *)(g_cd.work + at[4]), (uint16_t *)(g_cd.work + at[5]), (int *)(g_cd.work + at[6])};
-    g_cd.codes = (int *)(g_cd.work + at[7]);
+    g_cd.planes = cd_planes{(uint16_t *)(g_cd.work + at[3]), (uint16_t *)(g_cd.work + at[4]), (int *)(g_cd.work + at[5])};
     return 0;
 }
 
@@ -730,16 +730,19 @@ static int cd_wave(float *samples, const cd_product &p, int t0, int t1) {
 
 static int cd_enqueue_all(const int *codes, int n_frames, float *d_samples) { return cd_wave(d_samples, cd_enqueue(codes, n_frames), 0, n_frames * 8); }
 
+#define CD_MAX_FRAMES 4096
 static int cd_ready(const char *who, int n_frames) {
     if (!g_vt.initialized || !g_cd.uploaded) { vt_set_error("%s: codec weights not uploaded", who); return -1; }
-    if (n_frames < 1 || n_frames > 4096) { vt_set_error("%s: n_frames %d out of range", who, n_frames); return -1; }
+    if (n_frames < 1 || n_frames > CD_MAX_FRAMES) { vt_set_error("%s: n_frames %d out of range", who, n_frames); return -1; }
     if (cd_reserve(n_frames)) { vt_set_error("%s: out of device memory for %d frames", who, n_frames); return -1; }
     return 0;
 }
 
-/* pinned memory and the events of the waveform's parts */
+/* pinned memory and the events of the waveform's parts. */
 #define CD_WAVE_PART_BYTES (480 << 10)
-static int cd_host(size_t bytes) {
+#define CD_HOST_FRAME_BYTES (sizeof(float) * 8 * CD_PATCH + sizeof(int) * 37)
+static int cd_pin(int n_frames) {
+    size_t bytes = n_frames * CD_HOST_FRAME_BYTES;
     for (int i = 0; i < CD_WAVE_PARTS; i++)
         if (!g_cd.written[i] && vt_check(hipEventCreateWithFlags(&g_cd.written[i], hipEventDisableTiming), "codec event")) return -1;
     if (bytes <= g_cd.host_bytes) return 0;
@@ -769,7 +772,7 @@ extern "C" void tts_hip_codec_decode(const int *codes, int n_frames, float **out
     if (cd_ready("tts_hip_codec_decode", n_frames)) return;
     const int rows = n_frames * 8, n = rows * CD_PATCH;
     const size_t code_bytes = (size_t)n_frames * 37 * sizeof(int);
-    if (cd_host((size_t)n * sizeof(float) + code_bytes)) { vt_set_error("tts_hip_codec_decode: out of host memory"); return; }
+    if (cd_pin(n_frames)) { vt_set_error("tts_hip_codec_decode: out of host memory"); return; }
     float *s = (float *)malloc((size_t)n * sizeof(float));
     if (!s) { vt_set_error("tts_hip_codec_decode: out of host memory"); return; }
     /* Codes and samples cross through pinned memory that the kernels read and write themselves; the caller's buffer is filled
@@ -800,12 +803,16 @@ extern "C" void tts_hip_codec_decode(const int *codes, int n_frames, float **out
 
 /* For other translation units of the library: one launch of the decoder's product kernel at the last
  * stage's 1600 rows with the q|k|v, output, gate|up or down matrix of layer 7 (which 0..3), or of the whole
- * decoder on 200 frames of resident codes (which 4), on the decoder's own work area.  vt_codec_probe_fill makes
+ * decoder on 200 frames of resident codes (which 4), on the decoder's own work area and a waveform and codes of the
+ * probe's.  vt_codec_probe_fill makes
  * the planes that which 0..3 read from fp32 values x [1600, k], k = 1024 or 4096. */
+#define CD_PROBE_FRAMES 200
 int vt_codec_probe_buffers(float **x, int **codes) {
     if (!g_cd.uploaded) { vt_set_error("codec weights not uploaded"); return -1; }
-    if (cd_reserve(200)) { vt_set_error("codec: out of device memory"); return -1; }
-    *x = g_cd.part; *codes = g_cd.codes;
+    if (cd_reserve(CD_PROBE_FRAMES)) { vt_set_error("codec: out of device memory"); return -1; }
+    if (!g_cd.probe_wave && !(g_cd.probe_wave = (float *)vt_dev_alloc(sizeof(float) * CD_PROBE_FRAMES * 8 * CD_PATCH))) return -1;
+    if (!g_cd.probe_codes && !(g_cd.probe_codes = (int *)vt_dev_alloc(sizeof(int) * CD_PROBE_FRAMES * 37))) return -1;
+    *x = g_cd.part; *codes = g_cd.probe_codes;
     return 0;
 }
 
@@ -823,10 +830,10 @@ void vt_codec_probe_fill(const float *x, int k) {
 }
 
 int vt_codec_probe_launch(int which) {
-    const int frames = 200;
+    const int frames = CD_PROBE_FRAMES;
     const cd_layer_dev *l = &g_cd.layers[CD_LAYERS - 1];
     const cd_matrix *w[4] = {&l->wqkv, &l->wo, &l->w13, &l->w2};
-    if (which == 4) return cd_enqueue_all(g_cd.codes, frames, g_cd.wave);
+    if (which == 4) return cd_enqueue_all(g_cd.probe_codes, frames, g_cd.probe_wave);
     if (which < 0 || which > 3) return -1;
     (void)cd_gemm(frames * 8, *w[which]);
     return 0;
