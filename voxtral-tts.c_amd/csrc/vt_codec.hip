@@ -738,7 +738,8 @@ static int cd_ready(const char *who, int n_frames) {
     return 0;
 }
 
-/* pinned memory and the events of the waveform's parts. */
+/* pinned memory and the events of the waveform's parts.  The memory doubles at least, up to what the longest decode takes (32 MB):
+ * decodes that slowly get longer pin it anew five times. */
 #define CD_WAVE_PART_BYTES (480 << 10)
 #define CD_HOST_FRAME_BYTES (sizeof(float) * 8 * CD_PATCH + sizeof(int) * 37)
 static int cd_pin(int n_frames) {
@@ -748,9 +749,10 @@ static int cd_pin(int n_frames) {
     if (bytes <= g_cd.host_bytes) return 0;
     (void)hipStreamSynchronize(g_vt.stream);
     if (g_cd.host) (void)hipHostFree(g_cd.host);
+    const size_t longest = CD_MAX_FRAMES * CD_HOST_FRAME_BYTES, twice = 2 * g_cd.host_bytes > 1 << 20 ? 2 * g_cd.host_bytes : 1 << 20;
+    bytes = bytes > twice ? bytes : twice < longest ? twice : longest;
     g_cd.host_bytes = 0;
     g_cd.host = NULL;
-    bytes = (bytes + ((1 << 20) - 1)) & ~(size_t)((1 << 20) - 1);
     if (vt_check(hipHostMalloc((void **)&g_cd.host, bytes, hipHostMallocDefault), "codec host memory")) { g_cd.host = NULL; return -1; }
     g_cd.host_bytes = bytes;
     return 0;
