@@ -10,13 +10,16 @@
  * long as the operands of its steps need to arrive (step_us: a step of the 128- and 192-column tiles is two K steps, half
  * of the waves at each) and item_us for sums and stores, but no less than the card's
  * power limit lets the matrix cores of its items run (pflops, executed, padding included: narrow tiles pay
- * for their bytes here, too); a launch takes 5 us; cut planes are written and read once more.
+ * for their bytes here, too); cut planes are written and read once more.  (The codec's item_us is what an item takes beside its steps and what its
+ * matrix instructions take beyond them: the choice depends on their sum.)
  * The backbone's 192 columns divide 6144 and 3072 into 32 and 16 tiles, so that 1, 2, 4, .. row tiles fill the 256 CUs
  * where 256-column tiles come in multiples of 192 items: q|k|v / output / down at 700 rows 57.5 / 40.7 / 79.4 -> 51.1 / 37.2 /
  * 72.5 us, at 1000 75.0 / 53.3 / 104.9 -> 68.5 / 49.2 / 97.0, output / down at 1531 73.3 / 149.4 -> 67.1 / 140.6.
- * Measured against every tile and cut count at 65 .. 1531 rows of the backbone's products and 84 .. 8024 of the codec's, the plan taken is
- * 0.9 to 1.0 and 0.4 % behind the fastest on average, at worst 9 to 12 % (q|k|v at 600 rows, whole 192-column tiles on 224 CUs
- * instead of 240 cut ones; output at 256 rows) and 5 to 6 %, on two boxes. */
+ * Measured against every tile and cut count at 65 .. 1531 rows of the backbone's products, the plan taken is 0.9 to 1.0 % behind the
+ * fastest on average, at worst 9 to 12 % (q|k|v at 600 rows, whole 192-column tiles on 224 CUs instead of 240 cut ones; output at 256
+ * rows), on two boxes; for the codec's at 110 row counts from 65 to 8024, 0.2 % and at worst 7 % (down at 1500 rows, 96 x 256 in 4 cuts
+ * instead of 96 x 128 in 2).  Constants fitted to every second of these are 0.3 % behind at the others; fitted to the nine that
+ * decodes of 21, 212 and 1003 frames have, 0.6 % and 20 % (gate|up at 105 rows, 128 x 128 in 4 cuts 25 us, 96 x 128 in 2 21). */
 struct gw_format {
     int products;                         /* matrix instructions per pair of operands */
     float launch_us, item_us, planes;     /* planes: passes over a cut column's planes */
@@ -24,7 +27,7 @@ struct gw_format {
     float pflops[3];                      /* [128, 192, 256 columns] */
 };
 static const gw_format gw_backbone = {2, 5.0f, 2.8f, 1.45f, {{1.28f, 0.f}, {1.97f, 2.96f}, {1.15f, 1.65f}}, {0.91f, 1.07f, 1.21f}};
-static const gw_format gw_codec = {3, 6.0f, 1.0f, 1.4f, {{1.76f, 2.81f}, {0.f, 0.f}, {1.89f, 2.44f}}, {0.865f, 0.f, 0.98f}};
+static const gw_format gw_codec = {3, 2.5f, 14.2f, 1.79f, {{1.53f, 2.78f}, {0.f, 0.f}, {1.68f, 2.37f}}, {0.795f, 0.f, 1.33f}};
 
 static float gw_rounds(int items, float item_us, float power_us) {
     const int full = items / g_vt.n_cu, rem = items % g_vt.n_cu;
