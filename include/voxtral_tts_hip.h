@@ -314,8 +314,10 @@ const char *tts_hip_last_error(void);
 
 /* The activation format of the sequence-level products: n fp32 values (n even, device pointers,
  * 8-byte aligned) -> two bf16 planes, hi = bf16(x) rounded to nearest even and lo = bf16(x - hi),
- * so that hi + lo carries x to about 2^-17 relative (tts_hip_linear_bf16 with seq_len >= 8 and
- * tts_hip_llm_prefill multiply every weight tile with both planes).  No counterpart in the
+ * so that hi + lo carries x to about 2^-17 relative (tts_hip_llm_prefill multiplies every weight tile
+ * with both planes, and so does tts_hip_linear_bf16 with seq_len >= 8, out_dim a multiple of 128 and
+ * in_dim of 64; except for up to 16 rows with in_dim a multiple of 512 and seq_len * in_dim <= 49152,
+ * whose products are fp32 like those of all other shapes).  No counterpart in the
  * reference, whose CPU products read the fp32 activations directly (voxtral_tts_kernels.c:127-138);
  * exported so that the format can be checked bit for bit.  Returns 0, or -1 on error. */
 int tts_hip_split_planes(uint16_t *d_hi, uint16_t *d_lo, const float *d_x, size_t n);

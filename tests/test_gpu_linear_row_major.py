@@ -22,10 +22,10 @@ def hip():
                                    (8, 128, 64), (20, 1024, 3072), (64, 640, 192), (65, 128, 64), (96, 384, 192), (97, 256, 1088),
                                    (128, 768, 320), (129, 9216, 192), (150, 1152, 3072), (300, 640, 4096), (300, 3072, 1088),
                                    (700, 8320, 192), (33, 32768, 128), (110, 640, 320),
-                                   # a short K goes to tiles of 128 x 128: either side of where, per group of rows; the edges above with a longer one
+                                   # short and long K, few and many columns: strips in 1 to 8 cuts, tiles whole and cut, tiles of 128 x 128
                                    (33, 384, 448), (33, 384, 512), (64, 640, 576), (20, 32768, 448), (65, 128, 1984), (65, 128, 2048), (96, 384, 2112),
                                    (150, 256, 2048), (96, 384, 128), (110, 384, 768), (257, 640, 448), (300, 256, 3072), (300, 256, 3136),
-                                   (512, 512, 2048), (512, 512, 2112), (300, 8320, 256)])
+                                   (512, 512, 2048), (512, 512, 2112), (300, 8320, 256), (16, 12288, 4096), (40, 131072, 64), (192, 5120, 1024)])
 @pytest.mark.parametrize("noalloc", [False, True])
 def test_rows(hip, m, n, k, noalloc):
     W = S.bf16_normal((n, k), 5000 + n + k)

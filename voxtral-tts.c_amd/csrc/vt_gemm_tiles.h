@@ -1,7 +1,7 @@
 /*
  * vt_gemm_tiles.h - the tile kernels of the sequence-level products C[M,N] = X[M,K] W[N,K]^T on the matrix cores,
- * fp32 accumulation, for weights in fragment order (vt_launch_frag_layout): vt_gemm_wide_kernel and, for few rows,
- * vt_gemm_rows_kernel.  Both are templates over the number format (gm_bf16, gm_f16x2 below).
+ * fp32 accumulation: vt_gemm_wide_kernel, for weights in fragment order (vt_launch_frag_layout) or, with FRAG false, row-major
+ * ones, and, for few rows and fragment order, vt_gemm_rows_kernel.  Both are templates over the number format (gm_bf16, gm_f16x2 below).
  */
 #ifndef VT_GEMM_TILES_H
 #define VT_GEMM_TILES_H

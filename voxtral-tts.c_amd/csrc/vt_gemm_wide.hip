@@ -23,11 +23,12 @@
 struct gw_format {
     int products;                         /* matrix instructions per pair of operands */
     float launch_us, item_us, planes;     /* planes: passes over a cut column's planes */
+    float sums_us, stream_tbps;           /* the launch that adds them (0: whoever reads the result does); the weights' rate (0: no bound) */
     float step_us[3][2];                  /* [128, 192, 256 columns][96, 128 rows]; 0: tile not used */
     float pflops[3];                      /* [128, 192, 256 columns] */
 };
-static const gw_format gw_backbone = {2, 5.0f, 2.8f, 1.45f, {{1.28f, 0.f}, {1.97f, 2.96f}, {1.15f, 1.65f}}, {0.91f, 1.07f, 1.21f}};
-static const gw_format gw_codec = {3, 2.5f, 14.2f, 1.79f, {{1.53f, 2.78f}, {0.f, 0.f}, {1.68f, 2.37f}}, {0.795f, 0.f, 1.33f}};
+static const gw_format gw_backbone = {2, 5.0f, 2.8f, 1.45f, 0.f, 0.f, {{1.28f, 0.f}, {1.97f, 2.96f}, {1.15f, 1.65f}}, {0.91f, 1.07f, 1.21f}};
+static const gw_format gw_codec = {3, 2.5f, 14.2f, 1.79f, 0.f, 0.f, {{1.53f, 2.78f}, {0.f, 0.f}, {1.68f, 2.37f}}, {0.795f, 0.f, 1.33f}};
 
 static float gw_rounds(int items, float item_us, float power_us) {
     const int full = items / g_vt.n_cu, rem = items % g_vt.n_cu;
@@ -42,12 +43,12 @@ static float gw_cost(const gw_format &f, int M, int N, int K, int mb, int tn, in
     float t = f.launch_us + gw_rounds(mt * n_main, (float)((K / 64 + kw - 1) / kw) * t_step + f.item_us, tile_us);
     if (rest) {
         t += gw_rounds(mt * rest * cuts, (float)((K / 64 + cuts * kw - 1) / (cuts * kw)) * t_step + f.item_us, tile_us / cuts);
-        if (cuts > 1 || swiglu) t += f.planes * cuts * M * (float)(rest * tn) * 4.f / 4.5e6f + (swiglu ? 4.5f : 0.f);
+        if (cuts > 1 || swiglu) t += f.planes * cuts * M * (float)(rest * tn) * 4.f / 4.5e6f + (swiglu ? 4.5f : cuts > 1 ? f.sums_us : 0.f);
     }
-    return t;
+    return f.stream_tbps > 0.f ? fmaxf(t, f.launch_us + N * 2.f * K / (f.stream_tbps * 1e6f)) : t;
 }
 
-static vt_gemm_plan gw_plan(const gw_format &f, int M, int N, int K, int swiglu, int most = VT_MAX_CUTS) {
+static vt_gemm_plan gw_plan(const gw_format &f, int M, int N, int K, int swiglu, int most = VT_MAX_CUTS, float *us = NULL) {
     vt_gemm_plan best = {0, 64, 0, 1};
     float best_cost = 0.f;
     for (int mb = 3; mb <= 4; mb++)
@@ -72,6 +73,7 @@ static vt_gemm_plan gw_plan(const gw_format &f, int M, int N, int K, int swiglu,
                 }
             }
         }
+    if (us) *us = best_cost;
     return best;
 }
 
@@ -125,19 +127,42 @@ static void gw_run(const vt_gemm_plan &pl, gw_part whole, gw_part cut, const uin
     launch[pl.row_major][pl.mb - 3][pl.tn / 64 - 2](list, d_Ahi, d_Alo, M, K);
 }
 
-/* The cost constants are those of fragment order: a lane's own row costs four times the lines per request, and with the steps
- * 15 % or a cut column's planes twice as dear the plans were no better at 65 to 300 rows.  A step's four requests of a line
- * stand one in each of its regions, as with fragments: all in the last one, 42 us instead of 39 for 9216 x 3072 at 150 rows.
- * Strips up to 64 rows, beyond 32 only while they are one per CU (32768 x 3072 at 64 rows: 63 us, tiles 52) */
-vt_gemm_plan vt_gemm_row_major_plan(int M, int N, int K, int most) {
-    vt_gemm_plan pl;
-    if (vt_gemm_rows_ok(M, N, K) && (M <= 32 || N <= 96 * g_vt.n_cu)) {
-        pl = vt_gemm_few_rows_plan(N, 0);
-        if (pl.cuts > most) pl.cuts = most;
-        if (pl.cuts > K / 64) pl.cuts = K / 64;
-    } else {
-        pl = gw_plan(gw_backbone, M, N, K, 0, most);
-        if (pl.cuts == 1) pl.col0 = N;
+/* Products on a caller's row-major weights: tiles (a lane's own row costs four times the lines per request, hence constants of
+ * their own; a step's four requests of a line stand one in each of its regions, as with fragments: all in the last one, 42 us instead of
+ * 39 for 9216 x 3072 at 150 rows), up to 64 rows strips of 96 columns, and the 128 x 128 tiles of vt_launch_gemm, two
+ * workgroups per CU, which stage the weights through LDS in whole lines.  Each is taken where it is expected to be the fastest.  Fitted
+ * to 1312 shapes, 28 of N and K from 512 x 8192 to 131072 x 3072 and 8 .. 1000 rows, the launch that adds planes included: the choice is
+ * 0.9 % behind the fastest of all tiles, strips and cuts on average, 3.2 % where bounds on M, N and K made it, and takes 0.882 of the time
+ * of 128 x 128 tiles alone, 0.902; above 1.05 of it at 3 shapes, 84 (18 rows of 4608 x 1024 1.25; at most 1.83).  No part of it came near
+ * the card's power limit (pflops). */
+static const gw_format gw_row_major = {2, 6.101f, 2.766f, 1.642f, 1.944f, 4.665f, {{1.379f, 0.f}, {1.894f, 1.962f}, {1.112f, 1.119f}}, {99.f, 99.f, 99.f}};
+
+/* Strips: a workgroup goes through its K steps three at a time, which takes longer by the group of 8 rows, and so do its sums; but no
+ * less than its or the card's share of the weights' rate allows */
+static float gw_strip_us(int M, int N, int K, int tn, int cuts) {
+    const int groups = (M + 7) / 8, rounds = ((N + tn - 1) / tn * cuts + g_vt.n_cu - 1) / g_vt.n_cu, steps = ((K / 64 + cuts - 1) / cuts + 2) / 3 * 3;
+    const float work = steps * (0.164f + 0.03824f * groups) + 6.692f + 0.1547f * groups, share = steps * 0.5741f;
+    const float t = 0.7534f + fmaxf(rounds * fmaxf(work, share), N * 2.f * K / 4.734e6f);
+    return cuts > 1 ? t + gw_row_major.sums_us + gw_row_major.planes * cuts * M * (float)N * 4.f / 4.5e6f : t;
+}
+
+float vt_gemm_equal_us(int M, int N, int K, int cuts) {
+    const int items = (M + 127) / 128 * (N / 128) * cuts, slots = 2 * g_vt.n_cu, rem = items % slots;
+    const float steps = K / cuts / 64, short_rows = 0.23f * (1.f - (M < 128 ? M : 128) / 128.f);
+    float t = 4.228f + items / slots * (steps * 1.664f + 3.324f);
+    if (rem) t += steps * ((rem <= g_vt.n_cu ? 0.8796f : 1.664f) - short_rows) + 3.324f;
+    return cuts > 1 ? t + gw_row_major.sums_us + 0.1771f * cuts + 0.8242f * (cuts + 1) * M * (float)N * 4.f / 4.5e6f : t;
+}
+
+vt_gemm_plan vt_gemm_row_major_plan(int M, int N, int K, int most, float *us) {
+    vt_gemm_plan pl = gw_plan(gw_row_major, M, N, K, 0, most, us);
+    if (pl.cuts == 1) pl.col0 = N;
+    if (vt_gemm_rows_ok(M, N, K)) {
+        const vt_gemm_plan strips = vt_gemm_few_rows_plan(N, 0);
+        for (int cuts = 1; cuts <= strips.cuts && cuts <= most && cuts <= K / 64; cuts++) {
+            const float t = gw_strip_us(M, N, K, strips.tn, cuts);
+            if (t < *us) { *us = t; pl = strips; pl.cuts = cuts; }
+        }
     }
     pl.row_major = 1;
     return pl;

@@ -432,34 +432,6 @@ static size_t linear_part_bytes(const linear_plan &p, int seq_len, int out_dim) 
     return cuts > 1 ? sizeof(float) * seq_len * (size_t)(out_dim - col0) * cuts : 0;
 }
 
-/* 128 x 128 tiles, two workgroups per CU, stage the weights through LDS in whole lines; the others read a lane's own row and have
- * one workgroup per CU.  us, these and the others, 9216 x 3072 at 17 / 64 / 96 / 150 / 300 / 700 rows: 26 / 28 / 30 / 53 / 65 / 103
- * and 18 / 25 / 29 / 39 / 59 / 87; 3072 x 9216 27 / 31 / 33 / 55 / 72 / 141 and 17 / 23 / 29 / 37 / 57 / 105; 1024 x 3072 15 / 17 / 18 /
- * 21 / 22 / 31 and 11 / 14 / 16 / 18 / 22 / 29.  The 128 x 128 tiles stay the faster ones (ratios are theirs to the others', kernel
- * times over 11 widths from 128 to 32768)
- *   for 97 to 128 rows, one of their tiles and two of 96 rows (9216 x 3072 at 110: 32 and 37);
- *   but not where the others need no cut and save a launch: 0.53 to 0.99 the other way round, K below 768;
- *   with two full rounds of them, unless the others have a quarter fewer rows to pad (131072 x 3072 at 37 / 65 / 150 / 300 rows: 203 /
- *   215 / 412 / 641 and 215 / 228 / 378 / 677);
- *   for columns that are no multiple of 192 or 256, beyond 512 rows, and beyond 256 rows of few columns, K up to 3072 (8320 x 3072 at 700 /
- *   1500 rows: 100 / 187 and 106 / 199; 24 tiles at most: 0.95 up to K 2048, from 4096 on 1.08);
- *   where they make full rounds and pad no more, K up to 2048 (512 x 2048 at 1000 rows 22 and 29, 2048 x 2048 at 512 28 and 33);
- *   and for a short K, whose steps are over before the others' requests ahead pay: below 512 up to 64 rows (0.81 to 0.97 at K 64 to 256;
- *   up to 32 rows only beyond a round of strips) and where nobody cuts (0.76 at 64, 0.84 at 128, 0.97 at 384; 8320 x 64 at 300 rows 9 and
- *   18), below 2048 where both cut up to 256 rows (0.84 at 192, 0.95 at 1536) or only the others do (8320 x 256 at 300 rows 13 and 25). */
-static int linear_equal_cuts(int M, int N, int K, int tiles, int equal, int cuts) {
-    const int pad96 = (M + 95) / 96 * 96, pad128 = (M + 127) / 128 * 128;
-    const bool saves = equal > 1 && cuts == 1;
-    if (M > 96 && M <= 128 && K >= 768) return 1;
-    if (saves) return 0;
-    if (M > 96 && M <= 128) return 1;
-    if (tiles >= 4 * g_vt.n_cu && (M <= 128 || 4 * pad96 > 3 * pad128)) return 1;
-    if (K <= 3072 && ((M > 512 && N % 192 != 0 && N % 256 != 0) || (M > 256 && tiles <= 24))) return 1;
-    if (K <= 2048 && M > 64 && tiles * equal % g_vt.n_cu == 0 && pad128 <= pad96) return 1;
-    if (M <= 64) return K < 512 && (M > 32 || N > 96 * g_vt.n_cu);
-    return K < (cuts == 1 ? 512 : M <= 256 || equal == 1 ? 2048 : 0);
-}
-
 static int linear_mfma_plan(const float *d_y, const float *d_x, const uint16_t *d_W, int seq_len, int in_dim,
                             int out_dim, linear_plan *p) {
     if (seq_len < 8 || linear_rows_before_planes(d_x, d_W, seq_len, in_dim, out_dim) || !vt_gemm_shape_ok(seq_len, out_dim, in_dim, 1) ||
@@ -472,15 +444,16 @@ static int linear_mfma_plan(const float *d_y, const float *d_x, const uint16_t *
         if (vt_gemm_shape_ok(seq_len, out_dim, in_dim, cand[i])) p->equal_cuts = cand[i];
     const size_t planes = 2 * sizeof(uint16_t) * (size_t)seq_len * in_dim, equal = linear_part_bytes(*p, seq_len, out_dim) + planes;
     p->bytes = equal;
-    p->tiles = vt_gemm_row_major_plan(seq_len, out_dim, in_dim, VT_MAX_CUTS);
-    if (linear_equal_cuts(seq_len, out_dim, in_dim, tiles, p->equal_cuts, p->tiles.cuts)) return 1;
-    p->equal_cuts = 0;
-    for (;; p->tiles = vt_gemm_row_major_plan(seq_len, out_dim, in_dim, p->tiles.cuts - 1)) {
+    const float equal_us = vt_gemm_equal_us(seq_len, out_dim, in_dim, p->equal_cuts);
+    const int equal_cuts = p->equal_cuts;
+    for (int most = VT_MAX_CUTS;; most = p->tiles.cuts - 1) {
+        float us;
+        p->tiles = vt_gemm_row_major_plan(seq_len, out_dim, in_dim, most, &us);
+        p->equal_cuts = us < equal_us ? 0 : equal_cuts;
         const size_t bytes = linear_part_bytes(*p, seq_len, out_dim) + planes;
         p->bytes = bytes > equal ? bytes : equal;
-        if (p->tiles.cuts == 1 || equal > VT_STATIC_SCRATCH_BYTES || bytes <= VT_STATIC_SCRATCH_BYTES) break;
+        if (p->equal_cuts || p->tiles.cuts == 1 || equal > VT_STATIC_SCRATCH_BYTES || bytes <= VT_STATIC_SCRATCH_BYTES) return 1;
     }
-    return 1;
 }
 
 static void linear_mfma_run(unsigned char *base, float *d_y, const float *d_x, const uint16_t *d_W, int seq_len,
