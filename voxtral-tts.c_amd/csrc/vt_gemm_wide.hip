@@ -18,7 +18,7 @@
  * Measured against every tile and cut count at 65 .. 1531 rows of the backbone's products, the plan taken is 0.9 to 1.0 % behind the
  * fastest on average, at worst 9 to 12 % (q|k|v at 600 rows, whole 192-column tiles on 224 CUs instead of 240 cut ones; output at 256
  * rows), on two boxes; for the codec's at 110 row counts from 65 to 8024, 0.2 % and at worst 7 % (down at 1500 rows, 96 x 256 in 4 cuts
- * instead of 96 x 128 in 2).  Constants fitted to every second of these are 0.3 % behind at the others; fitted to the nine that
+ * instead of 96 x 128 in 2), 0.5 and 8 % at half of them on a third box.  Constants fitted to every second of these are 0.3 % behind at the others; fitted to the nine that
  * decodes of 21, 212 and 1003 frames have, 0.6 % and 20 % (gate|up at 105 rows, 128 x 128 in 4 cuts 25 us, 96 x 128 in 2 21). */
 struct gw_format {
     int products;                         /* matrix instructions per pair of operands */
