@@ -133,25 +133,26 @@ static void gw_run(const vt_gemm_plan &pl, gw_part whole, gw_part cut, const uin
  * workgroups per CU, which stage the weights through LDS in whole lines.  Each is taken where it is expected to be the fastest.  Fitted
  * to 1312 shapes, 28 of N and K from 512 x 8192 to 131072 x 3072 and 8 .. 1000 rows, the launch that adds planes included: the choice is
  * 0.9 % behind the fastest of all tiles, strips and cuts on average, 3.2 % where bounds on M, N and K made it, and takes 0.882 of the time
- * of 128 x 128 tiles alone, 0.902; above 1.05 of it at 3 shapes, 84 (18 rows of 4608 x 1024 1.25; at most 1.83).  No part of it came near
+ * of 128 x 128 tiles alone, 0.902; above 1.05 of it at 5 shapes, 84 (18 rows of 4608 x 1024 1.25; at most 1.83).  No part of it came near
  * the card's power limit (pflops). */
-static const gw_format gw_row_major = {2, 6.101f, 2.766f, 1.642f, 1.944f, 4.665f, {{1.379f, 0.f}, {1.894f, 1.962f}, {1.112f, 1.119f}}, {99.f, 99.f, 99.f}};
+static const gw_format gw_row_major = {2, 6.875f, 2.226f, 1.892f, 2.173f, 4.638f, {{1.446f, 0.f}, {1.968f, 2.054f}, {1.138f, 1.189f}}, {99.f, 99.f, 99.f}};
 
 /* Strips: a workgroup goes through its K steps three at a time, which takes longer by the group of 8 rows, and so do its sums; but no
  * less than its or the card's share of the weights' rate allows */
 static float gw_strip_us(int M, int N, int K, int tn, int cuts) {
     const int groups = (M + 7) / 8, rounds = ((N + tn - 1) / tn * cuts + g_vt.n_cu - 1) / g_vt.n_cu, steps = ((K / 64 + cuts - 1) / cuts + 2) / 3 * 3;
-    const float work = steps * (0.164f + 0.03824f * groups) + 6.692f + 0.1547f * groups, share = steps * 0.5741f;
-    const float t = 0.7534f + fmaxf(rounds * fmaxf(work, share), N * 2.f * K / 4.734e6f);
+    const float work = steps * (0.2246f + 0.02967f * groups) + 3.623f + 0.3222f * groups, share = steps * 0.6939f;
+    const float t = 0.3942f + fmaxf(rounds * fmaxf(work, share), N * 2.f * K / 13.36e6f);
     return cuts > 1 ? t + gw_row_major.sums_us + gw_row_major.planes * cuts * M * (float)N * 4.f / 4.5e6f : t;
 }
 
+/* 128 x 128 tiles: a step takes longer the more CUs take one, and shorter with rows to pad */
 float vt_gemm_equal_us(int M, int N, int K, int cuts) {
     const int items = (M + 127) / 128 * (N / 128) * cuts, slots = 2 * g_vt.n_cu, rem = items % slots;
-    const float steps = K / cuts / 64, short_rows = 0.23f * (1.f - (M < 128 ? M : 128) / 128.f);
-    float t = 4.228f + items / slots * (steps * 1.664f + 3.324f);
-    if (rem) t += steps * ((rem <= g_vt.n_cu ? 0.8796f : 1.664f) - short_rows) + 3.324f;
-    return cuts > 1 ? t + gw_row_major.sums_us + 0.1771f * cuts + 0.8242f * (cuts + 1) * M * (float)N * 4.f / 4.5e6f : t;
+    const float steps = K / cuts / 64, short_rows = 0.3468f * (1.f - (M < 128 ? M : 128) / 128.f);
+    float t = 4.158f + items / slots * (steps * 1.737f + 3.122f);
+    if (rem) t += steps * ((rem <= g_vt.n_cu ? 0.8687f + 0.1399f * rem / g_vt.n_cu : 1.737f) - short_rows) + 3.122f;
+    return cuts > 1 ? t + gw_row_major.sums_us + 0.2854f * cuts + 0.7692f * (cuts + 1) * M * (float)N * 4.f / 4.5e6f : t;
 }
 
 vt_gemm_plan vt_gemm_row_major_plan(int M, int N, int K, int most, float *us) {
