@@ -312,10 +312,12 @@ vt_linear_rows_kernel(float *y, const float *x, const uint16_t *W, const float *
 }
 
 /* Whole lines for eight waves, 16-byte loads; and where it is the fastest: against a wave per weight row from 8 rows on, from 4
- * on matrices of 8 M weights and at 2 on those of 128 M (us at 3 / 4 rows, wave per row and this: 4096 x 3072 7 / 9 and 8.8 / 9.0,
- * 9216 x 3072 17 / 21 and 18.3 / 18.5; 1024 x 3072 at 5 / 7 rows 7 / 8 and 8 / 8.5), against planes
- * and strips while a workgroup's rows of x stay below 200 KB (16 rows of 9216 x 3072 and 131072 x 3072 21 / 149, strips at 17 rows 18 / 185,
- * of 4096 x 3072 11.5 / 13; 3072 x 4096 at 12 / 16 rows 13 / 15.3, strips 12.6 at 17; 3072 x 9216 at 12 rows 27, strips 16). */
+ * on matrices of 8 M weights and at 2 on those of 128 M (us a call, a wave per row and this.  One matrix again and again, out of the memory-side
+ * cache: 4096 x 3072 at 3 rows 7.5, at 4 9.0 and 8.8, 9216 x 3072 17.2, 20.6 and 17.8, 3072 x 4096 at 4 / 5 / 7 8.1 / 9.8 / 12.4 and 10.0 / 10.0 /
+ * 10.5, 1024 x 3072 at 7 7.8, at 8 8.4.  Weights from HBM: 4096 x 3072 at 3 10.2, at 4 11.6 and 9.8, 9216 x 3072 24.1, 28.3 and 19.1,
+ * 3072 x 4096 at 4 13.0 and 11.0, 1024 x 3072 at 7 9.8, at 8 8.6), against planes
+ * and strips while a workgroup's rows of x stay below 200 KB (16 rows of 9216 x 3072 and 131072 x 3072 22 / 143, at 17 22 / 191,
+ * of 4096 x 3072 12.4 and 14.7; 3072 x 4096 at 12 rows 14.5, at 16 on strips 12.9; 3072 x 9216 at 4 rows 21, at 8 on strips 18). */
 static int linear_rows_ok(const float *d_x, const uint16_t *d_W, int seq_len, int in_dim, int out_dim) {
     if (in_dim % 512 != 0 || (((uintptr_t)d_W | (uintptr_t)d_x) & 15)) return 0;
     const size_t weights = (size_t)out_dim * in_dim;
