@@ -77,7 +77,7 @@ static void cg_rows(const gr_list &plan, int grid, const uint16_t *d_hi, const u
 
 template <int MB, int CW>
 static void cg_wide(const gw_list &list, const uint16_t *d_hi, const uint16_t *d_lo, int M, int K) {
-    constexpr int LDS = 2 * (4 / CW) * 2 * 32 * MB * GM_STAGE_ROW;
+    constexpr int LDS = 2 * (4 / CW) * 2 * 32 * MB * GM_STAGE_ROW + 32 * MB * (int)sizeof(int);
     static int attr_set = 0;
     if (!attr_set) {
         if (vt_check(hipFuncSetAttribute((const void *)vt_gemm_wide_kernel<gm_f16x2, MB, CW, 2>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS), "product LDS size"))

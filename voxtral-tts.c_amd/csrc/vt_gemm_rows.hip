@@ -134,12 +134,12 @@ vt_gemm_strip_kernel(float *C, int ldc, size_t plane_stride, const uint16_t *Ahi
     }
 
     /* accumulator element v of lane l: row 8*(v/4) + 4*(l/32) + v%4 of the 16 (v < 8: hi, then lo), column l%32 */
-    float *out = C + (size_t)cut * plane_stride + strip * (32 * CB) + 32 * cb + (lane & 31);
+    const __amdgpu_buffer_rsrc_t out = __builtin_amdgcn_make_buffer_rsrc(C + (size_t)cut * plane_stride, 0, here ? M * ldc * 4 : 0, 0x00020000);
+    const int out_at = 4 * (lane >> 5) * ldc * 4 + (strip * (32 * CB) + 32 * cb + (lane & 31)) * 4;
     auto store = [&](int qd, const f32x4 &x) {
-        const int row0 = 8 * qd + 4 * (lane >> 5);
-#pragma unroll
-        for (int v = 0; v < 4; v++)
-            if (row0 + v < M && here) out[(size_t)(row0 + v) * ldc] = x[v];
+        const f32x4 q[1] = {x};
+        const int none[1] = {};
+        gm_store_quad<gm_bf16, 1>(out, out_at + 8 * qd * ldc * 4, ldc * 4, q, i32x4{}, none);
     };
     auto quad = [&](int qd) {
         const f32x16 &p = acc[qd / 2];

@@ -12,6 +12,7 @@
 typedef __bf16 gm_bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 gm_f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef int i32x4 __attribute__((ext_vector_type(4)));
 
 #define GM_STAGE_ROW 144                  /* bytes per staged row: 64 elements of 2 bytes + 16 (fragment reads cover all banks) */
 
@@ -83,21 +84,17 @@ __device__ __forceinline__ void gm_multiply(f32x16 (&acc)[MB][NB], const gm_frag
     }
 }
 
-/* rows row0 .. + 3 of NB columns 32 apart; C and col_exp point at the first of them, C at its row 0 */
+/* Results leave through a descriptor whose size is that of the rows that exist: a row past them is dropped by the range check, with
+ * no branch and no address beyond one addition per row (the row is in the vector offset, which the check counts in any case).
+ * `at`: byte offset of row 0 of the quad, in the first of NB columns 32 apart. */
 template <class T, int NB>
-__device__ __forceinline__ void gm_store_quad(float *C, int ldc, int row0, int M, const f32x4 (&q)[NB], const int *row_exp, const int *col_exp) {
-    int e[NB];
-    if constexpr (T::SCALED) {
-#pragma unroll
-        for (int b = 0; b < NB; b++) e[b] = col_exp[32 * b];
-    }
+__device__ __forceinline__ void gm_store_quad(__amdgpu_buffer_rsrc_t C, int at, int row_bytes, const f32x4 (&q)[NB], const i32x4 &er, const int (&ec)[NB]) {
 #pragma unroll
     for (int v = 0; v < 4; v++)
-        if (row0 + v < M) {
-            const int er = T::SCALED ? row_exp[row0 + v] : 0;
 #pragma unroll
-            for (int b = 0; b < NB; b++)
-                C[(size_t)(row0 + v) * ldc + 32 * b] = T::SCALED ? __builtin_amdgcn_ldexpf(q[b][v], -e[b] - er) : q[b][v];
+        for (int b = 0; b < NB; b++) {
+            const float x = T::SCALED ? __builtin_amdgcn_ldexpf(q[b][v], -ec[b] - er[v]) : q[b][v];
+            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(x), C, at + v * row_bytes + 128 * b, 0, 0);
         }
 }
 
@@ -183,6 +180,7 @@ vt_gemm_wide_kernel(gw_list list, const uint16_t *Ahi, const uint16_t *Alo, int 
      * they were not, a launch's first loads were spilled one by one, each behind a wait: 5 us). */
     constexpr bool EARLY = CW == 4 || MB == 3;
     constexpr int PLANE = TM * GM_STAGE_ROW, GROUP = 2 * PLANE, STAGE = KW * GROUP;
+    int *tile_exp = reinterpret_cast<int *>(lds + 2 * STAGE);      /* T::SCALED: the exponents of the tile's rows */
     const int lane = (int)threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int cw = wave % CW, kw = wave / CW;              /* column block of the tile; which of the KW K steps */
     const int tg = (int)threadIdx.x - kw * 64 * CW;
@@ -281,8 +279,19 @@ vt_gemm_wide_kernel(gw_list list, const uint16_t *Ahi, const uint16_t *Alo, int 
         GW_FENCE();
         fetch_b_slice(it, cur, i + 2, 3);
     };
-    /* the first requests of an item: the planes and weights of steps 0 and 1 */
+    /* The first requests of an item: T::SCALED: the exponents of its rows and of this lane's columns; the planes and weights of steps 0
+     * and 1.  (The exponents asked for where the sums are stored, four rows at a time, each behind the stores before it, took 4.6 us of a
+     * 12 us launch at 84 rows, and 10 of an item's 40 us at 1696.) */
+    int next_row_exp = 0, next_ec[NB] = {}, ec[NB];
     auto begin = [&](const gw_item &it) {
+        if constexpr (T::SCALED) {
+            const gw_part &P = list.part[it.part];
+            const int rows = it.ns > 0 ? min(M - it.mt * TM, TM) : 0;
+            next_row_exp = __builtin_amdgcn_raw_buffer_load_b32(__builtin_amdgcn_make_buffer_rsrc((void *)(P.row_exp + it.mt * TM), 0, rows * 4, 0x00020000), (int)threadIdx.x * 4, 0, 0);
+            const __amdgpu_buffer_rsrc_t d = __builtin_amdgcn_make_buffer_rsrc((void *)(P.col_exp + it.nt * TN), 0, it.ns > 0 ? TN * 4 : 0, 0x00020000);
+#pragma unroll
+            for (int b = 0; b < NB; b++) next_ec[b] = __builtin_amdgcn_raw_buffer_load_b32(d, (32 * (NB * cw + b) + (lane & 31)) * 4, 0, 0);
+        }
         fetch_a(it, Ahi, ra0.hi, 0);
         fetch_a(it, Alo, ra0.lo, 0);
 #pragma unroll
@@ -302,6 +311,11 @@ vt_gemm_wide_kernel(gw_list list, const uint16_t *Ahi, const uint16_t *Alo, int 
             for (int b = 0; b < NB; b++)
 #pragma unroll
                 for (int v = 0; v < 16; v++) acc[a][b][v] = 0.f;
+        if constexpr (T::SCALED) {
+            if ((int)threadIdx.x < TM) tile_exp[threadIdx.x] = next_row_exp;
+#pragma unroll
+            for (int b = 0; b < NB; b++) ec[b] = next_ec[b];
+        }
         store_a(ra0.hi, 0);
         store_a(ra0.lo, PLANE);
         fetch_a(it, Ahi, ra0.hi, AHEAD);
@@ -326,23 +340,28 @@ vt_gemm_wide_kernel(gw_list list, const uint16_t *Ahi, const uint16_t *Alo, int 
 
     /* accumulator element v of lane l: row 8*(v/4) + 4*(l/32) + v%4, column l%32; quads (a, vq) hold v = 4 vq .. + 3 */
     auto emit = [&](const gw_part &P, const gw_item &it, int a, int vq, const f32x4 (&q)[NB]) {
-        const int row0 = it.mt * TM + 32 * a + 8 * vq + 4 * (lane >> 5), c = lane & 31;
+        const int quad_row = 32 * a + 8 * vq, rows = min(M - it.mt * TM, TM), c = lane & 31;      /* of the tile; a lane's first one is 4 (l / 32) on */
         if constexpr (!T::SCALED && NB == 2) {
             if (P.h_hi) {
                 /* a wave's two column blocks are the gates and the ups of the same 32 h columns (voxtral_tts_llm.c:346-350) */
                 const vt_h_quad h = vt_silu_mul_quad(q[0], q[1]);
-                const size_t at = (size_t)(row0 + h.row) * P.ldh + it.nt * (TN / 2) + 32 * cw + (c & ~1);
+                const size_t tile = (size_t)it.mt * TM * P.ldh;
+                const __amdgpu_buffer_rsrc_t d_hi = __builtin_amdgcn_make_buffer_rsrc(P.h_hi + tile, 0, rows * P.ldh * 2, 0x00020000);
+                const __amdgpu_buffer_rsrc_t d_lo = __builtin_amdgcn_make_buffer_rsrc(P.h_lo + tile, 0, rows * P.ldh * 2, 0x00020000);
+                const int at = ((quad_row + 4 * (lane >> 5) + h.row) * P.ldh + it.nt * (TN / 2) + 32 * cw + (c & ~1)) * 2;
 #pragma unroll
-                for (int r = 0; r < 2; r++)
-                    if (row0 + h.row + r < M) {
-                        *reinterpret_cast<unsigned *>(P.h_hi + at + (size_t)r * P.ldh) = h.hi[r];
-                        *reinterpret_cast<unsigned *>(P.h_lo + at + (size_t)r * P.ldh) = h.lo[r];
-                    }
+                for (int r = 0; r < 2; r++) {
+                    __builtin_amdgcn_raw_buffer_store_b32(h.hi[r], d_hi, at + r * P.ldh * 2, 0, 0);
+                    __builtin_amdgcn_raw_buffer_store_b32(h.lo[r], d_lo, at + r * P.ldh * 2, 0, 0);
+                }
                 return;
             }
         }
-        const int col = it.nt * TN + 32 * NB * cw + c;
-        gm_store_quad<T, NB>(P.C + (size_t)it.sp * P.plane_stride + col, P.ldc, row0, M, q, P.row_exp, P.col_exp + col);
+        const __amdgpu_buffer_rsrc_t d = __builtin_amdgcn_make_buffer_rsrc(P.C + (size_t)it.sp * P.plane_stride + (size_t)it.mt * TM * P.ldc, 0, rows * P.ldc * 4, 0x00020000);
+        const int at = 4 * (lane >> 5) * P.ldc * 4 + (it.nt * TN + 32 * NB * cw + c) * 4 + quad_row * P.ldc * 4;
+        i32x4 er = {};
+        if constexpr (T::SCALED) er = *reinterpret_cast<const i32x4 *>(tile_exp + quad_row + 4 * (lane >> 5));
+        gm_store_quad<T, NB>(d, at, P.ldc * 4, q, er, ec);
     };
     auto quads = [&](f32x4 (&q)[NB], int a, int vq) {
 #pragma unroll
@@ -386,6 +405,7 @@ vt_gemm_wide_kernel(gw_list list, const uint16_t *Ahi, const uint16_t *Alo, int 
         }
     };
 
+    /* (one copy of the code that finishes an item: where it runs once, it comes from memory, and so do its instructions) */
     int part = 0, id = (int)blockIdx.x;
     gw_item it = gw_item_at<TN, WP>(list, 0, id, K);
     if constexpr (EARLY) begin(it);
@@ -397,14 +417,16 @@ vt_gemm_wide_kernel(gw_list list, const uint16_t *Ahi, const uint16_t *Alo, int 
             part++;
             id = (int)blockIdx.x;
         }
-        if (part >= list.n_parts) break;
-        const gw_item nx = gw_item_at<TN, WP>(list, part, id, K);
+        const bool more = part < list.n_parts;
+        gw_item nx = it;
+        if (more) nx = gw_item_at<TN, WP>(list, part, id, K);
+        else nx.ns = 0;                   /* requests with nothing to bring */
         if constexpr (EARLY) begin(nx);
         finish(it);
+        if (!more) break;
         __syncthreads();                  /* the next item stages over what this one read */
         it = nx;
     }
-    finish(it);
 }
 
 
@@ -517,8 +539,22 @@ vt_gemm_rows_kernel(gr_list P, const uint16_t *Ahi, const uint16_t *Alo, int M, 
     auto mma = [&](const frags &f, const gm_weights<WP, 2> &w, int ks) { gm_multiply<T, MB, 2>(acc, f, w, ks); };
     gm_weights<WP, 2> b0, b1;
     frags f0, f1;
-    /* the first requests of an item: the rows of step 0, the weights of steps 0 and 1 */
+    /* wave w finishes the quads w, w + NW, ...: rows 8 q + 4 (lane / 32) + 0..3, column lane % 32 of both blocks; T::SCALED: their exponents */
+    constexpr int NQ = (NP + NW - 1) / NW;
+    i32x4 er[NQ] = {};
+    int next_ec[2] = {}, ec[2];
+    if constexpr (T::SCALED) {
+        const __amdgpu_buffer_rsrc_t d = __builtin_amdgcn_make_buffer_rsrc((void *)P.row_exp, 0, M * 4, 0x00020000);
+#pragma unroll
+        for (int i = 0; i < NQ; i++) er[i] = __builtin_bit_cast(i32x4, gm_ldb(d, (8 * (wave + NW * i) + 4 * (lane >> 5)) * 4, 0));
+    }
+    /* the first requests of an item: the exponents of its columns, the rows of step 0, the weights of steps 0 and 1 */
     auto begin = [&](const gr_item &it) {
+        if constexpr (T::SCALED) {
+            const __amdgpu_buffer_rsrc_t d = __builtin_amdgcn_make_buffer_rsrc((void *)(P.col_exp + it.nt * GR_TN), 0, GR_TN * 4, 0x00020000);
+#pragma unroll
+            for (int b = 0; b < 2; b++) next_ec[b] = __builtin_amdgcn_raw_buffer_load_b32(d, (32 * b + (lane & 31)) * 4, 0, 0);
+        }
         fetch_a(it, 0);
 #pragma unroll
         for (int j = 0; j < 4; j++) fetch_b_slice(it, b0, 0, j);
@@ -555,6 +591,8 @@ vt_gemm_rows_kernel(gr_list P, const uint16_t *Ahi, const uint16_t *Alo, int M, 
             for (int b = 0; b < 2; b++)
 #pragma unroll
                 for (int v = 0; v < 16; v++) acc[a][b][v] = 0.f;
+#pragma unroll
+        for (int b = 0; b < 2; b++) ec[b] = next_ec[b];
         store_a();
         fetch_a(it, 1);
         __builtin_amdgcn_sched_barrier(0);
@@ -576,9 +614,11 @@ vt_gemm_rows_kernel(gr_list P, const uint16_t *Ahi, const uint16_t *Alo, int M, 
                     *reinterpret_cast<f32x4 *>(park + (((a * 4 + vq) * 2 + b) * 64 + lane) * 4) =
                         f32x4{acc[a][b][4 * vq], acc[a][b][4 * vq + 1], acc[a][b][4 * vq + 2], acc[a][b][4 * vq + 3]};
         __syncthreads();
-        /* wave w finishes the quads w, w + NW, ...: rows 8 q + 4 (lane / 32) + 0..3, column lane % 32 of both blocks */
+        const __amdgpu_buffer_rsrc_t d = __builtin_amdgcn_make_buffer_rsrc(P.C + (size_t)it.sp * P.plane_stride, 0, M * P.ldc * 4, 0x00020000);
 #pragma unroll
-        for (int qd = wave; qd < NP; qd += NW) {
+        for (int i = 0; i < NQ; i++) {
+            const int qd = wave + NW * i;
+            if (qd >= NP) break;
             f32x4 s[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
             for (int w = 0; w < NW; w++)
@@ -588,9 +628,7 @@ vt_gemm_rows_kernel(gr_list P, const uint16_t *Ahi, const uint16_t *Alo, int M, 
                     s[b].x = __fadd_rn(s[b].x, v.x); s[b].y = __fadd_rn(s[b].y, v.y);
                     s[b].z = __fadd_rn(s[b].z, v.z); s[b].w = __fadd_rn(s[b].w, v.w);
                 }
-            const int row0 = 8 * qd + 4 * (lane >> 5), c = lane & 31;
-            const int col = it.nt * GR_TN + c;
-            gm_store_quad<T, 2>(P.C + (size_t)it.sp * P.plane_stride + col, P.ldc, row0, M, s, P.row_exp, P.col_exp + col);
+            gm_store_quad<T, 2>(d, (8 * qd + 4 * (lane >> 5)) * P.ldc * 4 + (it.nt * GR_TN + (lane & 31)) * 4, P.ldc * 4, s, er[i], ec);
         }
     };
 
