@@ -54,8 +54,8 @@ int vt_codec_weight_layout(uint16_t *d_Wf, int *d_col_exp, const float *d_W, int
 void vt_launch_codec_gemm(float *d_C, const uint16_t *d_hi, const uint16_t *d_lo, const int *d_row_exp,
                           const uint16_t *d_Wf, const int *d_col_exp, int M, int N, int K, const vt_gemm_plan &pl);
 /* row-major bf16 W[N, K] -> the fragment-order copy (same size); N % 32 == 0, K % 64 == 0.  pair: W holds
- * (gate, up) rows interleaved and every 64 fragment columns become 32 gates followed by their 32 ups
- * (N % 64 == 0), the order vt_launch_gemm_frag_swiglu expects. */
+ * (gate, up) rows interleaved and every 32 fragment columns become 16 gates followed by their 16 ups, the order
+ * vt_launch_gemm_frag_swiglu expects. */
 void vt_launch_frag_layout(uint16_t *d_Wf, const uint16_t *d_W, int N, int K, int pair);
 void vt_launch_swiglu_pair_tail(uint16_t *d_hi, uint16_t *d_lo, int ldh, int h_col0, const float *d_tail, int planes,
                                 size_t stride, int rows, int tw);
@@ -89,34 +89,45 @@ __device__ __forceinline__ float vt_silu_mul_small(float g, float u) {       /* 
     return q * u;
 }
 #define VT_SILU_SMALL 83.0f       /* exp(-g) and its reciprocal stay normal, with room for the quotient */
-__device__ __forceinline__ f32x4 vt_silu_mul4(const f32x4 &g, const f32x4 &u) {
-    f32x4 h;
+/* h = silu(g) * u for N of them */
+template <int N>
+__device__ __forceinline__ void vt_silu_mul(float (&h)[N], const float (&g)[N], const float (&u)[N]) {
+    float m = 0.f;
 #pragma unroll
-    for (int v = 0; v < 4; v++) h[v] = vt_silu_mul_small(g[v], u[v]);
+    for (int v = 0; v < N; v++) {
+        h[v] = vt_silu_mul_small(g[v], u[v]);
+        m = fmaxf(m, fabsf(g[v]));
+    }
     /* beyond, infinities included, the formula itself (rare: skipped by waves that have no such gate) */
-    if (__builtin_expect(fmaxf(fmaxf(fabsf(g.x), fabsf(g.y)), fmaxf(fabsf(g.z), fabsf(g.w))) >= VT_SILU_SMALL, 0)) {
+    if (__builtin_expect(m >= VT_SILU_SMALL, 0)) {
 #pragma unroll
-        for (int v = 0; v < 4; v++)
+        for (int v = 0; v < N; v++)
             if (fabsf(g[v]) >= VT_SILU_SMALL) h[v] = __fmul_rn(__fdiv_rn(g[v], __fadd_rn(1.0f, expf(-g[v]))), u[v]);
     }
-    return h;
+}
+__device__ __forceinline__ f32x4 vt_silu_mul4(const f32x4 &g, const f32x4 &u) {
+    const float gs[4] = {g.x, g.y, g.z, g.w}, us[4] = {u.x, u.y, u.z, u.w};
+    float h[4];
+    vt_silu_mul<4>(h, gs, us);
+    return f32x4{h[0], h[1], h[2], h[3]};
 }
 
-/* Four gates and ups of one column (rows v = 0..3; the neighbouring lane holds the next column) -> plane words of two
- * columns and two rows: an even lane keeps rows 0 and 1, an odd one rows 2 and 3, so that a plane takes 4-byte
- * stores, two per quad instead of four of 2 bytes.  The words belong to columns c & ~1 and c | 1. */
-struct vt_h_quad { unsigned hi[2], lo[2]; int row; };
-__device__ __forceinline__ vt_h_quad vt_silu_mul_quad(const f32x4 &g, const f32x4 &u) {
-    const f32x4 h = vt_silu_mul4(g, u);
-    const bool odd = threadIdx.x & 1;
-    vt_h_quad o;
-    o.row = odd ? 2 : 0;
+/* Four rows v = 0..3 of a paired column block (16 gates in lanes 0..15 of 32, the ups of the same h columns in lanes 16..31): the
+ * rows 0 and 1 for the lanes below 16, 2 and 3 for those above, gate and up side by side. */
+__device__ __forceinline__ void vt_pair_rows(const f32x4 &q, float (&g)[2], float (&u)[2]) {
 #pragma unroll
     for (int r = 0; r < 2; r++) {
-        const float got = vt_dpp<0xB1>(odd ? h[r] : h[2 + r]);       /* the other lane's value of my row */
-        vt_split_planes2(odd ? got : h[r], odd ? h[2 + r] : got, o.hi[r], o.lo[r]);
+        const auto x = __builtin_amdgcn_permlane16_swap(__float_as_uint(q[r]), __float_as_uint(q[2 + r]), false, false);
+        g[r] = __uint_as_float(x[0]);
+        u[r] = __uint_as_float(x[1]);
     }
-    return o;
+}
+/* Those two rows of h -> plane words of two columns, so that a plane takes one store of 4 bytes per lane: an even lane's row 0, an odd
+ * one's row 1, columns c & ~1 and c | 1. */
+__device__ __forceinline__ void vt_pair_words(float h0, float h1, unsigned &hi, unsigned &lo) {
+    const bool odd = threadIdx.x & 1;
+    const float got = vt_dpp<0xB1>(odd ? h0 : h1);               /* the other lane's value of my row */
+    vt_split_planes2(odd ? got : h0, odd ? h1 : got, hi, lo);
 }
 #endif
 

@@ -168,9 +168,8 @@ static int gm_blocks(size_t n);
  * feeds to slice j of K step ks of column block nb = n / 32, i.e. W[n][64 ks + 32 g + 8 j .. + 8], go to
  * 16-byte slot ((nb * K/64 + ks) * 4 + j) * 64 + l.  A block of 32 rows occupies the same 32 K elements
  * in both layouts. */
-/* pair: W is a gate|up matrix with (gate, up) rows interleaved; fragment column n' of every 64 takes row
- * 64 (n'/64) + 2 (n' % 32) + (n' % 64) / 32, so that a wave of the product (64 columns) holds the gates of 32
- * h columns in its first column block and their ups in the second. */
+/* pair: W is a gate|up matrix with (gate, up) rows interleaved; fragment column n' of every 32 takes row
+ * 32 (n'/32) + 2 (n' % 16) + (n' % 32) / 16, so that a column block of the product holds 16 gates and their ups, and a wave any number of blocks. */
 __global__ void vt_frag_layout_kernel(u32x4 *out, const uint16_t *W, size_t n_slots, int K, int pair) {
     const int ksteps = K / GM_BK;
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n_slots; i += (size_t)gridDim.x * blockDim.x) {
@@ -179,7 +178,7 @@ __global__ void vt_frag_layout_kernel(u32x4 *out, const uint16_t *W, size_t n_sl
         const int ks = (int)(blk % ksteps);
         const size_t nb = blk / ksteps;
         size_t n = nb * 32 + (l & 31);
-        if (pair) n = (nb >> 1) * 64 + 2 * (l & 31) + (nb & 1);
+        if (pair) n = nb * 32 + 2 * (l & 15) + (l >> 4 & 1);
         out[i] = gm_ld(W + n * K + 64 * ks + 32 * (l >> 5) + 8 * j);
     }
 }
@@ -350,7 +349,7 @@ void vt_launch_swiglu_split(uint16_t *d_hi, uint16_t *d_lo, const float *d_gu, s
 }
 
 /* The K-cut tail of the paired gate|up product: tail [planes][rows, tw] fp32 in the paired column order
- * (of every 64 columns the first 32 are gates, the other 32 the ups of the same h columns) -> the
+ * (of every 32 columns the first 16 are gates, the other 16 the ups of the same h columns) -> the
  * (hi, lo) planes of SiLU(gate) * up at h columns h_col0 .. h_col0 + tw/2 (row pitch ldh).  A thread owns 4
  * consecutive h columns and requests all its planes at once. */
 template <int P>
@@ -360,13 +359,13 @@ __global__ void vt_swiglu_pair_tail_kernel(uint16_t *hi, uint16_t *lo, int ldh, 
     const size_t total = (size_t)rows * per_row;
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (size_t)gridDim.x * blockDim.x) {
         const int row = (int)(i / per_row), q = (int)(i % per_row);
-        const int blk = q >> 3, c = (q & 7) * 4;
-        const float *tp = tail + (size_t)row * tw + 64 * blk + c;
+        const int blk = q >> 2, c = (q & 3) * 4;
+        const float *tp = tail + (size_t)row * tw + 32 * blk + c;
         f32x4 gs[P], us[P];
 #pragma unroll
         for (int p = 0; p < P; p++) {
             gs[p] = *reinterpret_cast<const f32x4 *>(tp + p * stride);
-            us[p] = *reinterpret_cast<const f32x4 *>(tp + p * stride + 32);
+            us[p] = *reinterpret_cast<const f32x4 *>(tp + p * stride + 16);
         }
         f32x4 g = gs[0], u = us[0];
 #pragma unroll
@@ -377,7 +376,7 @@ __global__ void vt_swiglu_pair_tail_kernel(uint16_t *hi, uint16_t *lo, int ldh, 
         const f32x4 h = vt_silu_mul4(g, u);
         u32x2 sph, spl;
         vt_split_planes4(h.x, h.y, h.z, h.w, sph, spl);
-        const size_t at = (size_t)row * ldh + h_col0 + 32 * blk + c;
+        const size_t at = (size_t)row * ldh + h_col0 + 16 * blk + c;
         *reinterpret_cast<u32x2 *>(hi + at) = sph;
         *reinterpret_cast<u32x2 *>(lo + at) = spl;
     }

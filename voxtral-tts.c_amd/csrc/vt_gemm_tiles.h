@@ -104,8 +104,12 @@ __device__ __forceinline__ void gm_store_quad(__amdgpu_buffer_rsrc_t C, int at, 
  * only the activation planes pass through the LDS: 8 KB of fragment reads per 16 matrix instructions, half
  * the LDS bandwidth (a 64 x 64 wave tile with both operands in LDS, vt_gemm_mfma_kernel, needs three quarters).
  * One workgroup of four waves per CU (a wave may then use the whole register file of its SIMD: up to 128
- * accumulator registers, 192 with 96 columns, two sets of weight registers, two sets of fragments), in one of these shapes:
- *   CW = 4: four waves side by side, tile MB*32 x 256; the planes of one K step serve four waves;
+ * accumulator registers, 192 with 96 columns (all 512 are then in use), two sets of weight registers, two sets of fragments), in one of these shapes:
+ *   CW = 4: four waves side by side, tile MB*32 x 256 (NB = 2 blocks of 32 columns per wave) or x 384 (NB = 3); the planes of one K
+ *           step serve four waves.  With 384 columns a fragment read from LDS serves 3 blocks instead of 2: a third less LDS traffic
+ *           per matrix instruction, which is time and, under the card's power limit, clock: executed TFLOP/s at 4096 rows of
+ *           3072 x 9216 1146 with 128 x 256, 1253 with 128 x 192, 1420 with 128 x 384, of 6144 x 3072 1234 / 1153 / 1346 (96 x 512: 989,
+ *           spilled; 64 x 512 1234 and 160 x 384 1159 on a box 5 % slower).  In prefills of 1531 rows, q|k|v / gate|up 101 / 280 -> 87 / 259 us;
  *   CW = 2: two waves side by side and two K steps at a time, tile MB*32 x 128 (NB = 2 blocks of 32 columns per wave) or
  *           x 192 (NB = 3); the two halves of K are added through LDS at the end.  For row counts whose 256-column
  *           tiles do not deal out over the CUs, at the price of more plane traffic (L2 and LDS stores) per matrix
@@ -339,20 +343,29 @@ vt_gemm_wide_kernel(gw_list list, const uint16_t *Ahi, const uint16_t *Alo, int 
 #undef GW_FENCE
 
     /* accumulator element v of lane l: row 8*(v/4) + 4*(l/32) + v%4, column l%32; quads (a, vq) hold v = 4 vq .. + 3 */
-    auto emit = [&](const gw_part &P, const gw_item &it, int a, int vq, const f32x4 (&q)[NB]) {
+    auto emit = [&](const gw_part &P, const gw_item &it, int lane, int a, int vq, const f32x4 (&q)[NB]) {
         const int quad_row = 32 * a + 8 * vq, rows = min(M - it.mt * TM, TM), c = lane & 31;      /* of the tile; a lane's first one is 4 (l / 32) on */
-        if constexpr (!T::SCALED && NB == 2) {
+        if constexpr (!T::SCALED) {
             if (P.h_hi) {
-                /* a wave's two column blocks are the gates and the ups of the same 32 h columns (voxtral_tts_llm.c:346-350) */
-                const vt_h_quad h = vt_silu_mul_quad(q[0], q[1]);
+                /* a column block holds the gates and the ups of 16 h columns (voxtral_tts_llm.c:346-350) */
+                float g[2 * NB], u[2 * NB], h[2 * NB];
+#pragma unroll
+                for (int b = 0; b < NB; b++) {
+                    float g2[2], u2[2];
+                    vt_pair_rows(q[b], g2, u2);
+                    g[2 * b] = g2[0]; g[2 * b + 1] = g2[1]; u[2 * b] = u2[0]; u[2 * b + 1] = u2[1];
+                }
+                vt_silu_mul<2 * NB>(h, g, u);
                 const size_t tile = (size_t)it.mt * TM * P.ldh;
                 const __amdgpu_buffer_rsrc_t d_hi = __builtin_amdgcn_make_buffer_rsrc(P.h_hi + tile, 0, rows * P.ldh * 2, 0x00020000);
                 const __amdgpu_buffer_rsrc_t d_lo = __builtin_amdgcn_make_buffer_rsrc(P.h_lo + tile, 0, rows * P.ldh * 2, 0x00020000);
-                const int at = ((quad_row + 4 * (lane >> 5) + h.row) * P.ldh + it.nt * (TN / 2) + 32 * cw + (c & ~1)) * 2;
+                const int at = ((4 * (lane >> 5) + 2 * (lane >> 4 & 1) + (lane & 1)) * P.ldh + it.nt * (TN / 2) + 16 * NB * cw + (lane & 14)) * 2 + quad_row * P.ldh * 2;
 #pragma unroll
-                for (int r = 0; r < 2; r++) {
-                    __builtin_amdgcn_raw_buffer_store_b32(h.hi[r], d_hi, at + r * P.ldh * 2, 0, 0);
-                    __builtin_amdgcn_raw_buffer_store_b32(h.lo[r], d_lo, at + r * P.ldh * 2, 0, 0);
+                for (int b = 0; b < NB; b++) {
+                    unsigned hi, lo;
+                    vt_pair_words(h[2 * b], h[2 * b + 1], hi, lo);
+                    __builtin_amdgcn_raw_buffer_store_b32(hi, d_hi, at + 32 * b, 0, 0);
+                    __builtin_amdgcn_raw_buffer_store_b32(lo, d_lo, at + 32 * b, 0, 0);
                 }
                 return;
             }
@@ -369,12 +382,13 @@ vt_gemm_wide_kernel(gw_list list, const uint16_t *Ahi, const uint16_t *Alo, int 
     };
     auto finish = [&](const gw_item &it) {
         const gw_part &P = list.part[it.part];
+        const int lane = vt_lane();       /* offsets are made here, not kept through the steps (16 of them were spilled) */
         f32x4 q[NB];
         if constexpr (KW == 1) {
 #pragma unroll
             for (int a = 0; a < MB; a++)
 #pragma unroll
-                for (int vq = 0; vq < 4; vq++) { quads(q, a, vq); emit(P, it, a, vq, q); }
+                for (int vq = 0; vq < 4; vq++) { quads(q, a, vq); emit(P, it, lane, a, vq, q); }
         } else {
             /* the two waves of a column block hold the sums over the even and the odd K steps: each parks the half
              * of its quads that the other one finishes */
@@ -400,7 +414,7 @@ vt_gemm_wide_kernel(gw_list list, const uint16_t *Ahi, const uint16_t *Alo, int 
                         const f32x4 o = *reinterpret_cast<const f32x4 *>(theirs + (((a * 2 + h) * NB + b) * 64 + lane) * 4), m = q[b];
                         q[b] = f32x4{__fadd_rn(m.x, o.x), __fadd_rn(m.y, o.y), __fadd_rn(m.z, o.z), __fadd_rn(m.w, o.w)};
                     }
-                    emit(P, it, a, kw == 0 ? h : 2 + h, q);
+                    emit(P, it, lane, a, kw == 0 ? h : 2 + h, q);
                 }
         }
     };

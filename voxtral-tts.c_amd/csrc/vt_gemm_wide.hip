@@ -15,20 +15,20 @@
  * The backbone's 192 columns divide 6144 and 3072 into 32 and 16 tiles, so that 1, 2, 4, .. row tiles fill the 256 CUs
  * where 256-column tiles come in multiples of 192 items: q|k|v / output / down at 700 rows 57.5 / 40.7 / 79.4 -> 51.1 / 37.2 /
  * 72.5 us, at 1000 75.0 / 53.3 / 104.9 -> 68.5 / 49.2 / 97.0, output / down at 1531 73.3 / 149.4 -> 67.1 / 140.6.
- * Measured against every tile and cut count at 65 .. 1531 rows of the backbone's products, the plan taken is 0.9 to 1.0 % behind the
- * fastest on average, at worst 9 to 12 % (q|k|v at 600 rows, whole 192-column tiles on 224 CUs instead of 240 cut ones; output at 256
- * rows), on two boxes; for the codec's at 110 row counts from 65 to 8024, 0.2 % and at worst 7 % (down at 1500 rows, 96 x 256 in 4 cuts
- * instead of 96 x 128 in 2), 0.5 and 8 % at half of them on a third box.  Constants fitted to every second of these are 0.3 % behind at the others; fitted to the nine that
- * decodes of 21, 212 and 1003 frames have, 0.6 % and 20 % (gate|up at 105 rows, 128 x 128 in 4 cuts 25 us, 96 x 128 in 2 21). */
+ * Measured against every tile and cut count at 37 row counts from 65 to 2048 of the backbone's products, the plan taken is 0.5 % behind the
+ * fastest on average, at worst 4.4 % (q|k|v at 128 rows, 96 x 256 in 5 cuts instead of 4); for the codec's at 108 of 65 to 8024
+ * rows, 0.6 % and at worst 8.1 % (output at 128 rows).  96 and 128 x 384, which draw less power per product, are taken from 400 rows on (gate|up) and from
+ * 690 (down): below, too few items are left for the CUs. */
 struct gw_format {
     int products;                         /* matrix instructions per pair of operands */
     float launch_us, item_us, planes;     /* planes: passes over a cut column's planes */
     float sums_us, stream_tbps;           /* the launch that adds them (0: whoever reads the result does); the weights' rate (0: no bound) */
-    float step_us[3][2];                  /* [128, 192, 256 columns][96, 128 rows]; 0: tile not used */
-    float pflops[3];                      /* [128, 192, 256 columns] */
+    float step_us[4][2];                  /* [128, 192, 256, 384 columns][96, 128 rows]; 0: tile not used */
+    float pflops[4];                      /* [128, 192, 256, 384 columns] */
 };
-static const gw_format gw_backbone = {2, 5.0f, 2.8f, 1.45f, 0.f, 0.f, {{1.28f, 0.f}, {1.97f, 2.96f}, {1.15f, 1.65f}}, {0.91f, 1.07f, 1.21f}};
-static const gw_format gw_codec = {3, 2.5f, 14.2f, 1.79f, 0.f, 0.f, {{1.53f, 2.78f}, {0.f, 0.f}, {1.68f, 2.37f}}, {0.795f, 0.f, 1.33f}};
+static int gw_width(int tn) { return tn == 384 ? 3 : tn / 64 - 2; }
+static const gw_format gw_backbone = {2, 1.82f, 3.10f, 1.87f, 0.f, 0.f, {{1.293f, 0.f}, {2.031f, 2.591f}, {1.052f, 1.394f}, {1.601f, 2.088f}}, {0.947f, 1.30f, 1.28f, 99.f}};
+static const gw_format gw_codec = {3, 1.03f, 4.56f, 2.33f, 0.f, 0.f, {{1.874f, 2.375f}, {0.f, 0.f}, {1.45f, 1.944f}, {0.f, 0.f}}, {99.f, 0.f, 1.76f, 0.f}};
 
 static float gw_rounds(int items, float item_us, float power_us) {
     const int full = items / g_vt.n_cu, rem = items % g_vt.n_cu;
@@ -36,7 +36,7 @@ static float gw_rounds(int items, float item_us, float power_us) {
 }
 
 static float gw_cost(const gw_format &f, int M, int N, int K, int mb, int tn, int n_main, int cuts, int swiglu) {
-    const int kw = tn < 256 ? 2 : 1, mt = (M + 32 * mb - 1) / (32 * mb), w = tn / 64 - 2;
+    const int kw = tn < 256 ? 2 : 1, mt = (M + 32 * mb - 1) / (32 * mb), w = gw_width(tn);
     const float t_step = f.step_us[w][mb - 3];
     const float tile_us = 2.f * f.products * (32 * mb) * tn * (float)K / (f.pflops[w] * 1e9f);
     const int rest = N / tn - n_main;
@@ -52,9 +52,8 @@ static vt_gemm_plan gw_plan(const gw_format &f, int M, int N, int K, int swiglu,
     vt_gemm_plan best = {0, 64, 0, 1};
     float best_cost = 0.f;
     for (int mb = 3; mb <= 4; mb++)
-        for (int tn = 128; tn <= 256; tn += 64) {
-            /* 192 columns: gates and ups come in blocks of 64, which a wave's 96 columns do not end with */
-            if (N % tn || f.step_us[tn / 64 - 2][mb - 3] == 0.f || (tn == 192 && swiglu)) continue;
+        for (int tn : {128, 192, 256, 384}) {
+            if (N % tn || f.step_us[gw_width(tn)][mb - 3] == 0.f) continue;
             const int mt = (M + 32 * mb - 1) / (32 * mb), nt = N / tn;
             /* whole tiles: as many as make full rounds over the CUs, or one round fewer, or all */
             const int full = mt * nt / g_vt.n_cu;
@@ -121,10 +120,10 @@ static void gw_run(const vt_gemm_plan &pl, gw_part whole, gw_part cut, const uin
     cut.splits = pl.cuts;
     if (whole.n_tiles) list.part[list.n_parts++] = whole;
     if (cut.n_tiles) list.part[list.n_parts++] = cut;
-    static void (*const launch[2][2][3])(const gw_list &, const uint16_t *, const uint16_t *, int, int) = {
-        {{gw_launch<3, 2, 2>, gw_launch<3, 2, 3>, gw_launch<3, 4, 2>}, {NULL, gw_launch<4, 2, 3>, gw_launch<4, 4, 2>}},
-        {{gw_launch<3, 2, 2, false>, gw_launch<3, 2, 3, false>, gw_launch<3, 4, 2, false>}, {NULL, gw_launch<4, 2, 3, false>, gw_launch<4, 4, 2, false>}}};
-    launch[pl.row_major][pl.mb - 3][pl.tn / 64 - 2](list, d_Ahi, d_Alo, M, K);
+    static void (*const launch[2][2][4])(const gw_list &, const uint16_t *, const uint16_t *, int, int) = {
+        {{gw_launch<3, 2, 2>, gw_launch<3, 2, 3>, gw_launch<3, 4, 2>, gw_launch<3, 4, 3>}, {NULL, gw_launch<4, 2, 3>, gw_launch<4, 4, 2>, gw_launch<4, 4, 3>}},
+        {{gw_launch<3, 2, 2, false>, gw_launch<3, 2, 3, false>, gw_launch<3, 4, 2, false>, NULL}, {NULL, gw_launch<4, 2, 3, false>, gw_launch<4, 4, 2, false>, NULL}}};
+    launch[pl.row_major][pl.mb - 3][gw_width(pl.tn)](list, d_Ahi, d_Alo, M, K);
 }
 
 /* Products on a caller's row-major weights: tiles (a lane's own row costs four times the lines per request, hence constants of
@@ -135,7 +134,7 @@ static void gw_run(const vt_gemm_plan &pl, gw_part whole, gw_part cut, const uin
  * 0.9 % behind the fastest of all tiles, strips and cuts on average, 3.2 % where bounds on M, N and K made it, and takes 0.882 of the time
  * of 128 x 128 tiles alone, 0.902; above 1.05 of it at 5 shapes, 84 (18 rows of 4608 x 1024 1.25; at most 1.83).  No part of it came near
  * the card's power limit (pflops). */
-static const gw_format gw_row_major = {2, 6.875f, 2.226f, 1.892f, 2.173f, 4.638f, {{1.446f, 0.f}, {1.968f, 2.054f}, {1.138f, 1.189f}}, {99.f, 99.f, 99.f}};
+static const gw_format gw_row_major = {2, 6.875f, 2.226f, 1.892f, 2.173f, 4.638f, {{1.446f, 0.f}, {1.968f, 2.054f}, {1.138f, 1.189f}, {0.f, 0.f}}, {99.f, 99.f, 99.f, 99.f}};
 
 /* Strips: a workgroup goes through its K steps three at a time, which takes longer by the group of 8 rows, and so do its sums; but no
  * less than its or the card's share of the weights' rate allows */
