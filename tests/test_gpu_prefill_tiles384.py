@@ -1,6 +1,5 @@
-"""Prefill products on tiles of 384 columns: 96 and 128 rows, whole columns (450, 515 rows), whole columns of gate|up beside K cuts of the
-others (697, 1050 rows, the latter in many cuts), the down projection in cuts only (697), q|k|v whole and in part cut with the boundary among
-the v columns (1450, 1600); the last rows of a tile each time.  Against the oracle."""
+"""Prefill products on tiles of 384 columns: 96 and 128 rows, gate|up whole (450, 515 rows) and whole beside K cuts (1050: 96 rows, 1600: 128),
+down in cuts (697), q|k|v whole (1450); the last rows of a tile each time.  Against the oracle."""
 import pytest
 
 from test_gpu_prefill_mfma import _prefill_case

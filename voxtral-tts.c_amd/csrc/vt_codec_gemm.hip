@@ -77,7 +77,7 @@ static void cg_rows(const gr_list &plan, int grid, const uint16_t *d_hi, const u
 
 template <int MB, int CW>
 static void cg_wide(const gw_list &list, const uint16_t *d_hi, const uint16_t *d_lo, int M, int K) {
-    constexpr int LDS = 2 * (4 / CW) * 2 * 32 * MB * GM_STAGE_ROW + 32 * MB * (int)sizeof(int);
+    constexpr int LDS = 2 * gw_shape<MB, CW, false>::STAGE + gw_shape<MB, CW, false>::TM * (int)sizeof(int);
     static int attr_set = 0;
     if (!attr_set) {
         if (vt_check(hipFuncSetAttribute((const void *)vt_gemm_wide_kernel<gm_f16x2, MB, CW, 2>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS), "product LDS size"))
@@ -90,7 +90,7 @@ static void cg_wide(const gw_list &list, const uint16_t *d_hi, const uint16_t *d
 
 void vt_launch_codec_gemm(float *d_C, const uint16_t *d_hi, const uint16_t *d_lo, const int *d_row_exp,
                           const uint16_t *d_Wf, const int *d_col_exp, int M, int N, int K, const vt_gemm_plan &pl) {
-    if (pl.mb == 0) {
+    if (pl.tm == 0) {
         const gr_list plan = {d_C, d_Wf, (size_t)M * N, N, N / GR_TN, pl.cuts, d_row_exp, d_col_exp};
         const int items = plan.n_tiles * pl.cuts, grid = items < g_vt.n_cu ? items : g_vt.n_cu;
         static void (*const launch[4])(const gr_list &, int, const uint16_t *, const uint16_t *, int, int) = {cg_rows<2>, cg_rows<4>, cg_rows<6>, cg_rows<8>};
@@ -98,12 +98,12 @@ void vt_launch_codec_gemm(float *d_C, const uint16_t *d_hi, const uint16_t *d_lo
         return;
     }
     gw_list list = {};
-    list.m_tiles = (M + 32 * pl.mb - 1) / (32 * pl.mb);
+    list.m_tiles = (M + pl.tm - 1) / pl.tm;
     gw_part whole = {d_C, d_Wf, 0, pl.col0, pl.col0 / pl.tn, 1, NULL, NULL, 0, d_row_exp, d_col_exp};
     gw_part cut = {d_C + (size_t)M * pl.col0, d_Wf + (size_t)pl.col0 * K * 2, (size_t)M * (N - pl.col0), N - pl.col0, (N - pl.col0) / pl.tn, pl.cuts, NULL, NULL, 0,
                    d_row_exp, d_col_exp + pl.col0};
     if (whole.n_tiles) list.part[list.n_parts++] = whole;
     if (cut.n_tiles) list.part[list.n_parts++] = cut;
     static void (*const launch[2][2])(const gw_list &, const uint16_t *, const uint16_t *, int, int) = {{cg_wide<3, 2>, cg_wide<3, 4>}, {cg_wide<4, 2>, cg_wide<4, 4>}};
-    launch[pl.mb - 3][pl.tn == 256](list, d_hi, d_lo, M, K);
+    launch[pl.tm == 128][pl.tn == 256](list, d_hi, d_lo, M, K);
 }

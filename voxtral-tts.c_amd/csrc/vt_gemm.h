@@ -18,10 +18,10 @@ void vt_launch_gemm_ex(float *d_C, int ldc, size_t plane_stride, const uint16_t 
                        const uint16_t *d_W, int M, int N, int K, int splits);
 /* How a product of the backbone is done on fragment-order weights (vt_launch_frag_layout): the columns below
  * col0 as whole tiles (one plane), the others with K in `cuts` cuts (that many partial planes, to be added in
- * order by whoever reads the result).  mb, tn: the tile, 32 mb rows x tn columns
- * (vt_gemm_wide.hip; mb 0: vt_gemm_rows.hip).  col0 is a multiple of 128. */
+ * order by whoever reads the result).  tm, tn: rows and columns of the tile
+ * (vt_gemm_wide.hip; tm 0: vt_gemm_rows.hip).  col0 is a multiple of 128. */
 #define VT_MAX_CUTS 8
-struct vt_gemm_plan { int mb, tn, col0, cuts, row_major; };      /* row_major: W as it is (vt_gemm_row_major_plan) */
+struct vt_gemm_plan { int tm, tn, col0, cuts, row_major; };      /* row_major: W as it is (vt_gemm_row_major_plan) */
 /* K % 64 == 0; N % 256 == 0, up to 64 rows N % 96 == 0 (swiglu: % 288); swiglu: for vt_launch_gemm_frag_swiglu */
 vt_gemm_plan vt_gemm_frag_plan(int M, int N, int K, int swiglu);
 /* The same on row-major weights W[N, K], N % 128 == 0, K % 64 == 0, in at most `most` cuts: d_y [M, N]; d_part: pl.cuts planes of

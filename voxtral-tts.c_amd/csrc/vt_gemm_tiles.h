@@ -9,6 +9,8 @@
 #include "vt_state.h"
 #include "vt_gemm.h"
 
+#include <type_traits>
+
 typedef __bf16 gm_bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 gm_f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
@@ -40,6 +42,7 @@ struct gm_f16x2 {
 
 template <int WP, int NB> struct gm_weights { u32x4 v[WP][NB][4]; };      /* one 64-wide K step: [plane][block of 32 columns][16-wide slice] */
 template <int MB> struct gm_frags { u32x4 hi[MB], lo[MB]; };      /* one 16-wide slice of MB blocks of 32 rows, both planes */
+template <int MB> struct gm_paired { u32x4 v[MB]; };      /* of MB groups of 16 rows, lanes 0..15 (of 32) their hi, 16..31 their lo plane */
 
 /* A request through a descriptor: one whose size is 0, and a byte offset beyond the size, load nothing (zeros) */
 __device__ __forceinline__ u32x4 gm_ldb(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
@@ -82,6 +85,15 @@ __device__ __forceinline__ void gm_multiply(f32x16 (&acc)[MB][NB], const gm_frag
 #pragma unroll
             for (int b = 0; b < NB; b++) acc[a][b] = T::mfma(f.hi[a], w.v[0][b][ks], acc[a][b]);
     }
+}
+
+/* the same for paired planes: the sums of both planes' products stand apart, 16 rows above 16 */
+template <class T, int MB, int NB>
+__device__ __forceinline__ void gm_multiply(f32x16 (&acc)[MB][NB], const gm_paired<MB> &f, const gm_weights<T::WP, NB> &w, int ks) {
+#pragma unroll
+    for (int a = 0; a < MB; a++)
+#pragma unroll
+        for (int b = 0; b < NB; b++) acc[a][b] = T::mfma(f.v[a], w.v[0][b][ks], acc[a][b]);
 }
 
 /* Results leave through a descriptor whose size is that of the rows that exist: a row past them is dropped by the range check, with
@@ -172,18 +184,27 @@ __device__ __forceinline__ gw_item gw_item_at(const gw_list &list, int part, int
     return it;
 }
 
+/* A tile's shape.  PAIR false: MB blocks of 32 rows.  PAIR true (WP 1): MB groups of 16, hi and lo plane of a group the 32 rows of one matrix
+ * instruction: row counts between, for twice the accumulator registers per row. */
+template <int MB, int CW, bool PAIR> struct gw_shape {
+    static constexpr int TM = (PAIR ? 16 : 32) * MB;
+    static constexpr int NP = (TM + 8 * CW - 1) / (8 * CW);                  /* staging passes over a plane, 8 * CW rows each */
+    static constexpr int PLANE = NP * 8 * CW * GM_STAGE_ROW, STAGE = 4 / CW * 2 * PLANE;
+};
+
 /* FRAG false: row-major weights (WP 1), a caller's own: the same operands, a lane's 16 bytes of each slice from its own row */
-template <class T, int MB, int CW, int NB, bool FRAG = true>
+template <class T, int MB, int CW, int NB, bool FRAG = true, bool PAIR = false>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
 vt_gemm_wide_kernel(gw_list list, const uint16_t *Ahi, const uint16_t *Alo, int M, int K) {
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-    constexpr int WP = T::WP, KW = 4 / CW, TM = 32 * MB, TN = 32 * NB * CW;
-    constexpr int NP = 4 * MB / CW;                        /* staging passes over a plane, 8 * CW rows each */
-    constexpr int AHEAD = MB * NB > 9 ? 1 : 2;             /* steps between the request of a step's planes and their store (registers) */
+    typedef gw_shape<MB, CW, PAIR> shape;
+    constexpr int WP = T::WP, KW = 4 / CW, TM = shape::TM, TN = 32 * NB * CW, NP = shape::NP;
+    constexpr int READS = PAIR ? MB : 2 * MB;              /* fragment reads of a slice */
+    constexpr int AHEAD = MB * NB > (PAIR ? 14 : 9) ? 1 : 2;       /* steps between the request of a step's planes and their store (registers) */
     /* The first requests of an item go out in front of the stores of the one before it, where registers for both are left (where
      * they were not, a launch's first loads were spilled one by one, each behind a wait: 5 us). */
-    constexpr bool EARLY = CW == 4 || MB == 3;
-    constexpr int PLANE = TM * GM_STAGE_ROW, GROUP = 2 * PLANE, STAGE = KW * GROUP;
+    constexpr bool EARLY = CW == 4 || MB == 3 || (PAIR && NB == 2);
+    constexpr int PLANE = shape::PLANE, GROUP = 2 * PLANE, STAGE = shape::STAGE;
     int *tile_exp = reinterpret_cast<int *>(lds + 2 * STAGE);      /* T::SCALED: the exponents of the tile's rows */
     const int lane = (int)threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int cw = wave % CW, kw = wave / CW;              /* column block of the tile; which of the KW K steps */
@@ -191,7 +212,7 @@ vt_gemm_wide_kernel(gw_list list, const uint16_t *Ahi, const uint16_t *Alo, int 
     const int lr = tg >> 3, lc = tg & 7;                   /* staging: row lr + 8 CW p, 16-byte chunk lc */
     const int a_voff = (lr * K + lc * 8) * 2, a_pass = 16 * CW * K, blk_bytes = 64 * K * WP;
     const int st_off = kw * GROUP + lr * GM_STAGE_ROW + lc * 16;
-    const int fa_off = kw * GROUP + (lane & 31) * GM_STAGE_ROW + (lane >> 5) * 64;
+    const int fa_off = kw * GROUP + (PAIR ? (lane & 15) * GM_STAGE_ROW + (lane >> 4 & 1) * PLANE : (lane & 31) * GM_STAGE_ROW) + (lane >> 5) * 64;
 
     const int w_voff = FRAG ? lane * 16 : (lane & 31) * K * 2 + (lane >> 5) * 64;
 
@@ -219,13 +240,17 @@ vt_gemm_wide_kernel(gw_list list, const uint16_t *Ahi, const uint16_t *Alo, int 
 #pragma unroll
         for (int p = 0; p < NP; p++) *reinterpret_cast<u32x4 *>(lds + at + st_off + 8 * CW * p * GM_STAGE_ROW) = r[p];
     };
-    typedef gm_frags<MB> frags;
+    typedef typename std::conditional<PAIR, gm_paired<MB>, gm_frags<MB>>::type frags;
     auto read_frags = [&](frags &f, int stage, int ks) {
         const unsigned char *base = lds + stage * STAGE + fa_off + ks * 16;
 #pragma unroll
         for (int a = 0; a < MB; a++) {
-            f.hi[a] = *reinterpret_cast<const u32x4 *>(base + 32 * a * GM_STAGE_ROW);
-            f.lo[a] = *reinterpret_cast<const u32x4 *>(base + PLANE + 32 * a * GM_STAGE_ROW);
+            if constexpr (PAIR) {
+                f.v[a] = *reinterpret_cast<const u32x4 *>(base + 16 * a * GM_STAGE_ROW);
+            } else {
+                f.hi[a] = *reinterpret_cast<const u32x4 *>(base + 32 * a * GM_STAGE_ROW);
+                f.lo[a] = *reinterpret_cast<const u32x4 *>(base + PLANE + 32 * a * GM_STAGE_ROW);
+            }
         }
     };
     f32x16 acc[MB][NB];
@@ -233,7 +258,7 @@ vt_gemm_wide_kernel(gw_list list, const uint16_t *Ahi, const uint16_t *Alo, int 
 
     /* One step: stage `stage` holds the planes of step i and `cur` its weights; ra holds the planes of step
      * i + 1 (requested two steps ago: with one step between request and store, the step takes as long as a load,
-     * 1.2 us, whatever the tile); f0 already holds the fragments of slice 0.  Four regions of 4 MB (6 MB with
+     * 1.2 us, whatever the tile); f0 already holds the fragments of slice 0.  Four regions of 2 MB NB (PAIR: MB NB; 3 MB NB with
      * two weight planes) matrix instructions each; the other instructions of a region (the fragment reads of the next slice, in the first
      * two also the LDS stores of a plane of step i + 1 and its requests of step i + 3, in all but the first the
      * weight requests that refill the slice just used) are dealt out between the matrix instructions, one
@@ -257,7 +282,7 @@ vt_gemm_wide_kernel(gw_list list, const uint16_t *Ahi, const uint16_t *Alo, int 
         read_frags(f1, stage, 1);
         mma(f0, cur, 0);
 #pragma unroll
-        for (int k = 0; k < 2 * MB; k++) { GW_MFMA(); GW_DSR1(); if (k < NP) { GW_DSW1(); GW_VMR1(); } }
+        for (int k = 0; k < READS; k++) { GW_MFMA(); GW_DSR1(); if (k < NP) { GW_DSW1(); GW_VMR1(); } }
         GW_FENCE();
         store_a(ra.lo, other + PLANE);
         fetch_a(it, Alo, ra.lo, i + 1 + AHEAD);
@@ -265,13 +290,13 @@ vt_gemm_wide_kernel(gw_list list, const uint16_t *Ahi, const uint16_t *Alo, int 
         read_frags(f0, stage, 2);
         mma(f1, cur, 1);
 #pragma unroll
-        for (int k = 0; k < 2 * MB; k++) { GW_MFMA(); GW_DSR1(); if (k < NP) { GW_DSW1(); GW_VMR1(); } if (k < NB * WP) GW_VMR1(); }
+        for (int k = 0; k < READS; k++) { GW_MFMA(); GW_DSR1(); if (k < NP) { GW_DSW1(); GW_VMR1(); } if (k < NB * WP) GW_VMR1(); }
         GW_FENCE();
         fetch_b_slice(it, cur, i + 2, 1);
         read_frags(f1, stage, 3);
         mma(f0, cur, 2);
 #pragma unroll
-        for (int k = 0; k < 2 * MB; k++) { GW_MFMA(); GW_DSR1(); if (k < NB * WP) GW_VMR1(); }
+        for (int k = 0; k < READS; k++) { GW_MFMA(); GW_DSR1(); if (k < NB * WP) GW_VMR1(); }
         GW_FENCE();
         __syncthreads();
         GW_FENCE();
@@ -279,7 +304,7 @@ vt_gemm_wide_kernel(gw_list list, const uint16_t *Ahi, const uint16_t *Alo, int 
         read_frags(f0, stage ^ 1, 0);
         mma(f1, cur, 3);
 #pragma unroll
-        for (int k = 0; k < 2 * MB; k++) { GW_MFMA(); GW_DSR1(); if (k < NB * WP) GW_VMR1(); }
+        for (int k = 0; k < READS; k++) { GW_MFMA(); GW_DSR1(); if (k < NB * WP) GW_VMR1(); }
         GW_FENCE();
         fetch_b_slice(it, cur, i + 2, 3);
     };
@@ -344,7 +369,7 @@ vt_gemm_wide_kernel(gw_list list, const uint16_t *Ahi, const uint16_t *Alo, int 
 
     /* accumulator element v of lane l: row 8*(v/4) + 4*(l/32) + v%4, column l%32; quads (a, vq) hold v = 4 vq .. + 3 */
     auto emit = [&](const gw_part &P, const gw_item &it, int lane, int a, int vq, const f32x4 (&q)[NB]) {
-        const int quad_row = 32 * a + 8 * vq, rows = min(M - it.mt * TM, TM), c = lane & 31;      /* of the tile; a lane's first one is 4 (l / 32) on */
+        const int quad_row = (PAIR ? 16 : 32) * a + 8 * vq, rows = min(M - it.mt * TM, TM), c = lane & 31;      /* of the tile; a lane's first one is 4 (l / 32) on */
         if constexpr (!T::SCALED) {
             if (P.h_hi) {
                 /* a column block holds the gates and the ups of 16 h columns (voxtral_tts_llm.c:346-350) */
@@ -376,9 +401,16 @@ vt_gemm_wide_kernel(gw_list list, const uint16_t *Ahi, const uint16_t *Alo, int 
         if constexpr (T::SCALED) er = *reinterpret_cast<const i32x4 *>(tile_exp + quad_row + 4 * (lane >> 5));
         gm_store_quad<T, NB>(d, at, P.ldc * 4, q, er, ec);
     };
+    constexpr int QUADS = PAIR ? 2 : 4, HALF = QUADS / 2;        /* quads per a; PAIR: elements 8 + v are row v's sums over the lo plane */
     auto quads = [&](f32x4 (&q)[NB], int a, int vq) {
 #pragma unroll
-        for (int b = 0; b < NB; b++) q[b] = f32x4{acc[a][b][4 * vq], acc[a][b][4 * vq + 1], acc[a][b][4 * vq + 2], acc[a][b][4 * vq + 3]};
+        for (int b = 0; b < NB; b++) {
+            q[b] = f32x4{acc[a][b][4 * vq], acc[a][b][4 * vq + 1], acc[a][b][4 * vq + 2], acc[a][b][4 * vq + 3]};
+            if constexpr (PAIR) {
+#pragma unroll
+                for (int v = 0; v < 4; v++) q[b][v] = __fadd_rn(q[b][v], acc[a][b][8 + 4 * vq + v]);
+            }
+        }
     };
     auto finish = [&](const gw_item &it) {
         const gw_part &P = list.part[it.part];
@@ -388,33 +420,33 @@ vt_gemm_wide_kernel(gw_list list, const uint16_t *Ahi, const uint16_t *Alo, int 
 #pragma unroll
             for (int a = 0; a < MB; a++)
 #pragma unroll
-                for (int vq = 0; vq < 4; vq++) { quads(q, a, vq); emit(P, it, lane, a, vq, q); }
+                for (int vq = 0; vq < QUADS; vq++) { quads(q, a, vq); emit(P, it, lane, a, vq, q); }
         } else {
             /* the two waves of a column block hold the sums over the even and the odd K steps: each parks the half
              * of its quads that the other one finishes */
-            float *park = reinterpret_cast<float *>(lds) + (size_t)wave * (MB * NB * 2 * 256);
-            const float *theirs = reinterpret_cast<const float *>(lds) + (size_t)(wave ^ CW) * (MB * NB * 2 * 256);
+            float *park = reinterpret_cast<float *>(lds) + (size_t)wave * (MB * NB * HALF * 256);
+            const float *theirs = reinterpret_cast<const float *>(lds) + (size_t)(wave ^ CW) * (MB * NB * HALF * 256);
             __syncthreads();
 #pragma unroll
             for (int a = 0; a < MB; a++)
 #pragma unroll
-                for (int h = 0; h < 2; h++) {
-                    if (kw == 0) quads(q, a, 2 + h); else quads(q, a, h);
+                for (int h = 0; h < HALF; h++) {
+                    if (kw == 0) quads(q, a, HALF + h); else quads(q, a, h);
 #pragma unroll
-                    for (int b = 0; b < NB; b++) *reinterpret_cast<f32x4 *>(park + (((a * 2 + h) * NB + b) * 64 + lane) * 4) = q[b];
+                    for (int b = 0; b < NB; b++) *reinterpret_cast<f32x4 *>(park + (((a * HALF + h) * NB + b) * 64 + lane) * 4) = q[b];
                 }
             __syncthreads();
 #pragma unroll
             for (int a = 0; a < MB; a++)
 #pragma unroll
-                for (int h = 0; h < 2; h++) {
-                    if (kw == 0) quads(q, a, h); else quads(q, a, 2 + h);
+                for (int h = 0; h < HALF; h++) {
+                    if (kw == 0) quads(q, a, h); else quads(q, a, HALF + h);
 #pragma unroll
                     for (int b = 0; b < NB; b++) {
-                        const f32x4 o = *reinterpret_cast<const f32x4 *>(theirs + (((a * 2 + h) * NB + b) * 64 + lane) * 4), m = q[b];
+                        const f32x4 o = *reinterpret_cast<const f32x4 *>(theirs + (((a * HALF + h) * NB + b) * 64 + lane) * 4), m = q[b];
                         q[b] = f32x4{__fadd_rn(m.x, o.x), __fadd_rn(m.y, o.y), __fadd_rn(m.z, o.z), __fadd_rn(m.w, o.w)};
                     }
-                    emit(P, it, lane, a, kw == 0 ? h : 2 + h, q);
+                    emit(P, it, lane, a, kw == 0 ? h : HALF + h, q);
                 }
         }
     };

@@ -15,34 +15,39 @@
  * The backbone's 192 columns divide 6144 and 3072 into 32 and 16 tiles, so that 1, 2, 4, .. row tiles fill the 256 CUs
  * where 256-column tiles come in multiples of 192 items: q|k|v / output / down at 700 rows 57.5 / 40.7 / 79.4 -> 51.1 / 37.2 /
  * 72.5 us, at 1000 75.0 / 53.3 / 104.9 -> 68.5 / 49.2 / 97.0, output / down at 1531 73.3 / 149.4 -> 67.1 / 140.6.
- * Measured against every tile and cut count at 37 row counts from 65 to 2048 of the backbone's products, the plan taken is 0.5 % behind the
- * fastest on average, at worst 4.4 % (q|k|v at 128 rows, 96 x 256 in 5 cuts instead of 4); for the codec's at 108 of 65 to 8024
- * rows, 0.6 % and at worst 8.1 % (output at 128 rows).  96 and 128 x 384, which draw less power per product, are taken from 400 rows on (gate|up) and from
- * 690 (down): below, too few items are left for the CUs. */
+ * Measured against every tile and cut count at 47 row counts from 65 to 2048 of the backbone's products, the plan taken is 0.3 % behind the
+ * fastest on average, at worst 5.5 % (q|k|v at 113 rows, 80 x 256 in 5 cuts instead of 4); for the codec's at 108 of 65 to 8024
+ * rows, 0.6 % and at worst 8.1 % (output at 128 rows).  Single products exchanged inside prefills of 150 to 1531 rows were at most 2.7 %
+ * of the prefill faster (gate|up at 700 rows, 96 x 384 in part cut).  Tiles x 384, which draw less power per product, are taken from 400 rows on
+ * (gate|up) and from 690 (down): below, too few items are left for the CUs.  80 and 112 rows, where those of 96 and 128 have many to pad: us of
+ * the four products at 200 / 226 / 290 / 400 / 800 rows 140 / 144 / 173 / 197 / 334 -> 130 / 136 / 163 / 186 / 322, a prefill of 226 rows 4274 -> 4020. */
 struct gw_format {
     int products;                         /* matrix instructions per pair of operands */
-    float launch_us, item_us, planes;     /* planes: passes over a cut column's planes */
+    float launch_us, planes;              /* planes: passes over a cut column's planes */
     float sums_us, stream_tbps;           /* the launch that adds them (0: whoever reads the result does); the weights' rate (0: no bound) */
-    float step_us[4][2];                  /* [128, 192, 256, 384 columns][96, 128 rows]; 0: tile not used */
+    float item_us[4];                     /* [128, 192, 256, 384 columns] */
+    float step_us[4][4];                  /* [128, 192, 256, 384 columns][80, 96, 112, 128 rows]; 0: tile not used */
     float pflops[4];                      /* [128, 192, 256, 384 columns] */
 };
 static int gw_width(int tn) { return tn == 384 ? 3 : tn / 64 - 2; }
-static const gw_format gw_backbone = {2, 1.82f, 3.10f, 1.87f, 0.f, 0.f, {{1.293f, 0.f}, {2.031f, 2.591f}, {1.052f, 1.394f}, {1.601f, 2.088f}}, {0.947f, 1.30f, 1.28f, 99.f}};
-static const gw_format gw_codec = {3, 1.03f, 4.56f, 2.33f, 0.f, 0.f, {{1.874f, 2.375f}, {0.f, 0.f}, {1.45f, 1.944f}, {0.f, 0.f}}, {99.f, 0.f, 1.76f, 0.f}};
+static int gw_height(int tm) { return tm / 16 - 5; }
+static const gw_format gw_backbone = {2, 0.f, 2.60f, 0.f, 0.f, {1.47f, 3.96f, 0.09f, 2.37f}, {{0.f, 1.397f, 0.f, 0.f}, {1.521f, 1.652f, 0.f, 1.967f}, {0.904f, 0.976f, 1.206f, 1.202f},
+    {1.302f, 1.398f, 0.f, 1.714f}}, {99.f, 1.381f, 1.496f, 99.f}};
+static const gw_format gw_codec = {3, 1.03f, 2.33f, 0.f, 0.f, {4.56f, 0.f, 4.56f, 0.f}, {{0.f, 1.874f, 0.f, 2.375f}, {}, {0.f, 1.45f, 0.f, 1.944f}, {}}, {99.f, 0.f, 1.76f, 0.f}};
 
 static float gw_rounds(int items, float item_us, float power_us) {
     const int full = items / g_vt.n_cu, rem = items % g_vt.n_cu;
     return full * fmaxf(item_us, g_vt.n_cu * power_us) + (rem ? fmaxf(item_us, rem * power_us) : 0.f);
 }
 
-static float gw_cost(const gw_format &f, int M, int N, int K, int mb, int tn, int n_main, int cuts, int swiglu) {
-    const int kw = tn < 256 ? 2 : 1, mt = (M + 32 * mb - 1) / (32 * mb), w = gw_width(tn);
-    const float t_step = f.step_us[w][mb - 3];
-    const float tile_us = 2.f * f.products * (32 * mb) * tn * (float)K / (f.pflops[w] * 1e9f);
+static float gw_cost(const gw_format &f, int M, int N, int K, int tm, int tn, int n_main, int cuts, int swiglu) {
+    const int kw = tn < 256 ? 2 : 1, mt = (M + tm - 1) / tm, w = gw_width(tn);
+    const float t_step = f.step_us[w][gw_height(tm)];
+    const float tile_us = 2.f * f.products * tm * tn * (float)K / (f.pflops[w] * 1e9f);
     const int rest = N / tn - n_main;
-    float t = f.launch_us + gw_rounds(mt * n_main, (float)((K / 64 + kw - 1) / kw) * t_step + f.item_us, tile_us);
+    float t = f.launch_us + gw_rounds(mt * n_main, (float)((K / 64 + kw - 1) / kw) * t_step + f.item_us[w], tile_us);
     if (rest) {
-        t += gw_rounds(mt * rest * cuts, (float)((K / 64 + cuts * kw - 1) / (cuts * kw)) * t_step + f.item_us, tile_us / cuts);
+        t += gw_rounds(mt * rest * cuts, (float)((K / 64 + cuts * kw - 1) / (cuts * kw)) * t_step + f.item_us[w], tile_us / cuts);
         if (cuts > 1 || swiglu) t += f.planes * cuts * M * (float)(rest * tn) * 4.f / 4.5e6f + (swiglu ? 4.5f : cuts > 1 ? f.sums_us : 0.f);
     }
     return f.stream_tbps > 0.f ? fmaxf(t, f.launch_us + N * 2.f * K / (f.stream_tbps * 1e6f)) : t;
@@ -51,10 +56,10 @@ static float gw_cost(const gw_format &f, int M, int N, int K, int mb, int tn, in
 static vt_gemm_plan gw_plan(const gw_format &f, int M, int N, int K, int swiglu, int most = VT_MAX_CUTS, float *us = NULL) {
     vt_gemm_plan best = {0, 64, 0, 1};
     float best_cost = 0.f;
-    for (int mb = 3; mb <= 4; mb++)
+    for (int tm = 80; tm <= 128; tm += 16)
         for (int tn : {128, 192, 256, 384}) {
-            if (N % tn || f.step_us[gw_width(tn)][mb - 3] == 0.f) continue;
-            const int mt = (M + 32 * mb - 1) / (32 * mb), nt = N / tn;
+            if (N % tn || f.step_us[gw_width(tn)][gw_height(tm)] == 0.f) continue;
+            const int mt = (M + tm - 1) / tm, nt = N / tn;
             /* whole tiles: as many as make full rounds over the CUs, or one round fewer, or all */
             const int full = mt * nt / g_vt.n_cu;
             for (int pick = 0; pick < 3; pick++) {
@@ -64,10 +69,10 @@ static vt_gemm_plan gw_plan(const gw_format &f, int M, int N, int K, int swiglu,
                 for (int cuts = 1; cuts <= most && cuts <= K / 64; cuts++) {
                     if (n_main == nt && cuts > 1) break;
                     if (swiglu && n_main < nt && cuts == 1) continue;
-                    const float c = gw_cost(f, M, N, K, mb, tn, n_main, cuts, swiglu);
+                    const float c = gw_cost(f, M, N, K, tm, tn, n_main, cuts, swiglu);
                     if (best_cost == 0.f || c < best_cost) {
                         best_cost = c;
-                        best = vt_gemm_plan{mb, tn, n_main * tn, n_main == nt ? 1 : cuts};
+                        best = vt_gemm_plan{tm, tn, n_main * tn, n_main == nt ? 1 : cuts};
                     }
                 }
             }
@@ -85,14 +90,12 @@ vt_gemm_plan vt_codec_gemm_plan(int M, int N, int K) {
     return gw_plan(gw_codec, M, N, K, 0);
 }
 
-template <int MB, int CW>
-struct gw_lds { static constexpr int bytes = 2 * (4 / CW) * 2 * 32 * MB * GM_STAGE_ROW; };
-
-template <int MB, int CW, int NB, bool FRAG = true>
+template <int MB, int CW, int NB, bool FRAG = true, bool PAIR = false>
 static int gw_prepare(void) {
     static int attr_device = -1;
     if (attr_device == g_vt.device) return 0;
-    if (vt_check(hipFuncSetAttribute((const void *)vt_gemm_wide_kernel<gm_bf16, MB, CW, NB, FRAG>, hipFuncAttributeMaxDynamicSharedMemorySize, gw_lds<MB, CW>::bytes), "product LDS size"))
+    if (vt_check(hipFuncSetAttribute((const void *)vt_gemm_wide_kernel<gm_bf16, MB, CW, NB, FRAG, PAIR>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                     2 * gw_shape<MB, CW, PAIR>::STAGE), "product LDS size"))
         return -1;
     attr_device = g_vt.device;
     return 0;
@@ -103,27 +106,31 @@ int vt_gemm_row_major_prepare(void) {
     return gw_prepare<3, 2, 2, false>() || gw_prepare<3, 2, 3, false>() || gw_prepare<3, 4, 2, false>() || gw_prepare<4, 2, 3, false>() || gw_prepare<4, 4, 2, false>() ? -1 : 0;
 }
 
-template <int MB, int CW, int NB, bool FRAG = true>
+template <int MB, int CW, int NB, bool FRAG = true, bool PAIR = false>
 static void gw_launch(const gw_list &list, const uint16_t *d_Ahi, const uint16_t *d_Alo, int M, int K) {
-    constexpr int LDS = gw_lds<MB, CW>::bytes;
-    if (gw_prepare<MB, CW, NB, FRAG>()) return;
+    constexpr int LDS = 2 * gw_shape<MB, CW, PAIR>::STAGE;
+    if (gw_prepare<MB, CW, NB, FRAG, PAIR>()) return;
     const int items = list.m_tiles * list.part[0].n_tiles * list.part[0].splits;      /* every workgroup takes an item of the first part */
-    hipLaunchKernelGGL((vt_gemm_wide_kernel<gm_bf16, MB, CW, NB, FRAG>), dim3(items < g_vt.n_cu ? items : g_vt.n_cu), dim3(256), LDS, g_vt.stream, list, d_Ahi, d_Alo, M, K);
+    hipLaunchKernelGGL((vt_gemm_wide_kernel<gm_bf16, MB, CW, NB, FRAG, PAIR>), dim3(items < g_vt.n_cu ? items : g_vt.n_cu), dim3(256), LDS, g_vt.stream,
+                       list, d_Ahi, d_Alo, M, K);
 }
 
 static void gw_run(const vt_gemm_plan &pl, gw_part whole, gw_part cut, const uint16_t *d_Ahi, const uint16_t *d_Alo, int M, int N, int K) {
     gw_list list = {};
-    list.m_tiles = (M + 32 * pl.mb - 1) / (32 * pl.mb);
+    list.m_tiles = (M + pl.tm - 1) / pl.tm;
     whole.n_tiles = pl.col0 / pl.tn;
     whole.splits = 1;
     cut.n_tiles = (N - pl.col0) / pl.tn;
     cut.splits = pl.cuts;
     if (whole.n_tiles) list.part[list.n_parts++] = whole;
     if (cut.n_tiles) list.part[list.n_parts++] = cut;
-    static void (*const launch[2][2][4])(const gw_list &, const uint16_t *, const uint16_t *, int, int) = {
-        {{gw_launch<3, 2, 2>, gw_launch<3, 2, 3>, gw_launch<3, 4, 2>, gw_launch<3, 4, 3>}, {NULL, gw_launch<4, 2, 3>, gw_launch<4, 4, 2>, gw_launch<4, 4, 3>}},
-        {{gw_launch<3, 2, 2, false>, gw_launch<3, 2, 3, false>, gw_launch<3, 4, 2, false>, NULL}, {NULL, gw_launch<4, 2, 3, false>, gw_launch<4, 4, 2, false>, NULL}}};
-    launch[pl.row_major][pl.mb - 3][gw_width(pl.tn)](list, d_Ahi, d_Alo, M, K);
+    typedef void (*fn)(const gw_list &, const uint16_t *, const uint16_t *, int, int);
+    static const fn launch[4][4] = {{NULL, gw_launch<5, 2, 3, true, true>, gw_launch<5, 4, 2, true, true>, gw_launch<5, 4, 3, true, true>},
+                                    {gw_launch<3, 2, 2>, gw_launch<3, 2, 3>, gw_launch<3, 4, 2>, gw_launch<3, 4, 3>},
+                                    {NULL, NULL, gw_launch<7, 4, 2, true, true>, NULL},
+                                    {NULL, gw_launch<4, 2, 3>, gw_launch<4, 4, 2>, gw_launch<4, 4, 3>}};
+    static const fn row_major[2][3] = {{gw_launch<3, 2, 2, false>, gw_launch<3, 2, 3, false>, gw_launch<3, 4, 2, false>}, {NULL, gw_launch<4, 2, 3, false>, gw_launch<4, 4, 2, false>}};
+    (pl.row_major ? row_major[pl.tm == 128][gw_width(pl.tn)] : launch[gw_height(pl.tm)][gw_width(pl.tn)])(list, d_Ahi, d_Alo, M, K);
 }
 
 /* Products on a caller's row-major weights: tiles (a lane's own row costs four times the lines per request, hence constants of
@@ -134,7 +141,7 @@ static void gw_run(const vt_gemm_plan &pl, gw_part whole, gw_part cut, const uin
  * 0.9 % behind the fastest of all tiles, strips and cuts on average, 3.2 % where bounds on M, N and K made it, and takes 0.882 of the time
  * of 128 x 128 tiles alone, 0.902; above 1.05 of it at 5 shapes, 84 (18 rows of 4608 x 1024 1.25; at most 1.83).  No part of it came near
  * the card's power limit (pflops). */
-static const gw_format gw_row_major = {2, 6.875f, 2.226f, 1.892f, 2.173f, 4.638f, {{1.446f, 0.f}, {1.968f, 2.054f}, {1.138f, 1.189f}, {0.f, 0.f}}, {99.f, 99.f, 99.f, 99.f}};
+static const gw_format gw_row_major = {2, 6.875f, 1.892f, 2.173f, 4.638f, {2.226f, 2.226f, 2.226f, 0.f}, {{0.f, 1.446f, 0.f, 0.f}, {0.f, 1.968f, 0.f, 2.054f}, {0.f, 1.138f, 0.f, 1.189f}, {}}, {99.f, 99.f, 99.f, 99.f}};
 
 /* Strips: a workgroup goes through its K steps three at a time, which takes longer by the group of 8 rows, and so do its sums; but no
  * less than its or the card's share of the weights' rate allows */
@@ -188,7 +195,7 @@ void vt_launch_gemm_row_major(float *d_y, float *d_part, const uint16_t *d_Ahi, 
                               const vt_gemm_plan &pl) {
     const int cut = N - pl.col0;
     const size_t plane = (size_t)M * cut;
-    if (pl.mb == 0) vt_launch_gemm_few_rows(pl.cuts > 1 ? d_part : d_y, N, plane, d_Ahi, d_Alo, d_W, M, N, K, pl);
+    if (pl.tm == 0) vt_launch_gemm_few_rows(pl.cuts > 1 ? d_part : d_y, N, plane, d_Ahi, d_Alo, d_W, M, N, K, pl);
     else gw_run(pl, gw_part{d_y, d_W, 0, N, 0, 0, NULL, NULL, 0, NULL, NULL},
                 gw_part{d_part, d_W + (size_t)pl.col0 * K, plane, cut, 0, 0, NULL, NULL, 0, NULL, NULL}, d_Ahi, d_Alo, M, N, K);
     if (pl.cuts > 1) {
@@ -199,7 +206,7 @@ void vt_launch_gemm_row_major(float *d_y, float *d_part, const uint16_t *d_Ahi, 
 
 void vt_launch_gemm_frag(float *d_C, int ldc, size_t plane_stride, const uint16_t *d_Ahi, const uint16_t *d_Alo,
                          const uint16_t *d_Wf, int M, int N, int K, const vt_gemm_plan &pl) {
-    if (pl.mb == 0) { vt_launch_gemm_few_rows(d_C, ldc, plane_stride, d_Ahi, d_Alo, d_Wf, M, N, K, pl); return; }
+    if (pl.tm == 0) { vt_launch_gemm_few_rows(d_C, ldc, plane_stride, d_Ahi, d_Alo, d_Wf, M, N, K, pl); return; }
     gw_run(pl, gw_part{d_C, d_Wf, plane_stride, ldc, 0, 0, NULL, NULL, 0, NULL, NULL},
            gw_part{d_C + pl.col0, d_Wf + (size_t)pl.col0 * K, plane_stride, ldc, 0, 0, NULL, NULL, 0, NULL, NULL}, d_Ahi, d_Alo, M, N, K);
 }
@@ -207,7 +214,7 @@ void vt_launch_gemm_frag(float *d_C, int ldc, size_t plane_stride, const uint16_
 void vt_launch_gemm_frag_swiglu(uint16_t *d_hhi, uint16_t *d_hlo, int ldh, float *d_tail, const uint16_t *d_Ahi,
                                 const uint16_t *d_Alo, const uint16_t *d_Wf, int M, int N, int K, const vt_gemm_plan &pl) {
     const int tail = N - pl.col0;
-    if (pl.mb == 0)
+    if (pl.tm == 0)
         vt_launch_gemm_few_rows(d_tail, N, (size_t)M * N, d_Ahi, d_Alo, d_Wf, M, N, K, pl);
     else
         gw_run(pl, gw_part{NULL, d_Wf, 0, 0, 0, 0, d_hhi, d_hlo, ldh, NULL, NULL},
