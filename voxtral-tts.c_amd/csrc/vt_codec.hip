@@ -49,17 +49,15 @@
 
 /* ---- row kernels ------------------------------------------------------------------------- */
 
-/* block-wide sum and maximum over 256 threads (4 waves), the same value in every thread */
+/* block-wide sum and maximum over 256 threads (4 waves), the same value in every thread; red: 4 floats for this one reduction */
 __device__ __forceinline__ float cd_block_sum(float v, float *red) {
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-    __syncthreads();
+    v = vt_wave_sum(v);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
     __syncthreads();
     return (red[0] + red[1]) + (red[2] + red[3]);
 }
 __device__ __forceinline__ float cd_block_max(float v, float *red) {
-    for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o));
-    __syncthreads();
+    v = vt_wave_max(v);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
     __syncthreads();
     return fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
@@ -106,7 +104,7 @@ template <int C, bool UP>
 __global__ void __launch_bounds__(256)
 vt_codec_row_kernel(float *x_out, cd_planes xn, const float *x_in, cd_product in, const float *__restrict__ bias,
                     const float *__restrict__ scale, const float *__restrict__ norm_w, float eps) {
-    __shared__ float red[4];
+    __shared__ float red[2][4];
     const int row = blockIdx.x, c = threadIdx.x * 4;
     const size_t at = (size_t)row * CD_DIM + c;
     f32x4 r = {0.f, 0.f, 0.f, 0.f};
@@ -124,11 +122,11 @@ vt_codec_row_kernel(float *x_out, cd_planes xn, const float *x_in, cd_product in
     v += r;
     if (norm_w) {
         *(f32x4 *)(x_out + at) = v;
-        const float ss = cd_block_sum(v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w, red);
+        const float ss = cd_block_sum(v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w, red[0]);
         const float inv = 1.0f / sqrtf(ss / (float)CD_DIM + eps);
         v = v * inv * *(const f32x4 *)(norm_w + c);
     }
-    const int e = vt_f16_exp(cd_block_max(cd_max4(v), red));
+    const int e = vt_f16_exp(cd_block_max(cd_max4(v), red[1]));
     cd_put4(xn, at, v, e);
     if (threadIdx.x == 0) xn.exp[row] = e;
 }
@@ -138,7 +136,7 @@ vt_codec_row_kernel(float *x_out, cd_planes xn, const float *x_in, cd_product in
 template <int C>
 __global__ void __launch_bounds__(256)
 vt_codec_qkv_kernel(float *__restrict__ qkv, cd_product in, const float *__restrict__ q_norm, const float *__restrict__ k_norm) {
-    __shared__ float red[4];
+    __shared__ float red[2][4];
     const int row = blockIdx.x, c = threadIdx.x * 4;
     const size_t at = (size_t)row * (3 * CD_DIM) + c;
     f32x4 v[3];
@@ -148,7 +146,7 @@ vt_codec_qkv_kernel(float *__restrict__ qkv, cd_product in, const float *__restr
     for (int part = 0; part < 3; part++) {
         const float *nw = part == 0 ? q_norm : part == 1 ? k_norm : nullptr;
         if (nw) {
-            const float ss = cd_block_sum(v[part].x * v[part].x + v[part].y * v[part].y + v[part].z * v[part].z + v[part].w * v[part].w, red);
+            const float ss = cd_block_sum(v[part].x * v[part].x + v[part].y * v[part].y + v[part].z * v[part].z + v[part].w * v[part].w, red[part]);
             const float inv = 1.0f / sqrtf(ss / (float)CD_DIM + CD_QK_EPS);
             v[part] = v[part] * inv * *(const f32x4 *)(nw + c);
         }
@@ -305,26 +303,27 @@ vt_codec_attention_split_kernel(cd_planes out, const float *__restrict__ qkv, in
         const cd_head_row k = cd_load_row(kr), v = cd_load_row(kr + CD_DIM);
         s.add(cd_row_dot(q, k) * scale + slope * (float)(j - i), v);
     }
-    float mx = s.mx;
-    for (int o = 8; o < 64; o <<= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+    auto ror8 = [](float v) { return vt_dpp<0x128>(v); };        /* the lane 8 away in its row of 16 */
+    const float mx = vt_rows_max(fmaxf(s.mx, ror8(s.mx)));
     const float f = s.mx == mx ? 1.0f : expf(s.mx - mx);
-    float se = s.se * f;
-    for (int o = 8; o < 64; o <<= 1) se += __shfl_xor(se, o);
+    const float sf = s.se * f, se = vt_rows_sum(sf + ror8(sf));
     const bool b3 = lane & 8, b4 = lane & 16, b5 = lane & 32;
     f32x4 r2[2], r1;
 #pragma unroll
     for (int e = 0; e < 2; e++) {
         const f32x4 keep = (b3 ? s.o.v[2 + e] : s.o.v[e]) * f, give = (b3 ? s.o.v[e] : s.o.v[2 + e]) * f;
 #pragma unroll
-        for (int n = 0; n < 4; n++) r2[e][n] = keep[n] + __shfl_xor(give[n], 8);
+        for (int n = 0; n < 4; n++) r2[e][n] = keep[n] + ror8(give[n]);
     }
 #pragma unroll
-    for (int n = 0; n < 4; n++) r1[n] = (b4 ? r2[1][n] : r2[0][n]) + __shfl_xor(b4 ? r2[0][n] : r2[1][n], 16);
+    for (int n = 0; n < 4; n++) {
+        const f32x2 r = vt_swap16(r2[0][n], r2[1][n]);
+        r1[n] = r.x + r.y;
+    }
     const float inv = se > 0.f ? 1.0f / se : 1.0f;
-    const float x = ((b5 ? r1[2] : r1[0]) + __shfl_xor(b5 ? r1[0] : r1[2], 32)) * inv;
-    const float y = ((b5 ? r1[3] : r1[1]) + __shfl_xor(b5 ? r1[1] : r1[3], 32)) * inv;
-    float m = fmaxf(fabsf(x), fabsf(y));
-    for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
+    const f32x2 rx = vt_swap32(r1[0], r1[2]), ry = vt_swap32(r1[1], r1[3]);
+    const float x = (rx.x + rx.y) * inv, y = (ry.x + ry.y) * inv;
+    float m = vt_wave_max(fmaxf(fabsf(x), fabsf(y)));
     if (lane == 0) red[h] = m;
     __syncthreads();
 #pragma unroll

@@ -84,26 +84,25 @@ static void cg_wide(const gw_list &list, const uint16_t *d_hi, const uint16_t *d
             return;
         attr_set = 1;
     }
-    const int items = list.m_tiles * list.part[0].n_tiles * list.part[0].splits;
+    const int items = list.part[0].items;
     hipLaunchKernelGGL((vt_gemm_wide_kernel<gm_f16x2, MB, CW, 2>), dim3(items < g_vt.n_cu ? items : g_vt.n_cu), dim3(256), LDS, g_vt.stream, list, d_hi, d_lo, M, K);
 }
 
 void vt_launch_codec_gemm(float *d_C, const uint16_t *d_hi, const uint16_t *d_lo, const int *d_row_exp,
                           const uint16_t *d_Wf, const int *d_col_exp, int M, int N, int K, const vt_gemm_plan &pl) {
     if (pl.tm == 0) {
-        const gr_list plan = {d_C, d_Wf, (size_t)M * N, N, N / GR_TN, pl.cuts, d_row_exp, d_col_exp};
-        const int items = plan.n_tiles * pl.cuts, grid = items < g_vt.n_cu ? items : g_vt.n_cu;
+        const int items = N / GR_TN * pl.cuts, grid = items < g_vt.n_cu ? items : g_vt.n_cu;
+        const gr_list plan = {d_C, d_Wf, (size_t)M * N, N, items, vt_divisor_of(N / GR_TN, items), gm_cuts_of(K, pl.cuts), d_row_exp, d_col_exp};
         static void (*const launch[4])(const gr_list &, int, const uint16_t *, const uint16_t *, int, int) = {cg_rows<2>, cg_rows<4>, cg_rows<6>, cg_rows<8>};
         launch[(M + 15) / 16 - 1](plan, grid, d_hi, d_lo, M, K);
         return;
     }
     gw_list list = {};
-    list.m_tiles = (M + pl.tm - 1) / pl.tm;
     gw_part whole = {d_C, d_Wf, 0, pl.col0, pl.col0 / pl.tn, 1, NULL, NULL, 0, d_row_exp, d_col_exp};
     gw_part cut = {d_C + (size_t)M * pl.col0, d_Wf + (size_t)pl.col0 * K * 2, (size_t)M * (N - pl.col0), N - pl.col0, (N - pl.col0) / pl.tn, pl.cuts, NULL, NULL, 0,
                    d_row_exp, d_col_exp + pl.col0};
-    if (whole.n_tiles) list.part[list.n_parts++] = whole;
-    if (cut.n_tiles) list.part[list.n_parts++] = cut;
+    gw_add(list, whole, M, pl.tm, K);
+    gw_add(list, cut, M, pl.tm, K);
     static void (*const launch[2][2])(const gw_list &, const uint16_t *, const uint16_t *, int, int) = {{cg_wide<3, 2>, cg_wide<3, 4>}, {cg_wide<4, 2>, cg_wide<4, 4>}};
     launch[pl.tm == 128][pl.tn == 256](list, d_hi, d_lo, M, K);
 }

@@ -78,6 +78,32 @@ __device__ __forceinline__ float vt_wave_sum(float v) {
     return a + b;
 }
 
+/* Reductions over the lanes 16 and 32 apart, in registers (a __shfl_xor is a trip through the LDS' crossbar of about 50 ns).  vt_swap16:
+ * x and y with the odd rows of 16 lanes of x and the even ones of y exchanged, so that x + y are x's pair sums in the even rows and y's
+ * in the odd ones; vt_swap32 the same for halves of the wave. */
+__device__ __forceinline__ f32x2 vt_swap16(float x, float y) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+    return f32x2{__uint_as_float(r[0]), __uint_as_float(r[1])};
+}
+__device__ __forceinline__ f32x2 vt_swap32(float x, float y) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+    return f32x2{__uint_as_float(r[0]), __uint_as_float(r[1])};
+}
+/* max and sum over the lanes with the same lane % 16 */
+__device__ __forceinline__ float vt_rows_max(float v) {
+    f32x2 r = vt_swap16(v, v);
+    v = fmaxf(r.x, r.y);
+    r = vt_swap32(v, v);
+    return fmaxf(r.x, r.y);
+}
+__device__ __forceinline__ float vt_rows_sum(float v) {
+    f32x2 r = vt_swap16(v, v);
+    v = r.x + r.y;
+    r = vt_swap32(v, v);
+    return r.x + r.y;
+}
+__device__ __forceinline__ float vt_wave_max(float v) { return vt_rows_max(vt_row16_max(v)); }
+
 /* Full wave64 sum that ends in lane 63 only (other lanes hold partial sums):
  * 4 steps inside each row of 16, then row_bcast:15 into rows 1 and 3 and
  * row_bcast:31 into rows 2 and 3.  No scalar round trip. */

@@ -43,7 +43,7 @@ template <int N> struct gs_int { static constexpr int v = N; };
 template <int NP, int KW, bool FRAG>
 __global__ void __launch_bounds__(64 * GS_WAVES)
 vt_gemm_strip_kernel(float *C, int ldc, size_t plane_stride, const uint16_t *Ahi, const uint16_t *Alo, const uint16_t *Wf, int M, int N, int K,
-                     int strips, int cuts) {
+                     vt_divisor strips, gm_cuts cuts) {
     constexpr int MG = (NP + 1) / 2, CB = GS_WAVES / KW, STEP = MG * 4096, BUF = GS_CHUNK * STEP;
     constexpr int SPW = GS_CHUNK / KW, D = 3;                                /* a wave's steps per chunk; steps ahead */
     constexpr int ND = (2 * GS_CHUNK * NP + GS_WAVES - 1) / GS_WAVES;        /* requests of rows per wave and chunk */
@@ -51,10 +51,9 @@ vt_gemm_strip_kernel(float *C, int ldc, size_t plane_stride, const uint16_t *Ahi
     const int lane = (int)threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int cb = wave / KW, kw = wave % KW;
     /* slot id lands on XCD id % 8: an XCD takes a run of items, strip fastest, i.e. few cuts, whose rows its L2 then holds */
-    const int id = (int)blockIdx.x, items = strips * cuts, li = (items & 7) == 0 ? (id & 7) * (items >> 3) + (id >> 3) : id;
-    const int strip = li % strips, cut = li / strips;
-    const int steps = K / 64, q = steps / cuts, rem = steps % cuts;
-    const int ns = q + (cut < rem ? 1 : 0), s0 = cut * q + min(cut, rem);
+    const int id = (int)blockIdx.x, items = strips.d * cuts.n, li = (items & 7) == 0 ? (id & 7) * (items >> 3) + (id >> 3) : id;
+    const int cut = vt_div(li, strips), strip = li - cut * strips.d;
+    const int ns = cuts.steps + (cut < cuts.longer ? 1 : 0), s0 = cut * cuts.steps + min(cut, cuts.longer);
     const int chunks = (ns + GS_CHUNK - 1) / GS_CHUNK;
 
     const int a_voff = (lane >> 3) * K * 2 + ((lane & 7) ^ (lane >> 3)) * 16;
@@ -184,7 +183,7 @@ template <int NP, int KW, bool FRAG>
 static void gs_launch(float *d_C, int ldc, size_t plane_stride, const uint16_t *d_Ahi, const uint16_t *d_Alo, const uint16_t *d_Wf, int M, int N, int K, int cuts) {
     const int tn = 32 * GS_WAVES / KW, strips = (N + tn - 1) / tn;
     hipLaunchKernelGGL((vt_gemm_strip_kernel<NP, KW, FRAG>), dim3(strips * cuts), dim3(64 * GS_WAVES), 0, g_vt.stream, d_C, ldc, plane_stride, d_Ahi, d_Alo, d_Wf, M, N, K,
-                       strips, cuts);
+                       vt_divisor_of(strips, strips * cuts), gm_cuts_of(K, cuts));
 }
 
 vt_gemm_plan vt_gemm_few_rows_plan(int N, int swiglu) {

@@ -8,6 +8,7 @@
 
 #include "vt_state.h"
 #include "vt_gemm.h"
+#include "vt_requests.h"
 
 #include <type_traits>
 
@@ -15,6 +16,10 @@ typedef __bf16 gm_bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 gm_f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef int i32x4 __attribute__((ext_vector_type(4)));
+
+/* K in n cuts, of `steps` steps of 64 each and one more in the first `longer` of them */
+struct gm_cuts { int n, steps, longer; };
+static inline gm_cuts gm_cuts_of(int K, int n) { return gm_cuts{n, K / 64 / n, K / 64 % n}; }
 
 #define GM_STAGE_ROW 144                  /* bytes per staged row: 64 elements of 2 bytes + 16 (fragment reads cover all banks) */
 
@@ -155,8 +160,22 @@ struct gw_part {
     uint16_t *h_hi, *h_lo;
     int ldh;
     const int *row_exp, *col_exp;         /* T::SCALED: exponents of the rows and of the set's columns */
+    /* gw_add: */
+    int items;
+    vt_divisor by_n_tiles;
+    gm_cuts cuts;
 };
-struct gw_list { gw_part part[2]; int n_parts, m_tiles; };
+struct gw_list { gw_part part[2]; int n_parts, m_tiles; vt_divisor by_m_tiles; };
+static inline void gw_add(gw_list &list, const gw_part &p, int M, int tm, int K) {
+    if (!p.n_tiles) return;
+    gw_part &q = list.part[list.n_parts++];
+    q = p;
+    list.m_tiles = (M + tm - 1) / tm;
+    q.items = list.m_tiles * p.n_tiles * p.splits;
+    list.by_m_tiles = vt_divisor_of(list.m_tiles, q.items > list.part[0].items ? q.items : list.part[0].items);
+    q.by_n_tiles = vt_divisor_of(p.n_tiles, p.n_tiles * (long long)p.splits);
+    q.cuts = gm_cuts_of(K, p.splits);
+}
 
 struct gw_item {
     const unsigned char *w;               /* weights of the tile's first column */
@@ -169,17 +188,16 @@ __device__ __forceinline__ gw_item gw_item_at(const gw_list &list, int part, int
     /* Slot id lands on XCD id % 8.  An XCD takes a run of consecutive items, row tile fastest, then N tile,
      * then K cut: the row tiles of a (K cut, N tile) pair share its weights, the N tiles of a K cut share the
      * activation planes of that cut, and both leave the memory side once per XCD instead of once per workgroup. */
-    const int items = list.m_tiles * P.n_tiles * P.splits, x = id & 7, run = items >> 3, rem = items & 7;
+    const int x = id & 7, run = P.items >> 3, rem = P.items & 7;
     const int li = x * run + min(x, rem) + (id >> 3);
     gw_item it;
     it.part = part;
-    it.mt = li % list.m_tiles;
-    const int ci = li / list.m_tiles;
-    it.nt = ci % P.n_tiles;
-    it.sp = ci / P.n_tiles;
-    const int steps = K / 64, q = steps / P.splits, r = steps % P.splits;
-    it.ns = q + (it.sp < r ? 1 : 0);
-    it.s0 = it.sp * q + min(it.sp, r);
+    const int ci = vt_div(li, list.by_m_tiles);
+    it.mt = li - ci * list.m_tiles;
+    it.sp = vt_div(ci, P.by_n_tiles);
+    it.nt = ci - it.sp * P.n_tiles;
+    it.ns = P.cuts.steps + (it.sp < P.cuts.longer ? 1 : 0);
+    it.s0 = it.sp * P.cuts.steps + min(it.sp, P.cuts.longer);
     it.w = (const unsigned char *)(P.Wf + (size_t)it.nt * TN * K * WP);
     return it;
 }
@@ -459,7 +477,7 @@ vt_gemm_wide_kernel(gw_list list, const uint16_t *Ahi, const uint16_t *Alo, int 
         if constexpr (!EARLY) begin(it);
         multiply(it);
         id += (int)gridDim.x;
-        while (part < list.n_parts && id >= list.m_tiles * list.part[part].n_tiles * list.part[part].splits) {
+        while (part < list.n_parts && id >= list.part[part].items) {
             part++;
             id = (int)blockIdx.x;
         }
@@ -494,10 +512,12 @@ vt_gemm_wide_kernel(gw_list list, const uint16_t *Ahi, const uint16_t *Alo, int 
 #define GR_TN 64
 
 struct gr_list {
-    float *C;                             /* `splits` planes of [M, ldc], plane_stride floats apart */
+    float *C;                             /* cuts.n planes of [M, ldc], plane_stride floats apart */
     const uint16_t *Wf;                   /* fragment-order weights */
     size_t plane_stride;
-    int ldc, n_tiles, splits;
+    int ldc, items;
+    vt_divisor n_tiles;
+    gm_cuts cuts;
     const int *row_exp, *col_exp;         /* T::SCALED: exponents of the rows and of the columns */
 };
 
@@ -516,14 +536,12 @@ template <int NW, int WP>
 __device__ __forceinline__ gr_item gr_item_at(const gr_list &P, int id, int K, int wave) {
     /* slot id lands on XCD id % 8: an XCD takes a run of items, N tile fastest, i.e. few K cuts: the slice of
      * the planes that its L2 has to fetch is that of its cuts */
-    const int items = P.n_tiles * P.splits;
-    const int li = (items & 7) == 0 ? (id & 7) * (items >> 3) + (id >> 3) : id;
+    const int li = (P.items & 7) == 0 ? (id & 7) * (P.items >> 3) + (id >> 3) : id;
     gr_item it;
-    it.nt = li % P.n_tiles;
-    it.sp = li / P.n_tiles;
-    const int steps = K / 64, q = steps / P.splits, rem = steps % P.splits;
-    const int ns = q + (it.sp < rem ? 1 : 0);
-    it.s0 = it.sp * q + min(it.sp, rem);
+    it.sp = vt_div(li, P.n_tiles);
+    it.nt = li - it.sp * P.n_tiles.d;
+    const int ns = P.cuts.steps + (it.sp < P.cuts.longer ? 1 : 0);
+    it.s0 = it.sp * P.cuts.steps + min(it.sp, P.cuts.longer);
     it.n = ns > wave ? (ns - wave + NW - 1) / NW : 0;
     it.w = (const unsigned char *)(P.Wf + (size_t)it.nt * GR_TN * K * WP);
     return it;
@@ -685,7 +703,7 @@ vt_gemm_rows_kernel(gr_list P, const uint16_t *Ahi, const uint16_t *Alo, int M, 
     for (;;) {
         multiply(it);
         id += (int)gridDim.x;
-        if (id >= P.n_tiles * P.splits) break;
+        if (id >= P.items) break;
         const gr_item nx = gr_item_at<NW, WP>(P, id, K, wave);
         begin(nx);
         finish(it);

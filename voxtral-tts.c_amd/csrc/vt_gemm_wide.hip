@@ -110,20 +110,19 @@ template <int MB, int CW, int NB, bool FRAG = true, bool PAIR = false>
 static void gw_launch(const gw_list &list, const uint16_t *d_Ahi, const uint16_t *d_Alo, int M, int K) {
     constexpr int LDS = 2 * gw_shape<MB, CW, PAIR>::STAGE;
     if (gw_prepare<MB, CW, NB, FRAG, PAIR>()) return;
-    const int items = list.m_tiles * list.part[0].n_tiles * list.part[0].splits;      /* every workgroup takes an item of the first part */
+    const int items = list.part[0].items;      /* every workgroup takes an item of the first part */
     hipLaunchKernelGGL((vt_gemm_wide_kernel<gm_bf16, MB, CW, NB, FRAG, PAIR>), dim3(items < g_vt.n_cu ? items : g_vt.n_cu), dim3(256), LDS, g_vt.stream,
                        list, d_Ahi, d_Alo, M, K);
 }
 
 static void gw_run(const vt_gemm_plan &pl, gw_part whole, gw_part cut, const uint16_t *d_Ahi, const uint16_t *d_Alo, int M, int N, int K) {
     gw_list list = {};
-    list.m_tiles = (M + pl.tm - 1) / pl.tm;
     whole.n_tiles = pl.col0 / pl.tn;
     whole.splits = 1;
     cut.n_tiles = (N - pl.col0) / pl.tn;
     cut.splits = pl.cuts;
-    if (whole.n_tiles) list.part[list.n_parts++] = whole;
-    if (cut.n_tiles) list.part[list.n_parts++] = cut;
+    gw_add(list, whole, M, pl.tm, K);
+    gw_add(list, cut, M, pl.tm, K);
     typedef void (*fn)(const gw_list &, const uint16_t *, const uint16_t *, int, int);
     static const fn launch[4][4] = {{NULL, gw_launch<5, 2, 3, true, true>, gw_launch<5, 4, 2, true, true>, gw_launch<5, 4, 3, true, true>},
                                     {gw_launch<3, 2, 2>, gw_launch<3, 2, 3>, gw_launch<3, 4, 2>, gw_launch<3, 4, 3>},

@@ -26,4 +26,13 @@ VT_HD vt_request vt_rows_request(int t, int n, int H, int P, int passes, int row
     return vt_request{live ? block : 0, live ? (left < 16 ? left : 16) * in_dim * 2 : 0, live ? ((at / P * 8 + wave) * P + at % P) * 128 * H : 0};
 }
 
+/* Division by a number that the host knows: n / d = (n m) >> 32 with m = 2^32 / d + 1 rounded down, exact where n d < 2^32; where that
+ * does not hold for every n up to `largest`, and for d = 1, m is 0 and the kernel divides.  (A division by a kernel's argument is a
+ * chain of 20 to 30 instructions that run once, in front of a launch's first request.) */
+struct vt_divisor { unsigned m; int d; };
+VT_HD vt_divisor vt_divisor_of(int d, long long largest) {
+    return vt_divisor{d > 1 && largest * d < (1ll << 32) ? (unsigned)((1ull << 32) / (unsigned)d + 1) : 0u, d};
+}
+VT_HD int vt_div(int n, const vt_divisor &by) { return by.m ? (int)((unsigned long long)(unsigned)n * by.m >> 32) : n / by.d; }
+
 #endif /* VT_REQUESTS_H */
