@@ -333,9 +333,9 @@ vt_gemm_wide_kernel(gw_list list, const uint16_t *Ahi, const uint16_t *Alo, int 
     auto begin = [&](const gw_item &it) {
         if constexpr (T::SCALED) {
             const gw_part &P = list.part[it.part];
-            const int rows = it.ns > 0 ? min(M - it.mt * TM, TM) : 0;
+            const int rows = min(M - it.mt * TM, TM);
             next_row_exp = __builtin_amdgcn_raw_buffer_load_b32(__builtin_amdgcn_make_buffer_rsrc((void *)(P.row_exp + it.mt * TM), 0, rows * 4, 0x00020000), (int)threadIdx.x * 4, 0, 0);
-            const __amdgpu_buffer_rsrc_t d = __builtin_amdgcn_make_buffer_rsrc((void *)(P.col_exp + it.nt * TN), 0, it.ns > 0 ? TN * 4 : 0, 0x00020000);
+            const __amdgpu_buffer_rsrc_t d = __builtin_amdgcn_make_buffer_rsrc((void *)(P.col_exp + it.nt * TN), 0, TN * 4, 0x00020000);
 #pragma unroll
             for (int b = 0; b < NB; b++) next_ec[b] = __builtin_amdgcn_raw_buffer_load_b32(d, (32 * (NB * cw + b) + (lane & 31)) * 4, 0, 0);
         }
@@ -483,9 +483,10 @@ vt_gemm_wide_kernel(gw_list list, const uint16_t *Ahi, const uint16_t *Alo, int 
         }
         const bool more = part < list.n_parts;
         gw_item nx = it;
-        if (more) nx = gw_item_at<TN, WP>(list, part, id, K);
-        else nx.ns = 0;                   /* requests with nothing to bring */
-        if constexpr (EARLY) begin(nx);
+        if (more) {
+            nx = gw_item_at<TN, WP>(list, part, id, K);
+            if constexpr (EARLY) begin(nx);
+        }
         finish(it);
         if (!more) break;
         __syncthreads();                  /* the next item stages over what this one read */

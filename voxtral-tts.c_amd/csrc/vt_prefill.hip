@@ -50,6 +50,12 @@
 #define PA_SHORT_QT 16
 #define PA_LONG_QT 32
 #define PA_SHORT_ROWS 1200
+/* Up to this many rows in all, the cached ones included, the attention's workgroups make the (at most two) tiles themselves instead of
+ * reading what a launch of its own has made: with the strips' shorter code (vt_gemm_rows.hip) prefills of 6 / 20 / 37 / 64 rows 1780 / 2010 / 2356 / 2840 ->
+ * 1701 / 1861 / 2244 / 2599 us.  With three and four tiles a workgroup makes them two at a time, and every one of six or eight workgroups per
+ * head makes its own: 3177 us instead of 3130 at 96 rows, the same at 128.  (Asking for the rows in front of the queries' work needs 160 registers, and
+ * its code twice: 2387 us at 37 rows.) */
+#define PA_HERE_ROWS 64
 #define PA_PLANE 8192             /* bytes of a plane of a tile: 8 slices of K, 4 dim blocks x 2 key halves of V, 1 KB each */
 #define PA_TILE_BYTES (4 * PA_PLANE)                  /* K hi, K lo, V hi, V lo */
 
@@ -71,88 +77,115 @@ __device__ __forceinline__ void pa_planes8(const f32x4 &a, const f32x4 &b, bf16x
  * lane l = dim 32 b + l%32, keys 16 t + 4 (l/32) + 0..3 and the four 8 further on.  Workgroup = (tile, kv head), 128
  * threads for K and 128 for V; thread (sg, cg) owns the dims 4*cg .. + 4 of the 8 keys that lane group sg % 2 meets in
  * key half sg / 2, so that the transposed V write is one 16-byte store per dim and plane.
- * Rows [start_pos, start_pos + S) come from the q|k|v product when qkv != NULL: the sum of `planes`
- * split-K planes (`plane_stride` floats apart, fixed order; only the columns from col0 on are cut, a multiple
- * of 128), k rotated (adjacent pairs,
- * voxtral_tts_kernels.c:616-634; the table holds (cos, sin) per pair), and are appended to the cache on the
- * way (voxtral_tts_llm.c:317-324).  Earlier rows come from the cache; rows from kv_rows on are zeros (their
- * keys are masked).  qkv == NULL: all rows are in the cache (rope is not read). */
+ * The rows from `start` on come from the q|k|v product: the sum of `planes` split-K planes (`plane_stride` floats apart, fixed order; only
+ * the columns from col0 on are cut, a multiple of 128), k rotated (adjacent pairs, voxtral_tts_kernels.c:616-634; the table holds
+ * (cos, sin) per pair), and are appended to the cache on the way (voxtral_tts_llm.c:317-324).  Earlier rows come from the cache; rows
+ * from kv_rows on are zeros (their keys are masked).
+ *
+ * Every request goes through a descriptor that covers the rows which this source has, and brings zeros for the others, so that a row is the sum
+ * of what its sources brought: no address of 64 bits and no branch per row.  Up to three planes are in flight beside the first:
+ * with one after the other a launch at 37 rows in four cuts took 7.3 us.  (What runs once comes from memory, instructions included:
+ * with addresses and branches per row the kernel had 7.4 KB of code instead of 4.1, and at 96 rows a launch took 7.0 us instead of 6.3.) */
 __device__ __forceinline__ int pa_key(int sg, int i) { return 16 * (sg >> 1) + 4 * (sg & 1) + 8 * (i >> 2) + (i & 3); }
-__global__ void __launch_bounds__(256)
-vt_kv_image_kernel(unsigned char *img, int img_tiles, const float *qkv, int col0, int planes, size_t plane_stride,
-                   float *kc, float *vc, const float *rope, int start_pos, int kv_rows) {
-    /* threads 0..127 make the K planes of the tile, threads 128..255 the V planes */
-    const int tile = (int)blockIdx.x, kvh = (int)blockIdx.y;
-    const bool is_v = threadIdx.x >= 128;
-    const int tl = (int)threadIdx.x & 127, sg = tl >> 5, cg = tl & 31;
-    const int col = kvh * VT_HEAD_DIM + 4 * cg;
-    const int wide_col = VT_Q_DIM + (is_v ? VT_KV_DIM : 0) + col;                /* in the product's rows */
-    if (!qkv || VT_Q_DIM + (is_v ? VT_KV_DIM : 0) + kvh * VT_HEAD_DIM < col0) planes = 1;      /* a head whose columns are not cut */
-    float *cache = is_v ? vc : kc;
-    f32x4 r8[8], cs[8];
-    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-    /* Every request up front (a row that is not there asks for the last one, a plane that is not there for the last one again):
-     * with one row or plane after the other a launch at 37 rows in four cuts took 7.3 us. */
-    const float *src[8];
-    bool fresh[8];
+
+struct pa_rows {
+    const float *qkv;             /* [kv_rows - start, 6144] planes */
+    int col0, planes;
+    size_t plane_stride;
+    float *kc, *vc;               /* [kv_rows, 1024] */
+    const float *rope;
+    int start, kv_rows;
+};
+
+/* (a clamped size is made by a vector instruction; without the move to a scalar register each request becomes a loop over the lanes' descriptors) */
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t pa_buffer(const void *p, int bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, __builtin_amdgcn_readfirstlane(bytes), 0x00020000);
+}
+__device__ __forceinline__ f32x4 pa_load(__amdgpu_buffer_rsrc_t r, int at) {
+    return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, at, 0, 0));
+}
+
+/* 256 threads make the K planes of tile `tile` of kv head kvh at Kt (threads 0..127) and its V planes at Vt (threads 128..255); of the
+ * rows from `start` on, first .. first + n - 1 are appended to the cache. */
+template <class PTR>
+__device__ __forceinline__ void pa_make_tile(PTR Kt, PTR Vt, const pa_rows &in, int kvh, int tile, int thread, int first, int n) {
+    const bool is_v = __builtin_amdgcn_readfirstlane(thread >> 7);           /* a wave is all K or all V */
+    const int tl = thread & 127, sg = tl >> 5, cg = tl & 31;
+    const int wide = VT_Q_DIM + (is_v ? VT_KV_DIM : 0) + kvh * VT_HEAD_DIM, col = kvh * VT_HEAD_DIM + 4 * cg;
+    const int planes = wide < in.col0 ? 1 : in.planes;                       /* a head whose columns are not cut has one */
+    /* descriptors begin at the tile's first row, or the source's where that lies within (rows in front of it: beyond any size) */
+    const int t0 = tile * 32, row0 = t0 + pa_key(sg, 0), f0 = max(t0, in.start), fresh_bytes = max(min(in.kv_rows - f0, 32), 0) * VT_QKV_DIM * 4;
+    const float *fresh = in.qkv + (size_t)(f0 - in.start) * VT_QKV_DIM;
+    float *const kc = in.kc, *const vc = in.vc, *const cache = is_v ? vc : kc;
+    const int at = (row0 - f0) * (VT_QKV_DIM * 4) + (wide + 4 * cg) * 4;
+    auto off = [](int i, int pitch) { return (8 * (i >> 2) + (i & 3)) * pitch; };
+    f32x4 r8[8], cs[8], w[3][8];
+    const __amdgpu_buffer_rsrc_t d0 = pa_buffer(fresh, fresh_bytes);
+    /* (a caller's own K and V may have more rows than the table: nothing of it is read for rows that are not rotated) */
+    const __amdgpu_buffer_rsrc_t dc = pa_buffer(in.rope + (size_t)t0 * VT_HEAD_DIM, is_v || fresh_bytes == 0 ? 0 : min(in.kv_rows - t0, 32) * VT_HEAD_DIM * 4);
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
-        const int r = min(tile * 32 + pa_key(sg, i), kv_rows - 1);
-        fresh[i] = qkv && r >= start_pos;
-        src[i] = fresh[i] ? qkv + (size_t)(r - start_pos) * VT_QKV_DIM + wide_col : cache + (size_t)r * VT_KV_DIM + col;
-        r8[i] = *reinterpret_cast<const f32x4 *>(src[i]);
-        cs[i] = qkv && !is_v ? *reinterpret_cast<const f32x4 *>(rope + (size_t)r * VT_HEAD_DIM + 4 * cg) : zero;
-    }
+    for (int i = 0; i < 8; i++) r8[i] = pa_load(d0, at + off(i, VT_QKV_DIM * 4));
+#pragma unroll
+    for (int i = 0; i < 8; i++) cs[i] = pa_load(dc, (row0 - t0) * (VT_HEAD_DIM * 4) + 16 * cg + off(i, VT_HEAD_DIM * 4));
     for (int p = 1; p < planes; p += 3) {
-        f32x4 w[3][8];
 #pragma unroll
-        for (int z = 0; z < 3; z++)
+        for (int z = 0; z < 3; z++) {
+            const __amdgpu_buffer_rsrc_t d = pa_buffer(fresh + (size_t)min(p + z, planes - 1) * in.plane_stride, p + z < planes ? fresh_bytes : 0);
 #pragma unroll
-            for (int i = 0; i < 8; i++) w[z][i] = *reinterpret_cast<const f32x4 *>(src[i] + (fresh[i] ? min(p + z, planes - 1) * plane_stride : 0));
-#pragma unroll
-        for (int z = 0; z < 3; z++)
-            if (p + z < planes) {
-#pragma unroll
-                for (int i = 0; i < 8; i++)
-                    if (fresh[i]) {
-                        r8[i].x = __fadd_rn(r8[i].x, w[z][i].x); r8[i].y = __fadd_rn(r8[i].y, w[z][i].y);
-                        r8[i].z = __fadd_rn(r8[i].z, w[z][i].z); r8[i].w = __fadd_rn(r8[i].w, w[z][i].w);
-                    }
-            }
-    }
-#pragma unroll
-    for (int i = 0; i < 8; i++) {
-        const int r = tile * 32 + pa_key(sg, i);
-        if (fresh[i]) {
-            if (!is_v) {
-                const f32x4 k = r8[i], c = cs[i];
-                r8[i] = f32x4{__fsub_rn(__fmul_rn(k.x, c.x), __fmul_rn(k.y, c.y)), __fadd_rn(__fmul_rn(k.x, c.y), __fmul_rn(k.y, c.x)),
-                              __fsub_rn(__fmul_rn(k.z, c.z), __fmul_rn(k.w, c.w)), __fadd_rn(__fmul_rn(k.z, c.w), __fmul_rn(k.w, c.z))};
-            }
-            if (r < kv_rows) *reinterpret_cast<f32x4 *>(cache + (size_t)r * VT_KV_DIM + col) = r8[i];
+            for (int i = 0; i < 8; i++) w[z][i] = pa_load(d, at + off(i, VT_QKV_DIM * 4));
         }
-        if (r >= kv_rows) r8[i] = zero;
+#pragma unroll
+        for (int z = 0; z < 3; z++)
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                r8[i].x = __fadd_rn(r8[i].x, w[z][i].x); r8[i].y = __fadd_rn(r8[i].y, w[z][i].y);
+                r8[i].z = __fadd_rn(r8[i].z, w[z][i].z); r8[i].w = __fadd_rn(r8[i].w, w[z][i].w);
+            }
     }
-    unsigned char *Kt = img + ((size_t)kvh * img_tiles + tile) * PA_TILE_BYTES, *Vt = Kt + 2 * PA_PLANE;
     if (!is_v) {
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const f32x4 k = r8[i], c = cs[i];
+            r8[i] = f32x4{__fsub_rn(__fmul_rn(k.x, c.x), __fmul_rn(k.y, c.y)), __fadd_rn(__fmul_rn(k.x, c.y), __fmul_rn(k.y, c.x)),
+                          __fsub_rn(__fmul_rn(k.z, c.z), __fmul_rn(k.w, c.w)), __fadd_rn(__fmul_rn(k.z, c.w), __fmul_rn(k.w, c.z))};
+        }
+    }
+    const int s0 = max(t0, first);
+    const __amdgpu_buffer_rsrc_t ds = pa_buffer(cache + (size_t)s0 * VT_KV_DIM, max(min(min(first + n, in.kv_rows), t0 + 32) - s0, 0) * VT_KV_DIM * 4);
+#pragma unroll
+    for (int i = 0; i < 8; i++)
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, r8[i]), ds, (row0 - s0) * (VT_KV_DIM * 4) + col * 4 + off(i, VT_KV_DIM * 4), 0, 0);
+    if (t0 < in.start) {                                 /* earlier rows */
+        const __amdgpu_buffer_rsrc_t d = pa_buffer(cache + (size_t)t0 * VT_KV_DIM, min(in.start - t0, 32) * VT_KV_DIM * 4);
+#pragma unroll
+        for (int i = 0; i < 8; i++) w[0][i] = pa_load(d, (row0 - t0) * (VT_KV_DIM * 4) + col * 4 + off(i, VT_KV_DIM * 4));
+#pragma unroll
+        for (int i = 0; i < 8; i++) r8[i] += w[0][i];
+    }
+    if (!is_v) {
+        PTR to = Kt + (cg >> 2) * 1024 + ((cg >> 1) & 1) * 512 + pa_key(sg, 0) * 16 + (cg & 1) * 8;
 #pragma unroll
         for (int i = 0; i < 8; i++) {
             u32x2 h, l;
             vt_split_planes4(r8[i].x, r8[i].y, r8[i].z, r8[i].w, h, l);
-            unsigned char *at = Kt + (cg >> 2) * 1024 + ((cg >> 1) & 1) * 512 + pa_key(sg, i) * 16 + (cg & 1) * 8;
-            *reinterpret_cast<u32x2 *>(at) = h;
-            *reinterpret_cast<u32x2 *>(at + PA_PLANE) = l;
+            *reinterpret_cast<u32x2 *>(to + off(i, 16)) = h;
+            *reinterpret_cast<u32x2 *>(to + off(i, 16) + PA_PLANE) = l;
         }
     } else {
+        PTR to = Vt + ((cg >> 3) * 2 + (sg >> 1)) * 1024 + ((sg & 1) * 32 + (4 * cg) % 32) * 16;
 #pragma unroll
         for (int d = 0; d < 4; d++) {
             bf16x8 h, l;
             pa_planes8(f32x4{r8[0][d], r8[1][d], r8[2][d], r8[3][d]}, f32x4{r8[4][d], r8[5][d], r8[6][d], r8[7][d]}, h, l);
-            unsigned char *at = Vt + ((cg >> 3) * 2 + (sg >> 1)) * 1024 + ((sg & 1) * 32 + (4 * cg + d) % 32) * 16;
-            *reinterpret_cast<bf16x8 *>(at) = h;
-            *reinterpret_cast<bf16x8 *>(at + PA_PLANE) = l;
+            *reinterpret_cast<bf16x8 *>(to + 16 * d) = h;
+            *reinterpret_cast<bf16x8 *>(to + 16 * d + PA_PLANE) = l;
         }
     }
+}
+
+__global__ void __launch_bounds__(256) vt_kv_image_kernel(unsigned char *img, int img_tiles, pa_rows in) {
+    unsigned char *Kt = img + ((size_t)blockIdx.y * img_tiles + blockIdx.x) * PA_TILE_BYTES;
+    pa_make_tile(Kt, Kt + 2 * PA_PLANE, in, (int)blockIdx.y, (int)blockIdx.x, (int)threadIdx.x, in.start, in.kv_rows - in.start);
 }
 
 typedef float pa_f32x16 __attribute__((ext_vector_type(16)));
@@ -165,11 +198,14 @@ __device__ __forceinline__ float pa_max_halves(float x) {
     return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
 }
 
-template <int QB>
+/* HERE (QB 16, at most two tiles in all): no images; a workgroup makes the tiles that its queries see in its own LDS, from the rows
+ * `in`, and appends its queries' rows to the cache. */
+template <int QB, bool HERE>
 __global__ void __launch_bounds__(512)
 vt_prefill_attention_kernel(float *out, uint16_t *out_hi, uint16_t *out_lo, const float *Q,
                             int q_stride, int q_col0, int q_planes, size_t q_plane_stride, const float *rope,
-                            const unsigned char *img, int img_tiles, int S, int start_pos, float scale) {
+                            const unsigned char *img, int img_tiles, int S, int start_pos, float scale, pa_rows in) {
+    static_assert(!HERE || QB == 16, "a residue each for two tiles");
     constexpr int HW = QB / 8, NS = 8 / HW;              /* waves of a residue, residues */
     /* QB 32: a tile of each residue of the even and of the odd steps; QB 16: K and V of a tile of each residue */
     __shared__ __attribute__((aligned(16))) unsigned char pa_a[65536], pa_b[65536];
@@ -196,7 +232,7 @@ vt_prefill_attention_kernel(float *out, uint16_t *out_hi, uint16_t *out_lo, cons
             __builtin_amdgcn_raw_ptr_buffer_load_lds(t_rs, (__attribute__((address_space(3))) void *)(buf + pz * KB * 1024 + (i * HW + hq) * 1024), 16,
                                                      (i * HW + hq) * 1024 + lane * 16, rq.soff, 0, 0);
     };
-    fetch(pa_a, 0, 0);
+    if constexpr (!HERE) fetch(pa_a, 0, 0);
 
     /* The queries of the four heads, QB rows x 512 columns: Q as it is, or (rope != NULL) the raw product: the sum of
      * q_planes split-K planes, rotated here (adjacent pairs, voxtral_tts_kernels.c:616-634; the table holds (cos, sin)
@@ -320,7 +356,13 @@ vt_prefill_attention_kernel(float *out, uint16_t *out_hi, uint16_t *out_lo, cons
     /* every wave waits for what it asked for, then for all the others: they have then also read what is written next */
 #define PA_LANDED() do { __builtin_amdgcn_s_waitcnt(0x0f70); __syncthreads(); } while (0)     /* vmcnt(0) */
     PA_LANDED();
-    if constexpr (QB == 32) {
+    if constexpr (HERE) {
+        const int tile = wave >> 2;                      /* half of the waves for each */
+        if (tile < ntiles) pa_make_tile(pa_a + tile * 2 * PA_PLANE, pa_b + tile * 2 * PA_PLANE, in, kvh, tile, t & 255, start_pos + q0, QB);
+        __syncthreads();
+        if (pz < ntiles) { scores(pa_a + pz * 2 * PA_PLANE); weigh(pa_b + pz * 2 * PA_PLANE, pz); }
+        __syncthreads();
+    } else if constexpr (QB == 32) {
         /* the next tile arrives while this one is worked on: one barrier per tile */
         const unsigned char *even = pa_a + pz * PA_TILE_BYTES, *odd = pa_b + pz * PA_TILE_BYTES;
         for (int step = 0; step < nsteps; step += 2) {
@@ -441,8 +483,8 @@ unsigned char *vt_pa_image(int rows) {
 void vt_pa_launch_image(unsigned char *d_img, const float *d_qkv, int col0, int planes, size_t plane_stride, float *d_K,
                         float *d_V, int S, int start_pos) {
     const int rows = start_pos + S;
-    hipLaunchKernelGGL(vt_kv_image_kernel, dim3(pa_tiles(rows), VT_KV_HEADS), dim3(256), 0, g_vt.stream, d_img,
-                       pa_tiles(rows), d_qkv, col0, planes, plane_stride, d_K, d_V, g_vt.d_rope, start_pos, rows);
+    hipLaunchKernelGGL(vt_kv_image_kernel, dim3(pa_tiles(rows), VT_KV_HEADS), dim3(256), 0, g_vt.stream, d_img, pa_tiles(rows),
+                       pa_rows{d_qkv, col0, planes, plane_stride, d_K, d_V, g_vt.d_rope, d_qkv ? start_pos : rows, rows});
 }
 
 /* Q rows are q_stride floats apart; out / (out_hi, out_lo) are [S,4096], each optional.  d_rope != NULL: d_Q
@@ -455,11 +497,25 @@ void vt_launch_prefill_attention_raw(float *d_out, uint16_t *d_hi, uint16_t *d_l
     const bool lng = S > PA_SHORT_ROWS;
     const int qb = lng ? PA_LONG_QT : PA_SHORT_QT;
     const dim3 grid(VT_KV_HEADS, (S + qb - 1) / qb);
-#define CALL(QB) hipLaunchKernelGGL(vt_prefill_attention_kernel<QB>, grid, dim3(512), 0, g_vt.stream, d_out, d_hi, d_lo, d_Q, q_stride, q_col0, \
-                                    q_planes, q_plane_stride, d_rope, d_img, pa_tiles(start_pos + S), S, start_pos, scale)
+#define CALL(QB) hipLaunchKernelGGL((vt_prefill_attention_kernel<QB, false>), grid, dim3(512), 0, g_vt.stream, d_out, d_hi, d_lo, d_Q, q_stride, q_col0, \
+                                    q_planes, q_plane_stride, d_rope, d_img, pa_tiles(start_pos + S), S, start_pos, scale, pa_rows{})
     if (lng) CALL(PA_LONG_QT);
     else CALL(PA_SHORT_QT);
 #undef CALL
+}
+
+/* A layer's attention on the raw q|k|v product and the cache rows in front of it, rows start_pos .. + S - 1 appended; with up to
+ * PA_HERE_ROWS rows in all as one launch */
+static void pa_launch_layer(uint16_t *d_hi, uint16_t *d_lo, const float *d_qkv, int col0, int planes, size_t plane_stride, float *d_K, float *d_V,
+                            unsigned char *d_img, int S, int start_pos) {
+    if (start_pos + S <= PA_HERE_ROWS) {
+        hipLaunchKernelGGL((vt_prefill_attention_kernel<16, true>), dim3(VT_KV_HEADS, (S + 15) / 16), dim3(512), 0, g_vt.stream, (float *)NULL, d_hi, d_lo, d_qkv, VT_QKV_DIM,
+                           col0, planes, plane_stride, g_vt.d_rope, (const unsigned char *)NULL, 0, S, start_pos, VT_ATT_SCALE,
+                           pa_rows{d_qkv, col0, planes, plane_stride, d_K, d_V, g_vt.d_rope, start_pos, start_pos + S});
+        return;
+    }
+    vt_pa_launch_image(d_img, d_qkv, col0, planes, plane_stride, d_K, d_V, S, start_pos);
+    vt_launch_prefill_attention_raw(NULL, d_hi, d_lo, d_qkv, VT_QKV_DIM, col0, planes, plane_stride, g_vt.d_rope, d_img, S, start_pos, VT_ATT_SCALE);
 }
 
 void vt_launch_prefill_attention(float *d_out, uint16_t *d_hi, uint16_t *d_lo, const float *d_Q,
@@ -538,9 +594,7 @@ extern "C" void tts_hip_llm_prefill_out(const float *embeds, int seq_len, int st
         else vt_launch_gemm(wide, hi, lo, L->wqkv, seq_len, VT_QKV_DIM, VT_DIM, pq.cuts);
         /* k (rotated) and v into the cache and, with the earlier rows, into the attention's tile images; the
          * attention takes q from the product's planes itself */
-        vt_pa_launch_image(img, wide, pq.col0, pq.cuts, S * VT_QKV_DIM, kc, vc, seq_len, start_pos);
-        vt_launch_prefill_attention_raw(NULL, hi, lo, wide, VT_QKV_DIM, pq.col0, pq.cuts, S * VT_QKV_DIM, g_vt.d_rope, img,
-                                        seq_len, start_pos, VT_ATT_SCALE);
+        pa_launch_layer(hi, lo, wide, pq.col0, pq.cuts, S * VT_QKV_DIM, kc, vc, img, seq_len, start_pos);
         if (frag) vt_launch_gemm_frag(part, VT_DIM, ps, hi, lo, F->wo, seq_len, VT_DIM, VT_Q_DIM, po);
         else vt_launch_gemm(part, hi, lo, L->wo, seq_len, VT_DIM, VT_Q_DIM, po.cuts);
         vt_launch_residual_norm_split(x, part, po.col0, po.cuts, ps, L->ffn_norm, hi, lo, seq_len);
