@@ -78,23 +78,27 @@ __device__ __forceinline__ void cd_put4(const cd_planes &p, size_t at, const f32
  * partial planes of the others, [rows, n - col0] */
 struct cd_product { const float *p; int rows, n, col0, cuts; };
 
-/* Four columns of a row, partial planes in order.  Up to C of them, all requested before the first is used (one after
- * the other they cost a memory latency each); those that do not exist repeat plane 0. */
+/* Four columns of a row: the whole column and each plane of a cut one, which bring zeros for the columns that they do not have (and
+ * planes that do not exist, for all).  The kernels ask for all that they need and put cd_asked() behind it (one after the other the
+ * planes cost a memory latency each); total() adds the planes in order. */
 template <int C>
-__device__ __forceinline__ f32x4 cd_sum(const cd_product &r, int row, int col) {
-    const bool cut = col >= r.col0;
-    const int pitch = cut ? r.n - r.col0 : r.col0, n = cut ? r.cuts : 1;
-    const size_t stride = (size_t)r.rows * pitch;
-    const float *p = r.p + (cut ? (size_t)r.rows * r.col0 : 0) + (size_t)row * pitch + (cut ? col - r.col0 : col);
-    f32x4 q[C];
+struct cd_quads {
+    f32x4 whole, q[C];
+    __device__ __forceinline__ void ask(const cd_product &r, int row, int col) {
+        const int cut = r.n - r.col0;
+        whole = vt_buffer_ld4(vt_buffer(r.p + (size_t)row * r.col0, r.col0 * 4), 4 * col);
+        const float *pc = r.p + (size_t)r.rows * r.col0 + (size_t)row * cut;
 #pragma unroll
-    for (int s = 0; s < C; s++) q[s] = *(const f32x4 *)(p + (s < n ? s : 0) * stride);
-    f32x4 v = q[0];
+        for (int s = 0; s < C; s++) q[s] = vt_buffer_ld4(vt_buffer(pc + (size_t)(s < r.cuts ? s : 0) * ((size_t)r.rows * cut), s < r.cuts ? cut * 4 : 0), 4 * (col - r.col0));
+    }
+    __device__ __forceinline__ f32x4 total() const {
+        f32x4 v = whole;
 #pragma unroll
-    for (int s = 1; s < C; s++)
-        if (s < n) v += q[s];
-    return v;
-}
+        for (int s = 0; s < C; s++) v += q[s];
+        return v;
+    }
+};
+__device__ __forceinline__ void cd_asked() { __builtin_amdgcn_sched_barrier(0); }
 
 /* One row of 1024: val = the product's result (+ bias) (* scale) (+ residual).  With a norm weight val -> x_out and
  * val * rsqrt(mean(val^2) + eps) * norm_w (tts_rms_norm, voxtral_tts_kernels.c:333-349) as planes; without one the
@@ -112,10 +116,17 @@ vt_codec_row_kernel(float *x_out, cd_planes xn, const float *x_in, cd_product in
     f32x4 v;
     if (UP) {
         const int j = row >> 1, col = (row & 1) * CD_DIM + c;
-        v = cd_sum<C>(in, j, col);
-        if (j > 0) v += cd_sum<C>(in, j - 1, 2 * CD_DIM + col);
+        cd_quads<C> q, before;
+        q.ask(in, j, col);
+        before.ask(in, max(j - 1, 0), 2 * CD_DIM + col);
+        cd_asked();
+        v = q.total();
+        if (j > 0) v += before.total();
     } else {
-        v = cd_sum<C>(in, row, c);
+        cd_quads<C> q;
+        q.ask(in, row, c);
+        cd_asked();
+        v = q.total();
     }
     if (bias) v += *(const f32x4 *)(bias + c);
     if (scale) v *= *(const f32x4 *)(scale + c);
@@ -140,8 +151,12 @@ vt_codec_qkv_kernel(float *__restrict__ qkv, cd_product in, const float *__restr
     const int row = blockIdx.x, c = threadIdx.x * 4;
     const size_t at = (size_t)row * (3 * CD_DIM) + c;
     f32x4 v[3];
+    cd_quads<C> q[3];
 #pragma unroll
-    for (int part = 0; part < 3; part++) v[part] = cd_sum<C>(in, row, part * CD_DIM + c);
+    for (int part = 0; part < 3; part++) q[part].ask(in, row, part * CD_DIM + c);
+    cd_asked();
+#pragma unroll
+    for (int part = 0; part < 3; part++) v[part] = q[part].total();
 #pragma unroll
     for (int part = 0; part < 3; part++) {
         const float *nw = part == 0 ? q_norm : part == 1 ? k_norm : nullptr;
@@ -162,12 +177,21 @@ vt_codec_swiglu_kernel(cd_planes h, cd_product gu) {
     const int row = blockIdx.x;
     f32x4 v[CD_HID / 1024];
     float m = 0.f;
+    constexpr int AT_ONCE = C > 4 ? 2 : CD_HID / 1024;        /* registers */
 #pragma unroll
-    for (int j = 0; j < CD_HID / 1024; j++) {
-        const int c = 4 * ((int)threadIdx.x + 256 * j);
-        const f32x4 g = cd_sum<C>(gu, row, c), u = cd_sum<C>(gu, row, CD_HID + c);
-        v[j] = vt_silu_mul4(g, u);
-        m = fmaxf(m, cd_max4(v[j]));
+    for (int j0 = 0; j0 < CD_HID / 1024; j0 += AT_ONCE) {
+        cd_quads<C> g[AT_ONCE], u[AT_ONCE];
+#pragma unroll
+        for (int j = 0; j < AT_ONCE; j++) {
+            g[j].ask(gu, row, 4 * ((int)threadIdx.x + 256 * (j0 + j)));
+            u[j].ask(gu, row, CD_HID + 4 * ((int)threadIdx.x + 256 * (j0 + j)));
+        }
+        cd_asked();
+#pragma unroll
+        for (int j = 0; j < AT_ONCE; j++) {
+            v[j0 + j] = vt_silu_mul4(g[j].total(), u[j].total());
+            m = fmaxf(m, cd_max4(v[j0 + j]));
+        }
     }
     const int e = vt_f16_exp(cd_block_max(m, red));
 #pragma unroll
@@ -385,13 +409,14 @@ vt_codec_wave_kernel(float *__restrict__ out, cd_product in, const float *__rest
     const int t = t0 + blockIdx.x, c = threadIdx.x * 4;
     if (c >= CD_PATCH) return;
     f32x4 v = {0.f, 0.f, 0.f, 0.f};
+    auto src = [&](int k) { return abs(t + k - (CD_OUT_TAPS - 1)); };
+    cd_quads<C> q[CD_OUT_TAPS];
 #pragma unroll
-    for (int k = 0; k < CD_OUT_TAPS; k++) {
-        int src = t + k - (CD_OUT_TAPS - 1);
-        if (src < 0) src = -src;
-        const f32x4 p = cd_sum<C>(in, src < in.rows ? src : 0, k * CD_OUT_PITCH + c);
-        if (src < in.rows) v += p;
-    }
+    for (int k = 0; k < CD_OUT_TAPS; k++) q[k].ask(in, src(k) < in.rows ? src(k) : 0, k * CD_OUT_PITCH + c);
+    if (C <= 4) cd_asked();                              /* (of eight planes the registers do not hold all) */
+#pragma unroll
+    for (int k = 0; k < CD_OUT_TAPS; k++)
+        if (src(k) < in.rows) v += q[k].total();
     if (bias) v += *(const f32x4 *)(bias + c);
     *(f32x4 *)(out + (size_t)t * CD_PATCH + c) = v;
 }

@@ -27,6 +27,22 @@ __device__ __forceinline__ int vt_tid() { int t = (int)threadIdx.x; asm volatile
 __device__ __forceinline__ int vt_lane() { return vt_tid() & (VT_WAVE - 1); }
 __device__ __forceinline__ int vt_wave() { return vt_tid() >> 6; }
 
+/* Memory through a buffer descriptor: what lies beyond `bytes`, a negative offset included, reads as zeros and is not written.  Where a
+ * source has some of the columns or rows only, that takes the place of a branch or a selection per element, and a base in scalar
+ * registers that of 64-bit additions per lane: the kernels between the products run each instruction once, from a cold
+ * instruction cache, where 300 instructions are about 1.5 us.  (A clamped size is made by a vector instruction; without the move to a scalar
+ * register each request becomes a loop over the lanes' descriptors.) */
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t vt_buffer(const void *p, int bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, __builtin_amdgcn_readfirstlane(bytes), 0x00020000);
+}
+__device__ __forceinline__ f32x4 vt_buffer_ld4(__amdgpu_buffer_rsrc_t r, int at) {
+    return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, at, 0, 0));
+}
+__device__ __forceinline__ void vt_buffer_st4(__amdgpu_buffer_rsrc_t r, int at, const f32x4 &v) {
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), r, at, 0, 0);
+}
+__device__ __forceinline__ void vt_buffer_st2(__amdgpu_buffer_rsrc_t r, int at, const u32x2 &v) { __builtin_amdgcn_raw_buffer_store_b64(v, r, at, 0, 0); }
+
 /* bf16 pair packed in a dword: element 0 in the low half. Widening is exact. */
 __device__ __forceinline__ float vt_bf16_lo(unsigned int w) { return __uint_as_float(w << 16); }
 __device__ __forceinline__ float vt_bf16_hi(unsigned int w) { return __uint_as_float(w & 0xffff0000u); }

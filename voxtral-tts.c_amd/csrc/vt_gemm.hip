@@ -234,7 +234,7 @@ static_assert(VT_MAX_CUTS == 8, "GM_BY_PLANES");
  *   (hi, lo)[row] = split(rmsnorm(x[row]) * w)                                   (w != NULL)
  * The residual add and the normalisation of voxtral_tts_llm.c:332-336,354 /
  * :338-341 in one pass over the row.  Up to a few hundred rows a launch is one chain of memory latencies per
- * workgroup, so everything is requested in front of the first sum (columns that are not cut ask for plane 0 again);
+ * workgroup, so everything is requested in front of the first sum;
  * with the planes in a loop that waited for each of them a launch took 8.5 us at 226 rows and takes 6.0 to 6.6 now; us per
  * prefill of 37 / 226 / 512 / 1531 rows 2632 / 4414 / 7236 / 20457 -> 2481 / 4326 / 7186 / 20181, results the same. */
 template <int C>
@@ -246,33 +246,37 @@ vt_residual_norm_split_kernel(float *x, const float *part, int col0, size_t part
     __shared__ float red[4];
     const size_t row = blockIdx.x;
     constexpr int NJ = VT_DIM / 1024;
+    const __amdgpu_buffer_rsrc_t dx = vt_buffer(x + row * VT_DIM, VT_DIM * 4);
+    const int at = 16 * (int)threadIdx.x;
     f32x4 v[NJ], g[NJ], p[NJ][C > 0 ? C : 1];
 #pragma unroll
-    for (int j = 0; j < NJ; j++) {
-        const int c = 4 * ((int)threadIdx.x + 256 * j);
-        const size_t i = row * VT_DIM + c;
-        v[j] = *reinterpret_cast<const f32x4 *>(x + i);
+    for (int j = 0; j < NJ; j++) v[j] = vt_buffer_ld4(dx, at + 4096 * j);
 #pragma unroll
-        for (int s = 0; s < C; s++) p[j][s] = *reinterpret_cast<const f32x4 *>(part + (c < col0 ? 0 : s) * part_stride + i);
-        g[j] = v[j];
-        if (w) g[j] = *reinterpret_cast<const f32x4 *>(w + c);
+    for (int s = 0; s < C; s++) {
+        /* the planes behind the first have the columns from col0 on, and zeros for the others */
+        const int from = s ? col0 : 0;
+        const __amdgpu_buffer_rsrc_t d = vt_buffer(part + s * part_stride + row * VT_DIM + from, (VT_DIM - from) * 4);
+#pragma unroll
+        for (int j = 0; j < NJ; j++) p[j][s] = vt_buffer_ld4(d, at + 4096 * j - from * 4);
     }
+    const __amdgpu_buffer_rsrc_t dw = vt_buffer(w, w ? VT_DIM * 4 : 0);
+#pragma unroll
+    for (int j = 0; j < NJ; j++) g[j] = vt_buffer_ld4(dw, at + 4096 * j);
+    __builtin_amdgcn_sched_barrier(0);
     float ss = 0.f;
 #pragma unroll
     for (int j = 0; j < NJ; j++) {
-        const int c = 4 * ((int)threadIdx.x + 256 * j);
         f32x4 a = v[j];
         if (C > 0) {
             f32x4 q = p[j][0];
 #pragma unroll
-            for (int s = 1; s < C; s++)
-                if (c >= col0) {
-                    q.x = __fadd_rn(q.x, p[j][s].x); q.y = __fadd_rn(q.y, p[j][s].y);
-                    q.z = __fadd_rn(q.z, p[j][s].z); q.w = __fadd_rn(q.w, p[j][s].w);
-                }
+            for (int s = 1; s < C; s++) {
+                q.x = __fadd_rn(q.x, p[j][s].x); q.y = __fadd_rn(q.y, p[j][s].y);
+                q.z = __fadd_rn(q.z, p[j][s].z); q.w = __fadd_rn(q.w, p[j][s].w);
+            }
             a.x = __fadd_rn(a.x, q.x); a.y = __fadd_rn(a.y, q.y);
             a.z = __fadd_rn(a.z, q.z); a.w = __fadd_rn(a.w, q.w);
-            *reinterpret_cast<f32x4 *>(x + row * VT_DIM + c) = a;
+            vt_buffer_st4(dx, at + 4096 * j, a);
         }
         v[j] = a;
         ss = fmaf(a.x, a.x, ss); ss = fmaf(a.y, a.y, ss);
@@ -284,14 +288,14 @@ vt_residual_norm_split_kernel(float *x, const float *part, int col0, size_t part
     __syncthreads();
     const float tot = (red[0] + red[1]) + (red[2] + red[3]);
     const float inv = 1.0f / sqrtf(tot / (float)VT_DIM + eps);
+    const __amdgpu_buffer_rsrc_t dh = vt_buffer(hi + row * VT_DIM, VT_DIM * 2), dl = vt_buffer(lo + row * VT_DIM, VT_DIM * 2);
 #pragma unroll
     for (int j = 0; j < NJ; j++) {
-        const int c = 4 * ((int)threadIdx.x + 256 * j);
         u32x2 sph, spl;
         vt_split_planes4(__fmul_rn(__fmul_rn(v[j].x, inv), g[j].x), __fmul_rn(__fmul_rn(v[j].y, inv), g[j].y),
                          __fmul_rn(__fmul_rn(v[j].z, inv), g[j].z), __fmul_rn(__fmul_rn(v[j].w, inv), g[j].w), sph, spl);
-        *reinterpret_cast<u32x2 *>(hi + row * VT_DIM + c) = sph;
-        *reinterpret_cast<u32x2 *>(lo + row * VT_DIM + c) = spl;
+        vt_buffer_st2(dh, at / 2 + 2048 * j, sph);
+        vt_buffer_st2(dl, at / 2 + 2048 * j, spl);
     }
 }
 
@@ -353,20 +357,19 @@ void vt_launch_swiglu_split(uint16_t *d_hi, uint16_t *d_lo, const float *d_gu, s
  * (hi, lo) planes of SiLU(gate) * up at h columns h_col0 .. h_col0 + tw/2 (row pitch ldh).  A thread owns 4
  * consecutive h columns and requests all its planes at once. */
 template <int P>
-__global__ void vt_swiglu_pair_tail_kernel(uint16_t *hi, uint16_t *lo, int ldh, int h_col0, const float *tail,
-                                           size_t stride, int rows, int tw) {
-    const int per_row = tw / 8;                                   /* threads per row */
-    const size_t total = (size_t)rows * per_row;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (size_t)gridDim.x * blockDim.x) {
-        const int row = (int)(i / per_row), q = (int)(i % per_row);
-        const int blk = q >> 2, c = (q & 3) * 4;
-        const float *tp = tail + (size_t)row * tw + 32 * blk + c;
+__global__ void __launch_bounds__(256) vt_swiglu_pair_tail_kernel(uint16_t *hi, uint16_t *lo, int ldh, int h_col0, const float *tail,
+                                                                  size_t stride, int rows, int tw) {
+    const int q = (int)(blockIdx.x * 256 + threadIdx.x), blk = q >> 2, c = (q & 3) * 4;
+    if (q >= tw / 8) return;
+    for (size_t row = blockIdx.y; row < (size_t)rows; row += gridDim.y) {
         f32x4 gs[P], us[P];
 #pragma unroll
         for (int p = 0; p < P; p++) {
-            gs[p] = *reinterpret_cast<const f32x4 *>(tp + p * stride);
-            us[p] = *reinterpret_cast<const f32x4 *>(tp + p * stride + 16);
+            const __amdgpu_buffer_rsrc_t d = vt_buffer(tail + p * stride + row * tw, tw * 4);
+            gs[p] = vt_buffer_ld4(d, (32 * blk + c) * 4);
+            us[p] = vt_buffer_ld4(d, (32 * blk + c) * 4 + 64);
         }
+        __builtin_amdgcn_sched_barrier(0);
         f32x4 g = gs[0], u = us[0];
 #pragma unroll
         for (int p = 1; p < P; p++) {
@@ -376,15 +379,15 @@ __global__ void vt_swiglu_pair_tail_kernel(uint16_t *hi, uint16_t *lo, int ldh, 
         const f32x4 h = vt_silu_mul4(g, u);
         u32x2 sph, spl;
         vt_split_planes4(h.x, h.y, h.z, h.w, sph, spl);
-        const size_t at = (size_t)row * ldh + h_col0 + 16 * blk + c;
-        *reinterpret_cast<u32x2 *>(hi + at) = sph;
-        *reinterpret_cast<u32x2 *>(lo + at) = spl;
+        const size_t at = row * ldh + h_col0;
+        vt_buffer_st2(vt_buffer(hi + at, tw), (16 * blk + c) * 2, sph);
+        vt_buffer_st2(vt_buffer(lo + at, tw), (16 * blk + c) * 2, spl);
     }
 }
 
 void vt_launch_swiglu_pair_tail(uint16_t *d_hi, uint16_t *d_lo, int ldh, int h_col0, const float *d_tail, int planes,
                                 size_t stride, int rows, int tw) {
-#define CALL(P) hipLaunchKernelGGL(vt_swiglu_pair_tail_kernel<P>, dim3(gm_blocks((size_t)rows * tw / 8)), dim3(256), 0, g_vt.stream, \
+#define CALL(P) hipLaunchKernelGGL(vt_swiglu_pair_tail_kernel<P>, dim3((tw / 8 + 255) / 256, rows < 65535 ? rows : 65535), dim3(256), 0, g_vt.stream, \
                                    d_hi, d_lo, ldh, h_col0, d_tail, stride, rows, tw)
     GM_BY_PLANES(planes, CALL);
 #undef CALL

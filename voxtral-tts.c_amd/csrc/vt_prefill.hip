@@ -97,14 +97,6 @@ struct pa_rows {
     int start, kv_rows;
 };
 
-/* (a clamped size is made by a vector instruction; without the move to a scalar register each request becomes a loop over the lanes' descriptors) */
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t pa_buffer(const void *p, int bytes) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, __builtin_amdgcn_readfirstlane(bytes), 0x00020000);
-}
-__device__ __forceinline__ f32x4 pa_load(__amdgpu_buffer_rsrc_t r, int at) {
-    return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, at, 0, 0));
-}
-
 /* 256 threads make the K planes of tile `tile` of kv head kvh at Kt (threads 0..127) and its V planes at Vt (threads 128..255); of the
  * rows from `start` on, first .. first + n - 1 are appended to the cache. */
 template <class PTR>
@@ -120,19 +112,19 @@ __device__ __forceinline__ void pa_make_tile(PTR Kt, PTR Vt, const pa_rows &in, 
     const int at = (row0 - f0) * (VT_QKV_DIM * 4) + (wide + 4 * cg) * 4;
     auto off = [](int i, int pitch) { return (8 * (i >> 2) + (i & 3)) * pitch; };
     f32x4 r8[8], cs[8], w[3][8];
-    const __amdgpu_buffer_rsrc_t d0 = pa_buffer(fresh, fresh_bytes);
+    const __amdgpu_buffer_rsrc_t d0 = vt_buffer(fresh, fresh_bytes);
     /* (a caller's own K and V may have more rows than the table: nothing of it is read for rows that are not rotated) */
-    const __amdgpu_buffer_rsrc_t dc = pa_buffer(in.rope + (size_t)t0 * VT_HEAD_DIM, is_v || fresh_bytes == 0 ? 0 : min(in.kv_rows - t0, 32) * VT_HEAD_DIM * 4);
+    const __amdgpu_buffer_rsrc_t dc = vt_buffer(in.rope + (size_t)t0 * VT_HEAD_DIM, is_v || fresh_bytes == 0 ? 0 : min(in.kv_rows - t0, 32) * VT_HEAD_DIM * 4);
 #pragma unroll
-    for (int i = 0; i < 8; i++) r8[i] = pa_load(d0, at + off(i, VT_QKV_DIM * 4));
+    for (int i = 0; i < 8; i++) r8[i] = vt_buffer_ld4(d0, at + off(i, VT_QKV_DIM * 4));
 #pragma unroll
-    for (int i = 0; i < 8; i++) cs[i] = pa_load(dc, (row0 - t0) * (VT_HEAD_DIM * 4) + 16 * cg + off(i, VT_HEAD_DIM * 4));
+    for (int i = 0; i < 8; i++) cs[i] = vt_buffer_ld4(dc, (row0 - t0) * (VT_HEAD_DIM * 4) + 16 * cg + off(i, VT_HEAD_DIM * 4));
     for (int p = 1; p < planes; p += 3) {
 #pragma unroll
         for (int z = 0; z < 3; z++) {
-            const __amdgpu_buffer_rsrc_t d = pa_buffer(fresh + (size_t)min(p + z, planes - 1) * in.plane_stride, p + z < planes ? fresh_bytes : 0);
+            const __amdgpu_buffer_rsrc_t d = vt_buffer(fresh + (size_t)min(p + z, planes - 1) * in.plane_stride, p + z < planes ? fresh_bytes : 0);
 #pragma unroll
-            for (int i = 0; i < 8; i++) w[z][i] = pa_load(d, at + off(i, VT_QKV_DIM * 4));
+            for (int i = 0; i < 8; i++) w[z][i] = vt_buffer_ld4(d, at + off(i, VT_QKV_DIM * 4));
         }
 #pragma unroll
         for (int z = 0; z < 3; z++)
@@ -151,14 +143,14 @@ __device__ __forceinline__ void pa_make_tile(PTR Kt, PTR Vt, const pa_rows &in, 
         }
     }
     const int s0 = max(t0, first);
-    const __amdgpu_buffer_rsrc_t ds = pa_buffer(cache + (size_t)s0 * VT_KV_DIM, max(min(min(first + n, in.kv_rows), t0 + 32) - s0, 0) * VT_KV_DIM * 4);
+    const __amdgpu_buffer_rsrc_t ds = vt_buffer(cache + (size_t)s0 * VT_KV_DIM, max(min(min(first + n, in.kv_rows), t0 + 32) - s0, 0) * VT_KV_DIM * 4);
 #pragma unroll
     for (int i = 0; i < 8; i++)
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, r8[i]), ds, (row0 - s0) * (VT_KV_DIM * 4) + col * 4 + off(i, VT_KV_DIM * 4), 0, 0);
+        vt_buffer_st4(ds, (row0 - s0) * (VT_KV_DIM * 4) + col * 4 + off(i, VT_KV_DIM * 4), r8[i]);
     if (t0 < in.start) {                                 /* earlier rows */
-        const __amdgpu_buffer_rsrc_t d = pa_buffer(cache + (size_t)t0 * VT_KV_DIM, min(in.start - t0, 32) * VT_KV_DIM * 4);
+        const __amdgpu_buffer_rsrc_t d = vt_buffer(cache + (size_t)t0 * VT_KV_DIM, min(in.start - t0, 32) * VT_KV_DIM * 4);
 #pragma unroll
-        for (int i = 0; i < 8; i++) w[0][i] = pa_load(d, (row0 - t0) * (VT_KV_DIM * 4) + col * 4 + off(i, VT_KV_DIM * 4));
+        for (int i = 0; i < 8; i++) w[0][i] = vt_buffer_ld4(d, (row0 - t0) * (VT_KV_DIM * 4) + col * 4 + off(i, VT_KV_DIM * 4));
 #pragma unroll
         for (int i = 0; i < 8; i++) r8[i] += w[0][i];
     }
