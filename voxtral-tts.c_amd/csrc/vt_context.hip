@@ -139,6 +139,7 @@ static int init_context(int kv_cache_max) {
         VT_TRY(hipMemset(*bufs[i].p, 0, bufs[i].bytes));
     }
     g_vt.bar_epoch = 0;
+    VT_TRY(hipHostMalloc((void **)&g_vt.h_rows, sizeof(float) * VT_DIM * (kv_cache_max < VT_PIN_ROWS ? kv_cache_max : VT_PIN_ROWS), hipHostMallocDefault));
     VT_TRY(hipHostMalloc((void **)&g_vt.h_pin, sizeof(float) * VT_PIN_FLOATS, hipHostMallocDefault));
     if (vt_gemm_row_major_prepare()) return -1;
     VT_TRY(hipDeviceSynchronize());
@@ -214,6 +215,7 @@ static void teardown(void) {
     for (size_t i = 0; i < sizeof ptrs / sizeof ptrs[0]; i++)
         if (ptrs[i]) (void)hipFree(ptrs[i]);
     if (g_vt.h_pin) (void)hipHostFree(g_vt.h_pin);
+    if (g_vt.h_rows) (void)hipHostFree(g_vt.h_rows);
     if (g_vt.ev0) (void)hipEventDestroy(g_vt.ev0);
     if (g_vt.ev1) (void)hipEventDestroy(g_vt.ev1);
     if (g_vt.stream) (void)hipStreamDestroy(g_vt.stream);

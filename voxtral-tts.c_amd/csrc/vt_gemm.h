@@ -61,9 +61,9 @@ void vt_launch_swiglu_pair_tail(uint16_t *d_hi, uint16_t *d_lo, int ldh, int h_c
                                 size_t stride, int rows, int tw);
 /* n even */
 void vt_launch_split(uint16_t *d_hi, uint16_t *d_lo, const float *d_x, size_t n);
-/* rows of 3072: x += the product (cuts > 0; one plane below col0, the sum of `cuts` from there on), then planes
- * of rmsnorm(x)*w (d_w != NULL) */
-void vt_launch_residual_norm_split(float *d_x, const float *d_part, int col0, int cuts, size_t part_stride,
+/* rows of 3072: x = x_in (d_x itself, or rows in memory that the device reads) + the product (cuts > 0; one plane below col0, the
+ * sum of `cuts` from there on), then planes of rmsnorm(x)*w (d_w != NULL) */
+void vt_launch_residual_norm_split(float *d_x, const float *x_in, const float *d_part, int col0, int cuts, size_t part_stride,
                                    const float *d_w, uint16_t *d_hi, uint16_t *d_lo, int rows);
 /* n_out a multiple of 4, tail_col0 of 8: planes of silu(gate)*up from interleaved (gate, up) pairs */
 void vt_launch_swiglu_split(uint16_t *d_hi, uint16_t *d_lo, const float *d_gu, size_t n_out, int tail_col0,

@@ -232,6 +232,7 @@ static_assert(VT_MAX_CUTS == 8, "GM_BY_PLANES");
 /* One workgroup per row of 3072 floats (256 threads x 12):
  *   x[row] += part[0][row] (+ part[1][row] + ... for the columns from col0 on)   (C > 0 cuts; fixed order)
  *   (hi, lo)[row] = split(rmsnorm(x[row]) * w)                                   (w != NULL)
+ * x before the sum comes from x_in: x itself or, for a prefill's input rows, host memory.
  * The residual add and the normalisation of voxtral_tts_llm.c:332-336,354 /
  * :338-341 in one pass over the row.  Up to a few hundred rows a launch is one chain of memory latencies per
  * workgroup, so everything is requested in front of the first sum;
@@ -239,7 +240,7 @@ static_assert(VT_MAX_CUTS == 8, "GM_BY_PLANES");
  * prefill of 37 / 226 / 512 / 1531 rows 2632 / 4414 / 7236 / 20457 -> 2481 / 4326 / 7186 / 20181, results the same. */
 template <int C>
 __global__ void __launch_bounds__(256)
-vt_residual_norm_split_kernel(float *x, const float *part, int col0, size_t part_stride,
+vt_residual_norm_split_kernel(float *x, const float *x_in, const float *part, int col0, size_t part_stride,
                               const float *w, uint16_t *hi, uint16_t *lo, float eps) {
     /* a thread owns 4 consecutive columns at 4 (t + 256 j): 16-byte loads and stores, 8-byte plane
      * stores (a quarter of the memory instructions of element-wise accesses) */
@@ -250,7 +251,7 @@ vt_residual_norm_split_kernel(float *x, const float *part, int col0, size_t part
     const int at = 16 * (int)threadIdx.x;
     f32x4 v[NJ], g[NJ], p[NJ][C > 0 ? C : 1];
 #pragma unroll
-    for (int j = 0; j < NJ; j++) v[j] = vt_buffer_ld4(dx, at + 4096 * j);
+    for (int j = 0; j < NJ; j++) v[j] = vt_buffer_ld4(vt_buffer(x_in + row * VT_DIM, VT_DIM * 4), at + 4096 * j);
 #pragma unroll
     for (int s = 0; s < C; s++) {
         /* the planes behind the first have the columns from col0 on, and zeros for the others */
@@ -276,8 +277,8 @@ vt_residual_norm_split_kernel(float *x, const float *part, int col0, size_t part
             }
             a.x = __fadd_rn(a.x, q.x); a.y = __fadd_rn(a.y, q.y);
             a.z = __fadd_rn(a.z, q.z); a.w = __fadd_rn(a.w, q.w);
-            vt_buffer_st4(dx, at + 4096 * j, a);
         }
+        if (C > 0 || x != x_in) vt_buffer_st4(dx, at + 4096 * j, a);
         v[j] = a;
         ss = fmaf(a.x, a.x, ss); ss = fmaf(a.y, a.y, ss);
         ss = fmaf(a.z, a.z, ss); ss = fmaf(a.w, a.w, ss);
@@ -299,9 +300,9 @@ vt_residual_norm_split_kernel(float *x, const float *part, int col0, size_t part
     }
 }
 
-void vt_launch_residual_norm_split(float *d_x, const float *d_part, int col0, int cuts, size_t part_stride,
+void vt_launch_residual_norm_split(float *d_x, const float *x_in, const float *d_part, int col0, int cuts, size_t part_stride,
                                    const float *d_w, uint16_t *d_hi, uint16_t *d_lo, int rows) {
-#define CALL(C) hipLaunchKernelGGL(vt_residual_norm_split_kernel<C>, dim3(rows), dim3(256), 0, g_vt.stream, d_x, d_part, \
+#define CALL(C) hipLaunchKernelGGL(vt_residual_norm_split_kernel<C>, dim3(rows), dim3(256), 0, g_vt.stream, d_x, x_in, d_part, \
                                    col0, part_stride, d_w, d_hi, d_lo, VT_EPS)
     if (cuts <= 0) CALL(0);
     else GM_BY_PLANES(cuts, CALL);

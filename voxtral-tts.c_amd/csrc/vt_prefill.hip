@@ -15,6 +15,7 @@
 #include "vt_requests.h"
 
 #include <math.h>
+#include <string.h>
 
 
 /* ---- causal attention, 32 query rows x 32 keys per matrix-core tile ----------------
@@ -522,6 +523,29 @@ void vt_launch_prefill_attention(float *d_out, uint16_t *d_hi, uint16_t *d_lo, c
 
 /* ---- backbone prefill ------------------------------------------------------------ */
 
+/* The input rows -> x and the planes of their RMSNorm.  Pageable rows of a longer prompt go piece by piece through pinned memory that the
+ * kernel reads itself, a launch per piece, while the next piece is copied: a prefill of 226 / 512 / 1531 rows takes 80 / 210 / 930 us
+ * longer than one of rows on the device; 140 / 290 / 1000 with the runtime's own staging in front of the first kernel, which up to PF_STAGED_ROWS
+ * rows is as fast (30 us at 37).  What is left is the copy, 20 GB/s from memory that is in no cache; three more threads copying
+ * made it 410 us at 800 rows and 440 at 1000, as long, and 570 to 690 at 1531: not kept. */
+#define PF_STAGED_ROWS 96
+#define PF_PIECE_ROWS 64
+static int pf_take_rows(float *x, const float *rows, int n, uint16_t *hi, uint16_t *lo) {
+    const float *norm = g_vt.h_layers[0].attn_norm;
+    if (n <= PF_STAGED_ROWS || n > VT_PIN_ROWS || !vt_pageable(rows)) {
+        VT_TRY(hipMemcpyAsync(x, rows, sizeof(float) * VT_DIM * n, hipMemcpyDefault, g_vt.stream));
+        vt_launch_residual_norm_split(x, x, NULL, 0, 0, 0, norm, hi, lo, n);
+        return 0;
+    }
+    for (int i = 0; i < n; i += PF_PIECE_ROWS) {
+        const int m = n - i < PF_PIECE_ROWS ? n - i : PF_PIECE_ROWS;
+        const size_t at = (size_t)i * VT_DIM;
+        memcpy(g_vt.h_rows + at, rows + at, sizeof(float) * VT_DIM * m);
+        vt_launch_residual_norm_split(x + at, g_vt.h_rows + at, NULL, 0, 0, 0, norm, hi + at, lo + at, m);
+    }
+    return 0;
+}
+
 extern "C" void tts_hip_llm_prefill_out(const float *embeds, int seq_len, int start_pos, float *out_x) {
     if (!g_vt.initialized || g_vt.n_dec_layers < 1) { vt_set_error("tts_hip_llm_prefill: no weights uploaded"); return; }
     if (seq_len < 1 || start_pos < 0 || start_pos + seq_len > g_vt.kv_max) {
@@ -566,8 +590,7 @@ extern "C" void tts_hip_llm_prefill_out(const float *embeds, int seq_len, int st
     uint16_t *hi = (uint16_t *)(tail + n_tail), *lo = hi + n_plane, *h_hi = lo + n_plane, *h_lo = h_hi + n_plane;
     const size_t ps = S * VT_DIM;
 
-    VT_TRYV(hipMemcpyAsync(x, embeds, sizeof(float) * n_x, hipMemcpyDefault, st));
-    vt_launch_residual_norm_split(x, NULL, 0, 0, 0, g_vt.h_layers[0].attn_norm, hi, lo, seq_len);
+    if (pf_take_rows(x, embeds, seq_len, hi, lo)) return;
     for (int l = 0; l < g_vt.n_dec_layers; l++) {
         const vt_layer_dev *L = &g_vt.h_layers[l];
         float *kc = g_hip.kv_cache_k_gpu + (size_t)l * g_vt.kv_max * VT_KV_DIM;
@@ -589,7 +612,7 @@ extern "C" void tts_hip_llm_prefill_out(const float *embeds, int seq_len, int st
         pa_launch_layer(hi, lo, wide, pq.col0, pq.cuts, S * VT_QKV_DIM, kc, vc, img, seq_len, start_pos);
         if (frag) vt_launch_gemm_frag(part, VT_DIM, ps, hi, lo, F->wo, seq_len, VT_DIM, VT_Q_DIM, po);
         else vt_launch_gemm(part, hi, lo, L->wo, seq_len, VT_DIM, VT_Q_DIM, po.cuts);
-        vt_launch_residual_norm_split(x, part, po.col0, po.cuts, ps, L->ffn_norm, hi, lo, seq_len);
+        vt_launch_residual_norm_split(x, x, part, po.col0, po.cuts, ps, L->ffn_norm, hi, lo, seq_len);
         if (frag) {
             vt_launch_gemm_frag_swiglu(h_hi, h_lo, VT_FFN, tail, hi, lo, F->w13, seq_len, 2 * VT_FFN, VT_DIM, pg);
         } else {
@@ -601,10 +624,11 @@ extern "C" void tts_hip_llm_prefill_out(const float *embeds, int seq_len, int st
         if (frag) vt_launch_gemm_frag(part, VT_DIM, ps, h_hi, h_lo, F->w2, seq_len, VT_DIM, VT_FFN, pd);
         else vt_launch_gemm(part, h_hi, h_lo, L->w2, seq_len, VT_DIM, VT_FFN, pd.cuts);
         const float *next_norm = l + 1 < g_vt.n_dec_layers ? g_vt.h_layers[l + 1].attn_norm : NULL;
-        vt_launch_residual_norm_split(x, part, pd.col0, pd.cuts, ps, next_norm, hi, lo, seq_len);
+        vt_launch_residual_norm_split(x, x, part, pd.col0, pd.cuts, ps, next_norm, hi, lo, seq_len);
     }
-    VT_TRYV(hipGetLastError());
-    VT_TRYV(hipStreamSynchronize(st));
+    const hipError_t launched = hipGetLastError();
+    VT_TRYV(hipStreamSynchronize(st));    /* in any case: the pinned rows are free for the next call */
+    VT_TRYV(launched);
     if (out_x) VT_TRYV(hipMemcpy(out_x, x, sizeof(float) * n_x, hipMemcpyDefault));
 }
 

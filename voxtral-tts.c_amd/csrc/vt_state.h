@@ -21,6 +21,8 @@
 #define VT_SEM_PADDED 8320
 #define VT_SEM_VALID_END 8194     /* 2 special + 8192 codes */
 
+#define VT_PIN_ROWS 2048          /* 25 MB */
+
 /* Second copy of a backbone layer's four matrices, in the order the 128 x 256 tile product reads them
  * (vt_launch_frag_layout); the decode step streams the row-major copy. */
 struct vt_layer_frag { uint16_t *wqkv, *wo, *w13, *w2; };
@@ -79,6 +81,7 @@ struct vt_state {
     unsigned long long bar_timeout; /* spin budget of a barrier in 100 MHz ticks; 0 = default */
     int *d_abort;
     uint16_t *d_dummy;            /* small resident block requested in place of a layer beyond the last */
+    float *h_rows;                /* pinned: a prefill's input rows on their way to the device, up to VT_PIN_ROWS */
     float *h_pin;                 /* pinned staging: [3072 in][3072 out + flag], and a frame's hidden state, noise and results */
 
     /* generic scratch (prefill / acoustic / linear) */
