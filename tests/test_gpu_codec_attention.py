@@ -50,3 +50,26 @@ def test_an_odd_token_count_on_workgroups_of_16():
         close(whole[tail], part[tail])
     finally:
         hip.close()
+
+
+@pytest.mark.parametrize("n_frames", [513, 1030, 2049])
+def test_four_tokens_to_a_lane_group(n_frames):
+    """Rows that give two tokens to a lane group more workgroups than compute units: 4104 and 8240 rows in the last
+    stage, and 4098 already in the second, where the last lane group has two of its four.  With windows of 2, 4,
+    8 and 16 a sample depends on fewer than 40 frames in front of it, so the ends of a long decode are those of short
+    ones, up to the sums of another plan."""
+    hc = K.HostCodec(8, distinct_layers=2)
+    cs = hc.struct()
+    hip = H.Hip(kv_max=8)
+    try:
+        assert hip.lib.tts_hip_upload_codec_weights(C.addressof(cs)) == 0, hip.lib.tts_hip_last_error()
+        codes = K.random_codes(n_frames, 78)
+        print(f"codec of {n_frames} frames", flush=True)
+        whole = hip_decode(hip, codes)
+        head, tail = hip_decode(hip, codes[:100]), hip_decode(hip, codes[-100:])
+        close(whole[:head.size], head)
+        close(whole[-60 * 1920:], tail[-60 * 1920:])
+        mid = n_frames // 2
+        close(whole[(mid - 60) * 1920:mid * 1920], hip_decode(hip, codes[mid - 100:mid])[-60 * 1920:])
+    finally:
+        hip.close()

@@ -238,72 +238,71 @@ struct cd_softmax {
     }
 };
 
-/* Many tokens: one workgroup for 16 of them, wave h for head h, eight lanes for two neighbouring tokens, which share
- * all but two of their keys.  The rows of the next key are requested in front of the work on this one; with its
- * value rows requested late instead (118 registers, two workgroups to a CU) the eight launches of 1003 frames took
- * 258 us instead of 196: a workgroup's rows in flight are twice the L1 already.  us per launch at 4012 rows, window
- * 8 / 8024 rows, window 16: 42 / 96 with the kernel below, 20 / 59 with this one. */
-/* Fewer rows than this: the kernel below.  Measured, this kernel / the one below: 848 rows, window 8, 11.3 / 11.3
+/* Many tokens: one workgroup for 8 NT of them, wave h for head h, eight lanes for NT neighbouring tokens, which share
+ * all but NT of their keys: a key's rows are read once per NT tokens, and that reading (L2: what a CU's waves have in
+ * flight is twice its L1) bounds the kernel.  The rows of the next key are requested in front of the work on this one;
+ * with its value rows requested late instead (118 registers at NT = 2, two workgroups to a CU) the eight launches of
+ * 1003 frames took 258 us instead of 196.  Tokens past the last one work as the last one and store nothing. */
+/* Fewer rows than this: the kernel below.  Measured, NT = 2 / the one below: 848 rows, window 8, 11.3 / 11.3
  * us; 1003 rows, window 2, 8 / 8.5; 1696 rows, window 16, 17.5 / 23.4; 168 rows, window 16, 16 / 5.5. */
-#define CD_ATT_TOKENS 16
 #define CD_ATT_SPLIT_BELOW 1024
+/* NT = 4 has one workgroup to a CU (233 registers) that takes 1.3 .. 1.8 times as long as two tokens' does, so it pays
+ * from where NT = 2 has more than one to a CU on.  Measured, us, NT = 2 / 4: 2800 rows, window 8, 14.8 / 18.8; 4000,
+ * window 8, 20 / 23; 4008, window 16, 30.4 / 29.7; 5600, window 16, 48 / 40; 6000, window 8, 33 / 30; 8024, window 16,
+ * 67 / 56; 12000, window 16, 106 / 86. */
+template <int NT>
 __global__ void __launch_bounds__(64 * CD_HEADS)
 vt_codec_attention_kernel(cd_planes out, const float *__restrict__ qkv, int T, int window,
                           const float *__restrict__ slopes, float scale) {
-    __shared__ float red[CD_HEADS][CD_ATT_TOKENS];
+    __shared__ float red[CD_HEADS][8 * NT];
     const int h = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane >> 3, sub = lane & 7;
-    const int i0 = blockIdx.x * CD_ATT_TOKENS + 2 * g;
-    const bool live[2] = {i0 < T, i0 + 1 < T};
-    const int a = live[0] ? i0 : T - 1, b = a + 1;
+    const int i0 = (blockIdx.x * 8 + g) * NT;
     const float slope = slopes[h];
     const float *base = qkv + h * CD_HEAD_DIM + 4 * sub;
     auto row = [&](int j, int part) { return cd_load_row(base + (size_t)j * (3 * CD_DIM) + part * CD_DIM); };
-    const cd_head_row qa = row(a, 0), qb = row(live[1] ? b : a, 0);
-    const int ja = (window > 0 && a - window + 1 > 0) ? a - window + 1 : 0, jb = (window > 0 && b - window + 1 > 0) ? b - window + 1 : 0;
-    cd_softmax sa, sb;
-    int j = ja;
-    cd_head_row k = row(j, 1), v = row(j, 2);
-    if (jb > ja) {                                /* the one key that only the first token sees */
-        const int nx = j < a ? j + 1 : live[1] ? b : a;
-        const cd_head_row nk = row(nx, 1), nv = row(nx, 2);
-        sa.add(cd_row_dot(qa, k) * scale + slope * (float)(j - a), v);
-        k = nk; v = nv;
-        j++;
-    }
-    for (; j <= a; j++) {
-        const int nx = j < a ? j + 1 : live[1] ? b : a;
-        const cd_head_row nk = row(nx, 1), nv = row(nx, 2);
-        const float ka = cd_row_dot(qa, k), kb = cd_row_dot(qb, k);
-        sa.add(ka * scale + slope * (float)(j - a), v);
-        sb.add(kb * scale + slope * (float)(j - b), v);
-        k = nk; v = nv;
-    }
-    if (live[1]) sb.add(cd_row_dot(qb, k) * scale, v);      /* the second token's own key */
-    cd_softmax *st[2] = {&sa, &sb};
+    int tok[NT], from[NT];
+    cd_head_row q[NT];
+    cd_softmax st[NT];
 #pragma unroll
-    for (int t = 0; t < 2; t++) {
-        const float inv = st[t]->se > 0.f ? 1.0f / st[t]->se : 1.0f;
+    for (int t = 0; t < NT; t++) {
+        tok[t] = min(i0 + t, T - 1);
+        from[t] = window > 0 && tok[t] - window + 1 > 0 ? tok[t] - window + 1 : 0;
+        q[t] = row(tok[t], 0);
+    }
+    cd_head_row k = row(from[0], 1), v = row(from[0], 2);
+    for (int j = from[0]; j <= tok[NT - 1]; j++) {
+        const int nx = min(j + 1, tok[NT - 1]);
+        const cd_head_row nk = row(nx, 1), nv = row(nx, 2);
+#pragma unroll
+        for (int t = 0; t < NT; t++)
+            if (j >= from[t] && j <= tok[t])
+                st[t].add(cd_row_dot(q[t], k) * scale + slope * (float)(j - tok[t]), v);
+        k = nk; v = nv;
+    }
+#pragma unroll
+    for (int t = 0; t < NT; t++) {
+        const float inv = st[t].se > 0.f ? 1.0f / st[t].se : 1.0f;
         float m = 0.f;
 #pragma unroll
         for (int e = 0; e < 4; e++) {
-            st[t]->o.v[e] *= inv;
-            m = fmaxf(m, cd_max4(st[t]->o.v[e]));
+            st[t].o.v[e] *= inv;
+            m = fmaxf(m, cd_max4(st[t].o.v[e]));
         }
         m = fmaxf(m, vt_dpp<0xB1>(m));
         m = fmaxf(m, vt_dpp<0x4E>(m));
         m = fmaxf(m, vt_dpp<0x141>(m));
-        if (sub == 0) red[h][2 * g + t] = m;
+        if (sub == 0) red[h][NT * g + t] = m;
     }
     __syncthreads();
 #pragma unroll
-    for (int t = 0; t < 2; t++) {
+    for (int t = 0; t < NT; t++) {
         float m = 0.f;
 #pragma unroll
-        for (int w = 0; w < CD_HEADS; w++) m = fmaxf(m, red[w][2 * g + t]);
+        for (int w = 0; w < CD_HEADS; w++) m = fmaxf(m, red[w][NT * g + t]);
         const int ex = vt_f16_exp(m);
-        if (live[t]) {
+        if (i0 + t < T) {
 #pragma unroll
-            for (int e = 0; e < 4; e++) cd_put4(out, (size_t)(i0 + t) * CD_DIM + h * CD_HEAD_DIM + 32 * e + 4 * sub, st[t]->o.v[e], ex);
+            for (int e = 0; e < 4; e++) cd_put4(out, (size_t)(i0 + t) * CD_DIM + h * CD_HEAD_DIM + 32 * e + 4 * sub, st[t].o.v[e], ex);
             if (h == 0 && sub == 0) out.exp[i0 + t] = ex;
         }
     }
@@ -722,9 +721,10 @@ static cd_product cd_enqueue(const int *codes, int n_frames) {
 #undef CALL
         if (T < CD_ATT_SPLIT_BELOW)
             hipLaunchKernelGGL(vt_codec_attention_split_kernel, dim3(T), dim3(64 * CD_HEADS), 0, g_vt.stream, g_cd.planes, g_cd.qkv, T, l->window, g_cd.slopes, scale);
+        else if ((T + 15) / 16 <= g_vt.n_cu)
+            hipLaunchKernelGGL(vt_codec_attention_kernel<2>, dim3((T + 15) / 16), dim3(64 * CD_HEADS), 0, g_vt.stream, g_cd.planes, g_cd.qkv, T, l->window, g_cd.slopes, scale);
         else
-            hipLaunchKernelGGL(vt_codec_attention_kernel, dim3((T + CD_ATT_TOKENS - 1) / CD_ATT_TOKENS), dim3(64 * CD_HEADS), 0, g_vt.stream, g_cd.planes,
-                               g_cd.qkv, T, l->window, g_cd.slopes, scale);
+            hipLaunchKernelGGL(vt_codec_attention_kernel<4>, dim3((T + 31) / 32), dim3(64 * CD_HEADS), 0, g_vt.stream, g_cd.planes, g_cd.qkv, T, l->window, g_cd.slopes, scale);
         p = cd_gemm(T, l->wo);
         cd_row(p, false, g_cd.x, NULL, l->attn_scale, l->ffn_norm);
         p = cd_gemm(T, l->w13);
