@@ -47,3 +47,28 @@ def test_rows(hip, m, n, k, noalloc):
     assert np.all(np.abs(got[:m] - want) <= tol), float((np.abs(got[:m] - want) / tol).max())
     for b in (dx, dW, dy):
         b.free()
+
+
+@pytest.mark.parametrize("m", [64, 128])
+def test_rows_of_more_than_32_bits_of_bytes(hip, m):
+    """8,388,864 columns: 64 and 128 rows of results are 2 and 4 GiB, more than a tile's rows may be apart where one
+    descriptor stores them.  The weights repeat 99 times.  Bound as above."""
+    n0, reps, k = 84736, 99, 64
+    n = n0 * reps
+    W = S.bf16_normal((n0, k), 5301)
+    x = S.f32_normal((m, k), 5302)
+    want = x.astype(np.float64) @ S.bf16_to_f32(W).astype(np.float64).T
+    size = np.abs(x).astype(np.float64) @ np.abs(S.bf16_to_f32(W)).astype(np.float64).T
+    dx, dW = H.DevBuf.from_numpy(hip.lib, x), H.DevBuf.from_numpy(hip.lib, np.tile(W, (reps, 1)))
+    dy = H.DevBuf.from_numpy(hip.lib, np.full((m + 1, n), 7.0, np.float32))
+    print(f"{m} rows of {n} columns", flush=True)
+    hip.lib.tts_hip_linear_bf16(dy.ptr, dx.ptr, None, m, k, n, dW.ptr)
+    hip.lib.tts_hip_sync()
+    hip.check()
+    got = dy.to_numpy(np.float32, (m + 1, n))
+    assert np.all(got[m] == 7.0)
+    tol = (2.0 ** -24 * (k / 16 + 40) + 2.0 ** -16) * size
+    for row in sorted({0, 1, 31, 32, 63, m // 2, m - 2, m - 1}):
+        assert np.all(np.abs(got[row].reshape(reps, n0) - want[row]) <= tol[row]), row
+    for b in (dx, dW, dy):
+        b.free()

@@ -448,10 +448,13 @@ static int linear_mfma_plan(const float *d_y, const float *d_x, const uint16_t *
     p->bytes = equal;
     const float equal_us = vt_gemm_equal_us(seq_len, out_dim, in_dim, p->equal_cuts);
     const int equal_cuts = p->equal_cuts;
+    /* strips and the backbone's tiles store the rows of a tile through one descriptor, whose offsets have 32 bits; the tiles of
+     * 128 x 128 have an address per row */
+    const bool stores_fit = (seq_len < 128 ? seq_len : 128) * (long long)out_dim * (long long)sizeof(float) <= 0x7fffffff;
     for (int most = VT_MAX_CUTS;; most = p->tiles.cuts - 1) {
         float us;
         p->tiles = vt_gemm_row_major_plan(seq_len, out_dim, in_dim, most, &us);
-        p->equal_cuts = us < equal_us ? 0 : equal_cuts;
+        p->equal_cuts = us < equal_us && stores_fit ? 0 : equal_cuts;
         const size_t bytes = linear_part_bytes(*p, seq_len, out_dim) + planes;
         p->bytes = bytes > equal ? bytes : equal;
         if (p->equal_cuts || p->tiles.cuts == 1 || equal > VT_STATIC_SCRATCH_BYTES || bytes <= VT_STATIC_SCRATCH_BYTES) return 1;
