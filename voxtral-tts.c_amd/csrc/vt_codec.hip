@@ -16,7 +16,7 @@
  *     = w[ic][oc][p + 2q].  Output (taps 7): W'[k * 256 + oc][ic] = w[oc][ic][k].  The sums are those
  *     of a product over shifted copies of the rows, in two and seven pieces, without four launches that
  *     write the copies (100 us of a 1003-frame decode); us per decode of 21 / 212 / 1003 frames:
- *     731 / 1595 / 4983 -> 712 / 1558 / 4890.
+ *     731 / 1595 / 4983 -> 712 / 1558 / 4890 (584 / 1359 / 4212 now, with the products and row kernels as they are).
  * Every product runs on the fp16 matrix cores with both operands as two fp16 planes
  * (vt_codec_gemm.hip); whoever produces a product's input leaves it as planes with one exponent
  * per row.  Where a launch would not fill the chip K is cut, and the kernel that reads the
@@ -804,7 +804,7 @@ extern "C" void tts_hip_codec_decode(const int *codes, int n_frames, float **out
     /* Codes and samples cross through pinned memory that the kernels read and write themselves; the caller's buffer is filled
      * part by part behind the last kernel's launches.  Where the codes and the waveform were copied
      * from and into pageable memory, calls of 2 / 21 / 212 / 1003 frames took 508 / 737 / 1630 / 5020 us; 453 / 695 / 1596 / 4791
-     * now, of which 8 / 21 / 95 / 273 behind the device's work. */
+     * with this, of which 8 / 21 / 95 / 273 behind the device's work. */
     float *wave = (float *)g_cd.host;
     int *host_codes = (int *)(wave + n);
     if (vt_pageable(codes)) memcpy(host_codes, codes, code_bytes);

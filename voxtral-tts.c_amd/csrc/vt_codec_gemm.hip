@@ -15,7 +15,7 @@
  * the weights 2^20 / 2^24 times the others, 1.4e-7 / 4.4e-7 at K = 1024 (2.1e-7 / 4.6e-7 at 4096); without it the operands alone
  * leave 2.4e-6 / 3.7e-5 at K = 1024.  hi times 2^-6, which it takes, costs 0.7 / 1.6 / 1.5 % of a decode of 21 / 212 / 1003 frames.
  * Rates, TFLOP/s of the product itself (v_mfma_f32_32x32x2f32 in 128 x 128 tiles before: 75 .. 105): gate|up
- * 8192 x 1024 at 212 / 848 / 1696 / 8024 rows 152 / 281 / 292 / 331, down 1024 x 4096 105 / 242 / 282 / 391.
+ * 8192 x 1024 at 212 / 848 / 1696 / 8024 rows 170 / 329 / 329 / 377, down 1024 x 4096 125 / 254 / 323 / 409.
  */
 #include "vt_gemm_tiles.h"
 
