@@ -34,6 +34,24 @@ def test_windows_and_token_counts(n_frames, windows):
         S.oracle().orc_set_threads(1)
 
 
+@pytest.mark.parametrize("n_frames", [151, 212, 255])
+def test_v_where_the_product_left_it(n_frames):
+    """From 1024 rows on v is read from the q|k|v product's result where its columns are whole or in one plane (1208 and
+    1696 rows here, 2040 in the last stage of 255 frames); fewer rows have it copied or summed from several planes."""
+    S.oracle().orc_set_threads(16)
+    hc = K.HostCodec(9, distinct_layers=2)
+    cs = hc.struct()
+    hip = H.Hip(kv_max=8)
+    try:
+        assert hip.lib.tts_hip_upload_codec_weights(C.addressof(cs)) == 0, hip.lib.tts_hip_last_error()
+        codes = K.random_codes(n_frames, 90 + n_frames)
+        print(f"codec of {n_frames} frames", flush=True)
+        close(K.oracle_decode(cs, codes), hip_decode(hip, codes))
+    finally:
+        hip.close()
+        S.oracle().orc_set_threads(1)
+
+
 def test_an_odd_token_count_on_workgroups_of_16():
     """1025 rows in the first stage leave the last workgroup one token.  The decoder is causal: the samples are the
     first ones of a longer decode, up to the sums of another plan."""

@@ -143,22 +143,24 @@ vt_codec_row_kernel(float *x_out, cd_planes xn, const float *x_in, cd_product in
 }
 
 /* q|k|v [T, 3072] summed, with the RMSNorm over the whole 1024-wide q row and k row (tts_qk_norm,
- * voxtral_tts_kernels.c:351-355, eps 1e-6) when the layer has those weights. */
-template <int C>
+ * voxtral_tts_kernels.c:351-355, eps 1e-6) when the layer has those weights.  PARTS 2: q and k only, where v has nothing to be added and
+ * the attention reads it where the product left it (cd_v_rows): the kernel is bound by memory, and a decode of 1003 frames takes 4345 us
+ * instead of 4377.  Below CD_ATT_SPLIT_BELOW rows it gained nothing (21 frames 596 us, 594 without). */
+template <int C, int PARTS>
 __global__ void __launch_bounds__(256)
 vt_codec_qkv_kernel(float *__restrict__ qkv, cd_product in, const float *__restrict__ q_norm, const float *__restrict__ k_norm) {
     __shared__ float red[2][4];
     const int row = blockIdx.x, c = threadIdx.x * 4;
     const size_t at = (size_t)row * (3 * CD_DIM) + c;
-    f32x4 v[3];
-    cd_quads<C> q[3];
+    f32x4 v[PARTS];
+    cd_quads<C> q[PARTS];
 #pragma unroll
-    for (int part = 0; part < 3; part++) q[part].ask(in, row, part * CD_DIM + c);
+    for (int part = 0; part < PARTS; part++) q[part].ask(in, row, part * CD_DIM + c);
     cd_asked();
 #pragma unroll
-    for (int part = 0; part < 3; part++) v[part] = q[part].total();
+    for (int part = 0; part < PARTS; part++) v[part] = q[part].total();
 #pragma unroll
-    for (int part = 0; part < 3; part++) {
+    for (int part = 0; part < PARTS; part++) {
         const float *nw = part == 0 ? q_norm : part == 1 ? k_norm : nullptr;
         if (nw) {
             const float ss = cd_block_sum(v[part].x * v[part].x + v[part].y * v[part].y + v[part].z * v[part].z + v[part].w * v[part].w, red[part]);
@@ -167,6 +169,15 @@ vt_codec_qkv_kernel(float *__restrict__ qkv, cd_product in, const float *__restr
         }
         *(f32x4 *)(qkv + at + part * CD_DIM) = v[part];
     }
+}
+
+/* The v rows of the attention for many tokens, `stride` floats apart */
+struct cd_v_rows { const float *p; int stride; };
+/* p NULL: some of the v columns of this q|k|v product are in several planes, or whole and cut ones meet among them */
+static cd_v_rows cd_v_in_place(const cd_product &in) {
+    if (in.col0 == in.n) return cd_v_rows{in.p + 2 * CD_DIM, in.n};
+    if (in.cuts > 1 || in.col0 > 2 * CD_DIM) return cd_v_rows{NULL, 0};
+    return cd_v_rows{in.p + (size_t)in.rows * in.col0 + (2 * CD_DIM - in.col0), in.n - in.col0};
 }
 
 /* gate|up [T, 8192] -> h = silu(gate) * up [T, 4096] (tts_silu, tts_mul_inplace) as planes; one workgroup per row */
@@ -252,14 +263,15 @@ struct cd_softmax {
  * 67 / 56; 12000, window 16, 106 / 86. */
 template <int NT>
 __global__ void __launch_bounds__(64 * CD_HEADS)
-vt_codec_attention_kernel(cd_planes out, const float *__restrict__ qkv, int T, int window,
+vt_codec_attention_kernel(cd_planes out, const float *__restrict__ qkv, cd_v_rows vs, int T, int window,
                           const float *__restrict__ slopes, float scale) {
     __shared__ float red[CD_HEADS][8 * NT];
     const int h = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane >> 3, sub = lane & 7;
     const int i0 = (blockIdx.x * 8 + g) * NT;
     const float slope = slopes[h];
-    const float *base = qkv + h * CD_HEAD_DIM + 4 * sub;
+    const float *base = qkv + h * CD_HEAD_DIM + 4 * sub, *v_base = vs.p + h * CD_HEAD_DIM + 4 * sub;
     auto row = [&](int j, int part) { return cd_load_row(base + (size_t)j * (3 * CD_DIM) + part * CD_DIM); };
+    auto v_row = [&](int j) { return cd_load_row(v_base + (size_t)j * vs.stride); };
     int tok[NT], from[NT];
     cd_head_row q[NT];
     cd_softmax st[NT];
@@ -269,10 +281,10 @@ vt_codec_attention_kernel(cd_planes out, const float *__restrict__ qkv, int T, i
         from[t] = window > 0 && tok[t] - window + 1 > 0 ? tok[t] - window + 1 : 0;
         q[t] = row(tok[t], 0);
     }
-    cd_head_row k = row(from[0], 1), v = row(from[0], 2);
+    cd_head_row k = row(from[0], 1), v = v_row(from[0]);
     for (int j = from[0]; j <= tok[NT - 1]; j++) {
         const int nx = min(j + 1, tok[NT - 1]);
-        const cd_head_row nk = row(nx, 1), nv = row(nx, 2);
+        const cd_head_row nk = row(nx, 1), nv = v_row(nx);
 #pragma unroll
         for (int t = 0; t < NT; t++)
             if (j >= from[t] && j <= tok[t])
@@ -716,15 +728,20 @@ static cd_product cd_enqueue(const int *codes, int n_frames) {
     for (int li = 0; li < CD_LAYERS; li++) {
         const cd_layer_dev *l = &g_cd.layers[li];
         p = cd_gemm(T, l->wqkv);
-#define CALL(C) hipLaunchKernelGGL(vt_codec_qkv_kernel<C>, dim3(T), dim3(256), 0, g_vt.stream, g_cd.qkv, p, l->q_norm, l->k_norm)
-        CD_BY_CUTS(p.cuts, CALL);
+        cd_v_rows v = T < CD_ATT_SPLIT_BELOW ? cd_v_rows{NULL, 0} : cd_v_in_place(p);
+#define CALL(C) hipLaunchKernelGGL((vt_codec_qkv_kernel<C, 3>), dim3(T), dim3(256), 0, g_vt.stream, g_cd.qkv, p, l->q_norm, l->k_norm)
+        if (v.p) hipLaunchKernelGGL((vt_codec_qkv_kernel<1, 2>), dim3(T), dim3(256), 0, g_vt.stream, g_cd.qkv, p, l->q_norm, l->k_norm);
+        else {
+            CD_BY_CUTS(p.cuts, CALL);
+            v = cd_v_rows{g_cd.qkv + 2 * CD_DIM, 3 * CD_DIM};
+        }
 #undef CALL
         if (T < CD_ATT_SPLIT_BELOW)
             hipLaunchKernelGGL(vt_codec_attention_split_kernel, dim3(T), dim3(64 * CD_HEADS), 0, g_vt.stream, g_cd.planes, g_cd.qkv, T, l->window, g_cd.slopes, scale);
         else if ((T + 15) / 16 <= g_vt.n_cu)
-            hipLaunchKernelGGL(vt_codec_attention_kernel<2>, dim3((T + 15) / 16), dim3(64 * CD_HEADS), 0, g_vt.stream, g_cd.planes, g_cd.qkv, T, l->window, g_cd.slopes, scale);
+            hipLaunchKernelGGL(vt_codec_attention_kernel<2>, dim3((T + 15) / 16), dim3(64 * CD_HEADS), 0, g_vt.stream, g_cd.planes, g_cd.qkv, v, T, l->window, g_cd.slopes, scale);
         else
-            hipLaunchKernelGGL(vt_codec_attention_kernel<4>, dim3((T + 31) / 32), dim3(64 * CD_HEADS), 0, g_vt.stream, g_cd.planes, g_cd.qkv, T, l->window, g_cd.slopes, scale);
+            hipLaunchKernelGGL(vt_codec_attention_kernel<4>, dim3((T + 31) / 32), dim3(64 * CD_HEADS), 0, g_vt.stream, g_cd.planes, g_cd.qkv, v, T, l->window, g_cd.slopes, scale);
         p = cd_gemm(T, l->wo);
         cd_row(p, false, g_cd.x, NULL, l->attn_scale, l->ffn_norm);
         p = cd_gemm(T, l->w13);
