@@ -8,6 +8,8 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include "vt_gemm_plans.h"
+
 /* N a multiple of 128, K/splits a multiple of 64 */
 int vt_gemm_shape_ok(int M, int N, int K, int splits);
 /* d_C: `splits` planes of [M, N] fp32, plane s holds the sum over K range s */
@@ -16,12 +18,6 @@ void vt_launch_gemm(float *d_C, const uint16_t *d_Ahi, const uint16_t *d_Alo, co
 /* the same with the row pitch of C and the distance between planes given */
 void vt_launch_gemm_ex(float *d_C, int ldc, size_t plane_stride, const uint16_t *d_Ahi, const uint16_t *d_Alo,
                        const uint16_t *d_W, int M, int N, int K, int splits);
-/* How a product of the backbone is done on fragment-order weights (vt_launch_frag_layout): the columns below
- * col0 as whole tiles (one plane), the others with K in `cuts` cuts (that many partial planes, to be added in
- * order by whoever reads the result).  tm, tn: rows and columns of the tile
- * (vt_gemm_wide.hip; tm 0: vt_gemm_rows.hip).  col0 is a multiple of 128. */
-#define VT_MAX_CUTS 8
-struct vt_gemm_plan { int tm, tn, col0, cuts, row_major; };      /* row_major: W as it is (vt_gemm_row_major_plan) */
 /* K % 64 == 0; N % 256 == 0, up to 64 rows N % 96 == 0 (swiglu: % 288); swiglu: for vt_launch_gemm_frag_swiglu */
 vt_gemm_plan vt_gemm_frag_plan(int M, int N, int K, int swiglu);
 /* The same on row-major weights W[N, K], N % 128 == 0, K % 64 == 0, in at most `most` cuts: d_y [M, N]; d_part: pl.cuts planes of
@@ -39,12 +35,8 @@ void vt_launch_gemm_frag_swiglu(uint16_t *d_hhi, uint16_t *d_hlo, int ldh, float
                                 const uint16_t *d_Alo, const uint16_t *d_Wf, int M, int N, int K, const vt_gemm_plan &pl);
 /* The same for M <= 64 rows on strips of 96 columns, or 288 for the gate|up product (vt_gemm_rows.hip), weights in the same
  * fragment order: N a multiple of those; the cuts need not divide K. */
-int vt_gemm_rows_ok(int M, int N, int K);
-vt_gemm_plan vt_gemm_few_rows_plan(int N, int swiglu);
 void vt_launch_gemm_few_rows(float *d_C, int ldc, size_t plane_stride, const uint16_t *d_Ahi, const uint16_t *d_Alo,
                              const uint16_t *d_Wf, int M, int N, int K, const vt_gemm_plan &pl);
-int vt_gemm_rows_cuts(int waves, int N, int K, int most);      /* waves of a workgroup of vt_gemm_rows_kernel */
-#define VT_CODEC_ROW_WAVES 4     /* with two weight planes a wave's registers do not fit two waves per SIMD */
 /* The codec's products (vt_codec_gemm.hip): activations as two fp16 planes [M, K] with an exponent per row, weights in
  * fragment order with an exponent per column, from fp32 W[N, K] by vt_codec_weight_layout (d_Wf: 2 N K elements; 0 / -1).
  * N % 64 == 0 (more than 64 rows: % 256), K % 64 == 0.  d_C: [M, pl.col0] and, behind it, pl.cuts planes of

@@ -3,20 +3,6 @@
  */
 #include "vt_gemm_tiles.h"
 
-int vt_gemm_rows_ok(int M, int N, int K) { return M >= 1 && M <= 64 && N % GR_TN == 0 && K % 64 == 0; }
-
-int vt_gemm_rows_cuts(int nw, int N, int K, int most) {
-    /* of the cut counts that leave every CU at most one item, the fewest planes among those with the fewest
-     * K steps on the busiest wave */
-    const int tiles = N / GR_TN, steps = K / 64;
-    int best = 1, best_cost = steps;
-    for (int c = 1; c <= most && tiles * c <= g_vt.n_cu; c++) {
-        const int cost = ((steps + c - 1) / c + nw - 1) / nw;
-        if (c == 1 || cost < best_cost) { best = c; best_cost = cost; }
-    }
-    return best;
-}
-
 /* ---- the backbone: column strips of 288 or 96, the rows of a K cut shared by a workgroup -----------------------
  * With so few rows the product is a weight stream: what counts is that every CU has an equal share of the weights, and
  * moves little else.  A workgroup owns a strip of columns over a K cut, so that strips times cuts make one item per CU:
@@ -177,20 +163,11 @@ vt_gemm_strip_kernel(float *C, int ldc, size_t plane_stride, const uint16_t *Ahi
     }
 }
 
-/* Columns of a strip */
-#define GS_WIDE 288
-#define GS_NARROW 96
-
 template <int NP, int KW, bool FRAG>
 static void gs_launch(float *d_C, int ldc, size_t plane_stride, const uint16_t *d_Ahi, const uint16_t *d_Alo, const uint16_t *d_Wf, int M, int N, int K, int cuts) {
     const int tn = 32 * GS_WAVES / KW, strips = (N + tn - 1) / tn;
     hipLaunchKernelGGL((vt_gemm_strip_kernel<NP, KW, FRAG>), dim3(strips * cuts), dim3(64 * GS_WAVES), 0, g_vt.stream, d_C, ldc, plane_stride, d_Ahi, d_Alo, d_Wf, M, N, K,
                        vt_divisor_of(strips, strips * cuts), gm_cuts_of(K, cuts));
-}
-
-vt_gemm_plan vt_gemm_few_rows_plan(int N, int swiglu) {
-    const int tn = swiglu ? GS_WIDE : GS_NARROW, cuts = g_vt.n_cu / ((N + tn - 1) / tn);
-    return vt_gemm_plan{0, tn, 0, cuts < 1 ? 1 : cuts < VT_MAX_CUTS ? cuts : VT_MAX_CUTS};
 }
 
 void vt_launch_gemm_few_rows(float *d_C, int ldc, size_t plane_stride, const uint16_t *d_Ahi, const uint16_t *d_Alo,

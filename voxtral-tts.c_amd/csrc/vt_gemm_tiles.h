@@ -512,8 +512,6 @@ vt_gemm_wide_kernel(gw_list list, const uint16_t *Ahi, const uint16_t *Alo, int 
  * one and rows past M ask for nothing, without a branch (behind a branch the compiler would wait for all
  * outstanding loads).
  */
-#define GR_TN 64
-
 struct gr_list {
     float *C;                             /* cuts.n planes of [M, ldc], plane_stride floats apart */
     const uint16_t *Wf;                   /* fragment-order weights */
