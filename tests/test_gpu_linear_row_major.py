@@ -49,11 +49,12 @@ def test_rows(hip, m, n, k, noalloc):
         b.free()
 
 
-@pytest.mark.parametrize("m", [64, 128])
-def test_rows_of_more_than_32_bits_of_bytes(hip, m):
-    """8,388,864 columns: 64 and 128 rows of results are 2 and 4 GiB, more than a tile's rows may be apart where one
-    descriptor stores them.  The weights repeat 99 times.  Bound as above."""
-    n0, reps, k = 84736, 99, 64
+# Columns of which a tile's rows are more than 32 bits of bytes apart: 2 and 4 GiB of rows that exist; fewer rows, whose tiles have room for
+# rows past them at offsets beyond 2^32; the last number of columns that tiles of 96 rows can store, and the first that they cannot.
+@pytest.mark.parametrize("m,reps", [(64, 99), (128, 99), (8, 196), (16, 196), (40, 196), (8, 65), (70, 65), (70, 66)])
+def test_rows_of_more_than_32_bits_of_bytes(hip, m, reps):
+    """The weights repeat.  Bound as above."""
+    n0, k = 84736, 64
     n = n0 * reps
     W = S.bf16_normal((n0, k), 5301)
     x = S.f32_normal((m, k), 5302)
@@ -68,7 +69,7 @@ def test_rows_of_more_than_32_bits_of_bytes(hip, m):
     got = dy.to_numpy(np.float32, (m + 1, n))
     assert np.all(got[m] == 7.0)
     tol = (2.0 ** -24 * (k / 16 + 40) + 2.0 ** -16) * size
-    for row in sorted({0, 1, 31, 32, 63, m // 2, m - 2, m - 1}):
+    for row in range(m) if m < 64 else sorted({0, 1, 31, 32, 63, m // 2, m - 2, m - 1}):
         assert np.all(np.abs(got[row].reshape(reps, n0) - want[row]) <= tol[row]), row
     for b in (dx, dW, dy):
         b.free()

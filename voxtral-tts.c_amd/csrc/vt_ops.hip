@@ -423,7 +423,8 @@ void vt_launch_linear(float *d_y, const float *d_x, const uint16_t *d_W, const f
  * planes summed in a fixed order.  linear_mfma_plan says whether the shape qualifies, how the product is divided and how many
  * bytes of work area (partial planes, then the two activation planes) the launches need; linear_mfma_run queues them on that
  * work area.  The products are the backbone's strips and tiles on the caller's weights as they lie (equal_cuts 0), or tiles
- * of 128 x 128 whose K is cut into equal ranges.
+ * of 128 x 128 whose K is cut into equal ranges, the only ones with an address per row of results (of more than 4 to 67 million
+ * columns, by the rows).
  * The fixed work area of the entry point without allocation holds what equal ranges that make 192 such tiles take, and a shape
  * beyond that is refused there: where it holds that, the plan is one that fits too. */
 #define VT_STATIC_SCRATCH_BYTES ((size_t)16 << 20)
@@ -448,13 +449,10 @@ static int linear_mfma_plan(const float *d_y, const float *d_x, const uint16_t *
     p->bytes = equal;
     const float equal_us = vt_gemm_equal_us(seq_len, out_dim, in_dim, p->equal_cuts);
     const int equal_cuts = p->equal_cuts;
-    /* strips and the backbone's tiles store the rows of a tile through one descriptor, whose offsets have 32 bits; the tiles of
-     * 128 x 128 have an address per row */
-    const bool stores_fit = (seq_len < 128 ? seq_len : 128) * (long long)out_dim * (long long)sizeof(float) <= 0x7fffffff;
     for (int most = VT_MAX_CUTS;; most = p->tiles.cuts - 1) {
         float us;
         p->tiles = vt_gemm_row_major_plan(seq_len, out_dim, in_dim, most, &us);
-        p->equal_cuts = us < equal_us && stores_fit ? 0 : equal_cuts;
+        p->equal_cuts = us < equal_us ? 0 : equal_cuts;
         const size_t bytes = linear_part_bytes(*p, seq_len, out_dim) + planes;
         p->bytes = bytes > equal ? bytes : equal;
         if (p->equal_cuts || p->tiles.cuts == 1 || equal > VT_STATIC_SCRATCH_BYTES || bytes <= VT_STATIC_SCRATCH_BYTES) return 1;
