@@ -1,7 +1,11 @@
 """Input rows of a prefill in pageable memory, which cross in pieces of 64 through pinned memory from 97 rows on: the same rows in
 pageable, pinned and device memory leave the same residual stream and cache rows, bit for bit, at the edges of a piece and of that rule, with a
-longer prompt and a shorter one behind it, and the caller's buffer is free behind the call."""
+longer prompt and a shorter one behind it, and the caller's buffer is free behind the call.  And where that pinned memory cannot be had, the
+same rows cross without it."""
 import ctypes as C
+import os
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -43,3 +47,49 @@ def test_rows_from_any_memory():
             assert libhip.hipHostFree(pinned) == 0
     finally:
         hip.close()
+
+
+# Stands in front of the runtime's function where it is loaded first: no pinned block of more than 1 MB
+REFUSE = r"""
+#include <dlfcn.h>
+#include <stddef.h>
+int refused = 0;
+int hipHostMalloc(void **p, size_t n, unsigned flags) {
+    if (n > (1u << 20)) { refused++; *p = NULL; return 2; }
+    return ((int (*)(void **, size_t, unsigned))dlsym(dlopen("libamdhip64.so.7", RTLD_LAZY), "hipHostMalloc"))(p, n, flags);
+}
+"""
+
+# prefills of rows in pageable memory, in a process of their own; saves the residual streams
+PREFILLS = """
+import ctypes as C, sys
+sys.path.insert(0, sys.argv[1])
+refuse = C.CDLL(sys.argv[3], mode=C.RTLD_GLOBAL) if len(sys.argv) > 3 else None
+import numpy as np
+import hipsupport as H, vtsupport as S
+hip = H.Hip(kv_max=600)
+assert refuse is None or C.c_int.in_dll(refuse, "refused").value > 0
+hip.upload_decoder([S.Layer(12)], S.norm_weight(S.DIM, 97), 1)
+out = {}
+for n in (97, 300, 600):
+    print("prefill of", n, "rows", flush=True)
+    hip.pos = 0
+    out[str(n)] = hip.llm_prefill(S.f32_normal((n, S.DIM), 70 + n), want_x=True)
+assert hip.lib.tts_hip_error_count() == 0
+hip.close()
+np.savez(sys.argv[2], **out)
+"""
+
+
+def test_without_pinned_rows(tmp_path):
+    src, lib = tmp_path / "refuse.c", tmp_path / "librefuse.so"
+    src.write_text(REFUSE)
+    subprocess.check_call(["gcc", "-shared", "-fPIC", "-o", str(lib), str(src), "-ldl"])
+    got = []
+    for i, extra in enumerate(([], [str(lib)])):
+        npz = str(tmp_path / f"{i}.npz")
+        subprocess.check_call([sys.executable, "-c", PREFILLS, os.path.dirname(os.path.abspath(__file__)), npz] + extra, timeout=100)
+        got.append(np.load(npz))
+    for n in got[0].files:
+        assert np.isfinite(got[0][n]).all()
+        assert np.array_equal(got[0][n].view(np.uint32), got[1][n].view(np.uint32)), n

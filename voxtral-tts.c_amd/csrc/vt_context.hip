@@ -139,7 +139,11 @@ static int init_context(int kv_cache_max) {
         VT_TRY(hipMemset(*bufs[i].p, 0, bufs[i].bytes));
     }
     g_vt.bar_epoch = 0;
-    VT_TRY(hipHostMalloc((void **)&g_vt.h_rows, sizeof(float) * VT_DIM * (kv_cache_max < VT_PIN_ROWS ? kv_cache_max : VT_PIN_ROWS), hipHostMallocDefault));
+    /* (not to be had: prompts take the runtime's own copy) */
+    if (hipHostMalloc((void **)&g_vt.h_rows, sizeof(float) * VT_DIM * (kv_cache_max < VT_PIN_ROWS ? kv_cache_max : VT_PIN_ROWS), hipHostMallocDefault) != hipSuccess) {
+        g_vt.h_rows = NULL;
+        (void)hipGetLastError();
+    }
     VT_TRY(hipHostMalloc((void **)&g_vt.h_pin, sizeof(float) * VT_PIN_FLOATS, hipHostMallocDefault));
     if (vt_gemm_row_major_prepare()) return -1;
     VT_TRY(hipDeviceSynchronize());

@@ -532,7 +532,7 @@ void vt_launch_prefill_attention(float *d_out, uint16_t *d_hi, uint16_t *d_lo, c
 #define PF_PIECE_ROWS 64
 static int pf_take_rows(float *x, const float *rows, int n, uint16_t *hi, uint16_t *lo) {
     const float *norm = g_vt.h_layers[0].attn_norm;
-    if (n <= PF_STAGED_ROWS || n > VT_PIN_ROWS || !vt_pageable(rows)) {
+    if (n <= PF_STAGED_ROWS || n > VT_PIN_ROWS || !g_vt.h_rows || !vt_pageable(rows)) {
         VT_TRY(hipMemcpyAsync(x, rows, sizeof(float) * VT_DIM * n, hipMemcpyDefault, g_vt.stream));
         vt_launch_residual_norm_split(x, x, NULL, 0, 0, 0, norm, hi, lo, n);
         return 0;

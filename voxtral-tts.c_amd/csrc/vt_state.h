@@ -81,7 +81,7 @@ struct vt_state {
     unsigned long long bar_timeout; /* spin budget of a barrier in 100 MHz ticks; 0 = default */
     int *d_abort;
     uint16_t *d_dummy;            /* small resident block requested in place of a layer beyond the last */
-    float *h_rows;                /* pinned: a prefill's input rows on their way to the device, up to VT_PIN_ROWS */
+    float *h_rows;                /* pinned: a prefill's input rows on their way to the device, up to VT_PIN_ROWS; or NULL */
     float *h_pin;                 /* pinned staging: [3072 in][3072 out + flag], and a frame's hidden state, noise and results */
 
     /* generic scratch (prefill / acoustic / linear) */
