@@ -1110,6 +1110,7 @@ extern "C" int tts_hip_upload_audio_embeddings(const uint16_t *emb_bf16, int tot
     if (!(ac->audio_offsets = (int *)vt_dev_alloc(sizeof(int) * 2 * (1 + VT_AC_DIM_IN)))) return -1;
     VT_TRY(hipMemcpy(ac->audio_emb, emb_bf16, bytes, hipMemcpyDefault));
     VT_TRY(hipMemcpy(ac->audio_offsets, offsets, sizeof(int) * (1 + VT_AC_DIM_IN), hipMemcpyDefault));
+    VT_TRY(hipStreamSynchronize(NULL));      /* sources may have been device memory */
     ac->audio_rows = total_rows;
     return 0;
 }

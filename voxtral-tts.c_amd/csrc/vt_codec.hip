@@ -648,6 +648,7 @@ extern "C" int tts_hip_upload_codec_weights(void *codec_ptr) {
         l->ffn_scale = s->ffn_scale ? cd_upload(s->ffn_scale, CD_DIM) : NULL;
         l->window = s->window_size;
     }
+    ok = ok && !vt_check(hipStreamSynchronize(NULL), "codec weight copy");      /* sources may have been device memory */
     if (!ok) { vt_codec_free(); return -1; }
     g_cd.uploaded = 1;
     return 0;

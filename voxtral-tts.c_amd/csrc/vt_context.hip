@@ -251,7 +251,8 @@ static void *upload(const void *src, size_t bytes) {
     return d;
 }
 
-/* Sources may be host or device memory (hipMemcpyDefault resolves the kind). */
+/* Sources may be host or device memory (hipMemcpyDefault resolves the kind).  Copies of device memory return before they are made, on a
+ * stream that the kernels' does not wait for: every upload waits for its own. */
 static int upload_layer(vt_layer_dev *dst, const tts_hip_host_layer_t *s) {
     if (!s->wq_bf16 || !s->wk_bf16 || !s->wv_bf16 || !s->wo_bf16 || !s->w1_bf16 ||
         !s->w2_bf16 || !s->w3_bf16 || !s->attention_norm || !s->ffn_norm) {
@@ -277,6 +278,7 @@ static int upload_layer(vt_layer_dev *dst, const tts_hip_host_layer_t *s) {
     if (!(dst->w2 = (uint16_t *)upload(s->w2_bf16, (size_t)VT_DIM * VT_FFN * 2))) return -1;
     if (!(dst->attn_norm = (float *)upload(s->attention_norm, sizeof(float) * VT_DIM))) return -1;
     if (!(dst->ffn_norm = (float *)upload(s->ffn_norm, sizeof(float) * VT_DIM))) return -1;
+    VT_TRY(hipStreamSynchronize(NULL));
     return 0;
 }
 
@@ -319,6 +321,7 @@ extern "C" int tts_hip_upload_llm_norm(const float *norm) {
     if (need_init("tts_hip_upload_llm_norm")) return -1;
     if (!norm) { vt_set_error("tts_hip_upload_llm_norm: NULL"); return -1; }
     VT_TRY(hipMemcpy(g_vt.d_dec_norm, norm, sizeof(float) * VT_DIM, hipMemcpyDefault));
+    VT_TRY(hipStreamSynchronize(NULL));
     return 0;
 }
 
