@@ -251,6 +251,23 @@ static void *upload(const void *src, size_t bytes) {
     return d;
 }
 
+/* Rows of 3072 bf16 -> every second row of d (d: the first of them); a workgroup per row, 19 us per 9216 of them.  The upload of a layer from
+ * pageable memory takes 9 ms; 177 with the runtime's strided copies, which are made row by row. */
+__global__ void __launch_bounds__(VT_DIM / 8) vt_every_second_row_kernel(u32x4 *d, const u32x4 *s) {
+    d[(size_t)blockIdx.x * (2 * VT_DIM / 8) + threadIdx.x] = s[(size_t)blockIdx.x * (VT_DIM / 8) + threadIdx.x];
+}
+
+/* w [9216, 3072] -> every second row of d, by way of `stage`.  (Plain copies: under rocprofv3 the runtime's strided one, hipMemcpy2D,
+ * leaves its destination as it was where the source came from some allocators, and profiles then show products on zeros.) */
+static int upload_every_second_row(uint16_t *d, uint16_t *stage, const void *w) {
+    VT_TRY(hipMemcpy(stage, w, (size_t)VT_FFN * VT_DIM * 2, hipMemcpyDefault));
+    VT_TRY(hipStreamSynchronize(NULL));
+    hipLaunchKernelGGL(vt_every_second_row_kernel, dim3(VT_FFN), dim3(VT_DIM / 8), 0, g_vt.stream, (u32x4 *)d, (const u32x4 *)stage);
+    VT_TRY(hipGetLastError());
+    VT_TRY(hipStreamSynchronize(g_vt.stream));
+    return 0;
+}
+
 /* Sources may be host or device memory (hipMemcpyDefault resolves the kind).  Copies of device memory return before they are made, on a
  * stream that the kernels' does not wait for: every upload waits for its own. */
 static int upload_layer(vt_layer_dev *dst, const tts_hip_host_layer_t *s) {
@@ -267,15 +284,17 @@ static int upload_layer(vt_layer_dev *dst, const tts_hip_host_layer_t *s) {
     dst->wqkv = wqkv;
     uint16_t *w13 = (uint16_t *)vt_dev_alloc((size_t)2 * VT_FFN * row);
     dst->w13 = w13;
-    if (!wqkv || !w13) return -1;
+    uint16_t *w2 = (uint16_t *)vt_dev_alloc((size_t)VT_DIM * VT_FFN * 2);
+    dst->w2 = w2;
+    if (!wqkv || !w13 || !w2) return -1;
     VT_TRY(hipMemcpy(wqkv, s->wq_bf16, (size_t)VT_Q_DIM * row, hipMemcpyDefault));
     VT_TRY(hipMemcpy(wqkv + (size_t)VT_Q_DIM * VT_DIM, s->wk_bf16, (size_t)VT_KV_DIM * row, hipMemcpyDefault));
     VT_TRY(hipMemcpy(wqkv + (size_t)(VT_Q_DIM + VT_KV_DIM) * VT_DIM, s->wv_bf16, (size_t)VT_KV_DIM * row,
                      hipMemcpyDefault));
-    VT_TRY(hipMemcpy2D(w13, 2 * row, s->w1_bf16, row, row, VT_FFN, hipMemcpyDefault));
-    VT_TRY(hipMemcpy2D(w13 + VT_DIM, 2 * row, s->w3_bf16, row, row, VT_FFN, hipMemcpyDefault));
+    /* w2's place has the size of w1 and w3 */
+    if (upload_every_second_row(w13, w2, s->w1_bf16) || upload_every_second_row(w13 + VT_DIM, w2, s->w3_bf16)) return -1;
+    VT_TRY(hipMemcpy(w2, s->w2_bf16, (size_t)VT_DIM * VT_FFN * 2, hipMemcpyDefault));
     if (!(dst->wo = (uint16_t *)upload(s->wo_bf16, (size_t)VT_DIM * VT_Q_DIM * 2))) return -1;
-    if (!(dst->w2 = (uint16_t *)upload(s->w2_bf16, (size_t)VT_DIM * VT_FFN * 2))) return -1;
     if (!(dst->attn_norm = (float *)upload(s->attention_norm, sizeof(float) * VT_DIM))) return -1;
     if (!(dst->ffn_norm = (float *)upload(s->ffn_norm, sizeof(float) * VT_DIM))) return -1;
     VT_TRY(hipStreamSynchronize(NULL));
