@@ -22,7 +22,7 @@ void vt_launch_gemm_ex(float *d_C, int ldc, size_t plane_stride, const uint16_t 
 vt_gemm_plan vt_gemm_frag_plan(int M, int N, int K, int swiglu);
 /* The same on row-major weights W[N, K], N % 128 == 0, K % 64 == 0, in at most `most` cuts: d_y [M, N]; d_part: pl.cuts planes of
  * [M, N - pl.col0] (pl.cuts 1: not used) */
-vt_gemm_plan vt_gemm_row_major_plan(int M, int N, int K, int most, float *us);      /* us: what it is expected to take; infinite where no strip or tile can store N columns */
+vt_gemm_plan vt_gemm_row_major_plan(int M, int N, int K, int most, float *us);      /* us: what it is expected to take; infinite where no strip or tile takes so many columns or such a K */
 float vt_gemm_equal_us(int M, int N, int K, int cuts);      /* the same of vt_launch_gemm and, with cuts, the sum of its planes */
 int vt_gemm_row_major_prepare(void);      /* once per context; 0 / -1 */
 void vt_launch_gemm_row_major(float *d_y, float *d_part, const uint16_t *d_Ahi, const uint16_t *d_Alo, const uint16_t *d_W, int M, int N, int K,

@@ -93,15 +93,15 @@ static inline float gw_cost(int n_cu, const gw_format &f, int M, int N, int K, i
 
 /* Strips and these tiles store the rows that they have room for through one descriptor, whose size drops those past the last one.  Its
  * offsets have 32 bits, so all of these rows have to lie within them, not only those that exist: at 16,640,000 columns row 65 of a tile
- * would be row 0. */
-static inline int gw_stores_fit(int rows, int N) { return 4ll * rows * N <= 0x7fffffff; }
+ * would be row 0.  The same holds for what they load: rows of activations and, up to 96 of a wave, of weights, 2 K bytes each. */
+static inline int gw_fits(int rows, int N, int K) { return 4ll * rows * N <= 0x7fffffff && 2ll * (rows > 96 ? rows : 96) * K <= 0x7fffffff; }
 
 static inline vt_gemm_plan gw_plan(int n_cu, const gw_format &f, int M, int N, int K, int swiglu, int most = VT_MAX_CUTS, float *us = NULL) {
     vt_gemm_plan best = {0, 64, 0, 1};
     float best_cost = 0.f;
     for (int tm = 80; tm <= 128; tm += 16)
         for (int tn : {128, 192, 256, 384}) {
-            if (N % tn || f.step_us[gw_width(tn)][gw_height(tm)] == 0.f || !gw_stores_fit(tm, N)) continue;
+            if (N % tn || f.step_us[gw_width(tn)][gw_height(tm)] == 0.f || !gw_fits(tm, N, K)) continue;
             const int mt = (M + tm - 1) / tm, nt = N / tn;
             /* whole tiles: as many as make full rounds over the CUs, or one round fewer, or all */
             const int full = mt * nt / n_cu;
@@ -164,7 +164,7 @@ static inline float gp_equal_us(int n_cu, int M, int N, int K, int cuts) {
 static inline vt_gemm_plan gp_row_major(int n_cu, int M, int N, int K, int most, float *us) {
     vt_gemm_plan pl = gw_plan(n_cu, gw_row_major, M, N, K, 0, most, us);
     if (pl.cuts == 1) pl.col0 = N;
-    if (vt_gemm_rows_ok(M, N, K) && gw_stores_fit((M + 7) / 8 * 8, N)) {
+    if (vt_gemm_rows_ok(M, N, K) && gw_fits((M + 7) / 8 * 8, N, K)) {
         const vt_gemm_plan strips = gp_few_rows(n_cu, N, 0);
         for (int cuts = 1; cuts <= strips.cuts && cuts <= most && cuts <= K / 64; cuts++) {
             const float t = gw_strip_us(n_cu, M, N, K, strips.tn, cuts);

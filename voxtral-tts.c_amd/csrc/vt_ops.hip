@@ -423,8 +423,8 @@ void vt_launch_linear(float *d_y, const float *d_x, const uint16_t *d_W, const f
  * planes summed in a fixed order.  linear_mfma_plan says whether the shape qualifies, how the product is divided and how many
  * bytes of work area (partial planes, then the two activation planes) the launches need; linear_mfma_run queues them on that
  * work area.  The products are the backbone's strips and tiles on the caller's weights as they lie (equal_cuts 0), or tiles
- * of 128 x 128 whose K is cut into equal ranges, the only ones with an address per row of results (of more than 4 to 67 million
- * columns, by the rows).
+ * of 128 x 128 whose K is cut into equal ranges, the only ones with an address per row (of more than 4 to 67 million
+ * columns, by the rows, or a K of more than 8 to 11 million).
  * The fixed work area of the entry point without allocation holds what equal ranges that make 192 such tiles take, and a shape
  * beyond that is refused there: where it holds that, the plan is one that fits too. */
 #define VT_STATIC_SCRATCH_BYTES ((size_t)16 << 20)
