@@ -34,10 +34,14 @@ def test_windows_and_token_counts(n_frames, windows):
         S.oracle().orc_set_threads(1)
 
 
-@pytest.mark.parametrize("n_frames", [151, 212, 255])
+IN_PLACE = [151, 212, 255]
+
+
+@pytest.mark.parametrize("n_frames", IN_PLACE)
 def test_v_where_the_product_left_it(n_frames):
-    """From 1024 rows on v is read from the q|k|v product's result where its columns are whole or in one plane (1208 and
-    1696 rows here, 2040 in the last stage of 255 frames); fewer rows have it copied or summed from several planes."""
+    """From 1024 rows on v is read from the q|k|v product's result where its columns are in one plane (1208, 1696 and 2040 rows
+    here, all columns in one; all whole, and some: 512 and 527 frames in test_gpu_mixed_plans.py); fewer rows have it copied or summed from
+    several planes."""
     S.oracle().orc_set_threads(16)
     hc = K.HostCodec(9, distinct_layers=2)
     cs = hc.struct()

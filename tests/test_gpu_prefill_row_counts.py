@@ -1,5 +1,5 @@
-"""The prefill's products take their tiles and K cuts from the row count: up to 64 rows the 64-column tiles of
-vt_gemm_rows.hip (one instance per 8 rows, 8 waves up to 40 rows and 4 beyond), then the 96- and 128-row tiles
+"""The prefill's products take their tiles and K cuts from the row count: up to 64 rows the column strips of
+vt_gemm_rows.hip (one instance per 8 rows), then the tiles of 80 to 128 rows
 of vt_gemm_wide.hip.  Row counts at the edges of those, alone and as a continued prompt, against the oracle
 (rows, cache rows, and the decode step that reads them)."""
 import pytest
@@ -14,7 +14,11 @@ def test_prefill_row_counts_of_the_few_row_tiles(chunks):
     _prefill_case(2, chunks, sum(chunks) + 4, lambda n: range(n))
 
 
-@pytest.mark.parametrize("chunks", [[96, 97], [128, 129], [192, 193], [225], [256, 257], [288, 289]])
+# the last three: 128 x 256 whole with SiLU, 96 x 256 whole, 128 x 256 in cuts (test_plans_cpu.py: every tile is run by one of the lists)
+WIDE = [[96, 97], [128, 129], [192, 193], [225], [256, 257], [288, 289], [350], [850], [1130]]
+
+
+@pytest.mark.parametrize("chunks", WIDE)
 def test_prefill_row_counts_of_the_wide_tiles(chunks):
     _prefill_case(1, chunks, sum(chunks) + 4, lambda n: range(0, n, 3))
 
