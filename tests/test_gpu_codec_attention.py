@@ -76,8 +76,8 @@ def test_an_odd_token_count_on_workgroups_of_16():
 
 @pytest.mark.parametrize("n_frames", [513, 1030, 2049])
 def test_four_tokens_to_a_lane_group(n_frames):
-    """Rows that give two tokens to a lane group more workgroups than compute units: 4104 and 8240 rows in the last
-    stage, and 4098 already in the second, where the last lane group has two of its four.  With windows of 2, 4,
+    """Rows that give two tokens to a lane group more workgroups than compute units: 4104, 8240 and 16392 rows in the last
+    stage, 4120 in the third, and 4098 already in the second, where the last lane group has two of its four.  With windows of 2, 4,
     8 and 16 a sample depends on fewer than 40 frames in front of it, so the ends of a long decode are those of short
     ones, up to the sums of another plan."""
     hc = K.HostCodec(8, distinct_layers=2)

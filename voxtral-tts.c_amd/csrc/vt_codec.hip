@@ -258,9 +258,11 @@ struct cd_softmax {
  * us; 1003 rows, window 2, 8 / 8.5; 1696 rows, window 16, 17.5 / 23.4; 168 rows, window 16, 16 / 5.5. */
 #define CD_ATT_SPLIT_BELOW 1024
 /* NT = 4 has one workgroup to a CU (233 registers) that takes 1.3 .. 1.8 times as long as two tokens' does, so it pays
- * from where NT = 2 has more than one to a CU on.  Measured, us, NT = 2 / 4: 2800 rows, window 8, 14.8 / 18.8; 4000,
- * window 8, 20 / 23; 4008, window 16, 30.4 / 29.7; 5600, window 16, 48 / 40; 6000, window 8, 33 / 30; 8024, window 16,
- * 67 / 56; 12000, window 16, 106 / 86. */
+ * from where NT = 2 has more than one to a CU on (4097 rows).  Measured, us, NT = 2 / 4: window 8: 2800 rows 14.8 / 18.8, 4000 20 / 23,
+ * 4120 27.0 / 23.0, 4800 28.2 / 24.5, 5600 34.2 / 27.3, 8240 46.6 / 47.2, 11200 56.7 / 55.8; window 16: 4160 41.5 / 31.6, 5600
+ * 48.5 / 39.1, 8024 67 / 56, 8240 70.0 / 69.0, 8800 70.0 / 76.3, 9600 73.4 / 78.1, 10400 76.3 / 81.5, 11200 82.5 / 83.3, 16480 140.6 / 132.7,
+ * 22400 191.7 / 164.7; window 4: 4120 20.9 / 18.7.  (With two tokens from 8200 to 10900 rows decodes of 1100 to 1300 frames, 5.0 to 5.6 ms, take
+ * as long: not kept.) */
 template <int NT>
 __global__ void __launch_bounds__(64 * CD_HEADS)
 vt_codec_attention_kernel(cd_planes out, const float *__restrict__ qkv, cd_v_rows vs, int T, int window,

@@ -53,9 +53,10 @@ static inline vt_gemm_plan gp_few_rows(int n_cu, int N, int swiglu) {
  * The backbone's 192 columns divide 6144 and 3072 into 32 and 16 tiles, so that 1, 2, 4, .. row tiles fill the 256 CUs
  * where 256-column tiles come in multiples of 192 items: q|k|v / output / down at 700 rows 57.5 / 40.7 / 79.4 -> 51.1 / 37.2 /
  * 72.5 us, at 1000 75.0 / 53.3 / 104.9 -> 68.5 / 49.2 / 97.0, output / down at 1531 73.3 / 149.4 -> 67.1 / 140.6.
- * Measured against every tile and cut count at 47 row counts from 65 to 2048 of the backbone's products, the plan taken is 0.3 % behind the
- * fastest on average, at worst 5.5 % (q|k|v at 113 rows, 80 x 256 in 5 cuts instead of 4); for the codec's at 108 of 65 to 8024
- * rows, 0.6 % and at worst 8.1 % (output at 128 rows).  Single products exchanged inside prefills of 150 to 1531 rows were at most 2.7 %
+ * Measured against every tile and cut count at 19 row counts from 65 to 1531 of the backbone's four products, the plan taken is 0.8 % behind
+ * the fastest on average, at worst 5.2 % (down at 1200 rows, 128 x 384 in 3 cuts instead of 80 x 384 in 2); for the codec's at 17 row counts from
+ * 84 to 8024, 0.6 % and at worst 6.9 %, which is how far two measurements of one division of the work (listed as whole and as cut columns)
+ * are apart.  Single products exchanged inside prefills of 150 to 1531 rows were at most 2.7 %
  * of the prefill faster (gate|up at 700 rows, 96 x 384 in part cut).  Tiles x 384, which draw less power per product, are taken from 400 rows on
  * (gate|up) and from 690 (down): below, too few items are left for the CUs.  80 and 112 rows, where those of 96 and 128 have many to pad: us of
  * the four products at 200 / 226 / 290 / 400 / 800 rows 140 / 144 / 173 / 197 / 334 -> 130 / 136 / 163 / 186 / 322, a prefill of 226 rows 4274 -> 4020. */

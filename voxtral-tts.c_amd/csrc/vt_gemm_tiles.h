@@ -118,18 +118,20 @@ __device__ __forceinline__ void gm_store_quad(__amdgpu_buffer_rsrc_t C, int at, 
 }
 
 /* ---- more than 64 rows ---------------------------------------------------------------------------------
- * A wave owns MB x 32 rows (MB 3 or 4) x 64 or 96 columns: the weights of its columns are nobody else's among the
+ * A wave owns 80 to 128 rows (gw_shape) x 64 or 96 columns: the weights of its columns are nobody else's among the
  * waves that work on the same K step, so they go from global memory straight into the B operand registers, and
  * only the activation planes pass through the LDS: 8 KB of fragment reads per 16 matrix instructions, half
  * the LDS bandwidth (a 64 x 64 wave tile with both operands in LDS, vt_gemm_mfma_kernel, needs three quarters).
  * One workgroup of four waves per CU (a wave may then use the whole register file of its SIMD: up to 128
- * accumulator registers, 192 with 96 columns (all 512 are then in use), two sets of weight registers, two sets of fragments), in one of these shapes:
- *   CW = 4: four waves side by side, tile MB*32 x 256 (NB = 2 blocks of 32 columns per wave) or x 384 (NB = 3); the planes of one K
+ * accumulator registers, 192 with 96 columns, in paired tiles 160 (80 x 256), 224 (112 x 256) and 240 (80 rows, 96 columns); two sets of weight
+ * registers, two sets of fragments.  With 96 columns and in the paired tiles all 512 are about used up: 112 x 256 spills 12 and 80 x 384 one,
+ * which their times in vt_gemm_plans.h hold), in one of these shapes:
+ *   CW = 4: four waves side by side, tiles x 256 (NB = 2 blocks of 32 columns per wave) or x 384 (NB = 3); the planes of one K
  *           step serve four waves.  With 384 columns a fragment read from LDS serves 3 blocks instead of 2: a third less LDS traffic
  *           per matrix instruction, which is time and, under the card's power limit, clock: executed TFLOP/s at 4096 rows of
  *           3072 x 9216 1146 with 128 x 256, 1253 with 128 x 192, 1420 with 128 x 384, of 6144 x 3072 1234 / 1153 / 1346 (96 x 512: 989,
  *           spilled; 64 x 512 1234 and 160 x 384 1159 on a box 5 % slower).  In prefills of 1531 rows, q|k|v / gate|up 101 / 280 -> 87 / 259 us;
- *   CW = 2: two waves side by side and two K steps at a time, tile MB*32 x 128 (NB = 2 blocks of 32 columns per wave) or
+ *   CW = 2: two waves side by side and two K steps at a time, tiles x 128 (NB = 2 blocks of 32 columns per wave) or
  *           x 192 (NB = 3); the two halves of K are added through LDS at the end.  For row counts whose 256-column
  *           tiles do not deal out over the CUs, at the price of more plane traffic (L2 and LDS stores) per matrix
  *           instruction: operand bytes per cycle of matrix instructions 32 (128 x 256), 37 (128 x 192), 47 (128 x 128).
@@ -223,7 +225,7 @@ vt_gemm_wide_kernel(gw_list list, const uint16_t *Ahi, const uint16_t *Alo, int 
     constexpr int AHEAD = MB * NB > (PAIR ? 14 : 9) ? 1 : 2;       /* steps between the request of a step's planes and their store (registers) */
     /* The first requests of an item go out in front of the stores of the one before it, where registers for both are left (where
      * they were not, a launch's first loads were spilled one by one, each behind a wait: 5 us). */
-    constexpr bool EARLY = CW == 4 || MB == 3 || (PAIR && NB == 2);
+    constexpr bool EARLY = CW == 4 || MB == 3;
     constexpr int PLANE = shape::PLANE, GROUP = 2 * PLANE, STAGE = shape::STAGE;
     int *tile_exp = reinterpret_cast<int *>(lds + 2 * STAGE);      /* T::SCALED: the exponents of the tile's rows */
     const int lane = (int)threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);

@@ -43,7 +43,7 @@
  * 7 to 9 us in front and behind (queries 2.1, their planes 1.5, merge and stores 2.5: each of them code that is run once and
  * comes from memory).  us per launch inside a prefill of 37 / 226 / 512 / 1531 rows: 7.7 / 12.2 / 17.8 /
  * 65.6, where 16 queries per wave on 16 x 16 x 32 instructions, four waves and tiles copied through registers took 9.0 / 15.8 /
- * 24.5 / 125.5; at 37 rows 9.4 now with the tiles made here (PA_HERE_ROWS), which took a launch of 6.1. */
+ * 24.5 / 125.5; at 37 rows 10.9 now with the tiles made here (PA_HERE_ROWS), which took a launch of 6.1. */
 /* Queries per workgroup: 16 as long as that gives the CUs more to do at once (twice the workgroups, each half as many
  * rounds of tiles), 32 from where every CU is busy either way and the tiles are copied half as often.  us per launch
  * at 37 / 226 / 512 / 1000 / 1531 / 3000 rows, 16: 7.5 / 10.5 / 16.4 / 34.4 / 70.1 / 236.7, 32: 9.0 / 14.3 / 22.4 / 39.5 /
